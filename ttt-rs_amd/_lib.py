@@ -3,10 +3,12 @@ been built: there is no CPU fallback anywhere in this package."""
 from __future__ import annotations
 
 import ctypes as C
+import importlib.util
 import os
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(HERE, "lib", "libttt_mi355x.so")
+HOST_PATH = os.path.join(HERE, "lib", "_ttt_torch.so")
 
 TTT_OK, TTT_ERR_SHAPE, TTT_ERR_UNSUPPORTED, TTT_ERR_HIP, TTT_ERR_NULL = 0, -1, -2, -3, -4
 TTT_F32, TTT_BF16 = 0, 1
@@ -107,3 +109,24 @@ def lib() -> C.CDLL:
 def check(rc: int):
     if rc != TTT_OK:
         raise TttError(rc, lib().ttt_last_error().decode())
+
+
+_host = None
+
+
+def host():
+    """The native host path (csrc/ttt_torch.cpp): checks, allocates and calls the library for the functions of inner.py."""
+    global _host
+    if _host is None:
+        lib()
+        if not os.path.exists(HOST_PATH):
+            raise ImportError(
+                f"{HOST_PATH} is missing: build it first (python ttt-rs_amd/build.py); "
+                "this package has no fallback path")
+        import torch  # noqa: F401  (its libraries have to be loaded before the extension)
+        spec = importlib.util.spec_from_file_location("_ttt_torch", HOST_PATH)
+        m = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(m)
+        m.set_error(TttError)
+        _host = m
+    return _host

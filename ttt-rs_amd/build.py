@@ -87,6 +87,34 @@ def build_host_driver() -> str:
     return DRIVER_PATH
 
 
+TORCH_PATH = os.path.join(LIB_DIR, "_ttt_torch.so")
+
+
+def build_torch_binding() -> str:
+    """The host path between torch tensors and the C ABI (csrc/ttt_torch.cpp), a CPython extension: plain host code
+    (g++), linked against the library and torch."""
+    import sysconfig
+
+    import torch
+    root = os.path.dirname(torch.__file__)
+    rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
+    abi = int(torch._C._GLIBCXX_USE_CXX11_ABI)
+    cmd = ["g++", "-std=c++17", "-O2", "-Wall", "-Wextra", "-fPIC", "-shared", "-fvisibility=hidden",
+           f"-D_GLIBCXX_USE_CXX11_ABI={abi}", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           "-isystem", os.path.join(root, "include"),
+           "-isystem", os.path.join(root, "include", "torch", "csrc", "api", "include"),
+           "-isystem", os.path.join(rocm, "include"), "-isystem", sysconfig.get_paths()["include"],
+           os.path.join(HERE, "csrc", "ttt_torch.cpp"), "-o", TORCH_PATH,
+           "-L", LIB_DIR, "-lttt_mi355x", "-L", os.path.join(root, "lib"), "-ltorch_python", "-ltorch_cpu", "-ltorch_hip",
+           "-lc10", "-lc10_hip", "-Wl,-rpath,$ORIGIN"]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        sys.stderr.write(res.stdout + res.stderr)
+        raise RuntimeError("g++ failed building " + TORCH_PATH)
+    return TORCH_PATH
+
+
 if __name__ == "__main__":
     print(build_library(verbose=True))
     print(build_host_driver())
+    print(build_torch_binding())

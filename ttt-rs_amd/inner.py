@@ -17,7 +17,7 @@ from typing import Optional
 import torch
 
 from . import _lib
-from ._lib import TttDesc, check, lib
+from ._lib import TttDesc, check, host, lib
 
 
 @dataclass
@@ -68,18 +68,6 @@ class TTTLinearState:
     bias: torch.Tensor
 
 
-def _ptr(t: Optional[torch.Tensor]):
-    return None if t is None else C.c_void_p(t.data_ptr())
-
-
-def _io_dtype(t: torch.Tensor) -> int:
-    if t.dtype == torch.float32:
-        return _lib.TTT_F32
-    if t.dtype == torch.bfloat16:
-        return _lib.TTT_BF16
-    raise _lib.TttError(_lib.TTT_ERR_UNSUPPORTED, f"activation dtype {t.dtype} (f32 or bf16 only)")
-
-
 def _need(t: torch.Tensor, shape, dtype, name):
     if tuple(t.shape) != tuple(shape):
         raise _lib.TttError(_lib.TTT_ERR_SHAPE, f"{name}: shape {tuple(t.shape)} != {tuple(shape)}")
@@ -88,39 +76,6 @@ def _need(t: torch.Tensor, shape, dtype, name):
     if not t.is_cuda:
         raise _lib.TttError(_lib.TTT_ERR_NULL, f"{name} is not a device tensor")
     return t.contiguous()
-
-
-def _seq_pitch(t: torch.Tensor) -> Optional[int]:
-    """Tokens between consecutive (batch, head) units if `t` ([B,H,seq,d] or [B,H,seq]) is a
-    window along seq of a dense tensor (what slicing dim 2 of a contiguous tensor gives), else None."""
-    trail = t.shape[3] if t.dim() == 4 else 1
-    st = t.stride()
-    if t.dim() == 4 and (st[3] != 1 or st[2] != trail):
-        return None
-    if t.dim() == 3 and st[2] != 1:
-        return None
-    if st[1] % trail or st[0] != t.shape[1] * st[1]:
-        return None
-    pitch = st[1] // trail
-    return pitch if pitch >= t.shape[2] else None
-
-
-def _common_pitch(seq: int, *tensors) -> int:
-    """The shared sequence pitch of the given windows, or 0 when they have to be packed."""
-    pitches = {_seq_pitch(t) for t in tensors}
-    if len(pitches) == 1 and None not in pitches:
-        p = pitches.pop()
-        return 0 if p == seq else p
-    return 0
-
-
-def _need_win(t: torch.Tensor, shape, dtype, name, pitch: int):
-    """Like _need, but keeps a sequence window in place when a pitch is in use."""
-    if pitch == 0:
-        return _need(t, shape, dtype, name)
-    if tuple(t.shape) != tuple(shape) or t.dtype != dtype or not t.is_cuda:
-        raise _lib.TttError(_lib.TTT_ERR_SHAPE, f"{name}: expected {tuple(shape)} {dtype} on the device")
-    return t
 
 
 def ttt_linear_forward_raw(xq, xk, xv, weight, bias, token_eta, ttt_lr_eta, ln_weight, ln_bias,
@@ -137,50 +92,9 @@ def ttt_linear_forward_raw(xq, xk, xv, weight, bias, token_eta, ttt_lr_eta, ln_w
     instead of states.  The result is to be handed to ttt_linear_backward_raw with the same value; the tensors keep
     their f32 [B,H,n,d,d] / [B,H,n,d] allocations whatever the format.
     """
-    B, H, seq, d = xq.shape
-    io = xq.dtype
-    # sequence windows of dense tensors are processed in place (desc.seq_stride) when inputs and
-    # the caller's output window share one pitch; anything else is packed first
-    pitch = _common_pitch(seq, xq, xk, xv, ttt_lr_eta, out) if out is not None else 0
-    xq = _need_win(xq, (B, H, seq, d), io, "xq", pitch)
-    xk = _need_win(xk, (B, H, seq, d), io, "xk", pitch)
-    xv = _need_win(xv, (B, H, seq, d), io, "xv", pitch)
-    lr = _need_win(ttt_lr_eta, (B, H, seq), io, "ttt_lr_eta", pitch)
-    per_batch = weight.dim() == 4
-    weight = _need(weight, (B, H, d, d) if per_batch else (H, d, d), torch.float32, "weight")
-    bias = _need(bias, (B, H, d) if per_batch else (H, d), torch.float32, "bias")
-    ln_weight = _need(ln_weight, (H, d), torch.float32, "ln_weight")
-    ln_bias = _need(ln_bias, (H, d), torch.float32, "ln_bias")
-    if token_eta.numel() < mini_batch:
-        raise _lib.TttError(_lib.TTT_ERR_SHAPE, "token_eta shorter than mini_batch")
-    te = token_eta.to(torch.float32).contiguous()
-    desc = TttDesc(B, H, seq, d, mini_batch, eps, checkpoint_interval, _io_dtype(xq), int(per_batch), pitch,
-                   int(packed_checkpoints), kernel_hint)
-    check(lib().ttt_linear_supported(C.byref(desc)))
-    dev = xq.device
-    if out is None or (pitch == 0 and not out.is_contiguous()):
-        dst, out = out, torch.empty((B, H, seq, d), dtype=io, device=dev)
-    else:
-        dst = None
-        out = _need_win(out, (B, H, seq, d), io, "out", pitch)
-    w_out = torch.empty((B, H, d, d), dtype=torch.float32, device=dev)
-    b_out = torch.empty((B, H, d), dtype=torch.float32, device=dev)
-    w_ck = b_ck = None
-    if want_checkpoints:
-        n = lib().ttt_linear_num_checkpoints(C.byref(desc))
-        w_ck = torch.empty((B, H, n, d, d), dtype=torch.float32, device=dev)
-        b_ck = torch.empty((B, H, n, d), dtype=torch.float32, device=dev)
-    stream = C.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
-    with torch.cuda.device(dev):
-        check(lib().ttt_linear_fwd(C.byref(desc), _ptr(xq), _ptr(xk), _ptr(xv), _ptr(weight), _ptr(bias),
-                                   _ptr(te), _ptr(lr), _ptr(ln_weight), _ptr(ln_bias), _ptr(out),
-                                   _ptr(w_out), _ptr(b_out), _ptr(w_ck), _ptr(b_ck), stream))
-    if dst is not None:
-        dst.copy_(out)
-        out = dst
-    if want_checkpoints:
-        return out, w_out, b_out, w_ck, b_ck
-    return out, w_out, b_out
+    return host().linear_forward(xq, xk, xv, weight, bias, token_eta, ttt_lr_eta, ln_weight, ln_bias, mini_batch, eps,
+                                 checkpoint_interval, want_checkpoints, out, int(packed_checkpoints), kernel_hint)
+
 
 
 def ttt_linear_adam_forward_raw(xq, xk, xv, weight, bias, token_eta, ttt_lr_eta, ln_weight, ln_bias, mini_batch: int,
@@ -190,38 +104,9 @@ def ttt_linear_adam_forward_raw(xq, xk, xv, weight, bias, token_eta, ttt_lr_eta,
     (rust/core/src/linear_adam.rs:183-236 looped as rust/core/src/inner.rs:25-50).  Arguments as
     ttt_linear_forward_raw; moments = (weight_m, bias_m, weight_v, bias_v) per batch element to continue an earlier call
     at `step`, or None for a fresh state.  Returns (output, weight, bias, (weight_m, bias_m, weight_v, bias_v), step)."""
-    B, H, seq, d = xq.shape
-    io = xq.dtype
-    xq = _need(xq, (B, H, seq, d), io, "xq")
-    xk = _need(xk, (B, H, seq, d), io, "xk")
-    xv = _need(xv, (B, H, seq, d), io, "xv")
-    per_batch = weight.dim() == 4
-    W0 = _need(weight, (B, H, d, d) if per_batch else (H, d, d), torch.float32, "weight")
-    b0 = _need(bias, (B, H, d) if per_batch else (H, d), torch.float32, "bias")
-    te = _need(token_eta[:mini_batch], (mini_batch,), torch.float32, "token_eta")
-    lr = _need(ttt_lr_eta, (B, H, seq), io, "ttt_lr_eta")
-    gam = _need(ln_weight, (H, d), torch.float32, "ln_weight")
-    bet = _need(ln_bias, (H, d), torch.float32, "ln_bias")
-    dev = xq.device
-    f32 = dict(dtype=torch.float32, device=dev)
-    null = C.c_void_p(None)
-    m_in = [null] * 4
-    if moments is not None:
-        shapes = ((B, H, d, d), (B, H, d), (B, H, d, d), (B, H, d))
-        m_in = [_ptr(_need(t, sh, torch.float32, "moment")) for t, sh in zip(moments, shapes)]
-    desc = TttDesc(B, H, seq, d, mini_batch, eps, 1, _io_dtype(xq), 1 if per_batch else 0, 0, 0, 0)
-    check(lib().ttt_linear_adam_supported(C.byref(desc)))
-    out = torch.empty((B, H, seq, d), dtype=io, device=dev)
-    W, b = torch.empty((B, H, d, d), **f32), torch.empty((B, H, d), **f32)
-    mo = (torch.empty((B, H, d, d), **f32), torch.empty((B, H, d), **f32), torch.empty((B, H, d, d), **f32),
-          torch.empty((B, H, d), **f32))
-    stream = C.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
-    with torch.cuda.device(dev):
-        check(lib().ttt_linear_adam_fwd(C.byref(desc), _ptr(xq), _ptr(xk), _ptr(xv), _ptr(W0), _ptr(b0), *m_in, int(step),
-                                        C.c_float(beta1), C.c_float(beta2), C.c_float(adam_eps), C.c_float(adam_lr),
-                                        _ptr(te), _ptr(lr), _ptr(gam), _ptr(bet), _ptr(out), _ptr(W), _ptr(b),
-                                        *[_ptr(t) for t in mo], stream))
-    return out, W, b, mo, step + seq // mini_batch
+    return host().linear_adam_forward(xq, xk, xv, weight, bias, token_eta, ttt_lr_eta, ln_weight, ln_bias, mini_batch,
+                                      beta1, beta2, adam_eps, adam_lr, moments, int(step), eps)
+
 
 
 def ttt_linear_backward_raw(xq, xk, xv, weight, bias, token_eta, ttt_lr_eta, ln_weight, ln_bias,
@@ -237,58 +122,10 @@ def ttt_linear_backward_raw(xq, xk, xv, weight, bias, token_eta, ttt_lr_eta, ln_
     (backward/launch.rs:427-437): grad_xq, grad_xk, grad_xv, grad_weight [B,H,d,d],
     grad_bias [B,H,d], grad_ttt_lr_eta, grad_token_eta [seq], grad_ln_weight, grad_ln_bias.
     """
-    B, H, seq, d = xq.shape
-    io = xq.dtype
-    xq = _need(xq, (B, H, seq, d), io, "xq")
-    xk = _need(xk, (B, H, seq, d), io, "xk")
-    xv = _need(xv, (B, H, seq, d), io, "xv")
-    go = _need(grad_output, (B, H, seq, d), io, "grad_output")
-    lr = _need(ttt_lr_eta, (B, H, seq), io, "ttt_lr_eta")
-    per_batch = weight.dim() == 4
-    weight = _need(weight, (B, H, d, d) if per_batch else (H, d, d), torch.float32, "weight")
-    bias = _need(bias, (B, H, d) if per_batch else (H, d), torch.float32, "bias")
-    ln_weight = _need(ln_weight, (H, d), torch.float32, "ln_weight")
-    ln_bias = _need(ln_bias, (H, d), torch.float32, "ln_bias")
-    te = token_eta.to(torch.float32).contiguous()
-    desc = TttDesc(B, H, seq, d, mini_batch, eps, checkpoint_interval, _io_dtype(xq), int(per_batch), 0,
-                   int(packed_checkpoints), kernel_hint)
-    check(lib().ttt_linear_bwd_supported(C.byref(desc)))
-    n = lib().ttt_linear_num_checkpoints(C.byref(desc))
-    w_ck = _need(weight_ckpt, (B, H, n, d, d), torch.float32, "weight_ckpt")
-    b_ck = _need(bias_ckpt, (B, H, n, d), torch.float32, "bias_ckpt")
-    if grad_weight_out is not None:
-        grad_weight_out = _need(grad_weight_out, (B, H, d, d), torch.float32, "grad_weight_out")
-        grad_bias_out = _need(grad_bias_out, (B, H, d), torch.float32, "grad_bias_out")
-    dev = xq.device
-    g = dict(
-        grad_xq=torch.empty_like(xq), grad_xk=torch.empty_like(xq), grad_xv=torch.empty_like(xq),
-        grad_weight=torch.empty((B, H, d, d), dtype=torch.float32, device=dev),
-        grad_bias=torch.empty((B, H, d), dtype=torch.float32, device=dev),
-        grad_ttt_lr_eta=torch.empty_like(lr),
-        grad_token_eta=torch.empty((seq,), dtype=torch.float32, device=dev),
-        grad_ln_weight=torch.empty((H, d), dtype=torch.float32, device=dev),
-        grad_ln_bias=torch.empty((H, d), dtype=torch.float32, device=dev),
-    )
-    stream = C.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
-    # a desc whose backward can use a workspace (two workgroups per unit) gets one: ttt_linear_bwd_ws
-    ws_bytes = lib().ttt_linear_bwd_workspace_bytes(C.byref(desc))
-    if ws_bytes < 0:
-        check(int(ws_bytes))
-    args = (C.byref(desc), _ptr(xq), _ptr(xk), _ptr(xv), _ptr(weight), _ptr(bias), _ptr(te), _ptr(lr),
-            _ptr(ln_weight), _ptr(ln_bias), _ptr(w_ck), _ptr(b_ck), _ptr(go), _ptr(grad_weight_out),
-            _ptr(grad_bias_out), _ptr(g["grad_xq"]), _ptr(g["grad_xk"]), _ptr(g["grad_xv"]),
-            _ptr(g["grad_weight"]), _ptr(g["grad_bias"]), _ptr(g["grad_ttt_lr_eta"]),
-            _ptr(g["grad_token_eta"]), _ptr(g["grad_ln_weight"]), _ptr(g["grad_ln_bias"]))
-    with torch.cuda.device(dev):
-        if ws_bytes > 0 and workspace is not False:
-            if workspace is None or workspace is True:
-                workspace = torch.empty((int(ws_bytes),), dtype=torch.uint8, device=dev)
-            if workspace.numel() * workspace.element_size() < ws_bytes:
-                raise _lib.TttError(_lib.TTT_ERR_SHAPE, f"workspace holds fewer than {ws_bytes} bytes")
-            check(lib().ttt_linear_bwd_ws(*args, _ptr(workspace), stream))
-        else:
-            check(lib().ttt_linear_bwd(*args, stream))
-    return g
+    return host().linear_backward(xq, xk, xv, weight, bias, token_eta, ttt_lr_eta, ln_weight, ln_bias, weight_ckpt,
+                                  bias_ckpt, grad_output, mini_batch, eps, checkpoint_interval, grad_weight_out,
+                                  grad_bias_out, int(packed_checkpoints), kernel_hint, workspace)
+
 
 
 def ttt_mlp_forward_raw(xq, xk, xv, w1, b1, w2, b2, token_eta, ttt_lr_eta, ln_weight, ln_bias,
@@ -299,46 +136,9 @@ def ttt_mlp_forward_raw(xq, xk, xv, w1, b1, w2, b2, token_eta, ttt_lr_eta, ln_we
     Returns (output, w1_out, b1_out, w2_out, b2_out), state per batch element.
     save_for_backward: call ttt_mlp_fwd_saving instead and return a sixth element, the `saved` buffer that
     ttt_mlp_backward_raw(saved=...) consumes (the backward then skips its own forward sweep)."""
-    B, H, seq, d = xq.shape
-    m = w1.shape[-1]
-    io = xq.dtype
-    xq = _need(xq, (B, H, seq, d), io, "xq")
-    xk = _need(xk, (B, H, seq, d), io, "xk")
-    xv = _need(xv, (B, H, seq, d), io, "xv")
-    lr = _need(ttt_lr_eta, (B, H, seq), io, "ttt_lr_eta")
-    per_batch = w1.dim() == 4
-    lead = (B, H) if per_batch else (H,)
-    if m != 4 * d:
-        raise _lib.TttError(_lib.TTT_ERR_UNSUPPORTED, f"mlp_dim {m} != 4*head_dim (only expansion 4)")
-    w1 = _need(w1, lead + (d, m), torch.float32, "w1")
-    b1 = _need(b1, lead + (m,), torch.float32, "b1")
-    w2 = _need(w2, lead + (m, d), torch.float32, "w2")
-    b2 = _need(b2, lead + (d,), torch.float32, "b2")
-    ln_weight = _need(ln_weight, (H, d), torch.float32, "ln_weight")
-    ln_bias = _need(ln_bias, (H, d), torch.float32, "ln_bias")
-    if token_eta.numel() < mini_batch:
-        raise _lib.TttError(_lib.TTT_ERR_SHAPE, "token_eta shorter than mini_batch")
-    te = token_eta.to(torch.float32).contiguous()
-    desc = TttDesc(B, H, seq, d, mini_batch, eps, 1, _io_dtype(xq), int(per_batch), 0, 0, kernel_hint)
-    check(lib().ttt_mlp_supported(C.byref(desc)))
-    dev = xq.device
-    f32 = dict(dtype=torch.float32, device=dev)
-    out = torch.empty_like(xq)
-    o = [torch.empty((B, H, d, m), **f32), torch.empty((B, H, m), **f32),
-         torch.empty((B, H, m, d), **f32), torch.empty((B, H, d), **f32)]
-    stream = C.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
-    with torch.cuda.device(dev):
-        if save_for_backward:
-            check(lib().ttt_mlp_fwd_saving_supported(C.byref(desc)))
-            saved = torch.empty((lib().ttt_mlp_bwd_workspace_bytes(C.byref(desc)) + 3) // 4, **f32)
-            check(lib().ttt_mlp_fwd_saving(C.byref(desc), _ptr(xq), _ptr(xk), _ptr(xv), _ptr(w1), _ptr(b1), _ptr(w2),
-                                           _ptr(b2), _ptr(te), _ptr(lr), _ptr(ln_weight), _ptr(ln_bias), _ptr(out),
-                                           *[_ptr(x) for x in o], _ptr(saved), stream))
-            return (out, *o, saved)
-        check(lib().ttt_mlp_fwd(C.byref(desc), _ptr(xq), _ptr(xk), _ptr(xv), _ptr(w1), _ptr(b1), _ptr(w2),
-                                _ptr(b2), _ptr(te), _ptr(lr), _ptr(ln_weight), _ptr(ln_bias), _ptr(out),
-                                *[_ptr(x) for x in o], stream))
-    return (out, *o)
+    return host().mlp_forward(xq, xk, xv, w1, b1, w2, b2, token_eta, ttt_lr_eta, ln_weight, ln_bias, mini_batch, eps,
+                              kernel_hint, save_for_backward)
+
 
 
 def ttt_mlpn_forward_raw(xq, xk, xv, weights, biases, token_eta, ttt_lr_eta, ln_weight, ln_bias, mini_batch: int,
@@ -346,34 +146,9 @@ def ttt_mlpn_forward_raw(xq, xk, xv, weights, biases, token_eta, ttt_lr_eta, ln_
     """One call of ttt_mlpn_fwd on the current stream: TTTMLP2/3/4::forward (rust/core/src/mlp2.rs, mlp3.rs, mlp4.rs
     looped as rust/core/src/inner.rs:25-50).  weights / biases: lists of the n_hidden + 1 layers, [H,in,out] / [H,out] or
     with a leading batch dimension.  Returns (output, weights_out, biases_out), state per batch element."""
-    B, H, seq, d = xq.shape
-    io = xq.dtype
-    n_hidden = len(weights) - 1
-    m = 4 * d
-    dims = [d] + [m] * n_hidden + [d]
-    xq = _need(xq, (B, H, seq, d), io, "xq")
-    xk = _need(xk, (B, H, seq, d), io, "xk")
-    xv = _need(xv, (B, H, seq, d), io, "xv")
-    per_batch = weights[0].dim() == 4
-    lead = (B, H) if per_batch else (H,)
-    Ws = [_need(w, lead + (dims[i], dims[i + 1]), torch.float32, f"weights[{i}]") for i, w in enumerate(weights)]
-    bs = [_need(b, lead + (dims[i + 1],), torch.float32, f"biases[{i}]") for i, b in enumerate(biases)]
-    te = _need(token_eta[:mini_batch], (mini_batch,), torch.float32, "token_eta")
-    lr = _need(ttt_lr_eta, (B, H, seq), io, "ttt_lr_eta")
-    gam = _need(ln_weight, (H, d), torch.float32, "ln_weight")
-    bet = _need(ln_bias, (H, d), torch.float32, "ln_bias")
-    dev = xq.device
-    desc = TttDesc(B, H, seq, d, mini_batch, eps, 1, _io_dtype(xq), 1 if per_batch else 0, 0, 0, 0)
-    check(lib().ttt_mlpn_supported(C.byref(desc), n_hidden))
-    out = torch.empty((B, H, seq, d), dtype=io, device=dev)
-    Wo = [torch.empty((B, H, dims[i], dims[i + 1]), dtype=torch.float32, device=dev) for i in range(n_hidden + 1)]
-    bo = [torch.empty((B, H, dims[i + 1]), dtype=torch.float32, device=dev) for i in range(n_hidden + 1)]
-    arr = lambda ts: (C.c_void_p * len(ts))(*[t.data_ptr() for t in ts])
-    stream = C.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
-    with torch.cuda.device(dev):
-        check(lib().ttt_mlpn_fwd(C.byref(desc), n_hidden, _ptr(xq), _ptr(xk), _ptr(xv), arr(Ws), arr(bs), _ptr(te),
-                                 _ptr(lr), _ptr(gam), _ptr(bet), _ptr(out), arr(Wo), arr(bo), stream))
-    return out, Wo, bo
+    return host().mlpn_forward(xq, xk, xv, list(weights), list(biases), token_eta, ttt_lr_eta, ln_weight, ln_bias,
+                               mini_batch, eps)
+
 
 
 def ttt_mlp_backward_raw(xq, xk, xv, w1, b1, w2, b2, token_eta, ttt_lr_eta, ln_weight, ln_bias, d_out,
@@ -391,71 +166,9 @@ def ttt_mlp_backward_raw(xq, xk, xv, w1, b1, w2, b2, token_eta, ttt_lr_eta, ln_w
     reverse scan's products in f32 where it would round their operands to bf16 (bf16 I/O, head_dim <= 96).
     saved: the buffer a forward with save_for_backward=True returned (same inputs, same hint): ttt_mlp_bwd_saved, which
     consumes it."""
-    B, H, seq, d = xq.shape
-    m = w1.shape[-1]
-    io = xq.dtype
-    xq = _need(xq, (B, H, seq, d), io, "xq")
-    xk = _need(xk, (B, H, seq, d), io, "xk")
-    xv = _need(xv, (B, H, seq, d), io, "xv")
-    d_out = _need(d_out, (B, H, seq, d), io, "d_out")
-    lr = _need(ttt_lr_eta, (B, H, seq), io, "ttt_lr_eta")
-    per_batch = w1.dim() == 4
-    lead = (B, H) if per_batch else (H,)
-    if m != 4 * d:
-        raise _lib.TttError(_lib.TTT_ERR_UNSUPPORTED, f"mlp_dim {m} != 4*head_dim (only expansion 4)")
-    w1 = _need(w1, lead + (d, m), torch.float32, "w1")
-    b1 = _need(b1, lead + (m,), torch.float32, "b1")
-    w2 = _need(w2, lead + (m, d), torch.float32, "w2")
-    b2 = _need(b2, lead + (d,), torch.float32, "b2")
-    ln_weight = _need(ln_weight, (H, d), torch.float32, "ln_weight")
-    ln_bias = _need(ln_bias, (H, d), torch.float32, "ln_bias")
-    if token_eta.numel() < mini_batch:
-        raise _lib.TttError(_lib.TTT_ERR_SHAPE, "token_eta shorter than mini_batch")
-    te = token_eta.to(torch.float32).contiguous()
-    desc = TttDesc(B, H, seq, d, mini_batch, eps, 1, _io_dtype(xq), int(per_batch), 0)
-    desc.kernel_hint = int(kernel_hint)
-    check(lib().ttt_mlp_supported(C.byref(desc)))
-    dev = xq.device
-    f32 = dict(dtype=torch.float32, device=dev)
-    shapes = [(B, H, d, m), (B, H, m), (B, H, m, d), (B, H, d)]
-    up = [None] * 4
-    if d_state_out is not None:
-        up = [_need(g, sh, torch.float32, "d_state_out") for g, sh in zip(d_state_out, shapes)]
-    if into is not None:
-        g_act = [into["d_xq"], into["d_xk"], into["d_xv"]]
-        g_st = [into["d_W1"], into["d_b1"], into["d_W2"], into["d_b2"]]
-        g_lr, g_te, g_gam, g_bet = into["d_lr"], into["d_token_eta"], into["d_gamma"], into["d_beta"]
-        for t, sh in zip(g_act + g_st + [g_lr, g_te, g_gam, g_bet],
-                         [xq.shape] * 3 + shapes + [lr.shape, (seq,), (H, d), (H, d)]):
-            if tuple(t.shape) != tuple(sh) or not t.is_contiguous() or not t.is_cuda:
-                raise _lib.TttError(_lib.TTT_ERR_SHAPE, "into: a gradient tensor has the wrong shape or layout")
-    else:
-        g_act = [torch.empty_like(xq) for _ in range(3)]
-        g_st = [torch.empty(sh, **f32) for sh in shapes]
-        g_lr = torch.empty_like(lr)
-        g_te = torch.empty(seq, **f32)
-        g_gam, g_bet = torch.empty((H, d), **f32), torch.empty((H, d), **f32)
-    stream = C.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
-    null = C.c_void_p(None)
-    args = [C.byref(desc), _ptr(xq), _ptr(xk), _ptr(xv), _ptr(w1), _ptr(b1), _ptr(w2), _ptr(b2), _ptr(te), _ptr(lr),
-            _ptr(ln_weight), _ptr(ln_bias), _ptr(d_out), *[null if g is None else _ptr(g) for g in up],
-            *[_ptr(g) for g in g_act], *[_ptr(g) for g in g_st], _ptr(g_lr), _ptr(g_te), _ptr(g_gam), _ptr(g_bet)]
-    with torch.cuda.device(dev):
-        if saved is not None:
-            if saved.numel() * saved.element_size() < lib().ttt_mlp_bwd_workspace_bytes(C.byref(desc)):
-                raise _lib.TttError(_lib.TTT_ERR_SHAPE, "saved is smaller than this desc's workspace (a forward with "
-                                                         "another kernel_hint?)")
-            check(lib().ttt_mlp_bwd_saved(*args, _ptr(saved), stream))
-        elif static_scratch:
-            check(lib().ttt_mlp_bwd_static(*args, stream))
-        else:
-            nbytes = lib().ttt_mlp_bwd_workspace_bytes(C.byref(desc))
-            if nbytes < 0:
-                raise _lib.TttError(_lib.TTT_ERR_SHAPE, "ttt_mlp_bwd_workspace_bytes failed")
-            ws = torch.empty((nbytes + 3) // 4, **f32)
-            check(lib().ttt_mlp_bwd(*args, _ptr(ws), stream))
-    return dict(d_xq=g_act[0], d_xk=g_act[1], d_xv=g_act[2], d_W1=g_st[0], d_b1=g_st[1], d_W2=g_st[2],
-                d_b2=g_st[3], d_lr=g_lr, d_token_eta=g_te, d_gamma=g_gam, d_beta=g_bet)
+    return host().mlp_backward(xq, xk, xv, w1, b1, w2, b2, token_eta, ttt_lr_eta, ln_weight, ln_bias, d_out, mini_batch,
+                               eps, d_state_out, static_scratch, into, int(kernel_hint), saved)
+
 
 
 @dataclass
@@ -579,34 +292,24 @@ class FusedTileMulti:
         return TTTLinearState(self.weight_init.unsqueeze(0).repeat(batch_size, 1, 1, 1),
                               self.bias_init.unsqueeze(0).repeat(batch_size, 1, 1))
 
-    def _launch(self, state: TTTLinearState, inputs: TTTInputsInner, mini_batch: int, out=None):
-        t = self.config.ttt
-        out, w, b = ttt_linear_forward_raw(
-            inputs.qkv.xq, inputs.qkv.xk, inputs.qkv.xv, state.weight, state.bias, inputs.token_eta,
-            inputs.ttt_lr_eta, self.ln_weight, self.ln_bias, mini_batch, t.epsilon,
-            t.checkpoint_interval, out=out)
-        state.weight, state.bias = w, b
+    def _pass(self, state: TTTLinearState, inputs: TTTInputsInner, start: int, stop: int):
+        q, t = inputs.qkv, self.config.ttt
+        out, state.weight, state.bias = host().linear_layer_forward(
+            q.xq, q.xk, q.xv, state.weight, state.bias, inputs.token_eta, inputs.ttt_lr_eta, self.ln_weight,
+            self.ln_bias, t.mini_batch_size, t.epsilon, t.checkpoint_interval, start, stop)
         return out
 
     def forward(self, state: TTTLinearState, inputs: TTTInputsInner) -> torch.Tensor:
         """wrapper.rs:102-164: all full mini-batches in one launch; a trailing remainder is one
-        short mini-batch, as the Burn-op model does it (inner.rs:40-47)."""
-        K = self.config.ttt.mini_batch_size
-        seq = inputs.qkv.xq.shape[2]
-        full = (seq // K) * K
-        # one output tensor; both launches read and write sequence windows in place
-        output = torch.empty(inputs.qkv.xq.shape, dtype=inputs.qkv.xq.dtype, device=inputs.qkv.xq.device)
-        if full > 0:
-            self._launch(state, inputs.slice_seq(range(0, full)), K, out=output[:, :, :full])
-        if full < seq:
-            self._launch(state, inputs.slice_seq(range(full, seq)), seq - full, out=output[:, :, full:])
-        return output
+        short mini-batch, as the Burn-op model does it (inner.rs:40-47).  Both launches read and write
+        windows of the sequence in place."""
+        return self._pass(state, inputs, 0, inputs.qkv.xq.shape[2])
 
     def forward_mini_batch(self, state: TTTLinearState, inputs: TTTInputsInner, r: range) -> torch.Tensor:
         """wrapper.rs:166-211: one mini-batch (len(r) <= mini_batch_size)."""
         if len(r) > self.config.ttt.mini_batch_size or len(r) == 0:
             raise _lib.TttError(_lib.TTT_ERR_SHAPE, "range longer than mini_batch_size")
-        return self._launch(state, inputs.slice_seq(r), len(r))
+        return self._pass(state, inputs, r.start, r.stop)
 
 
 @dataclass
@@ -786,75 +489,13 @@ def ttt_stack_forward_raw(layers, token_eta, mini_batch: int, eps: float = 1e-6,
     With check_lost the call waits for the device, reads that word before and after and raises if it moved.
     Default (None): checked unless the current stream is being captured into a graph; callers that must not
     synchronise (timed loops) pass False and compare mlp_fwd_lost_workgroups() around their own region."""
-    B, H, seq, d = layers[0]["pq"].shape
-    io = layers[0]["pq"].dtype
-    dev = layers[0]["pq"].device
-    f32 = dict(dtype=torch.float32, device=dev)
-    desc = TttDesc(B, H, seq, d, mini_batch, eps, 1, _io_dtype(layers[0]["pq"]), 0, 0, 0, kernel_hint)
-    te = _need(token_eta.to(torch.float32), (token_eta.numel(),), torch.float32, "token_eta")
-    if te.numel() < mini_batch:
-        raise _lib.TttError(_lib.TTT_ERR_SHAPE, "token_eta shorter than mini_batch")
-    arr = (_lib.TttStackLayer * len(layers))()
-    keep, states = [], []
-    for i, L in enumerate(layers):
-        mlp = "W2" in L
-        m = 4 * d
-        t = {k: _need(L[k], (B, H, seq, d), io, k) for k in ("pq", "pk", "pv")}
-        t["lr"] = _need(L["lr"], (B, H, seq), io, "lr")
-        t["gamma"] = _need(L["gamma"], (H, d), torch.float32, "gamma")
-        t["beta"] = _need(L["beta"], (H, d), torch.float32, "beta")
-        if mlp:
-            t["W1"] = _need(L["W1"], (H, d, m), torch.float32, "W1")
-            t["b1"] = _need(L["b1"], (H, m), torch.float32, "b1")
-            t["W2"] = _need(L["W2"], (H, m, d), torch.float32, "W2")
-            t["b2"] = _need(L["b2"], (H, d), torch.float32, "b2")
-            st = [torch.empty((B, H, d, m), **f32), torch.empty((B, H, m), **f32), torch.empty((B, H, m, d), **f32),
-                  torch.empty((B, H, d), **f32)]
-        else:
-            t["W1"] = _need(L["W0"], (H, d, d), torch.float32, "W0")
-            t["b1"] = _need(L["b0"], (H, d), torch.float32, "b0")
-            st = [torch.empty((B, H, d, d), **f32), torch.empty((B, H, d), **f32)]
-        keep.append(t)
-        states.append(st)
-        a = arr[i]
-        a.kind = 1 if mlp else 0
-        for k in ("pq", "pk", "pv", "W1", "b1", "lr", "gamma", "beta"):
-            setattr(a, k, t[k].data_ptr())
-        a.W2 = t["W2"].data_ptr() if mlp else None
-        a.b2 = t["b2"].data_ptr() if mlp else None
-        a.W1_out, a.b1_out = st[0].data_ptr(), st[1].data_ptr()
-        a.W2_out = st[2].data_ptr() if mlp else None
-        a.b2_out = st[3].data_ptr() if mlp else None
-    nbytes = lib().ttt_stack_fwd_workspace_bytes(C.byref(desc), len(layers), arr, chunk_tokens)
-    if nbytes < 0:
-        raise _lib.TttError(_lib.TTT_ERR_SHAPE, lib().ttt_last_error().decode())
-    if workspace is None:
-        workspace = torch.empty(nbytes, dtype=torch.uint8, device=dev)
-    elif workspace.numel() * workspace.element_size() < nbytes:
-        raise _lib.TttError(_lib.TTT_ERR_SHAPE, "workspace too small")
-    out = torch.empty((B, H, seq, d), dtype=io, device=dev)
-    stream = C.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
-    two_cu = (d == 128 or (d == 96 and kernel_hint & _lib.TTT_HINT_TWO_CU)) and io == torch.bfloat16 and \
-        any("W2" in L for L in layers) and not (kernel_hint & _lib.TTT_HINT_LDS_TILES)
     if check_lost is None:
-        check_lost = two_cu and not torch.cuda.is_current_stream_capturing()
-    with torch.cuda.device(dev):
-        lost_before = 0
-        if check_lost and two_cu:
-            torch.cuda.synchronize(dev)
-            lost_before = mlp_fwd_lost_workgroups()
-        check(lib().ttt_stack_fwd(C.byref(desc), len(layers), arr, _ptr(te), _ptr(out), _ptr(workspace),
-                                  chunk_tokens, C.c_void_p(aux_stream.cuda_stream) if aux_stream is not None else None,
-                                  stream))
-        if check_lost and two_cu:
-            torch.cuda.synchronize(dev)
-            lost = mlp_fwd_lost_workgroups() - lost_before
-            if lost and not (kernel_hint & _lib.TTT_HINT_TEST_LOST_PARTNER):
-                raise _lib.TttError(_lib.TTT_ERR_HIP, f"ttt_stack_fwd: {lost} workgroups of the two-CU TTT-MLP kernel "
-                                    "waited for their partner in vain; the outputs of their units are NaN")
+        check_lost = not torch.cuda.is_current_stream_capturing()
     # aux_stream reads and writes tensors that torch's allocator ties to the current stream only; the call joins
     # it into the current stream before it returns, so later work on that stream is ordered after it
-    return out, states
+    return host().stack_forward(layers, token_eta, mini_batch, eps, kernel_hint, workspace, chunk_tokens,
+                                0 if aux_stream is None else aux_stream.cuda_stream, int(check_lost))
+
 
 
 # --------------------------------------------------------------------------- either side of the inner loop
@@ -884,35 +525,11 @@ def inner_loop_inputs_raw(xq, xk, xv, lr_logits, lr_bias, base_lr: float, token_
     """One call of ttt_inner_inputs: TTT::get_inner_loop_inputs after the projections
     (rust/layer/src/ttt.rs:147-194, 205-227, 247-268).  xq,xk,xv [B,seq,H,d]; lr_logits [B,seq,H];
     rope = (cos, sin) tables [npos, d/2] f32 or None."""
-    B, seq, H, d = xq.shape
-    io = xq.dtype
-    xq = _need(xq, (B, seq, H, d), io, "xq")
-    xk = _need(xk, (B, seq, H, d), io, "xk")
-    xv = _need(xv, (B, seq, H, d), io, "xv")
-    lg = _need(lr_logits, (B, seq, H), io, "lr_logits")
-    lb = _need(lr_bias.reshape(-1), (H,), torch.float32, "lr_bias")
-    ti = _need(token_idx, (mini_batch,), torch.float32, "token_idx")
-    lti = _need(learnable_token_idx, (mini_batch,), torch.float32, "learnable_token_idx")
-    null = C.c_void_p(None)
-    cos = sin = None
-    if rope is not None:
-        cos = _need(rope[0], (rope[0].shape[0], d // 2), torch.float32, "rope cos")
-        sin = _need(rope[1], (rope[0].shape[0], d // 2), torch.float32, "rope sin")
-        last = (pos_offset + seq - 1) if pos_wrap == 0 else min(pos_wrap - 1, pos_offset + seq - 1)
-        if last >= cos.shape[0]:
-            raise _lib.TttError(_lib.TTT_ERR_SHAPE, "rope table shorter than the positions used")
-    dev = xq.device
-    q, k, v = (torch.empty((B, H, seq, d), dtype=io, device=dev) for _ in range(3))
-    lr = torch.empty((B, H, seq), dtype=io, device=dev)
-    te = torch.empty(seq, dtype=torch.float32, device=dev)
-    desc = TttDesc(B, H, seq, d, mini_batch, 0.0, 1, _io_dtype(xq), 0, 0)
-    stream = C.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
-    with torch.cuda.device(dev):
-        check(lib().ttt_inner_inputs(C.byref(desc), _ptr(xq), _ptr(xk), _ptr(xv), _ptr(lg), _ptr(lb),
-                                     C.c_float(base_lr), _ptr(ti), _ptr(lti),
-                                     null if cos is None else _ptr(cos), null if sin is None else _ptr(sin),
-                                     pos_offset, pos_wrap, _ptr(q), _ptr(k), _ptr(v), _ptr(lr), _ptr(te), stream))
+    cos, sin = (None, None) if rope is None else rope
+    q, k, v, lr, te = host().inner_inputs(xq, xk, xv, lr_logits, lr_bias, token_idx, learnable_token_idx, cos, sin,
+                                          pos_offset, pos_wrap, mini_batch, base_lr)
     return TTTInputsInner(Qkv(q, k, v), te, lr)
+
 
 
 def ttt_linear_forward_fused_inputs_raw(xq, xk, xv, lr_logits, lr_bias, base_lr: float, token_idx,
@@ -925,73 +542,19 @@ def ttt_linear_forward_fused_inputs_raw(xq, xk, xv, lr_logits, lr_bias, base_lr:
     lr_logits [B,seq,H]; rope = (cos, sin) tables [npos, d/2] f32 or None; weight/bias/ln_* as for
     ttt_linear_forward_raw.  Returns (output, weight_out, bias_out[, weight_ckpt, bias_ckpt][, TTTInputsInner]):
     the last item, with save_inputs, holds the operands as the kernel used them (what the backward needs)."""
-    B, seq, H, d = xq.shape
-    io = xq.dtype
-    xq = _need(xq, (B, seq, H, d), io, "xq")
-    xk = _need(xk, (B, seq, H, d), io, "xk")
-    xv = _need(xv, (B, seq, H, d), io, "xv")
-    lg = _need(lr_logits, (B, seq, H), io, "lr_logits")
-    lb = _need(lr_bias.reshape(-1), (H,), torch.float32, "lr_bias")
-    ti = _need(token_idx, (mini_batch,), torch.float32, "token_idx")
-    lti = _need(learnable_token_idx, (mini_batch,), torch.float32, "learnable_token_idx")
-    per_batch = weight.dim() == 4
-    W0 = _need(weight, (B, H, d, d) if per_batch else (H, d, d), torch.float32, "weight")
-    b0 = _need(bias, (B, H, d) if per_batch else (H, d), torch.float32, "bias")
-    gam = _need(ln_weight, (H, d), torch.float32, "ln_weight")
-    bet = _need(ln_bias, (H, d), torch.float32, "ln_bias")
-    null = C.c_void_p(None)
-    cos = sin = None
-    if rope is not None:
-        cos = _need(rope[0], (rope[0].shape[0], d // 2), torch.float32, "rope cos")
-        sin = _need(rope[1], (rope[0].shape[0], d // 2), torch.float32, "rope sin")
-        last = (pos_offset + seq - 1) if pos_wrap == 0 else min(pos_wrap - 1, pos_offset + seq - 1)
-        if last >= cos.shape[0]:
-            raise _lib.TttError(_lib.TTT_ERR_SHAPE, "rope table shorter than the positions used")
-    dev = xq.device
-    desc = TttDesc(B, H, seq, d, mini_batch, eps, checkpoint_interval, _io_dtype(xq), 1 if per_batch else 0, 0,
-                   int(packed_checkpoints), 0)
-    check(lib().ttt_linear_fwd_fused_inputs_supported(C.byref(desc), pos_wrap, 0 if rope is None else 1))
-    out = torch.empty((B, H, seq, d), dtype=io, device=dev)
-    W_out = torch.empty((B, H, d, d), dtype=torch.float32, device=dev)
-    b_out = torch.empty((B, H, d), dtype=torch.float32, device=dev)
-    Wc = bc = None
-    if want_checkpoints:
-        n = int(lib().ttt_linear_num_checkpoints(C.byref(desc)))
-        Wc = torch.empty((B, H, n, d, d), dtype=torch.float32, device=dev)
-        bc = torch.empty((B, H, n, d), dtype=torch.float32, device=dev)
-    q = k = v = lr = te = None
-    if save_inputs:
-        q, k, v = (torch.empty((B, H, seq, d), dtype=io, device=dev) for _ in range(3))
-        lr = torch.empty((B, H, seq), dtype=io, device=dev)
-        te = torch.empty(seq, dtype=torch.float32, device=dev)
-    opt = lambda t: null if t is None else _ptr(t)
-    stream = C.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
-    with torch.cuda.device(dev):
-        check(lib().ttt_linear_fwd_fused_inputs(
-            C.byref(desc), _ptr(xq), _ptr(xk), _ptr(xv), _ptr(lg), _ptr(lb), C.c_float(base_lr), _ptr(ti), _ptr(lti),
-            opt(cos), opt(sin), pos_offset, pos_wrap, _ptr(W0), _ptr(b0), _ptr(gam), _ptr(bet), _ptr(out), _ptr(W_out),
-            _ptr(b_out), opt(Wc), opt(bc), opt(q), opt(k), opt(v), opt(lr), opt(te), stream))
-    res = [out, W_out, b_out]
-    if want_checkpoints:
-        res += [Wc, bc]
-    if save_inputs:
-        res.append(TTTInputsInner(Qkv(q, k, v), te, lr))
-    return tuple(res)
+    cos, sin = (None, None) if rope is None else rope
+    r = host().linear_forward_fused_inputs(xq, xk, xv, lr_logits, lr_bias, token_idx, learnable_token_idx, cos, sin,
+                                           pos_offset, pos_wrap, mini_batch, base_lr, weight, bias, ln_weight, ln_bias,
+                                           eps, checkpoint_interval, want_checkpoints, int(packed_checkpoints),
+                                           save_inputs)
+    if not save_inputs:
+        return r
+    q, k, v, lr, te = r[-5:]
+    return r[:-5] + (TTTInputsInner(Qkv(q, k, v), te, lr),)
+
 
 
 def layer_epilogue_raw(inner_out, post_norm_weight, post_norm_bias, gate=None, eps: float = 1e-6):
     """One call of ttt_layer_epilogue: head merge + post_norm LayerNorm (+ tanh-GELU gate) of
     TTT::forward (rust/layer/src/ttt.rs:285-297).  inner_out [B,H,seq,d] -> [B,seq,H*d]."""
-    B, H, seq, d = inner_out.shape
-    io = inner_out.dtype
-    x = _need(inner_out, (B, H, seq, d), io, "inner_out")
-    g = _need(post_norm_weight, (H * d,), torch.float32, "post_norm_weight")
-    b = _need(post_norm_bias, (H * d,), torch.float32, "post_norm_bias")
-    gt = None if gate is None else _need(gate, (B, seq, H * d), io, "gate")
-    out = torch.empty((B, seq, H * d), dtype=io, device=x.device)
-    desc = TttDesc(B, H, seq, d, 1, eps, 1, _io_dtype(x), 0, 0)
-    stream = C.c_void_p(torch.cuda.current_stream(x.device).cuda_stream)
-    with torch.cuda.device(x.device):
-        check(lib().ttt_layer_epilogue(C.byref(desc), _ptr(x), _ptr(g), _ptr(b), C.c_float(eps),
-                                       C.c_void_p(None) if gt is None else _ptr(gt), _ptr(out), stream))
-    return out
+    return host().layer_epilogue(inner_out, post_norm_weight, post_norm_bias, gate, eps)
