@@ -1,0 +1,45 @@
+"""GPU parity of the backward on sparse checkpoints (one every ci > 1 mini-batches) with a workspace: the states between
+two checkpoints are computed first, all segments at once, and the dense-checkpoint kernels read them."""
+import importlib
+
+import pytest
+import torch
+
+from helpers import TOL, assert_close, to_dev
+from test_linear_bwd_gpu import NAMES, compare, oracle_bwd, run_bwd
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def P():
+    return importlib.import_module("ttt-rs_amd")
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["f32", "bf16"])
+@pytest.mark.parametrize("B,H,d,K,N,ci", [
+    (1, 1, 64, 16, 1, 2),     # a segment cut short to one mini-batch, one segment
+    (2, 2, 64, 16, 5, 4),     # the last segment of one mini-batch
+    (1, 3, 64, 16, 7, 3), (2, 2, 32, 16, 6, 2), (1, 2, 32, 8, 9, 16),
+    (2, 1, 64, 11, 8, 5)])    # short mini-batches: masked rows
+def test_sparse_backward_against_oracle(P, B, H, d, K, N, ci, dtype):
+    print(f"case sparse bwd B{B} H{H} d{d} K{K} N{N} ci{ci} {dtype}", flush=True)
+    c = P.synthetic.reference_test_inputs(300 + N + ci + d, B, H, N * K, d, K, io_dtype=dtype)
+    g = torch.Generator().manual_seed(N)
+    dO = torch.randn(B, H, N * K, d, generator=g).to(dtype)
+    sg = (torch.randn(B, H, d, d, generator=g), torch.randn(B, H, d, generator=g))
+    compare(run_bwd(P, c, dO, K, ci, sg), oracle_bwd(c, dO, K, sg), TOL[dtype])
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["f32", "bf16"])
+@pytest.mark.parametrize("B,H,N,ci", [
+    (34, 16, 33, 4),     # the states of a sequence exceed the workspace's bound: two launches, the first of one segment
+    (6, 16, 24, 5)])     # two workgroups per unit (f32)
+def test_sparse_backward_against_dense_checkpoints(P, B, H, N, ci, dtype):
+    d, K = 64, 16
+    print(f"case sparse vs dense bwd B{B} H{H} N{N} ci{ci} {dtype}", flush=True)
+    c = P.synthetic.baseline_inputs(7, B, H, N * K, d, K, io_dtype=dtype, with_dout=True)
+    dO = c.pop("d_out")
+    g1, g0 = run_bwd(P, c, dO, K, ci), run_bwd(P, c, dO, K, 1)
+    for name, _ in NAMES:
+        assert_close(g1[name], g0[name].double(), TOL[dtype], name, min_frac=0.99)

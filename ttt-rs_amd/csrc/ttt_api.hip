@@ -1079,97 +1079,9 @@ LinBwdPairWs linear_bwd_pair_ws(const ttt_desc* d) {
   return w;
 }
 
-int linear_bwd_impl(const ttt_desc* d, const void* xq, const void* xk, const void* xv,
-                    const float* W0, const float* b0, const float* token_eta, const void* lr,
-                    const float* gamma, const float* beta, const float* W_ckpt,
-                    const float* b_ckpt, const void* d_out, const float* d_W_out,
-                    const float* d_b_out, void* d_xq, void* d_xk, void* d_xv, float* d_W0,
-                    float* d_b0, void* d_lr, float* d_token_eta, float* d_gamma, float* d_beta,
-                    void* workspace, void* stream) {
-  // the kernel is chosen (and a desc without one refused) before anything is enqueued
-  LinearBwdChoice ch;
-  int rc = choose_linear_bwd(d, &ch);
-  if (rc != TTT_OK) return rc;
-  bool pair = workspace != nullptr && linear_bwd_pair_wanted(d);
-  if (pair) {
-    if (!aligned16(workspace)) return fail(TTT_ERR_SHAPE, "ttt_linear_bwd_ws: workspace must be 16-byte aligned");
-    int cus = 0;
-    rc = device_cus(&cus);
-    if (rc != TTT_OK) return rc;
-    pair = 2 * (int64_t)d->batch * d->heads <= cus;  // every workgroup a CU of its own, both sides resident together
-  }
-  // W0/b0 are part of the saved state for interface parity; the state entering every stage is
-  // rebuilt from the checkpoints (checkpoint 0 equals the initial state).
-  (void)W0;
-  (void)b0;
-  if (!xq || !xk || !xv || !token_eta || !lr || !gamma || !beta || !d_out || !d_xq || !d_xk ||
-      !d_xv || !d_W0 || !d_b0 || !d_lr || !d_token_eta || !d_gamma || !d_beta)
-    return fail(TTT_ERR_NULL, "ttt_linear_bwd: a required pointer is NULL");
-  if (!W_ckpt || !b_ckpt)
-    return fail(TTT_ERR_NULL, "ttt_linear_bwd needs the W/b checkpoints written by ttt_linear_fwd");
-  ttt::LinearBwdArgs a;
-  a.xq = xq; a.xk = xk; a.xv = xv; a.token_eta = token_eta; a.lr = lr; a.gamma = gamma; a.beta = beta;
-  a.W_ckpt = W_ckpt; a.b_ckpt = b_ckpt; a.d_out = d_out; a.d_W_out = d_W_out; a.d_b_out = d_b_out;
-  a.d_xq = d_xq; a.d_xk = d_xk; a.d_xv = d_xv; a.d_W0 = d_W0; a.d_b0 = d_b0; a.d_lr = d_lr;
-  a.d_token_eta = d_token_eta; a.d_gamma = d_gamma; a.d_beta = d_beta;
-  a.B = d->batch; a.H = d->heads; a.seq = d->seq; a.K = d->mini_batch;
-  a.seq_stride = d->seq_stride > 0 ? d->seq_stride : d->seq;
-  a.n_stages = d->seq / d->mini_batch;
-  a.ckpt_interval = d->checkpoint_interval;
-  a.n_ckpt = (int)ttt_linear_num_checkpoints(d);
-  a.ckpt_packed = ckpt_format_of(d) == TTT_CKPT_PACKED ? 1 : ckpt_format_of(d) == TTT_CKPT_FACTORS ? ttt::kCkptFactors : 0;
-  a.eps = d->eps;
-  const int D = d->head_dim;
-  if (ch.kind != LinearBwdChoice::LDS &&
-      (!aligned16(xq) || !aligned16(xk) || !aligned16(xv) || !aligned16(d_out) || !aligned16(d_xq) ||
-       !aligned16(d_xk) || !aligned16(d_xv) || !aligned16(W_ckpt) || !aligned16(b_ckpt) ||
-       ((size_t)a.seq_stride * D) % 8 != 0))
-    return fail(TTT_ERR_SHAPE, "ttt_linear_bwd: tensors must be 16-byte aligned");
-  if ((ch.w_global || ch.dw_global) && (!aligned16(W_ckpt) || !aligned16(d_W0)))
-    return fail(TTT_ERR_SHAPE, "ttt_linear_bwd: W_ckpt and d_W0 must be 16-byte aligned");
-  hipStream_t s = static_cast<hipStream_t>(stream);
-  // accumulated outputs start from zero; a fill kernel (not a memset node) so the sequence
-  // can be captured into a graph
-  const size_t hd = (size_t)d->heads * d->head_dim;
-  {
-    const size_t nmax = (size_t)d->seq > hd ? (size_t)d->seq : hd;
-    hipLaunchKernelGGL(ttt::ttt_fill_zero3_kernel, dim3((unsigned)((nmax + 255) / 256)), dim3(256), 0, s, d_token_eta,
-                       (size_t)d->seq, d_gamma, hd, d_beta, hd);
-  }
+// the register-resident kernels on one workgroup per unit (one checkpoint per mini-batch)
+int launch_linear_bwd_reg(const ttt::LinearBwdArgs& a, int D, bool f32, int waves, hipStream_t s) {
   const unsigned grid = (unsigned)(a.B * a.H);
-  const bool f32 = d->io_dtype == TTT_F32;
-  const int waves = ch.waves;
-  if (pair) {
-    const LinBwdPairWs w = linear_bwd_pair_ws(d);
-    ttt::LinearBwdPairArgs pa;
-    pa.a = a;
-    pa.hand = static_cast<unsigned char*>(workspace) + w.hand;
-    pa.flags = reinterpret_cast<unsigned*>(static_cast<unsigned char*>(workspace) + w.flags);
-    pa.spin_limit = (d->kernel_hint & TTT_HINT_TEST_LOST_PARTNER) ? 0u : (1u << 21);
-    pa.agent_release = (d->kernel_hint & TTT_HINT_TEST_OTHER_XCD) ? 1 : 0;
-    copy_or_zero(reinterpret_cast<float*>(pa.flags), nullptr, (size_t)grid * ttt::kLinBwdPairFlagWords, s);
-    if (a.ckpt_packed)
-      return D == 64 ? launch_linear_bwd_pair<64, true>(pa, s) : launch_linear_bwd_pair<32, true>(pa, s);
-    return D == 64 ? launch_linear_bwd_pair<64, false>(pa, s) : launch_linear_bwd_pair<32, false>(pa, s);
-  }
-  if (ch.kind == LinearBwdChoice::LDS) {
-    if (ch.w_global) return launch_linear_bwd<ttt::F32, 128, 1, true, true>(a, grid, s);
-    // bf16 I/O: operands rounded to bf16 like the register-resident kernels, unless f32 products were asked for
-    const bool bfops = !f32 && !(d->kernel_hint & TTT_HINT_LDS_TILES);
-    if (ch.dw_global)
-      return f32     ? launch_linear_bwd<ttt::F32, 96, 1, false, true>(a, grid, s)
-             : bfops ? launch_linear_bwd<ttt::BF16, 96, 1, false, true, true>(a, grid, s)
-                     : launch_linear_bwd<ttt::BF16, 96, 1, false, true>(a, grid, s);
-    if (d->mini_batch > 16)
-      return f32     ? launch_linear_bwd<ttt::F32, 32, 2>(a, grid, s)
-             : bfops ? launch_linear_bwd<ttt::BF16, 32, 2, false, false, true>(a, grid, s)
-                     : launch_linear_bwd<ttt::BF16, 32, 2>(a, grid, s);
-    if (f32) return D == 64 ? launch_linear_bwd<ttt::F32, 64>(a, grid, s) : launch_linear_bwd<ttt::F32, 32>(a, grid, s);
-    if (bfops)
-      return D == 64 ? launch_linear_bwd<ttt::BF16, 64, 1, false, false, true>(a, grid, s)
-                     : launch_linear_bwd<ttt::BF16, 32, 1, false, false, true>(a, grid, s);
-    return D == 64 ? launch_linear_bwd<ttt::BF16, 64>(a, grid, s) : launch_linear_bwd<ttt::BF16, 32>(a, grid, s);
-  }
   if (a.ckpt_packed == ttt::kCkptFactors) {
     if (D == 32) return launch_linear_bwd_mw<ttt::BF16, 32, 2, true, true>(a, grid, s);
     if (D == 64)
@@ -1206,6 +1118,192 @@ int linear_bwd_impl(const ttt_desc* d, const void* xq, const void* xk, const voi
   if (D == 96) return launch_linear_bwd_mw<ttt::BF16, 96, 3>(a, grid, s);
   return launch_linear_bwd_mw<ttt::BF16, 128, 4>(a, grid, s);
 }
+// ... on two workgroups per unit
+int launch_linear_bwd_pairs(const ttt::LinearBwdArgs& a, const ttt_desc* d, const LinBwdPairWs& w, void* workspace,
+                            hipStream_t s) {
+  ttt::LinearBwdPairArgs pa;
+  pa.a = a;
+  pa.hand = static_cast<unsigned char*>(workspace) + w.hand;
+  pa.flags = reinterpret_cast<unsigned*>(static_cast<unsigned char*>(workspace) + w.flags);
+  pa.spin_limit = (d->kernel_hint & TTT_HINT_TEST_LOST_PARTNER) ? 0u : (1u << 21);
+  pa.agent_release = (d->kernel_hint & TTT_HINT_TEST_OTHER_XCD) ? 1 : 0;
+  copy_or_zero(reinterpret_cast<float*>(pa.flags), nullptr, (size_t)a.B * a.H * ttt::kLinBwdPairFlagWords, s);
+  if (a.ckpt_packed)
+    return d->head_dim == 64 ? launch_linear_bwd_pair<64, true>(pa, s) : launch_linear_bwd_pair<32, true>(pa, s);
+  return d->head_dim == 64 ? launch_linear_bwd_pair<64, false>(pa, s) : launch_linear_bwd_pair<32, false>(pa, s);
+}
+
+// ---- Sparse checkpoints (one every ci > 1 mini-batches), with a workspace.
+// The LDS-tile kernel re-simulates the state from the last checkpoint for every mini-batch of the reverse scan, on the
+// CU that carries the scan: ci / 2 extra forward mini-batches in front of each.  With a workspace the states are
+// computed first, all segments at once (ttt_linear_states_kernel), and the dense-checkpoint kernels read them: at the
+// 125M shape (f32, 96 units, 2048 tokens, ci = 16) 3.21 -> 0.56 ms.
+// The workspace is bounded: a launch takes as many whole segments as kLinStatesMaxBytes holds states for (at least one),
+// from the end of the sequence to its beginning; the state gradient of a launch is the upstream gradient of the next.
+constexpr size_t kLinStatesMaxBytes = (size_t)256 << 20;
+struct LinStatesPlan {
+  ttt_desc dense;     // the desc of the backward that reads the states
+  bool pair;          // ... on two workgroups per unit
+  LinBwdPairWs pw;
+  int segments;       // per unit and launch, but for the last of a sequence
+  size_t W, b, total; // byte offsets in the workspace
+};
+bool plan_linear_states(const ttt_desc* d, LinStatesPlan* p) {
+  if (d->checkpoint_interval == 1 || d->mini_batch > 16 || d->head_dim > 64 || d->checkpoint_format != TTT_CKPT_F32 ||
+      (d->kernel_hint & TTT_HINT_LDS_TILES) != 0)
+    return false;
+  p->dense = *d;
+  p->dense.checkpoint_interval = 1;
+  p->dense.checkpoint_format = TTT_CKPT_PACKED;
+  p->pair = linear_bwd_pair_wanted(&p->dense);
+  p->pw = p->pair ? linear_bwd_pair_ws(&p->dense) : LinBwdPairWs{0, 0, 0};
+  const size_t U = (size_t)d->batch * d->heads, D = d->head_dim, N = d->seq / d->mini_batch, ci = d->checkpoint_interval;
+  const size_t C = (N + ci - 1) / ci, per_segment = U * ci * D * (D + 1) * sizeof(float);
+  size_t seg = kLinStatesMaxBytes / per_segment;
+  seg = seg < 1 ? 1 : seg > C ? C : seg;
+  p->segments = (int)seg;
+  const size_t stages = seg * ci < N ? seg * ci : N;
+  p->W = (p->pw.total + 255) / 256 * 256;
+  p->b = p->W + U * stages * D * D * sizeof(float);
+  p->total = p->b + U * stages * D * sizeof(float);
+  return true;
+}
+template <class T, int D, int NW>
+int launch_linear_states(const ttt::LinearFwdArgs& a, const ttt::LinearSegments& sg, hipStream_t s) {
+  const dim3 grid((unsigned)(a.B * a.H) * (unsigned)sg.n_seg), block(64 * NW);
+  if (a.K == 16)
+    hipLaunchKernelGGL((ttt::ttt_linear_states_kernel<T, D, NW, true>), grid, block, 0, s, a, sg);
+  else
+    hipLaunchKernelGGL((ttt::ttt_linear_states_kernel<T, D, NW, false>), grid, block, 0, s, a, sg);
+  return hip_status(hipGetLastError(), "ttt_linear_bwd_ws (states between checkpoints) launch");
+}
+int linear_bwd_sparse(const ttt_desc* d, const LinStatesPlan& p, bool pair, const ttt::LinearBwdArgs& base, void* workspace,
+                      hipStream_t s) {
+  LinearBwdChoice ch;
+  int rc = choose_linear_bwd(&p.dense, &ch);
+  if (rc != TTT_OK) return rc;
+  const bool f32 = d->io_dtype == TTT_F32;
+  const int D = d->head_dim, N = base.n_stages, ci = d->checkpoint_interval, C = base.n_ckpt;
+  const size_t es = f32 ? 4 : 2;
+  unsigned char* ws = static_cast<unsigned char*>(workspace);
+  float *Ws = reinterpret_cast<float*>(ws + p.W), *bs = reinterpret_cast<float*>(ws + p.b);
+  for (int c0 = (C - 1) / p.segments * p.segments; c0 >= 0; c0 -= p.segments) {
+    const int first = c0 * ci, stages = (N - first < p.segments * ci) ? N - first : p.segments * ci;
+    const size_t tok = (size_t)first * d->mini_batch;
+    auto in = [&](const void* q, size_t per_token) { return static_cast<const void*>(static_cast<const char*>(q) + tok * per_token); };
+    auto out = [&](void* q, size_t per_token) { return static_cast<void*>(static_cast<char*>(q) + tok * per_token); };
+    ttt::LinearFwdArgs f{};
+    f.xq = in(base.xq, D * es); f.xk = in(base.xk, D * es); f.xv = in(base.xv, D * es); f.lr = in(base.lr, es);
+    f.token_eta = base.token_eta; f.gamma = base.gamma; f.beta = base.beta;
+    f.W_ckpt = Ws; f.b_ckpt = bs;
+    f.B = base.B; f.H = base.H; f.seq = stages * d->mini_batch; f.K = base.K; f.seq_stride = base.seq_stride;
+    f.n_stages = f.n_ckpt = stages; f.ckpt_interval = 1; f.state_per_batch = 1; f.ckpt_packed = 1; f.eps = base.eps;
+    ttt::LinearSegments sg{base.W_ckpt, base.b_ckpt, C, c0, (stages + ci - 1) / ci, ci};
+    if (D == 64) rc = f32 ? launch_linear_states<ttt::F32, 64, 4>(f, sg, s) : launch_linear_states<ttt::BF16, 64, 2>(f, sg, s);
+    else rc = f32 ? launch_linear_states<ttt::F32, 32, 2>(f, sg, s) : launch_linear_states<ttt::BF16, 32, 2>(f, sg, s);
+    if (rc != TTT_OK) return rc;
+    ttt::LinearBwdArgs a = base;
+    a.xq = f.xq; a.xk = f.xk; a.xv = f.xv; a.lr = f.lr; a.d_out = in(base.d_out, D * es);
+    a.d_xq = out(base.d_xq, D * es); a.d_xk = out(base.d_xk, D * es); a.d_xv = out(base.d_xv, D * es);
+    a.d_lr = out(base.d_lr, es); a.d_token_eta = base.d_token_eta + tok;
+    a.W_ckpt = Ws; a.b_ckpt = bs; a.ckpt_packed = 1; a.ckpt_interval = 1;
+    a.seq = f.seq; a.n_stages = a.n_ckpt = stages;
+    if (first + stages < N) {
+      a.d_W_out = base.d_W0;
+      a.d_b_out = base.d_b0;
+    }
+    rc = pair && stages > 1 ? launch_linear_bwd_pairs(a, &p.dense, p.pw, workspace, s)
+                            : launch_linear_bwd_reg(a, D, f32, ch.waves, s);
+    if (rc != TTT_OK) return rc;
+  }
+  return TTT_OK;
+}
+
+int linear_bwd_impl(const ttt_desc* d, const void* xq, const void* xk, const void* xv,
+                    const float* W0, const float* b0, const float* token_eta, const void* lr,
+                    const float* gamma, const float* beta, const float* W_ckpt,
+                    const float* b_ckpt, const void* d_out, const float* d_W_out,
+                    const float* d_b_out, void* d_xq, void* d_xk, void* d_xv, float* d_W0,
+                    float* d_b0, void* d_lr, float* d_token_eta, float* d_gamma, float* d_beta,
+                    void* workspace, void* stream) {
+  // the kernel is chosen (and a desc without one refused) before anything is enqueued
+  LinearBwdChoice ch;
+  int rc = choose_linear_bwd(d, &ch);
+  if (rc != TTT_OK) return rc;
+  LinStatesPlan sparse;
+  const bool states = workspace != nullptr && plan_linear_states(d, &sparse);
+  bool pair = workspace != nullptr && (states ? sparse.pair : linear_bwd_pair_wanted(d));
+  if (workspace != nullptr && !aligned16(workspace))
+    return fail(TTT_ERR_SHAPE, "ttt_linear_bwd_ws: workspace must be 16-byte aligned");
+  if (pair) {
+    int cus = 0;
+    rc = device_cus(&cus);
+    if (rc != TTT_OK) return rc;
+    pair = 2 * (int64_t)d->batch * d->heads <= cus;  // every workgroup a CU of its own, both sides resident together
+  }
+  // W0/b0 are part of the saved state for interface parity; the state entering every stage is
+  // rebuilt from the checkpoints (checkpoint 0 equals the initial state).
+  (void)W0;
+  (void)b0;
+  if (!xq || !xk || !xv || !token_eta || !lr || !gamma || !beta || !d_out || !d_xq || !d_xk ||
+      !d_xv || !d_W0 || !d_b0 || !d_lr || !d_token_eta || !d_gamma || !d_beta)
+    return fail(TTT_ERR_NULL, "ttt_linear_bwd: a required pointer is NULL");
+  if (!W_ckpt || !b_ckpt)
+    return fail(TTT_ERR_NULL, "ttt_linear_bwd needs the W/b checkpoints written by ttt_linear_fwd");
+  ttt::LinearBwdArgs a;
+  a.xq = xq; a.xk = xk; a.xv = xv; a.token_eta = token_eta; a.lr = lr; a.gamma = gamma; a.beta = beta;
+  a.W_ckpt = W_ckpt; a.b_ckpt = b_ckpt; a.d_out = d_out; a.d_W_out = d_W_out; a.d_b_out = d_b_out;
+  a.d_xq = d_xq; a.d_xk = d_xk; a.d_xv = d_xv; a.d_W0 = d_W0; a.d_b0 = d_b0; a.d_lr = d_lr;
+  a.d_token_eta = d_token_eta; a.d_gamma = d_gamma; a.d_beta = d_beta;
+  a.B = d->batch; a.H = d->heads; a.seq = d->seq; a.K = d->mini_batch;
+  a.seq_stride = d->seq_stride > 0 ? d->seq_stride : d->seq;
+  a.n_stages = d->seq / d->mini_batch;
+  a.ckpt_interval = d->checkpoint_interval;
+  a.n_ckpt = (int)ttt_linear_num_checkpoints(d);
+  a.ckpt_packed = ckpt_format_of(d) == TTT_CKPT_PACKED ? 1 : ckpt_format_of(d) == TTT_CKPT_FACTORS ? ttt::kCkptFactors : 0;
+  a.eps = d->eps;
+  const int D = d->head_dim;
+  if ((states || ch.kind != LinearBwdChoice::LDS) &&
+      (!aligned16(xq) || !aligned16(xk) || !aligned16(xv) || !aligned16(d_out) || !aligned16(d_xq) ||
+       !aligned16(d_xk) || !aligned16(d_xv) || !aligned16(W_ckpt) || !aligned16(b_ckpt) ||
+       ((size_t)a.seq_stride * D) % 8 != 0))
+    return fail(TTT_ERR_SHAPE, "ttt_linear_bwd: tensors must be 16-byte aligned");
+  if ((ch.w_global || ch.dw_global) && (!aligned16(W_ckpt) || !aligned16(d_W0)))
+    return fail(TTT_ERR_SHAPE, "ttt_linear_bwd: W_ckpt and d_W0 must be 16-byte aligned");
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  // accumulated outputs start from zero; a fill kernel (not a memset node) so the sequence
+  // can be captured into a graph
+  const size_t hd = (size_t)d->heads * d->head_dim;
+  {
+    const size_t nmax = (size_t)d->seq > hd ? (size_t)d->seq : hd;
+    hipLaunchKernelGGL(ttt::ttt_fill_zero3_kernel, dim3((unsigned)((nmax + 255) / 256)), dim3(256), 0, s, d_token_eta,
+                       (size_t)d->seq, d_gamma, hd, d_beta, hd);
+  }
+  const unsigned grid = (unsigned)(a.B * a.H);
+  const bool f32 = d->io_dtype == TTT_F32;
+  const int waves = ch.waves;
+  if (states) return linear_bwd_sparse(d, sparse, pair, a, workspace, s);
+  if (pair) return launch_linear_bwd_pairs(a, d, linear_bwd_pair_ws(d), workspace, s);
+  if (ch.kind == LinearBwdChoice::LDS) {
+    if (ch.w_global) return launch_linear_bwd<ttt::F32, 128, 1, true, true>(a, grid, s);
+    // bf16 I/O: operands rounded to bf16 like the register-resident kernels, unless f32 products were asked for
+    const bool bfops = !f32 && !(d->kernel_hint & TTT_HINT_LDS_TILES);
+    if (ch.dw_global)
+      return f32     ? launch_linear_bwd<ttt::F32, 96, 1, false, true>(a, grid, s)
+             : bfops ? launch_linear_bwd<ttt::BF16, 96, 1, false, true, true>(a, grid, s)
+                     : launch_linear_bwd<ttt::BF16, 96, 1, false, true>(a, grid, s);
+    if (d->mini_batch > 16)
+      return f32     ? launch_linear_bwd<ttt::F32, 32, 2>(a, grid, s)
+             : bfops ? launch_linear_bwd<ttt::BF16, 32, 2, false, false, true>(a, grid, s)
+                     : launch_linear_bwd<ttt::BF16, 32, 2>(a, grid, s);
+    if (f32) return D == 64 ? launch_linear_bwd<ttt::F32, 64>(a, grid, s) : launch_linear_bwd<ttt::F32, 32>(a, grid, s);
+    if (bfops)
+      return D == 64 ? launch_linear_bwd<ttt::BF16, 64, 1, false, false, true>(a, grid, s)
+                     : launch_linear_bwd<ttt::BF16, 32, 1, false, false, true>(a, grid, s);
+    return D == 64 ? launch_linear_bwd<ttt::BF16, 64>(a, grid, s) : launch_linear_bwd<ttt::BF16, 32>(a, grid, s);
+  }
+  return launch_linear_bwd_reg(a, D, f32, waves, s);
+}
 }  // namespace
 
 extern "C" {
@@ -1225,6 +1323,8 @@ int64_t ttt_linear_bwd_workspace_bytes(const ttt_desc* d) {
   LinearBwdChoice ch;
   const int rc = choose_linear_bwd(d, &ch);
   if (rc != TTT_OK) return rc;
+  LinStatesPlan sparse;
+  if (plan_linear_states(d, &sparse)) return (int64_t)sparse.total;
   return linear_bwd_pair_wanted(d) ? (int64_t)linear_bwd_pair_ws(d).total : 0;
 }
 

@@ -49,10 +49,14 @@ namespace ttt {
 // zero accumulator, the moments live in registers beside the state (three times the state's registers), bias
 // corrections come from running powers of beta1, beta2.  Everything else -- products, LayerNorm, output -- is the
 // plain kernel's; the output of a mini-batch does not see its own update in either.
-template <class T, int D, int NW, int PF, bool FULL, bool FAC, int RAW, bool ADAM = false>
+// STATES: only the recurrence runs, from a given state, and the state entering every one of n_stages + 1 mini-batches is
+// written as a checkpoint: no output, no attention block, no final state (see ttt_linear_states_kernel).  The unit and the
+// index of its initial state are then given (unit, state) instead of following from the workgroup's index.
+template <class T, int D, int NW, int PF, bool FULL, bool FAC, int RAW, bool ADAM = false, bool STATES = false>
 __device__ __forceinline__ void linear_fwd_sk_body(const LinearFwdArgs& a, const FusedInputsArgs* fip,
-                                                   const AdamArgs* adam = nullptr) {
+                                                   const AdamArgs* adam = nullptr, size_t unit = 0, size_t state = 0) {
   static_assert(!ADAM || (D <= 64 && !FAC && RAW == 0), "Adam inner optimiser: head_dim <= 64, no checkpoints");
+  static_assert(!STATES || (D <= 64 && !FAC && RAW == 0 && !ADAM), "states alone: head_dim <= 64, operands given");
   using IO = Io<T>;
   using frag = typename IO::frag;
   using elem = typename IO::elem;
@@ -75,9 +79,9 @@ __device__ __forceinline__ void linear_fwd_sk_body(const LinearFwdArgs& a, const
   // wave 0 does (w == 0: valid loads, LDS writes of the same values) and it stores nothing
   const bool ctlw = DMA && __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) == NW;
   const int c = lane & 15, g = lane >> 4;
-  const size_t bh = blockIdx.x;
+  const size_t bh = STATES ? unit : blockIdx.x;
   const int h = (int)(bh % a.H);
-  const int K = a.K, n_stages_ = a.n_stages;
+  const int K = a.K, n_stages_ = a.n_stages + (STATES ? 1 : 0);
   const UnitBase<T, D> ub(a, bh);
 
   // same scale folding as the unskewed kernel: G'' = -sc lr G, M'' = (token_eta[t]/sc)(1 + A)
@@ -93,7 +97,7 @@ __device__ __forceinline__ void linear_fwd_sk_body(const LinearFwdArgs& a, const
   const frag ident = identity_frag<T>(c, g);
   const frag nident = identity_frag<T>(c, g, -1.f);
   const frag ones = splat_frag<T>(1.f);
-  const size_t sb = a.state_per_batch ? bh : (size_t)h;
+  const size_t sb = STATES ? state : a.state_per_batch ? bh : (size_t)h;
   f32x4 gam[TPW], bet[TPW], bT[TPW], a2[TPW];
   float sum_a = 0.f;
 #pragma unroll
@@ -563,11 +567,11 @@ __device__ __forceinline__ void linear_fwd_sk_body(const LinearFwdArgs& a, const
         for (int jj = 0; jj < TPW; ++jj) {
           const frag w0 = IO::to_frag(Wc[2 * q][jj]), w1 = IO::to_frag(Wc[2 * q + 1][jj]);
           IO::mma2(z1[jj], w0, w1, cur.k[2 * q], cur.k[2 * q + 1]);
-          IO::mma2(zb[jj], w0, w1, cur.q[2 * q], cur.q[2 * q + 1]);
+          if constexpr (!STATES) IO::mma2(zb[jj], w0, w1, cur.q[2 * q], cur.q[2 * q + 1]);
         }
-        if constexpr (!SHARE) IO::mma2(At, cur.k[2 * q], cur.k[2 * q + 1], cur.q[2 * q], cur.q[2 * q + 1]);
+        if constexpr (!SHARE && !STATES) IO::mma2(At, cur.k[2 * q], cur.k[2 * q + 1], cur.q[2 * q], cur.q[2 * q + 1]);
       }
-      if constexpr (SHARE) {
+      if constexpr (SHARE && !STATES) {
         IO::mma(At, cur.ko[0], cur.qo[0]);  // over the own 16 features
         atx[st & 1][w][lane] = At;
       }
@@ -610,7 +614,9 @@ __device__ __forceinline__ void linear_fwd_sk_body(const LinearFwdArgs& a, const
       exchange8_publish(S, st & 1);
       // ---- the output pending since two mini-batches (sums known since the last exchange): nothing waits
       // for it, and here it runs while this exchange is in flight (LDS write, barrier, LDS read)
-      if (!CHECKED || st > 1) emit_output(so0, so1, st - 2, zbo, qoo);
+      if constexpr (!STATES) {
+        if (!CHECKED || st > 1) emit_output(so0, so1, st - 2, zbo, qoo);
+      }
       exchange8_collect(S, st & 1);
       // RAW: the rows of the next mini-batch, rotated by their owners before this barrier
       if constexpr (DMA) gather_dma(buf[(u + 1) % R], st + 1);
@@ -625,9 +631,11 @@ __device__ __forceinline__ void linear_fwd_sk_body(const LinearFwdArgs& a, const
       if constexpr (SHARE) {
 #pragma unroll
         for (int I = 0; I < NT; ++I) kd[I] = IO::to_frag(kdx[st & 1][I][lane]);
-        At = atx[st & 1][0][lane];
+        if constexpr (!STATES) {
+          At = atx[st & 1][0][lane];
 #pragma unroll
-        for (int ww = 1; ww < NW; ++ww) At += atx[st & 1][ww][lane];
+          for (int ww = 1; ww < NW; ++ww) At += atx[st & 1][ww][lane];
+        }
       }
 
       // ---- recurrence: G'' , causal correction, state update
@@ -654,7 +662,7 @@ __device__ __forceinline__ void linear_fwd_sk_body(const LinearFwdArgs& a, const
         store_factor<TPW>(fac, Gd, w, lane);
         fac += 32 * D;
       }
-      {
+      if constexpr (!STATES) {
         f32x4 m;
 #pragma unroll
         for (int r = 0; r < 4; ++r) m[r] = (4 * g + r <= c) ? rho_c * (1.f + At[r]) : 0.f;
@@ -690,12 +698,14 @@ __device__ __forceinline__ void linear_fwd_sk_body(const LinearFwdArgs& a, const
       }
       // this mini-batch's Zbar and xq become the pending output; its in-lane sums are formed here, in the
       // shadow of the state update, not between the next Z1 and its exchange
+      if constexpr (!STATES) {
 #pragma unroll
-      for (int jj = 0; jj < TPW; ++jj) {
-        zbp[jj] = zb[jj];
-        qop[jj] = cur.qo[jj];
+        for (int jj = 0; jj < TPW; ++jj) {
+          zbp[jj] = zb[jj];
+          qop[jj] = cur.qo[jj];
+        }
+        pend_sums(zbp, ps0, ps1);
       }
-      pend_sums(zbp, ps0, ps1);
       // RAW: the own features of the mini-batch after the next, loaded during the previous pass of the loop; read
       // back by every wave behind the next barrier.  LDS buffer st & 1 was last read behind the barrier of the
       // previous mini-batch, which every wave has left.
@@ -846,6 +856,11 @@ __device__ __forceinline__ void linear_fwd_sk_body(const LinearFwdArgs& a, const
 
   }
 
+  if constexpr (STATES) {  // the state entering the last mini-batch
+    store_ckpt_packed<T, NT, TPW>(ck.W, Wc, w, lane);
+    store_bias_true<D, TPW>(ck.b, bT, b_mean, w, c, g);
+    return;
+  }
   // ---- flush the last mini-batch's output
   {
     float S[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
@@ -903,6 +918,38 @@ template <class T, int D, int NW, int PF, bool FULL, bool FAC, int RAW>
 __global__ void __launch_bounds__(64 * NW) ttt_linear_fwd_fi_kernel(LinearFwdArgs a, FusedInputsArgs fi) {
   static_assert(RAW == 1 || RAW == 2, "RAW selects how positions are looked up");
   linear_fwd_sk_body<T, D, NW, PF, FULL, FAC, RAW>(a, &fi);
+}
+
+// The states between two sparse checkpoints, for a backward that was given a checkpoint every ci mini-batches only: a
+// workgroup takes one segment (the mini-batches from one checkpoint to the next) and writes the state entering each of
+// them as a packed checkpoint, which the dense-checkpoint backward kernels then read.  Segments are independent, so the
+// launch has units x segments workgroups where the reverse scan has one or two per unit: at 96 units and 8 segments of 16
+// mini-batches (d = 64, f32) the 12 288 states take 90 us, bound by the chain of 15 dependent mini-batches and by writing
+// 200 MB.  Same arithmetic as the forward that wrote the checkpoints.
+struct LinearSegments {
+  const float* W_in;  // [units, n_in, d, d]: the sparse checkpoints
+  const float* b_in;  // [units, n_in, d]
+  int n_in, first;    // checkpoints per unit; the first segment of this launch
+  int n_seg, every;   // segments per unit in this launch; mini-batches of a segment
+};
+// a: rows, lr, ... at the first token of the launch; W_ckpt, b_ckpt [units, n_ckpt, ..] for its n_ckpt mini-batches
+template <class T, int D, int NW, bool FULL>
+__global__ void __launch_bounds__(64 * NW, 2) ttt_linear_states_kernel(LinearFwdArgs a, LinearSegments sg) {
+  using elem = typename Io<T>::elem;
+  const size_t unit = blockIdx.x / (unsigned)sg.n_seg, seg = blockIdx.x % (unsigned)sg.n_seg;
+  const size_t at = seg * (size_t)sg.every, tok = at * (size_t)a.K;
+  LinearFwdArgs b = a;
+  b.xq = static_cast<const elem*>(a.xq) + tok * D;
+  b.xk = static_cast<const elem*>(a.xk) + tok * D;
+  b.xv = static_cast<const elem*>(a.xv) + tok * D;
+  b.lr = static_cast<const elem*>(a.lr) + tok;
+  b.W0 = sg.W_in;
+  b.b0 = sg.b_in;
+  b.W_ckpt = a.W_ckpt + at * (D * D);
+  b.b_ckpt = a.b_ckpt + at * D;
+  b.n_stages = min(sg.every, a.n_ckpt - (int)at) - 1;
+  linear_fwd_sk_body<T, D, NW, 2, FULL, false, 0, false, true>(b, nullptr, nullptr, unit,
+                                                               unit * (size_t)sg.n_in + sg.first + seg);
 }
 
 }  // namespace ttt
