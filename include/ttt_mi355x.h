@@ -111,7 +111,7 @@ typedef struct ttt_desc {
 #define TTT_HINT_ALL_LOADS 0x2000
 /* ttt_mlp_bwd / ttt_mlp_bwd_static, bf16 I/O up to head_dim 96: the reverse scan normally rounds the operands of its
  * products to bf16, as the forward of the step did (f32 accumulation, f32 state and gradient accumulators);
- * TTT_HINT_F32_PRODUCTS keeps every product of the scan in f32 (about twice the time).  Ignored elsewhere: f32 I/O and
+ * TTT_HINT_F32_PRODUCTS keeps every product of the scan in f32 (about four times the time).  Ignored elsewhere: f32 I/O and
  * head_dim 128 always compute in f32. */
 #define TTT_HINT_F32_PRODUCTS 0x4000
 /* ttt_mlp_bwd and its variants: with at most 128 (batch, head) units every unit is worked on by two workgroups on two

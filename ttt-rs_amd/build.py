@@ -12,10 +12,11 @@ import sys
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_DIR = os.path.join(HERE, "lib")
 LIB_PATH = os.path.join(LIB_DIR, "libttt_mi355x.so")
-SOURCES = [os.path.join(HERE, "csrc", "ttt_api.hip")]
+# translation units, compiled side by side
+SOURCES = [os.path.join(HERE, "csrc", f) for f in ("ttt_api.hip", "ttt_mlp_bwd_rp.hip")]
 
 HIPCC_FLAGS = [
-    "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-shared",
+    "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC",
     # keep the compiler from forming packed-f32 VALU ops
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     # let MFMA results live in ordinary VGPRs: the kernels consume them with VALU code right away,
@@ -34,11 +35,18 @@ def build_library(verbose: bool = False, extra_flags=()) -> str:
     shutil.rmtree(tmp, ignore_errors=True)
     os.makedirs(tmp)
     out = os.path.join(tmp, os.path.basename(LIB_PATH))
-    cmd = [hipcc, *HIPCC_FLAGS, *extra_flags, "-save-temps=obj", "-o", out, *SOURCES]
-    res = subprocess.run(cmd, capture_output=True, text=True)
+    objs = [os.path.join(tmp, os.path.splitext(os.path.basename(s))[0] + ".o") for s in SOURCES]
+    jobs = [subprocess.Popen([hipcc, *HIPCC_FLAGS, *extra_flags, "-save-temps=obj", "-c", "-o", o, s],
+                             stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+            for s, o in zip(SOURCES, objs)]
+    log = "".join([j.communicate()[0] for j in jobs])
+    if any(j.returncode != 0 for j in jobs):
+        sys.stderr.write(log)
+        raise RuntimeError("hipcc failed building " + LIB_PATH)
+    res = subprocess.run([hipcc, "--offload-arch=gfx950", "-shared", "-o", out, *objs], capture_output=True, text=True)
     if res.returncode != 0:
         sys.stderr.write(res.stdout + res.stderr)
-        raise RuntimeError("hipcc failed building " + LIB_PATH)
+        raise RuntimeError("hipcc failed linking " + LIB_PATH)
     sys.path.insert(0, HERE)
     try:
         import isa_check
@@ -65,7 +73,7 @@ def build_library(verbose: bool = False, extra_flags=()) -> str:
     shutil.rmtree(os.path.join(HERE, "build"), ignore_errors=True)
     if verbose:
         # the host pass does not know the gfx950 feature flag and says so; drop that noise
-        for line in (res.stdout + res.stderr).splitlines():
+        for line in (log + res.stdout + res.stderr).splitlines():
             if "packed-fp32-ops" not in line:
                 print(line)
     return LIB_PATH

@@ -21,6 +21,7 @@
 #include "ttt_linear_fwd_mw.hip.h"
 #include "ttt_linear_fwd_sk.hip.h"
 #include "ttt_mlp_bwd.hip.h"
+#include "ttt_mlp_bwd_rp.hip.h"
 #include "ttt_mlp_fwd_cl2.hip.h"
 #include "ttt_mlp_fwd_rr.hip.h"
 #include "ttt_mlpn_fwd.hip.h"
@@ -28,6 +29,10 @@
 
 // Scratch of ttt_mlp_bwd_static (file scope, outside any namespace so that HIP_SYMBOL names it plainly).
 static __device__ __align__(256) unsigned char ttt_mlp_bwd_scratch_mem[TTT_MLP_BWD_STATIC_MAX_BYTES];
+
+namespace ttt {
+hipError_t launch_mlp_bwd_rp(int head_dim, const MlpBwdRpArgs& a, hipStream_t s);  // ttt_mlp_bwd_rp.hip
+}
 
 namespace {
 
@@ -304,10 +309,10 @@ int launch_mlp_fwd(const ttt::MlpFwdArgs* probs, unsigned ny, hipStream_t s) {
 }
 
 // register-resident kernel (d <= 96, bf16 operands on the matrix cores)
-template <class T, int D>
+template <class T, int D, bool SAVE = false>
 int launch_mlp_fwd_rr(const ttt::MlpFwdArgs* probs, unsigned ny, hipStream_t s) {
   const ttt::MlpFwdArgs& a = probs[0];
-  constexpr auto kern = ttt::ttt_mlp_fwd_rr_kernel<T, D>;
+  constexpr auto kern = ttt::ttt_mlp_fwd_rr_kernel<T, D, SAVE>;
   constexpr size_t bytes = ttt::MlpRrLds<D, sizeof(typename ttt::Io<T>::elem)>::BYTES;
   int rc = opt_in_lds<kern>(bytes);
   if (rc != TTT_OK) return rc;
@@ -445,9 +450,9 @@ int launch_linear_bwd_pair(const ttt::LinearBwdPairArgs& pa, hipStream_t s) {
   return hip_status(hipGetLastError(), "ttt_linear_bwd_ws (two workgroups per unit) launch");
 }
 
-template <class T, int D, bool BF, bool PIPE>
+template <class T, int D, bool PIPE>
 int launch_mlp_bwd_as(const ttt::MlpBwdArgs& a, hipStream_t s) {
-  constexpr auto kern = ttt::ttt_mlp_bwd_kernel<T, D, BF, PIPE>;
+  constexpr auto kern = ttt::ttt_mlp_bwd_kernel<T, D, PIPE>;
   constexpr size_t bytes = ttt::MlpBwdLds<D>::BYTES;
   int rc = opt_in_lds<kern>(bytes);
   if (rc != TTT_OK) return rc;
@@ -456,12 +461,12 @@ int launch_mlp_bwd_as(const ttt::MlpBwdArgs& a, hipStream_t s) {
   hipLaunchKernelGGL(kern, dim3(grid), dim3(512), bytes, s, a);
   return hip_status(hipGetLastError(), "ttt_mlp_bwd launch");
 }
-template <class T, int D, bool BF = false>
+template <class T, int D>
 int launch_mlp_bwd(const ttt::MlpBwdArgs& a, hipStream_t s) {
   static_assert(ttt::MlpBwdPipe<D>::FLOATS == 4 * D * 4 * D + ttt::kMlpBwdSharedTiles * 16 * 4 * D + 2 * ((48 * D + 4 * 256 + 16 + D + 3) / 4 * 4),
                 "MlpBwdWs computes the same size");
-  if (a.pipe != nullptr) return launch_mlp_bwd_as<T, D, BF, true>(a, s);
-  return launch_mlp_bwd_as<T, D, BF, false>(a, s);
+  if (a.pipe != nullptr) return launch_mlp_bwd_as<T, D, true>(a, s);
+  return launch_mlp_bwd_as<T, D, false>(a, s);
 }
 
 // Which TTT-Linear backward kernel serves a desc (and whether one does).
@@ -616,6 +621,85 @@ bool mlp_rr_sweep(const ttt_desc* d) {
   return d->io_dtype != TTT_F32 && d->head_dim <= 96 && !(d->kernel_hint & TTT_HINT_LDS_TILES);
 }
 
+// Whether the backward runs on the register-resident kernel (ttt_mlp_bwd_rp.hip.h): where its products take bf16 operands.
+bool mlp_rp(const ttt_desc* d) { return mlp_rr_sweep(d) && !(d->kernel_hint & TTT_HINT_F32_PRODUCTS); }
+
+// byte offsets of the pieces of its workspace, within what MlpBwdWs describes for the other kernel where that is enough
+struct MlpRpWs {
+  size_t state, b1, b2, fac, hand, flags, total;
+  int slots;
+  explicit MlpRpWs(const ttt_desc* d) {
+    const size_t U = (size_t)d->batch * d->heads, D = d->head_dim, M = 4 * D, N = d->seq / d->mini_batch;
+    const size_t facb = D == 32 ? ttt::MlpRp<32>::FAC : D == 64 ? ttt::MlpRp<64>::FAC : ttt::MlpRp<96>::FAC;
+    const size_t slot = D == 32 ? ttt::MlpRp<32>::SLOT : D == 64 ? ttt::MlpRp<64>::SLOT : ttt::MlpRp<96>::SLOT;
+    state = 0;
+    b1 = state + U * 2 * D * M * sizeof(float);
+    b2 = b1 + U * M * sizeof(float);
+    fac = b2 + U * D * sizeof(float);
+    hand = fac + U * N * facb;
+    const size_t room = MlpBwdWs(d).total * sizeof(float), fix = hand + U * ttt::kMlpRpFlagWords * sizeof(unsigned);
+    // one workgroup per unit: the roles run in turn over as many mini-batches as there are slots
+    size_t n = mlp_bwd_pipe(d) ? 3 : room > fix ? (room - fix) / (U * slot) : 1;
+    n = n < 1 ? 1 : n > 16 ? 16 : n > N && !mlp_bwd_pipe(d) ? N : n;
+    slots = (int)n;
+    flags = hand + U * n * slot;
+    total = flags + U * ttt::kMlpRpFlagWords * sizeof(unsigned);
+    if (total < room) total = room;
+  }
+};
+
+// address of the status word on the current device
+std::atomic<void*> g_lost_word[kMaxDevices];
+int lost_word(unsigned** out) {
+  int dev = -1;
+  int rc = hip_status(hipGetDevice(&dev), "hipGetDevice");
+  if (rc != TTT_OK) return rc;
+  if (dev < 0 || dev >= kMaxDevices) return fail(TTT_ERR_UNSUPPORTED, "device ordinal %d out of range", dev);
+  void* p = g_lost_word[dev].load(std::memory_order_acquire);
+  if (p == nullptr) {
+    rc = hip_status(hipGetSymbolAddress(&p, HIP_SYMBOL(ttt::g_mlp_fwd_lost_workgroups)), "hipGetSymbolAddress(status word)");
+    if (rc != TTT_OK) return rc;
+    g_lost_word[dev].store(p, std::memory_order_release);
+  }
+  *out = static_cast<unsigned*>(p);
+  return TTT_OK;
+}
+
+// the reverse scan on it: two workgroups per unit, or producer and consumer in turn, a few mini-batches at a time
+int run_mlp_bwd_rp(const ttt_desc* d, ttt::MlpBwdRpArgs& a, const MlpRpWs& w, void* workspace, hipStream_t s) {
+  unsigned char* ws = static_cast<unsigned char*>(workspace);
+  a.state = reinterpret_cast<float*>(ws + w.state);
+  a.b1 = reinterpret_cast<float*>(ws + w.b1);
+  a.b2 = reinterpret_cast<float*>(ws + w.b2);
+  a.fac = ws + w.fac;
+  a.hand = ws + w.hand;
+  a.flags = reinterpret_cast<unsigned*>(ws + w.flags);
+  a.B = d->batch; a.H = d->heads; a.K = d->mini_batch; a.n_stages = d->seq / d->mini_batch;
+  a.seq_stride = d->seq_stride > 0 ? d->seq_stride : d->seq;
+  a.eps = d->eps; a.slots = w.slots;
+  a.spin_limit = (d->kernel_hint & TTT_HINT_TEST_LOST_PARTNER) ? 0u : 1u << 21;
+  a.agent_release = (d->kernel_hint & TTT_HINT_TEST_OTHER_XCD) ? 1 : 0;
+  int rc = lost_word(&a.lost_count);
+  if (rc != TTT_OK) return rc;
+  const int64_t U = (int64_t)d->batch * d->heads;
+  int cus = 0;
+  rc = device_cus(&cus);
+  if (rc != TTT_OK) return rc;
+  if (mlp_bwd_pipe(d) && (U + 7) / 8 * 16 <= cus) {  // both workgroups of every unit resident together
+    copy_or_zero(reinterpret_cast<float*>(a.flags), nullptr, (size_t)U * ttt::kMlpRpFlagWords, s);
+    a.first = 0; a.last = a.n_stages; a.role = 2;
+    return hip_status(ttt::launch_mlp_bwd_rp(d->head_dim, a, s), "ttt_mlp_bwd launch");
+  }
+  for (a.last = a.n_stages; a.last > 0; a.last = a.first) {
+    a.first = a.last > a.slots ? a.last - a.slots : 0;
+    for (a.role = 0; a.role < 2; ++a.role) {
+      rc = hip_status(ttt::launch_mlp_bwd_rp(d->head_dim, a, s), "ttt_mlp_bwd launch");
+      if (rc != TTT_OK) return rc;
+    }
+  }
+  return TTT_OK;
+}
+
 // sweep = false: the workspace already holds what the sweep leaves there (ttt_mlp_fwd_saving wrote it)
 int mlp_bwd_impl(const ttt_desc* d, const void* xq, const void* xk, const void* xv,
                 const float* W1_0, const float* b1_0, const float* W2_0, const float* b2_0,
@@ -655,14 +739,24 @@ int mlp_bwd_impl(const ttt_desc* d, const void* xq, const void* xk, const void* 
   fa.n_stages = d->seq / d->mini_batch;
   fa.state_per_batch = d->state_per_batch ? 1 : 0;
   fa.eps = d->eps;
+  const bool rp = mlp_rp(d);
+  if (rp) {
+    const MlpRpWs rw(d);
+    unsigned char* wb = static_cast<unsigned char*>(workspace);
+    fa.W1 = fa.b1 = fa.W2 = fa.b2 = fa.G1_save = fa.G2_save = nullptr;
+    fa.fac_save = wb + rw.fac;
+    fa.state_save = reinterpret_cast<float*>(wb + rw.state);
+    fa.b1_save = reinterpret_cast<float*>(wb + rw.b1);
+    fa.b2_save = reinterpret_cast<float*>(wb + rw.b2);
+  }
   if (!sweep) {
     rc = TTT_OK;
   } else if (rr_sweep) {
     fa.out = d_xq;
     switch (d->head_dim) {
-      case 32: rc = launch_mlp_fwd_rr<ttt::BF16, 32>(&fa, 1, s); break;
-      case 64: rc = launch_mlp_fwd_rr<ttt::BF16, 64>(&fa, 1, s); break;
-      default: rc = launch_mlp_fwd_rr<ttt::BF16, 96>(&fa, 1, s); break;
+      case 32: rc = launch_mlp_fwd_rr<ttt::BF16, 32, true>(&fa, 1, s); break;
+      case 64: rc = launch_mlp_fwd_rr<ttt::BF16, 64, true>(&fa, 1, s); break;
+      default: rc = launch_mlp_fwd_rr<ttt::BF16, 96, true>(&fa, 1, s); break;
     }
   } else
   switch (d->head_dim) {
@@ -673,17 +767,27 @@ int mlp_bwd_impl(const ttt_desc* d, const void* xq, const void* xk, const void* 
   }
   if (rc != TTT_OK) return rc;
 
-  // gradient accumulators start from the upstream state gradients (or zero); the reductions over
-  // batch / heads start from zero
-  copy_or_zero(d_W1, d_W1_out, U * D * M, s);
-  copy_or_zero(d_b1, d_b1_out, U * M, s);
-  copy_or_zero(d_W2, d_W2_out, U * M * D, s);
-  copy_or_zero(d_b2, d_b2_out, U * D, s);
+  // the reductions over batch / heads start from zero
   {
     const size_t hd = (size_t)d->heads * D, nmax = (size_t)d->seq > hd ? (size_t)d->seq : hd;
     hipLaunchKernelGGL(ttt::ttt_fill_zero3_kernel, dim3((unsigned)((nmax + 255) / 256)), dim3(256), 0, s, d_token_eta,
                        (size_t)d->seq, d_gamma, hd, d_beta, hd);
   }
+  if (rp) {
+    ttt::MlpBwdRpArgs ra{};
+    ra.xq = xq; ra.xk = xk; ra.xv = xv; ra.d_out = d_out; ra.lr = lr;
+    ra.token_eta = token_eta; ra.gamma = gamma; ra.beta = beta;
+    ra.up_W1 = d_W1_out; ra.up_b1 = d_b1_out; ra.up_W2 = d_W2_out; ra.up_b2 = d_b2_out;
+    ra.d_W1 = d_W1; ra.d_b1 = d_b1; ra.d_W2 = d_W2; ra.d_b2 = d_b2;
+    ra.d_xq = d_xq; ra.d_xk = d_xk; ra.d_xv = d_xv; ra.d_lr = d_lr;
+    ra.d_token_eta = d_token_eta; ra.d_gamma = d_gamma; ra.d_beta = d_beta;
+    return run_mlp_bwd_rp(d, ra, MlpRpWs(d), workspace, s);
+  }
+  // gradient accumulators start from the upstream state gradients (or zero)
+  copy_or_zero(d_W1, d_W1_out, U * D * M, s);
+  copy_or_zero(d_b1, d_b1_out, U * M, s);
+  copy_or_zero(d_W2, d_W2_out, U * M * D, s);
+  copy_or_zero(d_b2, d_b2_out, U * D, s);
   rc = hip_status(hipGetLastError(), "ttt_mlp_bwd fills");
   if (rc != TTT_OK) return rc;
 
@@ -711,13 +815,6 @@ int mlp_bwd_impl(const ttt_desc* d, const void* xq, const void* xk, const void* 
       if (rc != TTT_OK) return rc;
     }
   }
-  // behind the register-resident sweep the scan takes bf16 operands too (the states it walks back through were
-  // formed from bf16 operands); TTT_HINT_F32_PRODUCTS keeps the scan's products in f32
-  if (rr_sweep && !(d->kernel_hint & TTT_HINT_F32_PRODUCTS)) switch (d->head_dim) {
-      case 32: return launch_mlp_bwd<ttt::BF16, 32, true>(a, s);
-      case 64: return launch_mlp_bwd<ttt::BF16, 64, true>(a, s);
-      default: return launch_mlp_bwd<ttt::BF16, 96, true>(a, s);
-    }
   switch (d->head_dim) {
     case 32: return f32 ? launch_mlp_bwd<ttt::F32, 32>(a, s) : launch_mlp_bwd<ttt::BF16, 32>(a, s);
     case 64: return f32 ? launch_mlp_bwd<ttt::F32, 64>(a, s) : launch_mlp_bwd<ttt::BF16, 64>(a, s);
@@ -1383,10 +1480,11 @@ int dispatch_mlp_fwd_pack(const ttt_desc* d, const ttt::MlpFwdArgs* a, unsigned 
   const bool f32 = d->io_dtype == TTT_F32;
   const bool want_lds = (d->kernel_hint & TTT_HINT_LDS_TILES) != 0;
   if (!f32 && d->head_dim <= 96 && !want_lds) {
+    const bool save = a[0].fac_save != nullptr || a[0].G1_save != nullptr;
     switch (d->head_dim) {
-      case 32: return launch_mlp_fwd_rr<ttt::BF16, 32>(a, ny, s);
-      case 64: return launch_mlp_fwd_rr<ttt::BF16, 64>(a, ny, s);
-      default: return launch_mlp_fwd_rr<ttt::BF16, 96>(a, ny, s);
+      case 32: return save ? launch_mlp_fwd_rr<ttt::BF16, 32, true>(a, ny, s) : launch_mlp_fwd_rr<ttt::BF16, 32>(a, ny, s);
+      case 64: return save ? launch_mlp_fwd_rr<ttt::BF16, 64, true>(a, ny, s) : launch_mlp_fwd_rr<ttt::BF16, 64>(a, ny, s);
+      default: return save ? launch_mlp_fwd_rr<ttt::BF16, 96, true>(a, ny, s) : launch_mlp_fwd_rr<ttt::BF16, 96>(a, ny, s);
     }
   }
   switch (d->head_dim) {
@@ -1439,7 +1537,7 @@ int ttt_mlp_fwd_lost_workgroups(int64_t* count) {
 
 int64_t ttt_mlp_bwd_workspace_bytes(const ttt_desc* d) {
   if (ttt_mlp_supported(d) != TTT_OK) return -1;
-  return (int64_t)(MlpBwdWs(d).total * sizeof(float));
+  return (int64_t)(mlp_rp(d) ? MlpRpWs(d).total : MlpBwdWs(d).total * sizeof(float));
 }
 
 int ttt_mlp_bwd(const ttt_desc* d, const void* xq, const void* xk, const void* xv,
@@ -1479,11 +1577,20 @@ int ttt_mlp_fwd_saving(const ttt_desc* d, const void* xq, const void* xk, const 
   rc = prepare_mlp_fwd(d, xq, xk, xv, W1_0, b1_0, W2_0, b2_0, token_eta, lr, gamma, beta, out, W1_out, b1_out, W2_out,
                        b2_out, &a);
   if (rc != TTT_OK) return rc;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  if (mlp_rp(d)) {
+    const MlpRpWs w(d);
+    unsigned char* wb = static_cast<unsigned char*>(saved);
+    a.fac_save = wb + w.fac;
+    a.state_save = reinterpret_cast<float*>(wb + w.state);
+    a.b1_save = reinterpret_cast<float*>(wb + w.b1);
+    a.b2_save = reinterpret_cast<float*>(wb + w.b2);
+    return dispatch_mlp_fwd_pack(d, &a, 1, s);
+  }
   const MlpBwdWs w(d);
   float* ws = static_cast<float*>(saved);
   a.G1_save = ws + w.G1s;
   a.G2_save = ws + w.G2s;
-  hipStream_t s = static_cast<hipStream_t>(stream);
   rc = dispatch_mlp_fwd_pack(d, &a, 1, s);
   if (rc != TTT_OK) return rc;
   // the reverse scan walks the state back in place: it gets a copy of the final state of its own

@@ -210,6 +210,13 @@ struct MlpFwdArgs {
   // eta_last * G1 [B*H][N][16][M] and eta_last * G2 [B*H][N][16][D], for ttt_mlp_bwd; out may then be null
   float* G1_save;
   float* G2_save;
+  // optional (register-resident kernel only): what the register-resident backward starts from -- the factors as the
+  // fragments the update multiplies (MlpRp<d>::FAC bytes per mini-batch), the final state in accumulator order (second
+  // layer centred) and its biases
+  unsigned char* fac_save = nullptr;
+  float* state_save = nullptr;
+  float* b1_save = nullptr;
+  float* b2_save = nullptr;
   int B, H, seq, seq_stride, K, n_stages, state_per_batch;
   float eps;
   int unit_base;  // two-CU kernel only: first (batch, head) unit of this launch (the units are launched in batches)

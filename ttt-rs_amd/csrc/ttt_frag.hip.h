@@ -269,6 +269,26 @@ __device__ __forceinline__ f32x4 rope_rotate4(f32x4 x, f32x2 cs, f32x2 sn) {
 // ttt_lr_eta of a token: scale * sigmoid(z), scale = base_lr / head_dim (reference rust/layer/src/ttt.rs:205-227)
 __device__ __forceinline__ float lr_gate(float z, float scale) { return scale / (1.f + __expf(-z)); }
 
+// The same through the hardware exp2 / rcp (absolute error about 1e-7): for the kernels whose VALU issue
+// is the bottleneck.
+// y = gelu_tanh(x), dy = its derivative.  With r = 1 / (1 + exp(2u)), u = c (x + a x^3):
+// (1 + tanh u) / 2 = 1 - r and 1 - tanh^2 u = 4 r (1 - r).
+__device__ __forceinline__ void gelu_fast_pair(float x, float& y, float& dy) {
+  const float c2 = 2.f * 0.7978845608f;
+  const float x2 = x * x;
+  const float u = x * __builtin_fmaf(0.044715f, x2, 1.f);
+  const float e = __builtin_amdgcn_exp2f(u * (c2 * 1.4426950409f));
+  const float r = __builtin_amdgcn_rcpf(1.f + e);
+  const float hp = 1.f - r;
+  y = x * hp;
+  dy = hp * __builtin_fmaf(c2 * __builtin_fmaf(3.f * 0.044715f, x2, 1.f), x * r, 1.f);
+}
+__device__ __forceinline__ float gelu_fast(float x) {
+  const float u = x * __builtin_fmaf(0.044715f, x * x, 1.f);
+  const float e = __builtin_amdgcn_exp2f(u * (2.f * 0.7978845608f * 1.4426950409f));
+  return x - x * __builtin_amdgcn_rcpf(1.f + e);
+}
+
 // A launch may carry several independent problems of one shape, gridDim.y of them (windows of different layers of
 // a stack that are ready at the same time: one layer's 64 units alone leave three quarters of the CUs idle).  The
 // argument blocks of all of them travel as kernel arguments and workgroup (x, y) works on block y: the index is

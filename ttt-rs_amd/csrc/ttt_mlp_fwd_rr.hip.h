@@ -105,7 +105,9 @@ __device__ __forceinline__ float mean_of(const float* p, int d, float inv_d) {
 // phase makes them cheap phase-local recomputations instead.
 #define RELANE() asm volatile("" : "+v"(lane))
 
-template <class T, int D>
+// SAVE: also leave what a backward starts from (MlpFwdArgs::fac_save or G1_save).  A compilation of its own: the pointers
+// and branches cost the plain forward 3 % of its time in registers.
+template <class T, int D, bool SAVE>
 __global__ void __launch_bounds__(512) ttt_mlp_fwd_rr_kernel(Problems<MlpFwdArgs> problems) {
   const MlpFwdArgs& a = problems.p[blockIdx.y];
   using IO = Io<T>;
@@ -434,7 +436,10 @@ __global__ void __launch_bounds__(512) ttt_mlp_fwd_rr_kernel(Problems<MlpFwdArgs
     // (G'' = -eta_last * lr * G); zeros when token_eta[K-1] = 0 switches the update off.  Stored behind B3 so
     // that the counted waits of phase C see the same memory operations as without them.
     const size_t save_row = (bh * (size_t)a.n_stages + st) * 16 + c;
-    if (a.G2_save != nullptr && red) {
+    unsigned char* const facp =
+        SAVE && a.fac_save != nullptr ? a.fac_save + (bh * (size_t)a.n_stages + st) * ((NW * HT + NT) * 512) : nullptr;
+    if (SAVE && facp != nullptr && red) *reinterpret_cast<frag*>(facp + (NW * HT + w) * 512 + lane * 8) = GD[w * 64 + lane];
+    if (SAVE && a.G2_save != nullptr && red) {
       const f32x4 v = upd ? -IO::to_f32(g2_saved) : f32x4{0.f, 0.f, 0.f, 0.f};
       *reinterpret_cast<f32x4*>(a.G2_save + save_row * D + own) = v;
     }
@@ -457,7 +462,8 @@ __global__ void __launch_bounds__(512) ttt_mlp_fwd_rr_kernel(Problems<MlpFwdArgs
       const frag g1b = IO::to_frag(acc * dg[j]);
       IO::mma(t, g1b, ident);
       G1d[j] = IO::to_frag(t);
-      if (a.G1_save != nullptr) {
+      if (SAVE && facp != nullptr) *reinterpret_cast<frag*>(facp + (w * HT + j) * 512 + lane * 8) = G1d[j];
+      if (SAVE && a.G1_save != nullptr) {
         const f32x4 v = upd ? -IO::to_f32(g1b) : f32x4{0.f, 0.f, 0.f, 0.f};
         *reinterpret_cast<f32x4*>(a.G1_save + save_row * F + 16 * (w * HT + j) + 4 * g) = v;
       }
@@ -552,6 +558,22 @@ __global__ void __launch_bounds__(512) ttt_mlp_fwd_rr_kernel(Problems<MlpFwdArgs
   lds_barrier();
   if (outw) output_emit(a.n_stages - 1);
 
+  if (SAVE && a.state_save != nullptr) {
+    f32x4* s1 = reinterpret_cast<f32x4*>(a.state_save + bh * (size_t)(2 * D * F)) + (w * NT * HT) * 64 + lane;
+    f32x4* s2 = s1 + NW * NT * HT * 64;
+#pragma unroll
+    for (int j = 0; j < HT; ++j) {
+#pragma unroll
+      for (int I = 0; I < NT; ++I) {
+        s1[(I * HT + j) * 64] = W1c[I][j];
+        s2[(j * NT + I) * 64] = W2c[j][I];
+      }
+      const int hb = 16 * (w * HT + j);
+      if (c == 0) store4<F32>(a.b1_save + bh * F + hb + 4 * g, *reinterpret_cast<const f32x4*>(B1s + hb + 4 * g));
+    }
+    if (red && c == 0) store4<F32>(a.b2_save + bh * D + own, b2T);
+  }
+  if (SAVE && a.W1 == nullptr) return;
   // ---- final state.  Second layer: initial value + (centred value now - centred value at the start), the start
   // value formed again exactly as above, so a sequence that never updates the state returns it bit for bit.
   {
