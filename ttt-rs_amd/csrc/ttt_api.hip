@@ -998,6 +998,41 @@ int ttt_mlpn_fwd(const ttt_desc* d, int n_hidden, const void* xq, const void* xk
   }
 }
 
+}  // extern "C"
+namespace {
+template <class T, int D, int NW, int PF, int RAW, bool COMPACT, int OCC>
+void launch_linear_adam_variant(const ttt::LinearFwdArgs& a, const ttt::AdamArgs& ad, hipStream_t s) {
+  const dim3 grid((unsigned)(a.B * a.H)), block(64 * (NW + (RAW == 5)));
+  if constexpr (RAW != 5) {  // (the control wave copies whole mini-batches of 16 tokens only)
+    if (a.K != 16) {
+      hipLaunchKernelGGL((ttt::ttt_linear_adam_fwd_kernel<T, D, NW, PF, false, RAW, COMPACT, OCC>), grid, block, 0, s, a, ad);
+      return;
+    }
+  }
+  hipLaunchKernelGGL((ttt::ttt_linear_adam_fwd_kernel<T, D, NW, PF, true, RAW, COMPACT, OCC>), grid, block, 0, s, a, ad);
+}
+// head_dim 64: a wave per feature tile while every unit has a CU to itself.  Beyond that two waves per unit with bf16 I/O
+// (four would put two on a SIMD: 324 us at 384 units, against 237); with f32 I/O the products fill a second wave's gaps
+// and four stay ahead (538 against 551), two to a SIMD.  head_dim 32: two waves, alone on their SIMDs up to two units per
+// CU.  (2048 tokens.)
+template <class T>
+void launch_linear_adam(int head_dim, int64_t units, int cus, const ttt::LinearFwdArgs& a, const ttt::AdamArgs& ad, hipStream_t s) {
+  constexpr bool f32 = sizeof(typename ttt::Io<T>::elem) == 4;
+  if (head_dim == 32) {
+    constexpr int PF = f32 ? 2 : 1;
+    if (units <= 2 * (int64_t)cus) launch_linear_adam_variant<T, 32, 2, PF, 0, false, 1>(a, ad, s);
+    else launch_linear_adam_variant<T, 32, 2, PF, 0, false, 2>(a, ad, s);
+  } else if constexpr (f32) {
+    if (units <= cus && a.K == 16) launch_linear_adam_variant<T, 64, 4, 2, 5, false, 2>(a, ad, s);
+    else launch_linear_adam_variant<T, 64, 4, 1, 0, true, 2>(a, ad, s);
+  } else {
+    if (units <= cus) launch_linear_adam_variant<T, 64, 4, 2, 3, true, 1>(a, ad, s);
+    else launch_linear_adam_variant<T, 64, 2, 2, 3, false, 1>(a, ad, s);
+  }
+}
+}  // namespace
+extern "C" {
+
 int ttt_linear_adam_supported(const ttt_desc* d) {
   int rc = ttt_linear_supported(d);
   if (rc != TTT_OK) return rc;
@@ -1034,21 +1069,13 @@ int ttt_linear_adam_fwd(const ttt_desc* d, const void* xq, const void* xk, const
   ad.Wm0 = Wm0; ad.bm0 = bm0; ad.Wv0 = Wv0; ad.bv0 = bv0;
   ad.Wm_out = Wm_out; ad.bm_out = bm_out; ad.Wv_out = Wv_out; ad.bv_out = bv_out;
   ad.beta1 = beta1; ad.beta2 = beta2; ad.eps = adam_eps; ad.lr = adam_lr; ad.step0 = step0;
-  const dim3 grid((unsigned)(a.B * a.H)), block(128);
+  int cus = 0;
+  rc = device_cus(&cus);
+  if (rc != TTT_OK) return rc;
+  const int64_t units = (int64_t)a.B * a.H;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const bool full = d->mini_batch == 16, f32 = d->io_dtype == TTT_F32;
-  // head_dim 64 holds state and both moments in 96 registers per wave: the rows are prefetched one mini-batch ahead
-  // there (two ahead would spill hundreds of registers), two ahead at head_dim 32
-#define TTT_ADAM_LAUNCH(T_, D_, FULL_) \
-  hipLaunchKernelGGL((ttt::ttt_linear_adam_fwd_kernel<T_, D_, 2, (D_ == 64 ? 1 : 2), FULL_>), grid, block, 0, s, a, ad)
-  if (d->head_dim == 64) {
-    if (f32) { if (full) TTT_ADAM_LAUNCH(ttt::F32, 64, true); else TTT_ADAM_LAUNCH(ttt::F32, 64, false); }
-    else { if (full) TTT_ADAM_LAUNCH(ttt::BF16, 64, true); else TTT_ADAM_LAUNCH(ttt::BF16, 64, false); }
-  } else {
-    if (f32) { if (full) TTT_ADAM_LAUNCH(ttt::F32, 32, true); else TTT_ADAM_LAUNCH(ttt::F32, 32, false); }
-    else { if (full) TTT_ADAM_LAUNCH(ttt::BF16, 32, true); else TTT_ADAM_LAUNCH(ttt::BF16, 32, false); }
-  }
-#undef TTT_ADAM_LAUNCH
+  if (d->io_dtype == TTT_F32) launch_linear_adam<ttt::F32>(d->head_dim, units, cus, a, ad, s);
+  else launch_linear_adam<ttt::BF16>(d->head_dim, units, cus, a, ad, s);
   return hip_status(hipGetLastError(), "ttt_linear_adam_fwd launch");
 }
 

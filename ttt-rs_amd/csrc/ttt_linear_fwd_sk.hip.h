@@ -49,13 +49,14 @@ namespace ttt {
 // zero accumulator, the moments live in registers beside the state (three times the state's registers), bias
 // corrections come from running powers of beta1, beta2.  Everything else -- products, LayerNorm, output -- is the
 // plain kernel's; the output of a mini-batch does not see its own update in either.
+// COMPACT: one loop body per ring slot, with the branches of the first and the last pass (see `pass` below).
 // STATES: only the recurrence runs, from a given state, and the state entering every one of n_stages + 1 mini-batches is
 // written as a checkpoint: no output, no attention block, no final state (see ttt_linear_states_kernel).  The unit and the
 // index of its initial state are then given (unit, state) instead of following from the workgroup's index.
-template <class T, int D, int NW, int PF, bool FULL, bool FAC, int RAW, bool ADAM = false, bool STATES = false>
+template <class T, int D, int NW, int PF, bool FULL, bool FAC, int RAW, bool ADAM = false, bool STATES = false, bool COMPACT = false>
 __device__ __forceinline__ void linear_fwd_sk_body(const LinearFwdArgs& a, const FusedInputsArgs* fip,
                                                    const AdamArgs* adam = nullptr, size_t unit = 0, size_t state = 0) {
-  static_assert(!ADAM || (D <= 64 && !FAC && RAW == 0), "Adam inner optimiser: head_dim <= 64, no checkpoints");
+  static_assert(!ADAM || (D <= 64 && !FAC && (RAW == 0 || RAW == 3 || RAW == 5)), "Adam inner optimiser: head_dim <= 64, operands given, no checkpoints");
   static_assert(!STATES || (D <= 64 && !FAC && RAW == 0 && !ADAM), "states alone: head_dim <= 64, operands given");
   using IO = Io<T>;
   using frag = typename IO::frag;
@@ -131,6 +132,7 @@ __device__ __forceinline__ void linear_fwd_sk_body(const LinearFwdArgs& a, const
   float pw1 = 1.f, pw2 = 1.f;
   if constexpr (ADAM) {
     const bool have = adam->Wm0 != nullptr;
+    const float um = 1.f / (1.f - adam->beta1), uv = 1.f / (1.f - adam->beta2);
 #pragma unroll
     for (int I = 0; I < NT; ++I)
 #pragma unroll
@@ -138,34 +140,36 @@ __device__ __forceinline__ void linear_fwd_sk_body(const LinearFwdArgs& a, const
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           const size_t at = bh * D * D + feat(I, 4 * g + r) * D + feat(w * TPW + jj, c);
-          Wm[I][jj][r] = have ? adam->Wm0[at] : 0.f;
-          Wv[I][jj][r] = have ? adam->Wv0[at] : 0.f;
+          Wm[I][jj][r] = have ? adam->Wm0[at] * um : 0.f;
+          Wv[I][jj][r] = have ? adam->Wv0[at] * uv : 0.f;
         }
 #pragma unroll
     for (int jj = 0; jj < TPW; ++jj)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const size_t at = bh * D + own_offset<TPW>(w, jj, g) + r;
-        bm[jj][r] = have ? adam->bm0[at] : 0.f;
-        bv[jj][r] = have ? adam->bv0[at] : 0.f;
+        bm[jj][r] = have ? adam->bm0[at] * um : 0.f;
+        bv[jj][r] = have ? adam->bv0[at] * uv : 0.f;
       }
     for (int i = 0; i < adam->step0; ++i) {
       pw1 *= adam->beta1;
       pw2 *= adam->beta2;
     }
   }
-  // one Adam step on a tile: gneg = -gradient (what the plain kernel would add to the state)
-  float ad_a1 = 0.f, ad_ic2 = 0.f;  // lr / (1 - beta1^t), 1 / (1 - beta2^t) of the current step
+  // One Adam step on a tile: gneg = -gradient (what the plain kernel would add to the state).  The moments are carried
+  // as m / (1 - beta1) and v / (1 - beta2), so that each decays and takes its new term in one or two instructions, and
+  // lr m^ / (sqrt(v^) + eps) is taken as ad_k m / (sqrt(v) + ad_e) with the bias corrections in the two scalars: eight
+  // instructions per element, two of them transcendental, where the step as written has eleven.
+  float ad_k = 0.f, ad_e = 0.f;
   auto adam_tile = [&](f32x4& x, f32x4& m, f32x4& v, f32x4 gneg) {
     if constexpr (ADAM) {
       const float b1 = adam->beta1, b2 = adam->beta2;
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const float gr = -gneg[r];
-        m[r] = __builtin_fmaf(b1, m[r], (1.f - b1) * gr);
-        v[r] = __builtin_fmaf(b2, v[r], (1.f - b2) * (gr * gr));
-        const float den = __builtin_amdgcn_sqrtf(v[r] * ad_ic2) + adam->eps;  // 1 ulp; v is far above the denormals
-        x[r] = __builtin_fmaf(-(ad_a1 * m[r]), __builtin_amdgcn_rcpf(den), x[r]);
+        m[r] = __builtin_fmaf(b1, m[r], -gneg[r]);
+        v[r] = __builtin_fmaf(b2, v[r], gneg[r] * gneg[r]);
+        const float den = __builtin_amdgcn_sqrtf(v[r]) + ad_e;  // 1 ulp; v is far above the denormals
+        x[r] = __builtin_fmaf(ad_k, m[r] * __builtin_amdgcn_rcpf(den), x[r]);
       }
     }
   };
@@ -601,7 +605,7 @@ __device__ __forceinline__ void linear_fwd_sk_body(const LinearFwdArgs& a, const
       }
       // ---- checkpoint of the state entering this mini-batch (W and b change only behind the barrier);
       // placed at the barrier so that its branch does not cut the stretch in two
-      if (ck.due()) {
+      if (!ADAM && ck.due()) {
         if (ck.packed) {
           store_ckpt_packed<T, NT, TPW>(ck.W, Wc, w, lane);
           store_bias_true<D, TPW>(ck.b, bT, b_mean, w, c, g);
@@ -610,7 +614,7 @@ __device__ __forceinline__ void linear_fwd_sk_body(const LinearFwdArgs& a, const
         }
         ck.advance();
       }
-      ck.next_stage();
+      if constexpr (!ADAM) ck.next_stage();
       exchange8_publish(S, st & 1);
       // ---- the output pending since two mini-batches (sums known since the last exchange): nothing waits
       // for it, and here it runs while this exchange is in flight (LDS write, barrier, LDS read)
@@ -673,8 +677,12 @@ __device__ __forceinline__ void linear_fwd_sk_body(const LinearFwdArgs& a, const
       if constexpr (ADAM) {
         pw1 *= adam->beta1;
         pw2 *= adam->beta2;
-        ad_a1 = adam->lr / (1.f - pw1);
-        ad_ic2 = 1.f / (1.f - pw2);
+        {
+          // v^ = v c2, m^ = m c1: lr m^ / (sqrt(v^) + eps) = (lr c1 / sqrt(c2)) m / (sqrt(v) + eps / sqrt(c2))
+          const float c1 = (1.f - adam->beta1) / (1.f - pw1), rc2 = sqrtf((1.f - pw2) / (1.f - adam->beta2));
+          ad_k = -adam->lr * c1 * rc2;
+          ad_e = adam->eps * rc2;
+        }
 #pragma unroll
         for (int I = 0; I < NT; ++I)
 #pragma unroll
@@ -712,7 +720,9 @@ __device__ __forceinline__ void linear_fwd_sk_body(const LinearFwdArgs& a, const
       if constexpr (RAW != 0) rotate_share(raw[(u + 2) % R], buf[(u + 2) % R], st + 2, st & 1);
     }
   };
-  if constexpr (NT <= 4) {
+  if constexpr (COMPACT) {
+    for (int st0 = 0; st0 < a.n_stages; st0 += R) pass(std::true_type{}, st0);
+  } else if constexpr (NT <= 4) {
     int st0 = 0;
     pass(std::true_type{}, st0);
     for (st0 = R; st0 + R <= a.n_stages; st0 += R) pass(std::false_type{}, st0);
@@ -878,15 +888,15 @@ __device__ __forceinline__ void linear_fwd_sk_body(const LinearFwdArgs& a, const
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           const size_t at = bh * D * D + feat(I, 4 * g + r) * D + feat(w * TPW + jj, c);
-          adam->Wm_out[at] = Wm[I][jj][r];
-          adam->Wv_out[at] = Wv[I][jj][r];
+          adam->Wm_out[at] = Wm[I][jj][r] * (1.f - adam->beta1);
+          adam->Wv_out[at] = Wv[I][jj][r] * (1.f - adam->beta2);
         }
     if (c == 0) {
 #pragma unroll
       for (int jj = 0; jj < TPW; ++jj) {
         const size_t at = bh * D + own_offset<TPW>(w, jj, g);
-        *reinterpret_cast<f32x4*>(adam->bm_out + at) = bm[jj];
-        *reinterpret_cast<f32x4*>(adam->bv_out + at) = bv[jj];
+        *reinterpret_cast<f32x4*>(adam->bm_out + at) = bm[jj] * (1.f - adam->beta1);
+        *reinterpret_cast<f32x4*>(adam->bv_out + at) = bv[jj] * (1.f - adam->beta2);
       }
     }
   }
@@ -907,10 +917,17 @@ __global__ void __launch_bounds__(64 * (NW + 1)) ttt_linear_fwd_dma_kernel(Probl
   linear_fwd_sk_body<T, D, NW, PF, true, false, 5>(problems.p[blockIdx.y], nullptr);
 }
 
-// TTT-Linear with the Adam inner optimiser: see ADAM above.
-template <class T, int D, int NW, int PF, bool FULL>
-__global__ void __launch_bounds__(64 * NW) ttt_linear_adam_fwd_kernel(LinearFwdArgs a, AdamArgs ad) {
-  linear_fwd_sk_body<T, D, NW, PF, FULL, false, 0, true>(a, nullptr, &ad);
+// TTT-Linear with the Adam inner optimiser: see ADAM above.  Bound by the chain of a mini-batch, and in it by the issue
+// of the optimiser's step (eight instructions per element of the state, two of them transcendental at a quarter of the
+// rate) and by fetching instructions.  Hence one wave per feature tile where a unit has a CU to itself, rows loaded by
+// their owners and shared through LDS (bf16) or copied in by a control wave (f32), and the loop without its branch-free
+// copies where a body is long (COMPACT: 207 us instead of 161).  OCC: waves per SIMD that the register allocation
+// allows; with one, the two waves of a second workgroup on a CU land on the other two SIMDs (d = 32, 384 units: 174 us
+// with two, 114 with one).  2048 tokens, d = 64, bf16: 96 units 260 -> 162 us, 384 units 263 -> 231; f32: 96 units 534 ->
+// 285, 384 units 545 -> 538.
+template <class T, int D, int NW, int PF, bool FULL, int RAW, bool COMPACT, int OCC>
+__global__ void __launch_bounds__(64 * (NW + (RAW == 5))) __attribute__((amdgpu_waves_per_eu(OCC, OCC))) ttt_linear_adam_fwd_kernel(LinearFwdArgs a, AdamArgs ad) {
+  linear_fwd_sk_body<T, D, NW, PF, FULL, false, RAW, true, false, COMPACT>(a, nullptr, &ad);
 }
 
 // The same forward on the projections as they leave the GEMMs: see RAW above.
