@@ -13,7 +13,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_DIR = os.path.join(HERE, "lib")
 LIB_PATH = os.path.join(LIB_DIR, "libttt_mi355x.so")
 # translation units, compiled side by side
-SOURCES = [os.path.join(HERE, "csrc", f) for f in ("ttt_api.hip", "ttt_mlp_bwd_rp.hip")]
+SOURCES = [os.path.join(HERE, "csrc", f) for f in ("ttt_api.hip", "ttt_mlp_bwd_rp.hip", "ttt_mlpn_fwd.hip")]
 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC",

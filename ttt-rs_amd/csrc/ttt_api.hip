@@ -32,6 +32,19 @@ static __device__ __align__(256) unsigned char ttt_mlp_bwd_scratch_mem[TTT_MLP_B
 
 namespace ttt {
 hipError_t launch_mlp_bwd_rp(int head_dim, const MlpBwdRpArgs& a, hipStream_t s);  // ttt_mlp_bwd_rp.hip
+
+__global__ void ttt_fill_zero_kernel(float* p, size_t n) {
+  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) p[i] = 0.f;
+}
+// three small buffers in one launch (the accumulated outputs of a backward: every launch costs a few microseconds
+// on the stream whatever it does)
+__global__ void ttt_fill_zero3_kernel(float* p0, size_t n0, float* p1, size_t n1, float* p2, size_t n2) {
+  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n0) p0[i] = 0.f;
+  if (i < n1) p1[i] = 0.f;
+  if (i < n2) p2[i] = 0.f;
+}
 }
 
 namespace {
@@ -927,18 +940,6 @@ int dispatch_linear_fwd(const ttt_desc* d, const ttt::LinearFwdArgs* probs, int 
 }
 }  // namespace
 
-namespace {
-template <class T, int D, int NL>
-int launch_mlpn(const ttt::MlpNFwdArgs& a, hipStream_t s) {
-  constexpr auto kern = ttt::ttt_mlpn_fwd_kernel<T, D, NL>;
-  constexpr size_t bytes = ttt::MlpNLds<D, NL>::BYTES;
-  int rc = opt_in_lds<kern>(bytes);
-  if (rc != TTT_OK) return rc;
-  hipLaunchKernelGGL(kern, dim3((unsigned)(a.B * a.H)), dim3(512), bytes, s, a);
-  return hip_status(hipGetLastError(), "ttt_mlpn_fwd launch");
-}
-}  // namespace
-
 extern "C" {
 
 int ttt_linear_fwd(const ttt_desc* d, const void* xq, const void* xk, const void* xv,
@@ -989,13 +990,7 @@ int ttt_mlpn_fwd(const ttt_desc* d, int n_hidden, const void* xq, const void* xk
   a.state_per_batch = d->state_per_batch ? 1 : 0;
   a.eps = d->eps;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const bool f32 = d->io_dtype == TTT_F32;
-  if (d->head_dim == 64) return f32 ? launch_mlpn<ttt::F32, 64, 2>(a, s) : launch_mlpn<ttt::BF16, 64, 2>(a, s);
-  switch (n_hidden) {
-    case 2: return f32 ? launch_mlpn<ttt::F32, 32, 2>(a, s) : launch_mlpn<ttt::BF16, 32, 2>(a, s);
-    case 3: return f32 ? launch_mlpn<ttt::F32, 32, 3>(a, s) : launch_mlpn<ttt::BF16, 32, 3>(a, s);
-    default: return f32 ? launch_mlpn<ttt::F32, 32, 4>(a, s) : launch_mlpn<ttt::BF16, 32, 4>(a, s);
-  }
+  return hip_status(ttt::launch_mlpn_fwd(d->io_dtype == TTT_F32, d->head_dim, n_hidden, a, s), "ttt_mlpn_fwd launch");
 }
 
 }  // extern "C"

@@ -548,23 +548,27 @@ __device__ __forceinline__ float rowgroup_sum(float v) {
 }
 __device__ __forceinline__ float row16_sum(float v) { return rowgroup_sum<16>(v); }
 
-__global__ void ttt_fill_zero_kernel(float* p, size_t n) {
-  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) p[i] = 0.f;
-}
-// three small buffers in one launch (the accumulated outputs of a backward: every launch costs a few microseconds
-// on the stream whatever it does)
-__global__ void ttt_fill_zero3_kernel(float* p0, size_t n0, float* p1, size_t n1, float* p2, size_t n2) {
-  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n0) p0[i] = 0.f;
-  if (i < n1) p1[i] = 0.f;
-  if (i < n2) p2[i] = 0.f;
+// tanh without a branch: a polynomial in u^2 for |u| < 0.6 (own fit: weighted least squares on Chebyshev nodes, weights
+// iterated until the relative error is level, 2.8e-9), 1 - 2 / (1 + exp(2 |u|)) above.  The 2-norm error of gelu and
+// gelu' built on it is that of a correctly rounded tanh to three digits for N(0, s^2) inputs, s = 0.02 .. 10.  tanhf
+// branches on its argument, which a wave with both kinds of it walks twice, one evaluation after the other.
+__device__ __forceinline__ float tanh_nobranch(float u) {
+  const float s = u * u, v = __builtin_fabsf(u);
+  float p = -0.005895157344639301f;
+  p = __builtin_fmaf(p, s, 0.020795971155166626f);
+  p = __builtin_fmaf(p, s, -0.053783830255270004f);
+  p = __builtin_fmaf(p, s, 0.13331924378871918f);
+  p = __builtin_fmaf(p, s, -0.33333298563957214f);
+  const float small = __builtin_fmaf(u, s * p, u);
+  const float r = __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(v * (2.f * 1.4426950409f)));
+  const float large = __builtin_copysignf(__builtin_fmaf(-2.f, r, 1.f), u);
+  return v < 0.6f ? small : large;
 }
 
 // tanh-approximated GELU and its derivative (reference rust/thundercube/src/unary_ops.rs:136-173)
 __device__ __forceinline__ void gelu_tanh_pair(float x, float& y, float& dy) {
   const float c = 0.7978845608f, a = 0.044715f;
-  const float t = tanhf(c * (x + a * x * x * x));
+  const float t = tanh_nobranch(c * (x + a * x * x * x));
   y = 0.5f * x * (1.f + t);
   dy = 0.5f * (1.f + t) + 0.5f * x * (1.f - t * t) * c * (1.f + 3.f * a * x * x);
 }

@@ -103,7 +103,7 @@ struct MlpBwdLds {
 // tanh-GELU with first and second derivative
 __device__ __forceinline__ void gelu_tanh_all(float x, float& y, float& dy, float& ddy) {
   const float c = 0.7978845608f, a = 0.044715f;
-  const float t = tanhf(c * (x + a * x * x * x));
+  const float t = tanh_nobranch(c * (x + a * x * x * x));
   const float du = c * (1.f + 3.f * a * x * x), ddu = 6.f * a * c * x, s = 1.f - t * t;
   y = 0.5f * x * (1.f + t);
   dy = 0.5f * (1.f + t) + 0.5f * x * s * du;

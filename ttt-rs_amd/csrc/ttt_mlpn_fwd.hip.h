@@ -9,11 +9,23 @@
 //   output chain    Xb[0] = XQ;  Zb[i] = Xb[i] W[i] - (eta (1 + tril(Xb[i] X[i]^T))) G[i] + b[i];  Xb[i+1] = gelu(Zb[i])
 //   out = XQ + LN(Zb[NL]);   W[i] -= (eta_last X[i])^T G[i];   b[i] -= colsum(eta_last G[i])
 //
-// One workgroup of 8 waves per (batch, head).  The state (up to 4 d x 4 d floats per hidden-to-hidden layer) lives in
-// the caller's output buffers, is read in place as a matrix operand and updated in place (an L2-resident working
-// set); the [16 x 4d] and [16 x d] tiles of a mini-batch, the biases and the 16 x 16 matrices are in LDS.  All
-// products are f32 matrix instructions for both I/O types.  LDS holds 2 NL + 2 hidden-wide tiles, which bounds the
-// shapes: head_dim 32 with up to four hidden layers, head_dim 64 with two.
+// One workgroup of 8 waves per (batch, head).  The weights stay in registers over the whole sequence, as accumulator
+// tiles of the f32 matrix instructions: register r of lane 16 g + c holds row 4 g + r, column c of a 16 x 16 tile, which
+// is at the same time a B operand over the rows (k step r takes row 4 g + r; the A operand is one 16-byte LDS read for
+// four k steps) and the accumulator of the rank-16 update.  A wave owns M / 8 hidden columns: the same columns of
+// W[0 .. NL-1] and the same rows of W[NL], so that elementwise work, gradients, biases and updates of a layer need no
+// exchange; products over k = M take the other waves' columns of X from LDS, products with W[NL] and the attention
+// blocks are summed over the waves.  G[i+1] W[i+1]^T contracts over the columns, the one product the layout does not
+// give: the tiles go through LDS (CH tile rows at a time) and are read back transposed.  (By 32 columns, written by two
+// waves while the others multiply the chunk before, half the barriers: 2138 us against 2087; the two writers hold up the
+// rest.)  At head_dim 64 all of it is 192 registers of a wave's 256; W[0], 32 of them, is therefore written to the output
+// buffer at the end of a mini-batch and read back for the next update.
+//
+// Bound by the f32 matrix instructions, 774 per wave and mini-batch at head_dim 64 with two hidden layers: two waves to
+// a SIMD, 32 cycles each, 20.6 of 32.2 us at 2.4 GHz; the rest are the barriers and the activations between the
+// products.  96 units of 64 mini-batches, bf16: 3128 us with the state read from the L2 for every product and update,
+// 2062 so.  All products are f32 for both I/O types.  LDS bounds the shapes: head_dim 32 with up to four hidden layers,
+// head_dim 64 with two.
 #pragma once
 #include "ttt_engine_fwd.hip.h"
 
@@ -40,52 +52,92 @@ struct MlpNFwdArgs {
 
 template <int D, int NL>
 struct MlpNLds {
-  static constexpr int M = 4 * D, LD = D + 4, LM = M + 4, LK = 17, KK = 16 * LK;
+  static constexpr int NW = 8, M = 4 * D, LD = D + 4, LM = M + 4;  // pitches: 4 mod 16 banks, 16-byte rows
   static constexpr int TD = 16 * LD, TM = 16 * LM;
-  // hidden-wide tiles: BA[i] (Z[i] -> gelu'(Z[i]) -> G[i]) and BB[i] (X[i+1]) per hidden layer, two for the output
-  // chain (Zb[i] -> Xb[i+1], used alternately)
-  static constexpr int BA = 0, BB = BA + NL * TM, BC = BB + NL * TM;
-  static constexpr int XQ = BC + 2 * TM, XK = XQ + TD, TG = XK + TD, ZL = TG + TD, ZBL = ZL + TD;
-  static constexpr int PART = ZBL + TD;  // eight [16 x 16] split-k partials of an attention block
-  static constexpr int AT = PART + 8 * 256, MX = AT + KK, ETA = MX + KK;
-  static constexpr int bh = ETA + KK;       // NL hidden biases
-  static constexpr int bl = bh + NL * M;    // bias of the last layer
+  static constexpr int NTD = D / 16, NTM = M / 16, NBM = NTM / NW;
+  static constexpr int CH = D == 32 ? NTM : 4;  // tile rows of W[i+1] in LDS at a time for G[i+1] W[i+1]^T
+  static constexpr int XI = 0;                  // X[1 .. NL]
+  static constexpr int GT = XI + NL * TM;       // G[i+1] as an operand
+  // one after the other: partials of Z[NL]; W[NL] transposed per wave; W[i+1] transposed and its partials; Xb[i] (two,
+  // in turn) beside the partials of Zb[NL]
+  static constexpr int POOL = GT + TM, PZ = POOL + 2 * TM;
+  static constexpr int S0 = CH * 16 * LM, S1 = NW * NBM * 16 * LD, S2 = 2 * TM + NW * NTD * 256, S3 = 4 * TM;
+  static constexpr int S01 = S0 > S1 ? S0 : S1, S23 = S2 > S3 ? S2 : S3, POOL_N = S01 > S23 ? S01 : S23;
+  static constexpr int XQ = POOL + POOL_N, XK = XQ + TD, TG = XK + TD, ZL = TG + TD, ZBL = ZL + TD;
+  static constexpr int PART = ZBL + TD;         // partials of an attention block, two blocks in turn
+  static constexpr int bl = PART + 2 * NW * 256;  // bias of the last layer
   static constexpr int gam = bl + D, bet = gam + D, lr = bet + D, te = lr + 16, END = te + 16;
   static constexpr size_t BYTES = sizeof(float) * END;
   static_assert(BYTES <= 160 * 1024, "exceeds the 160 KiB of LDS of a gfx950 CU");
 };
+
+// acc += A B over 16 k: k step r takes the four k with index 4 g + r
+__device__ __forceinline__ void mlpn_mma(f32x4& acc, f32x4 a, f32x4 b) {
+#pragma unroll
+  for (int r = 0; r < 4; ++r) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[r], b[r], acc, 0, 0, 0);
+}
+__device__ __forceinline__ f32x4 mlpn_ld4(const float* p) { return *reinterpret_cast<const f32x4*>(p); }
+__device__ __forceinline__ void mlpn_st4(float* p, f32x4 v) { *reinterpret_cast<f32x4*>(p) = v; }
+// rows 4 g .. 4 g + 3 of a column: the transposed operand of a rank-16 update, or its B operand
+__device__ __forceinline__ f32x4 mlpn_col4(const float* p, int ld) { return f32x4{p[0], p[ld], p[2 * ld], p[3 * ld]}; }
+// LDS written by a wave's lanes and read by other lanes of the same wave
+__device__ __forceinline__ void mlpn_wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
 
 template <class T, int D, int NL>
 __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) ttt_mlpn_fwd_kernel(MlpNFwdArgs a) {
   using IO = Io<T>;
   using elem = typename IO::elem;
   using L = MlpNLds<D, NL>;
-  constexpr int M = L::M, LD = L::LD, LM = L::LM, LK = L::LK, TM = L::TM;
-  constexpr int NW = 8, GW = 32, NJD = D / GW, NJM = M / GW, NTD = D / 16, NTM = M / 16;
-  constexpr int NBM = NTM / NW;  // hidden-side tile columns per job: one job per wave
-  constexpr int NBD = NTD % 3 == 0 ? 3 : (NTD % 2 == 0 ? 2 : 1);
-  static_assert(NTM % NW == 0, "hidden tiles must divide among the waves");
+  constexpr int M = L::M, LD = L::LD, LM = L::LM, TM = L::TM, NW = L::NW;
+  constexpr int GW = 32, NJD = D / GW, NTD = L::NTD, NTM = L::NTM, NBM = L::NBM;
+  constexpr int CH = L::CH, NCH = NTM / CH, SPLIT = NW / CH;
+  constexpr bool STREAM = D == 64;  // W[0] waits in the output buffer while the other products run
+  static_assert(NTM % NW == 0 && NTM % CH == 0 && NW % CH == 0 && (SPLIT > 1 || NBM == 1), "tiles must divide among the waves");
   extern __shared__ __attribute__((aligned(16))) float lds[];
   int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  int t = tid >> 5, cg = tid & 31;
+  int t = tid >> 5, cg = tid & 31, c = lane & 15, g = lane >> 4;
   const size_t bh = blockIdx.x;
   const int h = (int)(bh % a.H), K = a.K;
   float *sbl = lds + L::bl, *sgam = lds + L::gam, *sbet = lds + L::bet, *slr = lds + L::lr, *ste = lds + L::te;
   const size_t sbase = a.state_per_batch ? bh : (size_t)h;
-  auto in_dim = [](int i) { return i == 0 ? D : M; };
-  auto out_dim = [](int i) { return i == NL ? D : M; };
 
-  // ---- initial state -> live buffers
-  float* W[NL + 1];
+  // tile (row tile q, column tile n) of a row-major matrix of ld columns <-> registers.  q and n are known at compile
+  // time; the lane's own part of the address is the 32-bit offset o.
+  auto lane_off = [&](int ld, int row, int col) { return (unsigned)((row + 4 * g) * ld + col + c); };
+  auto load_tile = [&](const float* p, int ld, int q, int n, unsigned o) {
+    p += 16 * q * ld + 16 * n;
+    return f32x4{p[o], (p + ld)[o], (p + 2 * ld)[o], (p + 3 * ld)[o]};
+  };
+  auto store_tile = [&](float* p, int ld, int q, int n, unsigned o, f32x4 v) {
+    p += 16 * q * ld + 16 * n;
 #pragma unroll
-  for (int i = 0; i <= NL; ++i) {
-    const size_t n = (size_t)in_dim(i) * out_dim(i);
-    W[i] = a.W[i] + bh * n;
-    for (size_t e = tid; e < n; e += 512) W[i][e] = a.W0[i][sbase * n + e];
+    for (int r = 0; r < 4; ++r) (p + r * ld)[o] = v[r];
+  };
+
+  // ---- initial state
+  f32x4 w0[NTD][NBM], w[NL - 1][NTM][NBM], wl[NBM][NTD];  // W[0], W[1 .. NL-1]: own columns; W[NL]: own rows
+  float bias[NL][NBM];
+  const unsigned oc = lane_off(M, 0, 16 * NBM * wave), orow = lane_off(D, 16 * NBM * wave, 0);
+#pragma unroll
+  for (int j = 0; j < NBM; ++j) {
+#pragma unroll
+    for (int q = 0; q < NTD; ++q) {
+      w0[q][j] = load_tile(a.W0[0] + sbase * D * M, M, q, j, oc);
+      if (STREAM) store_tile(a.W[0] + bh * D * M, M, q, j, oc, w0[q][j]);
+    }
+#pragma unroll
+    for (int i = 1; i < NL; ++i)
+#pragma unroll
+      for (int q = 0; q < NTM; ++q) w[i - 1][q][j] = load_tile(a.W0[i] + sbase * M * M, M, q, j, oc);
+#pragma unroll
+    for (int q = 0; q < NTD; ++q) wl[j][q] = load_tile(a.W0[NL] + sbase * M * D, D, j, q, orow);
+#pragma unroll
+    for (int i = 0; i < NL; ++i) bias[i][j] = a.b0[i][sbase * M + 16 * (wave * NBM + j) + c];
   }
-#pragma unroll
-  for (int i = 0; i < NL; ++i)
-    for (int e = tid; e < M; e += 512) lds[L::bh + i * M + e] = a.b0[i][sbase * M + e];
   for (int e = tid; e < D; e += 512) {
     sbl[e] = a.b0[NL][sbase * D + e];
     sgam[e] = a.gamma[h * D + e];
@@ -95,147 +147,364 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))
   __syncthreads();
   const float te_last = ste[K - 1];
 
-  // the next mini-batch's xq/xk/xv/lr are fetched into registers while this one computes
-  float pq[NJD], pk[NJD], pv[NJD], plr = 0.f;
-  auto fetch = [&](int stage) {
-    const size_t r = (bh * (size_t)a.seq_stride + (size_t)stage * K + t) * D;
-    const bool ok = t < K;
+  // The next mini-batch's xq/xk/xv/lr are fetched into registers while the last W[i] is updated, wait where X[1] lay while
+  // W[0] is in registers, and go to their places when the mini-batch begins.  All by the thread that fetched them.
+  elem pq[NJD], pk[NJD], pv[NJD], plr;
+  auto fetch = [&](int stage) {  // rows K .. 15 are zero
+    int x = tid;  // opaque: the offsets are formed here and not kept from the loop's beginning
+    asm volatile("" : "+v"(x));
+    const size_t r0 = bh * (size_t)a.seq_stride + (size_t)stage * K;
+    const elem* xq = static_cast<const elem*>(a.xq) + r0 * D;
+    const elem* xk = static_cast<const elem*>(a.xk) + r0 * D;
+    const elem* xv = static_cast<const elem*>(a.xv) + r0 * D;
+    const elem* lr = static_cast<const elem*>(a.lr) + r0;
+    const unsigned o = ((x >> 5) < K ? x >> 5 : 0) * D + (x & 31);
 #pragma unroll
     for (int j = 0; j < NJD; ++j) {
-      const int o = cg + GW * j;
-      pq[j] = ok ? IO::load1(static_cast<const elem*>(a.xq) + r + o) : 0.f;
-      pk[j] = ok ? IO::load1(static_cast<const elem*>(a.xk) + r + o) : 0.f;
-      pv[j] = ok ? IO::load1(static_cast<const elem*>(a.xv) + r + o) : 0.f;
+      pq[j] = xq[o + GW * j];
+      pk[j] = xk[o + GW * j];
+      pv[j] = xv[o + GW * j];
     }
-    if (tid < 16)
-      plr = (tid < K) ? IO::load1(static_cast<const elem*>(a.lr) + bh * (size_t)a.seq_stride + (size_t)stage * K + tid) : 0.f;
+    plr = lr[(unsigned)((x & 15) < K ? x & 15 : 0)];
   };
+  auto stage_rows = [&]() {
+    float* S = lds + L::XI + t * LD + cg;
+#pragma unroll
+    for (int j = 0; j < NJD; ++j) {
+      const float k = IO::load1(pk + j);
+      S[GW * j] = t < K ? IO::load1(pq + j) : 0.f;
+      S[L::TD + GW * j] = t < K ? k : 0.f;
+      S[2 * L::TD + GW * j] = t < K ? IO::load1(pv + j) - k : 0.f;
+    }
+    if (tid < 16) lds[L::XI + 3 * L::TD + tid] = tid < K ? IO::load1(&plr) : 0.f;
+  };
+  static_assert(3 * L::TD + 16 <= TM, "the staged rows take the place of X[1]");
   fetch(0);
+  stage_rows();
 
   for (int st = 0; st < a.n_stages; ++st) {
-    // re-derived from an opaque copy every mini-batch, so that the address arithmetic of the tile products is
-    // recomputed here instead of being hoisted out of the scan into (spilled) registers
+    // re-derived from an opaque copy every mini-batch, so that address arithmetic is recomputed here instead of being
+    // hoisted out of the scan into (spilled) registers
     asm volatile("" : "+v"(tid));
-    lane = tid & 63, wave = tid >> 6, t = tid >> 5, cg = tid & 31;
-    const size_t row = bh * (size_t)a.seq_stride + (size_t)st * K + t;
+    lane = tid & 63, wave = tid >> 6, t = tid >> 5, cg = tid & 31, c = lane & 15, g = lane >> 4;
+    const int own = 16 * NBM * wave;               // first own hidden column
+    const int am = c * LM + 4 * g, ad = c * LD + 4 * g;  // A operand: row c, k = 4 g ..
+    const int um = 4 * g * LM + c, ud = 4 * g * LD + c;  // rows 4 g .., column c
 #pragma unroll
     for (int j = 0; j < NJD; ++j) {
-      const int o = cg + GW * j;
-      lds[L::XQ + t * LD + o] = pq[j];
-      lds[L::XK + t * LD + o] = pk[j];
-      lds[L::TG + t * LD + o] = pv[j] - pk[j];
+      const int o = t * LD + cg + GW * j;
+      lds[L::XQ + o] = lds[L::XI + o];
+      lds[L::XK + o] = lds[L::XI + L::TD + o];
+      lds[L::TG + o] = lds[L::XI + 2 * L::TD + o];
     }
-    if (tid < 16) slr[tid] = plr;
+    if (tid < 16) slr[tid] = lds[L::XI + 3 * L::TD + tid];
     __syncthreads();
-    if (st + 1 < a.n_stages) fetch(st + 1);
 
-    // ---- forward chain: Z[i] = X[i] W[i]; X[i+1] = gelu(Z[i] + b[i]), gelu' kept in place of Z[i]
+    // ---- forward chain: Z[i] = X[i] W[i]; X[i+1] = gelu(Z[i] + b[i]); gelu' stays in registers.  XQ W[0] rides along.
+    // Attention blocks are held transposed, element [s = 4 g + r][t = c]: as registers they are the A operand of MX G.
+    f32x4 G[NL][NBM], zq[NBM];  // G: gelu'(Z[i]), later G[i]
+    auto hidden = [&](int i, const f32x4 (&z)[NBM]) {
+      float* X = lds + L::XI + i * TM + own;
 #pragma unroll
-    for (int i = 0; i < NL; ++i) {
-      float* BAi = lds + L::BA + i * TM;
-      float* BBi = lds + L::BB + i * TM;
-      if (i == 0)
-        mm_lds<0, NW, NBM>(BAi, LM, lds + L::XK, LD, 1, W[0], M, 1, 1, NTM, D, wave, lane);
-      else
-        mm_lds<0, NW, NBM>(BAi, LM, lds + L::BB + (i - 1) * TM, LM, 1, W[i], M, 1, 1, NTM, M, wave, lane);
-      __syncthreads();
-      const float* sb = lds + L::bh + i * M;
+      for (int j = 0; j < NBM; ++j)
 #pragma unroll
-      for (int j = 0; j < NJM; ++j) {
-        const int o = cg + GW * j;
-        float y, dy;
-        gelu_tanh_pair(BAi[t * LM + o] + sb[o], y, dy);
-        BBi[t * LM + o] = y;
-        BAi[t * LM + o] = dy;
+        for (int r = 0; r < 4; ++r) {
+          float y, dy;
+          gelu_tanh_pair(z[j][r] + bias[i][j], y, dy);
+          X[um + r * LM + 16 * j] = y;
+          G[i][j][r] = dy;
+        }
+    };
+    // X W over k = M, the operand read one tile ahead (the compiler, short of registers, would wait for each read)
+    auto product = [&](f32x4 (&z)[NBM], const float* X, const f32x4 (&W)[NTM][NBM]) {
+      f32x4 fx = mlpn_ld4(X + am);
+#pragma unroll
+      for (int j = 0; j < NBM; ++j) z[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int q = 0; q < NTM; ++q) {
+        const f32x4 nx = mlpn_ld4(X + am + 16 * (q + 1 < NTM ? q + 1 : q));
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int j = 0; j < NBM; ++j) mlpn_mma(z[j], fx, W[q][j]);
+        __builtin_amdgcn_sched_barrier(0);
+        fx = nx;
       }
-      __syncthreads();
+    };
+    {
+      f32x4 z[NBM], at = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int j = 0; j < NBM; ++j) z[j] = zq[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int q = 0; q < NTD; ++q) {
+        const f32x4 fk = mlpn_ld4(lds + L::XK + ad + 16 * q);
+#pragma unroll
+        for (int j = 0; j < NBM; ++j) mlpn_mma(z[j], fk, w0[q][j]);
+      }
+      // the attention block XQ XK^T: the waves share its k steps
+#pragma unroll
+      for (int e = 0; e < D / 4 / NW; ++e) {
+        const int ks = wave * (D / 4 / NW) + e, o = ad + 16 * (ks >> 2) + (ks & 3);
+        at = __builtin_amdgcn_mfma_f32_16x16x4f32(lds[L::XK + o], lds[L::XQ + o], at, 0, 0, 0);
+      }
+      mlpn_st4(lds + L::PART + wave * 256 + 4 * lane, at);
+      __builtin_amdgcn_sched_barrier(0);
+      // XQ W[0] runs beside the activations: a product of four matrix instructions, then an activation
+      static_assert(NTD <= 4, "products to go with the activations");
+      float* X = lds + L::XI + own;
+#pragma unroll
+      for (int e = 0; e < 4 * NBM; ++e) {
+        if (e < NTD * NBM) mlpn_mma(zq[e % NBM], mlpn_ld4(lds + L::XQ + ad + 16 * (e / NBM)), w0[e / NBM][e % NBM]);
+        float y, dy;
+        gelu_tanh_pair(z[e >> 2][e & 3] + bias[0][e >> 2], y, dy);
+        X[um + (e & 3) * LM + 16 * (e >> 2)] = y;
+        G[0][e >> 2][e & 3] = dy;
+        __builtin_amdgcn_sched_barrier(0);
+      }
     }
+    __syncthreads();
+#pragma unroll
+    for (int i = 1; i < NL; ++i) {
+      f32x4 z[NBM];
+      product(z, lds + L::XI + (i - 1) * TM, w[i - 1]);
+      hidden(i, z);
+      if (i + 1 < NL) __syncthreads();
+    }
+    mlpn_wave_sync();
+    // X W[NL] over the wave's own rows
+    auto last_product = [&](const float* X) {
+      f32x4 z[NTD];
+#pragma unroll
+      for (int n = 0; n < NTD; ++n) z[n] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int j = 0; j < NBM; ++j) {
+        const f32x4 fx = mlpn_ld4(X + am + own + 16 * j);
+#pragma unroll
+        for (int n = 0; n < NTD; ++n) mlpn_mma(z[n], fx, wl[j][n]);
+      }
+#pragma unroll
+      for (int n = 0; n < NTD; ++n) mlpn_st4(lds + L::PZ + (wave * NTD + n) * 256 + 4 * lane, z[n]);
+    };
     // ---- Z[NL] = X[NL] W[NL]; G[NL] = LN-L2 gradient of Z[NL] + b[NL] against the target
-    mm_lds<0, NW>(lds + L::ZL, LD, lds + L::BB + (NL - 1) * TM, LM, 1, W[NL], D, 1, 1, NTD, M, wave, lane);
-    if (tid < 256) {
-      const int tt = tid >> 4, s = tid & 15;
-      lds[L::ETA + tt * LK + s] = (s <= tt) ? ste[tt] * slr[s] : 0.f;
-    }
+    last_product(lds + L::XI + (NL - 1) * TM);
     __syncthreads();
     {
-      float Gv[NJD];
+      float Gv[NJD], z[NJD][NW];
+#pragma unroll
+      for (int j = 0; j < NJD; ++j) {
+        const int o = cg + GW * j;
+        const float* p = lds + L::PZ + (o >> 4) * 256 + 4 * (16 * (t >> 2) + (o & 15)) + (t & 3);
+#pragma unroll
+        for (int v = 0; v < NW; ++v) z[j][v] = p[v * NTD * 256];
+      }
+      __builtin_amdgcn_sched_barrier(0);  // all reads first: the compiler would wait for each
+#pragma unroll
+      for (int j = 0; j < NJD; ++j) {
+#pragma unroll
+        for (int v = 1; v < NW; ++v) z[j][0] += z[j][v];
+        lds[L::ZL + t * LD + cg + GW * j] = z[j][0];
+      }
       ln_l2_grad<D, GW>(lds + L::ZL + t * LD, sbl, lds + L::TG + t * LD, sgam, sbet, cg, a.eps, Gv);
 #pragma unroll
       for (int j = 0; j < NJD; ++j) lds[L::ZL + t * LD + cg + GW * j] = Gv[j];
     }
     __syncthreads();
-    // ---- G[i] = (G[i+1] W[i+1]^T) * gelu'(Z[i]), from the last hidden layer down
+    // ---- G[NL-1] = (G[NL] W[NL]^T) * gelu'(Z[NL-1]): own rows, transposed in the wave's own part of the pool
+    {
+      float* S = lds + L::POOL + wave * NBM * 16 * LD;
 #pragma unroll
-    for (int i = NL - 1; i >= 0; --i) {
-      float* BAi = lds + L::BA + i * TM;
-      if (i == NL - 1)
-        mm_lds<3, NW, NBM, 2, true>(BAi, LM, lds + L::ZL, LD, 1, W[NL], 1, D, 1, NTM, D, wave, lane);
-      else
-        mm_lds<3, NW, NBM, 2, true>(BAi, LM, lds + L::BA + (i + 1) * TM, LM, 1, W[i + 1], 1, M, 1, NTM, M, wave, lane);
-      __syncthreads();
+      for (int j = 0; j < NBM; ++j)
+#pragma unroll
+        for (int n = 0; n < NTD; ++n)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) S[16 * j * LD + ud + r * LD + 16 * n] = wl[j][n][r];
+      mlpn_wave_sync();
+      f32x4 z[NBM];
+#pragma unroll
+      for (int j = 0; j < NBM; ++j) z[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int n = 0; n < NTD; ++n) {
+        const f32x4 fg = mlpn_ld4(lds + L::ZL + ad + 16 * n);
+#pragma unroll
+        for (int j = 0; j < NBM; ++j) mlpn_mma(z[j], fg, mlpn_ld4(S + 16 * j * LD + ad + 16 * n));
+      }
+#pragma unroll
+      for (int j = 0; j < NBM; ++j) {
+        G[NL - 1][j] *= z[j];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) lds[L::GT + um + r * LM + own + 16 * j] = G[NL - 1][j][r];
+      }
     }
-    // ---- output chain
+    __syncthreads();
+    // ---- G[i] = (G[i+1] W[i+1]^T) * gelu'(Z[i]): a wave takes one tile row of each chunk, SPLIT waves share its k
 #pragma unroll
-    for (int i = 0; i <= NL; ++i) {
-      float* zb = i == NL ? lds + L::ZBL : lds + L::BC + (i & 1) * TM;
-      const float* xb = i == 0 ? lds + L::XQ : lds + L::BC + ((i - 1) & 1) * TM;
-      const float* gi = i == NL ? lds + L::ZL : lds + L::BA + i * TM;
-      if (i == 0) {
-        // attention block and product over k = d
-        mm_lds<0, NW>(lds + L::AT, LK, lds + L::XQ, LD, 1, lds + L::XK, 1, LD, 1, 1, D, wave, lane);
-        mm_lds<0, NW, NBM>(zb, LM, xb, LD, 1, W[0], M, 1, 1, NTM, D, wave, lane);
-      } else {
-        // attention block Xb[i] X[i]^T over k = M, split over the waves
-        {
-          const int c = lane & 15, g = lane >> 4;
-          constexpr int KS = M / NW;
-          f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-          const float* Ap = xb + c * LM + wave * KS + g;
-          const float* Bp = lds + L::BB + (i - 1) * TM + c * LM + wave * KS + g;
-#pragma unroll 4
-          for (int k = 0; k < KS; k += 4) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(Ap[k], Bp[k], acc, 0, 0, 0);
+    for (int i = NL - 2; i >= 0; --i) {
+      f32x4 z[NCH];
 #pragma unroll
-          for (int r = 0; r < 4; ++r) lds[L::PART + wave * 256 + (4 * g + r) * 16 + c] = acc[r];
+      for (int ch = 0; ch < NCH; ++ch) {
+#pragma unroll
+        for (int q = 0; q < CH; ++q)
+#pragma unroll
+          for (int j = 0; j < NBM; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+              lds[L::POOL + 16 * q * LM + um + r * LM + own + 16 * j] = w[i][ch * CH + q][j][r];
+        __syncthreads();
+        const int k0 = (wave / CH) * (M / SPLIT);
+        const float* Gp = lds + L::GT + am + k0;
+        const float* Wp = lds + L::POOL + 16 * (wave % CH) * LM + am + k0;
+        f32x4 z0[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}}, fg = mlpn_ld4(Gp), fw = mlpn_ld4(Wp);
+#pragma unroll
+        for (int k = 0; k < M / SPLIT; k += 16) {  // reads one tile ahead, as above
+          const int kn = k + 16 < M / SPLIT ? k + 16 : k;
+          const f32x4 ng = mlpn_ld4(Gp + kn), nw = mlpn_ld4(Wp + kn);
+          __builtin_amdgcn_sched_barrier(0);
+          mlpn_mma(z0[(k >> 4) & 1], fg, fw);
+          __builtin_amdgcn_sched_barrier(0);
+          fg = ng;
+          fw = nw;
         }
-        if (i < NL)
-          mm_lds<0, NW, NBM>(zb, LM, xb, LM, 1, W[i], M, 1, 1, NTM, M, wave, lane);
-        else
-          mm_lds<0, NW>(zb, LD, xb, LM, 1, W[NL], D, 1, 1, NTD, M, wave, lane);
-      }
-      __syncthreads();
-      if (tid < 256) {
-        const int tt = tid >> 4, s = tid & 15;
-        float at;
-        if (i == 0) {
-          at = lds[L::AT + tt * LK + s];
-        } else {
-          at = 0.f;
-#pragma unroll
-          for (int w = 0; w < NW; ++w) at += lds[L::PART + w * 256 + tt * 16 + s];
-        }
-        lds[L::MX + tt * LK + s] = lds[L::ETA + tt * LK + s] * (1.f + at);
-      }
-      __syncthreads();
-      if (i < NL)
-        mm_lds<2, NW, NBM, 4>(zb, LM, lds + L::MX, LK, 1, gi, LM, 1, 1, NTM, 16, wave, lane);
-      else
-        mm_lds<2, NW, 1, 4>(zb, LD, lds + L::MX, LK, 1, gi, LD, 1, 1, NTD, 16, wave, lane);
-      __syncthreads();
-      if (i < NL) {
-        const float* sb = lds + L::bh + i * M;
-#pragma unroll
-        for (int j = 0; j < NJM; ++j) {
-          const int o = cg + GW * j;
-          float y, dy;
-          gelu_tanh_pair(zb[t * LM + o] + sb[o], y, dy);
-          zb[t * LM + o] = y;
-        }
+        z[ch] = z0[0] + z0[1];
         __syncthreads();
       }
+      if constexpr (SPLIT == 1) {
+        G[i][0] *= z[0];
+      } else {
+        // (G[1] waited in LDS: eight registers more for the products)
+#pragma unroll
+        for (int j = 0; j < NBM; ++j) G[NL - 1][j] = mlpn_col4(lds + L::GT + um + own + 16 * j, LM);
+        static_assert(SPLIT == 1 || (SPLIT == 2 && NL == 2), "the partials lie where the next layer's chunk would");
+#pragma unroll
+        for (int ch = 0; ch < NCH; ++ch)
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            lds[L::PZ + (wave / CH) * TM + um + r * LM + 16 * (ch * CH + wave % CH)] = z[ch][r];
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < NBM; ++j)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const float* p = lds + L::PZ + um + r * LM + own + 16 * j;
+            G[i][j][r] *= p[0] + p[TM];
+          }
+      }
+      if (i > 0) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+          for (int j = 0; j < NBM; ++j) lds[L::GT + um + r * LM + own + 16 * j] = G[i][j][r];
+      }
     }
-    // ---- out = XQ + LN(Zb[NL] + b[NL]); the gradients scaled by eta_last for the update
+    // ---- output chain; W[i] is updated right behind its last product of the mini-batch
+    auto last = [&]() { return te_last * mlpn_ld4(slr + 4 * g); };  // of rows 4 g ..
+    auto sum8 = [&](const float* p, int stride) {  // the waves' partials of a tile
+      f32x4 v[NW];
+#pragma unroll
+      for (int u = 0; u < NW; ++u) v[u] = mlpn_ld4(p + u * stride);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int u = 1; u < NW; ++u) v[0] += v[u];
+      return v[0];
+    };
+    auto attention = [&](int i) {  // -eta (1 + tril(Xb[i] X[i]^T)), transposed
+      const float* p = lds + L::PART + (i & 1) * NW * 256 + 4 * lane;
+      const f32x4 at = sum8(p, 256), l = mlpn_ld4(slr + 4 * g);
+      const float te = -ste[c];
+      f32x4 mx;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) mx[r] = 4 * g + r <= c ? te * l[r] * (1.f + at[r]) : 0.f;
+      return mx;
+    };
+    auto hidden_out = [&](int i, f32x4 (&z)[NBM]) {  // z -> Xb[i+1] and the own part of its attention block
+      const f32x4 mx = attention(i);
+      float* X = lds + L::POOL + (i & 1) * TM + own;
+#pragma unroll
+      for (int j = 0; j < NBM; ++j) {
+        mlpn_mma(z[j], mx, G[i][j]);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          float y, dy;
+          gelu_tanh_pair(z[j][r] + bias[i][j], y, dy);
+          X[um + r * LM + 16 * j] = y;
+        }
+      }
+      mlpn_wave_sync();
+      f32x4 p = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int j = 0; j < NBM; ++j)
+        mlpn_mma(p, mlpn_ld4(lds + L::XI + i * TM + am + own + 16 * j), mlpn_ld4(X + am + 16 * j));
+      mlpn_st4(lds + L::PART + ((i + 1) & 1) * NW * 256 + wave * 256 + 4 * lane, p);
+      // the update's gradient and the bias
+      const f32x4 lst = last();
+#pragma unroll
+      for (int j = 0; j < NBM; ++j) {
+        G[i][j] *= lst;
+        float s = (G[i][j][0] + G[i][j][1]) + (G[i][j][2] + G[i][j][3]);
+        s += __shfl_xor(s, 16);
+        s += __shfl_xor(s, 32);
+        bias[i][j] -= s;
+      }
+    };
+    hidden_out(0, zq);
+#pragma unroll
+    for (int i = 1; i < NL; ++i) {
+      __syncthreads();
+      f32x4 z[NBM];
+      product(z, lds + L::POOL + ((i - 1) & 1) * TM, w[i - 1]);
+      hidden_out(i, z);
+      if (i == NL - 1) fetch(st + 1 < a.n_stages ? st + 1 : st);  // no branch: the registers would be kept through it
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int q = 0; q < NTM; ++q) {
+        const f32x4 fx = -mlpn_col4(lds + L::XI + (i - 1) * TM + um + 16 * q, LM);
+#pragma unroll
+        for (int j = 0; j < NBM; ++j) mlpn_mma(w[i - 1][q][j], fx, G[i][j]);
+      }
+    }
+    last_product(lds + L::POOL + ((NL - 1) & 1) * TM);
+    __syncthreads();
+    stage_rows();
+    if (wave < NTD) {
+      f32x4 z = sum8(lds + L::PZ + wave * 256 + 4 * lane, NTD * 256);
+      mlpn_mma(z, attention(NL), mlpn_col4(lds + L::ZL + ud + 16 * wave, LD));
+#pragma unroll
+      for (int r = 0; r < 4; ++r) lds[L::ZBL + ud + r * LD + 16 * wave] = z[r];
+    }
+    if (STREAM) {
+#pragma unroll
+      for (int q = 0; q < NTD; ++q)
+#pragma unroll
+        for (int j = 0; j < NBM; ++j) w0[q][j] = load_tile(a.W[0] + bh * D * M, M, q, j, lane_off(M, 0, own));
+    }
+    __builtin_amdgcn_sched_barrier(0);
     {
-      const float last = te_last * slr[t];
+      const f32x4 lst = last();
+      f32x4 fx[NBM];
+#pragma unroll
+      for (int j = 0; j < NBM; ++j) fx[j] = -mlpn_col4(lds + L::XI + (NL - 1) * TM + um + own + 16 * j, LM);
+#pragma unroll
+      for (int n = 0; n < NTD; ++n) {
+        const f32x4 gl = mlpn_col4(lds + L::ZL + ud + 16 * n, LD) * lst;
+#pragma unroll
+        for (int j = 0; j < NBM; ++j) mlpn_mma(wl[j][n], fx[j], gl);
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < NTD; ++q) {
+      const f32x4 fx = -mlpn_col4(lds + L::XK + ud + 16 * q, LD);
+#pragma unroll
+      for (int j = 0; j < NBM; ++j) {
+        mlpn_mma(w0[q][j], fx, G[0][j]);
+        if (STREAM) store_tile(a.W[0] + bh * D * M, M, q, j, lane_off(M, 0, own), w0[q][j]);
+      }
+    }
+    float db = 0.f;
+    if (tid >= 512 - D)  // a wave that had no tile of Zb[NL]
+#pragma unroll
+      for (int r = 0; r < 16; ++r) db += lds[L::ZL + r * LD + tid - (512 - D)] * (te_last * slr[r]);
+    __syncthreads();
+    // ---- out = XQ + LN(Zb[NL] + b[NL])
+    {
+      const size_t row = bh * (size_t)a.seq_stride + (size_t)st * K + t;
       float xh[NJD], rstd;
       ln_stats<D, GW>(lds + L::ZBL + t * LD, sbl, cg, a.eps, xh, rstd);
 #pragma unroll
@@ -243,38 +512,35 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))
         const int o = cg + GW * j;
         if (t < K)
           IO::store1(static_cast<elem*>(a.out) + row * D + o, lds[L::XQ + t * LD + o] + (sgam[o] * xh[j] + sbet[o]));
-        lds[L::ZL + t * LD + o] *= last;
       }
-#pragma unroll
-      for (int i = 0; i < NL; ++i)
-#pragma unroll
-        for (int j = 0; j < NJM; ++j) lds[L::BA + i * TM + t * LM + cg + GW * j] *= last;
     }
     __syncthreads();
-    // ---- W[i] -= X[i]^T G[i]l ; b[i] -= colsum(G[i]l)
-    mm_rank<2, NW, NBM, 4>(W[0], M, lds + L::XK, 1, LD, lds + L::BA, LM, 1, NTD, NTM, wave, lane);
+    if (tid >= 512 - D) sbl[tid - (512 - D)] -= db;
+  }
+
+  // ---- final state
+  const unsigned oc1 = lane_off(M, 0, 16 * NBM * wave), orow1 = lane_off(D, 16 * NBM * wave, 0);
+#pragma unroll
+  for (int j = 0; j < NBM; ++j) {
+    const int n = wave * NBM + j;
+    if (!STREAM) {
+#pragma unroll
+      for (int q = 0; q < NTD; ++q) store_tile(a.W[0] + bh * D * M, M, q, j, oc1, w0[q][j]);
+    }
 #pragma unroll
     for (int i = 1; i < NL; ++i)
-      mm_rank<2, NW, NBM, 4>(W[i], M, lds + L::BB + (i - 1) * TM, 1, LM, lds + L::BA + i * TM, LM, 1, NTM, NTM, wave, lane);
-    mm_rank<2, NW, NBD, 4>(W[NL], D, lds + L::BB + (NL - 1) * TM, 1, LM, lds + L::ZL, LD, 1, NTM, NTD, wave, lane);
+#pragma unroll
+      for (int q = 0; q < NTM; ++q) store_tile(a.W[i] + bh * M * M, M, q, j, oc1, w[i - 1][q][j]);
+#pragma unroll
+    for (int q = 0; q < NTD; ++q) store_tile(a.W[NL] + bh * M * D, D, j, q, orow1, wl[j][q]);
 #pragma unroll
     for (int i = 0; i < NL; ++i)
-      for (int e = tid; e < M; e += 512) {
-        float s = 0.f;
-        for (int r = 0; r < 16; ++r) s += lds[L::BA + i * TM + r * LM + e];
-        lds[L::bh + i * M + e] -= s;
-      }
-    if (tid < D) {
-      float s = 0.f;
-      for (int r = 0; r < 16; ++r) s += lds[L::ZL + r * LD + tid];
-      sbl[tid] -= s;
-    }
-    __syncthreads();
+      if (g == 0) a.b[i][bh * M + 16 * n + c] = bias[i][j];
   }
-#pragma unroll
-  for (int i = 0; i < NL; ++i)
-    for (int e = tid; e < M; e += 512) a.b[i][bh * M + e] = lds[L::bh + i * M + e];
-  for (int e = tid; e < D; e += 512) a.b[NL][bh * D + e] = sbl[e];
+  __syncthreads();
+  if (tid < D) a.b[NL][bh * D + tid] = sbl[tid];
 }
+
+hipError_t launch_mlpn_fwd(bool f32, int head_dim, int n_hidden, const MlpNFwdArgs& a, hipStream_t s);  // ttt_mlpn_fwd.hip
 
 }  // namespace ttt
