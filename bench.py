@@ -523,14 +523,15 @@ def run_workload(name, a, pkg, torch):
         # backward runs no forward sweep of its own.
         flops = th * (224 * d * d)
         # bf16 I/O up to head_dim 96: every product of the scan takes bf16 operands (f32 accumulation, f32 state and
-        # gradient accumulators in memory); otherwise true-f32 products
+        # gradients in registers); otherwise true-f32 products
         bf = io == "bf16" and d <= 96
         peak = BF16_MFMA_PEAK_TF if bf else F32_MFMA_PEAK_TF
         out["dtype"] = "bf16" if bf else "f32"
         out["config"]["inner_model"] = "TTT-MLP"
         out["roofline"] = {"bound": "mfma", "achieved": flops / dev_s / 1e12, "peak": peak,
                            "unit": "TFLOP/s", "frac": flops / dev_s / 1e12 / peak, **counters,
-                           "kernel": "ttt_mlp_fwd_rr_kernel (forward, saving the update factors) + ttt_mlp_bwd_kernel (whole step)",
+                           "kernel": "ttt_mlp_fwd_rr_kernel (forward, saving the update factors) + " +
+                                     ("ttt_mlp_bwd_rp_kernel" if bf else "ttt_mlp_bwd_kernel") + " (whole step)",
                            "kernel_avg_us": dev_s * 1e6, "algorithmic_flops": flops}
     else:
         flops = th * (6 * (6 * d * d + 4 * K * d) + 2 * (56 * d * d + 20 * K * d))
