@@ -399,11 +399,8 @@ PyObject* linear_backward(PyObject* const* a) {
   const int64_t n = ttt_linear_num_checkpoints(&desc);
   const float* Wc = need_f32(a[9], {B, H, n, d, d}, "weight_ckpt", keep);
   const float* bc = need_f32(a[10], {B, H, n, d}, "bias_ckpt", keep);
-  const float *gW = nullptr, *gb = nullptr;
-  if (a[15] != Py_None) {
-    gW = need_f32(a[15], W4, "grad_weight_out", keep);
-    gb = need_f32(a[16], b3, "grad_bias_out", keep);
-  }
+  const float* gW = a[15] == Py_None ? nullptr : need_f32(a[15], W4, "grad_weight_out", keep);
+  const float* gb = a[16] == Py_None ? nullptr : need_f32(a[16], b3, "grad_bias_out", keep);
   at::Tensor dq = empty(rows, q.dtype, q.dev), dk = empty(rows, q.dtype, q.dev), dv = empty(rows, q.dtype, q.dev),
              dW = empty(W4, at::kFloat, q.dev), db = empty(b3, at::kFloat, q.dev), dl = empty(gates, q.dtype, q.dev),
              dt = empty({seq}, at::kFloat, q.dev), dg = empty(hd, at::kFloat, q.dev), de = empty(hd, at::kFloat, q.dev);
