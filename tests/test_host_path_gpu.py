@@ -34,3 +34,29 @@ def test_linear_backward_takes_each_state_gradient_alone(P, given, ci, dtype):
     got = P.ttt_linear_backward_raw(*a, Wc, bc, dO.to("cuda:0"), K, 1e-6, ci, **kw)
     torch.cuda.synchronize()
     compare(got, oracle_bwd(c, dO, K, sg), TOL[dtype])
+
+
+def layer_of(P, c, K):
+    v = to_dev(c)
+    H, d = v["W0"].shape[0], v["W0"].shape[1]
+    layer = P.FusedTileMulti(P.ModelConfig(H, d, P.TTTConfig(mini_batch_size=K)), v["W0"], v["b0"], v["gamma"], v["beta"])
+    return layer, P.TTTInputsInner(P.Qkv(v["xq"], v["xk"], v["xv"]), v["token_eta"], v["lr"])
+
+
+@pytest.mark.parametrize("seq", [48, 39, 7])
+def test_layer_takes_a_state_shared_over_the_batch(P, seq):
+    """The layer's own parameters ([H,d,d], [H,d]) as a state give what their repetition over the batch gives: whole
+    mini-batches, a remainder behind them, a remainder alone."""
+    print(f"case layer, shared state, {seq} tokens", flush=True)
+    B, H, d, K = 3, 2, 64, 16
+    c = P.synthetic.reference_test_inputs(77, B, H, 48, d, K, io_dtype=torch.float32)
+    for k in ("xq", "xk", "xv"):
+        c[k] = c[k][:, :, :seq].contiguous()
+    c["lr"] = c["lr"][:, :, :seq].contiguous()
+    c["token_eta"] = c["token_eta"].repeat(48)[:seq].contiguous()
+    layer, x = layer_of(P, c, K)
+    for call in (lambda s: layer.forward(s, x), lambda s: layer.forward_mini_batch(s, x, range(0, min(seq, K)))):
+        shared, full = P.TTTLinearState(layer.weight_init, layer.bias_init), layer.init_state(B)
+        o1, o2 = call(shared), call(full)
+        assert torch.equal(o1, o2) and torch.equal(shared.weight, full.weight) and torch.equal(shared.bias, full.bias)
+        assert shared.weight.shape == (B, H, d, d)

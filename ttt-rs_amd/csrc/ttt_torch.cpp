@@ -255,7 +255,8 @@ PyObject* linear_forward(PyObject* const* a) {
 
 // A layer's pass over the tokens start .. stop of its inputs: whole mini-batches in one launch, a remainder as one
 // short mini-batch behind it.  (xq, xk, xv, weight, bias, token_eta [seq], lr, ln_weight, ln_bias, mini_batch, eps,
-// checkpoint_interval, start, stop) -> (out, weight, bias); the state is per batch element.
+// checkpoint_interval, start, stop) -> (out, weight, bias); the state goes in shared over the batch ([H,d,d], [H,d]) or per
+// batch element and comes out per batch element.
 PyObject* linear_layer_forward(PyObject* const* a) {
   Keep keep;
   const Rows q(a[0]);
@@ -279,8 +280,9 @@ PyObject* linear_layer_forward(PyObject* const* a) {
   const std::array<int64_t, 4> W4 = {B, H, d, d};
   const std::array<int64_t, 3> b3 = {B, H, d};
   const std::array<int64_t, 2> hd = {H, d};
-  const float* W0 = need_f32(a[3], W4, "weight", keep);
-  const float* b0 = need_f32(a[4], b3, "bias", keep);
+  const bool per_batch = tensor(a[3], "weight").dim() == 4;
+  const float* W0 = need_f32(a[3], per_batch ? Shape(W4) : Shape(W4).slice(1), "weight", keep);
+  const float* b0 = need_f32(a[4], per_batch ? Shape(b3) : Shape(b3).slice(1), "bias", keep);
   const float* gam = need_f32(a[7], hd, "ln_weight", keep);
   const float* bet = need_f32(a[8], hd, "ln_bias", keep);
   const float* te = eta_of(a[5], stop, keep) + start;
@@ -291,8 +293,8 @@ PyObject* linear_layer_forward(PyObject* const* a) {
   // both launches' descs before anything is allocated or enqueued
   ttt_desc desc[2];
   int calls = 0;
-  if (full > 0) desc[calls++] = desc_of(B, H, full, d, K, eps, ci, io, true, rest > 0 ? n : 0, 0, 0);
-  if (rest > 0) desc[calls++] = desc_of(B, H, rest, d, rest, eps, ci, io, true, full > 0 ? n : 0, 0, 0);
+  if (full > 0) desc[calls++] = desc_of(B, H, full, d, K, eps, ci, io, per_batch, rest > 0 ? n : 0, 0, 0);
+  if (rest > 0) desc[calls++] = desc_of(B, H, rest, d, rest, eps, ci, io, per_batch || full > 0, full > 0 ? n : 0, 0, 0);
   for (int i = 0; i < calls; ++i) check(ttt_linear_supported(&desc[i]));
   at::Tensor out = empty(rows, q.dtype, q.dev), W[2], b[2];
   for (int i = 0; i < calls; ++i) {
