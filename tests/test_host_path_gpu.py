@@ -60,3 +60,23 @@ def test_layer_takes_a_state_shared_over_the_batch(P, seq):
         o1, o2 = call(shared), call(full)
         assert torch.equal(o1, o2) and torch.equal(shared.weight, full.weight) and torch.equal(shared.bias, full.bias)
         assert shared.weight.shape == (B, H, d, d)
+
+
+def test_layer_needs_token_eta_of_a_mini_batch_only(P):
+    """Whole mini-batches read the first K entries; a remainder reads those at its own tokens, and is refused without."""
+    print("case layer, token_eta of K entries", flush=True)
+    B, H, d, K = 2, 2, 64, 16
+    c = P.synthetic.reference_test_inputs(78, B, H, 48, d, K, io_dtype=torch.float32)
+    te = c["token_eta"][:K].contiguous()
+    c["token_eta"] = te.repeat(3)
+    layer, x = layer_of(P, c, K)
+    short = P.TTTInputsInner(x.qkv, te.to("cuda:0"), x.ttt_lr_eta)
+    s1, s2 = layer.init_state(B), layer.init_state(B)
+    assert torch.equal(layer.forward(s1, short), layer.forward(s2, x)) and torch.equal(s1.weight, s2.weight)
+    s1, s2 = layer.init_state(B), layer.init_state(B)
+    r = range(0, K)
+    assert torch.equal(layer.forward_mini_batch(s1, short, r), layer.forward_mini_batch(s2, x, r))
+    cut = lambda t: t[:, :, :39].contiguous()
+    short = P.TTTInputsInner(P.Qkv(cut(x.qkv.xq), cut(x.qkv.xk), cut(x.qkv.xv)), te.to("cuda:0"), cut(x.ttt_lr_eta))
+    with pytest.raises(P.TttError, match="token_eta"):
+        layer.forward(layer.init_state(B), short)

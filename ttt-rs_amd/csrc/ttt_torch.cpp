@@ -254,8 +254,9 @@ PyObject* linear_forward(PyObject* const* a) {
 }
 
 // A layer's pass over the tokens start .. stop of its inputs: whole mini-batches in one launch, a remainder as one
-// short mini-batch behind it.  (xq, xk, xv, weight, bias, token_eta [seq], lr, ln_weight, ln_bias, mini_batch, eps,
-// checkpoint_interval, start, stop) -> (out, weight, bias); the state goes in shared over the batch ([H,d,d], [H,d]) or per
+// short mini-batch behind it.  (xq, xk, xv, weight, bias, token_eta, lr, ln_weight, ln_bias, mini_batch, eps,
+// checkpoint_interval, start, stop) -> (out, weight, bias); of token_eta the first K entries from start on are read, and
+// those of a remainder; the state goes in shared over the batch ([H,d,d], [H,d]) or per
 // batch element and comes out per batch element.
 PyObject* linear_layer_forward(PyObject* const* a) {
   Keep keep;
@@ -285,9 +286,10 @@ PyObject* linear_layer_forward(PyObject* const* a) {
   const float* b0 = need_f32(a[4], per_batch ? Shape(b3) : Shape(b3).slice(1), "bias", keep);
   const float* gam = need_f32(a[7], hd, "ln_weight", keep);
   const float* bet = need_f32(a[8], hd, "ln_bias", keep);
-  const float* te = eta_of(a[5], stop, keep) + start;
   const int io = io_of(q.t);
   const int64_t size = io == TTT_F32 ? 4 : 2, full = n / K * K, rest = n - full;
+  // a launch reads as many entries as a mini-batch of it has tokens
+  const float* te = eta_of(a[5], rest > 0 ? stop : start + K, keep) + start;
   const float eps = real(a[10]);
   const int64_t ci = integer(a[11]);
   // both launches' descs before anything is allocated or enqueued
