@@ -80,3 +80,16 @@ def test_layer_needs_token_eta_of_a_mini_batch_only(P):
     short = P.TTTInputsInner(P.Qkv(cut(x.qkv.xq), cut(x.qkv.xk), cut(x.qkv.xv)), te.to("cuda:0"), cut(x.ttt_lr_eta))
     with pytest.raises(P.TttError, match="token_eta"):
         layer.forward(layer.init_state(B), short)
+
+
+def test_layer_takes_a_sequence_without_tokens(P):
+    print("case layer, empty sequence", flush=True)
+    c = P.synthetic.reference_test_inputs(79, 2, 2, 16, 64, 16, io_dtype=torch.bfloat16)
+    layer, x = layer_of(P, c, 16)
+    cut = lambda t: t[:, :, :0]
+    state = layer.init_state(2)
+    W, b = state.weight, state.bias
+    out = layer.forward(state, P.TTTInputsInner(P.Qkv(cut(x.qkv.xq), cut(x.qkv.xk), cut(x.qkv.xv)), x.token_eta[:0],
+                                                cut(x.ttt_lr_eta)))
+    assert out.shape == (2, 2, 0, 64) and out.dtype == torch.bfloat16
+    assert state.weight is W and state.bias is b

@@ -302,8 +302,9 @@ class FusedTileMulti:
     def forward(self, state: TTTLinearState, inputs: TTTInputsInner) -> torch.Tensor:
         """wrapper.rs:102-164: all full mini-batches in one launch; a trailing remainder is one
         short mini-batch, as the Burn-op model does it (inner.rs:40-47).  Both launches read and write
-        windows of the sequence in place."""
-        return self._pass(state, inputs, 0, inputs.qkv.xq.shape[2])
+        windows of the sequence in place.  A sequence without tokens leaves the state as it is."""
+        seq = inputs.qkv.xq.shape[2]
+        return self._pass(state, inputs, 0, seq) if seq > 0 else torch.empty_like(inputs.qkv.xq)
 
     def forward_mini_batch(self, state: TTTLinearState, inputs: TTTInputsInner, r: range) -> torch.Tensor:
         """wrapper.rs:166-211: one mini-batch (len(r) <= mini_batch_size)."""
