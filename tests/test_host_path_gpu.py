@@ -93,3 +93,11 @@ def test_layer_takes_a_sequence_without_tokens(P):
                                                 cut(x.ttt_lr_eta)))
     assert out.shape == (2, 2, 0, 64) and out.dtype == torch.bfloat16
     assert state.weight is W and state.bias is b
+
+
+def test_layer_refuses_a_mini_batch_without_tokens(P):
+    print("case layer, mini_batch 0", flush=True)
+    c = P.synthetic.reference_test_inputs(80, 1, 1, 16, 32, 16, io_dtype=torch.float32)
+    layer, x = layer_of(P, c, 0)
+    with pytest.raises(P.TttError, match="mini_batch 0"):
+        layer.forward(layer.init_state(1), x)

@@ -265,6 +265,7 @@ PyObject* linear_layer_forward(PyObject* const* a) {
   const int64_t n = stop - start;
   if (start < 0 || n <= 0 || stop > q.seq)
     fail(TTT_ERR_SHAPE, "tokens %lld .. %lld of a sequence of %lld", (long long)start, (long long)stop, (long long)q.seq);
+  if (K < 1) fail(TTT_ERR_SHAPE, "mini_batch %lld", (long long)K);
   const std::array<int64_t, 4> whole = q.shape(), rows = {B, H, n, d};
   const std::array<int64_t, 3> gates = {B, H, q.seq};
   const at::Tensor &xk = tensor(a[1], "xk"), &xv = tensor(a[2], "xv"), &lr = tensor(a[6], "ttt_lr_eta");
