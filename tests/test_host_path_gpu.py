@@ -101,3 +101,30 @@ def test_layer_refuses_a_mini_batch_without_tokens(P):
     layer, x = layer_of(P, c, 0)
     with pytest.raises(P.TttError, match="mini_batch 0"):
         layer.forward(layer.init_state(1), x)
+
+
+def off_by_one(t):
+    """The same contiguous tensor on the device, one element behind a 16-byte boundary."""
+    return torch.empty(t.numel() + 1, dtype=t.dtype, device="cuda:0")[1:].view(t.shape).copy_(t)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["f32", "bf16"])
+def test_sparse_linear_backward_takes_unaligned_tensors(P, dtype):
+    """Coarser checkpoints than one per mini-batch: the kernel without a workspace reads element by element, so the call
+    that is given one takes the same tensors (and workspaces)."""
+    print(f"case sparse linear bwd, unaligned {dtype}", flush=True)
+    B, H, d, K, N, ci = 2, 2, 64, 16, 5, 2
+    c = P.synthetic.reference_test_inputs(81, B, H, N * K, d, K, io_dtype=dtype)
+    dO = torch.randn(B, H, N * K, d, generator=torch.Generator().manual_seed(13)).to(dtype)
+    v = to_dev(c)
+    a = [v["xq"], v["xk"], v["xv"], v["W0"], v["b0"], v["token_eta"], v["lr"], v["gamma"], v["beta"]]
+    Wc, bc = P.ttt_linear_forward_raw(*a, K, 1e-6, ci, want_checkpoints=True)[3:]
+    ref = oracle_bwd(c, dO, K)
+    got = P.ttt_linear_backward_raw(*[off_by_one(t) for t in a[:3]], *a[3:], Wc, bc, off_by_one(dO), K, 1e-6, ci)
+    torch.cuda.synchronize()
+    compare(got, ref, TOL[dtype])
+    # a desc that needs no workspace ignores the one it is given
+    ws = torch.empty(65, dtype=torch.uint8, device="cuda:0")[1:]
+    got = P.ttt_linear_backward_raw(*a, Wc, bc, dO.to("cuda:0"), K, 1e-6, ci, kernel_hint=P.TTT_HINT_LDS_TILES, workspace=ws)
+    torch.cuda.synchronize()
+    compare(got, ref, TOL[dtype])

@@ -1349,10 +1349,14 @@ int linear_bwd_impl(const ttt_desc* d, const void* xq, const void* xk, const voi
   LinearBwdChoice ch;
   int rc = choose_linear_bwd(d, &ch);
   if (rc != TTT_OK) return rc;
+  // every kernel but the LDS-tile one reads and writes rows 16 bytes at a time; sparse checkpoints fall back to that one
+  const bool aligned = aligned16(xq) && aligned16(xk) && aligned16(xv) && aligned16(d_out) && aligned16(d_xq) &&
+                       aligned16(d_xk) && aligned16(d_xv) && aligned16(W_ckpt) && aligned16(b_ckpt) &&
+                       ((size_t)(d->seq_stride > 0 ? d->seq_stride : d->seq) * d->head_dim) % 8 == 0;
   LinStatesPlan sparse;
-  const bool states = workspace != nullptr && plan_linear_states(d, &sparse);
+  const bool states = workspace != nullptr && aligned && aligned16(d_b_out) && aligned16(d_b0) && plan_linear_states(d, &sparse);
   bool pair = workspace != nullptr && (states ? sparse.pair : linear_bwd_pair_wanted(d));
-  if (workspace != nullptr && !aligned16(workspace))
+  if ((pair || states) && !aligned16(workspace))
     return fail(TTT_ERR_SHAPE, "ttt_linear_bwd_ws: workspace must be 16-byte aligned");
   if (pair) {
     int cus = 0;
@@ -1382,10 +1386,7 @@ int linear_bwd_impl(const ttt_desc* d, const void* xq, const void* xk, const voi
   a.ckpt_packed = ckpt_format_of(d) == TTT_CKPT_PACKED ? 1 : ckpt_format_of(d) == TTT_CKPT_FACTORS ? ttt::kCkptFactors : 0;
   a.eps = d->eps;
   const int D = d->head_dim;
-  if ((states || ch.kind != LinearBwdChoice::LDS) &&
-      (!aligned16(xq) || !aligned16(xk) || !aligned16(xv) || !aligned16(d_out) || !aligned16(d_xq) ||
-       !aligned16(d_xk) || !aligned16(d_xv) || !aligned16(W_ckpt) || !aligned16(b_ckpt) ||
-       ((size_t)a.seq_stride * D) % 8 != 0))
+  if (ch.kind != LinearBwdChoice::LDS && !aligned)
     return fail(TTT_ERR_SHAPE, "ttt_linear_bwd: tensors must be 16-byte aligned");
   if ((ch.w_global || ch.dw_global) && (!aligned16(W_ckpt) || !aligned16(d_W0)))
     return fail(TTT_ERR_SHAPE, "ttt_linear_bwd: W_ckpt and d_W0 must be 16-byte aligned");
