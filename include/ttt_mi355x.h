@@ -314,7 +314,9 @@ int ttt_mlp_bwd(const ttt_desc* desc, const void* xq, const void* xk, const void
  * caller-owned) the two rank-16 factors of every mini-batch's state update and a copy of the final state, about
  * 2 K (5 d) floats per mini-batch and unit instead of the activations.  ttt_mlp_bwd_saved takes the arguments of
  * ttt_mlp_bwd with `saved` in place of the workspace, the same desc and the same inputs as the forward; it consumes
- * `saved` (the state in it is walked back), so a second backward needs a second forward or ttt_mlp_bwd.
+ * `saved` (the state in it is walked back), so a second backward needs a second forward or ttt_mlp_bwd.  The two calls'
+ * kernel_hint may differ as far as both descs need the same workspace: `saved` says in which form the forward left
+ * the factors, and a backward that takes them in another one runs the forward sweep as ttt_mlp_bwd does.
  * Exists where the forward's kernel is also the backward's sweep: bf16 I/O up to head_dim 96 (one CU per unit) and
  * f32 I/O; ttt_mlp_fwd_saving_supported says so beforehand (TTT_ERR_UNSUPPORTED for the forward on pairs of CUs:
  * head_dim 128 with bf16 I/O, TTT_HINT_TWO_CU).

@@ -5,8 +5,9 @@ import importlib
 import pytest
 import torch
 
-from helpers import TOL, assert_close
+from helpers import TOL, assert_close, to_dev
 from test_mlp_bwd_gpu import GRADS, run_case
+from test_mlp_fwd_gpu import mlp_case
 
 pytestmark = pytest.mark.gpu
 
@@ -29,3 +30,29 @@ def test_register_resident_backward(P, B, H, d, K, N, sg):
             assert_close(one[k], got[k].double(), 1e-5, k)
         else:
             assert torch.equal(one[k], got[k]), f"{k}: one workgroup per unit differs from two"
+
+
+def saving_pair(P, v, d_out, K, fwd_hint, bwd_hint):
+    a = (v["xq"], v["xk"], v["xv"], v["W1"], v["b1"], v["W2"], v["b2"], v["token_eta"], v["lr"], v["gamma"], v["beta"])
+    saved = P.ttt_mlp_forward_raw(*a, K, kernel_hint=fwd_hint, save_for_backward=True)[5]
+    return (P.ttt_mlp_backward_raw(*a, d_out, K, kernel_hint=bwd_hint, saved=saved),
+            P.ttt_mlp_backward_raw(*a, d_out, K, kernel_hint=bwd_hint))
+
+
+@pytest.mark.parametrize("d", [32, 96])
+@pytest.mark.parametrize("fwd,bwd", [(f, b) for f in ("", "F32_PRODUCTS", "LDS_TILES") for b in ("", "F32_PRODUCTS", "LDS_TILES")])
+def test_saved_buffer_says_which_form_it_has(P, fwd, bwd, d):
+    """Whatever hint the saving forward had, the backward's results are those of the call that saves nothing: the forms
+    of the saved factors differ between the kernels that the hints choose."""
+    print(f"case mlp saving pair, forward hint {fwd or 'none'}, backward hint {bwd or 'none'}, d{d}", flush=True)
+    K, N = 16, 5
+    c = mlp_case(P, 555 + d, 1, 2, N * K, d, K, torch.bfloat16, "baseline")
+    d_out = torch.randn(1, 2, N * K, d, generator=torch.Generator().manual_seed(8)).to(torch.bfloat16).to("cuda:0")
+    hint = lambda name: getattr(P, "TTT_HINT_" + name) if name else 0
+    got, ref = saving_pair(P, to_dev(c), d_out, K, hint(fwd), hint(bwd))
+    torch.cuda.synchronize()
+    for k in GRADS:
+        if k in ("d_token_eta", "d_gamma", "d_beta"):  # atomic additions: their order is not fixed
+            assert_close(got[k], ref[k].double(), 1e-5, k)
+        else:
+            assert torch.equal(got[k], ref[k]), k

@@ -661,6 +661,19 @@ struct MlpRpWs {
   }
 };
 
+// What ttt_mlp_fwd_saving leaves behind differs where a desc's hint chooses between kernels: fragments for the
+// register-resident scan, f32 matrices for the other, those with bf16 operands behind them or with f32 products.  Which of
+// them it is stands in the word at the start of the scratch tiles: behind everything that is saved in any form, at an
+// offset that no hint moves.  A backward that finds another form than its own sweep's runs that sweep.
+enum MlpSavedForm : unsigned { kMlpSavedFragments = 0x7fa5f4a6u, kMlpSavedMatrices = 0x7fa5a371u, kMlpSavedF32Matrices = 0x7fa5a372u };
+bool mlp_saved_has_forms(const ttt_desc* d) { return d->io_dtype != TTT_F32 && d->head_dim <= 96; }
+MlpSavedForm mlp_saved_form(const ttt_desc* d) {
+  return mlp_rp(d) ? kMlpSavedFragments : mlp_rr_sweep(d) ? kMlpSavedMatrices : kMlpSavedF32Matrices;
+}
+unsigned* mlp_saved_word(const ttt_desc* d, void* saved) {
+  return reinterpret_cast<unsigned*>(static_cast<float*>(saved) + MlpBwdWs(d).mt);
+}
+
 // address of the status word on the current device
 std::atomic<void*> g_lost_word[kMaxDevices];
 int lost_word(unsigned** out) {
@@ -713,14 +726,15 @@ int run_mlp_bwd_rp(const ttt_desc* d, ttt::MlpBwdRpArgs& a, const MlpRpWs& w, vo
   return TTT_OK;
 }
 
-// sweep = false: the workspace already holds what the sweep leaves there (ttt_mlp_fwd_saving wrote it)
+// saved: the workspace already holds what the sweep leaves there (ttt_mlp_fwd_saving wrote it), in the form that its word
+// names
 int mlp_bwd_impl(const ttt_desc* d, const void* xq, const void* xk, const void* xv,
                 const float* W1_0, const float* b1_0, const float* W2_0, const float* b2_0,
                 const float* token_eta, const void* lr, const float* gamma, const float* beta,
                 const void* d_out, const float* d_W1_out, const float* d_b1_out,
                 const float* d_W2_out, const float* d_b2_out, void* d_xq, void* d_xk, void* d_xv,
                 float* d_W1, float* d_b1, float* d_W2, float* d_b2, void* d_lr, float* d_token_eta,
-                float* d_gamma, float* d_beta, void* workspace, void* stream, bool sweep = true) {
+                float* d_gamma, float* d_beta, void* workspace, void* stream, bool saved = false) {
   int rc = ttt_mlp_supported(d);
   if (rc != TTT_OK) return rc;
   if (!xq || !xk || !xv || !W1_0 || !b1_0 || !W2_0 || !b2_0 || !token_eta || !lr || !gamma || !beta ||
@@ -762,7 +776,12 @@ int mlp_bwd_impl(const ttt_desc* d, const void* xq, const void* xk, const void* 
     fa.b1_save = reinterpret_cast<float*>(wb + rw.b1);
     fa.b2_save = reinterpret_cast<float*>(wb + rw.b2);
   }
-  if (!sweep) {
+  if (saved && mlp_saved_has_forms(d)) {
+    fa.layout_word = mlp_saved_word(d, workspace);
+    fa.layout = mlp_saved_form(d);
+    fa.if_other = 1;
+  }
+  if (saved && !mlp_saved_has_forms(d)) {
     rc = TTT_OK;
   } else if (rr_sweep) {
     fa.out = d_xq;
@@ -1601,6 +1620,10 @@ int ttt_mlp_fwd_saving(const ttt_desc* d, const void* xq, const void* xk, const 
                        b2_out, &a);
   if (rc != TTT_OK) return rc;
   hipStream_t s = static_cast<hipStream_t>(stream);
+  if (mlp_saved_has_forms(d)) {
+    a.layout_word = mlp_saved_word(d, saved);
+    a.layout = mlp_saved_form(d);
+  }
   if (mlp_rp(d)) {
     const MlpRpWs w(d);
     unsigned char* wb = static_cast<unsigned char*>(saved);
@@ -1636,7 +1659,7 @@ int ttt_mlp_bwd_saved(const ttt_desc* d, const void* xq, const void* xk, const v
   if (rc != TTT_OK) return rc;
   return mlp_bwd_impl(d, xq, xk, xv, W1_0, b1_0, W2_0, b2_0, token_eta, lr, gamma, beta, d_out, d_W1_out,
                       d_b1_out, d_W2_out, d_b2_out, d_xq, d_xk, d_xv, d_W1, d_b1, d_W2, d_b2, d_lr,
-                      d_token_eta, d_gamma, d_beta, saved, stream, /*sweep=*/false);
+                      d_token_eta, d_gamma, d_beta, saved, stream, /*saved=*/true);
 }
 
 int ttt_mlp_bwd_static(const ttt_desc* d, const void* xq, const void* xk, const void* xv,

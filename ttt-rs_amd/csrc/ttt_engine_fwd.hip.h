@@ -217,6 +217,11 @@ struct MlpFwdArgs {
   float* state_save = nullptr;
   float* b1_save = nullptr;
   float* b2_save = nullptr;
+  // with either: a word beside what is saved that names its form.  The forward writes `layout` there; a backward's own
+  // sweep (if_other) runs only if the word holds something else
+  unsigned* layout_word = nullptr;
+  unsigned layout = 0;
+  int if_other = 0;
   int B, H, seq, seq_stride, K, n_stages, state_per_batch;
   float eps;
   int unit_base;  // two-CU kernel only: first (batch, head) unit of this launch (the units are launched in batches)
@@ -224,6 +229,15 @@ struct MlpFwdArgs {
   int exchange_cleared;  // two-CU kernel only, read by the host: the exchange area (W2) has been zeroed by the caller
   int assume_other_xcd;  // two-CU kernel only: treat the partner as sitting on another XCD whatever it reports (testing)
 };
+
+// Whether a launch has nothing to do because what it would save is there (see MlpFwdArgs::layout_word), the same in every
+// lane; a launch that is to run whatever was there leaves its mark.
+__device__ __forceinline__ bool already_saved(const MlpFwdArgs& a) {
+  if (a.layout_word == nullptr) return false;
+  if (a.if_other) return __builtin_amdgcn_readfirstlane(*a.layout_word) == a.layout;
+  if (blockIdx.x == 0 && threadIdx.x == 0) *a.layout_word = a.layout;
+  return false;
+}
 
 template <int D>
 struct MlpLds {
@@ -252,6 +266,7 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))
   constexpr int NW = 8, GW = 32, NJD = D / GW, NJM = M / GW, NTD = D / 16, NTM = M / 16;
   constexpr int NBM = NTM / NW;  // hidden-side tile columns per job: one job per wave
   constexpr int NBD = NTD % 3 == 0 ? 3 : 2;
+  if (already_saved(a)) return;
   extern __shared__ __attribute__((aligned(16))) float lds[];
   // re-derived from an opaque copy at the top of every mini-batch, so that the address arithmetic of the
   // tile products is recomputed there instead of being hoisted out of the scan into (spilled) registers

@@ -117,6 +117,7 @@ __global__ void __launch_bounds__(512) ttt_mlp_fwd_rr_kernel(Problems<MlpFwdArgs
   using L = MlpRrLds<D, ES>;
   constexpr int NW = 8, NT = D / 16, F = 4 * D, HT = F / 16 / NW;
   constexpr float inv_d = 1.0f / D;
+  if (SAVE && already_saved(a)) return;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
 
   // the wave index is read through an SGPR so that everything keyed on it is scalar control flow
