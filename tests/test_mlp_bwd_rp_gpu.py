@@ -56,3 +56,35 @@ def test_saved_buffer_says_which_form_it_has(P, fwd, bwd, d):
             assert_close(got[k], ref[k].double(), 1e-5, k)
         else:
             assert torch.equal(got[k], ref[k]), k
+
+
+def off_by_one(t):
+    """The same contiguous tensor, one element behind a 16-byte boundary."""
+    return torch.empty(t.numel() + 1, dtype=t.dtype, device="cuda:0")[1:].view(t.shape).copy_(t)
+
+
+@pytest.mark.parametrize("save", [False, True])
+@pytest.mark.parametrize("which", ["xq", "d_out", "d_xk", "d_W2", "all"])
+def test_backward_takes_tensors_off_a_16_byte_boundary(P, which, save):
+    """The kernels that move rows 16 bytes at a time give way to those that read element by element: to the scan with f32
+    products, and where the rows of the forward are off to the sweep on LDS tiles as well."""
+    print(f"case mlp bwd, unaligned {which}, saved {save}", flush=True)
+    B, H, d, K, N = 1, 2, 64, 16, 4
+    c = mlp_case(P, 611, B, H, N * K, d, K, torch.bfloat16, "baseline")
+    d_out = torch.randn(B, H, N * K, d, generator=torch.Generator().manual_seed(8)).to(torch.bfloat16)
+    v = to_dev(c)
+    names = ("xq", "xk", "xv", "W1", "b1", "W2", "b2", "token_eta", "lr", "gamma", "beta")
+    a = [v[k] for k in names]
+    hint = P.TTT_HINT_LDS_TILES if which in ("xq", "all") else P.TTT_HINT_F32_PRODUCTS
+    ref = P.ttt_mlp_backward_raw(*a, d_out.to("cuda:0"), K, kernel_hint=hint)
+    saved = P.ttt_mlp_forward_raw(*a, K, save_for_backward=True)[5] if save else None
+    off = lambda k, t: off_by_one(t) if which in (k, "all") else t
+    into = {k: off(k, torch.full_like(t, float("nan"))) for k, t in ref.items()}
+    a = [off(k, t) if k in ("xq", "xk", "xv") else t for k, t in zip(names, a)]
+    got = P.ttt_mlp_backward_raw(*a, off("d_out", d_out.to("cuda:0")), K, into=into, saved=saved)
+    torch.cuda.synchronize()
+    for k in GRADS:
+        if k in ("d_token_eta", "d_gamma", "d_beta"):  # atomic additions: their order is not fixed
+            assert_close(got[k], ref[k].double(), 1e-5, k)
+        else:
+            assert torch.equal(got[k], ref[k]), k

@@ -755,7 +755,12 @@ int mlp_bwd_impl(const ttt_desc* d, const void* xq, const void* xk, const void* 
   // head_dim 96: the register-resident forward itself (the factors are then the ones the forward of this step
   // applied, rounded to bf16 as its matrix instructions took them); its output goes to d_xq, which the reverse
   // scan overwrites afterwards.  Otherwise the LDS-tile kernel (f32 products, no output).
-  const bool rr_sweep = mlp_rr_sweep(d);
+  // The register-resident kernels move rows, gradients and states 16 bytes at a time; the others read and write io tensors
+  // element by element, so a call with a tensor off a 16-byte boundary runs those.
+  const bool rows = aligned16(xq) && aligned16(xk) && aligned16(xv) && aligned16(d_xq);
+  const bool rr_sweep = mlp_rr_sweep(d) && rows;
+  const bool rp = mlp_rp(d) && rows && aligned16(d_out) && aligned16(d_xk) && aligned16(d_xv) && aligned16(d_W1) &&
+                  aligned16(d_W2) && aligned16(d_b2);
   ttt::MlpFwdArgs fa;
   fa.xq = xq; fa.xk = xk; fa.xv = xv; fa.W1_0 = W1_0; fa.b1_0 = b1_0; fa.W2_0 = W2_0; fa.b2_0 = b2_0;
   fa.token_eta = token_eta; fa.lr = lr; fa.gamma = gamma; fa.beta = beta; fa.out = nullptr;
@@ -766,7 +771,6 @@ int mlp_bwd_impl(const ttt_desc* d, const void* xq, const void* xk, const void* 
   fa.n_stages = d->seq / d->mini_batch;
   fa.state_per_batch = d->state_per_batch ? 1 : 0;
   fa.eps = d->eps;
-  const bool rp = mlp_rp(d);
   if (rp) {
     const MlpRpWs rw(d);
     unsigned char* wb = static_cast<unsigned char*>(workspace);
@@ -778,7 +782,7 @@ int mlp_bwd_impl(const ttt_desc* d, const void* xq, const void* xk, const void* 
   }
   if (saved && mlp_saved_has_forms(d)) {
     fa.layout_word = mlp_saved_word(d, workspace);
-    fa.layout = mlp_saved_form(d);
+    fa.layout = rp ? kMlpSavedFragments : rr_sweep ? kMlpSavedMatrices : kMlpSavedF32Matrices;
     fa.if_other = 1;
   }
   if (saved && !mlp_saved_has_forms(d)) {
