@@ -341,8 +341,9 @@ int ttt_mlp_bwd_saved(const ttt_desc* desc, const void* xq, const void* xk, cons
  * HIP graph capture, tight serving loops, harnesses that forbid hipMalloc).  Same arguments, results
  * and kernels as ttt_mlp_bwd; the workspace is a buffer of TTT_MLP_BWD_STATIC_MAX_BYTES that is part of
  * the library's device image (each GPU the library runs on holds it until the process ends).
- * A desc with ttt_mlp_bwd_workspace_bytes(desc) > TTT_MLP_BWD_STATIC_MAX_BYTES is refused with
- * TTT_ERR_SHAPE (use ttt_mlp_bwd then).  All calls on one GPU share that buffer: calls that overlap on
+ * A desc that needs more than that is refused with TTT_ERR_SHAPE (use ttt_mlp_bwd then); one whose
+ * ttt_mlp_bwd_workspace_bytes is above it but whose TTT_HINT_F32_PRODUCTS scan needs no more (a few mini-batches at
+ * head_dim 96 under TTT_HINT_ONE_WORKGROUP) runs that scan.  All calls on one GPU share that buffer: calls that overlap on
  * one GPU (different streams or threads) race; calls on one stream, or otherwise ordered, are safe.
  * Nothing in the buffer has to survive between calls.
  */

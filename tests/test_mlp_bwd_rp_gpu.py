@@ -1,5 +1,6 @@
 """GPU parity of the register-resident TTT-MLP backward (bf16 I/O, head_dim 32 / 64 / 96) where its own structure can go
 wrong: sequences longer than its hand-over slots, on two workgroups per unit (a ring) and on one (a launch per slots)."""
+import ctypes
 import importlib
 
 import pytest
@@ -82,6 +83,27 @@ def test_backward_takes_tensors_off_a_16_byte_boundary(P, which, save):
     into = {k: off(k, torch.full_like(t, float("nan"))) for k, t in ref.items()}
     a = [off(k, t) if k in ("xq", "xk", "xv") else t for k, t in zip(names, a)]
     got = P.ttt_mlp_backward_raw(*a, off("d_out", d_out.to("cuda:0")), K, into=into, saved=saved)
+    torch.cuda.synchronize()
+    for k in GRADS:
+        if k in ("d_token_eta", "d_gamma", "d_beta"):  # atomic additions: their order is not fixed
+            assert_close(got[k], ref[k].double(), 1e-5, k)
+        else:
+            assert torch.equal(got[k], ref[k]), k
+
+
+def test_static_scratch_takes_what_the_other_scan_fits(P):
+    """On one workgroup per unit the register-resident scan needs more scratch than the scan with f32 products for
+    sequences of a few mini-batches: a call whose scratch holds only the latter runs that."""
+    B, H, d, K, N = 1, 57, 96, 16, 1
+    print(f"case mlp bwd static B{B} H{H} d{d} N{N}", flush=True)
+    hint = P.TTT_HINT_ONE_WORKGROUP
+    desc = P.TttDesc(B, H, N * K, d, K, 1e-6, 1, P.TTT_BF16, 0, 0, 0, hint)
+    assert P.lib().ttt_mlp_bwd_workspace_bytes(ctypes.byref(desc)) > 32 << 20
+    v = to_dev(mlp_case(P, 613, B, H, N * K, d, K, torch.bfloat16, "baseline"))
+    a = [v[k] for k in ("xq", "xk", "xv", "W1", "b1", "W2", "b2", "token_eta", "lr", "gamma", "beta")]
+    d_out = torch.randn(B, H, N * K, d, generator=torch.Generator().manual_seed(8)).to(torch.bfloat16).to("cuda:0")
+    got = P.ttt_mlp_backward_raw(*a, d_out, K, kernel_hint=hint, static_scratch=True)
+    ref = P.ttt_mlp_backward_raw(*a, d_out, K, kernel_hint=hint | P.TTT_HINT_F32_PRODUCTS)
     torch.cuda.synchronize()
     for k in GRADS:
         if k in ("d_token_eta", "d_gamma", "d_beta"):  # atomic additions: their order is not fixed

@@ -727,14 +727,15 @@ int run_mlp_bwd_rp(const ttt_desc* d, ttt::MlpBwdRpArgs& a, const MlpRpWs& w, vo
 }
 
 // saved: the workspace already holds what the sweep leaves there (ttt_mlp_fwd_saving wrote it), in the form that its word
-// names
+// names.  room: bytes of the workspace (at least what MlpBwdWs asks for); the register-resident scan may need more.
 int mlp_bwd_impl(const ttt_desc* d, const void* xq, const void* xk, const void* xv,
                 const float* W1_0, const float* b1_0, const float* W2_0, const float* b2_0,
                 const float* token_eta, const void* lr, const float* gamma, const float* beta,
                 const void* d_out, const float* d_W1_out, const float* d_b1_out,
                 const float* d_W2_out, const float* d_b2_out, void* d_xq, void* d_xk, void* d_xv,
                 float* d_W1, float* d_b1, float* d_W2, float* d_b2, void* d_lr, float* d_token_eta,
-                float* d_gamma, float* d_beta, void* workspace, void* stream, bool saved = false) {
+                float* d_gamma, float* d_beta, void* workspace, void* stream, bool saved = false,
+                size_t room = SIZE_MAX) {
   int rc = ttt_mlp_supported(d);
   if (rc != TTT_OK) return rc;
   if (!xq || !xk || !xv || !W1_0 || !b1_0 || !W2_0 || !b2_0 || !token_eta || !lr || !gamma || !beta ||
@@ -760,7 +761,7 @@ int mlp_bwd_impl(const ttt_desc* d, const void* xq, const void* xk, const void* 
   const bool rows = aligned16(xq) && aligned16(xk) && aligned16(xv) && aligned16(d_xq);
   const bool rr_sweep = mlp_rr_sweep(d) && rows;
   const bool rp = mlp_rp(d) && rows && aligned16(d_out) && aligned16(d_xk) && aligned16(d_xv) && aligned16(d_W1) &&
-                  aligned16(d_W2) && aligned16(d_b2);
+                  aligned16(d_W2) && aligned16(d_b2) && MlpRpWs(d).total <= room;
   ttt::MlpFwdArgs fa;
   fa.xq = xq; fa.xk = xk; fa.xv = xv; fa.W1_0 = W1_0; fa.b1_0 = b1_0; fa.W2_0 = W2_0; fa.b2_0 = b2_0;
   fa.token_eta = token_eta; fa.lr = lr; fa.gamma = gamma; fa.beta = beta; fa.out = nullptr;
@@ -1675,8 +1676,8 @@ int ttt_mlp_bwd_static(const ttt_desc* d, const void* xq, const void* xk, const 
                        float* d_token_eta, float* d_gamma, float* d_beta, void* stream) {
   int rc = ttt_mlp_supported(d);
   if (rc != TTT_OK) return rc;
-  const int64_t need = ttt_mlp_bwd_workspace_bytes(d);
-  if (need < 0 || (uint64_t)need > kMlpBwdScratchBytes)
+  const int64_t need = (int64_t)(MlpBwdWs(d).total * sizeof(float));
+  if ((uint64_t)need > kMlpBwdScratchBytes)
     return fail(TTT_ERR_SHAPE,
                 "ttt_mlp_bwd_static: this shape needs %lld bytes of scratch, the built-in buffer holds %llu; "
                 "use ttt_mlp_bwd with a caller-owned workspace",
@@ -1686,7 +1687,7 @@ int ttt_mlp_bwd_static(const ttt_desc* d, const void* xq, const void* xk, const 
   if (rc != TTT_OK) return rc;
   return mlp_bwd_impl(d, xq, xk, xv, W1_0, b1_0, W2_0, b2_0, token_eta, lr, gamma, beta, d_out, d_W1_out,
                       d_b1_out, d_W2_out, d_b2_out, d_xq, d_xk, d_xv, d_W1, d_b1, d_W2, d_b2, d_lr,
-                      d_token_eta, d_gamma, d_beta, ws, stream);
+                      d_token_eta, d_gamma, d_beta, ws, stream, /*saved=*/false, kMlpBwdScratchBytes);
 }
 
 }  // extern "C"
