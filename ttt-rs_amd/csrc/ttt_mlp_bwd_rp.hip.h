@@ -45,8 +45,8 @@ struct MlpRp {
   // update factors of a mini-batch: [wave][hidden tile] fragments of G1'', then [feature tile] fragments of G2''
   static constexpr int FAC = (NW * HT + NT) * 512;
   // hand-over slot: per wave W2^T, W1^T images, hidden tiles; per feature tile LayerNorm tiles; small matrices, scalars
-  static constexpr int W2T = 0, W1T = W2T + HT * NQ * 1024, XT = W1T + HT * NQ * 1024, DT = XT + HT * 1024,
-                       DG = DT + HT * 1024, UG = DG + HT * 1024, WAVE = UG + HT * 1024;
+  static constexpr int W2T = 0, W1T = W2T + HT * NQ * 1024, XT = W1T + HT * NQ * 1024, DG = XT + HT * 1024,
+                       UG = DG + HT * 1024, G1 = UG + HT * 1024, DT = G1 + HT * 1024, WAVE = DT + HT * 512;
   static constexpr int XH = 0, GO = 1024, G2 = 2048, MZ = 3072, GG = 4096, ZD = 5120, TILE = ZD + 512;
   static constexpr int TILES = NW * WAVE, SMALL = TILES + NT * TILE;
   static constexpr int M1T = SMALL, A2T = M1T + 512, A1T = A2T + 512, SCAL = A1T + 512;  // SCAL: six rows of 16 floats
@@ -93,7 +93,7 @@ struct MlpRpLds {
   static constexpr int B2 = DB + NT * 1024;        // consumer: d b2 [d]
   static constexpr int BYTES = B2 + D * 4;
   static_assert(BYTES <= 160 * 1024, "exceeds the 160 KiB of LDS of a gfx950 CU");
-  static_assert(S::HT + (S::HT + 1) / 2 <= NT, "the wait for phase D fits a wave's partial tiles");
+  static_assert(2 * S::HT <= NT, "what waits for phase D fits a wave's partial tiles");
 };
 
 // tanh-GELU with first and second derivative, as gelu_fast_pair
@@ -526,9 +526,11 @@ __device__ __forceinline__ void producer(const MlpBwdRpArgs& a, unsigned char* s
         at<u32x4>(sw, S::W2T + (j * NQ + q) * 1024 + 16u * lane) = rp::pair(t0, t1);
         IO::mma2(acc, t0, t1, x.GT[(2 * q) * 64 + lane], x.GT[(2 * q + 1) * 64 + lane]);
       }
-      g1b[j] = IO::to_frag(acc * dg[j]);
+      const f32x4 g1 = acc * dg[j];
+      g1b[j] = IO::to_frag(g1);
       at<f32x4>(sw, S::DG + j * 1024 + 16u * lane) = dg[j];
       at<f32x4>(sw, S::UG + j * 1024 + 16u * lane) = acc * ddg[j];
+      at<f32x4>(sw, S::G1 + j * 1024 + 16u * lane) = g1;
       RP_FENCE();
     }
 #pragma unroll
@@ -644,7 +646,7 @@ __device__ __forceinline__ void producer(const MlpBwdRpArgs& a, unsigned char* s
       at<f32x4>(stl, S::MZ + 16u * lane) = mz;
     }
     // the next mini-batch's rows have landed: every wave has issued at least the stores of phase D behind their copies
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(HT * NQ + 3 * HT) : "memory");
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(HT * NQ + 4 * HT) : "memory");
     lds_barrier();  // ---- B6
     RP_RELANE();
 
@@ -679,7 +681,7 @@ __device__ __forceinline__ void producer(const MlpBwdRpArgs& a, unsigned char* s
       const f32x4 dz = acc * dgz[j], zs = token_sums(dz);
       if (c == 0) at<f32x4>(sl, S::ZB1 + (w * HT + j) * 64 + 16u * g) = zs;
       dzb[j] = IO::to_frag(dz);
-      at<u32x4>(sw, S::DT + j * 1024 + 16u * lane) = rp::pair(dzb[j], g1b[j]);
+      at<frag>(sw, S::DT + j * 512 + 8u * lane) = dzb[j];
       RP_FENCE();
     }
     {
@@ -895,12 +897,13 @@ __device__ __forceinline__ void consumer(const MlpBwdRpArgs& a, unsigned char* s
 
     // ================= A: d_xk, d_lr of the mini-batch before; S1 = XK dW1, dG1, dU; partial -last X2 dW2 + dU W2
     frag x2f[HT];
-    u32x4 dt[HT];  // (dZbar1, G1): fetched again for the last part of phase D
-    f32x4 dg[HT], ug[HT];
+    frag dt[HT];  // dZbar1: fetched again for the last part of phase D
+    f32x4 dg[HT], ug[HT], gg1[HT];
 #pragma unroll
     for (int j = 0; j < HT; ++j) {
       x2f[j] = at<const frag>(sw, S::XT + j * 1024 + 16u * lane);
-      dt[j] = at<const u32x4>(sw, S::DT + j * 1024 + 16u * lane);
+      dt[j] = at<const frag>(sw, S::DT + j * 512 + 8u * lane);
+      gg1[j] = at<const f32x4>(sw, S::G1 + j * 1024 + 16u * lane);
       dg[j] = at<const f32x4>(sw, S::DG + j * 1024 + 16u * lane);
       ug[j] = at<const f32x4>(sw, S::UG + j * 1024 + 16u * lane);
     }
@@ -941,14 +944,14 @@ __device__ __forceinline__ void consumer(const MlpBwdRpArgs& a, unsigned char* s
     }
     if (lane < 16 * HT) DB1[16 * w * HT + lane] += zb1;
     float qs = 0.f;
-    frag duf[HT];
+    frag duf[HT], g1b[HT];
 #pragma unroll
     for (int j = 0; j < HT; ++j) {
-      const f32x4 gg = IO::to_f32(hi(dt[j]));
 #pragma unroll
-      for (int r = 0; r < 4; ++r) qs += gg[r] * s1[j][r];
+      for (int r = 0; r < 4; ++r) qs += gg1[j][r] * s1[j][r];
+      g1b[j] = IO::to_frag(gg1[j]);
       f32x4 m = {0.f, 0.f, 0.f, 0.f};
-      IO::mma(m, flip(lo(dt[j]), x.ident), m1t);
+      IO::mma(m, flip(dt[j], x.ident), m1t);
       const f32x4 dG1 = -(last_c * s1[j] + m);
       duf[j] = IO::to_frag(dG1 * dg[j]);
       ug[j] = dG1 * ug[j];  // first term of dZ1
@@ -1019,11 +1022,14 @@ __device__ __forceinline__ void consumer(const MlpBwdRpArgs& a, unsigned char* s
       }
       x.publish(Q);
     }
-    // the first term of dZ1 and dU wait for phase D in the wave's part of the partial dK tiles, which are summed by now
+    // the first term of dZ1, dU and G1 as an operand wait for phase D in the wave's part of the partial dK tiles, which are
+    // summed by now
+    auto wait_frag = [&](int n) -> frag& { return reinterpret_cast<frag*>(x.PB + ((NW + w) * NT + HT) * 64)[n * 64 + lane]; };
 #pragma unroll
     for (int j = 0; j < HT; ++j) {
       x.PB[((NW + w) * NT + j) * 64 + lane] = ug[j];
-      reinterpret_cast<frag*>(x.PB + ((NW + w) * NT + HT) * 64)[j * 64 + lane] = duf[j];
+      wait_frag(j) = duf[j];
+      wait_frag(HT + j) = g1b[j];
     }
     lds_barrier();  // ---- C2
     RP_RELANE();
@@ -1087,7 +1093,7 @@ __device__ __forceinline__ void consumer(const MlpBwdRpArgs& a, unsigned char* s
       } else {
         load_w1(wt[0], 0);
 #pragma unroll
-        for (int n = 0; n < HT; ++n) dt[n] = at<const u32x4>(sw, S::DT + n * 1024 + 16u * lane);
+        for (int n = 0; n < HT; ++n) dt[n] = at<const frag>(sw, S::DT + n * 512 + 8u * lane);
       }
 #pragma unroll
       for (int q = 0; q < NQ; ++q) {
@@ -1109,7 +1115,7 @@ __device__ __forceinline__ void consumer(const MlpBwdRpArgs& a, unsigned char* s
       dz1[j] = IO::to_frag(dz);
       RP_FENCE();
       // dW2 += [X2 | dU]^T [dZ2 ; G2] + Xbar2^T dZbar2
-      const frag x2d = flip(x2, x.ident), dud = flip(reinterpret_cast<frag*>(x.PB + ((NW + w) * NT + HT) * 64)[j * 64 + lane], x.ident);
+      const frag x2d = flip(x2, x.ident), dud = flip(wait_frag(j), x.ident);
 #pragma unroll
       for (int I = 0; I < NT; ++I) {
         IO::mma2(dW2c[j][I], x2d, dud, ZDs[I * 64 + lane], GNs[I * 64 + lane]);
@@ -1126,6 +1132,8 @@ __device__ __forceinline__ void consumer(const MlpBwdRpArgs& a, unsigned char* s
 #pragma unroll
       for (int I = 0; I < NT; ++I) forget(dW1c[I][j]);
 #pragma unroll
+    for (int j = 0; j < HT; ++j) g1b[j] = wait_frag(HT + j);
+#pragma unroll
     for (int q = 0; q < NQ; ++q) {
       if (q + 1 < NQ) load_w1(wt[(q + 1) & 1], q + 1);
 #pragma unroll
@@ -1136,8 +1144,8 @@ __device__ __forceinline__ void consumer(const MlpBwdRpArgs& a, unsigned char* s
         for (int j = 0; j < HT; ++j) tn[j] = flip(IO::to_frag(dW1c[I][j]), x.ident);
         f32x4 p = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int j = 0; j + 1 < HT; j += 2) IO::mma2(p, tn[j], tn[j + 1], hi(dt[j]), hi(dt[j + 1]));
-        if (HT & 1) mmz(p, tn[HT - 1], hi(dt[HT - 1]));
+        for (int j = 0; j + 1 < HT; j += 2) IO::mma2(p, tn[j], tn[j + 1], g1b[j], g1b[j + 1]);
+        if (HT & 1) mmz(p, tn[HT - 1], g1b[HT - 1]);
         p *= -last_c;
 #pragma unroll
         for (int j = 0; j < HT; ++j) {
@@ -1155,7 +1163,7 @@ __device__ __forceinline__ void consumer(const MlpBwdRpArgs& a, unsigned char* s
     frag dzd[HT], dz1d[HT];
 #pragma unroll
     for (int j = 0; j < HT; ++j) {
-      dzd[j] = flip(lo(dt[j]), x.ident);
+      dzd[j] = flip(dt[j], x.ident);
       dz1d[j] = flip(dz1[j], x.ident);
     }
 #pragma unroll
