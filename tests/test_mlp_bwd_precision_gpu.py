@@ -1,0 +1,90 @@
+"""What the register-resident TTT-MLP backward (bf16 I/O) holds and multiplies in f32, element by element.
+
+One mini-batch, no gradient of the output and one element of an upstream state gradient: the last token's d_token_eta is
+then -lr * G1 * S1 (or G2 * S2) of a single token and hidden unit (or feature), the product of two numbers, and every matrix
+operand behind it is exact in bf16 or rounded in the expectation too."""
+import importlib
+import math
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+K, H_UNIT, F0, F1, TOK = 16, 5, 3, 17, 15  # tokens; the hidden unit, the features and the token that carry everything
+
+
+@pytest.fixture(scope="module")
+def P():
+    return importlib.import_module("ttt-rs_amd")
+
+
+def bf16(x):
+    return x.to(torch.bfloat16).to(x.dtype)
+
+
+def gelu_d(x):
+    """tanh-GELU and its derivative in float64"""
+    x = torch.as_tensor(x, dtype=torch.float64)
+    c = math.sqrt(2 / math.pi)
+    u = c * (x + 0.044715 * x**3)
+    return x * torch.sigmoid(2 * u), torch.sigmoid(2 * u) + 0.5 * x / torch.cosh(u) ** 2 * c * (1 + 3 * 0.044715 * x * x)
+
+
+def d_token_eta(P, d, x, through, seed=0):
+    """The last token's d_token_eta with b1 = x, and what it is in float64 (G1, S1 or G2, S2 and their product)."""
+    m = 4 * d
+    g = torch.Generator().manual_seed(seed + d)
+    xk, xv = torch.randn(1, 1, K, d, generator=g), torch.randn(1, 1, K, d, generator=g)
+    xk, xv = xk.bfloat16(), xv.bfloat16()
+    lr = torch.zeros(1, 1, K, dtype=torch.bfloat16)
+    lr[0, 0, TOK] = 2.0**-7
+    b2 = torch.randn(1, d, generator=g)
+    W2 = torch.zeros(1, m, d)
+    W2[0, H_UNIT, F0], W2[0, H_UNIT, F1] = 0.375, -0.375  # row mean 0: the kernels carry W2 centred
+    b1 = torch.full((1, m), float(x))
+    up = [torch.zeros(1, 1, d, m), torch.zeros(1, 1, m), torch.zeros(1, 1, m, d), torch.zeros(1, 1, d)]
+    if through == "G1":
+        up[0][0, 0, :, H_UNIT] = 0.25
+    else:
+        up[2][0, 0, H_UNIT, F0] = 0.75
+    dev = lambda t: t.to("cuda:0")
+    te = 1.0 / torch.arange(1, K + 1, dtype=torch.float32)
+    got = P.ttt_mlp_backward_raw(dev(xk), dev(xk), dev(xv), dev(torch.zeros(1, d, m)), dev(b1), dev(W2), dev(b2), dev(te),
+                                 dev(lr), dev(torch.ones(1, d)), dev(torch.zeros(1, d)),
+                                 dev(torch.zeros(1, 1, K, d, dtype=torch.bfloat16)), K, d_state_out=[dev(t) for t in up])
+    torch.cuda.synchronize()
+    y, dy = gelu_d(b1[0, H_UNIT].item())
+    x2 = bf16(y)
+    z = x2 * W2[0, H_UNIT].double() + b2[0].double()
+    rstd = (z.var(unbiased=False) + 1e-6) ** -0.5
+    xh = (z - z.mean()) * rstd
+    t = xv[0, 0, TOK].double() - xk[0, 0, TOK].double()
+    gx = xh - t
+    G2 = (gx - gx.mean() - xh * (gx * xh).mean()) * rstd
+    U = (bf16(G2) * W2[0, H_UNIT].double()).sum()
+    if through == "G1":
+        a, s = U * dy, xk[0, 0, TOK].double().sum() * 0.25
+    else:
+        a, s = G2[F0], x2 * 0.75
+    return got["d_token_eta"][K - 1].item(), -(2.0**-7) * (a * s).item(), (U * s).item() * 2.0**-7
+
+
+@pytest.mark.parametrize("d", [32, 64, 96])
+def test_g2_enters_d_lr_unrounded(P, d):
+    """X2 : T2, the kernel's form of G2 : S2, takes G2 in two bf16 parts: it may miss 2^-17 of it (two parts of 8 bits and
+    a sign), and the f32 products beside it."""
+    for seed in range(6):
+        print(f"case G2 in d_token_eta, d{d} seed {seed}", flush=True)
+        got, ref, _ = d_token_eta(P, d, 1.0, "G2", seed)
+        assert abs(got - ref) <= 2.0**-16 * abs(ref), (got, ref)
+
+
+@pytest.mark.parametrize("d", [32, 64, 96])
+def test_g1_enters_d_lr_in_f32(P, d):
+    """An operand's rounding would be up to 2^-9 of G1; f32 products and a sum of d terms of one size leave 2^-14 even where
+    the sum nearly cancels."""
+    for seed in range(6):
+        print(f"case G1 in d_token_eta, d{d} seed {seed}", flush=True)
+        got, ref, _ = d_token_eta(P, d, 0.0, "G1", seed)
+        assert abs(got - ref) <= 2.0**-14 * abs(ref), (got, ref)

@@ -91,7 +91,8 @@ struct MlpRpLds {
   static constexpr int CTL = QS + NW * 64;
   static constexpr int DB = CTL + 16;              // consumer: [NT][64] f32x4, d beta by lane (d gamma: in PA)
   static constexpr int B2 = DB + NT * 1024;        // consumer: d b2 [d]
-  static constexpr int BYTES = B2 + D * 4;
+  static constexpr int GL = B2 + D * 4;            // consumer: [NT][64] fragments of what G2 loses as an operand
+  static constexpr int BYTES = GL + NT * 512;
   static_assert(BYTES <= 160 * 1024, "exceeds the 160 KiB of LDS of a gfx950 CU");
   static_assert(2 * S::HT <= NT, "what waits for phase D fits a wave's partial tiles");
 };
@@ -803,6 +804,7 @@ __device__ __forceinline__ void consumer(const MlpBwdRpArgs& a, unsigned char* s
   // G2 in both orientations and dZbar2: where the staging area has room for two tensors more than are staged here
   frag* const GTs = reinterpret_cast<frag*>(smem + B::L::IN + 2 * B::L::TILE);
   frag* const GNs = GTs + NT * 64;
+  frag* const GLs = reinterpret_cast<frag*>(smem + B::L::GL);
   frag* const ZNs = reinterpret_cast<frag*>(smem + B::L::IN + B::L::IN1 + 2 * B::L::TILE);
   float* const DB1 = x.B1s;
 
@@ -1003,6 +1005,7 @@ __device__ __forceinline__ void consumer(const MlpBwdRpArgs& a, unsigned char* s
     if (red) {
       GTs[w * 64 + lane] = lo(gg);
       GNs[w * 64 + lane] = hi(gg);
+      GLs[w * 64 + lane] = IO::to_frag(G - IO::to_f32(lo(gg)));
       ZNs[w * 64 + lane] = zdn;
       const f32x4 db2T = db2();
       if (lane < 16) reinterpret_cast<float*>(smem + B::L::B2)[fb2] += zb2;  // behind the read: dG2 takes db2 as it was
@@ -1077,6 +1080,8 @@ __device__ __forceinline__ void consumer(const MlpBwdRpArgs& a, unsigned char* s
     RP_RELANE();
 
     // ================= D: T2, dX2, dZ1; partial dK; updates
+    // (X2 : T2 is the sum G2 : X2 dW2 behind d lr; it takes G2 in two bf16 parts, 16 bits of it, so that only the operands
+    // X2 and dW2 are rounded there)
     frag dz1[HT];
 #pragma unroll
     for (int j = 0; j < HT; ++j)
@@ -1097,8 +1102,9 @@ __device__ __forceinline__ void consumer(const MlpBwdRpArgs& a, unsigned char* s
       }
 #pragma unroll
       for (int q = 0; q < NQ; ++q) {
-        IO::mma2(t, flip(IO::to_frag(dW2c[j][2 * q]), x.ident), flip(IO::to_frag(dW2c[j][2 * q + 1]), x.ident),
-                 GTs[(2 * q) * 64 + lane], GTs[(2 * q + 1) * 64 + lane]);
+        const frag w0 = flip(IO::to_frag(dW2c[j][2 * q]), x.ident), w1 = flip(IO::to_frag(dW2c[j][2 * q + 1]), x.ident);
+        IO::mma2(t, w0, w1, GTs[(2 * q) * 64 + lane], GTs[(2 * q + 1) * 64 + lane]);
+        IO::mma2(t, w0, w1, GLs[(2 * q) * 64 + lane], GLs[(2 * q + 1) * 64 + lane]);
         const u32x4 v = wd[j & 1][q];
         IO::mma2(acc, lo(v), hi(v), x.ZT[(2 * q) * 64 + lane], x.ZT[(2 * q + 1) * 64 + lane]);
       }
