@@ -88,3 +88,22 @@ def test_g1_enters_d_lr_in_f32(P, d):
         print(f"case G1 in d_token_eta, d{d} seed {seed}", flush=True)
         got, ref, _ = d_token_eta(P, d, 0.0, "G1", seed)
         assert abs(got - ref) <= 2.0**-14 * abs(ref), (got, ref)
+
+
+def test_gelu_derivative_is_as_good_as_the_tanh_form(P):
+    """gelu'(x) = G1 / U where its terms cancel (x from -4.5 to -1.5), against float64: the error may be that of the tanh
+    form in float32 with a correctly rounded tanh, computed here at the same points, and half of it more for the products
+    around it.  (1 + tanh through exp2 and rcp, without a tanh, has 2.6 times that error.)"""
+    print("case gelu' through d_token_eta", flush=True)
+    c = math.sqrt(2 / math.pi)
+    err, ref = 0.0, 0.0
+    for i in range(40):
+        x = torch.tensor(-4.5 + 3.0 * (i + 0.37) / 40, dtype=torch.float32)
+        got, _, scale = d_token_eta(P, 32, x.item(), "G1", 1)
+        dy = gelu_d(x.item())[1].item()
+        t = torch.tanh((c * (x + 0.044715 * x * x * x)).double()).float()
+        f32 = 0.5 * (1 + t) + 0.5 * x * (1 - t * t) * c * (1 + 3 * 0.044715 * x * x)
+        err += (-got / scale - dy) ** 2
+        ref += (f32.double().item() - dy) ** 2
+    print(f"rms error {math.sqrt(err / 40):.3e}, of the tanh form in float32 {math.sqrt(ref / 40):.3e}")
+    assert err <= 1.5**2 * ref

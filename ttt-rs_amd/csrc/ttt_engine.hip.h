@@ -573,4 +573,14 @@ __device__ __forceinline__ void gelu_tanh_pair(float x, float& y, float& dy) {
   dy = 0.5f * (1.f + t) + 0.5f * x * (1.f - t * t) * c * (1.f + 3.f * a * x * x);
 }
 
+// tanh-GELU with first and second derivative
+__device__ __forceinline__ void gelu_tanh_all(float x, float& y, float& dy, float& ddy) {
+  const float c = 0.7978845608f, a = 0.044715f;
+  const float t = tanh_nobranch(c * (x + a * x * x * x));
+  const float du = c * (1.f + 3.f * a * x * x), ddu = 6.f * a * c * x, s = 1.f - t * t;
+  y = 0.5f * x * (1.f + t);
+  dy = 0.5f * (1.f + t) + 0.5f * x * s * du;
+  ddy = s * du + 0.5f * x * s * (ddu - 2.f * t * du * du);
+}
+
 }  // namespace ttt

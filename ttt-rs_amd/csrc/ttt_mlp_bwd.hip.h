@@ -100,16 +100,6 @@ struct MlpBwdLds {
   static_assert(BYTES <= 160 * 1024, "exceeds the 160 KiB of LDS of a gfx950 CU");
 };
 
-// tanh-GELU with first and second derivative
-__device__ __forceinline__ void gelu_tanh_all(float x, float& y, float& dy, float& ddy) {
-  const float c = 0.7978845608f, a = 0.044715f;
-  const float t = tanh_nobranch(c * (x + a * x * x * x));
-  const float du = c * (1.f + 3.f * a * x * x), ddu = 6.f * a * c * x, s = 1.f - t * t;
-  y = 0.5f * x * (1.f + t);
-  dy = 0.5f * (1.f + t) + 0.5f * x * s * du;
-  ddy = s * du + 0.5f * x * s * (ddu - 2.f * t * du * du);
-}
-
 // PIPE: two workgroups per unit on two CUs of one XCD.  A mini-batch's work falls into a part that needs only the
 // state walked back (steps 1 - 10: the roll-back and the recomputation of the forward's intermediates) and a part
 // that needs the gradient carried from the later mini-batches (steps 11 - 24).  The producer workgroup runs the

@@ -30,6 +30,7 @@
 // turn, launch by launch, over as many mini-batches as there are slots; the matrices are stored in accumulator order
 // between launches.  The same code and the same bits.
 #pragma once
+#include "ttt_engine.hip.h"
 #include "ttt_frag.hip.h"
 #include "ttt_linear_fwd_mw.hip.h"
 
@@ -96,20 +97,6 @@ struct MlpRpLds {
   static_assert(BYTES <= 160 * 1024, "exceeds the 160 KiB of LDS of a gfx950 CU");
   static_assert(2 * S::HT <= NT, "what waits for phase D fits a wave's partial tiles");
 };
-
-// tanh-GELU with first and second derivative, as gelu_fast_pair
-__device__ __forceinline__ void gelu_fast_all(float x, float& y, float& dy, float& ddy) {
-  const float c2 = 2.f * 0.7978845608f;
-  const float x2 = x * x;
-  const float u = x * __builtin_fmaf(0.044715f, x2, 1.f);
-  const float e = __builtin_amdgcn_exp2f(u * (c2 * 1.4426950409f));
-  const float r = __builtin_amdgcn_rcpf(1.f + e);
-  const float hp = 1.f - r;
-  const float w1 = c2 * __builtin_fmaf(3.f * 0.044715f, x2, 1.f), w2 = (c2 * 6.f * 0.044715f) * x, s = hp * r;
-  y = x * hp;
-  dy = hp * __builtin_fmaf(w1, x * r, 1.f);
-  ddy = s * __builtin_fmaf(x, __builtin_fmaf((r - hp) * w1, w1, w2), 2.f * w1);
-}
 
 // Lane coordinates formed anew: the addresses derived from them are many and all loop-invariant; hoisted out of the loop
 // they would be spilled and reloaded, and a reload waits for every load in flight (see ttt_mlp_fwd_rr.hip.h).
@@ -424,7 +411,7 @@ __device__ __forceinline__ void producer(const MlpBwdRpArgs& a, unsigned char* s
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         float yy, d1, d2;
-        gelu_fast_all(z1[j][r], yy, d1, d2);
+        gelu_tanh_all(z1[j][r], yy, d1, d2);
         y[r] = yy;
         dg[j][r] = d1;
         ddg[j][r] = d2;
@@ -567,7 +554,7 @@ __device__ __forceinline__ void producer(const MlpBwdRpArgs& a, unsigned char* s
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         float yy, d1;
-        gelu_fast_pair(zq[j][r], yy, d1);
+        gelu_tanh_pair(zq[j][r], yy, d1);
         y[r] = yy;
         dgz[j][r] = d1;
       }
