@@ -338,8 +338,6 @@ __device__ __forceinline__ void producer(const MlpBwdRpArgs& a, unsigned char* s
   }
   if (tid == 0) *x.lost = pair && a.spin_limit == 0 ? 1 : 0;
   const bool upd = x.te_last != 0.f;
-  const float sc = upd ? x.te_last : 1.f;
-  const float rho_c = x.te_c / sc;
 
   f32x4 W1c[NT][HT], W2c[HT][NT], b2T = {0.f, 0.f, 0.f, 0.f};
   f32x4* const st1 = reinterpret_cast<f32x4*>(a.state + bh * (size_t)(2 * D * F)) + (w * NT * HT) * 64 + lane;
@@ -486,6 +484,7 @@ __device__ __forceinline__ void producer(const MlpBwdRpArgs& a, unsigned char* s
       const f32x4 G = (gam * gO - s1 * inv_d - xh * (s2 * inv_d)) * rstd;
       const frag gt = IO::to_frag(G), gn = flip(gt, x.ident);
       x.GT[w * 64 + lane] = gt;
+      x.GS[w * 64 + lane] = gn;
       at<f32x4>(stl, S::XH + 16u * lane) = xh;
       at<f32x4>(stl, S::GO + 16u * lane) = gO;
       at<f32x4>(stl, S::G2 + 16u * lane) = G;
@@ -500,6 +499,11 @@ __device__ __forceinline__ void producer(const MlpBwdRpArgs& a, unsigned char* s
     RP_RELANE();
 
     // ================= D: U = G2 W2^T, G1; Zbar1, Xbar2; partial A2, Zbar2
+    // (Zbar1 and Zbar2 take G1, G2 and the causal blocks M1, M2 as the very operands that the gradient's products take: what
+    // an operand loses then shifts the point at which the gradient is taken, instead of adding to its error)
+    float lrs[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) lrs[r] = x.lr_of(st, 4 * g + r);
     frag g1b[HT];
 #pragma unroll
     for (int j = 0; j < HT; ++j)
@@ -541,10 +545,10 @@ __device__ __forceinline__ void producer(const MlpBwdRpArgs& a, unsigned char* s
     {
       f32x4 m;
 #pragma unroll
-      for (int r = 0; r < 4; ++r) m[r] = (4 * g + r <= c) ? rho_c * (1.f + At[r]) : 0.f;
-      const frag Mf = IO::to_frag(m);
+      for (int r = 0; r < 4; ++r) m[r] = (4 * g + r <= c) ? x.te_c * lrs[r] * (1.f + At[r]) : 0.f;
+      const frag Mf = neg(IO::to_frag(m));
 #pragma unroll
-      for (int j = 0; j < HT; ++j) mmz(zq[j], G1d[j], Mf);
+      for (int j = 0; j < HT; ++j) mmz(zq[j], flip(g1b[j], x.ident), Mf);
     }
     frag xbf[HT];
     f32x4 dgz[HT];
@@ -589,15 +593,16 @@ __device__ __forceinline__ void producer(const MlpBwdRpArgs& a, unsigned char* s
     // ================= E: reducers: output LayerNorm backward, dZbar2 (and the wave that forms d lr keeps A2)
     f32x4 at2 = {0.f, 0.f, 0.f, 0.f}, dO = at2, zb = at2;
     if (red || w == NW - 1) at2 = x.sum_block();
-    float lrs[4];
 #pragma unroll
     for (int r = 0; r < 4; ++r) lrs[r] = x.lr_of(st, 4 * g + r);
+    frag M2f = IO::zero();
     if (red) {
       f32x4 m;
 #pragma unroll
-      for (int r = 0; r < 4; ++r) m[r] = (4 * g + r <= c) ? rho_c * (1.f + at2[r]) : 0.f;
+      for (int r = 0; r < 4; ++r) m[r] = (4 * g + r <= c) ? x.te_c * lrs[r] * (1.f + at2[r]) : 0.f;
+      M2f = IO::to_frag(m);
       zb = x.sum_tile(par ^ 1, w) + b2T;
-      IO::mma(zb, x.GS[w * 64 + lane], IO::to_frag(m));
+      IO::mma(zb, x.GS[w * 64 + lane], neg(M2f));
       dO = IO::to_f32(load4<BF16>(x.row(st, 3) + x.own));
       const f32x4 gam = *reinterpret_cast<const f32x4*>(x.GAM + x.own);
       float Q[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
@@ -627,10 +632,8 @@ __device__ __forceinline__ void producer(const MlpBwdRpArgs& a, unsigned char* s
       dbet += dO;
       x.ZT[w * 64 + lane] = zt;
       at<frag>(stl, S::ZD + 8u * lane) = zd;
-      f32x4 m, mz = {0.f, 0.f, 0.f, 0.f};  // M2^T dZbar2
-#pragma unroll
-      for (int r = 0; r < 4; ++r) m[r] = (4 * g + r <= c) ? x.te_c * lrs[r] * (1.f + at2[r]) : 0.f;
-      IO::mma(mz, zd, flip(IO::to_frag(m), x.ident));
+      f32x4 mz = {0.f, 0.f, 0.f, 0.f};  // M2^T dZbar2
+      IO::mma(mz, zd, flip(M2f, x.ident));
       at<f32x4>(stl, S::MZ + 16u * lane) = mz;
     }
     // the next mini-batch's rows have landed: every wave has issued at least the stores of phase D behind their copies
