@@ -110,3 +110,23 @@ def test_static_scratch_takes_what_the_other_scan_fits(P):
             assert_close(got[k], ref[k].double(), 1e-5, k)
         else:
             assert torch.equal(got[k], ref[k]), k
+
+
+@pytest.mark.parametrize("B,H,d,N", [(8, 16, 32, 96), (1, 8, 96, 40)])
+def test_hand_over_slots_are_read_fresh(P, B, H, d, N):
+    """Many turns of the ring of slots, up to as many units as run on two workgroups: what the consumer reads is what the
+    producer stored this time, not what an earlier turn left in the consumer's vector cache (one workgroup per unit runs
+    the two sides as separate launches)."""
+    K = 16
+    print(f"case mlp bwd rp ring B{B} H{H} d{d} N{N}", flush=True)
+    v = to_dev(mlp_case(P, 612, B, H, N * K, d, K, torch.bfloat16, "baseline"))
+    a = [v[k] for k in ("xq", "xk", "xv", "W1", "b1", "W2", "b2", "token_eta", "lr", "gamma", "beta")]
+    d_out = torch.randn(B, H, N * K, d, generator=torch.Generator().manual_seed(8)).to(torch.bfloat16).to("cuda:0")
+    got = P.ttt_mlp_backward_raw(*a, d_out, K)
+    one = P.ttt_mlp_backward_raw(*a, d_out, K, kernel_hint=P.TTT_HINT_ONE_WORKGROUP)
+    torch.cuda.synchronize()
+    for k in GRADS:
+        if k in ("d_token_eta", "d_gamma", "d_beta"):  # atomic additions: their order is not fixed
+            assert_close(got[k], one[k].double(), 1e-4, k)
+        else:
+            assert torch.equal(got[k], one[k]), k

@@ -134,6 +134,27 @@ __device__ __forceinline__ V& at(const unsigned char* base, unsigned off) {
   return *reinterpret_cast<V*>(const_cast<unsigned char*>(base) + off);
 }
 
+// The consumer's reads of a slot: device-scope loads (sc1), which do not look in the CU's vector cache and so see what the
+// producer's CU stored into the L2 behind both.  (Dropping the cache instead takes an instruction of device scope, which
+// also drops lines of the L2; what one of workgroup scope does is not for other workgroups to rely on.)  A slot is read once
+// or twice, so the cache holds nothing worth keeping of it: forward and backward at 128 units of 2048 tokens, d = 96, take
+// 3554 us, with a device-scope acquire per mini-batch 3908 us.  Scalar offset + lane offset.
+struct Slot {
+  __amdgpu_buffer_rsrc_t rsrc;
+  __device__ __forceinline__ Slot(const unsigned char* base, int bytes)
+      : rsrc(__builtin_amdgcn_make_buffer_rsrc(const_cast<unsigned char*>(base), 0, bytes, 0x00027000)) {}
+  template <class V>
+  __device__ __forceinline__ V get(unsigned lane_off, unsigned off) const {
+    static_assert(sizeof(V) == 4 || sizeof(V) == 8 || sizeof(V) == 16, "");
+    if constexpr (sizeof(V) == 16)
+      return __builtin_bit_cast(V, __builtin_amdgcn_raw_buffer_load_b128(rsrc, lane_off, off, 16));
+    else if constexpr (sizeof(V) == 8)
+      return __builtin_bit_cast(V, __builtin_amdgcn_raw_buffer_load_b64(rsrc, lane_off, off, 16));
+    else
+      return __builtin_bit_cast(V, __builtin_amdgcn_raw_buffer_load_b32(rsrc, lane_off, off, 16));
+  }
+};
+
 // sums of a tile over its tokens (the lanes of a row), in every lane
 __device__ __forceinline__ f32x4 token_sums(f32x4 v) {
   f32x4 s;
@@ -867,20 +888,14 @@ __device__ __forceinline__ void consumer(const MlpBwdRpArgs& a, unsigned char* s
   };
 
   for (int st = a.last - 1; st >= a.first; --st) {
-    const unsigned char* const sl = x.slot(st);
-    const unsigned char* const sw = sl + w * S::WAVE;
-    const unsigned char* const stl = sl + S::TILES + (red ? w : 0) * S::TILE;
+    const Slot sl(x.slot(st), S::SLOT);
+    const unsigned sw = w * S::WAVE, stl = S::TILES + (red ? w : 0) * S::TILE;
     x.poll(fl, 0, a.n_stages - st);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     lds_barrier();  // ---- T: the slot is filled, this mini-batch's rows have landed, the slot before is no longer read
-    if (pair) {
-      // drop what this CU's vector cache holds; behind one L2 nothing else need go (an agent-scope acquire also drops
-      // lines of the L2, and the hand-over is read from there)
-      if (same_l2)
-        asm volatile("buffer_inv sc0" ::: "memory");
-      else
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-    }
+    // a producer behind another L2 writes its L2 back: drop the lines that this one's L2 and vector cache hold.  Behind one
+    // L2 nothing need go: the hand-over is read with device-scope loads (see Slot), which do not look in the vector cache
+    if (pair && !same_l2) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
     if (pair && !same_l2 && a.agent_release == 0)
       same_l2 = __builtin_amdgcn_readfirstlane(__hip_atomic_load(fl + 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) == (0x100u | my_xcc);
     x.raise(fl, 1, a.n_stages - 1 - st);
@@ -893,28 +908,28 @@ __device__ __forceinline__ void consumer(const MlpBwdRpArgs& a, unsigned char* s
     f32x4 dg[HT], ug[HT], gg1[HT];
 #pragma unroll
     for (int j = 0; j < HT; ++j) {
-      x2f[j] = at<const frag>(sw, S::XT + j * 1024 + 16u * lane);
-      dt[j] = at<const frag>(sw, S::DT + j * 512 + 8u * lane);
-      gg1[j] = at<const f32x4>(sw, S::G1 + j * 1024 + 16u * lane);
-      dg[j] = at<const f32x4>(sw, S::DG + j * 1024 + 16u * lane);
-      ug[j] = at<const f32x4>(sw, S::UG + j * 1024 + 16u * lane);
+      x2f[j] = sl.get<frag>(16u * lane, sw + S::XT + j * 1024);
+      dt[j] = sl.get<frag>(8u * lane, sw + S::DT + j * 512);
+      gg1[j] = sl.get<f32x4>(16u * lane, sw + S::G1 + j * 1024);
+      dg[j] = sl.get<f32x4>(16u * lane, sw + S::DG + j * 1024);
+      ug[j] = sl.get<f32x4>(16u * lane, sw + S::UG + j * 1024);
     }
-    const frag m1t = at<const frag>(sl, S::M1T + 8u * lane);
+    const frag m1t = sl.get<frag>(8u * lane, S::M1T);
     // the images of W2 and W1 are fetched a feature-tile pair ahead of their use
     auto load_w2 = [&](u32x4 (&t)[HT], int q) {
 #pragma unroll
-      for (int j = 0; j < HT; ++j) t[j] = at<const u32x4>(sw, S::W2T + (j * NQ + q) * 1024 + 16u * lane);
+      for (int j = 0; j < HT; ++j) t[j] = sl.get<u32x4>(16u * lane, sw + S::W2T + (j * NQ + q) * 1024);
     };
     auto load_w1 = [&](u32x4 (&t)[HT], int q) {
 #pragma unroll
-      for (int n = 0; n < HT; ++n) t[n] = at<const u32x4>(sw, S::W1T + (q * HT + n) * 1024 + 16u * lane);
+      for (int n = 0; n < HT; ++n) t[n] = sl.get<u32x4>(16u * lane, sw + S::W1T + (q * HT + n) * 1024);
     };
     u32x4 wt[2][HT];
     load_w2(wt[0], 0);
     // column sums of dZbar1 (own hidden slice) and, reducers, of dZbar2 (own features): one value a lane
-    const float zb1 = at<const float>(sl, S::ZB1 + w * HT * 64 + 4u * (lane < 16 * HT ? lane : 0));
+    const float zb1 = sl.get<float>(4u * (lane < 16 * HT ? lane : 0), S::ZB1 + w * HT * 64);
     const int fb2 = own_offset<1>(red ? w : 0, 0, (lane >> 2) & 3) + (lane & 3);
-    const float zb2 = at<const float>(sl, S::ZB2 + 4u * fb2);
+    const float zb2 = sl.get<float>(4u * fb2, S::ZB2);
     RP_FENCE();
     if (st + 1 < a.last) finish(st + 1);
     const float last_c = x.te_last * x.lr_of(st, c);
@@ -977,16 +992,16 @@ __device__ __forceinline__ void consumer(const MlpBwdRpArgs& a, unsigned char* s
     f32x4 xh = {0.f, 0.f, 0.f, 0.f}, gO = xh, uu = xh, G = xh, mz = xh;
     u32x4 gg = {0u, 0u, 0u, 0u};
     frag zdn = IO::zero();
-    const unsigned so = S::SCAL + 4u * c;
-    const float rstd = at<const float>(sl, so), sg = at<const float>(sl, so + 64), sgx = at<const float>(sl, so + 128),
-                sa1 = at<const float>(sl, so + 192), sa2 = at<const float>(sl, so + 256), dlp = at<const float>(sl, so + 320);
+    const unsigned so = 4u * c;
+    const float rstd = sl.get<float>(so, S::SCAL), sg = sl.get<float>(so, S::SCAL + 64), sgx = sl.get<float>(so, S::SCAL + 128),
+                sa1 = sl.get<float>(so, S::SCAL + 192), sa2 = sl.get<float>(so, S::SCAL + 256), dlp = sl.get<float>(so, S::SCAL + 320);
     if (red) {
-      xh = at<const f32x4>(stl, S::XH + 16u * lane);
-      gO = at<const f32x4>(stl, S::GO + 16u * lane);
-      G = at<const f32x4>(stl, S::G2 + 16u * lane);
-      mz = at<const f32x4>(stl, S::MZ + 16u * lane);
-      gg = at<const u32x4>(stl, S::GG + 16u * lane);
-      zdn = at<const frag>(stl, S::ZD + 8u * lane);
+      xh = sl.get<f32x4>(16u * lane, stl + S::XH);
+      gO = sl.get<f32x4>(16u * lane, stl + S::GO);
+      G = sl.get<f32x4>(16u * lane, stl + S::G2);
+      mz = sl.get<f32x4>(16u * lane, stl + S::MZ);
+      gg = sl.get<u32x4>(16u * lane, stl + S::GG);
+      zdn = sl.get<frag>(8u * lane, stl + S::ZD);
     }
     lds_barrier();  // ---- C1
     RP_RELANE();
@@ -1029,17 +1044,17 @@ __device__ __forceinline__ void consumer(const MlpBwdRpArgs& a, unsigned char* s
     u32x4 wd[2][NQ];  // W2^T by hidden tile, for dX2
     auto load_w2j = [&](u32x4 (&t)[NQ], int j) {
 #pragma unroll
-      for (int q = 0; q < NQ; ++q) t[q] = at<const u32x4>(sw, S::W2T + (j * NQ + q) * 1024 + 16u * lane);
+      for (int q = 0; q < NQ; ++q) t[q] = sl.get<u32x4>(16u * lane, sw + S::W2T + (j * NQ + q) * 1024);
     };
     u32x4 xd[2];
     f32x4 dd[2];  // (X2, Xbar2) and gelu'(Z1), fetched again rather than held since phase A
     auto load_xd = [&](int j) {
-      xd[j & 1] = at<const u32x4>(sw, S::XT + j * 1024 + 16u * lane);
-      dd[j & 1] = at<const f32x4>(sw, S::DG + j * 1024 + 16u * lane);
+      xd[j & 1] = sl.get<u32x4>(16u * lane, sw + S::XT + j * 1024);
+      dd[j & 1] = sl.get<f32x4>(16u * lane, sw + S::DG + j * 1024);
     };
     load_w2j(wd[0], 0);
     load_xd(0);
-    const frag a2t = at<const frag>(sl, S::A2T + 8u * lane), a1t = at<const frag>(sl, S::A1T + 8u * lane);
+    const frag a2t = sl.get<frag>(8u * lane, S::A2T), a1t = sl.get<frag>(8u * lane, S::A1T);
 
     // ================= C: reducers: dZ2, dT
     if (red) {
@@ -1088,7 +1103,7 @@ __device__ __forceinline__ void consumer(const MlpBwdRpArgs& a, unsigned char* s
       } else {
         load_w1(wt[0], 0);
 #pragma unroll
-        for (int n = 0; n < HT; ++n) dt[n] = at<const frag>(sw, S::DT + n * 512 + 8u * lane);
+        for (int n = 0; n < HT; ++n) dt[n] = sl.get<frag>(8u * lane, sw + S::DT + n * 512);
       }
 #pragma unroll
       for (int q = 0; q < NQ; ++q) {
