@@ -202,15 +202,25 @@ int ttt_linear_bwd(const ttt_desc* desc, const void* xq, const void* xk, const v
  * ttt_linear_bwd with a caller-owned workspace: the same call (same interface of the reference replaced, same
  * arguments, same results to rounding) for a caller that can hold ttt_linear_bwd_workspace_bytes(desc) bytes of
  * device memory (16-byte aligned, ordinary hipMalloc memory, nothing in it has to be kept between calls).  The
- * workspace argument itself has no counterpart in the reference.  Where that size is above zero -- f32 I/O,
- * checkpoint_interval 1 (row-major or packed checkpoints), head_dim 32 or 64, at most 128 (batch, head) units, no
- * TTT_HINT_ONE_WORKGROUP or wave hint -- and the device has two CUs per unit, the reverse scan of a unit runs on two
+ * workspace argument itself has no counterpart in the reference.  That size is above zero in two cases.
+ *
+ * checkpoint_interval > 1 (f32 checkpoints, mini_batch <= 16, head_dim 32 or 64, no TTT_HINT_LDS_TILES): the states between the checkpoints are computed first, all
+ * segments side by side, into the workspace, and the kernels for one checkpoint per mini-batch read them, where the call
+ * without a workspace simulates them again on the CU that carries the scan (head_dim 64, interval 16, 96 units of 2048
+ * tokens: 3.28 -> 0.56 ms with f32 I/O, 2.71 -> 0.38 ms with bf16 I/O).  The states take at most 256 MiB (one segment of a
+ * single unit may exceed that): a longer sequence or a larger batch goes through the workspace in several launches.  So the
+ * call holds, while it runs, up to what dense checkpoints would take; a caller without that memory passes NULL.  Tensors
+ * off a 16-byte boundary run as without a workspace.
+ *
+ * f32 I/O, checkpoint_interval 1 (row-major or packed checkpoints), head_dim 32 or 64, at most 128 (batch, head) units,
+ * no TTT_HINT_ONE_WORKGROUP or wave hint: where the device has two CUs per unit, the reverse scan of a unit runs on two
  * workgroups on two CUs: one recomputes what depends only on the saved state (Z1, G, Zbar, dZbar, the attention
  * block's gradients, d_xq), the other carries the state gradient (dZ1, d_xk, d_xv, d_lr, d_token_eta, dW, db); they
  * hand their data over through a ring of three slots per unit in the workspace and follow each other through two
  * counters there.  The f32 backward is bound by the matrix instructions of the CUs that hold a unit, and a batch of
  * 8 x 12 heads leaves 160 of 256 CUs idle: at that shape (head_dim 64, 2048 tokens) the backward takes 0.44 instead of
  * 0.72 ms.
+ * (The scan behind sparse checkpoints with f32 I/O runs this way too, under the same conditions.)
  * Both workgroups must be resident together, and what ttt_mlp_fwd says of a GPU shared with other work holds here: a
  * workgroup that waits for its partner in vain (2^21 polls, seconds) gives up, both run to the end without waiting
  * again, the unit's d_b0 is NaN in every element (its other gradients are then meaningless) and

@@ -193,3 +193,16 @@ def test_eta_logit_gradient_helper_matches_the_oracle_chain(P):
     got = P.ttt_lr_eta_logit_grad(d_lr, z, 1.5, 64).double().numpy()
     ref = orc.lr_logit_grad(d_lr.double().numpy(), z.double().numpy(), 1.5, 64)
     assert np.abs(got - ref).max() <= 1e-6 * np.abs(ref).max()
+
+
+@pytest.mark.parametrize("io", ["TTT_F32", "TTT_BF16"])
+@pytest.mark.parametrize("B,H,d,N,ci", [
+    (8, 12, 64, 128, 16), (32, 16, 64, 128, 128), (64, 16, 64, 512, 512), (1, 16, 64, 2048, 2048), (3, 5, 64, 8192, 8000),
+    (16, 16, 32, 4096, 4096), (1, 1, 64, 8192, 8192), (1000, 3, 64, 40, 39), (8, 16, 64, 4, 1 << 30)])
+def test_sparse_backward_workspace_is_bounded(pkg, B, H, d, N, ci, io):
+    """The states of a launch take at most 256 MiB (beside the hand-over ring of units on two workgroups), or those of one
+    segment of one unit."""
+    state, ring = d * (d + 1) * 4, 128 * 3 * 48 * 1024
+    desc = pkg.TttDesc(B, H, N * 16, d, 16, 1e-6, ci, getattr(pkg, io))
+    n = pkg.lib().ttt_linear_bwd_workspace_bytes(C.byref(desc))
+    assert 0 < n <= max(256 << 20, min(ci, N) * state) + ring

@@ -43,3 +43,19 @@ def test_sparse_backward_against_dense_checkpoints(P, B, H, N, ci, dtype):
     g1, g0 = run_bwd(P, c, dO, K, ci), run_bwd(P, c, dO, K, 1)
     for name, _ in NAMES:
         assert_close(g1[name], g0[name].double(), TOL[dtype], name, min_frac=0.99)
+
+
+@pytest.mark.parametrize("B,H,N,ci,dtype", [
+    (34, 16, 35, 33, torch.float32), (34, 16, 33, 40, torch.bfloat16),  # a segment of all units exceeds the workspace's bound: batch elements
+    (2, 16, 1040, 1039, torch.bfloat16)])  # ... of one batch element's: heads, and segments of them
+def test_sparse_backward_in_launches_over_units(P, B, H, N, ci, dtype):
+    d, K = 64, 16
+    print(f"case sparse bwd over units B{B} H{H} N{N} ci{ci} {dtype}", flush=True)
+    c = P.synthetic.baseline_inputs(8, B, H, N * K, d, K, io_dtype=dtype, with_dout=True)
+    dO = c.pop("d_out")
+    g = torch.Generator().manual_seed(N)
+    c["gamma"], c["beta"] = 1 + 0.1 * torch.randn(H, d, generator=g), 0.1 * torch.randn(H, d, generator=g)
+    sg = (torch.randn(B, H, d, d, generator=g), torch.randn(B, H, d, generator=g))
+    g1, g0 = run_bwd(P, c, dO, K, ci, sg), run_bwd(P, c, dO, K, 1, sg)
+    for name, _ in NAMES:
+        assert_close(g1[name], g0[name].double(), TOL[dtype], name, min_frac=0.99)

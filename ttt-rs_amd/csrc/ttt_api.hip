@@ -1281,11 +1281,15 @@ int launch_linear_bwd_pairs(const ttt::LinearBwdArgs& a, const ttt_desc* d, cons
 // CU that carries the scan: ci / 2 extra forward mini-batches in front of each.  With a workspace the states are
 // computed first, all segments at once (ttt_linear_states_kernel), and the dense-checkpoint kernels read them: at the
 // 125M shape (f32, 96 units, 2048 tokens, ci = 16) 3.21 -> 0.56 ms.
-// The workspace is bounded: a launch takes as many whole segments as kLinStatesMaxBytes holds states for (at least one),
-// from the end of the sequence to its beginning; the state gradient of a launch is the upstream gradient of the next.
+// The workspace is bounded: a launch takes as many whole segments of all units as kLinStatesMaxBytes holds states for, from
+// the end of the sequence to its beginning (the state gradient of a launch is the upstream gradient of the next); where one
+// segment of all units is too much, one segment of as many batch elements, or of as many heads of one, as it holds.  Only
+// the segment of a single unit may exceed it.  The bound: launches of fewer segments cost chains of their own.  96 units of
+// 2048 tokens, d = 64, ci = 16 (every state: 195 MiB) take 563 / 380 us (f32 / bf16) in one launch, 605 / 402 within
+// 128 MiB, 654 / 438 within 64, 857 / 529 within 32.
 constexpr size_t kLinStatesMaxBytes = (size_t)256 << 20;
 struct LinStatesPlan {
-  ttt_desc dense;     // the desc of the backward that reads the states
+  ttt_desc dense;     // the desc of the backward that reads the states of a launch: its batch elements and heads
   bool pair;          // ... on two workgroups per unit
   LinBwdPairWs pw;
   int segments;       // per unit and launch, but for the last of a sequence
@@ -1295,17 +1299,34 @@ bool plan_linear_states(const ttt_desc* d, LinStatesPlan* p) {
   if (d->checkpoint_interval == 1 || d->mini_batch > 16 || d->head_dim > 64 || d->checkpoint_format != TTT_CKPT_F32 ||
       (d->kernel_hint & TTT_HINT_LDS_TILES) != 0)
     return false;
+  const size_t B = d->batch, H = d->heads, D = d->head_dim, N = d->seq / d->mini_batch;
+  const size_t ci = (size_t)d->checkpoint_interval < N ? d->checkpoint_interval : N, C = (N + ci - 1) / ci;
+  const size_t held = kLinStatesMaxBytes / (ci * D * (D + 1) * sizeof(float));  // segments of one unit
+  size_t nb = B, nh = H, seg = held / (B * H);
+  auto even = [](size_t all, size_t most) {  // parts of at most `most`, as even as can be
+    const size_t parts = (all + most - 1) / most;
+    return (all + parts - 1) / parts;
+  };
+  if (seg < 1) {
+    seg = 1;
+    if (held >= H) {
+      nb = even(B, held / H);
+    } else {
+      nb = 1;
+      nh = even(H, held < 1 ? 1 : held);
+    }
+  } else if (seg > C) {
+    seg = C;
+  }
+  p->segments = (int)seg;
   p->dense = *d;
+  p->dense.batch = (int32_t)nb;
+  p->dense.heads = (int32_t)nh;
   p->dense.checkpoint_interval = 1;
   p->dense.checkpoint_format = TTT_CKPT_PACKED;
   p->pair = linear_bwd_pair_wanted(&p->dense);
   p->pw = p->pair ? linear_bwd_pair_ws(&p->dense) : LinBwdPairWs{0, 0, 0};
-  const size_t U = (size_t)d->batch * d->heads, D = d->head_dim, N = d->seq / d->mini_batch, ci = d->checkpoint_interval;
-  const size_t C = (N + ci - 1) / ci, per_segment = U * ci * D * (D + 1) * sizeof(float);
-  size_t seg = kLinStatesMaxBytes / per_segment;
-  seg = seg < 1 ? 1 : seg > C ? C : seg;
-  p->segments = (int)seg;
-  const size_t stages = seg * ci < N ? seg * ci : N;
+  const size_t stages = seg * ci < N ? seg * ci : N, U = nb * nh;
   p->W = (p->pw.total + 255) / 256 * 256;
   p->b = p->W + U * stages * D * D * sizeof(float);
   p->total = p->b + U * stages * D * sizeof(float);
@@ -1330,35 +1351,48 @@ int linear_bwd_sparse(const ttt_desc* d, const LinStatesPlan& p, bool pair, cons
   const size_t es = f32 ? 4 : 2;
   unsigned char* ws = static_cast<unsigned char*>(workspace);
   float *Ws = reinterpret_cast<float*>(ws + p.W), *bs = reinterpret_cast<float*>(ws + p.b);
-  for (int c0 = (C - 1) / p.segments * p.segments; c0 >= 0; c0 -= p.segments) {
+  // batch elements b0 .. b0 + nb, heads h0 .. h0 + nh of them (of one only if not all), from segment c0 on
+  auto launch = [&](int b0, int nb, int h0, int nh, int c0) {
+    const size_t u0 = (size_t)b0 * d->heads + h0, row0 = u0 * base.seq_stride;
     const int first = c0 * ci, stages = (N - first < p.segments * ci) ? N - first : p.segments * ci;
     const size_t tok = (size_t)first * d->mini_batch;
-    auto in = [&](const void* q, size_t per_token) { return static_cast<const void*>(static_cast<const char*>(q) + tok * per_token); };
-    auto out = [&](void* q, size_t per_token) { return static_cast<void*>(static_cast<char*>(q) + tok * per_token); };
+    auto in = [&](const void* q, size_t per_token) { return static_cast<const void*>(static_cast<const char*>(q) + (row0 + tok) * per_token); };
+    auto out = [&](void* q, size_t per_token) { return static_cast<void*>(static_cast<char*>(q) + (row0 + tok) * per_token); };
+    auto of_units = [&](auto* q, size_t per_unit) { return q == nullptr ? q : q + u0 * per_unit; };
     ttt::LinearFwdArgs f{};
     f.xq = in(base.xq, D * es); f.xk = in(base.xk, D * es); f.xv = in(base.xv, D * es); f.lr = in(base.lr, es);
-    f.token_eta = base.token_eta; f.gamma = base.gamma; f.beta = base.beta;
+    f.token_eta = base.token_eta; f.gamma = base.gamma + (size_t)h0 * D; f.beta = base.beta + (size_t)h0 * D;
     f.W_ckpt = Ws; f.b_ckpt = bs;
-    f.B = base.B; f.H = base.H; f.seq = stages * d->mini_batch; f.K = base.K; f.seq_stride = base.seq_stride;
+    f.B = nb; f.H = nh; f.seq = stages * d->mini_batch; f.K = base.K; f.seq_stride = base.seq_stride;
     f.n_stages = f.n_ckpt = stages; f.ckpt_interval = 1; f.state_per_batch = 1; f.ckpt_packed = 1; f.eps = base.eps;
-    ttt::LinearSegments sg{base.W_ckpt, base.b_ckpt, C, c0, (stages + ci - 1) / ci, ci};
-    if (D == 64) rc = f32 ? launch_linear_states<ttt::F32, 64, 4>(f, sg, s) : launch_linear_states<ttt::BF16, 64, 2>(f, sg, s);
-    else rc = f32 ? launch_linear_states<ttt::F32, 32, 2>(f, sg, s) : launch_linear_states<ttt::BF16, 32, 2>(f, sg, s);
-    if (rc != TTT_OK) return rc;
+    ttt::LinearSegments sg{of_units(base.W_ckpt, (size_t)C * D * D), of_units(base.b_ckpt, (size_t)C * D), C, c0,
+                           (stages + ci - 1) / ci, ci};
+    int r;
+    if (D == 64) r = f32 ? launch_linear_states<ttt::F32, 64, 4>(f, sg, s) : launch_linear_states<ttt::BF16, 64, 2>(f, sg, s);
+    else r = f32 ? launch_linear_states<ttt::F32, 32, 2>(f, sg, s) : launch_linear_states<ttt::BF16, 32, 2>(f, sg, s);
+    if (r != TTT_OK) return r;
     ttt::LinearBwdArgs a = base;
     a.xq = f.xq; a.xk = f.xk; a.xv = f.xv; a.lr = f.lr; a.d_out = in(base.d_out, D * es);
+    a.gamma = f.gamma; a.beta = f.beta;
     a.d_xq = out(base.d_xq, D * es); a.d_xk = out(base.d_xk, D * es); a.d_xv = out(base.d_xv, D * es);
     a.d_lr = out(base.d_lr, es); a.d_token_eta = base.d_token_eta + tok;
+    a.d_gamma = base.d_gamma + (size_t)h0 * D; a.d_beta = base.d_beta + (size_t)h0 * D;
+    a.d_W0 = of_units(base.d_W0, (size_t)D * D); a.d_b0 = of_units(base.d_b0, D);
     a.W_ckpt = Ws; a.b_ckpt = bs; a.ckpt_packed = 1; a.ckpt_interval = 1;
-    a.seq = f.seq; a.n_stages = a.n_ckpt = stages;
-    if (first + stages < N) {
-      a.d_W_out = base.d_W0;
-      a.d_b_out = base.d_b0;
-    }
-    rc = pair && stages > 1 ? launch_linear_bwd_pairs(a, &p.dense, p.pw, workspace, s)
-                            : launch_linear_bwd_reg(a, D, f32, ch.waves, s);
-    if (rc != TTT_OK) return rc;
-  }
+    a.B = nb; a.H = nh; a.seq = f.seq; a.n_stages = a.n_ckpt = stages;
+    const bool last = first + stages == N;
+    a.d_W_out = last ? of_units(base.d_W_out, (size_t)D * D) : a.d_W0;
+    a.d_b_out = last ? of_units(base.d_b_out, D) : a.d_b0;
+    return pair && stages > 1 ? launch_linear_bwd_pairs(a, &p.dense, p.pw, workspace, s)
+                              : launch_linear_bwd_reg(a, D, f32, ch.waves, s);
+  };
+  const int B = d->batch, H = d->heads, nb = p.dense.batch, nh = p.dense.heads;
+  for (int b0 = 0; b0 < B; b0 += nb)
+    for (int h0 = 0; h0 < H; h0 += nh)
+      for (int c0 = (C - 1) / p.segments * p.segments; c0 >= 0; c0 -= p.segments) {
+        rc = launch(b0, B - b0 < nb ? B - b0 : nb, h0, H - h0 < nh ? H - h0 : nh, c0);
+        if (rc != TTT_OK) return rc;
+      }
   return TTT_OK;
 }
 
@@ -1386,7 +1420,8 @@ int linear_bwd_impl(const ttt_desc* d, const void* xq, const void* xk, const voi
     int cus = 0;
     rc = device_cus(&cus);
     if (rc != TTT_OK) return rc;
-    pair = 2 * (int64_t)d->batch * d->heads <= cus;  // every workgroup a CU of its own, both sides resident together
+    const int64_t units = states ? (int64_t)sparse.dense.batch * sparse.dense.heads : (int64_t)d->batch * d->heads;
+    pair = 2 * units <= cus;  // every workgroup a CU of its own, both sides resident together
   }
   // W0/b0 are part of the saved state for interface parity; the state entering every stage is
   // rebuilt from the checkpoints (checkpoint 0 equals the initial state).

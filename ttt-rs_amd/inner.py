@@ -114,8 +114,10 @@ def ttt_linear_backward_raw(xq, xk, xv, weight, bias, token_eta, ttt_lr_eta, ln_
                             checkpoint_interval: int = 1, grad_weight_out=None, grad_bias_out=None, packed_checkpoints: bool = False,
                             kernel_hint: int = 0, workspace=None):
     """One call of ttt_linear_bwd (or ttt_linear_bwd_ws, where the library has a kernel that uses a workspace: f32
-    I/O up to 128 units runs every unit on two workgroups) on the current stream.  workspace: a device tensor of
-    ttt_linear_bwd_workspace_bytes(desc) bytes, None to allocate one, False to call the entry point without.
+    I/O up to 128 units runs every unit on two workgroups; with checkpoint_interval > 1 the states between the checkpoints
+    are computed first, into up to 256 MiB) on the current stream.  workspace: a device tensor of
+    ttt_linear_bwd_workspace_bytes(desc) bytes, None to allocate one for the call, False to call the entry point without
+    (the memory of sparse checkpoints and nothing else, at several times the time).
 
     Counterpart of backward_multi (rust/fused/src/linear_fused_tile/backward/launch.rs:332-438).
     Returns a dict with the nine input gradients named as TttGradInputs
