@@ -204,7 +204,8 @@ int ttt_linear_bwd(const ttt_desc* desc, const void* xq, const void* xk, const v
  * device memory (16-byte aligned, ordinary hipMalloc memory, nothing in it has to be kept between calls).  The
  * workspace argument itself has no counterpart in the reference.  That size is above zero in two cases.
  *
- * checkpoint_interval > 1 (f32 checkpoints, mini_batch <= 16, head_dim 32 or 64, no TTT_HINT_LDS_TILES): the states between the checkpoints are computed first, all
+ * checkpoint_interval > 1 (f32 checkpoints, mini_batch <= 16, head_dim 32 or 64, no TTT_HINT_LDS_TILES; not f32 I/O at
+ * head_dim 32 with an interval up to 3 and more than 256 units): the states between the checkpoints are computed first, all
  * segments side by side, into the workspace, and the kernels for one checkpoint per mini-batch read them, where the call
  * without a workspace simulates them again on the CU that carries the scan (head_dim 64, interval 16, 96 units of 2048
  * tokens: 3.28 -> 0.56 ms with f32 I/O, 2.71 -> 0.38 ms with bf16 I/O).  The states take at most 256 MiB (one segment of a

@@ -206,3 +206,11 @@ def test_sparse_backward_workspace_is_bounded(pkg, B, H, d, N, ci, io):
     desc = pkg.TttDesc(B, H, N * 16, d, 16, 1e-6, ci, getattr(pkg, io))
     n = pkg.lib().ttt_linear_bwd_workspace_bytes(C.byref(desc))
     assert 0 < n <= max(256 << 20, min(ci, N) * state) + ring
+
+
+def test_sparse_backward_workspace_only_where_it_is_faster(pkg):
+    size = lambda B, d, ci, io: pkg.lib().ttt_linear_bwd_workspace_bytes(
+        C.byref(pkg.TttDesc(B, 16, 1024, d, 16, 1e-6, ci, getattr(pkg, io))))
+    assert size(24, 32, 2, "TTT_F32") == 0 and size(24, 32, 3, "TTT_F32") == 0
+    for case in ((24, 32, 4, "TTT_F32"), (16, 32, 2, "TTT_F32"), (24, 32, 2, "TTT_BF16"), (24, 64, 2, "TTT_F32")):
+        assert size(*case) > 0, case

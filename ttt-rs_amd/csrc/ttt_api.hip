@@ -1299,6 +1299,11 @@ bool plan_linear_states(const ttt_desc* d, LinStatesPlan* p) {
   if (d->checkpoint_interval == 1 || d->mini_batch > 16 || d->head_dim > 64 || d->checkpoint_format != TTT_CKPT_F32 ||
       (d->kernel_hint & TTT_HINT_LDS_TILES) != 0)
     return false;
+  // f32 at head_dim 32: with a second and third unit on a CU the scan that simulates one or two mini-batches again is the
+  // shorter one (384 units of 1024 tokens, interval 2: 427 against 503 us, 4: 541 against 476).  Everything else gains, from
+  // 96 to 1024 units and from interval 2 on (the least: f32, d = 64, interval 2, 2471 -> 2320 us at 1024 units).
+  if (d->io_dtype == TTT_F32 && d->head_dim == 32 && d->checkpoint_interval <= 3 && (int64_t)d->batch * d->heads > 256)
+    return false;
   const size_t B = d->batch, H = d->heads, D = d->head_dim, N = d->seq / d->mini_batch;
   const size_t ci = (size_t)d->checkpoint_interval < N ? d->checkpoint_interval : N, C = (N + ci - 1) / ci;
   const size_t held = kLinStatesMaxBytes / (ci * D * (D + 1) * sizeof(float));  // segments of one unit
