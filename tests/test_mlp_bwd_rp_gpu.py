@@ -25,8 +25,12 @@ def test_register_resident_backward(P, B, H, d, K, N, sg):
     got, ref = run_case(P, B, H, d, K, N, torch.bfloat16, "baseline", sg)
     one, _ = run_case(P, B, H, d, K, N, torch.bfloat16, "baseline", sg, kernel_hint=P.TTT_HINT_ONE_WORKGROUP)
     for k in GRADS:
-        # d_token_eta is a sum over units with alternating signs: few mini-batches leave little but rounding
-        assert_close(got[k], ref[k], TOL[torch.bfloat16] * (5 if k == "d_token_eta" else 1), k, min_frac=0.8)
+        # The usual bars: long sequences of one or two units leave up to 4 % of d_b1 outside the elementwise band, as they do
+        # with the scan on tiles in memory.  d_token_eta is a sum over units with alternating signs: after two mini-batches
+        # little but rounding is left of it (that scan misses it by 0.10 and has 31 % outside).
+        few = k == "d_token_eta" and N == 2
+        assert_close(got[k], ref[k], TOL[torch.bfloat16] * (5 if few else 1.25 if k == "d_token_eta" else 1), k,
+                     min_frac=0.65 if few else 0.95)
         if k in ("d_token_eta", "d_gamma", "d_beta"):  # atomic additions: their order is not fixed
             assert_close(one[k], got[k].double(), 1e-5, k)
         else:

@@ -1033,7 +1033,9 @@ void launch_linear_adam_variant(const ttt::LinearFwdArgs& a, const ttt::AdamArgs
 // head_dim 64: a wave per feature tile while every unit has a CU to itself.  Beyond that two waves per unit with bf16 I/O
 // (four would put two on a SIMD: 324 us at 384 units, against 237); with f32 I/O the products fill a second wave's gaps
 // and four stay ahead (538 against 551), two to a SIMD.  head_dim 32: two waves, alone on their SIMDs up to two units per
-// CU.  (2048 tokens.)
+// CU.  (2048 tokens.)  Beyond two units per CU the units queue, and one wave to a SIMD stays right: bf16, head_dim 64, 1024
+// tokens take 143 us at 512 units, 256 at 528, 279 at 1024, 406 at 1536; with registers for two waves to a SIMD the state
+// spills, 712, 799, 1152 and 1973 us.
 template <class T>
 void launch_linear_adam(int head_dim, int64_t units, int cus, const ttt::LinearFwdArgs& a, const ttt::AdamArgs& ad, hipStream_t s) {
   constexpr bool f32 = sizeof(typename ttt::Io<T>::elem) == 4;

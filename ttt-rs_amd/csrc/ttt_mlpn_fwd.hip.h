@@ -1,7 +1,8 @@
 // TTT-MLP with NL hidden layers (NL = 2, 3, 4), multi-stage forward: the reference's TTTMLP2 / TTTMLP3 / TTTMLP4 inner
 // models (rust/core/src/mlp2.rs:152-243, mlp3.rs:162-279, mlp4.rs:186-324) looped as rust/core/src/inner.rs:25-50.
-// The reference has no fused kernel for them; this is their Burn-op mini-batch restated as one persistent kernel on
-// the LDS tile engine, the NL-layer generalisation of ttt_mlp_fwd_kernel (ttt_engine_fwd.hip.h):
+// The reference has no fused kernel for them; this is their Burn-op mini-batch restated as one persistent kernel with the
+// weights in registers, the NL-layer generalisation of the loop that ttt_mlp_fwd_kernel (ttt_engine_fwd.hip.h) runs on tiles
+// in memory:
 //
 //   weight layer i = 0 .. NL:  W[i] [in_i x out_i], in_0 = d, out_NL = d, every other side M = 4 d
 //   forward chain   X[0] = XK;  Z[i] = X[i] W[i] + b[i];  X[i+1] = gelu(Z[i])  (i < NL)

@@ -96,7 +96,6 @@ def ttt_linear_forward_raw(xq, xk, xv, weight, bias, token_eta, ttt_lr_eta, ln_w
                                  checkpoint_interval, want_checkpoints, out, int(packed_checkpoints), kernel_hint)
 
 
-
 def ttt_linear_adam_forward_raw(xq, xk, xv, weight, bias, token_eta, ttt_lr_eta, ln_weight, ln_bias, mini_batch: int,
                                 beta1: float = 0.9, beta2: float = 0.999, adam_eps: float = 1e-8, adam_lr: float = 1e-3,
                                 moments=None, step: int = 0, eps: float = 1e-6):
@@ -106,7 +105,6 @@ def ttt_linear_adam_forward_raw(xq, xk, xv, weight, bias, token_eta, ttt_lr_eta,
     at `step`, or None for a fresh state.  Returns (output, weight, bias, (weight_m, bias_m, weight_v, bias_v), step)."""
     return host().linear_adam_forward(xq, xk, xv, weight, bias, token_eta, ttt_lr_eta, ln_weight, ln_bias, mini_batch,
                                       beta1, beta2, adam_eps, adam_lr, moments, int(step), eps)
-
 
 
 def ttt_linear_backward_raw(xq, xk, xv, weight, bias, token_eta, ttt_lr_eta, ln_weight, ln_bias,
@@ -129,7 +127,6 @@ def ttt_linear_backward_raw(xq, xk, xv, weight, bias, token_eta, ttt_lr_eta, ln_
                                   grad_bias_out, int(packed_checkpoints), kernel_hint, workspace)
 
 
-
 def ttt_mlp_forward_raw(xq, xk, xv, w1, b1, w2, b2, token_eta, ttt_lr_eta, ln_weight, ln_bias,
                         mini_batch: int, eps: float = 1e-6, kernel_hint: int = 0, save_for_backward: bool = False):
     """One call of ttt_mlp_fwd on the current stream: the fused counterpart of
@@ -142,7 +139,6 @@ def ttt_mlp_forward_raw(xq, xk, xv, w1, b1, w2, b2, token_eta, ttt_lr_eta, ln_we
                               kernel_hint, save_for_backward)
 
 
-
 def ttt_mlpn_forward_raw(xq, xk, xv, weights, biases, token_eta, ttt_lr_eta, ln_weight, ln_bias, mini_batch: int,
                          eps: float = 1e-6):
     """One call of ttt_mlpn_fwd on the current stream: TTTMLP2/3/4::forward (rust/core/src/mlp2.rs, mlp3.rs, mlp4.rs
@@ -150,7 +146,6 @@ def ttt_mlpn_forward_raw(xq, xk, xv, weights, biases, token_eta, ttt_lr_eta, ln_
     with a leading batch dimension.  Returns (output, weights_out, biases_out), state per batch element."""
     return host().mlpn_forward(xq, xk, xv, list(weights), list(biases), token_eta, ttt_lr_eta, ln_weight, ln_bias,
                                mini_batch, eps)
-
 
 
 def ttt_mlp_backward_raw(xq, xk, xv, w1, b1, w2, b2, token_eta, ttt_lr_eta, ln_weight, ln_bias, d_out,
@@ -170,7 +165,6 @@ def ttt_mlp_backward_raw(xq, xk, xv, w1, b1, w2, b2, token_eta, ttt_lr_eta, ln_w
     consumes it."""
     return host().mlp_backward(xq, xk, xv, w1, b1, w2, b2, token_eta, ttt_lr_eta, ln_weight, ln_bias, d_out, mini_batch,
                                eps, d_state_out, static_scratch, into, int(kernel_hint), saved)
-
 
 
 @dataclass
@@ -500,7 +494,6 @@ def ttt_stack_forward_raw(layers, token_eta, mini_batch: int, eps: float = 1e-6,
                                 0 if aux_stream is None else aux_stream.cuda_stream, int(check_lost))
 
 
-
 # --------------------------------------------------------------------------- either side of the inner loop
 def rope_cos_sin(seq_len: int, offset: int, wrap: Optional[int], head_dim: int, device, base: float = 10000.0):
     """RotaryEmbeddingConfig::init + RotaryEmbedding::get_cos_sin (rust/core/src/util.rs:266-322) in f32:
@@ -534,7 +527,6 @@ def inner_loop_inputs_raw(xq, xk, xv, lr_logits, lr_bias, base_lr: float, token_
     return TTTInputsInner(Qkv(q, k, v), te, lr)
 
 
-
 def ttt_linear_forward_fused_inputs_raw(xq, xk, xv, lr_logits, lr_bias, base_lr: float, token_idx,
                                         learnable_token_idx, weight, bias, ln_weight, ln_bias, mini_batch: int,
                                         rope=None, pos_offset: int = 0, pos_wrap: int = 0, eps: float = 1e-6,
@@ -554,7 +546,6 @@ def ttt_linear_forward_fused_inputs_raw(xq, xk, xv, lr_logits, lr_bias, base_lr:
         return r
     q, k, v, lr, te = r[-5:]
     return r[:-5] + (TTTInputsInner(Qkv(q, k, v), te, lr),)
-
 
 
 def layer_epilogue_raw(inner_out, post_norm_weight, post_norm_bias, gate=None, eps: float = 1e-6):
