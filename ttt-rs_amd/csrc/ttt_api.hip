@@ -651,8 +651,10 @@ struct MlpRpWs {
     fac = b2 + U * D * sizeof(float);
     hand = fac + U * N * facb;
     const size_t room = MlpBwdWs(d).total * sizeof(float), fix = hand + U * ttt::kMlpRpFlagWords * sizeof(unsigned);
-    // one workgroup per unit: the roles run in turn over as many mini-batches as there are slots
-    size_t n = mlp_bwd_pipe(d) ? 3 : room > fix ? (room - fix) / (U * slot) : 1;
+    // one workgroup per unit: the roles run in turn over as many mini-batches as there are slots, and every turn loads and
+    // stores the matrices; a quarter of a slot more than the other scan's room buys one more (256 units, 32 mini-batches,
+    // d = 64: two slots 1329 us forward and backward, three 1149)
+    size_t n = mlp_bwd_pipe(d) ? 3 : room > fix ? (room - fix + U * slot / 4) / (U * slot) : 1;
     n = n < 1 ? 1 : n > 16 ? 16 : n > N && !mlp_bwd_pipe(d) ? N : n;
     slots = (int)n;
     flags = hand + U * n * slot;
