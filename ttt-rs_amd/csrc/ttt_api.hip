@@ -1387,7 +1387,7 @@ int linear_bwd_sparse(const ttt_desc* d, const LinStatesPlan& p, bool pair, cons
     a.d_lr = out(base.d_lr, es); a.d_token_eta = base.d_token_eta + tok;
     a.d_gamma = base.d_gamma + (size_t)h0 * D; a.d_beta = base.d_beta + (size_t)h0 * D;
     a.d_W0 = of_units(base.d_W0, (size_t)D * D); a.d_b0 = of_units(base.d_b0, D);
-    a.W_ckpt = Ws; a.b_ckpt = bs; a.ckpt_packed = 1; a.ckpt_interval = 1;
+    a.W_ckpt = Ws; a.b_ckpt = bs; a.ckpt_packed = 1; a.ckpt_interval = 1; a.tokens_db = 1;
     a.B = nb; a.H = nh; a.seq = f.seq; a.n_stages = a.n_ckpt = stages;
     const bool last = first + stages == N;
     a.d_W_out = last ? of_units(base.d_W_out, (size_t)D * D) : a.d_W0;

@@ -85,6 +85,16 @@ __device__ __forceinline__ float row16_sum_dpp(float v) {
   v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x121, 0xf, 0xf, false));  // row_ror:1
   return v;
 }
+// four of them: the sums of a tile over its tokens (the lanes of a row), in every lane
+__device__ __forceinline__ f32x4 over_tokens(f32x4 v) {
+  f32x4 s;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const float x = v[r];
+    s[r] = row16_sum_dpp(x);
+  }
+  return s;
+}
 // The value of the first lane (c = 0) of each row of 16 lanes, in every lane of that row.  A rotation sum leaves
 // every lane with the same terms added in a different order, i.e. possibly different last bits; where all lanes
 // of a row must hold the SAME number (a pivot subtracted from a whole matrix row), one lane's result is shared.

@@ -754,7 +754,9 @@ __global__ void __launch_bounds__(64 * (D / 16 + 1)) ttt_linear_bwd_pair_kernel(
         IO::mma2(dWc[I], qa, ka, Zd, Z1d);
         IO::mma2(DT[I], za, z1a, qdo, kdo);
       }
-      IO::mma2(dbT, Zd, Z1d, ones, ones);
+      f32x4 t = zero4;  // (the tokens' sum first, as in ttt_linear_bwd_mw_kernel)
+      IO::mma2(t, Zd, Z1d, ones, ones);
+      dbT += t;
     }
   }
 

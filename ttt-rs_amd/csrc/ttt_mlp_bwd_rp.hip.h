@@ -180,17 +180,6 @@ struct Slot {
   }
 };
 
-// sums of a tile over its tokens (the lanes of a row), in every lane
-__device__ __forceinline__ f32x4 token_sums(f32x4 v) {
-  f32x4 s;
-#pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const float x = v[r];
-    s[r] = row16_sum_dpp(x);
-  }
-  return s;
-}
-
 // What both roles need of their place: lane coordinates, LDS regions, input staging, exchange of row sums.
 template <int D, int TENSORS>
 struct Base {
@@ -672,7 +661,7 @@ __device__ __forceinline__ void producer(const MlpBwdRpArgs& a, unsigned char* s
       const float s1 = q2 * inv_d, s2 = rstd * (q3 - mu * q2) * inv_d;
       const f32x4 gam = *reinterpret_cast<const f32x4*>(x.GAM + x.own);
       const f32x4 xh = (zb - mu) * rstd;
-      const f32x4 dz = (gam * dO - s1 - xh * s2) * rstd, zs = token_sums(dz);
+      const f32x4 dz = (gam * dO - s1 - xh * s2) * rstd, zs = over_tokens(dz);
       if (c == 0) at<f32x4>(sl, S::ZB2 + 4u * x.own) = zs;
       const frag zt = IO::to_frag(dz), zd = flip(zt, x.ident);
       dgam += dO * xh;
@@ -716,7 +705,7 @@ __device__ __forceinline__ void producer(const MlpBwdRpArgs& a, unsigned char* s
         IO::mma2(acc, flip(IO::to_frag(W2c[j][2 * q]), x.ident), flip(IO::to_frag(W2c[j][2 * q + 1]), x.ident),
                  x.ZT[(2 * q) * 64 + lane], x.ZT[(2 * q + 1) * 64 + lane]);
       mmz(acc, x2d[j], dA2f);
-      const f32x4 dz = acc * dgz[j], zs = token_sums(dz);
+      const f32x4 dz = acc * dgz[j], zs = over_tokens(dz);
       if (c == 0) at<f32x4>(sl, S::ZB1 + (w * HT + j) * 64 + 16u * g) = zs;
       dzb[j] = IO::to_frag(dz);
       at<frag>(sw, S::DT + j * 512 + 8u * lane) = dzb[j];
@@ -1101,7 +1090,7 @@ __device__ __forceinline__ void consumer(const MlpBwdRpArgs& a, unsigned char* s
       const frag zt = IO::to_frag(dZ2), zd = flip(zt, x.ident);
       x.ZT[w * 64 + lane] = zt;
       ZDs[w * 64 + lane] = zd;
-      const f32x4 b = db2() + token_sums(dZ2);
+      const f32x4 b = db2() + over_tokens(dZ2);
       if (c == 0) db2() = b;
       dk_p = dy;  // -d target
       IO::mma(dk_p, QD[w * 64 + lane], a1t);
@@ -1146,7 +1135,7 @@ __device__ __forceinline__ void consumer(const MlpBwdRpArgs& a, unsigned char* s
       const f32x4 dz = x.PB[((NW + w) * NT + j) * 64 + lane] + dx2 * dd[j & 1];
       {
         f32x4* const bp = reinterpret_cast<f32x4*>(DB1 + 16 * (w * HT + j) + 4 * g);
-        const f32x4 b = *bp + token_sums(dz);  // (bias gradients are sums of f32 terms)
+        const f32x4 b = *bp + over_tokens(dz);  // (bias gradients are sums of f32 terms)
         if (c == 0) *bp = b;
       }
       dz1[j] = IO::to_frag(dz);
