@@ -63,7 +63,7 @@ def test_mlp_bwd_matches_oracle(P, B, H, d, K, N, style, state_grads, dtype):
 @pytest.mark.parametrize("d,N,style,sg", [(32, 3, "ref", False), (64, 4, "ref", True), (96, 3, "baseline", False)])
 def test_mlp_bwd_bf16_with_f32_products(P, d, N, style, sg):
     """bf16 I/O up to head_dim 96: the scan with its products kept in f32 (TTT_HINT_F32_PRODUCTS) and the default scan
-    (bf16 operands) are two compilations of the same kernel; both are held to the oracle, and to each other."""
+    (bf16 operands, in registers) are two kernels; both are held to the oracle, and to each other."""
     print(f"case mlp bwd bf16 f32-products d{d}", flush=True)
     got32, ref = run_case(P, 1, 2, d, 16, N, torch.bfloat16, style, sg, kernel_hint=P.TTT_HINT_F32_PRODUCTS)
     got16, _ = run_case(P, 1, 2, d, 16, N, torch.bfloat16, style, sg)
