@@ -413,9 +413,11 @@ int launch_linear_bwd(const ttt::LinearBwdArgs& a, unsigned grid, hipStream_t s)
 }
 
 // bf16 I/O, one checkpoint per mini-batch: one wave per (batch, head), state gradient in registers
-template <int D, bool PK = false>
+template <int D, bool PK = false, bool TDB = false>
 int launch_linear_bwd_rr(const ttt::LinearBwdArgs& a, unsigned grid, hipStream_t s) {
-  constexpr auto kern = ttt::ttt_linear_bwd_rr_kernel<ttt::BF16, D, PK>;
+  if constexpr (PK && !TDB)
+    if (a.tokens_db) return launch_linear_bwd_rr<D, PK, true>(a, grid, s);
+  constexpr auto kern = ttt::ttt_linear_bwd_rr_kernel<ttt::BF16, D, PK, TDB>;
   constexpr size_t bytes = ttt::LinBwdRrLds<D, PK>::BYTES;
   int rc = opt_in_lds<kern>(bytes);
   if (rc != TTT_OK) return rc;
@@ -424,20 +426,22 @@ int launch_linear_bwd_rr(const ttt::LinearBwdArgs& a, unsigned grid, hipStream_t
 }
 
 // one checkpoint per mini-batch, NW waves per (batch, head): feature axis split, exchanges through LDS
-template <class T, int D, int NW, bool PK = false, bool FM = false>
+template <class T, int D, int NW, bool PK = false, bool FM = false, bool TDB = false>
 int launch_linear_bwd_mw(const ttt::LinearBwdArgs& a, unsigned grid, hipStream_t s) {
+  if constexpr (PK && !FM && !TDB && D <= 64)  // (sparse checkpoints: d = 32 and 64)
+    if (a.tokens_db) return launch_linear_bwd_mw<T, D, NW, PK, FM, true>(a, grid, s);
   constexpr size_t bytes = ttt::LinBwdMwLds<D, NW, sizeof(typename ttt::Io<T>::elem), PK, FM>::BYTES;
   // opaque checkpoints (the training path): a variant for whole mini-batches of 16 tokens
   if constexpr (PK) {
     if (a.K == 16) {
-      constexpr auto kern16 = ttt::ttt_linear_bwd_mw_kernel<T, D, NW, PK, FM, true>;
+      constexpr auto kern16 = ttt::ttt_linear_bwd_mw_kernel<T, D, NW, PK, FM, true, TDB>;
       int rc = opt_in_lds<kern16>(bytes);
       if (rc != TTT_OK) return rc;
       hipLaunchKernelGGL(kern16, dim3(grid), dim3(64 * NW), bytes, s, a);
       return hip_status(hipGetLastError(), "ttt_linear_bwd (multi-wave register-resident kernel) launch");
     }
   }
-  constexpr auto kern = ttt::ttt_linear_bwd_mw_kernel<T, D, NW, PK, FM>;
+  constexpr auto kern = ttt::ttt_linear_bwd_mw_kernel<T, D, NW, PK, FM, false, TDB>;
   int rc = opt_in_lds<kern>(bytes);
   if (rc != TTT_OK) return rc;
   hipLaunchKernelGGL(kern, dim3(grid), dim3(64 * NW), bytes, s, a);

@@ -48,7 +48,7 @@ struct LinearBwdArgs {
   int B, H, seq, seq_stride, K, n_stages, ckpt_interval, n_ckpt;
   int ckpt_packed;  // W checkpoints as bf16 operand fragments (register-resident kernels, bf16 I/O)
   float eps;
-  int tokens_db = 0;  // register-resident kernels, bf16 I/O, packed checkpoints: the bias gradient as a sum of f32 terms
+  int tokens_db = 0;  // register-resident kernels, packed checkpoints: the bias gradient as f32 sums token by token
 };
 
 // MT tiles of 16 token rows: mini_batch <= KT = 16 MT.  MT = 2 serves the reference's (mini_batch 32, head_dim 32)

@@ -59,7 +59,7 @@ struct LinBwdMwLds {
 // Up to d = 64 with one feature tile per wave the kernel is held to 256 registers: two workgroups then share a compute
 // unit (two waves per SIMD), which is what 257 registers would silently halve (f32 I/O with f32 row-major checkpoints
 // excepted: it needs 265 and would spill).
-template <class T, int D, int NW, bool PK = false, bool FM = false, bool FULL = false>
+template <class T, int D, int NW, bool PK = false, bool FM = false, bool FULL = false, bool TDB = false>
 __global__ void __launch_bounds__(64 * NW, (D <= 64 && D / 16 == NW && (PK || sizeof(typename Io<T>::elem) == 2)) ? 2 : 1)
     ttt_linear_bwd_mw_kernel(LinearBwdArgs a) {
   using IO = Io<T>;
@@ -98,11 +98,11 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && D / 16 == NW && (PK || si
   const frag ident = identity_frag<T>(c, g);
   const frag ones = splat_frag<T>(1.f);
   const f32x4 zero4 = {0.f, 0.f, 0.f, 0.f};
-  // dbT: the bias gradient, in every lane; behind sparse checkpoints with bf16 I/O (tdb) of the token that the lane holds,
-  // in f32, and added up over the lanes where it is used.  As a product of bf16 operands with ones its error is 1.6 times
-  // as large, and that of d_beta, which S carries it into, 1.5 times: more than that of the LDS-tile kernel, which the
-  // route from sparse checkpoints stands in for.
-  const bool tdb = BF && PK && !FM && D <= 64 && a.tokens_db != 0;
+  // dbT: the bias gradient, in every lane; behind sparse checkpoints (TDB) of the token that the lane holds, in f32, and
+  // added up over the lanes where it is used.  As a product with ones its error is 1.6 times as large with bf16 operands
+  // and 1.7 times with f32 ones (a rounding of the whole gradient for every token): more than that of the LDS-tile
+  // kernel, which the route from sparse checkpoints stands in for.  Its own instantiation: as a branch in the one for
+  // dense checkpoints it costs that one 3.7 % with f32 I/O (d 64, 144 units x 2048 tokens: 960 -> 996 us).
   f32x4 gam[TPW], bet[TPW], a2[TPW], dgam[TPW], dbet[TPW], dbT[TPW];
   float sum_a = 0.f;
   for (int f = 0; f < D; ++f) sum_a += a.gamma[h * D + f] * a.gamma[h * D + f];
@@ -113,7 +113,7 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && D / 16 == NW && (PK || si
     bet[jj] = *reinterpret_cast<const f32x4*>(a.beta + h * D + f);
     a2[jj] = gam[jj] * gam[jj];
     dgam[jj] = dbet[jj] = zero4;
-    dbT[jj] = a.d_b_out && (!tdb || c == 0) ? *reinterpret_cast<const f32x4*>(a.d_b_out + bh * D + f) : zero4;
+    dbT[jj] = a.d_b_out && (!TDB || c == 0) ? *reinterpret_cast<const f32x4*>(a.d_b_out + bh * D + f) : zero4;
   }
   // dWc[I][jj]: rows i = feat(I, 4g+r), columns j = feat(own jj, c)
   // DT[J][ii]:  rows j = feat(J, 4g+r), columns i = feat(own ii, c)   (= dW[own rows][all columns], transposed)
@@ -489,7 +489,7 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && D / 16 == NW && (PK || si
 #pragma unroll
     for (int ii = 0; ii < TPW; ++ii) {
       S[ii] = dbT[ii];
-      if (tdb) S[ii] = over_tokens(dbT[ii]);
+      if constexpr (TDB) S[ii] = over_tokens(dbT[ii]);
 #pragma unroll
       for (int qq = 0; qq < NQ; ++qq)
         IO::mma2(S[ii], IO::to_frag(dWc[2 * qq][ii]), IO::to_frag(dWc[2 * qq + 1][ii]), k[2 * qq], k[2 * qq + 1]);
@@ -566,7 +566,7 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && D / 16 == NW && (PK || si
         dbet[jj] += dO;
         const f32x4 dzb = (gx2[jj] - m1 - x2 * m2) * rstd2;
         Zf[jj] = IO::to_frag(dzb);
-        if (tdb) dbT[jj] += dzb;
+        if constexpr (TDB) dbT[jj] += dzb;
         Zd[jj] = tokens_k(Zf[jj]);
         fr(ZF, w * TPW + jj) = Zf[jj];
         fr(ZD, w * TPW + jj) = Zd[jj];
@@ -712,7 +712,7 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && D / 16 == NW && (PK || si
         const f32x4 dxh = dy * gam[jj] + gx[jj] * s2 + u[jj] * sgx;
         const f32x4 dz1 = (dxh - q1) * rstd1 + xh[jj] * (dsig * inv_d);
         Z1f[jj] = IO::to_frag(dz1);
-        if (tdb) dbT[jj] += dz1;
+        if constexpr (TDB) dbT[jj] += dz1;
         Z1d[jj] = tokens_k(Z1f[jj]);
         fr(Z1F, w * TPW + jj) = Z1f[jj];
         fr(Z1D, w * TPW + jj) = Z1d[jj];
@@ -770,13 +770,7 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && D / 16 == NW && (PK || si
     }
 #pragma unroll
     for (int jj = 0; jj < TPW; ++jj) {
-      if constexpr (!BF) {  // (the tokens' sum first: 32 roundings at its size instead of the gradient's)
-        f32x4 t = zero4;
-        IO::mma2(t, Zd[jj], Z1d[jj], ones, ones);
-        dbT[jj] += t;
-      } else if (!tdb) {
-        IO::mma2(dbT[jj], Zd[jj], Z1d[jj], ones, ones);
-      }
+      if constexpr (!TDB) IO::mma2(dbT[jj], Zd[jj], Z1d[jj], ones, ones);
     }
     if constexpr (!FM) single_wave_outputs();
     // FM: the state entering the next mini-batch of the scan.  Placed last: its short dependent chain (transposes,
@@ -797,7 +791,7 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && D / 16 == NW && (PK || si
 #pragma unroll
   for (int jj = 0; jj < TPW; ++jj) {
     const int f = own_offset<TPW>(w, jj, g);
-    if (tdb) dbT[jj] = over_tokens(dbT[jj]);
+    if constexpr (TDB) dbT[jj] = over_tokens(dbT[jj]);
     if (c == 0) store4<F32>(a.d_b0 + bh * D + f, dbT[jj]);
 #pragma unroll
     for (int r = 0; r < 4; ++r) {

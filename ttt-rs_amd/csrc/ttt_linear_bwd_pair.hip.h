@@ -754,7 +754,7 @@ __global__ void __launch_bounds__(64 * (D / 16 + 1)) ttt_linear_bwd_pair_kernel(
         IO::mma2(dWc[I], qa, ka, Zd, Z1d);
         IO::mma2(DT[I], za, z1a, qdo, kdo);
       }
-      f32x4 t = zero4;  // (the tokens' sum first, as in ttt_linear_bwd_mw_kernel)
+      f32x4 t = zero4;  // (the tokens' sum first: its roundings are not at the gradient's size)
       IO::mma2(t, Zd, Z1d, ones, ones);
       dbT += t;
     }

@@ -41,7 +41,7 @@ struct LinBwdRrLds {
   static constexpr int BYTES = M0 + (D + 4) * 4;
 };
 
-template <class T, int D, bool PK = false>
+template <class T, int D, bool PK = false, bool TDB = false>
 __global__ void __launch_bounds__(64) ttt_linear_bwd_rr_kernel(LinearBwdArgs a) {
   using IO = Io<T>;
   using frag = typename IO::frag;
@@ -64,15 +64,14 @@ __global__ void __launch_bounds__(64) ttt_linear_bwd_rr_kernel(LinearBwdArgs a) 
   for (int r = 0; r < 4; ++r) te_s[r] = (4 * g + r < K) ? a.token_eta[4 * g + r] : 0.f;
   const frag ident = identity_frag<T>(c, g);
   const frag ones = splat_frag<T>(1.f);
-  const bool tdb = PK && a.tokens_db != 0;  // dbT of the token that the lane holds, see ttt_linear_bwd_mw_kernel
-  f32x4 gam[NT], bet[NT], dgam[NT], dbet[NT], dbT[NT];
+  f32x4 gam[NT], bet[NT], dgam[NT], dbet[NT], dbT[NT];  // TDB: dbT of the lane's token, see ttt_linear_bwd_mw_kernel
 #pragma unroll
   for (int J = 0; J < NT; ++J) {
     const int f = own_offset<NT>(0, J, g);
     gam[J] = *reinterpret_cast<const f32x4*>(a.gamma + h * D + f);
     bet[J] = *reinterpret_cast<const f32x4*>(a.beta + h * D + f);
     dgam[J] = dbet[J] = f32x4{0.f, 0.f, 0.f, 0.f};
-    dbT[J] = a.d_b_out && (!tdb || c == 0) ? *reinterpret_cast<const f32x4*>(a.d_b_out + bh * D + f) : f32x4{0.f, 0.f, 0.f, 0.f};
+    dbT[J] = a.d_b_out && (!TDB || c == 0) ? *reinterpret_cast<const f32x4*>(a.d_b_out + bh * D + f) : f32x4{0.f, 0.f, 0.f, 0.f};
   }
   // state gradient: dWc[I][J], rows i = feat(I, 4g+r) in registers, columns j = feat(J, c) on lanes
   f32x4 dWc[NT][NT];
@@ -380,7 +379,7 @@ __global__ void __launch_bounds__(64) ttt_linear_bwd_rr_kernel(LinearBwdArgs a) 
       for (int I = 0; I < NT; ++I) {
         dK[I] = DGM[I] = TMP[I] = zero4;
         S[I] = dbT[I];
-        if (tdb) {
+        if constexpr (TDB) {
           S[I] = over_tokens(dbT[I]);
           dbT[I] += DZB[I];
         }
@@ -434,7 +433,7 @@ __global__ void __launch_bounds__(64) ttt_linear_bwd_rr_kernel(LinearBwdArgs a) 
       for (int J = 0; J < NT; ++J) {
         const f32x4 dz1 = (dxh[J] - q1) * rstd1 + xh[J] * (dsig * inv_d);
         Z1f[J] = IO::to_frag(dz1);
-        if (tdb) dbT[J] += dz1;
+        if constexpr (TDB) dbT[J] += dz1;
         Z1d[J] = tokens_k(Z1f[J]);
         dK[J] += dy[J] - last * TMP[J];
         dy[J] = -dy[J];
@@ -477,9 +476,10 @@ __global__ void __launch_bounds__(64) ttt_linear_bwd_rr_kernel(LinearBwdArgs a) 
       for (int J = 0; J < NT; ++J) {
         IO::mma2(dWc[I][J], qd[I], kd[I], Zd[J], Z1d[J]);
       }
-    if (!tdb)
+    if constexpr (!TDB) {
 #pragma unroll
       for (int J = 0; J < NT; ++J) IO::mma2(dbT[J], Zd[J], Z1d[J], ones, ones);
+    }
     // The next mini-batch's copies to LDS must have landed; this mini-batch's stores and atomics, all issued
     // after them, need not have (the atomics of all units meet on one cache line and take long).  Vector
     // memory operations retire in order on this counter, so the wait leaves exactly those outstanding:
@@ -501,7 +501,7 @@ __global__ void __launch_bounds__(64) ttt_linear_bwd_rr_kernel(LinearBwdArgs a) 
 #pragma unroll
   for (int J = 0; J < NT; ++J) {
     const int f = own_offset<NT>(0, J, g);
-    if (tdb) dbT[J] = over_tokens(dbT[J]);
+    if constexpr (TDB) dbT[J] = over_tokens(dbT[J]);
     if (c == 0) store4<F32>(a.d_b0 + bh * D + f, dbT[J]);
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
