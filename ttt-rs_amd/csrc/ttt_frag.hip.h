@@ -284,19 +284,18 @@ __device__ __forceinline__ float lr_gate(float z, float scale) { return scale / 
 // y = gelu_tanh(x), dy = its derivative.  With r = 1 / (1 + exp(2u)), u = c (x + a x^3):
 // (1 + tanh u) / 2 = 1 - r and 1 - tanh^2 u = 4 r (1 - r).
 __device__ __forceinline__ void gelu_fast_pair(float x, float& y, float& dy) {
-  const float c2 = 2.f * 0.7978845608f;
+  constexpr float c2 = 2.f * 0.7978845608f, a = 0.044715f, l = 1.4426950409f;
   const float x2 = x * x;
-  const float u = x * __builtin_fmaf(0.044715f, x2, 1.f);
-  const float e = __builtin_amdgcn_exp2f(u * (c2 * 1.4426950409f));
+  const float e = __builtin_amdgcn_exp2f(x * __builtin_fmaf(c2 * a * l, x2, c2 * l));
   const float r = __builtin_amdgcn_rcpf(1.f + e);
   const float hp = 1.f - r;
   y = x * hp;
-  dy = hp * __builtin_fmaf(c2 * __builtin_fmaf(3.f * 0.044715f, x2, 1.f), x * r, 1.f);
+  dy = hp * __builtin_fmaf(__builtin_fmaf(3.f * a * c2, x2, c2), x * r, 1.f);
 }
 __device__ __forceinline__ float gelu_fast(float x) {
-  const float u = x * __builtin_fmaf(0.044715f, x * x, 1.f);
-  const float e = __builtin_amdgcn_exp2f(u * (2.f * 0.7978845608f * 1.4426950409f));
-  return x - x * __builtin_amdgcn_rcpf(1.f + e);
+  constexpr float c2 = 2.f * 0.7978845608f, a = 0.044715f, l = 1.4426950409f;
+  const float e = __builtin_amdgcn_exp2f(x * __builtin_fmaf(c2 * a * l, x * x, c2 * l));
+  return __builtin_fmaf(-x, __builtin_amdgcn_rcpf(1.f + e), x);
 }
 
 // A launch may carry several independent problems of one shape, gridDim.y of them (windows of different layers of

@@ -16,19 +16,27 @@
 //
 // Per mini-batch there are three barriers on the recurrence W -> Z1 -> X2 -> Z2 -> G2 -> G1 -> W':
 //   B1  partial Z2 tiles (and last mini-batch's partial Zbar2 / A2) are in LDS
-//   B2  the reducers' row moments (six for the LN-L2 gradient of this mini-batch, two for the output
-//       LayerNorm of the previous one) are in LDS
-//   B3  G2 (as both operand orientations, already scaled by -eta_last) is in LDS
-// The output of mini-batch t needs nothing the recurrence waits for, so it is finished one
-// mini-batch late, inside the reducers' part of mini-batch t+1, and shares its barriers.
+//   B2  the reducers' row moments for the LN-L2 gradient are in LDS
+//   B3  G2 (already scaled by -eta_last) is in LDS, and the row moments of last mini-batch's output
+// The output of mini-batch t needs nothing the recurrence waits for: it is finished one mini-batch late, and between B1
+// and B3 it is the work of the waves that reduce nothing, so that the reducers' chain is the only thing there.
+//
+// What bounds it.  Phases A and D (the products) by the issue of a SIMD's two waves: matrix instructions and vector
+// instructions of 16x16 tiles hardly overlap, not across waves either (probe: a matrix instruction and three FMAs, two
+// waves, 23.3 cycles against 16 + 7.5).  Phases B and C by latency.  Cycles of a mini-batch at d = 96 and 128 units,
+// before -> after the last revision: A 4.9 -> 4.7 k (XQ W1 now shares the operands of XK W1), B 2.9 -> 2.0 k, C 2.2 -> 1.3 k
+// (output off the chain, loads in one go, sums by lane group), D 7.4 -> 6.4 k (independent products side by side, transposes
+// read from LDS).  8 x 16 units x 2048 tokens: d = 96 840 -> 667 us, d = 64 488 -> 433 us, d = 32 286 -> 266 us.
 //
 // An odd hidden tile at the end of a split-k chain is issued as a k = 32 MFMA with a zero second
 // half, not as a k = 16 one: a 16x16x16 bf16 MFMA accumulating straight onto the result of a
 // 16x16x32 one was measured to give wrong sums on gfx950 with this toolchain.
 //
-// Contractions over the d axis against W2 (G1 = G2 W2^T) need W2 tiles with d in the k position;
-// the accumulator layout has it across lanes, so those operand tiles are transposed on the matrix
-// pipe (one 16x16x16 MFMA against an identity fragment each).
+// Operands that are needed with their axes exchanged.  What lies in LDS anyway (the staged rows of XK, G2) or is not waited
+// for (X2 at d = 96) is read with the transposing LDS load.  W2 tiles with d in the k position (G1 = G2 W2^T) and G1 are
+// transposed on the matrix pipe, one 16x16x16 MFMA against an identity fragment each: G1 is on the chain, where a round trip
+// through LDS takes longer, and for W2 (74 KB at d = 96) LDS has no room beside the partial tiles.  (Shared by the two kinds
+// of partial tile, it has: 726 us, the waits for the region cost what the transposes save.)
 #pragma once
 #include "ttt_engine_fwd.hip.h"
 #include "ttt_linear_fwd_mw.hip.h"
@@ -38,22 +46,27 @@ namespace ttt {
 template <int D, int ES>
 struct MlpRrLds {
   static constexpr int NW = 8, NT = D / 16;
+  static constexpr int XS = D > 64 ? 2 : 0;   // hidden tiles of a wave whose X2 is transposed by LDS: as many as there is room for
   static constexpr int TILE = 16 * D * ES;    // one [16 x d] input tile, rows unpadded
   static constexpr int IN1 = 3 * TILE;        // xq, xk, xv tiles of one mini-batch
   static constexpr int IN = 0;                // [3 buffers][3][16][d]
   static constexpr int LR = IN + 3 * IN1;     // [3][16] floats
-  static constexpr int P1 = LR + 3 * 64 + 64;  // [NW][NT][64] f32x4: partial Z2^T tiles
+  static constexpr int PRM = LR + 3 * 64 + 64;  // gamma[d], beta[d], b1[4d] floats
+  static constexpr int EX = PRM + 6 * D * 4;    // [6 sums][2][16 tokens] f32x4 (reducer index % 4)
+  static constexpr int EXO = EX + 6 * 2 * 16 * 16;      // [2 sums][2][16 tokens] f32x4 (output tile % 4)
+  static constexpr int P1 = EXO + 2 * 2 * 16 * 16;  // [NW][NT][64] f32x4: partial Z2^T tiles
   static constexpr int P2 = P1 + NW * NT * 1024;  // partial Zbar2^T tiles
   static constexpr int PA = P2 + NW * NT * 1024;  // [NW][64] f32x4: partial A2^T
-  static constexpr int EX = PA + NW * 1024;       // [8 sums][2][16 tokens] f32x4 (reducer index % 4)
-  static constexpr int GT = EX + 8 * 2 * 16 * 16;  // [NT][64] frag: G2^T tiles (d along k)
-  static constexpr int GD = GT + NT * 64 * 4 * ES;  // [NT][64] frag: G2 tiles (tokens along k)
-  static constexpr int KD = GD + NT * 64 * 4 * ES;  // [2][NT][64] frag: XK tiles (tokens along k)
-  static constexpr int PRM = KD + 2 * NT * 64 * 4 * ES;  // gamma[d], beta[d], b1[4d] floats
-  static constexpr int EXO = PRM + (2 * D + 4 * D) * 4;    // [2 sums][2][16 tokens] f32x4 (output tile % 4)
-  static constexpr int BYTES = EXO + 2 * 2 * 16 * 16;
+  static constexpr int ZB = PA + NW * 1024;       // [NT][64] f32x4: Zbar2^T tiles of the previous mini-batch
+  static constexpr int GT = ZB + NT * 1024;       // [2][NT][64] frag: G2^T tiles (d along k)
+  static constexpr int X2S = GT + 2 * NT * 64 * 4 * ES;  // [NW][XS][64] frag: X2^T tiles
+  static constexpr int M1 = X2S + NW * XS * 64 * 4 * ES;  // [2][64] frag: M1 of this mini-batch
+  static constexpr int ID = M1 + 2 * 64 * 4 * ES;  // [64] frag: identity
+  static constexpr int RHO = ID + 64 * 4 * ES;  // [16] token_eta / sc
+  static constexpr int BYTES = RHO + 64;
   static_assert(BYTES <= 160 * 1024, "exceeds the 160 KiB of LDS of a gfx950 CU");
   static_assert(NT <= NW && D % 32 == 0, "one reducer wave per d-feature tile");
+  static_assert(ES == 2, "the transposing LDS load takes 16-bit elements");
   static_assert(TILE % 1024 == 0 && P1 % 16 == 0, "input tiles are staged in 1 KiB wave blocks");
 };
 
@@ -99,11 +112,40 @@ __device__ __forceinline__ float mean_of(const float* p, int d, float inv_d) {
   return s;
 }
 
+// A fragment's transpose: element (m, k) of the tile that lies in LDS as a fragment (lane order) -> the fragment with the
+// two axes exchanged.  Within each group of sixteen lanes the instruction takes four rows of sixteen elements, a row from
+// four lanes, and gives every lane a column.
+__device__ __forceinline__ bf16x4 read_tr(const void* p) {
+  typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
+  return __builtin_bit_cast(bf16x4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)p));
+}
+// the lane whose fragment starts the row that this lane supplies
+__device__ __forceinline__ int tr_lane(int lane) { return (lane & 3) * 16 + (lane >> 4) * 4 + ((lane >> 2) & 3); }
+
+// All of v in registers here: loads that feed v are issued together and waited for once.  (Short of registers the scheduler
+// otherwise loads, waits and uses them one at a time, an LDS round trip each.)
+template <int N>
+__device__ __forceinline__ void together(f32x4 (&v)[N]) {
+  if constexpr (N == 4) asm volatile("" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]));
+  if constexpr (N == 8)
+    asm volatile("" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]), "+v"(v[4]), "+v"(v[5]), "+v"(v[6]), "+v"(v[7]));
+}
+
 // The LDS addresses derived from the lane index are many (the regions span 150 KiB, beyond the
 // 64 KiB reach of an instruction offset) and all loop-invariant: hoisted out of the loop they are
 // spilled and reloaded from scratch.  Hiding the lane index from the optimiser at the start of each
-// phase makes them cheap phase-local recomputations instead.
-#define RELANE() asm volatile("" : "+v"(lane))
+// phase makes them cheap phase-local recomputations instead.  At d = 96 the lane coordinates and the constant operands
+// (identity, rho) are formed anew or read from LDS as well: held in registers they spill, and a reload from scratch waits for
+// the copies in flight (871 against 770 us); at d <= 64 there is room for them (471 against 434 us).
+#define RELANE()                               \
+  do {                                         \
+    asm volatile("" : "+v"(lane));             \
+    if constexpr (D > 64) {                    \
+      c = lane & 15;                           \
+      g = lane >> 4;                           \
+      own = own_offset<1>(red ? w : 0, 0, g);  \
+    }                                          \
+  } while (0)
 
 // SAVE: also leave what a backward starts from (MlpFwdArgs::fac_save or G1_save).  A compilation of its own: the pointers
 // and branches cost the plain forward 3 % of its time in registers.
@@ -123,7 +165,7 @@ __global__ void __launch_bounds__(512) ttt_mlp_fwd_rr_kernel(Problems<MlpFwdArgs
   // the wave index is read through an SGPR so that everything keyed on it is scalar control flow
   const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   int lane = tid & 63;  // refreshed (see RELANE) at every phase of the main loop
-  const int c = lane & 15, g = lane >> 4;
+  int c = lane & 15, g = lane >> 4;
   const size_t bh = blockIdx.x;
   const int h = (int)(bh % a.H), K = a.K;
   const bool red = w < NT;  // this wave reduces d-feature tile w
@@ -133,9 +175,12 @@ __global__ void __launch_bounds__(512) ttt_mlp_fwd_rr_kernel(Problems<MlpFwdArgs
   f32x4* const PA = reinterpret_cast<f32x4*>(smem + L::PA);
   float* const EX = reinterpret_cast<float*>(smem + L::EX);
   float* const EXO = reinterpret_cast<float*>(smem + L::EXO);
+  frag* const IDs = reinterpret_cast<frag*>(smem + L::ID);
+  float* const RHO = reinterpret_cast<float*>(smem + L::RHO);
+  frag* const M1s = reinterpret_cast<frag*>(smem + L::M1);
+  f32x4* const ZB = reinterpret_cast<f32x4*>(smem + L::ZB);
   frag* const GT = reinterpret_cast<frag*>(smem + L::GT);
-  frag* const GD = reinterpret_cast<frag*>(smem + L::GD);
-  frag* const KD = reinterpret_cast<frag*>(smem + L::KD);
+  frag* const X2S = reinterpret_cast<frag*>(smem + L::X2S) + w * L::XS * 64;
   uint32_t* const LRs = reinterpret_cast<uint32_t*>(smem + L::LR);
   float* const GAM = reinterpret_cast<float*>(smem + L::PRM);
   float* const BET = GAM + D;
@@ -145,11 +190,12 @@ __global__ void __launch_bounds__(512) ttt_mlp_fwd_rr_kernel(Problems<MlpFwdArgs
   const float te_last = a.token_eta[K - 1];
   const bool upd = te_last != 0.f;
   const float sc = upd ? te_last : 1.f;
-  const float rho_c = (c < K) ? a.token_eta[c] / sc : 0.f;
-  const frag ident = identity_frag<T>(c, g);
-  const frag ones = splat_frag<T>(1.f);
+  const float rho_r = (c < K) ? a.token_eta[c] / sc : 0.f;
+  const frag ident_r = identity_frag<T>(c, g);
+  auto rho = [&]() { return D > 64 ? RHO[c] : rho_r; };
+  auto identity = [&]() { return D > 64 ? IDs[lane] : ident_r; };
   const size_t sb = a.state_per_batch ? bh : (size_t)h;
-  const int own = own_offset<1>(red ? w : 0, 0, g);  // first of this lane's four features of tile w
+  int own = own_offset<1>(red ? w : 0, 0, g);  // first of this lane's four features of tile w
 
   // ---- state and parameters
   f32x4 W1c[NT][HT], W2c[HT][NT];
@@ -170,6 +216,8 @@ __global__ void __launch_bounds__(512) ttt_mlp_fwd_rr_kernel(Problems<MlpFwdArgs
   }
   f32x4 b2T;
   float sum_a = 0.f;
+  if (tid < 16) RHO[tid] = tid < K ? a.token_eta[tid] / sc : 0.f;
+  if (w == 0) IDs[lane] = identity_frag<T>(c, g);
 #pragma unroll
   for (int r = 0; r < 4; ++r) b2T[r] = a.b2_0[sb * D + own + r];
   // the second layer is carried centred (see row_means16)
@@ -181,6 +229,7 @@ __global__ void __launch_bounds__(512) ttt_mlp_fwd_rr_kernel(Problems<MlpFwdArgs
   }
   b2T -= mean_of(a.b2_0 + sb * D, D, inv_d);
   for (int f = 0; f < D; ++f) sum_a += a.gamma[h * D + f] * a.gamma[h * D + f];
+  sum_a = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(sum_a)));
   for (int i = tid; i < D; i += 512) {
     GAM[i] = a.gamma[h * D + i];
     BET[i] = a.beta[h * D + i];
@@ -192,48 +241,49 @@ __global__ void __launch_bounds__(512) ttt_mlp_fwd_rr_kernel(Problems<MlpFwdArgs
   // whose token is past a short mini-batch are masked off and their LDS rows keep the zeros
   // written below.  Three buffers: mini-batch st+1 is fetched while st is computed, and rows of
   // st are still read (for the W1 update) after the slowest wave has started st+1's fetch.
+  // Per wave block a running source address, scalar like everything but the lane's offset.
   constexpr int NBLK = L::IN1 / 1024, NBI = (NBLK + NW - 1) / NW;
-  int goff[NBI];
+  const unsigned lds0 = __builtin_amdgcn_readfirstlane((unsigned)(size_t)(__attribute__((address_space(3))) unsigned char*)smem);
+  const unsigned step = (unsigned)(K * D * ES);
+  const unsigned char* srcp[NBI];
 #pragma unroll
   for (int it = 0; it < NBI; ++it) {
-    const int rem = (1024 * (w + NW * it) + 16 * lane) % L::TILE, tok = rem / (D * ES);
-    goff[it] = (tok < K) ? rem : -1;
+    const int b = w + NW * it, ten = (1024 * b) / L::TILE;
+    srcp[it] = static_cast<const unsigned char*>(ten == 0 ? a.xq : ten == 1 ? a.xk : a.xv) + bh * (size_t)a.seq_stride * (D * ES);
   }
+  const unsigned char* lrp = static_cast<const unsigned char*>(a.lr) + bh * (size_t)a.seq_stride * ES;
+  unsigned char* const outp = static_cast<unsigned char*>(a.out) + bh * (size_t)a.seq_stride * (D * ES);
+  unsigned fdst = lds0 + L::IN + 1024 * w, flr = lds0 + L::LR;  // where the next mini-batch goes
+  const int n_stages = a.n_stages;
   auto fetch = [&](int stage) {
-    if (stage >= a.n_stages) return;
-    unsigned char* dst = smem + L::IN + (stage % 3) * L::IN1;
-    const size_t tok0 = (bh * (size_t)a.seq_stride + (size_t)stage * K) * D * ES;
+    if (stage >= n_stages) return;
 #pragma unroll
     for (int it = 0; it < NBI; ++it) {
-      const int b = w + NW * it;  // wave-uniform
-      if (b < NBLK) {
-        const int ten = (1024 * b) / L::TILE;
-        const unsigned char* src =
-            static_cast<const unsigned char*>(ten == 0 ? a.xq : ten == 1 ? a.xk : a.xv) + tok0;
-        if (goff[it] >= 0)
-          lds_dma16(src, (unsigned)goff[it], (unsigned)(size_t)(__attribute__((address_space(3))) unsigned char*)(dst + 1024 * b));
-      }
+      const int b = w + NW * it;
+      const unsigned off = (1024u * b) % L::TILE + 16u * lane;
+      if (b < NBLK && off < step) lds_dma16(srcp[it], off, fdst + 1024 * NW * it);
+      srcp[it] += step;
     }
     // lr as zero-extended bf16 words, copied like the tiles (a register load here would make the compiler
     // wait for every copy in flight); absent tokens read a clamped position and are zeroed at use
-    if (tid < 16)
-      lds_dma2(static_cast<const elem*>(a.lr) + bh * (size_t)a.seq_stride + (size_t)stage * K, 2u * (unsigned)(tid < K ? tid : K - 1),
-               (unsigned)(size_t)(__attribute__((address_space(3))) uint32_t*)(LRs + (stage % 3) * 16));
+    if (w == 0 && lane < 16) lds_dma2(lrp, 2u * (unsigned)min(lane, K - 1), flr);
+    lrp += K * ES;
+    const bool wrap = stage % 3 == 2;
+    fdst += wrap ? -2 * L::IN1 : L::IN1;
+    flr += wrap ? -128 : 64;
   };
   // staged row of token c of tensor ten (0 xq, 1 xk, 2 xv)
   auto row = [&](int buf, int ten) -> const elem* {
     return reinterpret_cast<const elem*>(smem + L::IN + buf * L::IN1 + ten * L::TILE) + c * D;
   };
 
-  for (int i = tid; i < (L::P1 - L::IN) / 4; i += 512) reinterpret_cast<float*>(smem)[i] = 0.f;
-  for (int i = tid; i < 8 * 2 * 16 * 4; i += 512) EX[i] = 0.f;
+  for (int i = tid; i < (L::PRM - L::IN) / 4; i += 512) reinterpret_cast<float*>(smem)[i] = 0.f;
+  for (int i = tid; i < 6 * 2 * 16 * 4; i += 512) EX[i] = 0.f;
   if (tid < 2 * 2 * 16 * 4) EXO[tid] = 0.f;
   __syncthreads();
   fetch(0);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
-
-  // pending output of the previous mini-batch (reducers)
 
   // ---- reducers: lane group g publishes sums g and g + 4 (six in all) of reducer w
   auto publish = [&](const float (&S)[6]) {
@@ -242,97 +292,148 @@ __global__ void __launch_bounds__(512) ttt_mlp_fwd_rr_kernel(Problems<MlpFwdArgs
     EX[(((g)*2 + (w >> 2)) * 16 + c) * 4 + (w & 3)] = v0;
     if (g < 2) EX[(((g + 4) * 2 + (w >> 2)) * 16 + c) * 4 + (w & 3)] = v1;
   };
-  auto collect = [&](int i) -> float {
-    const f32x4 lo = *reinterpret_cast<const f32x4*>(EX + ((i * 2 + 0) * 16 + c) * 4);
-    float s = (lo[0] + lo[1]) + (lo[2] + lo[3]);
+  // sums i and j of those exchanged at ex
+  auto collect2 = [&](const float* ex, int i, int j, float& a, float& b) {
+    f32x4 v[4] = {};
+    v[0] = *reinterpret_cast<const f32x4*>(ex + ((i * 2 + 0) * 16 + c) * 4);
+    v[1] = *reinterpret_cast<const f32x4*>(ex + ((j * 2 + 0) * 16 + c) * 4);
     if (NT > 4) {
-      const f32x4 hi = *reinterpret_cast<const f32x4*>(EX + ((i * 2 + 1) * 16 + c) * 4);
-      s += (hi[0] + hi[1]) + (hi[2] + hi[3]);
+      v[2] = *reinterpret_cast<const f32x4*>(ex + ((i * 2 + 1) * 16 + c) * 4);
+      v[3] = *reinterpret_cast<const f32x4*>(ex + ((j * 2 + 1) * 16 + c) * 4);
     }
-    return s;
+    together(v);
+    a = (v[0][0] + v[0][1]) + (v[0][2] + v[0][3]);
+    b = (v[1][0] + v[1][1]) + (v[1][2] + v[1][3]);
+    if (NT > 4) {
+      a += (v[2][0] + v[2][1]) + (v[2][2] + v[2][3]);
+      b += (v[3][0] + v[3][1]) + (v[3][2] + v[3][3]);
+    }
   };
 
-  // ---- output path: finishing the OUTPUT of the previous mini-batch is spread over the waves with
-  // the most slack: d-feature tile I goes to wave (NT + I) % NW, i.e. first to the waves that reduce
-  // no Z2 tile, then to reducers 0, 1, ...  Each wave has at most one output tile.
-  const int otile = (w - NT + NW) % NW;  // this wave's output tile
-  const bool outw = otile < NT;
-  const int ooff = own_offset<1>(outw ? otile : 0, 0, g);
-  f32x4 zb = {0.f, 0.f, 0.f, 0.f};
-  // part 1 (before B2): Zbar2^T tile from the split-k partials, causal correction, row moments
-  auto output_reduce = [&]() {
-    f32x4 at = {0.f, 0.f, 0.f, 0.f};
+  // ---- output path.  The waves that reduce no Z2 tile (w >= NT) finish the previous mini-batch's Zbar2 beside the
+  // reducers' chain, wave w the tiles (w - NT) + (NW - NT) i: sums over the split-k partials in phase B, causal
+  // correction and row moments in phase C.  The reducers store it, a tile each, in phase D.  (By reducers as well, the
+  // older wave of each SIMD after its own tile, both phases took 0.8 k cycles longer.)
+  constexpr int NOW = NW - NT, OPW = (NT + NOW - 1) / NOW;
+  f32x4 zo[OPW];
+  frag m2f = IO::zero();
+  auto otile = [&](int i) { const int I = (w - NT) + NOW * i; return I < NT ? I : 0; };
+  auto output_sum = [&]() {
+    const f32x4* p = P2 + lane;
 #pragma unroll
-    for (int ww = 0; ww < NW; ++ww) at += PA[ww * 64 + lane];
-    pin(at);
+    for (int i = 0; i < OPW; ++i) {
+      const int I = otile(i);
+      f32x4 v[NW];
+#pragma unroll
+      for (int ww = 0; ww < NW; ++ww) v[ww] = p[(ww * NT + I) * 64];
+      together(v);
+      zo[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int ww = 0; ww < NW; ++ww) zo[i] += v[ww];
+    }
+  };
+  // M2[s][t] = (token_eta[t] / sc)(1 + A2[t][s]) for s <= t
+  auto output_m2 = [&]() {
+    const float rho_c = rho();
+    f32x4 at = {0.f, 0.f, 0.f, 0.f};
+    {
+      f32x4 v[NW];
+#pragma unroll
+      for (int ww = 0; ww < NW; ++ww) v[ww] = PA[ww * 64 + lane];
+      together(v);
+#pragma unroll
+      for (int ww = 0; ww < NW; ++ww) at += v[ww];
+    }
     f32x4 m;
 #pragma unroll
     for (int r = 0; r < 4; ++r) m[r] = (4 * g + r <= c) ? rho_c * (1.f + at[r]) : 0.f;
-    zb = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int ww = 0; ww < NW; ++ww) zb += P2[(ww * NT + otile) * 64 + lane];
-    pin(zb);
-    IO::mma(zb, GD[otile * 64 + lane], IO::to_frag(m));  // GD still holds the previous mini-batch's G2
-    float s0 = 0.f, s1 = 0.f;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      s0 += zb[r];
-      s1 += zb[r] * zb[r];
-    }
-    s0 = xg_sum(s0);
-    s1 = xg_sum(s1);
-    if (g == 0) {
-      EXO[((0 * 2 + (otile >> 2)) * 16 + c) * 4 + (otile & 3)] = s0;
-      EXO[((1 * 2 + (otile >> 2)) * 16 + c) * 4 + (otile & 3)] = s1;
-    }
+    m2f = IO::to_frag(m);
   };
-  auto collect_o = [&](int i) -> float {
-    const f32x4 lo = *reinterpret_cast<const f32x4*>(EXO + ((i * 2 + 0) * 16 + c) * 4);
-    float s = (lo[0] + lo[1]) + (lo[2] + lo[3]);
-    if (NT > 4) {
-      const f32x4 hi = *reinterpret_cast<const f32x4*>(EXO + ((i * 2 + 1) * 16 + c) * 4);
-      s += (hi[0] + hi[1]) + (hi[2] + hi[3]);
+  auto output_moments = [&](int stage) {
+    float s[2 * OPW];
+#pragma unroll
+    for (int i = 0; i < OPW; ++i) IO::mma(zo[i], read_tr(GT + (((stage & 1) * NT) + otile(i)) * 64 + tr_lane(lane)), m2f);
+#pragma unroll
+    for (int i = 0; i < OPW; ++i) {
+      s[2 * i] = s[2 * i + 1] = 0.f;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        s[2 * i] += zo[i][r];
+        s[2 * i + 1] += zo[i][r] * zo[i][r];
+      }
     }
-    return s;
+    // lane group g: sum g & 1 of this wave's tile i + g / 2
+#pragma unroll
+    for (int i = 0; i < OPW; i += 2) {
+      const bool two = i + 1 < OPW;
+      const float v = xg_sum4_scatter(s[2 * i], s[2 * i + 1], two ? s[2 * i + 2 * two] : 0.f, two ? s[2 * i + 2 * two + 1] : 0.f);
+      const int I = (w - NT) + NOW * (i + (g >> 1));
+      if (I < NT && (two || g < 2)) EXO[(((g & 1) * 2 + (I >> 2)) * 16 + c) * 4 + (I & 3)] = v;
+    }
+#pragma unroll
+    for (int i = 0; i < OPW; ++i)
+      if ((w - NT) + NOW * i < NT) ZB[((w - NT) + NOW * i) * 64 + lane] = zo[i];
   };
-  // part 2 (after B2): out = xq + gamma (zbar - mu) rstd + beta
-  auto output_emit = [&](int stage) {
-    const float mu = collect_o(0) * inv_d;
-    const float rstd = __builtin_amdgcn_rsqf(fmaxf(collect_o(1) * inv_d - mu * mu, 0.f) + a.eps);
+  // out = xq + gamma (zbar - mu) rstd + beta, tile w
+  auto output_emit = [&](int stage, frag qo) {
+    const f32x4 zb = ZB[w * 64 + lane];
+    float mu, ms;
+    collect2(EXO, 0, 1, mu, ms);
+    mu *= inv_d;
+    const float rstd = __builtin_amdgcn_rsqf(fmaxf(ms * inv_d - mu * mu, 0.f) + a.eps);
     if (c < K) {
-      const f32x4 gam = *reinterpret_cast<const f32x4*>(GAM + ooff), bet = *reinterpret_cast<const f32x4*>(BET + ooff);
-      const frag qo = load4<T>(row(stage % 3, 0) + ooff);
-      elem* po = static_cast<elem*>(a.out) + (bh * (size_t)a.seq_stride + (size_t)stage * K + c) * D + ooff;
+      const f32x4 gam = *reinterpret_cast<const f32x4*>(GAM + own), bet = *reinterpret_cast<const f32x4*>(BET + own);
+      elem* po = reinterpret_cast<elem*>(outp + (size_t)stage * step) + (c * D + own);
       store4<T>(po, IO::to_f32(qo) + bet + gam * ((zb - mu) * rstd));
     }
   };
+  // partial tiles of X W2 over this wave's hidden units, two at a time
+  auto partials = [&](f32x4* P, const frag (&x)[HT], bool bias) {
+    f32x4* p = P + w * NT * 64 + lane;
+#pragma unroll
+    for (int I = 0; I < NT; I += 2) {
+      f32x4 p0 = {0.f, 0.f, 0.f, 0.f}, p1 = p0;
+      if (bias && I == w) p0 = b2T;
+      if (bias && I + 1 == w) p1 = b2T;
+#pragma unroll
+      for (int j = 0; j + 1 < HT; j += 2) {
+        IO::mma2(p0, IO::to_frag(W2c[j][I]), IO::to_frag(W2c[j + 1][I]), x[j], x[j + 1]);
+        IO::mma2(p1, IO::to_frag(W2c[j][I + 1]), IO::to_frag(W2c[j + 1][I + 1]), x[j], x[j + 1]);
+      }
+      if (HT & 1) {
+        IO::mma2(p0, IO::to_frag(W2c[HT - 1][I]), IO::zero(), x[HT - 1], IO::zero());
+        IO::mma2(p1, IO::to_frag(W2c[HT - 1][I + 1]), IO::zero(), x[HT - 1], IO::zero());
+      }
+      p[I * 64] = p0;
+      p[(I + 1) * 64] = p1;
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
 
-  for (int st = 0; st < a.n_stages; ++st) {
-    const int buf = st % 3, par = st & 1;
+  for (int st = 0; st < n_stages; ++st) {
+    const int buf = st % 3;
+    frag* const GTc = GT + (st & 1) * NT * 64;
     RELANE();
     fetch(st + 1);
 
     // ================= phase A: everything that needs only W1, W2 and the inputs
-    f32x4 z1[HT];
-    // XK tile w with tokens along k, for everybody's W1 update
-    if (red) {
-      f32x4 t = {0.f, 0.f, 0.f, 0.f};
-      IO::mma(t, load4<T>(row(buf, 1) + own), ident);
-      KD[(par * NT + w) * 64 + lane] = IO::to_frag(t);
-    }
-    // Z1^T for this wave's hidden units
+    f32x4 z1[HT], zq[HT];
+    // Z1^T and (XQ W1 + b1)^T for this wave's hidden units
 #pragma unroll
-    for (int j = 0; j < HT; ++j) z1[j] = *reinterpret_cast<const f32x4*>(B1s + 16 * (w * HT + j) + 4 * g);
+    for (int j = 0; j < HT; ++j) zq[j] = z1[j] = *reinterpret_cast<const f32x4*>(B1s + 16 * (w * HT + j) + 4 * g);
 #pragma unroll
     for (int q = 0; q < NT / 2; ++q) {
-      frag k0, k1;
+      frag k0, k1, q0, q1;
       IO::load8(row(buf, 1) + 32 * q + 8 * g, true, k0, k1);
+      IO::load8(row(buf, 0) + 32 * q + 8 * g, true, q0, q1);
 #pragma unroll
-      for (int j = 0; j < HT; ++j)
-        IO::mma2(z1[j], IO::to_frag(W1c[2 * q][j]), IO::to_frag(W1c[2 * q + 1][j]), k0, k1);
+      for (int j = 0; j < HT; ++j) {
+        const frag w0 = IO::to_frag(W1c[2 * q][j]), w1 = IO::to_frag(W1c[2 * q + 1][j]);
+        IO::mma2(z1[j], w0, w1, k0, k1);
+        IO::mma2(zq[j], w0, w1, q0, q1);
+      }
       __builtin_amdgcn_sched_barrier(0);
     }
-    const float lrc = (c < K) ? __uint_as_float(LRs[buf * 16 + c] << 16) : 0.f;
     // X2 = gelu(Z1), gelu'(Z1)
     frag x2f[HT];
     f32x4 dg[HT];
@@ -353,32 +454,44 @@ __global__ void __launch_bounds__(512) ttt_mlp_fwd_rr_kernel(Problems<MlpFwdArgs
       asm volatile("" : "+v"(x2f[j]), "+v"(dg[j]));
       __builtin_amdgcn_sched_barrier(0);
     }
-    // partial Z2^T over this wave's hidden units
 #pragma unroll
-    for (int I = 0; I < NT; ++I) {
-      f32x4 p = {0.f, 0.f, 0.f, 0.f};
+    for (int j = 0; j < L::XS; ++j) X2S[j * 64 + lane] = x2f[j];
+    partials(P1, x2f, false);
+    // M1[s][t] = (token_eta[t] / sc)(1 + A1[t][s]) for s <= t.  By wave 3: of the two waves of a SIMD the older runs ahead
+    // and would wait at B1 for 2 k cycles
+    if (w == 3) {
+      const float rho_c = rho();
+      f32x4 At = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int j = 0; j + 1 < HT; j += 2)
-        IO::mma2(p, IO::to_frag(W2c[j][I]), IO::to_frag(W2c[j + 1][I]), x2f[j], x2f[j + 1]);
-      if (HT & 1) IO::mma2(p, IO::to_frag(W2c[HT - 1][I]), IO::zero(), x2f[HT - 1], IO::zero());
-      P1[(w * NT + I) * 64 + lane] = p;
-      __builtin_amdgcn_sched_barrier(0);
+      for (int q = 0; q < NT / 2; ++q) {
+        frag k0, k1, q0, q1;
+        IO::load8(row(buf, 1) + 32 * q + 8 * g, true, k0, k1);
+        IO::load8(row(buf, 0) + 32 * q + 8 * g, true, q0, q1);
+        IO::mma2(At, k0, k1, q0, q1);
+      }
+      f32x4 m;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) m[r] = (4 * g + r <= c) ? rho_c * (1.f + At[r]) : 0.f;
+      M1s[(st & 1) * 64 + lane] = IO::to_frag(m);
     }
     lds_barrier();  // ---- B1
     RELANE();
 
     // ================= phase B: reducers: full Z2 tile and its row moments;
-    //                          output waves: Zbar2 tiles of the previous mini-batch and their moments
+    //                          the other waves: Zbar2 tiles and causal correction of the previous mini-batch
     f32x4 z = {0.f, 0.f, 0.f, 0.f}, bq = z;
+    frag qo = IO::zero();
     if (red) {
-      z = b2T;
-#pragma unroll
-      for (int ww = 0; ww < NW; ++ww) {
-        z += P1[(ww * NT + w) * 64 + lane];
-        if ((ww & 3) == 3) pin(z);
-      }
+      const f32x4* p = P1 + w * 64 + lane;
       const frag ko = load4<T>(row(buf, 1) + own), vo = load4<T>(row(buf, 2) + own);
       const f32x4 gam = *reinterpret_cast<const f32x4*>(GAM + own), bet = *reinterpret_cast<const f32x4*>(BET + own);
+      f32x4 v[NW];
+#pragma unroll
+      for (int ww = 0; ww < NW; ++ww) v[ww] = p[ww * NT * 64];
+      together(v);
+      z = b2T;
+#pragma unroll
+      for (int ww = 0; ww < NW; ++ww) z += v[ww];
       bq = gam * (bet - (IO::to_f32(vo) - IO::to_f32(ko)));
       float S[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
       const f32x4 az = gam * gam * z;
@@ -392,18 +505,35 @@ __global__ void __launch_bounds__(512) ttt_mlp_fwd_rr_kernel(Problems<MlpFwdArgs
         S[5] += bq[r] * z[r];
       }
       publish(S);
+    } else if (st > 0) {
+      output_sum();
+      output_m2();
     }
-    if (outw && st > 0) output_reduce();
     lds_barrier();  // ---- B2
     RELANE();
 
-    // ================= phase C: reducers: G2'' in both orientations; output waves: store the output
+    // ================= phase C: reducers: G2''; the other waves: the rest of Zbar2
     frag g2_saved = IO::zero();
     if (red) {
+      const float lrc = (c < K) ? __uint_as_float(LRs[buf * 16 + c] << 16) : 0.f;
       float S[6];
-#pragma unroll
-      for (int i = 0; i < 6; ++i) {
-        S[i] = collect(i);
+      {
+        // lane group g adds up sums g and 4 + (g & 1), then all groups get all six
+        float v0, v1;
+        collect2(EX, g, 4 + (g & 1), v0, v1);
+        const uint32_t u = __float_as_uint(v0), v = __float_as_uint(v1);
+        const auto p = __builtin_amdgcn_permlane16_swap(u, u, false, false);  // rows: 0 0 2 2 / 1 1 3 3
+        const uint32_t p0 = p[0], p1 = p[1];
+        const auto q = __builtin_amdgcn_permlane32_swap(p0, p0, false, false);
+        const auto r = __builtin_amdgcn_permlane32_swap(p1, p1, false, false);
+        const auto t2 = __builtin_amdgcn_permlane16_swap(v, v, false, false);  // rows: 4 4 4 4 / 5 5 5 5
+        const uint32_t q0 = q[0], q1 = q[1], r0 = r[0], r1 = r[1], t0 = t2[0], t1 = t2[1];
+        S[0] = __uint_as_float(q0);
+        S[2] = __uint_as_float(q1);
+        S[1] = __uint_as_float(r0);
+        S[3] = __uint_as_float(r1);
+        S[4] = __uint_as_float(t0);
+        S[5] = __uint_as_float(t1);
       }
       const float mu = S[0] * inv_d;
       const float var = S[1] * inv_d - mu * mu;
@@ -415,31 +545,25 @@ __global__ void __launch_bounds__(512) ttt_mlp_fwd_rr_kernel(Problems<MlpFwdArgs
       const f32x4 gam = *reinterpret_cast<const f32x4*>(GAM + own);
       const f32x4 G = (z - mu) * (gam * gam * c1 + c2) + (bq * p + c3);
       const frag gt = IO::to_frag(G);
-      f32x4 t = {0.f, 0.f, 0.f, 0.f};
-      IO::mma(t, gt, ident);
-      GT[w * 64 + lane] = gt;
-      GD[w * 64 + lane] = IO::to_frag(t);
+      GTc[w * 64 + lane] = gt;
       g2_saved = gt;
+      if (st > 0) qo = load4<T>(row((st + 2) % 3, 0) + own);
+    } else if (st > 0) {
+      output_moments(st - 1);
     }
-    if (outw && st > 0) output_emit(st - 1);
-    // the next mini-batch's rows must have landed before anybody passes B3; the output store just issued
-    // (the only memory operation younger than the copies, which retire in order) may stay in flight
-    if (outw && st > 0)
-      asm volatile("s_waitcnt vmcnt(1)" ::: "memory");
-    else
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    // the next mini-batch's rows must have landed before anybody passes B3
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     lds_barrier();  // ---- B3
     RELANE();
 
     // ================= phase D: G1, Zbar1, Xbar2, split-k partials of the output path, updates
     // The factors of this mini-batch's state update for ttt_mlp_bwd, eta_last * G1 [16 x 4d] and eta_last * G2
     // [16 x d] (row = token), exactly as the update applies them: rounded to the operand type, sign undone
-    // (G'' = -eta_last * lr * G); zeros when token_eta[K-1] = 0 switches the update off.  Stored behind B3 so
-    // that the counted waits of phase C see the same memory operations as without them.
+    // (G'' = -eta_last * lr * G); zeros when token_eta[K-1] = 0 switches the update off.
     const size_t save_row = (bh * (size_t)a.n_stages + st) * 16 + c;
     unsigned char* const facp =
         SAVE && a.fac_save != nullptr ? a.fac_save + (bh * (size_t)a.n_stages + st) * ((NW * HT + NT) * 512) : nullptr;
-    if (SAVE && facp != nullptr && red) *reinterpret_cast<frag*>(facp + (NW * HT + w) * 512 + lane * 8) = GD[w * 64 + lane];
+    if (SAVE && facp != nullptr && red) *reinterpret_cast<frag*>(facp + (NW * HT + w) * 512 + lane * 8) = read_tr(GTc + w * 64 + tr_lane(lane));
     if (SAVE && a.G2_save != nullptr && red) {
       const f32x4 v = upd ? -IO::to_f32(g2_saved) : f32x4{0.f, 0.f, 0.f, 0.f};
       *reinterpret_cast<f32x4*>(a.G2_save + save_row * D + own) = v;
@@ -448,57 +572,52 @@ __global__ void __launch_bounds__(512) ttt_mlp_fwd_rr_kernel(Problems<MlpFwdArgs
     for (int j = 0; j < HT; ++j)
 #pragma unroll
       for (int I = 0; I < NT; ++I) forget(W2c[j][I]);
+    // G1''^T = (W2 G2''^T) gelu'(Z1)
     frag G1d[HT];
+    {
+      const frag ident = identity();
+      f32x4 acc[HT];
 #pragma unroll
-    for (int j = 0; j < HT; ++j) {
-      f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+      for (int j = 0; j < HT; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int q = 0; q < NT / 2; ++q) {
-        f32x4 t0 = {0.f, 0.f, 0.f, 0.f}, t1 = {0.f, 0.f, 0.f, 0.f};
-        IO::mma(t0, IO::to_frag(W2c[j][2 * q]), ident);
-        IO::mma(t1, IO::to_frag(W2c[j][2 * q + 1]), ident);
-        IO::mma2(acc, IO::to_frag(t0), IO::to_frag(t1), GT[(2 * q) * 64 + lane], GT[(2 * q + 1) * 64 + lane]);
+        const frag g0 = GTc[(2 * q) * 64 + lane], g1 = GTc[(2 * q + 1) * 64 + lane];
+        f32x4 t0[HT], t1[HT];
+#pragma unroll
+        for (int j = 0; j < HT; ++j) {
+          t0[j] = t1[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+          IO::mma(t0[j], IO::to_frag(W2c[j][2 * q]), ident);
+          IO::mma(t1[j], IO::to_frag(W2c[j][2 * q + 1]), ident);
+        }
+#pragma unroll
+        for (int j = 0; j < HT; ++j) IO::mma2(acc[j], IO::to_frag(t0[j]), IO::to_frag(t1[j]), g0, g1);
+        __builtin_amdgcn_sched_barrier(0);
       }
-      f32x4 t = {0.f, 0.f, 0.f, 0.f};
-      const frag g1b = IO::to_frag(acc * dg[j]);
-      IO::mma(t, g1b, ident);
-      G1d[j] = IO::to_frag(t);
-      if (SAVE && facp != nullptr) *reinterpret_cast<frag*>(facp + (w * HT + j) * 512 + lane * 8) = G1d[j];
-      if (SAVE && a.G1_save != nullptr) {
-        const f32x4 v = upd ? -IO::to_f32(g1b) : f32x4{0.f, 0.f, 0.f, 0.f};
-        *reinterpret_cast<f32x4*>(a.G1_save + save_row * F + 16 * (w * HT + j) + 4 * g) = v;
+      f32x4 t[HT];
+#pragma unroll
+      for (int j = 0; j < HT; ++j) {
+        const frag g1b = IO::to_frag(acc[j] * dg[j]);
+        t[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+        IO::mma(t[j], g1b, ident);
+        if (SAVE && a.G1_save != nullptr) {
+          const f32x4 v = upd ? -IO::to_f32(g1b) : f32x4{0.f, 0.f, 0.f, 0.f};
+          *reinterpret_cast<f32x4*>(a.G1_save + save_row * F + 16 * (w * HT + j) + 4 * g) = v;
+        }
       }
-      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int j = 0; j < HT; ++j) {
+        G1d[j] = IO::to_frag(t[j]);
+        if (SAVE && facp != nullptr) *reinterpret_cast<frag*>(facp + (w * HT + j) * 512 + lane * 8) = G1d[j];
+      }
     }
-    // Zbar1^T = (XQ W1 + b1)^T + G1''^T M1, with M1[s][t] = (token_eta[t] / sc)(1 + A1[t][s]) for s <= t.
-    // Computed here rather than next to Z1 so that it does not occupy registers across the barriers.
-#pragma unroll
-    for (int j = 0; j < HT; ++j)
-#pragma unroll
-      for (int I = 0; I < NT; ++I) forget(W1c[I][j]);
-    f32x4 zq[HT], At = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int j = 0; j < HT; ++j) zq[j] = *reinterpret_cast<const f32x4*>(B1s + 16 * (w * HT + j) + 4 * g);
-#pragma unroll
-    for (int q = 0; q < NT / 2; ++q) {
-      frag k0, k1, q0, q1;
-      IO::load8(row(buf, 1) + 32 * q + 8 * g, true, k0, k1);
-      IO::load8(row(buf, 0) + 32 * q + 8 * g, true, q0, q1);
-#pragma unroll
-      for (int j = 0; j < HT; ++j)
-        IO::mma2(zq[j], IO::to_frag(W1c[2 * q][j]), IO::to_frag(W1c[2 * q + 1][j]), q0, q1);
-      IO::mma2(At, k0, k1, q0, q1);
-      __builtin_amdgcn_sched_barrier(0);
-    }
+    // Zbar1^T = (XQ W1 + b1)^T + G1''^T M1
+    frag xbf[HT];
     {
-      f32x4 m;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) m[r] = (4 * g + r <= c) ? rho_c * (1.f + At[r]) : 0.f;
-      const frag Mf = IO::to_frag(m);
+      const frag Mf = M1s[(st & 1) * 64 + lane];
 #pragma unroll
       for (int j = 0; j < HT; ++j) IO::mma(zq[j], G1d[j], Mf);
     }
-    frag xbf[HT];
+    if (red && st > 0) output_emit(st - 1, qo);
 #pragma unroll
     for (int j = 0; j < HT; ++j) {
       f32x4 y;
@@ -518,46 +637,62 @@ __global__ void __launch_bounds__(512) ttt_mlp_fwd_rr_kernel(Problems<MlpFwdArgs
       if (HT & 1) IO::mma2(p, x2f[HT - 1], IO::zero(), xbf[HT - 1], IO::zero());
       PA[w * 64 + lane] = p;
     }
-#pragma unroll
-    for (int I = 0; I < NT; ++I) {
-      f32x4 p = (I == w) ? b2T : f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int j = 0; j + 1 < HT; j += 2)
-        IO::mma2(p, IO::to_frag(W2c[j][I]), IO::to_frag(W2c[j + 1][I]), xbf[j], xbf[j + 1]);
-      if (HT & 1) IO::mma2(p, IO::to_frag(W2c[HT - 1][I]), IO::zero(), xbf[HT - 1], IO::zero());
-      P2[(w * NT + I) * 64 + lane] = p;
-      __builtin_amdgcn_sched_barrier(0);
-    }
+    partials(P2, xbf, true);
     if (upd) {
       frag x2d[HT];
+      {
+        const frag ones = splat_frag<T>(1.f);
+        f32x4 b[HT];
 #pragma unroll
-      for (int j = 0; j < HT; ++j) {
-        f32x4 t = {0.f, 0.f, 0.f, 0.f};
-        IO::mma(t, x2f[j], ident);
-        x2d[j] = IO::to_frag(t);
-        f32x4 b = *reinterpret_cast<const f32x4*>(B1s + 16 * (w * HT + j) + 4 * g);
-        IO::mma(b, G1d[j], ones);
-        if (c == 0) *reinterpret_cast<f32x4*>(B1s + 16 * (w * HT + j) + 4 * g) = b;
+        for (int j = 0; j < HT; ++j) {
+          if (j < L::XS) {
+            x2d[j] = read_tr(X2S + j * 64 + tr_lane(lane));
+          } else {
+            f32x4 t = {0.f, 0.f, 0.f, 0.f};
+            IO::mma(t, x2f[j], identity());
+            x2d[j] = IO::to_frag(t);
+          }
+          b[j] = *reinterpret_cast<const f32x4*>(B1s + 16 * (w * HT + j) + 4 * g);
+        }
+#pragma unroll
+        for (int j = 0; j < HT; ++j) IO::mma(b[j], G1d[j], ones);
+#pragma unroll
+        for (int j = 0; j < HT; ++j)
+          if (c == 0) *reinterpret_cast<f32x4*>(B1s + 16 * (w * HT + j) + 4 * g) = b[j];
       }
+      // XK tiles with tokens along k, straight from the staged rows: lane l supplies four features of token 4g + c / 4
+      const elem* const kr = reinterpret_cast<const elem*>(smem + L::IN + buf * L::IN1 + L::TILE) + (4 * g + (c >> 2)) * D + 8 * (c & 3);
+      const frag* const gr = GTc + tr_lane(lane);
+      frag kd = read_tr(kr), g2d = read_tr(gr);
 #pragma unroll
       for (int I = 0; I < NT; ++I) {
-        const frag kd = KD[(par * NT + I) * 64 + lane], g2d = GD[I * 64 + lane];
+        const int In = I + 1 < NT ? I + 1 : I;
+        const frag kn = read_tr(kr + 32 * (In >> 1) + 4 * (In & 1)), gn = read_tr(gr + (I + 1 < NT ? I + 1 : w < NT ? w : 0) * 64);
 #pragma unroll
         for (int j = 0; j < HT; ++j) {
           IO::mma(W1c[I][j], kd, G1d[j]);
           IO::mma(W2c[j][I], x2d[j], g2d);
         }
+        kd = kn;
+        g2d = gn;
         __builtin_amdgcn_sched_barrier(0);
       }
-      if (red) IO::mma(b2T, GD[w * 64 + lane], ones);
+      if (red) IO::mma(b2T, g2d, splat_frag<T>(1.f));
     }
   }
 
   // ---- the last mini-batch's output
+  frag qo = IO::zero();
   lds_barrier();
-  if (outw) output_reduce();
+  if (!red) {
+    output_sum();
+    output_m2();
+    output_moments(n_stages - 1);
+  } else {
+    qo = load4<T>(row((a.n_stages - 1) % 3, 0) + own);
+  }
   lds_barrier();
-  if (outw) output_emit(a.n_stages - 1);
+  if (red) output_emit(a.n_stages - 1, qo);
 
   if (SAVE && a.state_save != nullptr) {
     f32x4* s1 = reinterpret_cast<f32x4*>(a.state_save + bh * (size_t)(2 * D * F)) + (w * NT * HT) * 64 + lane;
