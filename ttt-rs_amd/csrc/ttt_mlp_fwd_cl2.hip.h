@@ -18,7 +18,7 @@
 // 64-bit word together with a tag (mini-batch index + 1), written and polled with relaxed agent-scope
 // atomics, so a word is either old or complete and the caches are never flushed or invalidated (an
 // agent-scope release / acquire pair per mini-batch cost about 30 us here).  Lane l of wave I only
-// ever waits for lane l of wave I of the other CU.  There is no workspace argument in ttt_mlp_fwd, so
+// ever waits for lane l of wave I of the other CU (A2: wave 2 for wave 2).  There is no workspace argument in ttt_mlp_fwd, so
 // the exchange area is the unit's W2_out buffer, which is not needed until the final state is stored:
 // everything a CU polls lies in the rows of W2_out that this CU itself overwrites at the end, so its
 // final store is ordered after its last read by program order, and the partner never writes there
@@ -28,6 +28,15 @@
 // That placement is checked, not assumed: at start the two workgroups tell each other which XCD they run on
 // (device-scope words), and a pair that sits on two XCDs stores at device scope for the whole launch -- slower,
 // same results.  Every wait is bounded, so a missing partner ends in NaN outputs, never in a hang.
+//
+// What bounds it.  The products by the issue of a SIMD's two waves, as in ttt_mlp_fwd_rr.hip.h; between the first and the
+// second barrier a round trip through the L2, about 1.6 k cycles from the send to the tile in registers.  Cycles of a
+// mini-batch at d = 128 with all 256 CUs at work, before -> after the last revision: A 4.0 -> 5.2 k (XQ W1 moved here, where
+// it shares XK W1's operands), B 8.9 -> 4.0 k, C 1.8 -> 1.1 k, D 5.8 -> 6.7 k (CU 0; CU 1 6.0 k).  What it took in B: one load
+// of the tile when it is needed instead of a watch on one word first, the words of a tile next to each other in each load,
+// loads of a sum issued together, A2 and M1 formed by the older waves, which would wait at the first barrier, and the output
+// finished a phase later, its stores where the waves wait for the partner.  128 units x 2048 tokens: d = 128 1078 -> 826 us,
+// d = 96 838 -> 623 us.
 #pragma once
 #include "ttt_mlp_fwd_rr.hip.h"
 
@@ -43,17 +52,21 @@ struct MlpCl2Lds {
   static constexpr int P1 = LR + 2 * 64 + 128;  // [NW][NT][64] f32x4: partial Z2^T tiles
   static constexpr int P2 = P1 + NW * NT * 1024;  // [NW][NT][64] bf16x4: partial Zbar2^T tiles
   static constexpr int PA = P2 + NW * NT * 512;   // [NW][64] f32x4: partial A2^T
-  static constexpr int EX = PA + NW * 1024;       // [8 sums][2][16 tokens] f32x4
-  static constexpr int GT = EX + 8 * 2 * 16 * 16;
-  static constexpr int GD = GT + NT * 64 * 4 * ES;
-  static constexpr int KD = GD + NT * 64 * 4 * ES;  // [2][NT][64] frag
-  static constexpr int PRM = KD + 2 * NT * 64 * 4 * ES;  // gamma[d], beta[d], b1[FH] floats
-  static constexpr int EXO = PRM + (2 * D + FH) * 4;
-  static constexpr int LOST = EXO + 2 * 2 * 16 * 16;  // one word: a wait for the partner ran out
-  static constexpr int BYTES = LOST + 16;
+  static constexpr int EX = PA + NW * 1024;       // [6 sums][2][16 tokens] f32x4 (reducer index % 4)
+  static constexpr int EXO = EX + 6 * 2 * 16 * 16;
+  static constexpr int GT = EXO + 2 * 2 * 16 * 16;       // [2][NT][64] frag: G2^T tiles
+  static constexpr int X2S = GT + 2 * NT * 64 * 4 * ES;  // [NW][FH / 16 / NW][64] frag: X2^T tiles
+  static constexpr int M1 = X2S + FH / 16 * 64 * 4 * ES;  // [2][64] frag: M1 of this mini-batch
+  static constexpr int M2 = M1 + 2 * 64 * 4 * ES;     // [64] frag: M2 of the previous one
+  static constexpr int ID = M2 + 64 * 4 * ES;     // [64] frag: identity
+  static constexpr int RHO = ID + 64 * 4 * ES;    // [16] token_eta / sc
+  static constexpr int PRM = RHO + 64;            // gamma[d], beta[d], b1[FH] floats
+  static constexpr int LOST = PRM + (2 * D + FH) * 4;  // one word: a wait for the partner ran out
+  static constexpr int FL = LOST + 16;            // [NW] counters
+  static constexpr int BYTES = FL + 32;
   static_assert(BYTES <= 160 * 1024, "exceeds the 160 KiB of LDS of a gfx950 CU");
   static_assert(NT == NW && NW <= 8 && D % 32 == 0 && ES == 2, "one reducer and one output tile per wave, bf16 I/O");
-  static_assert(FH % (16 * NW) == 0, "whole hidden tiles per wave");
+  static_assert(FH % (32 * NW) == 0, "an even number of hidden tiles per wave");
   static_assert(TILE % 1024 == 0 && P1 % 16 == 0, "input tiles are staged in 1 KiB wave blocks");
   // exchange area inside this CU's rows of W2_out (bytes): two parities of X1 tiles, X2 tiles, A2 tile,
   // each tile as 64 lanes x 4 tagged 64-bit words
@@ -62,7 +75,7 @@ struct MlpCl2Lds {
   static_assert(XHELLO + 16 <= FH * D * 4, "exchange area exceeds this CU's rows of W2_out");
 };
 
-// One [16 x 16] f32 tile (this lane's four values) as four (value, tag) words.
+// One [16 x 16] f32 tile (this lane's four values) as four (value, tag) words, value r of lane l at word 64 r + l.
 // The two workgroups of a pair sit on CUs of one XCD (see the block numbering in the kernel), which share an L2.
 // The stores therefore carry workgroup scope: they leave the CU (its L1 writes through) and stay in that L2, where
 // the partner's device-scope loads, which bypass its own L1, find them.  Device-scope stores would also be written
@@ -73,60 +86,52 @@ __device__ __forceinline__ void send_tagged(unsigned long long* slot, f32x4 v, u
   if (same_xcd) {
 #pragma unroll
     for (int r = 0; r < 4; ++r)
-      __hip_atomic_store(slot + r, ((unsigned long long)tag << 32) | __float_as_uint(v[r]), __ATOMIC_RELAXED,
+      __hip_atomic_store(slot + 64 * r, ((unsigned long long)tag << 32) | __float_as_uint(v[r]), __ATOMIC_RELAXED,
                          __HIP_MEMORY_SCOPE_WORKGROUP);
   } else {
 #pragma unroll
     for (int r = 0; r < 4; ++r)
-      __hip_atomic_store(slot + r, ((unsigned long long)tag << 32) | __float_as_uint(v[r]), __ATOMIC_RELAXED,
+      __hip_atomic_store(slot + 64 * r, ((unsigned long long)tag << 32) | __float_as_uint(v[r]), __ATOMIC_RELAXED,
                          __HIP_MEMORY_SCOPE_AGENT);
   }
 }
-// Receives N tiles at once: polls until the four words of every slot carry that slot's tag, all
-// loads of a round in flight together (one memory round trip per round, not one per tile).  The wait
-// is bounded; after one wait has run out (`alive` cleared) no further wait is attempted: a lost
-// partner costs one time-out per wave, not one per mini-batch, and ends in NaNs in b1_out, never in a hang.
-template <int N>
-__device__ __forceinline__ void recv_tagged(const unsigned long long* const (&slot)[N], const unsigned (&tag)[N],
-                                            f32x4 (&out)[N], bool& alive, int spin_limit) {
-  unsigned long long wd[N][4];
-  int it = 0;
-  // light first stage: one lane watches the word stored last of the first slot, so that sixteen
-  // waiting waves do not flood the memory system with polls; the full check then usually passes at once
-  if (alive && (threadIdx.x & 63) == 0) {
-    const unsigned long long* last = slot[0] + 4 * 63 + 3;  // lane 63's fourth word (slot[] is lane 0's here)
-    while ((unsigned)(__hip_atomic_load(last, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >> 32) != tag[0]) {
-      if (++it >= spin_limit) break;
-      __builtin_amdgcn_s_sleep(1);
-    }
+// A tile on its way in: the four words as last loaded.
+struct Inbound {
+  unsigned long long wd[4];
+  __device__ __forceinline__ void load(const unsigned long long* slot) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) wd[r] = __hip_atomic_load(slot + 64 * r, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
-  it = 0;
-  while (true) {
-    bool ok = true;
+  // Loads again until the four words of every lane carry the tag.  The wait is bounded; after one wait has run out
+  // (`alive` cleared) no further wait is attempted: a lost partner costs one time-out per wave, not one per
+  // mini-batch, and ends in NaN outputs, never in a hang.
+  __device__ __forceinline__ f32x4 wait(const unsigned long long* slot, unsigned tag, bool& alive, int spin_limit) {
+    int it = 0;
+    while (true) {
+      bool ok = true;
 #pragma unroll
-    for (int n = 0; n < N; ++n)
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        wd[n][r] = __hip_atomic_load(slot[n] + r, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-#pragma unroll
-    for (int n = 0; n < N; ++n)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) ok = ok && (unsigned)(wd[n][r] >> 32) == tag[n];
-    // the whole wave leaves together: its lanes poll neighbouring words of the same tiles
-    if (__all(ok) || !alive) break;
-    if (++it >= spin_limit) {
-      alive = false;
-      break;
+      for (int r = 0; r < 4; ++r) ok = ok && (unsigned)(wd[r] >> 32) == tag;
+      // the whole wave leaves together: its lanes poll neighbouring words of the same tile
+      if (__all(ok) || !alive) break;
+      if (++it >= spin_limit) {
+        alive = false;
+        break;
+      }
+      load(slot);
     }
-    __builtin_amdgcn_s_sleep(1);
+    return f32x4{__uint_as_float((unsigned)wd[0]), __uint_as_float((unsigned)wd[1]), __uint_as_float((unsigned)wd[2]),
+                 __uint_as_float((unsigned)wd[3])};
   }
-#pragma unroll
-  for (int n = 0; n < N; ++n)
-    out[n] = f32x4{__uint_as_float((unsigned)wd[n][0]), __uint_as_float((unsigned)wd[n][1]),
-                   __uint_as_float((unsigned)wd[n][2]), __uint_as_float((unsigned)wd[n][3])};
-}
+};
 
-#define RELANE() asm volatile("" : "+v"(lane))
+// see ttt_mlp_fwd_rr.hip.h: lane coordinates and constants held across the loop spill here as well (62 registers)
+#define RELANE()                       \
+  do {                                 \
+    asm volatile("" : "+v"(lane));     \
+    c = lane & 15;                     \
+    g = lane >> 4;                     \
+    own = own_offset<1>(w, 0, g);      \
+  } while (0)
 
 template <class T, int D>
 __global__ void __launch_bounds__(64 * (D / 16)) ttt_mlp_fwd_cl2_kernel(Problems<MlpFwdArgs> problems) {
@@ -142,7 +147,7 @@ __global__ void __launch_bounds__(64 * (D / 16)) ttt_mlp_fwd_cl2_kernel(Problems
 
   const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   int lane = tid & 63;
-  const int c = lane & 15, g = lane >> 4;
+  int c = lane & 15, g = lane >> 4;
   // blocks (i, i + 8) of every group of sixteen form a pair
   const int blk = blockIdx.x;
   const int cu = (blk >> 3) & 1;
@@ -159,8 +164,12 @@ __global__ void __launch_bounds__(64 * (D / 16)) ttt_mlp_fwd_cl2_kernel(Problems
   float* const EX = reinterpret_cast<float*>(smem + L::EX);
   float* const EXO = reinterpret_cast<float*>(smem + L::EXO);
   frag* const GT = reinterpret_cast<frag*>(smem + L::GT);
-  frag* const GD = reinterpret_cast<frag*>(smem + L::GD);
-  frag* const KD = reinterpret_cast<frag*>(smem + L::KD);
+  frag* const X2S = reinterpret_cast<frag*>(smem + L::X2S) + w * HT * 64;
+  frag* const M1s = reinterpret_cast<frag*>(smem + L::M1);
+  frag* const M2s = reinterpret_cast<frag*>(smem + L::M2);
+  frag* const IDs = reinterpret_cast<frag*>(smem + L::ID);
+  volatile int* const FL = reinterpret_cast<volatile int*>(smem + L::FL);
+  float* const RHO = reinterpret_cast<float*>(smem + L::RHO);
   uint32_t* const LRs = reinterpret_cast<uint32_t*>(smem + L::LR);
   float* const GAM = reinterpret_cast<float*>(smem + L::PRM);
   float* const BET = GAM + D;
@@ -183,11 +192,11 @@ __global__ void __launch_bounds__(64 * (D / 16)) ttt_mlp_fwd_cl2_kernel(Problems
   const float te_last = a.token_eta[K - 1];
   const bool upd = te_last != 0.f;
   const float sc = upd ? te_last : 1.f;
-  const float rho_c = (c < K) ? a.token_eta[c] / sc : 0.f;
-  const frag ident = identity_frag<T>(c, g);
-  const frag ones = splat_frag<T>(1.f);
+  if (tid < 8) FL[tid] = tid < NW ? 0 : 0x7fffffff;
+  if (tid < 16) RHO[tid] = tid < K ? a.token_eta[tid] / sc : 0.f;
+  if (w == 0) IDs[lane] = identity_frag<T>(c, g);
   const size_t sb = a.state_per_batch ? bh : (size_t)h;
-  const int own = own_offset<1>(w, 0, g);  // first of this lane's four features of d-feature tile w
+  int own = own_offset<1>(w, 0, g);  // first of this lane's four features of d-feature tile w
 
   // ---- state and parameters
   f32x4 W1c[NT][HT], W2c[HT][NT];
@@ -219,6 +228,7 @@ __global__ void __launch_bounds__(64 * (D / 16)) ttt_mlp_fwd_cl2_kernel(Problems
   }
   b2T -= mean_of(a.b2_0 + sb * D, D, inv_d);
   for (int f = 0; f < D; ++f) sum_a += a.gamma[h * D + f] * a.gamma[h * D + f];
+  sum_a = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(sum_a)));
   for (int i = tid; i < D; i += NTHR) {
     GAM[i] = a.gamma[h * D + i];
     BET[i] = a.beta[h * D + i];
@@ -228,40 +238,41 @@ __global__ void __launch_bounds__(64 * (D / 16)) ttt_mlp_fwd_cl2_kernel(Problems
   // ---- staging of the xq / xk / xv rows: global -> LDS, two buffers.  The fetch of mini-batch st+1 is
   // issued after the first barrier of mini-batch st (every wave has then finished reading the buffer it
   // overwrites) and has landed before the third.
+  // Per wave block a running source address, scalar like everything but the lane's offset.
   constexpr int NBLK = L::IN1 / 1024, NBI = (NBLK + NW - 1) / NW;
-  int goff[NBI];
+  const unsigned lds0 = __builtin_amdgcn_readfirstlane((unsigned)(size_t)(__attribute__((address_space(3))) unsigned char*)smem);
+  const unsigned step = (unsigned)(K * D * ES);
+  const size_t unit0 = bh * (size_t)a.seq_stride * (D * ES);
+  const unsigned char* srcp[NBI];
 #pragma unroll
   for (int it = 0; it < NBI; ++it) {
-    const int rem = (1024 * (w + NW * it) + 16 * lane) % L::TILE, tok = rem / (D * ES);
-    goff[it] = (tok < K) ? rem : -1;
+    const int b = w + NW * it, ten = (1024 * b) / L::TILE;
+    srcp[it] = static_cast<const unsigned char*>(ten == 0 ? a.xq : ten == 1 ? a.xk : a.xv) + unit0;
   }
+  const unsigned char* lrp = static_cast<const unsigned char*>(a.lr) + bh * (size_t)a.seq_stride * ES;
+  unsigned char* const outp = static_cast<unsigned char*>(a.out) + unit0;
+  const int n_stages = a.n_stages;
   auto fetch = [&](int stage) {
-    if (stage >= a.n_stages) return;
-    unsigned char* dst = smem + L::IN + (stage & 1) * L::IN1;
-    const size_t tok0 = (bh * (size_t)a.seq_stride + (size_t)stage * K) * D * ES;
+    if (stage >= n_stages) return;
+    const unsigned dst = lds0 + L::IN + (stage & 1) * L::IN1 + 1024 * w;
 #pragma unroll
     for (int it = 0; it < NBI; ++it) {
-      const int b = w + NW * it;  // wave-uniform
-      if (b < NBLK) {
-        const int ten = (1024 * b) / L::TILE;
-        const unsigned char* src =
-            static_cast<const unsigned char*>(ten == 0 ? a.xq : ten == 1 ? a.xk : a.xv) + tok0;
-        if (goff[it] >= 0)
-          lds_dma16(src, (unsigned)goff[it], (unsigned)(size_t)(__attribute__((address_space(3))) unsigned char*)(dst + 1024 * b));
-      }
+      const int b = w + NW * it;
+      const unsigned off = (1024u * b) % L::TILE + 16u * lane;
+      if (b < NBLK && off < step) lds_dma16(srcp[it], off, dst + 1024 * NW * it);
+      srcp[it] += step;
     }
     // lr as zero-extended bf16 words, copied like the tiles (a register load here would make the compiler
     // wait for every copy in flight); absent tokens read a clamped position and are zeroed at use
-    if (tid < 16)
-      lds_dma2(static_cast<const elem*>(a.lr) + bh * (size_t)a.seq_stride + (size_t)stage * K, 2u * (unsigned)(tid < K ? tid : K - 1),
-               (unsigned)(size_t)(__attribute__((address_space(3))) uint32_t*)(LRs + (stage & 1) * 16));
+    if (w == 0 && lane < 16) lds_dma2(lrp, 2u * (unsigned)min(lane, K - 1), lds0 + L::LR + (stage & 1) * 64);
+    lrp += K * ES;
   };
   auto row = [&](int buf, int ten) -> const elem* {
     return reinterpret_cast<const elem*>(smem + L::IN + buf * L::IN1 + ten * L::TILE) + c * D;
   };
 
   for (int i = tid; i < (L::P1 - L::IN) / 4; i += NTHR) reinterpret_cast<float*>(smem)[i] = 0.f;
-  for (int i = tid; i < 8 * 2 * 16 * 4; i += NTHR) EX[i] = 0.f;
+  for (int i = tid; i < 6 * 2 * 16 * 4; i += NTHR) EX[i] = 0.f;
   if (tid < 2 * 2 * 16 * 4) EXO[tid] = 0.f;
   int& partner_xcc = *reinterpret_cast<int*>(smem + L::LOST + 4);  // -1: the partner never said
   if (tid == 0) {
@@ -287,96 +298,130 @@ __global__ void __launch_bounds__(64 * (D / 16)) ttt_mlp_fwd_cl2_kernel(Problems
     EX[(((g)*2 + (w >> 2)) * 16 + c) * 4 + (w & 3)] = v0;
     if (g < 2) EX[(((g + 4) * 2 + (w >> 2)) * 16 + c) * 4 + (w & 3)] = v1;
   };
-  auto collect = [&](const float* ex, int i) -> float {
-    const f32x4 lo = *reinterpret_cast<const f32x4*>(ex + ((i * 2 + 0) * 16 + c) * 4);
-    const f32x4 hi = *reinterpret_cast<const f32x4*>(ex + ((i * 2 + 1) * 16 + c) * 4);
-    return ((lo[0] + lo[1]) + (lo[2] + lo[3])) + ((hi[0] + hi[1]) + (hi[2] + hi[3]));
+  // sums i and j of those exchanged at ex
+  auto collect2 = [&](const float* ex, int i, int j, float& a, float& b) {
+    f32x4 v[4];
+    v[0] = *reinterpret_cast<const f32x4*>(ex + ((i * 2 + 0) * 16 + c) * 4);
+    v[1] = *reinterpret_cast<const f32x4*>(ex + ((j * 2 + 0) * 16 + c) * 4);
+    v[2] = *reinterpret_cast<const f32x4*>(ex + ((i * 2 + 1) * 16 + c) * 4);
+    v[3] = *reinterpret_cast<const f32x4*>(ex + ((j * 2 + 1) * 16 + c) * 4);
+    together(v);
+    a = ((v[0][0] + v[0][1]) + (v[0][2] + v[0][3])) + ((v[2][0] + v[2][1]) + (v[2][2] + v[2][3]));
+    b = ((v[1][0] + v[1][1]) + (v[1][2] + v[1][3])) + ((v[3][0] + v[3][1]) + (v[3][2] + v[3][3]));
   };
   // tile slot `idx` of parity `par`: X1 tiles 0..NT-1, X2 tiles NT..2NT-1, the A2 tile 2NT
   bool alive = a.spin_limit > 0;
   auto send_tile = [&](int par_, int idx, f32x4 v, unsigned tag) {
-    send_tagged(reinterpret_cast<unsigned long long*>(xout + par_ * L::XSLOT + idx * L::XTILE) + 4 * lane, v, tag, same_xcd);
+    send_tagged(reinterpret_cast<unsigned long long*>(xout + par_ * L::XSLOT + idx * L::XTILE) + lane, v, tag, same_xcd);
   };
   auto slot_in = [&](int par_, int idx) -> const unsigned long long* {
-    return reinterpret_cast<const unsigned long long*>(xin + par_ * L::XSLOT + idx * L::XTILE) + 4 * lane;
+    return reinterpret_cast<const unsigned long long*>(xin + par_ * L::XSLOT + idx * L::XTILE) + lane;
   };
 
-  // ---- output path (previous mini-batch), wave w owns d-feature tile w.  CU 1 reduces its half and
-  // sends it; CU 0 adds both halves, applies the causal correction and finishes the LayerNorm.
+  // ---- output path, wave w owns d-feature tile w.  While the Z2 tiles of mini-batch t + 1 cross, each CU sums its partial
+  // Zbar2 tiles of t and CU 1 sends its half off; CU 0 adds it in phase D, applies the causal correction and forms the row
+  // moments, and stores the output while the tiles of t + 2 cross.  A2 is summed by wave 2 of each CU at the end of phase
+  // A, as soon as every wave has written its partial block (a counter per wave; a wave's LDS operations take place in order).
   f32x4 zb = {0.f, 0.f, 0.f, 0.f};
-  frag qo_pend = IO::zero();  // xq tile of the mini-batch whose output is pending
-  f32x4 at2 = {0.f, 0.f, 0.f, 0.f};
-  // local half of the pending output: this CU's split-k sums; CU 1 sends them off at once
-  auto output_local = [&](int st_out) {  // st_out: the mini-batch the output belongs to
-    at2 = f32x4{0.f, 0.f, 0.f, 0.f};
+  frag qo1 = IO::zero(), qo2 = qo1;  // xq tiles of the last mini-batch and of the one before
+  auto a2_sum = [&]() -> f32x4 {
+    f32x4 v[NW], at = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int ww = 0; ww < NW; ++ww) at2 += PA[ww * 64 + lane];
-    pin(at2);
+    for (int ww = 0; ww < NW; ++ww) v[ww] = PA[ww * 64 + lane];
+    together(v);
+#pragma unroll
+    for (int ww = 0; ww < NW; ++ww) at += v[ww];
+    return at;
+  };
+  auto a2_early = [&](int stage) -> f32x4 {
+    while (__builtin_amdgcn_ballot_w64(FL[lane & 7] <= stage) != 0) {
+    }
+    asm volatile("" ::: "memory");
+    const f32x4 at = a2_sum();
+    if (cu == 1) send_tile(stage & 1, 2 * NT, at, (unsigned)stage + 1);
+    return at;
+  };
+  auto output_local = [&](int stage) {
+    const int par_ = stage & 1;
+    frag v[NW];
+#pragma unroll
+    for (int ww = 0; ww < NW; ++ww) v[ww] = P2[(ww * NT + w) * 64 + lane];
     zb = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int ww = 0; ww < NW; ++ww) zb += IO::to_f32(P2[(ww * NT + w) * 64 + lane]);
+    for (int ww = 0; ww < NW; ++ww) zb += IO::to_f32(v[ww]);
     pin(zb);
-    if (cu == 1) {
-      send_tile(st_out & 1, NT + w, zb, (unsigned)st_out + 1);
-      if (w == 0) send_tile(st_out & 1, 2 * NT, at2, (unsigned)st_out + 1);
-    }
+    if (cu == 1) send_tile(par_, NT + w, zb, (unsigned)stage + 1);
   };
-  // CU 0: add CU 1's half, causal correction, row moments
-  auto output_finish = [&](f32x4 zb_part, f32x4 at_part) {
-    if (cu == 1) return;
-    zb += zb_part;
-    at2 += at_part;
+  // wave 2 of CU 0: M2[s][t] = (token_eta[t] / sc)(1 + A2[t][s]) for s <= t
+  auto output_m2 = [&](f32x4 at) {
+    const float rho_c = RHO[c];
     f32x4 m;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) m[r] = (4 * g + r <= c) ? rho_c * (1.f + at2[r]) : 0.f;
-    IO::mma(zb, GD[w * 64 + lane], IO::to_frag(m));  // GD still holds the previous mini-batch's G2
+    for (int r = 0; r < 4; ++r) m[r] = (4 * g + r <= c) ? rho_c * (1.f + at[r]) : 0.f;
+    M2s[lane] = IO::to_frag(m);
+  };
+  // CU 0: add CU 1's half, causal correction, row moments
+  auto output_finish = [&](int stage, f32x4 zb_part) {
+    zb += zb_part;
+    IO::mma(zb, read_tr(GT + ((stage & 1) * NT + w) * 64 + tr_lane(lane)), M2s[lane]);
     float s0 = 0.f, s1 = 0.f;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       s0 += zb[r];
       s1 += zb[r] * zb[r];
     }
-    s0 = xg_sum(s0);
-    s1 = xg_sum(s1);
-    if (g == 0) {
-      EXO[((0 * 2 + (w >> 2)) * 16 + c) * 4 + (w & 3)] = s0;
-      EXO[((1 * 2 + (w >> 2)) * 16 + c) * 4 + (w & 3)] = s1;
-    }
+    const float v = xg_sum4_scatter(s0, s1, 0.f, 0.f);
+    if (g < 2) EXO[((g * 2 + (w >> 2)) * 16 + c) * 4 + (w & 3)] = v;
   };
   auto output_emit = [&](int stage) {
-    if (cu == 1) return;
-    const float mu = collect(EXO, 0) * inv_d;
-    const float rstd = __builtin_amdgcn_rsqf(fmaxf(collect(EXO, 1) * inv_d - mu * mu, 0.f) + a.eps);
+    float mu, ms;
+    collect2(EXO, 0, 1, mu, ms);
+    mu *= inv_d;
+    const float rstd = __builtin_amdgcn_rsqf(fmaxf(ms * inv_d - mu * mu, 0.f) + a.eps);
     if (c < K) {
       const f32x4 gam = *reinterpret_cast<const f32x4*>(GAM + own), bet = *reinterpret_cast<const f32x4*>(BET + own);
-      elem* po = static_cast<elem*>(a.out) + (bh * (size_t)a.seq_stride + (size_t)stage * K + c) * D + own;
-      store4<T>(po, IO::to_f32(qo_pend) + bet + gam * ((zb - mu) * rstd));
+      elem* po = reinterpret_cast<elem*>(outp + (size_t)stage * step) + (c * D + own);
+      store4<T>(po, IO::to_f32(qo2) + bet + gam * ((zb - mu) * rstd));
+    }
+  };
+  // partial tiles of X W2 over this wave's hidden units, two at a time (HT is even here)
+  auto partials = [&](const frag (&x)[HT], auto put) {
+#pragma unroll
+    for (int I = 0; I < NT; I += 2) {
+      f32x4 p0 = {0.f, 0.f, 0.f, 0.f}, p1 = p0;
+#pragma unroll
+      for (int j = 0; j < HT; j += 2) {
+        IO::mma2(p0, IO::to_frag(W2c[j][I]), IO::to_frag(W2c[j + 1][I]), x[j], x[j + 1]);
+        IO::mma2(p1, IO::to_frag(W2c[j][I + 1]), IO::to_frag(W2c[j + 1][I + 1]), x[j], x[j + 1]);
+      }
+      put(I, p0);
+      put(I + 1, p1);
+      __builtin_amdgcn_sched_barrier(0);
     }
   };
 
-  for (int st = 0; st < a.n_stages; ++st) {
+  for (int st = 0; st < n_stages; ++st) {
     const int buf = st & 1, par = st & 1;
+    frag* const GTc = GT + par * NT * 64;
     RELANE();
 
     // ================= phase A: everything that needs only W1, W2 and the inputs
-    f32x4 z1[HT];
-    {
-      f32x4 t = {0.f, 0.f, 0.f, 0.f};
-      IO::mma(t, load4<T>(row(buf, 1) + own), ident);
-      KD[(par * NT + w) * 64 + lane] = IO::to_frag(t);
-    }
+    f32x4 z1[HT], zq[HT];
 #pragma unroll
-    for (int j = 0; j < HT; ++j) z1[j] = *reinterpret_cast<const f32x4*>(B1s + 16 * (w * HT + j) + 4 * g);
+    for (int j = 0; j < HT; ++j) zq[j] = z1[j] = *reinterpret_cast<const f32x4*>(B1s + 16 * (w * HT + j) + 4 * g);
 #pragma unroll
     for (int q = 0; q < NT / 2; ++q) {
-      frag k0, k1;
+      frag k0, k1, q0, q1;
       IO::load8(row(buf, 1) + 32 * q + 8 * g, true, k0, k1);
+      IO::load8(row(buf, 0) + 32 * q + 8 * g, true, q0, q1);
 #pragma unroll
-      for (int j = 0; j < HT; ++j)
-        IO::mma2(z1[j], IO::to_frag(W1c[2 * q][j]), IO::to_frag(W1c[2 * q + 1][j]), k0, k1);
+      for (int j = 0; j < HT; ++j) {
+        const frag w0 = IO::to_frag(W1c[2 * q][j]), w1 = IO::to_frag(W1c[2 * q + 1][j]);
+        IO::mma2(z1[j], w0, w1, k0, k1);
+        IO::mma2(zq[j], w0, w1, q0, q1);
+      }
       __builtin_amdgcn_sched_barrier(0);
     }
-    const float lrc = (c < K) ? __uint_as_float(LRs[buf * 16 + c] << 16) : 0.f;
     frag x2f[HT];
     f32x4 dg[HT];
 #pragma unroll
@@ -394,81 +439,56 @@ __global__ void __launch_bounds__(64 * (D / 16)) ttt_mlp_fwd_cl2_kernel(Problems
       asm volatile("" : "+v"(x2f[j]), "+v"(dg[j]));
       __builtin_amdgcn_sched_barrier(0);
     }
-    // partial Z2^T over this wave's hidden units (HT is even here)
 #pragma unroll
-    for (int I = 0; I < NT; ++I) {
-      f32x4 p = {0.f, 0.f, 0.f, 0.f};
+    for (int j = 0; j < HT; ++j) X2S[j * 64 + lane] = x2f[j];
+    partials(x2f, [&](int I, f32x4 p) { P1[(w * NT + I) * 64 + lane] = p; });
+    f32x4 at = {0.f, 0.f, 0.f, 0.f};
+    if (w == 2 && st > 0) at = a2_early(st - 1);
+    // M1[s][t] = (token_eta[t] / sc)(1 + A1[t][s]) for s <= t
+    if (w == 3) {
+      const float rho_c = RHO[c];
+      f32x4 At = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int j = 0; j + 1 < HT; j += 2)
-        IO::mma2(p, IO::to_frag(W2c[j][I]), IO::to_frag(W2c[j + 1][I]), x2f[j], x2f[j + 1]);
-      if (HT & 1) IO::mma2(p, IO::to_frag(W2c[HT - 1][I]), IO::zero(), x2f[HT - 1], IO::zero());
-      P1[(w * NT + I) * 64 + lane] = p;
-      __builtin_amdgcn_sched_barrier(0);
+      for (int q = 0; q < NT / 2; ++q) {
+        frag k0, k1, q0, q1;
+        IO::load8(row(buf, 1) + 32 * q + 8 * g, true, k0, k1);
+        IO::load8(row(buf, 0) + 32 * q + 8 * g, true, q0, q1);
+        IO::mma2(At, k0, k1, q0, q1);
+      }
+      f32x4 m;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) m[r] = (4 * g + r <= c) ? rho_c * (1.f + At[r]) : 0.f;
+      M1s[par * 64 + lane] = IO::to_frag(m);
     }
     lds_barrier();  // ---- B1
     RELANE();
 
-    // ================= phase B: this CU's half of Z2 tile w, exchange with the partner, row moments;
-    //                          then the output path of the previous mini-batch
-    f32x4 z, bq, zq[HT];
-    frag Mf;
+    // ================= phase B: this CU's half of Z2 tile w, exchange with the partner, row moments
+    f32x4 z, bq;
+    Inbound zb_in;
     {
       f32x4 zloc = {0.f, 0.f, 0.f, 0.f};
+      {
+        f32x4 v[NW];
 #pragma unroll
-      for (int ww = 0; ww < NW; ++ww) {
-        zloc += P1[(ww * NT + w) * 64 + lane];
-        if ((ww & 3) == 3) pin(zloc);
+        for (int ww = 0; ww < NW; ++ww) v[ww] = P1[(ww * NT + w) * 64 + lane];
+        together(v);
+#pragma unroll
+        for (int ww = 0; ww < NW; ++ww) zloc += v[ww];
       }
       send_tile(par, w, zloc, (unsigned)st + 1);
-      // everything that does not need the partner goes between the send and the wait
+      // everything that does not need the partner goes between the send and the wait: the local half of the previous
+      // output
+      if (cu == 0 && st > 1) output_emit(st - 2);
       if (st > 0) output_local(st - 1);
-      // (XQ W1 + b1)^T for this wave's hidden units and the causal matrix M1: independent of the partner
-#pragma unroll
-      for (int j = 0; j < HT; ++j)
-#pragma unroll
-        for (int I = 0; I < NT; ++I) forget(W1c[I][j]);
-#pragma unroll
-      for (int j = 0; j < HT; ++j) zq[j] = *reinterpret_cast<const f32x4*>(B1s + 16 * (w * HT + j) + 4 * g);
-      {
-        f32x4 At = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int q = 0; q < NT / 2; ++q) {
-          frag k0, k1, q0, q1;
-          IO::load8(row(buf, 1) + 32 * q + 8 * g, true, k0, k1);
-          IO::load8(row(buf, 0) + 32 * q + 8 * g, true, q0, q1);
-#pragma unroll
-          for (int j = 0; j < HT; ++j)
-            IO::mma2(zq[j], IO::to_frag(W1c[2 * q][j]), IO::to_frag(W1c[2 * q + 1][j]), q0, q1);
-          IO::mma2(At, k0, k1, q0, q1);
-          __builtin_amdgcn_sched_barrier(0);
-        }
-        f32x4 m;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) m[r] = (4 * g + r <= c) ? rho_c * (1.f + At[r]) : 0.f;
-        Mf = IO::to_frag(m);
-      }
       const frag ko = load4<T>(row(buf, 1) + own), vo = load4<T>(row(buf, 2) + own);
       const f32x4 gam = *reinterpret_cast<const f32x4*>(GAM + own), bet = *reinterpret_cast<const f32x4*>(BET + own);
       bq = gam * (bet - (IO::to_f32(vo) - IO::to_f32(ko)));
-      // one wait for everything the partner sends this mini-batch: its half of Z2 tile w and (to CU 0)
-      // its half of the pending output
-      f32x4 zpart, zb_part = {0.f, 0.f, 0.f, 0.f}, at_part = zb_part;
-      if (cu == 0 && st > 0) {
-        const unsigned long long* const sl[3] = {slot_in(par, w), slot_in(par ^ 1, NT + w), slot_in(par ^ 1, 2 * NT)};
-        const unsigned tg[3] = {(unsigned)st + 1, (unsigned)st, (unsigned)st};
-        f32x4 rv[3];
-        recv_tagged<3>(sl, tg, rv, alive, a.spin_limit);
-        zpart = rv[0];
-        zb_part = rv[1];
-        at_part = rv[2];
-      } else {
-        const unsigned long long* const sl[1] = {slot_in(par, w)};
-        const unsigned tg[1] = {(unsigned)st + 1};
-        f32x4 rv[1];
-        recv_tagged<1>(sl, tg, rv, alive, a.spin_limit);
-        zpart = rv[0];
-      }
-      fetch(st + 1);
+      const bool m2w = cu == 0 && w == 2 && st > 0;  // CU 1 sent its A2 before its Z2 tiles
+      Inbound in, in2;
+      in.load(slot_in(par, w));
+      if (m2w) in2.load(slot_in(par ^ 1, 2 * NT));
+      const f32x4 zpart = in.wait(slot_in(par, w), (unsigned)st + 1, alive, a.spin_limit);
       z = b2T + (cu == 0 ? zloc + zpart : zpart + zloc);  // same order of the halves on both CUs
       float S[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
       const f32x4 az = gam * gam * z;
@@ -482,16 +502,37 @@ __global__ void __launch_bounds__(64 * (D / 16)) ttt_mlp_fwd_cl2_kernel(Problems
         S[5] += bq[r] * z[r];
       }
       publish(S);
-      if (st > 0) output_finish(zb_part, at_part);
+      if (cu == 0 && st > 0) {
+        if (m2w) output_m2(at + in2.wait(slot_in(par ^ 1, 2 * NT), (unsigned)st, alive, a.spin_limit));
+        zb_in.load(slot_in(par ^ 1, NT + w));
+      }
+      fetch(st + 1);
     }
     lds_barrier();  // ---- B2
     RELANE();
 
-    // ================= phase C: G2'' in both orientations; CU 0 stores the previous output
+    // ================= phase C: G2''
     {
+      const float lrc = (c < K) ? __uint_as_float(LRs[buf * 16 + c] << 16) : 0.f;
       float S[6];
-#pragma unroll
-      for (int i = 0; i < 6; ++i) S[i] = collect(EX, i);
+      {
+        // lane group g adds up sums g and 4 + (g & 1), then all groups get all six
+        float v0, v1;
+        collect2(EX, g, 4 + (g & 1), v0, v1);
+        const uint32_t u = __float_as_uint(v0), v = __float_as_uint(v1);
+        const auto p = __builtin_amdgcn_permlane16_swap(u, u, false, false);  // rows: 0 0 2 2 / 1 1 3 3
+        const uint32_t p0 = p[0], p1 = p[1];
+        const auto q = __builtin_amdgcn_permlane32_swap(p0, p0, false, false);
+        const auto r = __builtin_amdgcn_permlane32_swap(p1, p1, false, false);
+        const auto t2 = __builtin_amdgcn_permlane16_swap(v, v, false, false);  // rows: 4 4 4 4 / 5 5 5 5
+        const uint32_t q0 = q[0], q1 = q[1], r0 = r[0], r1 = r[1], t0 = t2[0], t1 = t2[1];
+        S[0] = __uint_as_float(q0);
+        S[2] = __uint_as_float(q1);
+        S[1] = __uint_as_float(r0);
+        S[3] = __uint_as_float(r1);
+        S[4] = __uint_as_float(t0);
+        S[5] = __uint_as_float(t1);
+      }
       const float mu = S[0] * inv_d;
       const float var = S[1] * inv_d - mu * mu;
       const float rstd = __builtin_amdgcn_rsqf(fmaxf(var, 0.f) + a.eps);
@@ -501,20 +542,10 @@ __global__ void __launch_bounds__(64 * (D / 16)) ttt_mlp_fwd_cl2_kernel(Problems
       const float c1 = p * rstd, c2 = -c1 * s2 * inv_d, c3 = -p * s1 * inv_d;
       const f32x4 gam = *reinterpret_cast<const f32x4*>(GAM + own);
       const f32x4 G = (z - mu) * (gam * gam * c1 + c2) + (bq * p + c3);
-      const frag gt = IO::to_frag(G);
-      f32x4 t = {0.f, 0.f, 0.f, 0.f};
-      IO::mma(t, gt, ident);
-      GT[w * 64 + lane] = gt;
-      GD[w * 64 + lane] = IO::to_frag(t);
+      GTc[w * 64 + lane] = IO::to_frag(G);
     }
-    if (st > 0) output_emit(st - 1);
-    qo_pend = load4<T>(row(buf, 0) + own);
-    // the next mini-batch's rows must have landed; CU 0's output store, the only memory operation younger
-    // than the copies (which retire in order), may stay in flight
-    if (cu == 0 && st > 0)
-      asm volatile("s_waitcnt vmcnt(1)" ::: "memory");
-    else
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    // the next mini-batch's rows must have landed before anybody passes B3
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     lds_barrier();  // ---- B3
     RELANE();
 
@@ -523,24 +554,47 @@ __global__ void __launch_bounds__(64 * (D / 16)) ttt_mlp_fwd_cl2_kernel(Problems
     for (int j = 0; j < HT; ++j)
 #pragma unroll
       for (int I = 0; I < NT; ++I) forget(W2c[j][I]);
+    // G1''^T = (W2 G2''^T) gelu'(Z1)
     frag G1d[HT];
+    {
+      const frag ident = IDs[lane];
+      f32x4 acc[HT];
 #pragma unroll
-    for (int j = 0; j < HT; ++j) {
-      f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+      for (int j = 0; j < HT; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int q = 0; q < NT / 2; ++q) {
-        f32x4 t0 = {0.f, 0.f, 0.f, 0.f}, t1 = {0.f, 0.f, 0.f, 0.f};
-        IO::mma(t0, IO::to_frag(W2c[j][2 * q]), ident);
-        IO::mma(t1, IO::to_frag(W2c[j][2 * q + 1]), ident);
-        IO::mma2(acc, IO::to_frag(t0), IO::to_frag(t1), GT[(2 * q) * 64 + lane], GT[(2 * q + 1) * 64 + lane]);
-      }
-      f32x4 t = {0.f, 0.f, 0.f, 0.f};
-      IO::mma(t, IO::to_frag(acc * dg[j]), ident);
-      G1d[j] = IO::to_frag(t);
-      __builtin_amdgcn_sched_barrier(0);
-    }
+        const frag g0 = GTc[(2 * q) * 64 + lane], g1 = GTc[(2 * q + 1) * 64 + lane];
+        f32x4 t0[HT], t1[HT];
 #pragma unroll
-    for (int j = 0; j < HT; ++j) IO::mma(zq[j], G1d[j], Mf);
+        for (int j = 0; j < HT; ++j) {
+          t0[j] = t1[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+          IO::mma(t0[j], IO::to_frag(W2c[j][2 * q]), ident);
+          IO::mma(t1[j], IO::to_frag(W2c[j][2 * q + 1]), ident);
+        }
+#pragma unroll
+        for (int j = 0; j < HT; ++j) IO::mma2(acc[j], IO::to_frag(t0[j]), IO::to_frag(t1[j]), g0, g1);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      f32x4 t[HT];
+#pragma unroll
+      for (int j = 0; j < HT; ++j) {
+        t[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+        IO::mma(t[j], IO::to_frag(acc[j] * dg[j]), ident);
+      }
+#pragma unroll
+      for (int j = 0; j < HT; ++j) G1d[j] = IO::to_frag(t[j]);
+    }
+    // Zbar1^T = (XQ W1 + b1)^T + G1''^T M1
+    {
+      const frag Mf = M1s[par * 64 + lane];
+#pragma unroll
+      for (int j = 0; j < HT; ++j) IO::mma(zq[j], G1d[j], Mf);
+    }
+    if (cu == 0) {
+      if (st > 0) output_finish(st - 1, zb_in.wait(slot_in(par ^ 1, NT + w), (unsigned)st, alive, a.spin_limit));
+      qo2 = qo1;
+      qo1 = load4<T>(row(buf, 0) + own);
+    }
     frag xbf[HT];
 #pragma unroll
     for (int j = 0; j < HT; ++j) {
@@ -557,59 +611,72 @@ __global__ void __launch_bounds__(64 * (D / 16)) ttt_mlp_fwd_cl2_kernel(Problems
     {
       f32x4 p = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int j = 0; j + 1 < HT; j += 2) IO::mma2(p, x2f[j], x2f[j + 1], xbf[j], xbf[j + 1]);
-      if (HT & 1) IO::mma2(p, x2f[HT - 1], IO::zero(), xbf[HT - 1], IO::zero());
+      for (int j = 0; j < HT; j += 2) IO::mma2(p, x2f[j], x2f[j + 1], xbf[j], xbf[j + 1]);
       PA[w * 64 + lane] = p;
+      asm volatile("" ::: "memory");
+      if (lane == 0) FL[w] = st + 1;
     }
-#pragma unroll
-    for (int I = 0; I < NT; ++I) {
-      // b2 enters the sum once: through wave I of CU 0
-      f32x4 p = (I == w && cu == 0) ? b2T : f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int j = 0; j + 1 < HT; j += 2)
-        IO::mma2(p, IO::to_frag(W2c[j][I]), IO::to_frag(W2c[j + 1][I]), xbf[j], xbf[j + 1]);
-      if (HT & 1) IO::mma2(p, IO::to_frag(W2c[HT - 1][I]), IO::zero(), xbf[HT - 1], IO::zero());
-      P2[(w * NT + I) * 64 + lane] = IO::to_frag(p);
-      __builtin_amdgcn_sched_barrier(0);
-    }
+    // (b2 enters the sum once: through wave I of CU 0)
+    partials(xbf, [&](int I, f32x4 p) { P2[(w * NT + I) * 64 + lane] = IO::to_frag(I == w && cu == 0 ? p + b2T : p); });
     if (upd) {
       frag x2d[HT];
+      {
+        const frag ones = splat_frag<T>(1.f);
+        f32x4 b[HT];
 #pragma unroll
-      for (int j = 0; j < HT; ++j) {
-        f32x4 t = {0.f, 0.f, 0.f, 0.f};
-        IO::mma(t, x2f[j], ident);
-        x2d[j] = IO::to_frag(t);
-        f32x4 b = *reinterpret_cast<const f32x4*>(B1s + 16 * (w * HT + j) + 4 * g);
-        IO::mma(b, G1d[j], ones);
-        if (c == 0) *reinterpret_cast<f32x4*>(B1s + 16 * (w * HT + j) + 4 * g) = b;
+        for (int j = 0; j < HT; ++j) {
+          x2d[j] = read_tr(X2S + j * 64 + tr_lane(lane));
+          b[j] = *reinterpret_cast<const f32x4*>(B1s + 16 * (w * HT + j) + 4 * g);
+        }
+#pragma unroll
+        for (int j = 0; j < HT; ++j) IO::mma(b[j], G1d[j], ones);
+#pragma unroll
+        for (int j = 0; j < HT; ++j)
+          if (c == 0) *reinterpret_cast<f32x4*>(B1s + 16 * (w * HT + j) + 4 * g) = b[j];
       }
+      // XK tiles with tokens along k, straight from the staged rows: lane l supplies four features of token 4g + c / 4
+      const elem* const kr = reinterpret_cast<const elem*>(smem + L::IN + buf * L::IN1 + L::TILE) + (4 * g + (c >> 2)) * D + 8 * (c & 3);
+      const frag* const gr = GTc + tr_lane(lane);
+      frag kd = read_tr(kr), g2d = read_tr(gr);
 #pragma unroll
       for (int I = 0; I < NT; ++I) {
-        const frag kd = KD[(par * NT + I) * 64 + lane], g2d = GD[I * 64 + lane];
+        const int In = I + 1 < NT ? I + 1 : I;
+        const frag kn = read_tr(kr + 32 * (In >> 1) + 4 * (In & 1)), gn = read_tr(gr + (I + 1 < NT ? I + 1 : w) * 64);
 #pragma unroll
         for (int j = 0; j < HT; ++j) {
           IO::mma(W1c[I][j], kd, G1d[j]);
           IO::mma(W2c[j][I], x2d[j], g2d);
         }
+        kd = kn;
+        g2d = gn;
         __builtin_amdgcn_sched_barrier(0);
       }
-      IO::mma(b2T, GD[w * 64 + lane], ones);
+      IO::mma(b2T, g2d, splat_frag<T>(1.f));
     }
   }
 
   // ---- the last mini-batch's output
   lds_barrier();
-  output_local(a.n_stages - 1);
-  if (cu == 0) {
-    const int lp = (a.n_stages - 1) & 1;
-    const unsigned long long* const sl[2] = {slot_in(lp, NT + w), slot_in(lp, 2 * NT)};
-    const unsigned tg[2] = {(unsigned)a.n_stages, (unsigned)a.n_stages};
-    f32x4 rv[2];
-    recv_tagged<2>(sl, tg, rv, alive, a.spin_limit);
-    output_finish(rv[0], rv[1]);
+  if (cu == 0 && n_stages > 1) output_emit(n_stages - 2);
+  qo2 = qo1;
+  output_local(n_stages - 1);
+  f32x4 at = {0.f, 0.f, 0.f, 0.f};
+  if (w == 2) at = a2_early(n_stages - 1);
+  if (cu == 0 && w == 2) {
+    const unsigned long long* const sl = slot_in((n_stages - 1) & 1, 2 * NT);
+    Inbound in;
+    in.load(sl);
+    output_m2(at + in.wait(sl, (unsigned)n_stages, alive, a.spin_limit));
   }
   lds_barrier();
-  output_emit(a.n_stages - 1);
+  if (cu == 0) {
+    const unsigned long long* const sl = slot_in((n_stages - 1) & 1, NT + w);
+    Inbound in;
+    in.load(sl);
+    output_finish(n_stages - 1, in.wait(sl, (unsigned)n_stages, alive, a.spin_limit));
+  }
+  lds_barrier();
+  if (cu == 0) output_emit(n_stages - 1);
 
   // ---- final state: this CU's hidden half.  Its rows of W2_out held the exchange area; every read of
   // it by this workgroup is above, every write of the partner into it was awaited above.
