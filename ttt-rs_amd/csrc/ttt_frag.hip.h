@@ -106,6 +106,26 @@ __device__ __forceinline__ void lds_barrier() {
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
 
+// A fragment's transpose: element (m, k) of the tile that lies in LDS as a fragment (lane order) -> the fragment with the
+// two axes exchanged.  Within each group of sixteen lanes the instruction takes four rows of sixteen elements, a row from
+// four lanes, and gives every lane a column.
+__device__ __forceinline__ bf16x4 read_tr(const void* p) {
+  typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
+  return __builtin_bit_cast(bf16x4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)p));
+}
+// the lane whose fragment starts the row that this lane supplies
+__device__ __forceinline__ int tr_lane(int lane) { return (lane & 3) * 16 + (lane >> 4) * 4 + ((lane >> 2) & 3); }
+
+// All of v in registers here: loads that feed v are issued together and waited for once.  (Short of registers the scheduler
+// otherwise loads, waits and uses them one at a time, an LDS round trip each.)
+template <int N>
+__device__ __forceinline__ void together(f32x4 (&v)[N]) {
+  if constexpr (N == 4) asm volatile("" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]));
+  if constexpr (N == 6) asm volatile("" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]), "+v"(v[4]), "+v"(v[5]));
+  if constexpr (N == 8)
+    asm volatile("" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]), "+v"(v[4]), "+v"(v[5]), "+v"(v[6]), "+v"(v[7]));
+}
+
 // 16 bytes per lane, global -> LDS at lds_base + 16 * lane, not passing registers.  Written as assembly
 // because the compiler makes every later LDS read wait for all copies it knows to be in flight (it cannot
 // tell the two stage buffers apart), which would turn the prefetch into a synchronous load; the waits

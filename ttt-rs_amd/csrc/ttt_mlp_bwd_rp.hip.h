@@ -5,9 +5,9 @@
 // with the second-order LayerNorm (rust/fused/src/linear_fused_tile/layer_norm.rs:428-709) and GELU'' terms.
 //
 // Why: the scan on tiles in memory (ttt_mlp_bwd.hip.h) passes over W1, W2, dW1, dW2 21 times per mini-batch, 57 GB at
-// 128 units x 2048 tokens of d = 96, and is bound by that traffic: 9.3 ms.  This kernel: 2.65 ms there, 15.6 GB, bound by the
-// hand-over of 289 KB per mini-batch and unit (more than the L2 of 16 units holds), at head_dim 32 and 64 by the producer's
-// vector instructions.  Nothing of the state moves here: a unit is worked on by two roles, each of which keeps its
+// 128 units x 2048 tokens of d = 96, and is bound by that traffic: 9.3 ms.  This kernel: 2.07 ms there, 1.76 ms for 16
+// units: bound by the producer's products, and on a full chip by the hand-over of 289 KB per mini-batch and unit besides
+// (more than the L2 of 16 units holds).  Nothing of the state moves here: a unit is worked on by two roles, each of which keeps its
 // matrices as MFMA accumulator tiles in the
 // registers of one workgroup of eight waves, the hidden axis (4 d) cut into eight slices as in the forward
 // (ttt_mlp_fwd_rr.hip.h):
@@ -31,6 +31,12 @@
 // check, the bounded waits and the poison value; they are the same here).  One workgroup per unit: the roles run in
 // turn, launch by launch, over as many mini-batches as there are slots; the matrices are stored in accumulator order
 // between launches.  The same code and the same bits.
+//
+// Registers.  At d = 96 a role holds 144 of 256 in its matrices, and a value spilled inside the loop is dear: its reload waits
+// for every load and store of the wave that is in flight, up to 5 k cycles on a full chip.  Hence what is read from LDS
+// (transposing loads of the staged rows, sums of gradients, parked tiles) or formed again rather than held, and the
+// scheduler's register tracking that the d = 96 instance is compiled with (build.py).  128 units x 2048 tokens, d = 96:
+// 2645 us with fourteen reloads in the two loops, 2167 with two, 2066 with none; d = 64 1440 -> 1375, d = 32 845 -> 818 us.
 #pragma once
 #include "ttt_engine.hip.h"
 #include "ttt_frag.hip.h"
@@ -87,12 +93,13 @@ struct MlpRpLds {
   static constexpr int PA = LR + 2 * 64 + 128;     // [NW][64] f32x4: partial [16 x 16] blocks
   static constexpr int PB = PA + NW * 1024;        // [2][NW][NT][64] f32x4: partial [16 x d] tiles
   static constexpr int GT = PB + 2 * NW * NT * 1024;  // fragments by feature tile
-  static constexpr int ZT = GT + NT * 512, KD = ZT + NT * 512, GS = KD + 2 * NT * 512;
+  static constexpr int ZT = GT + NT * 512, DG = ZT + NT * 512;  // DG: producer: [NT][64] f32x4, d gamma by lane
+  static constexpr int GS = DG + NT * 1024;
   static constexpr int EX = GS + NT * 512;         // [8 sums][2][16 tokens] f32x4 (reducer index % 4)
   static constexpr int PRM = EX + 8 * 2 * 16 * 16;  // gamma[d], beta[d], b1[4d]
   static constexpr int QS = PRM + 6 * D * 4;       // [NW][16] floats
   static constexpr int CTL = QS + NW * 64;
-  static constexpr int DB = CTL + 16;              // consumer: [NT][64] f32x4, d beta by lane (d gamma: in PA)
+  static constexpr int DB = CTL + 16;              // [NT][64] f32x4, d beta by lane (the consumer's d gamma: in PA)
   static constexpr int B2 = DB + NT * 1024;        // consumer: d b2 [d]
   static constexpr int GL = B2 + D * 4;            // consumer: [NT][64] fragments of what G2 loses as an operand
   static constexpr int BYTES = GL + NT * 512;
@@ -161,6 +168,23 @@ __device__ __forceinline__ V& at(const unsigned char* base, unsigned off) {
   return *reinterpret_cast<V*>(const_cast<unsigned char*>(base) + off);
 }
 
+// lds_dma16 and lds_dma4 with device scope (see Slot)
+__device__ __forceinline__ void lds_dma16_dev(const void* base, unsigned lane_off, unsigned lds_base) {
+  unsigned saved;
+  asm volatile(
+      "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 sc1\n\ts_nop 0\n\ts_mov_b32 m0, %0"
+      : "=&s"(saved)
+      : "v"(lane_off), "s"(uniform_ptr(base)), "s"(lds_base)
+      : "memory");
+}
+__device__ __forceinline__ void lds_dma4_dev(const void* base, unsigned lane_off, unsigned lds_base) {
+  unsigned saved;
+  asm volatile(
+      "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2 sc1\n\ts_nop 0\n\ts_mov_b32 m0, %0"
+      : "=&s"(saved)
+      : "v"(lane_off), "s"(uniform_ptr(base)), "s"(lds_base)
+      : "memory");
+}
 // The consumer's reads of a slot: device-scope loads (sc1), which do not look in the CU's vector cache and so see what the
 // producer's CU stored into the L2 behind both.  (Dropping the cache instead takes an instruction of device scope, which
 // also drops lines of the L2; what one of workgroup scope does is not for other workgroups to rely on.)  A slot is read once
@@ -189,13 +213,14 @@ struct Base {
   using L = MlpRpLds<D>;
   static constexpr int NW = S::NW, NT = S::NT, F = S::F, HT = S::HT, NQ = S::NQ;
   static constexpr float inv_d = 1.0f / D;
+  static constexpr bool ROOM = D <= 64;  // registers for more loads in flight beside the state (d = 96: spills, 2.3 ms)
   const MlpBwdRpArgs& a;
   unsigned char* smem;
   size_t bh;
   int tid, w, lane, c, g, K, h, own;
   bool red, pair;
   f32x4 *PA, *PB;
-  frag *GT, *ZT, *KD, *GS;
+  frag *GT, *ZT, *GS;
   float *EX, *GAM, *BET, *B1s, *QS;
   uint32_t* LRs;
   int* lost;
@@ -225,7 +250,6 @@ struct Base {
     PB = reinterpret_cast<f32x4*>(smem + L::PB);
     GT = reinterpret_cast<frag*>(smem + L::GT);
     ZT = reinterpret_cast<frag*>(smem + L::ZT);
-    KD = reinterpret_cast<frag*>(smem + L::KD);
     GS = reinterpret_cast<frag*>(smem + L::GS);
     EX = reinterpret_cast<float*>(smem + L::EX);
     GAM = reinterpret_cast<float*>(smem + L::PRM);
@@ -252,10 +276,14 @@ struct Base {
     for (int i = 0; i < TENSORS; ++i) src[i] = static_cast<const unsigned char*>(t[i]) + r0;
     lrp = static_cast<const unsigned char*>(a.lr) + bh * (size_t)a.seq_stride * 2;
   }
+  // the LDS address of the dynamic allocation, as a scalar
+  __device__ __forceinline__ unsigned lds0() const {
+    return __builtin_amdgcn_readfirstlane((unsigned)(size_t)(__attribute__((address_space(3))) unsigned char*)smem);
+  }
   // rows of a mini-batch, global -> LDS without passing registers; tokens past a short mini-batch keep the zeros
   __device__ __forceinline__ void fetch(int stage) {
     if (stage < a.first) return;
-    const unsigned in0 = __builtin_amdgcn_readfirstlane((unsigned)(size_t)(__attribute__((address_space(3))) unsigned char*)smem);
+    const unsigned in0 = lds0();
     const unsigned dst = in0 + L::IN + (stage & 1) * L::IN1;
     const size_t tok0 = (size_t)stage * (unsigned)(K * D * 2);
     // a tensor's tile is TILE / 1024 wave blocks; the blocks of all tensors are dealt to the waves in turn
@@ -272,6 +300,11 @@ struct Base {
   }
   __device__ __forceinline__ const uint16_t* row(int stage, int ten) const {
     return reinterpret_cast<const uint16_t*>(smem + L::IN + (stage & 1) * L::IN1 + ten * L::TILE) + c * D;
+  }
+  // tile I of a staged tensor with tokens along k: lane l supplies four features of token 4g + c / 4
+  __device__ __forceinline__ frag token_k(int stage, int ten, int I) const {
+    const unsigned char* t = smem + L::IN + (stage & 1) * L::IN1 + ten * L::TILE;
+    return read_tr(reinterpret_cast<const uint16_t*>(t) + (4 * g + (c >> 2)) * D + 8 * (c & 3) + 32 * (I >> 1) + 4 * (I & 1));
   }
   __device__ __forceinline__ float lr_of(int stage, int t) const {
     return t < K ? __uint_as_float(LRs[(stage & 1) * 16 + t] << 16) : 0.f;
@@ -304,27 +337,51 @@ struct Base {
     return s;
   }
   __device__ __forceinline__ f32x4 sum_tile(int buf, int I) const {
-    f32x4 z = {0.f, 0.f, 0.f, 0.f};
+    f32x4 v[NW], z = {0.f, 0.f, 0.f, 0.f};
+    if constexpr (ROOM) {
 #pragma unroll
-    for (int ww = 0; ww < NW; ++ww) {
-      z += PB[((buf * NW + ww) * NT + I) * 64 + lane];
-      if ((ww & 3) == 3) pin(z);
+      for (int ww = 0; ww < NW; ++ww) v[ww] = PB[((buf * NW + ww) * NT + I) * 64 + lane];
+      together(v);
+#pragma unroll
+      for (int ww = 0; ww < NW; ++ww) z += v[ww];
+    } else {
+#pragma unroll
+      for (int ww = 0; ww < NW; ++ww) {
+        z += PB[((buf * NW + ww) * NT + I) * 64 + lane];
+        if ((ww & 3) == 3) pin(z);
+      }
     }
     return z;
   }
   __device__ __forceinline__ f32x4 sum_block() const {
-    f32x4 z = {0.f, 0.f, 0.f, 0.f};
+    f32x4 v[NW], z = {0.f, 0.f, 0.f, 0.f};
+    if constexpr (ROOM) {
 #pragma unroll
-    for (int ww = 0; ww < NW; ++ww) z += PA[ww * 64 + lane];
-    pin(z);
+      for (int ww = 0; ww < NW; ++ww) v[ww] = PA[ww * 64 + lane];
+      together(v);
+#pragma unroll
+      for (int ww = 0; ww < NW; ++ww) z += v[ww];
+    } else {
+#pragma unroll
+      for (int ww = 0; ww < NW; ++ww) z += PA[ww * 64 + lane];
+      pin(z);
+    }
     return z;
   }
   // (moved to a scalar register by hand: see isa_check.py, the scalar select on a vector comparison)
   __device__ __forceinline__ bool is_lost() const { return __builtin_amdgcn_readfirstlane(*lost) != 0; }
   // bounded wait of thread 0 for the partner's counter; the barrier behind it is the caller's
+  // A look at the counter ahead of time: the poll that follows finds it in LDS and is spared the round trip it would begin
+  // with, up to 5 k cycles on a full chip (d = 96 2167 -> 2122 us).  Through LDS because a register for it spills others.
+  __device__ __forceinline__ void peek(const unsigned* fl, int which) {
+    if (pair && w == 0 && lane == 0) lds_dma4_dev(fl, 4u * which, lds0() + L::CTL + 4);
+  }
   __device__ __forceinline__ void poll(unsigned* fl, int which, int want) {
     if (!pair || want <= 0 || tid != 0 || is_lost()) return;
-    bool got = false;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    const unsigned seen = (unsigned)const_cast<volatile int*>(lost)[1];
+    bool got = seen != kMlpRpPoison && seen >= (unsigned)want;
+    if (got) return;
     for (unsigned i = 0; i < a.spin_limit; ++i) {
       const unsigned v = __hip_atomic_load(fl + which, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       if (v == kMlpRpPoison) break;
@@ -373,7 +430,7 @@ __device__ __forceinline__ void producer(const MlpBwdRpArgs& a, unsigned char* s
     my_xcc &= 15u;
     if (tid == 0) __hip_atomic_store(fl + 2, 0x100u | my_xcc, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
-  if (tid == 0) *x.lost = pair && a.spin_limit == 0 ? 1 : 0;
+  if (tid == 0) x.lost[0] = pair && a.spin_limit == 0 ? 1 : 0, x.lost[1] = 0;
   const bool upd = x.te_last != 0.f;
 
   f32x4 W1c[NT][HT], W2c[HT][NT], b2T = {0.f, 0.f, 0.f, 0.f};
@@ -388,7 +445,10 @@ __device__ __forceinline__ void producer(const MlpBwdRpArgs& a, unsigned char* s
     }
   for (int i = tid; i < F; i += 512) x.B1s[i] = a.b1[bh * F + i];
   if (red) b2T = *reinterpret_cast<const f32x4*>(a.b2 + bh * D + x.own);
-  f32x4 dgam = {0.f, 0.f, 0.f, 0.f}, dbet = dgam;
+  // sums that only the reducers touch, once per mini-batch, live in LDS: the registers are short
+  auto dgam = [&]() -> f32x4& { return reinterpret_cast<f32x4*>(smem + B::L::DG)[(red ? w : 0) * 64 + lane]; };
+  auto dbet = [&]() -> f32x4& { return reinterpret_cast<f32x4*>(smem + B::L::DB)[(red ? w : 0) * 64 + lane]; };
+  if (red) dgam() = dbet() = f32x4{0.f, 0.f, 0.f, 0.f};
 
   const unsigned char* const fac = a.fac + bh * (size_t)a.n_stages * S::FAC;
   frag G1d[HT], gd = IO::zero();
@@ -405,7 +465,6 @@ __device__ __forceinline__ void producer(const MlpBwdRpArgs& a, unsigned char* s
   __syncthreads();
   if (red) {
     x.GS[w * 64 + lane] = gd;
-    x.KD[(((a.last - 1) & 1) * NT + w) * 64 + lane] = flip(load4<BF16>(x.row(a.last - 1, 1) + x.own), x.ident);
   }
 
   for (int st = a.last - 1; st >= a.first; --st) {
@@ -417,28 +476,37 @@ __device__ __forceinline__ void producer(const MlpBwdRpArgs& a, unsigned char* s
     RP_RELANE();
 
     // ================= A: walk W1, b1 back; Z1, X2; walk W2, b2 back; partial Z2
-    f32x4 z1[HT];
+    f32x4 z1[HT], zq[HT];
+    frag kd[NT];
+#pragma unroll
+    for (int I = 0; I < NT; ++I) kd[I] = x.token_k(st, 1, I);
 #pragma unroll
     for (int j = 0; j < HT; ++j) {
       const frag ng = upd ? neg(G1d[j]) : IO::zero();
 #pragma unroll
-      for (int I = 0; I < NT; ++I) IO::mma(W1c[I][j], x.KD[(par * NT + I) * 64 + lane], ng);
+      for (int I = 0; I < NT; ++I) IO::mma(W1c[I][j], kd[I], ng);
       f32x4* const bp = reinterpret_cast<f32x4*>(x.B1s + 16 * (w * HT + j) + 4 * g);
       z1[j] = *bp;
       IO::mma(z1[j], ng, x.ones);
       if (c == 0) *bp = z1[j];
       asm volatile("s_nop 4" : "+v"(z1[j]));
+      zq[j] = z1[j];
       RP_FENCE();
     }
 #pragma unroll
     for (int q = 0; q < NQ; ++q) {
-      frag k0, k1;
+      frag k0, k1, q0, q1;
       IO::load8(x.row(st, 1) + 32 * q + 8 * g, true, k0, k1);
+      IO::load8(x.row(st, 0) + 32 * q + 8 * g, true, q0, q1);
 #pragma unroll
-      for (int j = 0; j < HT; ++j) IO::mma2(z1[j], IO::to_frag(W1c[2 * q][j]), IO::to_frag(W1c[2 * q + 1][j]), k0, k1);
+      for (int j = 0; j < HT; ++j) {
+        const frag w0 = IO::to_frag(W1c[2 * q][j]), w1 = IO::to_frag(W1c[2 * q + 1][j]);
+        IO::mma2(z1[j], w0, w1, k0, k1);
+        IO::mma2(zq[j], w0, w1, q0, q1);
+      }
       RP_FENCE();
     }
-    frag x2f[HT], x2d[HT];
+    frag x2f[HT];
     f32x4 dg[HT], ddg[HT];
 #pragma unroll
     for (int j = 0; j < HT; ++j) {
@@ -453,8 +521,7 @@ __device__ __forceinline__ void producer(const MlpBwdRpArgs& a, unsigned char* s
       }
       x2f[j] = IO::to_frag(y);
       asm volatile("" : "+v"(x2f[j]), "+v"(dg[j]), "+v"(ddg[j]));
-      x2d[j] = flip(x2f[j], x.ident);
-      const frag nx = upd ? neg(x2d[j]) : IO::zero();
+      const frag nx = upd ? neg(flip(x2f[j], x.ident)) : IO::zero();
 #pragma unroll
       for (int I = 0; I < NT; ++I) IO::mma(W2c[j][I], nx, x.GS[I * 64 + lane]);
       RP_FENCE();
@@ -546,39 +613,47 @@ __device__ __forceinline__ void producer(const MlpBwdRpArgs& a, unsigned char* s
     for (int j = 0; j < HT; ++j)
 #pragma unroll
       for (int I = 0; I < NT; ++I) forget(W2c[j][I]);
+    {
+      f32x4 acc[HT];
 #pragma unroll
-    for (int j = 0; j < HT; ++j) {
-      f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+      for (int j = 0; j < HT; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int q = 0; q < NQ; ++q) {
-        const frag t0 = flip(IO::to_frag(W2c[j][2 * q]), x.ident), t1 = flip(IO::to_frag(W2c[j][2 * q + 1]), x.ident);
-        at<u32x4>(sw, S::W2T + (j * NQ + q) * 1024 + 16u * lane) = rp::pair(t0, t1);
-        IO::mma2(acc, t0, t1, x.GT[(2 * q) * 64 + lane], x.GT[(2 * q + 1) * 64 + lane]);
+        const frag g0 = x.GT[(2 * q) * 64 + lane], g1 = x.GT[(2 * q + 1) * 64 + lane];
+        f32x4 f0[HT], f1[HT];
+#pragma unroll
+        for (int j = 0; j < HT; ++j) {
+          f0[j] = f1[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+          IO::mma(f0[j], IO::to_frag(W2c[j][2 * q]), x.ident);
+          IO::mma(f1[j], IO::to_frag(W2c[j][2 * q + 1]), x.ident);
+        }
+#pragma unroll
+        for (int j = 0; j < HT; ++j) {
+          const frag t0 = IO::to_frag(f0[j]), t1 = IO::to_frag(f1[j]);
+          at<u32x4>(sw, S::W2T + (j * NQ + q) * 1024 + 16u * lane) = rp::pair(t0, t1);
+          IO::mma2(acc[j], t0, t1, g0, g1);
+        }
+        RP_FENCE();
       }
-      const f32x4 g1 = acc * dg[j];
-      g1b[j] = IO::to_frag(g1);
-      g1n[j] = flip(g1b[j], x.ident);
-      at<f32x4>(sw, S::DG + j * 1024 + 16u * lane) = dg[j];
-      at<f32x4>(sw, S::UG + j * 1024 + 16u * lane) = acc * ddg[j];
-      at<f32x4>(sw, S::G1 + j * 1024 + 16u * lane) = g1;
-      RP_FENCE();
+#pragma unroll
+      for (int j = 0; j < HT; ++j) {
+        const f32x4 g1 = acc[j] * dg[j];
+        g1b[j] = IO::to_frag(g1);
+        at<f32x4>(sw, S::DG + j * 1024 + 16u * lane) = dg[j];
+        at<f32x4>(sw, S::UG + j * 1024 + 16u * lane) = acc[j] * ddg[j];
+        at<f32x4>(sw, S::G1 + j * 1024 + 16u * lane) = g1;
+      }
+#pragma unroll
+      for (int j = 0; j < HT; ++j) g1n[j] = flip(g1b[j], x.ident);
     }
-#pragma unroll
-    for (int j = 0; j < HT; ++j)
-#pragma unroll
-      for (int I = 0; I < NT; ++I) forget(W1c[I][j]);
-    f32x4 zq[HT], At = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int j = 0; j < HT; ++j) zq[j] = *reinterpret_cast<const f32x4*>(x.B1s + 16 * (w * HT + j) + 4 * g);
+    RP_FENCE();
+    f32x4 At = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int q = 0; q < NQ; ++q) {
       frag k0, k1, q0, q1;
       IO::load8(x.row(st, 1) + 32 * q + 8 * g, true, k0, k1);
       IO::load8(x.row(st, 0) + 32 * q + 8 * g, true, q0, q1);
-#pragma unroll
-      for (int j = 0; j < HT; ++j) IO::mma2(zq[j], IO::to_frag(W1c[2 * q][j]), IO::to_frag(W1c[2 * q + 1][j]), q0, q1);
       IO::mma2(At, k0, k1, q0, q1);
-      RP_FENCE();
     }
     {
       f32x4 m;
@@ -666,8 +741,8 @@ __device__ __forceinline__ void producer(const MlpBwdRpArgs& a, unsigned char* s
       const f32x4 dz = (gam * dO - s1 - xh * s2) * rstd, zs = over_tokens(dz);
       if (c == 0) at<f32x4>(sl, S::ZB2 + 4u * x.own) = zs;
       const frag zt = IO::to_frag(dz), zd = flip(zt, x.ident);
-      dgam += dO * xh;
-      dbet += dO;
+      dgam() += dO * xh;
+      dbet() += dO;
       x.ZT[w * 64 + lane] = zt;
       at<frag>(stl, S::ZD + 8u * lane) = zd;
       f32x4 mz = {0.f, 0.f, 0.f, 0.f};  // M2^T dZbar2
@@ -680,9 +755,8 @@ __device__ __forceinline__ void producer(const MlpBwdRpArgs& a, unsigned char* s
     RP_RELANE();
 
     // ================= F: dXbar2, dZbar1; partial P1 and dQ
-    if (red && st > a.first)
-      x.KD[((par ^ 1) * NT + w) * 64 + lane] = flip(load4<BF16>(x.row(st - 1, 1) + x.own), x.ident);
     if (st > a.first) load_factors(st - 1);
+    x.peek(fl, 1);
     f32x4 Pm = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int q = 0; q < NQ; ++q)
@@ -706,7 +780,7 @@ __device__ __forceinline__ void producer(const MlpBwdRpArgs& a, unsigned char* s
       for (int q = 0; q < NQ; ++q)
         IO::mma2(acc, flip(IO::to_frag(W2c[j][2 * q]), x.ident), flip(IO::to_frag(W2c[j][2 * q + 1]), x.ident),
                  x.ZT[(2 * q) * 64 + lane], x.ZT[(2 * q + 1) * 64 + lane]);
-      mmz(acc, x2d[j], dA2f);
+      mmz(acc, flip(x2f[j], x.ident), dA2f);
       const f32x4 dz = acc * dgz[j], zs = over_tokens(dz);
       if (c == 0) at<f32x4>(sl, S::ZB1 + (w * HT + j) * 64 + 16u * g) = zs;
       dzb[j] = IO::to_frag(dz);
@@ -756,7 +830,7 @@ __device__ __forceinline__ void producer(const MlpBwdRpArgs& a, unsigned char* s
       const frag dA1f = IO::to_frag(m);
       if (red) {
         f32x4 dq = x.sum_tile(par, w) + dO;
-        IO::mma(dq, x.KD[(par * NT + w) * 64 + lane], dA1f);
+        IO::mma(dq, x.token_k(st, 1, w), dA1f);
         if (c < K)
           store4<BF16>(x.out_row(a.d_xq, st), dq);
         x.GS[w * 64 + lane] = gd;
@@ -800,7 +874,7 @@ __device__ __forceinline__ void producer(const MlpBwdRpArgs& a, unsigned char* s
     for (int i = tid; i < F; i += 512) a.b1[bh * F + i] = x.B1s[i];
     if (red && c == 0) *reinterpret_cast<f32x4*>(a.b2 + bh * D + x.own) = b2T;
   }
-  x.add_norm_grads(dgam, dbet);
+  x.add_norm_grads(dgam(), dbet());
 }
 
 template <int D>
@@ -821,13 +895,12 @@ __device__ __forceinline__ void consumer(const MlpBwdRpArgs& a, unsigned char* s
     my_xcc &= 15u;
     if (tid == 0) __hip_atomic_store(fl + 3, 0x100u | my_xcc, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
-  if (tid == 0) *x.lost = pair && a.spin_limit == 0 ? 1 : 0;
+  if (tid == 0) x.lost[0] = pair && a.spin_limit == 0 ? 1 : 0, x.lost[1] = 0;
   // sums that only the reducers touch, once per mini-batch, live in LDS: the registers are short
   auto dgam = [&]() -> f32x4& { return x.PA[(red ? w : 0) * 64 + lane]; };
   auto dbet = [&]() -> f32x4& { return reinterpret_cast<f32x4*>(smem + B::L::DB)[(red ? w : 0) * 64 + lane]; };
   auto db2 = [&]() -> f32x4& { return *reinterpret_cast<f32x4*>(smem + B::L::B2 + 4 * x.own); };
-  // second use of LDS regions: XQ tiles with tokens along k where the producer keeps G2'', dZ2 beside its other orientation
-  frag* const QD = x.GS;
+  // second use of an LDS region: dZ2 beside its other orientation
   frag* const ZDs = x.GT;
   // G2 in both orientations and dZbar2: where the staging area has room for two tensors more than are staged here
   frag* const GTs = reinterpret_cast<frag*>(smem + B::L::IN + 2 * B::L::TILE);
@@ -923,15 +996,6 @@ __device__ __forceinline__ void consumer(const MlpBwdRpArgs& a, unsigned char* s
     frag x2f[HT];
     frag dt[HT];  // dZbar1: fetched again for the last part of phase D
     f32x4 dg[HT], ug[HT], gg1[HT];
-#pragma unroll
-    for (int j = 0; j < HT; ++j) {
-      x2f[j] = sl.get<frag>(16u * lane, sw + S::XT + j * 1024);
-      dt[j] = sl.get<frag>(8u * lane, sw + S::DT + j * 512);
-      gg1[j] = sl.get<f32x4>(16u * lane, sw + S::G1 + j * 1024);
-      dg[j] = sl.get<f32x4>(16u * lane, sw + S::DG + j * 1024);
-      ug[j] = sl.get<f32x4>(16u * lane, sw + S::UG + j * 1024);
-    }
-    const frag m1t = sl.get<frag>(8u * lane, S::M1T);
     // the images of W2 and W1 are fetched a feature-tile pair ahead of their use
     auto load_w2 = [&](u32x4 (&t)[HT], int q) {
 #pragma unroll
@@ -942,18 +1006,33 @@ __device__ __forceinline__ void consumer(const MlpBwdRpArgs& a, unsigned char* s
       for (int n = 0; n < HT; ++n) t[n] = sl.get<u32x4>(16u * lane, sw + S::W1T + (q * HT + n) * 1024);
     };
     u32x4 wt[2][HT];
-    load_w2(wt[0], 0);
     // column sums of dZbar1 (own hidden slice) and, reducers, of dZbar2 (own features): one value a lane
     const float zb1 = sl.get<float>(4u * (lane < 16 * HT ? lane : 0), S::ZB1 + w * HT * 64);
     const int fb2 = own_offset<1>(red ? w : 0, 0, (lane >> 2) & 3) + (lane & 3);
     const float zb2 = sl.get<float>(4u * fb2, S::ZB2);
     RP_FENCE();
     if (st + 1 < a.last) finish(st + 1);
-    const float last_c = x.te_last * x.lr_of(st, c);
-    if (red) {
-      x.KD[w * 64 + lane] = flip(load4<BF16>(x.row(st, 1) + x.own), x.ident);
-      QD[w * 64 + lane] = flip(load4<BF16>(x.row(st, 0) + x.own), x.ident);
+    RP_FENCE();
+    // gelu'(Z1) and U gelu''(Z1) wait in LDS, in the wave's own part of the partial tiles it is about to form
+    {
+      const unsigned char* const hs = x.slot(st) + sw;
+      const unsigned park = x.lds0() + B::L::PB + w * NT * 1024;
+#pragma unroll
+      for (int j = 0; j < HT; ++j) {
+        lds_dma16_dev(hs + S::DG + j * 1024, 16u * lane, park + j * 1024);
+        lds_dma16_dev(hs + S::UG + j * 1024, 16u * lane, park + (HT + j) * 1024);
+      }
     }
+#pragma unroll
+    for (int j = 0; j < HT; ++j) {
+      x2f[j] = sl.get<frag>(16u * lane, sw + S::XT + j * 1024);
+      dt[j] = sl.get<frag>(8u * lane, sw + S::DT + j * 512);
+      gg1[j] = sl.get<f32x4>(16u * lane, sw + S::G1 + j * 1024);
+    }
+    const frag m1t = sl.get<frag>(8u * lane, S::M1T);
+    load_w2(wt[0], 0);
+    RP_FENCE();
+    const float last_c = x.te_last * x.lr_of(st, c);
     f32x4 s1[HT];
 #pragma unroll
     for (int j = 0; j < HT; ++j) s1[j] = *reinterpret_cast<const f32x4*>(DB1 + 16 * (w * HT + j) + 4 * g);
@@ -969,6 +1048,12 @@ __device__ __forceinline__ void consumer(const MlpBwdRpArgs& a, unsigned char* s
     if (lane < 16 * HT) DB1[16 * w * HT + lane] += zb1;
     float qs = 0.f;
     frag duf[HT], g1b[HT];
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // what was copied to LDS has landed
+#pragma unroll
+    for (int j = 0; j < HT; ++j) {
+      dg[j] = x.PB[(w * NT + j) * 64 + lane];
+      ug[j] = x.PB[(w * NT + HT + j) * 64 + lane];
+    }
 #pragma unroll
     for (int j = 0; j < HT; ++j) {
 #pragma unroll
@@ -1058,19 +1143,12 @@ __device__ __forceinline__ void consumer(const MlpBwdRpArgs& a, unsigned char* s
     }
     lds_barrier();  // ---- C2
     RP_RELANE();
-    u32x4 wd[2][NQ];  // W2^T by hidden tile, for dX2
-    auto load_w2j = [&](u32x4 (&t)[NQ], int j) {
+    u32x4 xd[HT];  // (X2, Xbar2), fetched again rather than held since phase A
+    constexpr int AH = B::ROOM ? 2 : 1;  // feature-tile pairs of W2^T on their way
 #pragma unroll
-      for (int q = 0; q < NQ; ++q) t[q] = sl.get<u32x4>(16u * lane, sw + S::W2T + (j * NQ + q) * 1024);
-    };
-    u32x4 xd[2];
-    f32x4 dd[2];  // (X2, Xbar2) and gelu'(Z1), fetched again rather than held since phase A
-    auto load_xd = [&](int j) {
-      xd[j & 1] = sl.get<u32x4>(16u * lane, sw + S::XT + j * 1024);
-      dd[j & 1] = sl.get<f32x4>(16u * lane, sw + S::DG + j * 1024);
-    };
-    load_w2j(wd[0], 0);
-    load_xd(0);
+    for (int q = 0; q < AH && q < NQ; ++q) load_w2(wt[q], q);
+#pragma unroll
+    for (int j = 0; j < HT; ++j) xd[j] = sl.get<u32x4>(16u * lane, sw + S::XT + j * 1024);
     const frag a2t = sl.get<frag>(8u * lane, S::A2T), a1t = sl.get<frag>(8u * lane, S::A1T);
 
     // ================= C: reducers: dZ2, dT
@@ -1095,61 +1173,108 @@ __device__ __forceinline__ void consumer(const MlpBwdRpArgs& a, unsigned char* s
       const f32x4 b = db2() + over_tokens(dZ2);
       if (c == 0) db2() = b;
       dk_p = dy;  // -d target
-      IO::mma(dk_p, QD[w * 64 + lane], a1t);
+      IO::mma(dk_p, x.token_k(st, 0, w), a1t);
     }
     dl_p = dlp;
     lds_barrier();  // ---- C3
     RP_RELANE();
 
+    x.peek(fl, 0);
     // ================= D: T2, dX2, dZ1; partial dK; updates
     // (X2 : T2 is the sum G2 : X2 dW2 behind d lr; it takes G2 in two bf16 parts, 16 bits of it, so that only the operands
     // X2 and dW2 are rounded there)
-    frag dz1[HT];
+    frag dz1[HT], xbd[HT];
 #pragma unroll
     for (int j = 0; j < HT; ++j)
 #pragma unroll
       for (int I = 0; I < NT; ++I) forget(dW2c[j][I]);
+    {
+      f32x4 t[HT], acc[HT], dd[HT];  // T2; dX2; gelu'(Z1), fetched again
 #pragma unroll
-    for (int j = 0; j < HT; ++j) {
-      f32x4 t = {0.f, 0.f, 0.f, 0.f}, acc = t;
-      const frag x2 = lo(xd[j & 1]), xbd = flip(hi(xd[j & 1]), x.ident);
-      mmz(acc, xbd, a2t);
-      if (j + 1 < HT) {
-        load_w2j(wd[(j + 1) & 1], j + 1);
-        load_xd(j + 1);
-      } else {
-        load_w1(wt[0], 0);
-#pragma unroll
-        for (int n = 0; n < HT; ++n) dt[n] = sl.get<frag>(8u * lane, sw + S::DT + n * 512);
+      for (int j = 0; j < HT; ++j) {
+        xbd[j] = flip(hi(xd[j]), x.ident);
+        t[j] = acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+        mmz(acc[j], xbd[j], a2t);
       }
+      RP_FENCE();
 #pragma unroll
       for (int q = 0; q < NQ; ++q) {
-        const frag w0 = flip(IO::to_frag(dW2c[j][2 * q]), x.ident), w1 = flip(IO::to_frag(dW2c[j][2 * q + 1]), x.ident);
-        IO::mma2(t, w0, w1, GTs[(2 * q) * 64 + lane], GTs[(2 * q + 1) * 64 + lane]);
-        IO::mma2(t, w0, w1, GLs[(2 * q) * 64 + lane], GLs[(2 * q + 1) * 64 + lane]);
-        const u32x4 v = wd[j & 1][q];
-        IO::mma2(acc, lo(v), hi(v), x.ZT[(2 * q) * 64 + lane], x.ZT[(2 * q + 1) * 64 + lane]);
-      }
-      const f32x4 xf = IO::to_f32(x2);
+        const frag z0 = x.ZT[(2 * q) * 64 + lane], z1 = x.ZT[(2 * q + 1) * 64 + lane];
 #pragma unroll
-      for (int r = 0; r < 4; ++r) qs += xf[r] * t[r];
-      const f32x4 dx2 = acc - last_c * t;
-      const f32x4 dz = x.PB[((NW + w) * NT + j) * 64 + lane] + dx2 * dd[j & 1];
-      {
-        f32x4* const bp = reinterpret_cast<f32x4*>(DB1 + 16 * (w * HT + j) + 4 * g);
-        const f32x4 b = *bp + over_tokens(dz);  // (bias gradients are sums of f32 terms)
-        if (c == 0) *bp = b;
+        for (int j = 0; j < HT; ++j) IO::mma2(acc[j], lo(wt[q % AH][j]), hi(wt[q % AH][j]), z0, z1);
+        RP_FENCE();
+        if (q + AH < NQ) load_w2(wt[q % AH], q + AH);
+        if (q + 1 == NQ) {
+#pragma unroll
+          for (int j = 0; j < HT; ++j) dd[j] = sl.get<f32x4>(16u * lane, sw + S::DG + j * 1024);
+        }
+        const frag g0 = GTs[(2 * q) * 64 + lane], g1 = GTs[(2 * q + 1) * 64 + lane], l0 = GLs[(2 * q) * 64 + lane],
+                   l1 = GLs[(2 * q + 1) * 64 + lane];
+        frag w0[HT], w1[HT];
+        {
+          f32x4 f[HT];
+#pragma unroll
+          for (int j = 0; j < HT; ++j) {
+            f[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+            IO::mma(f[j], IO::to_frag(dW2c[j][2 * q]), x.ident);
+          }
+#pragma unroll
+          for (int j = 0; j < HT; ++j) w0[j] = IO::to_frag(f[j]);
+#pragma unroll
+          for (int j = 0; j < HT; ++j) {
+            f[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+            IO::mma(f[j], IO::to_frag(dW2c[j][2 * q + 1]), x.ident);
+          }
+#pragma unroll
+          for (int j = 0; j < HT; ++j) w1[j] = IO::to_frag(f[j]);
+        }
+#pragma unroll
+        for (int j = 0; j < HT; ++j) IO::mma2(t[j], w0[j], w1[j], g0, g1);
+#pragma unroll
+        for (int j = 0; j < HT; ++j) IO::mma2(t[j], w0[j], w1[j], l0, l1);
+        RP_FENCE();
       }
-      dz1[j] = IO::to_frag(dz);
-      RP_FENCE();
-      // dW2 += [X2 | dU]^T [dZ2 ; G2] + Xbar2^T dZbar2
-      const frag x2d = flip(x2, x.ident), dud = flip(wait_frag(j), x.ident);
+      load_w1(wt[0], 0);
+#pragma unroll
+      for (int n = 0; n < HT; ++n) dt[n] = sl.get<frag>(8u * lane, sw + S::DT + n * 512);
+#pragma unroll
+      for (int j = 0; j < HT; ++j) {
+        const f32x4 xf = IO::to_f32(lo(xd[j]));
+#pragma unroll
+        for (int r = 0; r < 4; ++r) qs += xf[r] * t[j][r];
+        const f32x4 dx2 = acc[j] - last_c * t[j];
+        const f32x4 dz = x.PB[((NW + w) * NT + j) * 64 + lane] + dx2 * dd[j];
+        {
+          f32x4* const bp = reinterpret_cast<f32x4*>(DB1 + 16 * (w * HT + j) + 4 * g);
+          const f32x4 b = *bp + over_tokens(dz);  // (bias gradients are sums of f32 terms)
+          if (c == 0) *bp = b;
+        }
+        dz1[j] = IO::to_frag(dz);
+      }
+    }
+    RP_FENCE();
+    // dW2 += [X2 | dU]^T [dZ2 ; G2] + Xbar2^T dZbar2
+    {
+      frag x2d[HT], dud[HT];
+#pragma unroll
+      for (int j = 0; j < HT; ++j) {
+        x2d[j] = flip(lo(xd[j]), x.ident);
+        dud[j] = flip(wait_frag(j), x.ident);
+      }
+      frag zd = ZDs[lane], gn = GNs[lane], zn = ZNs[lane];
 #pragma unroll
       for (int I = 0; I < NT; ++I) {
-        IO::mma2(dW2c[j][I], x2d, dud, ZDs[I * 64 + lane], GNs[I * 64 + lane]);
-        mmz(dW2c[j][I], xbd, ZNs[I * 64 + lane]);
+        const int In = (I + 1 < NT ? I + 1 : I) * 64;
+        const frag zd_ = ZDs[In + lane], gn_ = GNs[In + lane], zn_ = ZNs[In + lane];
+#pragma unroll
+        for (int j = 0; j < HT; ++j) IO::mma2(dW2c[j][I], x2d[j], dud[j], zd, gn);
+#pragma unroll
+        for (int j = 0; j < HT; ++j) mmz(dW2c[j][I], xbd[j], zn);
+        zd = zd_;
+        gn = gn_;
+        zn = zn_;
+        RP_FENCE();
       }
-      RP_FENCE();
     }
     {
       const float s = xg_sum(qs);
@@ -1164,27 +1289,46 @@ __device__ __forceinline__ void consumer(const MlpBwdRpArgs& a, unsigned char* s
 #pragma unroll
     for (int q = 0; q < NQ; ++q) {
       if (q + 1 < NQ) load_w1(wt[(q + 1) & 1], q + 1);
+f32x4 f[2][HT], p[2];
 #pragma unroll
       for (int u = 0; u < 2; ++u) {
-        const int I = 2 * q + u;
-        frag tn[HT];
+        p[u] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int j = 0; j < HT; ++j) tn[j] = flip(IO::to_frag(dW1c[I][j]), x.ident);
-        f32x4 p = {0.f, 0.f, 0.f, 0.f};
+        for (int j = 0; j < HT; ++j) {
+          f[u][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+          IO::mma(f[u][j], IO::to_frag(dW1c[2 * q + u][j]), x.ident);
+        }
+      }
+      frag tn[2][HT];
 #pragma unroll
-        for (int j = 0; j + 1 < HT; j += 2) IO::mma2(p, tn[j], tn[j + 1], g1b[j], g1b[j + 1]);
-        if (HT & 1) mmz(p, tn[HT - 1], g1b[HT - 1]);
-        p *= -last_c;
+      for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int j = 0; j < HT; ++j) tn[u][j] = IO::to_frag(f[u][j]);
+#pragma unroll
+      for (int j = 0; j + 1 < HT; j += 2)
+#pragma unroll
+        for (int u = 0; u < 2; ++u) IO::mma2(p[u], tn[u][j], tn[u][j + 1], g1b[j], g1b[j + 1]);
+      if (HT & 1)
+#pragma unroll
+        for (int u = 0; u < 2; ++u) mmz(p[u], tn[u][HT - 1], g1b[HT - 1]);
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        p[u] *= -last_c;
 #pragma unroll
         for (int j = 0; j < HT; ++j) {
           const int n = u * HT + j;
-          tn[j] = (n & 1) ? hi(wt[q & 1][n >> 1]) : lo(wt[q & 1][n >> 1]);
+          tn[u][j] = (n & 1) ? hi(wt[q & 1][n >> 1]) : lo(wt[q & 1][n >> 1]);
         }
-#pragma unroll
-        for (int j = 0; j + 1 < HT; j += 2) IO::mma2(p, tn[j], tn[j + 1], dz1[j], dz1[j + 1]);
-        if (HT & 1) mmz(p, tn[HT - 1], dz1[HT - 1]);
-        x.PB[((NW + w) * NT + I) * 64 + lane] = p;
       }
+#pragma unroll
+      for (int j = 0; j + 1 < HT; j += 2)
+#pragma unroll
+        for (int u = 0; u < 2; ++u) IO::mma2(p[u], tn[u][j], tn[u][j + 1], dz1[j], dz1[j + 1]);
+      if (HT & 1)
+#pragma unroll
+        for (int u = 0; u < 2; ++u) mmz(p[u], tn[u][HT - 1], dz1[HT - 1]);
+#pragma unroll
+      for (int u = 0; u < 2; ++u) x.PB[((NW + w) * NT + 2 * q + u) * 64 + lane] = p[u];
       RP_FENCE();
     }
     // dW1 += [XQ | XK]^T [dZbar1 ; dZ1]
@@ -1196,7 +1340,7 @@ __device__ __forceinline__ void consumer(const MlpBwdRpArgs& a, unsigned char* s
     }
 #pragma unroll
     for (int I = 0; I < NT; ++I) {
-      const frag qd = QD[I * 64 + lane], kd = x.KD[I * 64 + lane];
+      const frag qd = x.token_k(st, 0, I), kd = x.token_k(st, 1, I);
 #pragma unroll
       for (int j = 0; j < HT; ++j) IO::mma2(dW1c[I][j], qd, kd, dzd[j], dz1d[j]);
       RP_FENCE();
@@ -1260,5 +1404,17 @@ __global__ void __launch_bounds__(512) ttt_mlp_bwd_rp_kernel(MlpBwdRpArgs a) {
 
 #undef RP_RELANE
 #undef RP_FENCE
+
+template <int D>
+hipError_t launch_mlp_bwd_rp_d(const MlpBwdRpArgs& a, hipStream_t s) {
+  constexpr auto kern = ttt_mlp_bwd_rp_kernel<D>;
+  constexpr int bytes = MlpRpLds<D>::BYTES;
+  const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+  if (e != hipSuccess) return e;
+  // two workgroups per unit: workgroups b and b + 8 of every 16 share a unit
+  const unsigned units = (unsigned)(a.B * a.H), grid = a.role == 2 ? (units + 7) / 8 * 16 : units;
+  hipLaunchKernelGGL(kern, dim3(grid), dim3(512), bytes, s, a);
+  return hipGetLastError();
+}
 
 }  // namespace ttt
