@@ -494,7 +494,6 @@ __global__ void __launch_bounds__(512) ttt_mlp_fwd_rr_kernel(Problems<MlpFwdArgs
     RELANE();
 
     // ================= phase C: reducers: G2''; the other waves: the rest of Zbar2
-    frag g2_saved = IO::zero();
     if (red) {
       const float lrc = (c < K) ? __uint_as_float(LRs[buf * 16 + c] << 16) : 0.f;
       float S[6];
@@ -525,9 +524,7 @@ __global__ void __launch_bounds__(512) ttt_mlp_fwd_rr_kernel(Problems<MlpFwdArgs
       const float c1 = p * rstd, c2 = -c1 * s2 * inv_d, c3 = -p * s1 * inv_d;
       const f32x4 gam = *reinterpret_cast<const f32x4*>(GAM + own);
       const f32x4 G = (z - mu) * (gam * gam * c1 + c2) + (bq * p + c3);
-      const frag gt = IO::to_frag(G);
-      GTc[w * 64 + lane] = gt;
-      g2_saved = gt;
+      GTc[w * 64 + lane] = IO::to_frag(G);
       if (st > 0) qo = load4<T>(row((st + 2) % 3, 0) + own);
     } else if (st > 0) {
       output_moments(st - 1);
@@ -541,13 +538,13 @@ __global__ void __launch_bounds__(512) ttt_mlp_fwd_rr_kernel(Problems<MlpFwdArgs
     // The factors of this mini-batch's state update for ttt_mlp_bwd, eta_last * G1 [16 x 4d] and eta_last * G2
     // [16 x d] (row = token), exactly as the update applies them: rounded to the operand type, sign undone
     // (G'' = -eta_last * lr * G); zeros when token_eta[K-1] = 0 switches the update off.
-    const size_t save_row = (bh * (size_t)a.n_stages + st) * 16 + c;
-    unsigned char* const facp =
-        SAVE && a.fac_save != nullptr ? a.fac_save + (bh * (size_t)a.n_stages + st) * ((NW * HT + NT) * 512) : nullptr;
-    if (SAVE && facp != nullptr && red) *reinterpret_cast<frag*>(facp + (NW * HT + w) * 512 + lane * 8) = read_tr(GTc + w * 64 + tr_lane(lane));
+    const size_t saved_at = bh * (size_t)n_stages + st;
+    unsigned char* const facp = SAVE && a.fac_save != nullptr ? a.fac_save + saved_at * ((NW * HT + NT) * 512) : nullptr;
+    if (SAVE && facp != nullptr && red)
+      *reinterpret_cast<frag*>(facp + (NW * HT + w) * 512 + 8u * lane) = read_tr(GTc + w * 64 + tr_lane(lane));
     if (SAVE && a.G2_save != nullptr && red) {
-      const f32x4 v = upd ? -IO::to_f32(g2_saved) : f32x4{0.f, 0.f, 0.f, 0.f};
-      *reinterpret_cast<f32x4*>(a.G2_save + save_row * D + own) = v;
+      const f32x4 v = upd ? -IO::to_f32(GTc[w * 64 + lane]) : f32x4{0.f, 0.f, 0.f, 0.f};
+      *reinterpret_cast<f32x4*>(a.G2_save + saved_at * (16 * D) + (unsigned)(c * D + own)) = v;
     }
 #pragma unroll
     for (int j = 0; j < HT; ++j)
@@ -582,13 +579,13 @@ __global__ void __launch_bounds__(512) ttt_mlp_fwd_rr_kernel(Problems<MlpFwdArgs
         IO::mma(t[j], g1b, ident);
         if (SAVE && a.G1_save != nullptr) {
           const f32x4 v = upd ? -IO::to_f32(g1b) : f32x4{0.f, 0.f, 0.f, 0.f};
-          *reinterpret_cast<f32x4*>(a.G1_save + save_row * F + 16 * (w * HT + j) + 4 * g) = v;
+          *reinterpret_cast<f32x4*>(a.G1_save + saved_at * (16 * F) + 16 * (w * HT + j) + (unsigned)(c * F + 4 * g)) = v;
         }
       }
 #pragma unroll
       for (int j = 0; j < HT; ++j) {
         G1d[j] = IO::to_frag(t[j]);
-        if (SAVE && facp != nullptr) *reinterpret_cast<frag*>(facp + (w * HT + j) * 512 + lane * 8) = G1d[j];
+        if (SAVE && facp != nullptr) *reinterpret_cast<frag*>(facp + (w * HT + j) * 512 + 8u * lane) = G1d[j];
       }
     }
     // Zbar1^T = (XQ W1 + b1)^T + G1''^T M1
