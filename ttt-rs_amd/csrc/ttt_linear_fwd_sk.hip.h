@@ -75,6 +75,12 @@ __device__ __forceinline__ void linear_fwd_sk_body(const LinearFwdArgs& a, const
   __shared__ f32x4 atx[SHARE ? 2 : 1][SHARE ? NW : 1][64];
 
   constexpr bool DMA = RAW == 5;
+  // XK with tokens along k, for the state update: where the rows are shared through LDS anyway, the transposing LDS load
+  // gives it, instead of a matrix instruction and two conversions per tile (the waves are bound by what they issue; 384 units
+  // x 2048 tokens, d = 64: 127.0 -> 126.1 us, saving update factors 7 us less).  A zero token_eta[K-1] then masks G'' in the
+  // update, where it makes the transpose zero otherwise.  Not where the operands are formed here (a layer 199.3 -> 200.1 us)
+  // and not with the Adam step (230 -> 240 us), whose loops are scheduled worse with it.
+  constexpr bool TRK = RAW >= 3 && !DMA && BF && !ADAM;
   const int lane = threadIdx.x & 63, w = (threadIdx.x >> 6) % NW;
   // RAW = 5: the wave behind the compute waves is the control wave; up to the point where it branches off it does what
   // wave 0 does (w == 0: valid loads, LDS writes of the same values) and it stores nothing
@@ -272,6 +278,15 @@ __device__ __forceinline__ void linear_fwd_sk_body(const LinearFwdArgs& a, const
   };
   // token_eta[K-1] == 0 means "no state update": instead of a branch inside the loop the two operands
   // that carry tokens into the update (XK^T, the ones column of the bias update) are made zero
+  const unsigned upd_mask = upd ? ~0u : 0u;
+  auto and_mask = [](frag f, unsigned m) -> frag {
+    if constexpr (BF) {
+      const u32x2 v = __builtin_bit_cast(u32x2, f);
+      return __builtin_bit_cast(frag, u32x2{v[0] & m, v[1] & m});
+    } else {
+      return f;
+    }
+  };
   const frag ident_upd = upd ? ident : IO::zero();
   const frag ones_upd = upd ? ones : IO::zero();
 
@@ -550,6 +565,11 @@ __device__ __forceinline__ void linear_fwd_sk_body(const LinearFwdArgs& a, const
         f32x4 t = {0.f, 0.f, 0.f, 0.f};
         IO::mma(t, cur.ko[0], ident_upd);  // the own tile; the others come back from LDS behind the barrier
         kdx[st & 1][w][lane] = t;
+      } else if constexpr (TRK) {
+        // (the rows lie there as fragments, tokens across lanes; they are overwritten behind the next barrier)
+        const u32x4* const xk = xrot + ((st & 1) * 2 + 1) * (NT / 2) * 64 + tr_lane(lane);
+#pragma unroll
+        for (int I = 0; I < NT; ++I) kd[I] = read_tr(reinterpret_cast<const unsigned char*>(xk + (I >> 1) * 64) + 8 * (I & 1));
       } else {
 #pragma unroll
         for (int I = 0; I < NT; ++I) {
@@ -698,10 +718,13 @@ __device__ __forceinline__ void linear_fwd_sk_body(const LinearFwdArgs& a, const
           adam_tile(bT[jj], bm[jj], bv[jj], gneg);
         }
       } else {
+        frag Gu[TPW];
+#pragma unroll
+        for (int jj = 0; jj < TPW; ++jj) Gu[jj] = TRK ? and_mask(Gd[jj], upd_mask) : Gd[jj];
 #pragma unroll
         for (int I = 0; I < NT; ++I)
 #pragma unroll
-          for (int jj = 0; jj < TPW; ++jj) IO::mma(Wc[I][jj], kd[I], Gd[jj]);
+          for (int jj = 0; jj < TPW; ++jj) IO::mma(Wc[I][jj], kd[I], Gu[jj]);
         bias_update(bT, Gd, ones_upd);
       }
       // this mini-batch's Zbar and xq become the pending output; its in-lane sums are formed here, in the
@@ -716,7 +739,7 @@ __device__ __forceinline__ void linear_fwd_sk_body(const LinearFwdArgs& a, const
       }
       // RAW: the own features of the mini-batch after the next, loaded during the previous pass of the loop; read
       // back by every wave behind the next barrier.  LDS buffer st & 1 was last read behind the barrier of the
-      // previous mini-batch, which every wave has left.
+      // previous mini-batch (TRK: in front of this one's), which every wave has left.
       if constexpr (RAW != 0) rotate_share(raw[(u + 2) % R], buf[(u + 2) % R], st + 2, st & 1);
     }
   };
@@ -755,11 +778,17 @@ __device__ __forceinline__ void linear_fwd_sk_body(const LinearFwdArgs& a, const
         // ---- XK with tokens along k for the state update: depends on nothing computed here, so it
         // is issued first and fills the gaps of the dependent chain below
         frag kd[NT];
+        if constexpr (TRK) {
+          const u32x4* const xk = xrot + ((st & 1) * 2 + 1) * (NT / 2) * 64 + tr_lane(lane);
 #pragma unroll
-        for (int I = 0; I < NT; ++I) {
-          f32x4 t = {0.f, 0.f, 0.f, 0.f};
-          IO::mma(t, cur.k[I], ident);  // t[r] = XK[s = 4g+r][feat(I,c)]
-          kd[I] = IO::to_frag(t);
+          for (int I = 0; I < NT; ++I) kd[I] = read_tr(reinterpret_cast<const unsigned char*>(xk + (I >> 1) * 64) + 8 * (I & 1));
+        } else {
+#pragma unroll
+          for (int I = 0; I < NT; ++I) {
+            f32x4 t = {0.f, 0.f, 0.f, 0.f};
+            IO::mma(t, cur.k[I], ident);  // t[r] = XK[s = 4g+r][feat(I,c)]
+            kd[I] = IO::to_frag(t);
+          }
         }
         // ---- Z1^T, Zbar^T (this wave's feature rows) and the attention block
         f32x4 z1[TPW], zb[TPW], At = {0.f, 0.f, 0.f, 0.f};
