@@ -12,9 +12,9 @@
 //   X1  six raw moments of Z1 (mean, variance and both sums of the LN-L2 gradient follow from them), the
 //       partial attention blocks, XK^T / XQ^T fragments (tokens along k);
 //   X2  four raw moments of Zbar and of the output-LayerNorm backward; G fragments;
-//   X3  partial P = dZbar G^T, dZbar fragments in both forms, and the six sums of the second-order LayerNorm
+//   X3  partial P = dZbar G^T, dZbar fragments (f32 I/O: in both forms), and the six sums of the second-order LayerNorm
 //       (all its statistics are linear in them; none needs P, so one exchange carries both);
-//   X4  dZ1 fragments in both forms.
+//   X4  dZ1 fragments (f32 I/O: in both forms).
 // All matrix products with a d-deep contraction over the OTHER slices' features take those fragments as B
 // operands; products over tokens (rank-16) are local.  f32 I/O computes in true-f32 MFMA
 // (v_mfma_f32_16x16x4_f32), bf16 I/O in bf16 MFMA with f32 accumulation.
@@ -258,6 +258,23 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && D / 16 == NW && (PK || si
     IO::mma(t, x, ident);
     return IO::to_frag(t);
   };
+  // The same for a tile that lies in LDS as fragments, `step` bytes from lane to lane: bf16 takes it from there with the
+  // transposing load, which costs no matrix instruction and no conversion (d = 64: 11 of a mini-batch's 14 transposes; forward
+  // and backward, 384 units x 2048 tokens, 596 -> 568 us).  What a wave has just computed and needs at once stays with
+  // tokens_k: a write to LDS and a read back is the longer way.
+  const int trl = tr_lane(lane);
+  auto tokens_k_lds = [&](const void* tile, int step) -> frag {
+    const unsigned char* p = static_cast<const unsigned char*>(tile);
+    if constexpr (BF)
+      return read_tr(p + trl * step);
+    else
+      return tokens_k(*reinterpret_cast<const frag*>(p + lane * step));
+  };
+  auto tile_ptr = [&](int kind, int J) { return FRp + (kind * NT + J) * 64; };
+  // tile J of an activation tensor in the staging area
+  auto row_ptr = [&](int tensor, int J) {
+    return smem + L::X + (BF ? (tensor * XS + (J >> 1)) * 1024 + 8 * (J & 1) : (tensor * XS + J) * 1024);
+  };
   // acc += sum over the NT tiles of A[J] B[J]
   auto mma_all = [&](f32x4& acc, const frag (&A)[NT], const frag (&B)[NT]) {
 #pragma unroll
@@ -321,14 +338,9 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && D / 16 == NW && (PK || si
   // packed image of the current state is no longer read), so it is off the chain of dependent exchanges.
   auto walk_back = [&]() {
     if constexpr (FM) {
-      const unsigned char* sl = smem + lane * 16;
       frag kda[NT];
 #pragma unroll
-      for (int s = 0; s < XS; ++s) {
-        const u32x4 rk = *reinterpret_cast<const u32x4*>(sl + L::X + (1 * XS + s) * 1024);
-        kda[2 * s] = tokens_k(__builtin_bit_cast(frag, u32x2{rk[0], rk[1]}));
-        kda[2 * s + 1] = tokens_k(__builtin_bit_cast(frag, u32x2{rk[2], rk[3]}));
-      }
+      for (int I = 0; I < NT; ++I) kda[I] = tokens_k_lds(row_ptr(1, I), 16);
       frag nG[TPW];
 #pragma unroll
       for (int jj = 0; jj < TPW; ++jj) {
@@ -420,13 +432,13 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && D / 16 == NW && (PK || si
         bT[ii] = *reinterpret_cast<const f32x4*>(sl + L::Bv + Io * 1024) - bbar;
 #pragma unroll
       for (int J = 0; J < NT; ++J) {
-        if constexpr (PK)  // stored as (m = j, k = i): transposed on the matrix pipe
-          Wn[ii][J] = tokens_k(*reinterpret_cast<const frag*>(sl + pk_off(Io, J)));
+        if constexpr (PK)  // stored as (m = j, k = i)
+          Wn[ii][J] = tokens_k_lds(smem + pk_off(Io, J), 16);
         else
           Wn[ii][J] = IO::to_frag(*reinterpret_cast<const f32x4*>(sl + L::W + (Io * NT + J) * 1024) - mrowo[ii]);
       }
-      kdo[ii] = tokens_k(ko[ii]);
-      qdo[ii] = tokens_k(qo[ii]);
+      kdo[ii] = tokens_k_lds(row_ptr(1, Io), 16);
+      qdo[ii] = tokens_k_lds(row_ptr(0, Io), 16);
       fr(KD, Io) = kdo[ii];
       fr(QD, Io) = qdo[ii];
     }
@@ -569,7 +581,7 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && D / 16 == NW && (PK || si
         if constexpr (TDB) dbT[jj] += dzb;
         Zd[jj] = tokens_k(Zf[jj]);
         fr(ZF, w * TPW + jj) = Zf[jj];
-        fr(ZD, w * TPW + jj) = Zd[jj];
+        if constexpr (!BF) fr(ZD, w * TPW + jj) = Zd[jj];
         if (BF) {
           // P feeds the gradients of eta (small differences of large sums): bf16 head + tail of both factors
           Gl[jj] = IO::to_frag(G[jj] - IO::to_f32(Gf[jj]));
@@ -713,9 +725,8 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && D / 16 == NW && (PK || si
         const f32x4 dz1 = (dxh - q1) * rstd1 + xh[jj] * (dsig * inv_d);
         Z1f[jj] = IO::to_frag(dz1);
         if constexpr (TDB) dbT[jj] += dz1;
-        Z1d[jj] = tokens_k(Z1f[jj]);
         fr(Z1F, w * TPW + jj) = Z1f[jj];
-        fr(Z1D, w * TPW + jj) = Z1d[jj];
+        if constexpr (!BF) fr(Z1D, w * TPW + jj) = Z1d[jj] = tokens_k(Z1f[jj]);
         dK[jj] += dy - last * TMP[jj];
         ndy[jj] = -dy;
       }
@@ -759,9 +770,21 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && D / 16 == NW && (PK || si
     };
     if constexpr (FM) single_wave_outputs();
     // ---- state gradient: dW += XQ^T dZb + XK^T dZ1 (column slice and transposed row slice), db
+    if constexpr (BF) {
+#pragma unroll
+      for (int jj = 0; jj < TPW; ++jj) Z1d[jj] = read_tr(tile_ptr(Z1F, w * TPW + jj) + trl);
+    }
 #pragma unroll
     for (int I = 0; I < NT; ++I) {
-      const frag qa = fr(QD, I), ka = fr(KD, I), za = fr(ZD, I), z1a = fr(Z1D, I);
+      const frag qa = fr(QD, I), ka = fr(KD, I);
+      frag za, z1a;
+      if constexpr (BF) {
+        za = read_tr(tile_ptr(ZF, I) + trl);
+        z1a = read_tr(tile_ptr(Z1F, I) + trl);
+      } else {
+        za = fr(ZD, I);
+        z1a = fr(Z1D, I);
+      }
 #pragma unroll
       for (int jj = 0; jj < TPW; ++jj) {
         IO::mma2(dWc[I][jj], qa, ka, Zd[jj], Z1d[jj]);
