@@ -266,19 +266,30 @@ int launch_linear_fwd_wide(const ttt::LinearFwdArgs* probs, unsigned ny, hipStre
       return hip_status(hipGetLastError(), "ttt_linear_fwd launch");
     }
   }
-  if constexpr (!f32 && D == 96) {
-    if (a.ckpt_packed == ttt::kCkptFactors) {
-      if (a.K == 16)
-        hipLaunchKernelGGL((ttt::ttt_linear_fwd_sk_kernel<T, D, NW, PF, true, true>), grid, block, 0, s, P);
-      else
-        hipLaunchKernelGGL((ttt::ttt_linear_fwd_sk_kernel<T, D, NW, PF, false, true>), grid, block, 0, s, P);
-      return hip_status(hipGetLastError(), "ttt_linear_fwd launch");
+  // bf16 I/O: a wave loads only the features it owns, the full rows cross LDS (RAW = 3; same sizes and forms as RAW = 0, which
+  // every wave's loads of whole rows bound: 24 of 36 KB per mini-batch and unit at d = 128 were loads of what another
+  // wave loads too).  2048 tokens, d = 96: 4 units 159 -> 139 us, 64 184 -> 143, 512 381 -> 289; d = 128: 4 units 227 -> 161,
+  // 64 278 -> 168, 512 576 -> 342; four mini-batches and a single one gain as well, so no count of units keeps RAW = 0.
+  if constexpr (!f32) {
+    if constexpr (D == 96) {
+      if (a.ckpt_packed == ttt::kCkptFactors) {
+        if (a.K == 16)
+          hipLaunchKernelGGL((ttt::ttt_linear_fwd_sk_kernel<T, D, NW, PF, true, true, 1>), grid, block, 0, s, P);
+        else
+          hipLaunchKernelGGL((ttt::ttt_linear_fwd_sk_kernel<T, D, NW, PF, false, true, 1>), grid, block, 0, s, P);
+        return hip_status(hipGetLastError(), "ttt_linear_fwd launch");
+      }
     }
+    if (a.K == 16)
+      hipLaunchKernelGGL((ttt::ttt_linear_fwd_sk_kernel<T, D, NW, PF, true, false, 1>), grid, block, 0, s, P);
+    else
+      hipLaunchKernelGGL((ttt::ttt_linear_fwd_sk_kernel<T, D, NW, PF, false, false, 1>), grid, block, 0, s, P);
+  } else {
+    if (a.K == 16)
+      hipLaunchKernelGGL((ttt::ttt_linear_fwd_sk_kernel<T, D, NW, PF, true>), grid, block, 0, s, P);
+    else
+      hipLaunchKernelGGL((ttt::ttt_linear_fwd_sk_kernel<T, D, NW, PF, false>), grid, block, 0, s, P);
   }
-  if (a.K == 16)
-    hipLaunchKernelGGL((ttt::ttt_linear_fwd_sk_kernel<T, D, NW, PF, true>), grid, block, 0, s, P);
-  else
-    hipLaunchKernelGGL((ttt::ttt_linear_fwd_sk_kernel<T, D, NW, PF, false>), grid, block, 0, s, P);
   return hip_status(hipGetLastError(), "ttt_linear_fwd launch");
 }
 
