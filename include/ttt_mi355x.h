@@ -97,12 +97,12 @@ typedef struct ttt_desc {
 #define TTT_HINT_LDS_TILES 0x100
 /* ttt_mlp_fwd, bf16 I/O at head_dim 96: spread every (batch, head) unit over a pair of CUs, as head_dim 128 always is
  * (see ttt_mlp_fwd), when the units number at most half the device's CUs.  Not the default: measured on MI355X the
- * pair gains 2 - 3 % at 128 units.  Ignored where only one of the two kernels exists. */
+ * pair gains 7 % at 128 units.  Ignored where only one of the two kernels exists. */
 #define TTT_HINT_TWO_CU 0x400
-/* ttt_linear_fwd, bf16 I/O at head_dim 64 with two waves per unit: TTT_HINT_OWN_LOADS = every wave loads only the
+/* ttt_linear_fwd, bf16 I/O at head_dim 32 / 64 with two waves per unit: TTT_HINT_OWN_LOADS = every wave loads only the
  * features it owns of xq, xk, xv and the full rows reach the waves through LDS (half the vector loads; the library's
- * choice above 256 units, where two workgroups share a CU); TTT_HINT_ALL_LOADS = every wave loads every row (the
- * library's choice up to 256 units).  Same results bit for bit.  Ignored where only one of the two exists.
+ * choice but for long sequences of up to 32 units at head_dim 64); TTT_HINT_ALL_LOADS = every wave loads every row (the
+ * library's choice there).  Same results bit for bit.  Ignored where only one of the two exists.
  * ttt_linear_fwd, f32 I/O with one wave per feature tile (head_dim 32 / 64), whole mini-batches of 16 tokens and at
  * most one (batch, head) unit per CU: the library's choice is a kernel with a fifth wave that copies the operands
  * global -> LDS, so that the four compute waves issue no loads; TTT_HINT_ALL_LOADS keeps the loads in the compute

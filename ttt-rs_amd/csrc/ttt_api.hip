@@ -165,16 +165,17 @@ int launch_linear_fwd_nw(const ttt::LinearFwdArgs* probs, unsigned ny, hipStream
       hipLaunchKernelGGL((ttt::ttt_linear_fwd_mw_kernel<T, D, 1, PF, false>), grid, block, 0, s, P);
   } else {
     constexpr int NWS = NW > 1 ? NW : 2;  // the skewed kernel needs at least two waves
-    // bf16, head_dim 64, two waves per unit: the variant in which a wave loads only the features it owns and the
-    // full rows cross LDS (same bits).  Measured on MI355X (seq 2048): 24 units 117 us against 114 us, 252 units
-    // 120 against 120, 384 units 129 - 139 against 137 - 146: it pays once two workgroups share a CU's load path.
-    if constexpr (can_fac && NWS == 2 && D == 64) {
-      if (sums) {  // operands formed as x + projections (a layer of a stack); no checkpoints in that mode
-        if (a.K == 16)
-          hipLaunchKernelGGL((ttt::ttt_linear_fwd_sk_kernel<T, D, NWS, PF, true, false, 2>), grid, block, 0, s, P);
-        else
-          hipLaunchKernelGGL((ttt::ttt_linear_fwd_sk_kernel<T, D, NWS, PF, false, false, 2>), grid, block, 0, s, P);
-        return hip_status(hipGetLastError(), "ttt_linear_fwd launch");
+    // bf16, two waves per unit: the variant in which a wave loads only the features it owns and the full rows cross LDS
+    // (same bits), see launch_linear_fwd
+    if constexpr (can_fac && NWS == 2) {
+      if constexpr (D == 64) {
+        if (sums) {  // operands formed as x + projections (a layer of a stack); no checkpoints in that mode
+          if (a.K == 16)
+            hipLaunchKernelGGL((ttt::ttt_linear_fwd_sk_kernel<T, D, NWS, PF, true, false, 2>), grid, block, 0, s, P);
+          else
+            hipLaunchKernelGGL((ttt::ttt_linear_fwd_sk_kernel<T, D, NWS, PF, false, false, 2>), grid, block, 0, s, P);
+          return hip_status(hipGetLastError(), "ttt_linear_fwd launch");
+        }
       }
       if (own_loads) {
         if (fac) {
@@ -239,8 +240,12 @@ int launch_linear_fwd(const ttt::LinearFwdArgs* probs, int hint, unsigned ny, hi
   if constexpr (max_nw >= 4) {
     if (nw >= 4) return launch_linear_fwd_nw<T, D, 4>(probs, ny, s, false, ctl_wave);
   }
-  // a launch that puts two workgroups on a CU, or a caller that asks for it
-  const bool own_loads = units > 256 ? (hint & TTT_HINT_ALL_LOADS) == 0 : (hint & TTT_HINT_OWN_LOADS) != 0;
+  // bf16: own-feature loads, except for long sequences of a few units at d = 64, where the trip through LDS costs more than the
+  // loads it saves.  Every wave's loads of whole rows -> own features, 2048 tokens, d = 64: 4 units 112.3 -> 113.0 us, 24
+  // 114.0 -> 114.3, 96 122.6 -> 117.0, 256 127.6 -> 118.1, saving update factors 136.7 -> 122.0; d = 32: 4 units 83.0 -> 75.9,
+  // 256 100 -> 78, 512 119 -> 101.  One mini-batch, d = 64: 4 units 10.9 -> 10.5, 256 11.7 -> 11.1; four: 24 13.1 -> 12.8.
+  const bool own_rule = D < 64 || units > 32 || a.n_stages <= 8;
+  const bool own_loads = own_rule ? (hint & TTT_HINT_ALL_LOADS) == 0 : (hint & TTT_HINT_OWN_LOADS) != 0;
   if (nw >= 2) return launch_linear_fwd_nw<T, D, 2>(probs, ny, s, own_loads, ctl_wave && max_nw == 2);
   return launch_linear_fwd_nw<T, D, 1>(probs, ny, s);
 }
