@@ -401,8 +401,8 @@ int launch_mlp_fwd_cl2(const ttt::MlpFwdArgs* probs, int n, hipStream_t s) {
 // Whether ttt_mlp_fwd runs the two-CU kernel for this desc and this many problems of its shape in one dispatch:
 // bf16 I/O without TTT_HINT_LDS_TILES; head_dim 128 always (the state does not fit one CU); head_dim 96 on request
 // (TTT_HINT_TWO_CU), for a single problem with at most half as many units as the device has CUs.  Measured at
-// B = 8, H = 16, seq 2048 (128 units on 256 CUs): 0.83 - 0.85 ms on pairs against 0.86 ms on single CUs -- the
-// exchange through global memory costs what halving each CU's share of the hidden axis saves -- so it is not the default.
+// B = 8, H = 16, seq 2048 (128 units on 256 CUs): 0.623 ms on pairs against 0.668 ms on single CUs, which does not pay for
+// two CUs that have to be resident together, so it is not the default.
 int uses_two_cu_mlp(const ttt_desc* d, int n_problems, bool* yes) {
   *yes = false;
   if (d->io_dtype == TTT_F32 || (d->kernel_hint & TTT_HINT_LDS_TILES) != 0) return TTT_OK;
