@@ -1,0 +1,50 @@
+"""CPU: properties of the code that the compiler makes of single kernels which no result shows for certain: how two waves
+order what they hand to each other without a barrier, and what a kernel needs of the registers that other waves could use."""
+import importlib
+import os
+import re
+import shutil
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+HIPCC = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
+
+pytestmark = pytest.mark.skipif(not os.path.exists(HIPCC), reason="needs hipcc")
+
+
+def compile_kernels(tmp_path, header, kernels):
+    """{kernel (its mangled name): (its instructions and labels, its register figures)} of explicit instantiations."""
+    build = importlib.import_module("ttt-rs_amd.build")
+    src, asm = tmp_path / "kernels.hip", tmp_path / "kernels.s"
+    src.write_text(f'#include "{header}"\nnamespace ttt {{\n' + "".join(f"template __global__ void {k};\n" for k in kernels) + "}\n")
+    subprocess.run([HIPCC, *build.HIPCC_FLAGS, "-I", os.path.join(build.HERE, "csrc"), "--cuda-device-only", "-S", "-o", str(asm),
+                    str(src)], check=True, capture_output=True)
+    bodies, figures, func = {}, {}, None
+    meta = {}
+    for line in asm.read_text().splitlines():
+        m = re.match(r"(_Z\w+):", line)
+        if m:
+            func = bodies.setdefault(m.group(1), [])
+        elif line.startswith(".Lfunc_end"):
+            func = None
+        elif func is not None and line.split(";")[0].strip():
+            func.append(line.split(";")[0].strip())
+        m = re.match(r"[\s-]+\.(name|vgpr_count|vgpr_spill_count|wavefront_size):\s+(\S+)", line)
+        if m:
+            meta[m.group(1)] = m.group(2)
+            if m.group(1) == "wavefront_size":
+                figures[meta["name"]] = {k: int(v) for k, v in meta.items() if k != "name"}
+    assert len(figures) == len(kernels)
+    return {k: (bodies[k], figures[k]) for k in figures}
+
+
+def test_mlp_pair_hands_a2_over_in_lds(tmp_path):
+    """Wave 2 of the TTT-MLP forward on a pair of CUs sums A2 as soon as a counter per wave says that every wave's partial
+    block is written, with no barrier between.  That holds if block and counter are both LDS instructions: a FLAT access to the
+    counter takes another path than the block, in an order that nothing guarantees."""
+    for name, (body, _) in compile_kernels(tmp_path, "ttt_mlp_fwd_cl2.hip.h", [
+            f"ttt_mlp_fwd_cl2_kernel<BF16, {d}>(Problems<MlpFwdArgs>)" for d in (96, 128)]).items():
+        flat = [s for s in body if s.startswith("flat_")]
+        assert not flat, f"{name}: {flat}"

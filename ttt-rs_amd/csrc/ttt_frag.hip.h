@@ -106,6 +106,13 @@ __device__ __forceinline__ void lds_barrier() {
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
 
+// this wave's LDS operations so far are done
+__device__ __forceinline__ void lds_done() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
+// An int that is known to lie in LDS.  A volatile or atomic access through a generic pointer stays a FLAT instruction, whose
+// order with the wave's LDS instructions nothing guarantees and which counts as a vector memory operation besides
+// (isa_check.py refuses code that has one).
+typedef __attribute__((address_space(3))) int lds_int;
+
 // A fragment's transpose: element (m, k) of the tile that lies in LDS as a fragment (lane order) -> the fragment with the
 // two axes exchanged.  Within each group of sixteen lanes the instruction takes four rows of sixteen elements, a row from
 // four lanes, and gives every lane a column.

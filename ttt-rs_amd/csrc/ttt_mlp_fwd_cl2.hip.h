@@ -27,7 +27,7 @@
 // same XCD (shared L2), and the exchange then never leaves that L2 (workgroup-scope stores, see send_tagged).
 // That placement is checked, not assumed: at start the two workgroups tell each other which XCD they run on
 // (device-scope words), and a pair that sits on two XCDs stores at device scope for the whole launch -- slower,
-// same results.  Every wait is bounded, so a missing partner ends in NaN outputs, never in a hang.
+// same results.  Every wait for the partner is bounded, so a missing partner ends in NaN outputs, never in a hang.
 //
 // What bounds it.  The products by the issue of a SIMD's two waves, as in ttt_mlp_fwd_rr.hip.h; between the first and the
 // second barrier a round trip through the L2, about 1.6 k cycles from the send to the tile in registers.  Cycles of a
@@ -168,7 +168,7 @@ __global__ void __launch_bounds__(64 * (D / 16)) ttt_mlp_fwd_cl2_kernel(Problems
   frag* const M1s = reinterpret_cast<frag*>(smem + L::M1);
   frag* const M2s = reinterpret_cast<frag*>(smem + L::M2);
   frag* const IDs = reinterpret_cast<frag*>(smem + L::ID);
-  volatile int* const FL = reinterpret_cast<volatile int*>(smem + L::FL);
+  lds_int* const FL = (lds_int*)(smem + L::FL);
   float* const RHO = reinterpret_cast<float*>(smem + L::RHO);
   uint32_t* const LRs = reinterpret_cast<uint32_t*>(smem + L::LR);
   float* const GAM = reinterpret_cast<float*>(smem + L::PRM);
@@ -321,7 +321,10 @@ __global__ void __launch_bounds__(64 * (D / 16)) ttt_mlp_fwd_cl2_kernel(Problems
   // ---- output path, wave w owns d-feature tile w.  While the Z2 tiles of mini-batch t + 1 cross, each CU sums its partial
   // Zbar2 tiles of t and CU 1 sends its half off; CU 0 adds it in phase D, applies the causal correction and forms the row
   // moments, and stores the output while the tiles of t + 2 cross.  A2 is summed by wave 2 of each CU at the end of phase
-  // A, as soon as every wave has written its partial block (a counter per wave; a wave's LDS operations take place in order).
+  // A, as soon as every wave has written its partial block.  There is no barrier between: each wave waits for its block to
+  // be in LDS (lds_done) and then counts up its own word there, which wave 2 reads.  Block and word both have to be LDS
+  // instructions (FL carries the address space: through a generic pointer the word goes another way than the block).  This
+  // wait needs no bound: on its way from B3 to the counter a wave waits for nothing but, bounded, the partner's tile.
   f32x4 zb = {0.f, 0.f, 0.f, 0.f};
   frag qo1 = IO::zero(), qo2 = qo1;  // xq tiles of the last mini-batch and of the one before
   auto a2_sum = [&]() -> f32x4 {
@@ -334,9 +337,9 @@ __global__ void __launch_bounds__(64 * (D / 16)) ttt_mlp_fwd_cl2_kernel(Problems
     return at;
   };
   auto a2_early = [&](int stage) -> f32x4 {
-    while (__builtin_amdgcn_ballot_w64(FL[lane & 7] <= stage) != 0) {
+    while (__builtin_amdgcn_ballot_w64(__hip_atomic_load(FL + (lane & 7), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) <= stage) != 0) {
     }
-    asm volatile("" ::: "memory");
+    lds_done();
     const f32x4 at = a2_sum();
     if (cu == 1) send_tile(stage & 1, 2 * NT, at, (unsigned)stage + 1);
     return at;
@@ -613,8 +616,8 @@ __global__ void __launch_bounds__(64 * (D / 16)) ttt_mlp_fwd_cl2_kernel(Problems
 #pragma unroll
       for (int j = 0; j < HT; j += 2) IO::mma2(p, x2f[j], x2f[j + 1], xbf[j], xbf[j + 1]);
       PA[w * 64 + lane] = p;
-      asm volatile("" ::: "memory");
-      if (lane == 0) FL[w] = st + 1;
+      lds_done();  // the block is in LDS before its counter says so
+      if (lane == 0) __hip_atomic_store(FL + w, st + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     }
     // (b2 enters the sum once: through wave I of CU 0)
     partials(xbf, [&](int I, f32x4 p) { P2[(w * NT + I) * 64 + lane] = IO::to_frag(I == w && cu == 0 ? p + b2T : p); });
