@@ -40,6 +40,15 @@ def compile_kernels(tmp_path, header, kernels):
     return {k: (bodies[k], figures[k]) for k in figures}
 
 
+def scan_loop(body):
+    """The instructions of the loop over the mini-batches: the shortest of the loops with the most matrix instructions
+    (branches back from blocks that the compiler moved behind the loop span it as well)."""
+    at = {s[:-1]: i for i, s in enumerate(body) if s.endswith(":")}
+    loops = [body[at[m.group(1)]:i] for i, s in enumerate(body)
+             if (m := re.match(r"s_c?branch\w*\s+(\.LBB\w+)", s)) and at.get(m.group(1), i) < i]
+    return min(loops, key=lambda loop: (-sum(s.startswith("v_mfma") for s in loop), len(loop)))
+
+
 def test_mlp_pair_hands_a2_over_in_lds(tmp_path):
     """Wave 2 of the TTT-MLP forward on a pair of CUs sums A2 as soon as a counter per wave says that every wave's partial
     block is written, with no barrier between.  That holds if block and counter are both LDS instructions: a FLAT access to the
@@ -48,3 +57,14 @@ def test_mlp_pair_hands_a2_over_in_lds(tmp_path):
             f"ttt_mlp_fwd_cl2_kernel<BF16, {d}>(Problems<MlpFwdArgs>)" for d in (96, 128)]).items():
         flat = [s for s in body if s.startswith("flat_")]
         assert not flat, f"{name}: {flat}"
+
+
+def test_linear_backward_reloads_nothing_in_its_loop(tmp_path):
+    """head_dim 128, bf16 I/O with f32 row-major checkpoints, and head_dim 64, f32 I/O from sparse checkpoints: the kernels
+    that sit at the limit of their registers.  A value spilled inside the loop is reloaded behind every load and store of the
+    wave that is in flight."""
+    for name, (body, _) in compile_kernels(tmp_path, "ttt_linear_bwd_mw.hip.h", [
+            f"ttt_linear_bwd_mw_kernel<{k}>(LinearBwdArgs)" for k in (
+                "BF16, 128, 4, false, false, false, false", "F32, 64, 4, true, false, true, true")]).items():
+        reloads = [s for s in scan_loop(body) if s.startswith("scratch_load")]
+        assert not reloads, f"{name}: {reloads}"

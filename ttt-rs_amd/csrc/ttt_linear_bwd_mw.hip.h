@@ -12,9 +12,9 @@
 //   X1  six raw moments of Z1 (mean, variance and both sums of the LN-L2 gradient follow from them), the
 //       partial attention blocks, XK^T / XQ^T fragments (tokens along k);
 //   X2  four raw moments of Zbar and of the output-LayerNorm backward; G fragments;
-//   X3  partial P = dZbar G^T, dZbar fragments (f32 I/O: in both forms), and the six sums of the second-order LayerNorm
+//   X3  partial P = dZbar G^T, dZbar fragments (without TR, see below: in both forms), and the six sums of the second-order LayerNorm
 //       (all its statistics are linear in them; none needs P, so one exchange carries both);
-//   X4  dZ1 fragments (f32 I/O: in both forms).
+//   X4  dZ1 fragments (without TR: in both forms).
 // All matrix products with a d-deep contraction over the OTHER slices' features take those fragments as B
 // operands; products over tokens (rank-16) are local.  f32 I/O computes in true-f32 MFMA
 // (v_mfma_f32_16x16x4_f32), bf16 I/O in bf16 MFMA with f32 accumulation.
@@ -76,6 +76,8 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && D / 16 == NW && (PK || si
   // whole by every wave on the matrix pipe, from fragments that cross LDS anyway, instead of per-wave partial
   // blocks that are written, read NW times and added up on the VALU
   constexpr bool FULL_AT = BF && D <= 96;
+  // tiles with the other axis along k, of what lies in LDS, by the transposing load (see lds_tr)
+  constexpr bool TR = BF && (D <= 96 || PK);
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
 
   const int lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
@@ -270,23 +272,17 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && D / 16 == NW && (PK || si
     IO::mma(t, x, ident);
     return IO::to_frag(t);
   };
-  // The same for a tile that lies in LDS as fragments, `step` bytes from lane to lane: bf16 takes it from there with the
-  // transposing load, which costs no matrix instruction and no conversion (d = 64: 11 of a mini-batch's 14 transposes; forward
-  // and backward, 384 units x 2048 tokens, 596 -> 568 us).  What a wave has just computed and needs at once stays with
-  // tokens_k: a write to LDS and a read back is the longer way.
-  const int trl = tr_lane(lane);
-  auto tokens_k_lds = [&](const void* tile, int step) -> frag {
-    const unsigned char* p = static_cast<const unsigned char*>(tile);
-    if constexpr (BF)
-      return read_tr(p + trl * step);
-    else
-      return tokens_k(*reinterpret_cast<const frag*>(p + lane * step));
-  };
+  // TR: the same for a tile that lies in LDS as fragments, sixteen bytes from lane to lane: the transposing load takes it from
+  // there, which costs no matrix instruction and no conversion (bf16, d = 64: 11 of a mini-batch's 14 transposes; forward and
+  // backward, 384 units x 2048 tokens, 596 -> 568 us).  What a wave has just computed and needs at once stays with tokens_k: a
+  // write to LDS and a read back is the longer way.  So does everything where the addresses of these loads are registers
+  // too many: d = 128 with f32 row-major checkpoints, 128 units x 2048 tokens, 911 us, with these loads five reloads from
+  // scratch in the loop and 1034 us.
+  const int trl = TR ? tr_lane(lane) : 0;
+  auto lds_tr = [&](const unsigned char* tile) { return read_tr(tile + trl * 16); };
   auto tile_ptr = [&](int kind, int J) { return FRp + (kind * NT + J) * 64; };
   // tile J of an activation tensor in the staging area
-  auto row_ptr = [&](int tensor, int J) {
-    return smem + L::X + (BF ? (tensor * XS + (J >> 1)) * 1024 + 8 * (J & 1) : (tensor * XS + J) * 1024);
-  };
+  auto row_ptr = [&](int tensor, int J) { return smem + L::X + (tensor * XS + (J >> 1)) * 1024 + 8 * (J & 1); };
   // acc += sum over the NT tiles of A[J] B[J]
   auto mma_all = [&](f32x4& acc, const frag (&A)[NT], const frag (&B)[NT]) {
 #pragma unroll
@@ -352,7 +348,7 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && D / 16 == NW && (PK || si
     if constexpr (FM) {
       frag kda[NT];
 #pragma unroll
-      for (int I = 0; I < NT; ++I) kda[I] = tokens_k_lds(row_ptr(1, I), 16);
+      for (int I = 0; I < NT; ++I) kda[I] = lds_tr(row_ptr(1, I));
       frag nG[TPW];
 #pragma unroll
       for (int jj = 0; jj < TPW; ++jj) {
@@ -444,13 +440,20 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && D / 16 == NW && (PK || si
         bT[ii] = *reinterpret_cast<const f32x4*>(sl + L::Bv + Io * 1024) - bbar;
 #pragma unroll
       for (int J = 0; J < NT; ++J) {
-        if constexpr (PK)  // stored as (m = j, k = i)
-          Wn[ii][J] = tokens_k_lds(smem + pk_off(Io, J), 16);
+        if constexpr (PK && TR)  // stored as (m = j, k = i)
+          Wn[ii][J] = lds_tr(smem + pk_off(Io, J));
+        else if constexpr (PK)
+          Wn[ii][J] = tokens_k(*reinterpret_cast<const frag*>(sl + pk_off(Io, J)));
         else
           Wn[ii][J] = IO::to_frag(*reinterpret_cast<const f32x4*>(sl + L::W + (Io * NT + J) * 1024) - mrowo[ii]);
       }
-      kdo[ii] = tokens_k_lds(row_ptr(1, Io), 16);
-      qdo[ii] = tokens_k_lds(row_ptr(0, Io), 16);
+      if constexpr (TR) {
+        kdo[ii] = lds_tr(row_ptr(1, Io));
+        qdo[ii] = lds_tr(row_ptr(0, Io));
+      } else {
+        kdo[ii] = tokens_k(ko[ii]);
+        qdo[ii] = tokens_k(qo[ii]);
+      }
       fr(KD, Io) = kdo[ii];
       fr(QD, Io) = qdo[ii];
     }
@@ -593,7 +596,7 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && D / 16 == NW && (PK || si
         if constexpr (TDB) dbT[jj] += dzb;
         Zd[jj] = tokens_k(Zf[jj]);
         fr(ZF, w * TPW + jj) = Zf[jj];
-        if constexpr (!BF) fr(ZD, w * TPW + jj) = Zd[jj];
+        if constexpr (!TR) fr(ZD, w * TPW + jj) = Zd[jj];
         if (BF) {
           // P feeds the gradients of eta (small differences of large sums): bf16 head + tail of both factors
           Gl[jj] = IO::to_frag(G[jj] - IO::to_f32(Gf[jj]));
@@ -737,8 +740,9 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && D / 16 == NW && (PK || si
         const f32x4 dz1 = (dxh - q1) * rstd1 + xh[jj] * (dsig * inv_d);
         Z1f[jj] = IO::to_frag(dz1);
         if constexpr (TDB) dbT[jj] += dz1;
+        if constexpr (!TR) Z1d[jj] = tokens_k(Z1f[jj]);
         fr(Z1F, w * TPW + jj) = Z1f[jj];
-        if constexpr (!BF) fr(Z1D, w * TPW + jj) = Z1d[jj] = tokens_k(Z1f[jj]);
+        if constexpr (!TR) fr(Z1D, w * TPW + jj) = Z1d[jj];
         dK[jj] += dy - last * TMP[jj];
         ndy[jj] = -dy;
       }
@@ -782,7 +786,7 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && D / 16 == NW && (PK || si
     };
     if constexpr (FM) single_wave_outputs();
     // ---- state gradient: dW += XQ^T dZb + XK^T dZ1 (column slice and transposed row slice), db
-    if constexpr (BF) {
+    if constexpr (TR) {
 #pragma unroll
       for (int jj = 0; jj < TPW; ++jj) Z1d[jj] = read_tr(tile_ptr(Z1F, w * TPW + jj) + trl);
     }
@@ -790,7 +794,7 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && D / 16 == NW && (PK || si
     for (int I = 0; I < NT; ++I) {
       const frag qa = fr(QD, I), ka = fr(KD, I);
       frag za, z1a;
-      if constexpr (BF) {
+      if constexpr (TR) {
         za = read_tr(tile_ptr(ZF, I) + trl);
         z1a = read_tr(tile_ptr(Z1F, I) + trl);
       } else {
