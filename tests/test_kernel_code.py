@@ -68,3 +68,10 @@ def test_linear_backward_reloads_nothing_in_its_loop(tmp_path):
                 "BF16, 128, 4, false, false, false, false", "F32, 64, 4, true, false, true, true")]).items():
         reloads = [s for s in scan_loop(body) if s.startswith("scratch_load")]
         assert not reloads, f"{name}: {reloads}"
+
+
+def test_mlp_forward_d32_leaves_room_for_a_second_workgroup(tmp_path):
+    """Eight waves, two a SIMD: a CU takes two workgroups if a wave needs at most a quarter of a SIMD's 512 registers."""
+    for name, (body, figures) in compile_kernels(tmp_path, "ttt_mlp_fwd_rr.hip.h", [
+            f"ttt_mlp_fwd_rr_kernel<BF16, 32, {save}>(Problems<MlpFwdArgs>)" for save in ("false", "true")]).items():
+        assert figures["vgpr_count"] <= 128 and figures["vgpr_spill_count"] == 0, f"{name}: {figures}"

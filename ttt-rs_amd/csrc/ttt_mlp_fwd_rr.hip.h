@@ -26,7 +26,7 @@
 // waves, 23.3 cycles against 16 + 7.5).  Phases B and C by latency.  Cycles of a mini-batch at d = 96 and 128 units,
 // before -> after the last revision: A 4.9 -> 4.7 k (XQ W1 now shares the operands of XK W1), B 2.9 -> 2.0 k, C 2.2 -> 1.3 k
 // (output off the chain, loads in one go, sums by lane group), D 7.4 -> 6.4 k (independent products side by side, transposes
-// read from LDS).  8 x 16 units x 2048 tokens: d = 96 840 -> 667 us, d = 64 488 -> 433 us, d = 32 286 -> 266 us.
+// read from LDS).  8 x 16 units x 2048 tokens: d = 96 840 -> 667 us, d = 64 488 -> 433 us, d = 32 286 -> 261 us.
 //
 // An odd hidden tile at the end of a split-k chain is issued as a k = 32 MFMA with a zero second
 // half, not as a k = 16 one: a 16x16x16 bf16 MFMA accumulating straight onto the result of a
@@ -117,10 +117,12 @@ __device__ __forceinline__ float mean_of(const float* p, int d, float inv_d) {
 // spilled and reloaded from scratch.  Hiding the lane index from the optimiser at the start of each
 // phase makes them cheap phase-local recomputations instead.  At d = 96 the lane coordinates and the constant operands
 // (identity, rho) are formed anew or read from LDS as well: held in registers they spill, and a reload from scratch waits for
-// the copies in flight (871 against 770 us); at d <= 64 there is room for them (471 against 434 us).
+// the copies in flight (871 against 770 us); at d <= 64 there is room for them (471 against 434 us), but for one register
+// too many in the saving kernel at d = 32 (see the kernel's launch bounds).
 #define RELANE()                               \
   do {                                         \
     asm volatile("" : "+v"(lane));             \
+    if constexpr (D == 32 && SAVE) g = lane >> 4; \
     if constexpr (D > 64) {                    \
       c = lane & 15;                           \
       g = lane >> 4;                           \
@@ -130,8 +132,11 @@ __device__ __forceinline__ float mean_of(const float* p, int d, float inv_d) {
 
 // SAVE: also leave what a backward starts from (MlpFwdArgs::fac_save or G1_save).  A compilation of its own: the pointers
 // and branches cost the plain forward 3 % of its time in registers.
+// d = 32 is held to 128 registers, so that a CU takes two workgroups (LDS has room for them): each hides the other's waits
+// between the barriers.  512 units x 2048 tokens, with 130 registers -> 128: 530 -> 353 us, saving 574 -> 382 us; 128 units,
+// which have a CU each, 266 -> 261 and 287 -> 285 us.
 template <class T, int D, bool SAVE>
-__global__ void __launch_bounds__(512) ttt_mlp_fwd_rr_kernel(Problems<MlpFwdArgs> problems) {
+__global__ void __launch_bounds__(512, D == 32 ? 4 : 2) ttt_mlp_fwd_rr_kernel(Problems<MlpFwdArgs> problems) {
   const MlpFwdArgs& a = problems.p[blockIdx.y];
   using IO = Io<T>;
   using frag = typename IO::frag;
@@ -150,6 +155,8 @@ __global__ void __launch_bounds__(512) ttt_mlp_fwd_rr_kernel(Problems<MlpFwdArgs
   const size_t bh = blockIdx.x;
   const int h = (int)(bh % a.H), K = a.K;
   const bool red = w < NT;  // this wave reduces d-feature tile w
+  // this wave finishes output tiles (at d = 32 there are more waves left than tiles)
+  const bool outw = !red && (2 * NT >= NW || w < 2 * NT);
 
   f32x4* const P1 = reinterpret_cast<f32x4*>(smem + L::P1);
   f32x4* const P2 = reinterpret_cast<f32x4*>(smem + L::P2);
@@ -486,7 +493,7 @@ __global__ void __launch_bounds__(512) ttt_mlp_fwd_rr_kernel(Problems<MlpFwdArgs
         S[5] += bq[r] * z[r];
       }
       publish(S);
-    } else if (st > 0) {
+    } else if (outw && st > 0) {
       output_sum();
       output_m2();
     }
@@ -526,7 +533,7 @@ __global__ void __launch_bounds__(512) ttt_mlp_fwd_rr_kernel(Problems<MlpFwdArgs
       const f32x4 G = (z - mu) * (gam * gam * c1 + c2) + (bq * p + c3);
       GTc[w * 64 + lane] = IO::to_frag(G);
       if (st > 0) qo = load4<T>(row((st + 2) % 3, 0) + own);
-    } else if (st > 0) {
+    } else if (outw && st > 0) {
       output_moments(st - 1);
     }
     // the next mini-batch's rows must have landed before anybody passes B3
@@ -662,11 +669,11 @@ __global__ void __launch_bounds__(512) ttt_mlp_fwd_rr_kernel(Problems<MlpFwdArgs
   // ---- the last mini-batch's output
   frag qo = IO::zero();
   lds_barrier();
-  if (!red) {
+  if (outw) {
     output_sum();
     output_m2();
     output_moments(n_stages - 1);
-  } else {
+  } else if (red) {
     qo = load4<T>(row((a.n_stages - 1) % 3, 0) + own);
   }
   lds_barrier();
