@@ -48,6 +48,14 @@ def test_scanner_flags_a_scalar_select_on_a_vector_comparison():
     assert isa_check.scan_scc_select(["ttt_selftest_x:"] + wrong[1:]) == []
 
 
+def test_scanner_flags_flat_accesses():
+    """The third rule: a poll and a store of an LDS word through a generic pointer, as the compiler once left them."""
+    assert [b[1] for b in isa_check.scan_flat(["kern:", ".LBB0_1:", "\tflat_load_dword v1, v[2:3] sc0 sc1", "\ts_waitcnt vmcnt(0) lgkmcnt(0)",
+                                               "\tflat_store_dword v[2:3], v1 sc0 sc1"])] == [3, 5]
+    assert isa_check.scan_flat(["kern:", "\tds_read_b32 v1, v2", "\tglobal_load_dword v1, v[2:3], off", "\t; flat_load_dword v1, v[2:3]",
+                                "\t.set kern.uses_flat_scratch, 0"]) == []
+
+
 def test_scanner_flags_a_close_mixed_pair_in_place():
     assert len(flagged([K32.format(c="0"), K16.format(d="v[0:3]", c="v[0:3]")])) == 1
     assert len(flagged([K16.format(d="v[0:3]", c="0"), K32.format(c="v[0:3]")])) == 1

@@ -75,3 +75,12 @@ def test_mlp_forward_d32_leaves_room_for_a_second_workgroup(tmp_path):
     for name, (body, figures) in compile_kernels(tmp_path, "ttt_mlp_fwd_rr.hip.h", [
             f"ttt_mlp_fwd_rr_kernel<BF16, 32, {save}>(Problems<MlpFwdArgs>)" for save in ("false", "true")]).items():
         assert figures["vgpr_count"] <= 128 and figures["vgpr_spill_count"] == 0, f"{name}: {figures}"
+
+
+def test_mlp_backward_reads_its_look_ahead_from_lds(tmp_path):
+    """The look-ahead at the partner's counter is copied to LDS to spare a trip through the vector memory path: its reader may
+    not take that path either."""
+    for name, (body, _) in compile_kernels(tmp_path, "ttt_mlp_bwd_rp.hip.h", [
+            f"ttt_mlp_bwd_rp_kernel<{d}>(MlpBwdRpArgs)" for d in (32, 64)]).items():
+        flat = [s for s in body if s.startswith("flat_")]
+        assert not flat, f"{name}: {flat}"

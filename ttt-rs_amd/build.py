@@ -32,7 +32,7 @@ HIPCC_FLAGS = [
 
 def build_library(verbose: bool = False, extra_flags=()) -> str:
     """Compiles the library, then scans the gfx950 assembly the compiler produced on the way (isa_check.py: a
-    matrix-instruction hazard the compiler does not guard and the hardware does not interlock).  The library is
+    matrix-instruction hazard the compiler does not guard and the hardware does not interlock, and two more).  The library is
     installed only if the scan is clean."""
     hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
     os.makedirs(LIB_DIR, exist_ok=True)
@@ -73,6 +73,12 @@ def build_library(verbose: bool = False, extra_flags=()) -> str:
                 sys.stderr.write(f"{os.path.basename(path)}:{no}: in {func}: scalar select on a vector comparison\n    {a}\n    {b}\n")
             raise RuntimeError(f"{len(sel)} s_cselect instruction(s) read a condition code that the comparison in front "
                                "of them does not set (see isa_check.py); library not installed")
+        flat = isa_check.check_flat_file(path)
+        if flat:
+            for func, no, a in flat[:20]:
+                sys.stderr.write(f"{os.path.basename(path)}:{no}: in {func}: FLAT access\n    {a}\n")
+            raise RuntimeError(f"{len(flat)} FLAT access(es), whose order with LDS instructions nothing guarantees (see isa_check.py); "
+                               "library not installed")
     shutil.copyfile(out, LIB_PATH)
     shutil.copymode(out, LIB_PATH)
     shutil.rmtree(os.path.join(HERE, "build"), ignore_errors=True)

@@ -370,16 +370,16 @@ struct Base {
   }
   // (moved to a scalar register by hand: see isa_check.py, the scalar select on a vector comparison)
   __device__ __forceinline__ bool is_lost() const { return __builtin_amdgcn_readfirstlane(*lost) != 0; }
-  // bounded wait of thread 0 for the partner's counter; the barrier behind it is the caller's
   // A look at the counter ahead of time: the poll that follows finds it in LDS and is spared the round trip it would begin
   // with, up to 5 k cycles on a full chip (d = 96 2167 -> 2122 us).  Through LDS because a register for it spills others.
   __device__ __forceinline__ void peek(const unsigned* fl, int which) {
     if (pair && w == 0 && lane == 0) lds_dma4_dev(fl, 4u * which, lds0() + L::CTL + 4);
   }
+  // bounded wait of thread 0 for the partner's counter; the barrier behind it is the caller's
   __device__ __forceinline__ void poll(unsigned* fl, int which, int want) {
     if (!pair || want <= 0 || tid != 0 || is_lost()) return;
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    const unsigned seen = (unsigned)const_cast<volatile int*>(lost)[1];
+    const unsigned seen = (unsigned)lost[1];  // (as the copy left it: the wait above is a memory clobber)
     bool got = seen != kMlpRpPoison && seen >= (unsigned)want;
     if (got) return;
     for (unsigned i = 0; i < a.spin_limit; ++i) {
