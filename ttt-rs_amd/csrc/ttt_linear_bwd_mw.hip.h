@@ -239,18 +239,6 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && D / 16 == NW && (PK || si
   auto xcol = [&](int region, float (&S)[8]) {
     const float* e = SUMp + region * 8 * 16 * NW;
     lds_barrier();
-    if constexpr (NW == 4) {
-      // four sums (the second exchange): their loads are held together, see together(); the others' are issued so anyway
-      if (region == 1) {
-        f32x4 v[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) v[i] = *reinterpret_cast<const f32x4*>(e + (i * 16 + c) * NW);
-        together(v);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) S[i] = v[i][0] + v[i][1] + v[i][2] + v[i][3];
-        return;
-      }
-    }
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
       float s = 0.f;
