@@ -153,8 +153,8 @@ def test_mlp_bwd_repeat_calls(P, d, K, dtype):
 @pytest.mark.parametrize("B,H,K,N", [(2, 3, 16, 5), (1, 2, 7, 4), (1, 1, 16, 1), (2, 2, 16, 2), (3, 2, 5, 7)])
 def test_linear_fwd_own_loads_variant_gives_the_same_bits(P, B, H, K, N, fmt):
     """bf16, head_dim 64, two waves per unit: the variant in which a wave loads only the features it owns and the
-    full rows cross LDS (the library's choice above 256 units; TTT_HINT_OWN_LOADS asks for it at any size) against
-    the variant in which every wave loads every row (TTT_HINT_ALL_LOADS): the same arithmetic on the same values."""
+    full rows cross LDS (the library's choice, which TTT_HINT_OWN_LOADS asks for by name) against the variant in which
+    every wave loads every row (TTT_HINT_ALL_LOADS): the same arithmetic on the same values."""
     if fmt == 2 and N < 2:
         pytest.skip("one mini-batch is saved packed")
     d = 64

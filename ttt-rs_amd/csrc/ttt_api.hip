@@ -240,12 +240,12 @@ int launch_linear_fwd(const ttt::LinearFwdArgs* probs, int hint, unsigned ny, hi
   if constexpr (max_nw >= 4) {
     if (nw >= 4) return launch_linear_fwd_nw<T, D, 4>(probs, ny, s, false, ctl_wave);
   }
-  // bf16: own-feature loads, except for long sequences of a few units at d = 64, where the trip through LDS costs more than the
-  // loads it saves.  Every wave's loads of whole rows -> own features, 2048 tokens, d = 64: 4 units 112.3 -> 113.0 us, 24
-  // 114.0 -> 114.3, 96 122.6 -> 117.0, 256 127.6 -> 118.1, saving update factors 136.7 -> 122.0; d = 32: 4 units 83.0 -> 75.9,
-  // 256 100 -> 78, 512 119 -> 101.  One mini-batch, d = 64: 4 units 10.9 -> 10.5, 256 11.7 -> 11.1; four: 24 13.1 -> 12.8.
-  const bool own_rule = D < 64 || units > 32 || a.n_stages <= 8;
-  const bool own_loads = own_rule ? (hint & TTT_HINT_ALL_LOADS) == 0 : (hint & TTT_HINT_OWN_LOADS) != 0;
+  // bf16: own-feature loads.  Every wave's loads of whole rows -> own features, 2048 tokens, d = 64: 4 units 112.4 -> 113.2 us, 8
+  // 112.6 -> 113.4, 12 116.0 -> 113.9, 24 114.5 -> 114.2, 48 120.5 -> 115.7, 128 124.4 -> 118.4, 256 127.6 -> 118.1, saving
+  // update factors 136.7 -> 122.0; d = 32: 4 units 83.0 -> 75.9, 256 100 -> 78, 512 119 -> 101.  One mini-batch, d = 64: 4 units
+  // 10.9 -> 10.4, 128 11.3 -> 10.8.  Up to 8 units the trip through LDS costs up to 0.8 % at 64 and 128 mini-batches and nothing
+  // at 16, 32 and 256: no rule of its own.
+  const bool own_loads = (hint & TTT_HINT_ALL_LOADS) == 0;
   if (nw >= 2) return launch_linear_fwd_nw<T, D, 2>(probs, ny, s, own_loads, ctl_wave && max_nw == 2);
   return launch_linear_fwd_nw<T, D, 1>(probs, ny, s);
 }
