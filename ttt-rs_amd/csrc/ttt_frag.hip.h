@@ -127,6 +127,7 @@ __device__ __forceinline__ int tr_lane(int lane) { return (lane & 3) * 16 + (lan
 // otherwise loads, waits and uses them one at a time, an LDS round trip each.)
 template <int N>
 __device__ __forceinline__ void together(f32x4 (&v)[N]) {
+  static_assert(N == 4 || N == 6 || N == 8, "one operand list per size");
   if constexpr (N == 4) asm volatile("" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]));
   if constexpr (N == 6) asm volatile("" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]), "+v"(v[4]), "+v"(v[5]));
   if constexpr (N == 8)

@@ -36,6 +36,14 @@ struct LinBwdMwLds {
   static constexpr int NT = D / 16, TPW = NT / NW;
   static constexpr int XS = (ES == 2) ? NT / 2 : NT;  // 1 KiB slots per activation tensor
   static constexpr int FT = 64 * 4 * ES;              // bytes of one fragment tile
+  // tiles with the other axis along k, of what lies in LDS, by the transposing load (see lds_tr in the kernel)
+  static constexpr bool TR = ES == 2 && (D <= 96 || PK);
+  // bf16, d <= 96: the [16 x 16] blocks that contract over all d features (attention, P = dZbar G^T) are formed
+  // whole by every wave on the matrix pipe, from fragments that cross LDS anyway, instead of per-wave partial
+  // blocks that are written, read NW times and added up on the VALU
+  static constexpr bool FULL_AT = ES == 2 && D <= 96;
+  static constexpr int KINDS = 5 + (TR ? 0 : 2) + (FULL_AT ? 2 : 0);  // without TR ZD and Z1D, with FULL_AT GL and ZL
+  static_assert(TR || !FULL_AT, "the order of the kinds");
   static constexpr int W = 0;                         // NT*NT slots: slot I*NT+J, lane (c,g): W[feat(I,c)][feat(J,4g..4g+3)]
                                                       // packed: NT*NT/2 slots: slot I*NT/2+q = tiles (I,2q), (I,2q+1)
   static constexpr int WSLOTS = (PK && ES == 2) ? NT * NT / 2 : NT * NT;
@@ -44,8 +52,8 @@ struct LinBwdMwLds {
   static constexpr int LR = X + 4 * XS * 1024;        // 16 dwords: lr of token c (bf16 zero-extended, or f32)
   static constexpr int SUM = LR + 256;                // 3 exchanges x [8 sums][16 tokens][NW]
   static constexpr int PT = SUM + 3 * 8 * 16 * NW * 4;  // 4 kinds x [NW][64] f32x4: partial [16 x 16] blocks
-  static constexpr int FR = PT + 4 * NW * 1024;       // 9 kinds x [NT][64] fragments
-  static constexpr int M0 = FR + 9 * NT * FT;         // D row means of the initial W, then mean(b): the centred state
+  static constexpr int FR = PT + 4 * NW * 1024;       // KINDS x [NT][64] fragments
+  static constexpr int M0 = FR + KINDS * NT * FT;         // D row means of the initial W, then mean(b): the centred state
   static constexpr int GDS = M0 + (D + 4) * 4;         // FM: NT half slots: the factor fragments of tile J
   static constexpr int BYTES = GDS + (FM ? NT * 512 : 0);
   static_assert(!FM || (PK && ES == 2), "factors: bf16 I/O, packed image of the state");
@@ -70,14 +78,9 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && D / 16 == NW && (PK || si
   using L = LinBwdMwLds<D, NW, ES, PK, FM>;
   constexpr int NT = D / 16, TPW = NT / NW, NQ = NT / 2, XS = L::XS;
   constexpr float inv_d = 1.0f / D;
-  enum { KD = 0, QD, GF, ZF, ZD, Z1F, Z1D, GL, ZL };
+  enum { KD = 0, QD, GF, ZF, ZD, Z1F = L::TR ? 4 : 5, Z1D, GL = L::TR ? 5 : 7, ZL };
   enum { P_AT = 0, P_AT2, P_P, P_P2 };
-  // bf16, d <= 96: the [16 x 16] blocks that contract over all d features (attention, P = dZbar G^T) are formed
-  // whole by every wave on the matrix pipe, from fragments that cross LDS anyway, instead of per-wave partial
-  // blocks that are written, read NW times and added up on the VALU
-  constexpr bool FULL_AT = BF && D <= 96;
-  // tiles with the other axis along k, of what lies in LDS, by the transposing load (see lds_tr)
-  constexpr bool TR = BF && (D <= 96 || PK);
+  constexpr bool FULL_AT = L::FULL_AT, TR = L::TR;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
 
   const int lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
