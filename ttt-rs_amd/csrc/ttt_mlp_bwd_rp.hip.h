@@ -379,7 +379,8 @@ struct Base {
   __device__ __forceinline__ void poll(unsigned* fl, int which, int want) {
     if (!pair || want <= 0 || tid != 0 || is_lost()) return;
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    const unsigned seen = (unsigned)lost[1];  // (as the copy left it: the wait above is a memory clobber)
+    // as the copy left it (the wait above is a memory clobber); in a scalar register, as in is_lost: d = 32 803 -> 793 us
+    const unsigned seen = (unsigned)__builtin_amdgcn_readfirstlane(lost[1]);
     bool got = seen != kMlpRpPoison && seen >= (unsigned)want;
     if (got) return;
     for (unsigned i = 0; i < a.spin_limit; ++i) {
