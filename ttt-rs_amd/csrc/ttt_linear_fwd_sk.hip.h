@@ -77,7 +77,7 @@ __device__ __forceinline__ void linear_fwd_sk_body(const LinearFwdArgs& a, const
   constexpr bool DMA = RAW == 5;
   // XK with tokens along k, for the state update: where the rows are shared through LDS anyway, the transposing LDS load
   // gives it, instead of a matrix instruction and two conversions per tile (the waves are bound by what they issue; 384 units
-  // x 2048 tokens, d = 64: 127.0 -> 126.1 us, saving update factors 7 us less).  A zero token_eta[K-1] then masks G'' in the
+  // x 2048 tokens, d = 64: 128.3 -> 127.3 us, saving update factors 148.7 -> 140.6 us; runs of one side differ by 0.3 us).  A zero token_eta[K-1] then masks G'' in the
   // update, where it makes the transpose zero otherwise.  Not where the operands are formed here (a layer 199.3 -> 200.1 us)
   // and not with the Adam step (230 -> 240 us), whose loops are scheduled worse with it.
   constexpr bool TRK = RAW >= 3 && !DMA && BF && !ADAM;
