@@ -100,6 +100,17 @@ __device__ __forceinline__ f32x4 over_tokens(f32x4 v) {
 // of a row must hold the SAME number (a pivot subtracted from a whole matrix row), one lane's result is shared.
 __device__ __forceinline__ float row16_first(float v) { return __shfl(v, (int)(threadIdx.x & 48u), 64); }
 
+// A kernel argument in a scalar register from here on.  Short of scalar registers the compiler otherwise loads it again where
+// it is used, in every mini-batch: a round trip through the scalar cache, behind a barrier in the middle of the chain.
+__device__ __forceinline__ float held(float x) {
+  asm volatile("" : "+s"(x));
+  return x;
+}
+__device__ __forceinline__ int held(int x) {
+  asm volatile("" : "+s"(x));
+  return x;
+}
+
 // Workgroup barrier for LDS exchanges only: waits for this wave's LDS traffic, not for the
 // global prefetches in flight (a full __syncthreads() would drain those every mini-batch).
 __device__ __forceinline__ void lds_barrier() {

@@ -88,7 +88,15 @@ __device__ __forceinline__ void linear_fwd_sk_body(const LinearFwdArgs& a, const
   const int c = lane & 15, g = lane >> 4;
   const size_t bh = STATES ? unit : blockIdx.x;
   const int h = (int)(bh % a.H);
-  const int K = a.K, n_stages_ = a.n_stages + (STATES ? 1 : 0);
+  // Arguments of every mini-batch held in scalar registers (see held).  384 units x 2048 tokens, d = 64: 127 -> 117 us, saving
+  // update factors 142 -> 128; d = 32 99 -> 97; f32, 96 units 215.4 -> 214.2.  Not with the Adam step (230 -> 231), and the length
+  // only where the loop has a branch-free middle: held in the other loops (wide heads, d = 128: 193 -> 230 us; f32 215 -> 218; the
+  // Adam step 230 -> 258) it has the compiler take them apart.
+  constexpr bool HOLD_EPS = !ADAM, HOLD_N = BF && !ADAM && NT <= 4;
+  const int K = a.K, n_held = HOLD_N ? held(a.n_stages) : 0, n_stages_ = (HOLD_N ? n_held : a.n_stages) + (STATES ? 1 : 0);
+  const float eps_held = HOLD_EPS ? held(a.eps) : 0.f;
+  auto n_st = [&]() { return HOLD_N ? n_held : a.n_stages; };
+  auto eps = [&]() { return HOLD_EPS ? eps_held : a.eps; };
   const UnitBase<T, D> ub(a, bh);
 
   // same scale folding as the unskewed kernel: G'' = -sc lr G, M'' = (token_eta[t]/sc)(1 + A)
@@ -164,7 +172,7 @@ __device__ __forceinline__ void linear_fwd_sk_body(const LinearFwdArgs& a, const
   }
   // One Adam step on a tile: gneg = -gradient (what the plain kernel would add to the state).  The moments are carried
   // as m / (1 - beta1) and v / (1 - beta2), so that each decays and takes its new term in one or two instructions, and
-  // lr m^ / (sqrt(v^) + eps) is taken as ad_k m / (sqrt(v) + ad_e) with the bias corrections in the two scalars: eight
+  // lr m^ / (sqrt(v^) + eps()) is taken as ad_k m / (sqrt(v) + ad_e) with the bias corrections in the two scalars: eight
   // instructions per element, two of them transcendental, where the step as written has eleven.
   float ad_k = 0.f, ad_e = 0.f;
   auto adam_tile = [&](f32x4& x, f32x4& m, f32x4& v, f32x4 gneg) {
@@ -230,7 +238,7 @@ __device__ __forceinline__ void linear_fwd_sk_body(const LinearFwdArgs& a, const
   // out = xq + gamma (zbar - mu) rstd + beta for the pending mini-batch
   auto emit_output = [&](float s0, float s1, int stage, const f32x4 (&zbp)[TPW], const frag (&qop)[TPW]) {
     const float mu = s0 * inv_d;
-    const float rstd = __builtin_amdgcn_rsqf(fmaxf(s1 * inv_d - mu * mu, 0.f) + a.eps);
+    const float rstd = __builtin_amdgcn_rsqf(fmaxf(s1 * inv_d - mu * mu, 0.f) + eps());
     if (FULL || c < K) {
       elem* po = reinterpret_cast<elem*>(ub.out + UnitBase<T, D>::row_off(stage, K, c));
       f32x4 o[TPW];
@@ -286,6 +294,13 @@ __device__ __forceinline__ void linear_fwd_sk_body(const LinearFwdArgs& a, const
     } else {
       return f;
     }
+  };
+  // s2 of the LN-L2 gradient, a sum of two products of which one is rounded before the other is added.  Written out, `second`
+  // as the callers have it: left open, the compiler decides it in each copy of the body, anew after every change of the
+  // code around it, and a stack of layers carries a last bit on to 1 % of its outputs.
+  auto g_norm_sum = [&](const float (&S)[8], float mu, float rstd, bool second) {
+    const float m = S[5] - mu * S[4], q = S[3] - 2.f * mu * S[2] + mu * mu * sum_a, r2 = rstd * rstd;
+    return second ? __builtin_fmaf(r2, q, rstd * m) : __builtin_fmaf(m, rstd, r2 * q);
   };
   const frag ident_upd = upd ? ident : IO::zero();
   const frag ones_upd = upd ? ones : IO::zero();
@@ -546,8 +561,8 @@ __device__ __forceinline__ void linear_fwd_sk_body(const LinearFwdArgs& a, const
   const float b_mean = __builtin_amdgcn_readfirstlane(m0s[D]);  // mean of the initial bias (split off by centre_state)
   static_assert(!FAC || BF, "update factors are saved with bf16 I/O only");
   unsigned char* fac = FAC ? factor_base<D>(a.W_ckpt, a.n_ckpt, bh) : nullptr;
-  auto pass = [&](auto checked_tag, int st0) {
-    constexpr bool CHECKED = decltype(checked_tag)::value;
+  auto pass = [&](auto checked_tag, auto later_tag, int st0) {
+    constexpr bool CHECKED = decltype(checked_tag)::value, LATER = decltype(later_tag)::value;
 #pragma unroll
     for (int u = 0; u < R; ++u) {
       const int st = st0 + u;
@@ -555,7 +570,7 @@ __device__ __forceinline__ void linear_fwd_sk_body(const LinearFwdArgs& a, const
         load_raw(raw[u], st + R);  // its previous content, mini-batch st, was rotated two mini-batches ago
       else
         load_stage_mw<T, D, NW, FULL>(buf[(u + PF) % R], ub, K, n_stages_, st + PF, c, g, w);
-      if (CHECKED && st >= a.n_stages) continue;
+      if (CHECKED && st >= n_st()) continue;
       const StageInMw<T, NT, TPW>& cur = buf[u];
 
       // ---- XK with tokens along k for the state update: depends on nothing computed here, so it
@@ -667,9 +682,9 @@ __device__ __forceinline__ void linear_fwd_sk_body(const LinearFwdArgs& a, const
       {
         const float mu = S[0] * inv_d;
         const float var = S[1] * inv_d - mu * mu;
-        const float rstd = __builtin_amdgcn_rsqf(fmaxf(var, 0.f) + a.eps);
+        const float rstd = __builtin_amdgcn_rsqf(fmaxf(var, 0.f) + eps());
         const float s1 = rstd * (S[2] - mu * sum_a) + S[4];
-        const float s2 = rstd * rstd * (S[3] - 2.f * mu * S[2] + mu * mu * sum_a) + rstd * (S[5] - mu * S[4]);
+        const float s2 = g_norm_sum(S, mu, rstd, ADAM || FORM || STATES || (FULL && (u == 2 || LATER)));
         const float p = -sc * cur.lr * rstd;
         const float c1 = p * rstd, c2 = -c1 * s2 * inv_d, c3 = -p * s1 * inv_d;
 #pragma unroll
@@ -698,7 +713,7 @@ __device__ __forceinline__ void linear_fwd_sk_body(const LinearFwdArgs& a, const
         pw1 *= adam->beta1;
         pw2 *= adam->beta2;
         {
-          // v^ = v c2, m^ = m c1: lr m^ / (sqrt(v^) + eps) = (lr c1 / sqrt(c2)) m / (sqrt(v) + eps / sqrt(c2))
+          // v^ = v c2, m^ = m c1: lr m^ / (sqrt(v^) + eps()) = (lr c1 / sqrt(c2)) m / (sqrt(v) + eps / sqrt(c2))
           const float c1 = (1.f - adam->beta1) / (1.f - pw1), rc2 = sqrtf((1.f - pw2) / (1.f - adam->beta2));
           ad_k = -adam->lr * c1 * rc2;
           ad_e = adam->eps * rc2;
@@ -744,16 +759,16 @@ __device__ __forceinline__ void linear_fwd_sk_body(const LinearFwdArgs& a, const
     }
   };
   if constexpr (COMPACT) {
-    for (int st0 = 0; st0 < a.n_stages; st0 += R) pass(std::true_type{}, st0);
+    for (int st0 = 0; st0 < n_st(); st0 += R) pass(std::true_type{}, std::false_type{}, st0);
   } else if constexpr (NT <= 4) {
     int st0 = 0;
-    pass(std::true_type{}, st0);
-    for (st0 = R; st0 + R <= a.n_stages; st0 += R) pass(std::false_type{}, st0);
-    if (st0 < a.n_stages) pass(std::true_type{}, st0);
+    pass(std::true_type{}, std::false_type{}, st0);
+    for (st0 = R; st0 + R <= n_st(); st0 += R) pass(std::false_type{}, std::true_type{}, st0);
+    if (st0 < n_st()) pass(std::true_type{}, std::true_type{}, st0);
   } else {
     // Wide heads (d = 96, 128) keep the loop with its branches: in one long basic block the scheduler overlaps
     // so much that the state tiles no longer fit the register file (d = 128: 30 spilled registers).
-    for (int st0 = 0; st0 < a.n_stages; st0 += R) {
+    for (int st0 = 0; st0 < n_st(); st0 += R) {
 #pragma unroll
       for (int u = 0; u < R; ++u) {
         const int st = st0 + u;
@@ -761,7 +776,7 @@ __device__ __forceinline__ void linear_fwd_sk_body(const LinearFwdArgs& a, const
           load_raw(raw[u], st + R);
         else
           load_stage_mw<T, D, NW, FULL>(buf[(u + PF) % R], ub, K, n_stages_, st + PF, c, g, w);
-        if (st >= a.n_stages) continue;
+        if (st >= n_st()) continue;
         const StageInMw<T, NT, TPW>& cur = buf[u];
 
         if (ck.due()) {
@@ -849,9 +864,9 @@ __device__ __forceinline__ void linear_fwd_sk_body(const LinearFwdArgs& a, const
         {
           const float mu = S[0] * inv_d;
           const float var = S[1] * inv_d - mu * mu;
-          const float rstd = __builtin_amdgcn_rsqf(fmaxf(var, 0.f) + a.eps);
+          const float rstd = __builtin_amdgcn_rsqf(fmaxf(var, 0.f) + eps());
           const float s1 = rstd * (S[2] - mu * sum_a) + S[4];
-          const float s2 = rstd * rstd * (S[3] - 2.f * mu * S[2] + mu * mu * sum_a) + rstd * (S[5] - mu * S[4]);
+          const float s2 = g_norm_sum(S, mu, rstd, FULL && u == 2);
           const float p = -sc * cur.lr * rstd;
           const float c1 = p * rstd, c2 = -c1 * s2 * inv_d, c3 = -p * s1 * inv_d;
 #pragma unroll
@@ -904,9 +919,9 @@ __device__ __forceinline__ void linear_fwd_sk_body(const LinearFwdArgs& a, const
   {
     float S[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     pend_sums(zbp, S[6], S[7]);
-    exchange8(S, a.n_stages & 1);
-    if (a.n_stages >= 2) emit_output(so0, so1, a.n_stages - 2, zbo, qoo);
-    emit_output(S[6], S[7], a.n_stages - 1, zbp, qop);
+    exchange8(S, n_st() & 1);
+    if (n_st() >= 2) emit_output(so0, so1, n_st() - 2, zbo, qoo);
+    emit_output(S[6], S[7], n_st() - 1, zbp, qop);
   }
   store_state_final<D, TPW>(a.W_out + bh * D * D, a.b_out + bh * D, a.W0 + sb * D * D, a.b0 + sb * D, Wc, bT, m0s, w, c, g);
   if constexpr (ADAM) {
