@@ -135,3 +135,21 @@ def test_mixed_shapes_five_wait_states_apart_are_exact():
             if gap == 5:
                 assert exact, f"order {order}: five wait states between the two shapes no longer suffice"
     assert P.lib().ttt_selftest_mfma_mixed(4, 5, C.c_void_p(out.data_ptr()), stream) == P.TTT_ERR_SHAPE
+
+
+def test_scanner_flags_a_result_read_too_early_behind_a_branch():
+    """The compiler counts the wait states between a matrix instruction and a read of its result in straight code, not
+    across a branch: one instruction (the branch) in between read garbage on MI355X, one more did not."""
+    def code(between, behind):
+        return [K32.format(c="0")] + between + ["\ts_cbranch_vccnz .LBB0_2", "\ts_branch .LBB0_1", ".LBB0_1:", "\ts_nop 7", ".LBB0_2:"] + behind
+    read = "\tv_mul_f32_e32 v40, v41, v{r}"
+    assert [h[4] for h in flagged(code([], [read.format(r=0)]))] == [1]
+    assert [h[4] for h in flagged(code([], ["\tds_write_b32 v9, v3"]))] == [1]
+    assert [h[4] for h in flagged(code([], ["\tv_mov_b32_e32 v2, 0"]))] == [1]  # a write is overtaken as well
+    assert flagged(code(["\ts_add_i32 s0, s1, s2"], [read.format(r=0)])) == []
+    assert flagged(code([], ["\ts_nop 4", read.format(r=0)])) == []
+    assert flagged(code([], [read.format(r=12)])) == []
+    # straight code, and code behind a branch that is always taken, which the text order does not reach
+    assert [h[4] for h in flagged([K32.format(c="0"), "\ts_nop 2", read.format(r=1)])] == [3]
+    assert flagged([K32.format(c="0"), "\ts_nop 3", "\ts_nop 0", read.format(r=1)]) == []
+    assert flagged([K32.format(c="0"), "\ts_branch .LBB0_9", read.format(r=1), ".LBB0_9:", "\ts_endpgm"]) == []

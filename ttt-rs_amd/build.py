@@ -65,8 +65,8 @@ def build_library(verbose: bool = False, extra_flags=()) -> str:
         if bad:
             for func, no, a, b, ws in bad[:20]:
                 sys.stderr.write(f"{os.path.basename(path)}:{no}: in {func}: {ws} wait state(s) between\n    {a}\n    {b}\n")
-            raise RuntimeError(f"{len(bad)} in-place accumulations onto a matrix instruction of another shape sit closer "
-                               "than the hardware needs (see isa_check.py); library not installed")
+            raise RuntimeError(f"{len(bad)} uses of a matrix instruction's result sit closer to it than the hardware needs (see "
+                               "isa_check.py); library not installed")
         sel = isa_check.check_scc_select_file(path)
         if sel:
             for func, no, a, b in sel[:20]:

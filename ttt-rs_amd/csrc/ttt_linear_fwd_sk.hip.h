@@ -198,6 +198,10 @@ __device__ __forceinline__ void linear_fwd_sk_body(const LinearFwdArgs& a, const
     qop[jj] = qoo[jj] = IO::zero();
   }
 
+  // Every sum starts from its first term, not from zero: a wave is bound by the number of instructions it issues, and each
+  // sum from zero has one that adds nothing (d = 32, 384 units x 2048 tokens: 97.4 -> 95.4 us, d = 64 116.5 -> 114.7, d = 96, 128
+  // units 146.5 -> 143.6, d = 128, 64 units 193.7 -> 190.6; f32, d = 64, 96 units 215.7 -> 211.9).  Not with the Adam step (230 -> 235).
+  constexpr bool FIRST = !ADAM;
   // publish this lane group's two sums ...
   auto exchange8_publish = [&](const float (&S)[8], int parity) {
     // lane group g ends up with sums g and g+4 reduced over the wave, and publishes them
@@ -213,9 +217,9 @@ __device__ __forceinline__ void linear_fwd_sk_body(const LinearFwdArgs& a, const
     lds_barrier();
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-      float s = 0.f;
+      float s = FIRST ? e[(i * 16 + c) * NW] : 0.f;
 #pragma unroll
-      for (int ww = 0; ww < NW; ++ww) s += e[(i * 16 + c) * NW + ww];
+      for (int ww = FIRST; ww < NW; ++ww) s += e[(i * 16 + c) * NW + ww];
       S[i] = s;
     }
   };
@@ -231,9 +235,33 @@ __device__ __forceinline__ void linear_fwd_sk_body(const LinearFwdArgs& a, const
     for (int jj = 0; jj < TPW; ++jj)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        s0 += z[jj][r];
-        s1 = __builtin_fmaf(z[jj][r], z[jj][r], s1);
+        const bool first = FIRST && jj == 0 && r == 0;
+        s0 = first ? z[jj][r] : s0 + z[jj][r];
+        s1 = first ? z[jj][r] * z[jj][r] : __builtin_fmaf(z[jj][r], z[jj][r], s1);
       }
+  };
+  // the six moments of Z1, feature tile jj
+  float z_first = 0.f;
+  auto moments = [&](float (&S)[8], int jj, const f32x4& z, const f32x4& uu, const f32x4& bq) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const float az = a2[jj][r] * z[r];
+      if (jj == 0 && r == 0) z_first = z[r];
+      if (FIRST && jj == 0 && r == 0) {
+        S[0] = z[r];
+        S[2] = az;
+        S[3] = az * z[r];
+        S[4] = bq[r];
+        S[5] = bq[r] * z[r];
+      } else {
+        S[0] += z[r];
+        if (jj != 0 || r != 0) S[1] = jj == 0 && r == 1 ? __builtin_fmaf(z_first, z_first, z[r] * z[r]) : __builtin_fmaf(z[r], z[r], S[1]);
+        S[2] = __builtin_fmaf(a2[jj][r], z[r], S[2]);
+        S[3] = __builtin_fmaf(az, z[r], S[3]);
+        S[4] = __builtin_fmaf(gam[jj][r], uu[r], S[4]);
+        S[5] = __builtin_fmaf(bq[r], z[r], S[5]);
+      }
+    }
   };
   // out = xq + gamma (zbar - mu) rstd + beta for the pending mini-batch
   auto emit_output = [&](float s0, float s1, int stage, const f32x4 (&zbp)[TPW], const frag (&qop)[TPW]) {
@@ -614,28 +642,14 @@ __device__ __forceinline__ void linear_fwd_sk_body(const LinearFwdArgs& a, const
         IO::mma(At, cur.ko[0], cur.qo[0]);  // over the own 16 features
         atx[st & 1][w][lane] = At;
       }
-      // ---- row sums: six raw moments of Z1 (this mini-batch), two of the pending Zbar
-      f32x4 bq[TPW];
-      float S[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, ps0, ps1};  // the pending Zbar's in-lane sums are ready
+      f32x4 bq[TPW], uu[TPW];  // uu = beta - (xv - xk)
 #pragma unroll
       for (int jj = 0; jj < TPW; ++jj) {
-        f32x4 uu;  // beta - (xv - xk)
         if (BF) {
-          uu = bet[jj];
-          IO::mma2(uu, nident, ident, cur.vo[jj], cur.ko[jj]);
+          uu[jj] = bet[jj];
+          IO::mma2(uu[jj], nident, ident, cur.vo[jj], cur.ko[jj]);
         } else {
-          uu = bet[jj] - (IO::to_f32(cur.vo[jj]) - IO::to_f32(cur.ko[jj]));
-        }
-        bq[jj] = gam[jj] * uu;
-        const f32x4 az = a2[jj] * z1[jj];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          S[0] += z1[jj][r];
-          S[1] += z1[jj][r] * z1[jj][r];
-          S[2] += az[r];
-          S[3] += az[r] * z1[jj][r];
-          S[4] += bq[jj][r];
-          S[5] += bq[jj][r] * z1[jj][r];
+          uu[jj] = bet[jj] - (IO::to_f32(cur.vo[jj]) - IO::to_f32(cur.ko[jj]));
         }
       }
       // ---- checkpoint of the state entering this mini-batch (W and b change only behind the barrier);
@@ -650,6 +664,19 @@ __device__ __forceinline__ void linear_fwd_sk_body(const LinearFwdArgs& a, const
         ck.advance();
       }
       if constexpr (!ADAM) ck.next_stage();
+      // The compiler does not count the wait states between a matrix instruction and a read of its result behind a branch,
+      // and so few instructions are left in between that the read comes too early (isa_check.py).
+      if constexpr (BF && !ADAM) {
+        if constexpr (TPW == 1) asm volatile("s_nop 4" : "+v"(z1[0]), "+v"(uu[0]));
+        else asm volatile("s_nop 4" : "+v"(z1[0]), "+v"(uu[0]), "+v"(z1[1]), "+v"(uu[1]));
+      }
+      // ---- row sums: six raw moments of Z1 (this mini-batch), two of the pending Zbar
+      float S[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, ps0, ps1};  // the pending Zbar's in-lane sums are ready
+#pragma unroll
+      for (int jj = 0; jj < TPW; ++jj) {
+        bq[jj] = gam[jj] * uu[jj];
+        moments(S, jj, z1[jj], uu[jj], bq[jj]);
+      }
       exchange8_publish(S, st & 1);
       // ---- the output pending since two mini-batches (sums known since the last exchange): nothing waits
       // for it, and here it runs while this exchange is in flight (LDS write, barrier, LDS read)
@@ -835,16 +862,7 @@ __device__ __forceinline__ void linear_fwd_sk_body(const LinearFwdArgs& a, const
             uu = bet[jj] - (IO::to_f32(cur.vo[jj]) - IO::to_f32(cur.ko[jj]));
           }
           bq[jj] = gam[jj] * uu;
-          const f32x4 az = a2[jj] * z1[jj];
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            S[0] += z1[jj][r];
-            S[1] += z1[jj][r] * z1[jj][r];
-            S[2] += az[r];
-            S[3] += az[r] * z1[jj][r];
-            S[4] += bq[jj][r];
-            S[5] += bq[jj][r] * z1[jj][r];
-          }
+          moments(S, jj, z1[jj], uu, bq[jj]);
         }
         pend_sums(zbp, S[6], S[7]);
         exchange8_publish(S, st & 1);

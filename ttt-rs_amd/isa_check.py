@@ -13,6 +13,13 @@ not listed), counting every instruction in between as one wait state and `s_nop 
 text order and, from every branch, on into the branch target while an earlier matrix instruction can still matter
 (loop back edges included).
 
+The scan also reports a read or write of a matrix instruction's result by any other instruction within the same distance.  In
+straight code the compiler keeps more (eight wait states behind an instruction of four passes), but it loses count where a
+branch lies in between: a read directly behind a taken branch that follows the matrix instruction returned garbage in
+every mini-batch with two waves on a SIMD; with one more instruction in between it was right.  A taken branch therefore
+counts as four wait states for such a use (it counts as one for an accumulator).  (The cure in source is an s_nop behind
+the branch that names the registers as its operands.)
+
 Functions whose name contains "selftest" are skipped: the library's own test of this fact places such pairs on
 purpose, in inline assembly.
 
@@ -58,14 +65,29 @@ def _overlap(a, b):
 _BRANCH = re.compile(r"^s_c?branch\w*\s+(\.L\w+)")
 
 
+_READERS = ("v_", "ds_", "global_", "buffer_", "scratch_")
+_OPERAND = re.compile(r"^[-|]*([av])(?:\[(\d+):(\d+)\]|(\d+)\b)")
+
+
+def _operand(text: str):
+    """Register range of an operand, or None."""
+    m = _OPERAND.match(text.strip())
+    if not m:
+        return None
+    return (m.group(1), int(m.group(2)), int(m.group(3))) if m.group(2) else (m.group(1), int(m.group(4)), int(m.group(4)))
+
+
 def _states(s: str) -> int:
     n = re.match(r"s_nop\s+(\d+)", s)
     return int(n.group(1)) + 1 if n else 1
 
 
-def _step(window, s, m, func, no):
+TAKEN_BRANCH = 4
+
+
+def _step(window, s, m, func, no, taken=0):
     """Advances the window of recent MFMAs over instruction `s` (m: its MFMA match or None); returns the new window
-    and the hazards this instruction completes."""
+    and the hazards this instruction completes.  taken: wait states of a branch in front, beyond the one it counts as."""
     found = []
     if m:
         op, dst = m.group(1), (m.group(2), int(m.group(3)), int(m.group(4)))
@@ -74,6 +96,11 @@ def _step(window, s, m, func, no):
             for w in window:
                 if _overlap(w[1], c) and w[0] != op and w[2] < min_wait_states(w[0]):
                     found.append((func, no, w[3], s, w[2]))
+    elif "selftest" not in func and s.startswith(_READERS):
+        regs = [r for r in map(_operand, s.split(None, 1)[1].split(",")) if r is not None] if " " in s else []
+        for w in window:
+            if w[2] + taken < min_wait_states(w[0]) and any(_overlap(w[1], r) for r in regs):
+                found.append((func, no, w[3], s, w[2]))
     states = _states(s)
     # a write to the same registers by anything else ends the dependence; keeping the entry is conservative
     window = [[w[0], w[1], w[2] + states, w[3], w[4]] for w in window if w[2] + states < MAX_WINDOW]
@@ -134,7 +161,7 @@ def scan(lines):
                     break
                 if s2 is None:
                     continue
-                w2, found = _step(w2, s2, _MFMA.match("\t" + s2), func, no2)
+                w2, found = _step(w2, s2, _MFMA.match("\t" + s2), func, no2, TAKEN_BRANCH - 1)
                 # only what was in flight at the branch matters here: later instructions are met in text order
                 w2 = [w for w in w2 if w[4] <= no or w[4] > no2]
                 for h in found:
@@ -143,6 +170,8 @@ def scan(lines):
                         yield h
                 if s2.startswith("s_endpgm") or s2.startswith("s_branch"):
                     break
+        if s.startswith(("s_branch", "s_endpgm")):
+            window = []  # what follows in the text is reached through branches only
 
 
 def check_file(path: str):
@@ -228,7 +257,7 @@ if __name__ == "__main__":
     bad = check_file(sys.argv[1])
     for func, no, a, b, ws in bad:
         print(f"{sys.argv[1]}:{no}: in {func}: {ws} wait state(s) between\n    {a}\n    {b}")
-    print(f"{len(bad)} MFMA pair(s) of different shapes, the second accumulating from the first, closer than the first's passes + 1 wait states")
+    print(f"{len(bad)} use(s) of a matrix instruction's result closer than its passes + 1 wait states")
     sel = check_scc_select_file(sys.argv[1])
     for func, no, a, b in sel:
         print(f"{sys.argv[1]}:{no}: in {func}: scalar select on a vector comparison\n    {a}\n    {b}")
