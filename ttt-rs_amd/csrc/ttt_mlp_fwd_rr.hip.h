@@ -18,15 +18,19 @@
 //   B1  partial Z2 tiles (and last mini-batch's partial Zbar2 / A2) are in LDS
 //   B2  the reducers' row moments for the LN-L2 gradient are in LDS
 //   B3  G2 (already scaled by -eta_last) is in LDS, and the row moments of last mini-batch's output
-// The output of mini-batch t needs nothing the recurrence waits for: it is finished one mini-batch late, and between B1
-// and B3 it is the work of the waves that reduce nothing, so that the reducers' chain is the only thing there.
+// The output of mini-batch t needs nothing the recurrence waits for: it is finished one mini-batch late, where waves have time.
+// At d = 96 its sums are formed at the end of phase A by the older waves (0 - 3: of the two waves of a SIMD they run 2 k cycles
+// ahead and would wait at B1) and stored between B1 and B3 by the two waves that reduce nothing; at d = 32 and 64 there are
+// more such waves, and all of it is theirs.
 //
 // What bounds it.  Phases A and D (the products) by the issue of a SIMD's two waves: matrix instructions and vector
 // instructions of 16x16 tiles hardly overlap, not across waves either (probe: a matrix instruction and three FMAs, two
 // waves, 23.3 cycles against 16 + 7.5).  Phases B and C by latency.  Cycles of a mini-batch at d = 96 and 128 units,
-// before -> after the last revision: A 4.9 -> 4.7 k (XQ W1 now shares the operands of XK W1), B 2.9 -> 2.0 k, C 2.2 -> 1.3 k
-// (output off the chain, loads in one go, sums by lane group), D 7.4 -> 6.4 k (independent products side by side, transposes
-// read from LDS).  8 x 16 units x 2048 tokens: d = 96 840 -> 667 us, d = 64 488 -> 433 us, d = 32 286 -> 261 us.
+// before -> after the revision before last: A 4.9 -> 4.7 k (XQ W1 now shares the operands of XK W1), B 2.9 -> 2.0 k, C 2.2 -> 1.3 k
+// (sums by lane group), D 7.4 -> 6.4 k (independent products side by side, transposes read from LDS).  The last one took the
+// output out of B (three tiles of sums by two waves were its longest path, 2.1 k) and D, the staging copies from the younger
+// waves and a load of eps through the scalar cache from C.  8 x 16 units x 2048 tokens: d = 96 840 -> 661 -> 640 us, d = 64 488 -> 428 ->
+// 416, d = 32 286 -> 260 -> 247; saving d = 96 715 -> 687, d = 64 467 -> 444, d = 32 284 -> 270.
 //
 // An odd hidden tile at the end of a split-k chain is issued as a k = 32 MFMA with a zero second
 // half, not as a k = 16 one: a 16x16x16 bf16 MFMA accumulating straight onto the result of a
@@ -63,7 +67,8 @@ struct MlpRrLds {
   static constexpr int M1 = X2S + NW * XS * 64 * 4 * ES;  // [2][64] frag: M1 of this mini-batch
   static constexpr int ID = M1 + 2 * 64 * 4 * ES;  // [64] frag: identity
   static constexpr int RHO = ID + 64 * 4 * ES;  // [16] token_eta / sc
-  static constexpr int BYTES = RHO + 64;
+  static constexpr int FL = RHO + 64;           // [NW] counters
+  static constexpr int BYTES = FL + 4 * NW;
   static_assert(BYTES <= 160 * 1024, "exceeds the 160 KiB of LDS of a gfx950 CU");
   static_assert(NT <= NW && D % 32 == 0, "one reducer wave per d-feature tile");
   static_assert(ES == 2, "the transposing LDS load takes 16-bit elements");
@@ -154,9 +159,13 @@ __global__ void __launch_bounds__(512, D == 32 ? 4 : 2) ttt_mlp_fwd_rr_kernel(Pr
   int c = lane & 15, g = lane >> 4;
   const size_t bh = blockIdx.x;
   const int h = (int)(bh % a.H), K = a.K;
+  const float eps = held(a.eps);
   const bool red = w < NT;  // this wave reduces d-feature tile w
-  // this wave finishes output tiles (at d = 32 there are more waves left than tiles)
+  // this wave stores output tiles (at d = 32 there are more waves left than tiles)
   const bool outw = !red && (2 * NT >= NW || w < 2 * NT);
+  const bool older = w < 4;               // the first wave of its SIMD
+  constexpr bool LATE = D <= 64;
+  const bool outs = LATE ? outw : older;   // this wave adds up output tiles
 
   f32x4* const P1 = reinterpret_cast<f32x4*>(smem + L::P1);
   f32x4* const P2 = reinterpret_cast<f32x4*>(smem + L::P2);
@@ -166,6 +175,7 @@ __global__ void __launch_bounds__(512, D == 32 ? 4 : 2) ttt_mlp_fwd_rr_kernel(Pr
   frag* const IDs = reinterpret_cast<frag*>(smem + L::ID);
   float* const RHO = reinterpret_cast<float*>(smem + L::RHO);
   frag* const M1s = reinterpret_cast<frag*>(smem + L::M1);
+  lds_int* const FL = (lds_int*)(smem + L::FL);
   f32x4* const ZB = reinterpret_cast<f32x4*>(smem + L::ZB);
   frag* const GT = reinterpret_cast<frag*>(smem + L::GT);
   frag* const X2S = reinterpret_cast<frag*>(smem + L::X2S) + w * L::XS * 64;
@@ -230,26 +240,26 @@ __global__ void __launch_bounds__(512, D == 32 ? 4 : 2) ttt_mlp_fwd_rr_kernel(Pr
   // written below.  Three buffers: mini-batch st+1 is fetched while st is computed, and rows of
   // st are still read (for the W1 update) after the slowest wave has started st+1's fetch.
   // Per wave block a running source address, scalar like everything but the lane's offset.
-  constexpr int NBLK = L::IN1 / 1024, NBI = (NBLK + NW - 1) / NW;
+  constexpr int NBLK = L::IN1 / 1024, NBI = (NBLK + 3) / 4;
   const unsigned lds0 = __builtin_amdgcn_readfirstlane((unsigned)(size_t)(__attribute__((address_space(3))) unsigned char*)smem);
   const unsigned step = (unsigned)(K * D * ES);
   const unsigned char* srcp[NBI];
 #pragma unroll
   for (int it = 0; it < NBI; ++it) {
-    const int b = w + NW * it, ten = (1024 * b) / L::TILE;
+    const int b = (w & 3) + 4 * it, ten = (1024 * b) / L::TILE;
     srcp[it] = static_cast<const unsigned char*>(ten == 0 ? a.xq : ten == 1 ? a.xk : a.xv) + bh * (size_t)a.seq_stride * (D * ES);
   }
   const unsigned char* lrp = static_cast<const unsigned char*>(a.lr) + bh * (size_t)a.seq_stride * ES;
   unsigned char* const outp = static_cast<unsigned char*>(a.out) + bh * (size_t)a.seq_stride * (D * ES);
-  unsigned fdst = lds0 + L::IN + 1024 * w, flr = lds0 + L::LR;  // where the next mini-batch goes
+  unsigned fdst = lds0 + L::IN + 1024 * (w & 3), flr = lds0 + L::LR;  // where the next mini-batch goes
   const int n_stages = a.n_stages;
   auto fetch = [&](int stage) {
     if (stage >= n_stages) return;
 #pragma unroll
     for (int it = 0; it < NBI; ++it) {
-      const int b = w + NW * it;
+      const int b = w + 4 * it;
       const unsigned off = (1024u * b) % L::TILE + 16u * lane;
-      if (b < NBLK && off < step) lds_dma16(srcp[it], off, fdst + 1024 * NW * it);
+      if (b < NBLK && off < step) lds_dma16(srcp[it], off, fdst + 4096 * it);
       srcp[it] += step;
     }
     // lr as zero-extended bf16 words, copied like the tiles (a register load here would make the compiler
@@ -268,8 +278,9 @@ __global__ void __launch_bounds__(512, D == 32 ? 4 : 2) ttt_mlp_fwd_rr_kernel(Pr
   for (int i = tid; i < (L::PRM - L::IN) / 4; i += 512) reinterpret_cast<float*>(smem)[i] = 0.f;
   for (int i = tid; i < 6 * 2 * 16 * 4; i += 512) EX[i] = 0.f;
   if (tid < 2 * 2 * 16 * 4) EXO[tid] = 0.f;
+  if (tid < NW) FL[tid] = 0;
   __syncthreads();
-  fetch(0);
+  if (older) fetch(0);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
 
@@ -298,81 +309,82 @@ __global__ void __launch_bounds__(512, D == 32 ? 4 : 2) ttt_mlp_fwd_rr_kernel(Pr
     }
   };
 
-  // ---- output path.  The waves that reduce no Z2 tile (w >= NT) finish the previous mini-batch's Zbar2 beside the
-  // reducers' chain, wave w the tiles (w - NT) + (NW - NT) i: sums over the split-k partials in phase B, causal
-  // correction and row moments in phase C.  The reducers store it, a tile each, in phase D.  (By reducers as well, the
-  // older wave of each SIMD after its own tile, both phases took 0.8 k cycles longer.)
-  constexpr int NOW = NW - NT, OPW = (NT + NOW - 1) / NOW;
-  f32x4 zo[OPW];
-  frag m2f = IO::zero();
-  auto otile = [&](int i) { const int I = (w - NT) + NOW * i; return I < NT ? I : 0; };
-  auto output_sum = [&]() {
-    const f32x4* p = P2 + lane;
-#pragma unroll
-    for (int i = 0; i < OPW; ++i) {
-      const int I = otile(i);
-      f32x4 v[NW];
-#pragma unroll
-      for (int ww = 0; ww < NW; ++ww) v[ww] = p[(ww * NT + I) * 64];
-      together(v);
-      zo[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int ww = 0; ww < NW; ++ww) zo[i] += v[ww];
+  // ---- output path: the sums, causal correction and row moments of mini-batch t by the older waves at the end of phase A of
+  // t + 1, wave w the tiles w + 4 i; the stores by the waves that reduce no Z2 tile, beside the reducers in phase B.
+  // There is no barrier between a wave's partial blocks and the wave that adds them up: each wave waits for its blocks to
+  // be in LDS (lds_done) and then counts up its own word there.  Blocks and word are LDS instructions both (FL carries the
+  // address space).  The wait needs no bound: on its way from B3 to the counter a wave waits for nobody.
+  constexpr int EW = NW - NT, EPW = (NT + EW - 1) / EW, OPW = LATE ? 1 : (NT + 3) / 4;
+  static_assert(!LATE || EPW == 1, "one tile per wave");
+  auto otile = [&](int i) { return LATE ? w - NT : w + 4 * i; };
+  auto output_finish = [&](int stage) {
+    if (!LATE) {
+      while (__builtin_amdgcn_ballot_w64(__hip_atomic_load(FL + (lane & 7), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) <= stage) != 0) {
+      }
+      lds_done();
     }
-  };
-  // M2[s][t] = (token_eta[t] / sc)(1 + A2[t][s]) for s <= t
-  auto output_m2 = [&]() {
-    const float rho_c = rho();
-    f32x4 at = {0.f, 0.f, 0.f, 0.f};
+    frag m2f;
     {
+      // M2[s][t] = (token_eta[t] / sc)(1 + A2[t][s]) for s <= t
+      const float rho_c = rho();
+      f32x4 at = {0.f, 0.f, 0.f, 0.f};
       f32x4 v[NW];
 #pragma unroll
       for (int ww = 0; ww < NW; ++ww) v[ww] = PA[ww * 64 + lane];
       together(v);
 #pragma unroll
       for (int ww = 0; ww < NW; ++ww) at += v[ww];
-    }
-    f32x4 m;
+      f32x4 m;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) m[r] = (4 * g + r <= c) ? rho_c * (1.f + at[r]) : 0.f;
-    m2f = IO::to_frag(m);
-  };
-  auto output_moments = [&](int stage) {
+      for (int r = 0; r < 4; ++r) m[r] = (4 * g + r <= c) ? rho_c * (1.f + at[r]) : 0.f;
+      m2f = IO::to_frag(m);
+    }
     float s[2 * OPW];
 #pragma unroll
-    for (int i = 0; i < OPW; ++i) IO::mma(zo[i], read_tr(GT + (((stage & 1) * NT) + otile(i)) * 64 + tr_lane(lane)), m2f);
-#pragma unroll
     for (int i = 0; i < OPW; ++i) {
+      const int I = otile(i);
       s[2 * i] = s[2 * i + 1] = 0.f;
+      if (I >= NT) continue;
+      f32x4 v[NW], zo = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int ww = 0; ww < NW; ++ww) v[ww] = P2[(ww * NT + I) * 64 + lane];
+      together(v);
+#pragma unroll
+      for (int ww = 0; ww < NW; ++ww) zo += v[ww];
+      IO::mma(zo, read_tr(GT + (((stage & 1) * NT) + I) * 64 + tr_lane(lane)), m2f);
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        s[2 * i] += zo[i][r];
-        s[2 * i + 1] += zo[i][r] * zo[i][r];
+        s[2 * i] += zo[r];
+        s[2 * i + 1] += zo[r] * zo[r];
       }
+      ZB[I * 64 + lane] = zo;
     }
-    // lane group g: sum g & 1 of this wave's tile i + g / 2
-#pragma unroll
-    for (int i = 0; i < OPW; i += 2) {
-      const bool two = i + 1 < OPW;
-      const float v = xg_sum4_scatter(s[2 * i], s[2 * i + 1], two ? s[2 * i + 2 * two] : 0.f, two ? s[2 * i + 2 * two + 1] : 0.f);
-      const int I = (w - NT) + NOW * (i + (g >> 1));
-      if (I < NT && (two || g < 2)) EXO[(((g & 1) * 2 + (I >> 2)) * 16 + c) * 4 + (I & 3)] = v;
-    }
-#pragma unroll
-    for (int i = 0; i < OPW; ++i)
-      if ((w - NT) + NOW * i < NT) ZB[((w - NT) + NOW * i) * 64 + lane] = zo[i];
+    // lane group g: sum g & 1 of this wave's tile g / 2
+    static_assert(OPW <= 2, "two sums of two tiles, a lane group each");
+    const float v = xg_sum4_scatter(s[0], s[1], OPW > 1 ? s[2 * OPW - 2] : 0.f, OPW > 1 ? s[2 * OPW - 1] : 0.f);
+    const int I = otile(g >> 1);
+    if (I < NT && (OPW > 1 || g < 2)) EXO[(((g & 1) * 2 + (I >> 2)) * 16 + c) * 4 + (I & 3)] = v;
   };
-  // out = xq + gamma (zbar - mu) rstd + beta, tile w
-  auto output_emit = [&](int stage, frag qo) {
-    const f32x4 zb = ZB[w * 64 + lane];
-    float mu, ms;
-    collect2(EXO, 0, 1, mu, ms);
-    mu *= inv_d;
-    const float rstd = __builtin_amdgcn_rsqf(fmaxf(ms * inv_d - mu * mu, 0.f) + a.eps);
-    if (c < K) {
-      const f32x4 gam = *reinterpret_cast<const f32x4*>(GAM + own), bet = *reinterpret_cast<const f32x4*>(BET + own);
-      elem* po = reinterpret_cast<elem*>(outp + (size_t)stage * step) + (c * D + own);
-      store4<T>(po, IO::to_f32(qo) + bet + gam * ((zb - mu) * rstd));
+  // out = xq + gamma (zbar - mu) rstd + beta, tiles (w - NT) + EW i for i in [i0, i1)
+  float o_mu = 0.f, o_rstd = 0.f;
+  auto output_stats = [&]() {
+    float ms;
+    collect2(EXO, 0, 1, o_mu, ms);
+    o_mu *= inv_d;
+    o_rstd = __builtin_amdgcn_rsqf(fmaxf(ms * inv_d - o_mu * o_mu, 0.f) + eps);
+  };
+  auto output_emit = [&](int stage, int i0, int i1) {
+#pragma unroll
+    for (int i = i0; i < i1; ++i) {
+      const int I = (w - NT) + EW * i;
+      if (I >= NT) continue;
+      const int own_o = own_offset<1>(I, 0, g);
+      const f32x4 zb = ZB[I * 64 + lane];
+      const frag qo = load4<T>(row(stage % 3, 0) + own_o);
+      const f32x4 gam = *reinterpret_cast<const f32x4*>(GAM + own_o), bet = *reinterpret_cast<const f32x4*>(BET + own_o);
+      const f32x4 o = IO::to_f32(qo) + bet + gam * ((zb - o_mu) * o_rstd);
+      elem* po = reinterpret_cast<elem*>(outp + (size_t)stage * step) + (c * D + own_o);
+      if (c < K) store4<T>(po, o);
     }
   };
   // partial tiles of X W2 over this wave's hidden units, two at a time
@@ -402,7 +414,7 @@ __global__ void __launch_bounds__(512, D == 32 ? 4 : 2) ttt_mlp_fwd_rr_kernel(Pr
     const int buf = st % 3;
     frag* const GTc = GT + (st & 1) * NT * 64;
     RELANE();
-    fetch(st + 1);
+    if (older) fetch(st + 1);
 
     // ================= phase A: everything that needs only W1, W2 and the inputs
     f32x4 z1[HT], zq[HT];
@@ -445,8 +457,9 @@ __global__ void __launch_bounds__(512, D == 32 ? 4 : 2) ttt_mlp_fwd_rr_kernel(Pr
 #pragma unroll
     for (int j = 0; j < L::XS; ++j) X2S[j * 64 + lane] = x2f[j];
     partials(P1, x2f, false);
-    // M1[s][t] = (token_eta[t] / sc)(1 + A1[t][s]) for s <= t.  By wave 3: of the two waves of a SIMD the older runs ahead
-    // and would wait at B1 for 2 k cycles
+    // of the two waves of a SIMD the older runs ahead and would wait at B1 for 2 k cycles
+    if (!LATE && outs && st > 0) output_finish(st - 1);
+    // M1[s][t] = (token_eta[t] / sc)(1 + A1[t][s]) for s <= t
     if (w == 3) {
       const float rho_c = rho();
       f32x4 At = {0.f, 0.f, 0.f, 0.f};
@@ -466,9 +479,8 @@ __global__ void __launch_bounds__(512, D == 32 ? 4 : 2) ttt_mlp_fwd_rr_kernel(Pr
     RELANE();
 
     // ================= phase B: reducers: full Z2 tile and its row moments;
-    //                          the other waves: Zbar2 tiles and causal correction of the previous mini-batch
+    //                          the other waves: stores of the previous mini-batch's output
     f32x4 z = {0.f, 0.f, 0.f, 0.f}, bq = z;
-    frag qo = IO::zero();
     if (red) {
       const f32x4* p = P1 + w * 64 + lane;
       const frag ko = load4<T>(row(buf, 1) + own), vo = load4<T>(row(buf, 2) + own);
@@ -494,13 +506,17 @@ __global__ void __launch_bounds__(512, D == 32 ? 4 : 2) ttt_mlp_fwd_rr_kernel(Pr
       }
       publish(S);
     } else if (outw && st > 0) {
-      output_sum();
-      output_m2();
+      if (LATE) {
+        output_finish(st - 1);
+      } else {
+        output_stats();
+        output_emit(st - 1, 0, 1);
+      }
     }
     lds_barrier();  // ---- B2
     RELANE();
 
-    // ================= phase C: reducers: G2''; the other waves: the rest of Zbar2
+    // ================= phase C: reducers: G2''
     if (red) {
       const float lrc = (c < K) ? __uint_as_float(LRs[buf * 16 + c] << 16) : 0.f;
       float S[6];
@@ -524,20 +540,21 @@ __global__ void __launch_bounds__(512, D == 32 ? 4 : 2) ttt_mlp_fwd_rr_kernel(Pr
       }
       const float mu = S[0] * inv_d;
       const float var = S[1] * inv_d - mu * mu;
-      const float rstd = __builtin_amdgcn_rsqf(fmaxf(var, 0.f) + a.eps);
+      const float rstd = __builtin_amdgcn_rsqf(fmaxf(var, 0.f) + eps);
       const float s1 = rstd * (S[2] - mu * sum_a) + S[4];
-      const float s2 = rstd * rstd * (S[3] - 2.f * mu * S[2] + mu * mu * sum_a) + rstd * (S[5] - mu * S[4]);
+      const float m5 = S[5] - mu * S[4], q3 = S[3] - 2.f * mu * S[2] + mu * mu * sum_a, r2 = rstd * rstd;
+      const float s2 = __builtin_fmaf(m5, rstd, r2 * q3);
       const float p = -sc * lrc * rstd;
       const float c1 = p * rstd, c2 = -c1 * s2 * inv_d, c3 = -p * s1 * inv_d;
       const f32x4 gam = *reinterpret_cast<const f32x4*>(GAM + own);
       const f32x4 G = (z - mu) * (gam * gam * c1 + c2) + (bq * p + c3);
       GTc[w * 64 + lane] = IO::to_frag(G);
-      if (st > 0) qo = load4<T>(row((st + 2) % 3, 0) + own);
     } else if (outw && st > 0) {
-      output_moments(st - 1);
+      if (LATE) output_stats();
+      output_emit(st - 1, LATE ? 0 : 1, EPW);
     }
     // the next mini-batch's rows must have landed before anybody passes B3
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    if (older) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     lds_barrier();  // ---- B3
     RELANE();
 
@@ -602,7 +619,6 @@ __global__ void __launch_bounds__(512, D == 32 ? 4 : 2) ttt_mlp_fwd_rr_kernel(Pr
 #pragma unroll
       for (int j = 0; j < HT; ++j) IO::mma(zq[j], G1d[j], Mf);
     }
-    if (red && st > 0) output_emit(st - 1, qo);
 #pragma unroll
     for (int j = 0; j < HT; ++j) {
       f32x4 y;
@@ -623,6 +639,10 @@ __global__ void __launch_bounds__(512, D == 32 ? 4 : 2) ttt_mlp_fwd_rr_kernel(Pr
       PA[w * 64 + lane] = p;
     }
     partials(P2, xbf, true);
+    if (!LATE) {
+      lds_done();  // the blocks are in LDS before their counter says so
+      if (lane == 0) __hip_atomic_store(FL + w, st + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    }
     if (upd) {
       frag x2d[HT];
       {
@@ -667,17 +687,13 @@ __global__ void __launch_bounds__(512, D == 32 ? 4 : 2) ttt_mlp_fwd_rr_kernel(Pr
   }
 
   // ---- the last mini-batch's output
-  frag qo = IO::zero();
+  if (LATE) lds_barrier();
+  if (outs) output_finish(n_stages - 1);
   lds_barrier();
   if (outw) {
-    output_sum();
-    output_m2();
-    output_moments(n_stages - 1);
-  } else if (red) {
-    qo = load4<T>(row((a.n_stages - 1) % 3, 0) + own);
+    output_stats();
+    output_emit(n_stages - 1, 0, EPW);
   }
-  lds_barrier();
-  if (red) output_emit(a.n_stages - 1, qo);
 
   if (SAVE && a.state_save != nullptr) {
     f32x4* s1 = reinterpret_cast<f32x4*>(a.state_save + bh * (size_t)(2 * D * F)) + (w * NT * HT) * 64 + lane;
