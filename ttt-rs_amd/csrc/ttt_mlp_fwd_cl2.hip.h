@@ -155,7 +155,8 @@ __global__ void __launch_bounds__(64 * (D / 16)) ttt_mlp_fwd_cl2_kernel(Problems
   if (bh >= (size_t)a.B * a.H) return;
   int& lost = *reinterpret_cast<int*>(smem + L::LOST);  // set by a wave whose wait for the partner ran out
   if (tid == 0) lost = 0;
-  const int h = (int)(bh % a.H), K = a.K;
+  const int h = (int)(bh % a.H), K = a.K, spin_limit = held(a.spin_limit);
+  const float eps = held(a.eps);
   const int hoff = cu * FH;  // first hidden unit of this CU
 
   f32x4* const P1 = reinterpret_cast<f32x4*>(smem + L::P1);
@@ -280,7 +281,7 @@ __global__ void __launch_bounds__(64 * (D / 16)) ttt_mlp_fwd_cl2_kernel(Problems
     unsigned long long wd = 0;
     int it = 0;
     while ((unsigned)((wd = __hip_atomic_load(hello, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) >> 32) != 0xffffffffu) {
-      if (++it >= a.spin_limit) break;
+      if (++it >= spin_limit) break;
       __builtin_amdgcn_s_sleep(1);
     }
     partner_xcc = (unsigned)(wd >> 32) == 0xffffffffu ? (int)(wd & 15u) : -1;
@@ -310,7 +311,7 @@ __global__ void __launch_bounds__(64 * (D / 16)) ttt_mlp_fwd_cl2_kernel(Problems
     b = ((v[1][0] + v[1][1]) + (v[1][2] + v[1][3])) + ((v[3][0] + v[3][1]) + (v[3][2] + v[3][3]));
   };
   // tile slot `idx` of parity `par`: X1 tiles 0..NT-1, X2 tiles NT..2NT-1, the A2 tile 2NT
-  bool alive = a.spin_limit > 0;
+  bool alive = spin_limit > 0;
   auto send_tile = [&](int par_, int idx, f32x4 v, unsigned tag) {
     send_tagged(reinterpret_cast<unsigned long long*>(xout + par_ * L::XSLOT + idx * L::XTILE) + lane, v, tag, same_xcd);
   };
@@ -380,7 +381,7 @@ __global__ void __launch_bounds__(64 * (D / 16)) ttt_mlp_fwd_cl2_kernel(Problems
     float mu, ms;
     collect2(EXO, 0, 1, mu, ms);
     mu *= inv_d;
-    const float rstd = __builtin_amdgcn_rsqf(fmaxf(ms * inv_d - mu * mu, 0.f) + a.eps);
+    const float rstd = __builtin_amdgcn_rsqf(fmaxf(ms * inv_d - mu * mu, 0.f) + eps);
     if (c < K) {
       const f32x4 gam = *reinterpret_cast<const f32x4*>(GAM + own), bet = *reinterpret_cast<const f32x4*>(BET + own);
       elem* po = reinterpret_cast<elem*>(outp + (size_t)stage * step) + (c * D + own);
@@ -491,7 +492,7 @@ __global__ void __launch_bounds__(64 * (D / 16)) ttt_mlp_fwd_cl2_kernel(Problems
       Inbound in, in2;
       in.load(slot_in(par, w));
       if (m2w) in2.load(slot_in(par ^ 1, 2 * NT));
-      const f32x4 zpart = in.wait(slot_in(par, w), (unsigned)st + 1, alive, a.spin_limit);
+      const f32x4 zpart = in.wait(slot_in(par, w), (unsigned)st + 1, alive, spin_limit);
       z = b2T + (cu == 0 ? zloc + zpart : zpart + zloc);  // same order of the halves on both CUs
       float S[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
       const f32x4 az = gam * gam * z;
@@ -506,7 +507,7 @@ __global__ void __launch_bounds__(64 * (D / 16)) ttt_mlp_fwd_cl2_kernel(Problems
       }
       publish(S);
       if (cu == 0 && st > 0) {
-        if (m2w) output_m2(at + in2.wait(slot_in(par ^ 1, 2 * NT), (unsigned)st, alive, a.spin_limit));
+        if (m2w) output_m2(at + in2.wait(slot_in(par ^ 1, 2 * NT), (unsigned)st, alive, spin_limit));
         zb_in.load(slot_in(par ^ 1, NT + w));
       }
       fetch(st + 1);
@@ -538,7 +539,7 @@ __global__ void __launch_bounds__(64 * (D / 16)) ttt_mlp_fwd_cl2_kernel(Problems
       }
       const float mu = S[0] * inv_d;
       const float var = S[1] * inv_d - mu * mu;
-      const float rstd = __builtin_amdgcn_rsqf(fmaxf(var, 0.f) + a.eps);
+      const float rstd = __builtin_amdgcn_rsqf(fmaxf(var, 0.f) + eps);
       const float s1 = rstd * (S[2] - mu * sum_a) + S[4];
       const float s2 = rstd * rstd * (S[3] - 2.f * mu * S[2] + mu * mu * sum_a) + rstd * (S[5] - mu * S[4]);
       const float p = -sc * lrc * rstd;
@@ -594,7 +595,7 @@ __global__ void __launch_bounds__(64 * (D / 16)) ttt_mlp_fwd_cl2_kernel(Problems
       for (int j = 0; j < HT; ++j) IO::mma(zq[j], G1d[j], Mf);
     }
     if (cu == 0) {
-      if (st > 0) output_finish(st - 1, zb_in.wait(slot_in(par ^ 1, NT + w), (unsigned)st, alive, a.spin_limit));
+      if (st > 0) output_finish(st - 1, zb_in.wait(slot_in(par ^ 1, NT + w), (unsigned)st, alive, spin_limit));
       qo2 = qo1;
       qo1 = load4<T>(row(buf, 0) + own);
     }
@@ -669,14 +670,14 @@ __global__ void __launch_bounds__(64 * (D / 16)) ttt_mlp_fwd_cl2_kernel(Problems
     const unsigned long long* const sl = slot_in((n_stages - 1) & 1, 2 * NT);
     Inbound in;
     in.load(sl);
-    output_m2(at + in.wait(sl, (unsigned)n_stages, alive, a.spin_limit));
+    output_m2(at + in.wait(sl, (unsigned)n_stages, alive, spin_limit));
   }
   lds_barrier();
   if (cu == 0) {
     const unsigned long long* const sl = slot_in((n_stages - 1) & 1, NT + w);
     Inbound in;
     in.load(sl);
-    output_finish(n_stages - 1, in.wait(sl, (unsigned)n_stages, alive, a.spin_limit));
+    output_finish(n_stages - 1, in.wait(sl, (unsigned)n_stages, alive, spin_limit));
   }
   lds_barrier();
   if (cu == 0) output_emit(n_stages - 1);
