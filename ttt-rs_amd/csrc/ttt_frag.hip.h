@@ -76,6 +76,32 @@ __device__ __forceinline__ float xg_sum4_scatter(float a, float b, float c, floa
   return __uint_as_float(r0) + __uint_as_float(r1);            // rows: a, b, c, d
 }
 
+// Two values: lane groups 0 and 1 get the sum of a, 2 and 3 that of b (the same additions in the same order as above;
+// with zeros for c and d it would take a swap and an addition more).
+__device__ __forceinline__ float xg_sum2_scatter(float a, float b) {
+  const auto p = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  const uint32_t p0 = p[0], p1 = p[1];
+  const uint32_t ab = __float_as_uint(__uint_as_float(p0) + __uint_as_float(p1));
+  const auto q = __builtin_amdgcn_permlane16_swap(ab, ab, false, false);
+  const uint32_t q0 = q[0], q1 = q[1];
+  return __uint_as_float(q0) + __uint_as_float(q1);
+}
+// One term, or one product, of a sum that starts from its first one: from zero it would take an instruction more, and the
+// kernels of one or two waves per SIMD are bound by the number of instructions a wave issues.
+__device__ __forceinline__ void sum_term(float& s, bool first, float v) { s = first ? v : s + v; }
+__device__ __forceinline__ void sum_term(float& s, bool first, float x, float y) { s = first ? x * y : __builtin_fmaf(x, y, s); }
+// (the order in which the products are fused is written out: the forward kernels keep their bits)
+__device__ __forceinline__ float sum_squares(f32x4 z) {
+  return __builtin_fmaf(z[3], z[3], __builtin_fmaf(z[2], z[2], __builtin_fmaf(z[0], z[0], z[1] * z[1])));
+}
+template <int N>
+__device__ __forceinline__ f32x4 sum_tiles(const f32x4 (&v)[N]) {
+  f32x4 s = v[0];
+#pragma unroll
+  for (int i = 1; i < N; ++i) s += v[i];
+  return s;
+}
+
 // Sum over the 16 lanes of a row, in every lane: four rotations inside the row on the DPP path
 // (a shuffle goes through the LDS crossbar and costs an LDS round trip per step).
 __device__ __forceinline__ float row16_sum_dpp(float v) {

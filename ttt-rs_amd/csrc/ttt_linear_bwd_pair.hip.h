@@ -219,19 +219,20 @@ __global__ void __launch_bounds__(64 * (D / 16 + 1)) ttt_linear_bwd_pair_kernel(
 #pragma unroll
     for (int qq = 0; qq < NQ; ++qq) IO::mma2(acc, A[2 * qq], A[2 * qq + 1], B[2 * qq], B[2 * qq + 1]);
   };
-  auto xpub = [&](float* e, const float (&S)[8]) {
+  // four sums or six, each from its first term (96 units x 2048 tokens, f32: 427 -> 420 us)
+  auto xpub = [&](float* e, const auto& S) {
     const float v0 = xg_sum4_scatter(S[0], S[1], S[2], S[3]);
-    const float v1 = xg_sum4_scatter(S[4], S[5], S[6], S[7]);
     e[(g * 16 + c) * NW + w] = v0;
-    e[((g + 4) * 16 + c) * NW + w] = v1;
+    if constexpr (sizeof(S) > 4 * sizeof(float))  // six sums: two lane groups write the same value
+      e[((4 + (g >> 1)) * 16 + c) * NW + w] = xg_sum2_scatter(S[4], S[5]);
   };
-  auto xcol = [&](const float* e, float (&S)[8]) {
+  auto xcol = [&](const float* e, auto& S) {
     lds_barrier();
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      float s = 0.f;
+    for (int i = 0; i < (int)(sizeof(S) / sizeof(float)); ++i) {
+      float s = e[(i * 16 + c) * NW];
 #pragma unroll
-      for (int ww = 0; ww < NW; ++ww) s += e[(i * 16 + c) * NW + ww];
+      for (int ww = 1; ww < NW; ++ww) s += e[(i * 16 + c) * NW + ww];
       S[i] = s;
     }
   };
@@ -417,17 +418,17 @@ __global__ void __launch_bounds__(64 * (D / 16 + 1)) ttt_linear_bwd_pair_kernel(
       // ---- X1: raw moments of Z1
       const f32x4 tgt = bet - (vo - ko);
       const f32x4 bq = gam * tgt;
-      float S1[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+      float S1[6];
       {
         const f32x4 az = a2 * z1;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          S1[0] += z1[r];
-          S1[1] += z1[r] * z1[r];
-          S1[2] += az[r];
-          S1[3] += az[r] * z1[r];
-          S1[4] += bq[r];
-          S1[5] += bq[r] * z1[r];
+          sum_term(S1[0], r == 0, z1[r]);
+          sum_term(S1[1], r == 0, z1[r], z1[r]);
+          sum_term(S1[2], r == 0, az[r]);
+          sum_term(S1[3], r == 0, az[r], z1[r]);
+          sum_term(S1[4], r == 0, bq[r]);
+          sum_term(S1[5], r == 0, bq[r], z1[r]);
         }
       }
       xpub(SUMp, S1);
@@ -468,13 +469,13 @@ __global__ void __launch_bounds__(64 * (D / 16 + 1)) ttt_linear_bwd_pair_kernel(
       // ---- Zb = XQ W + b - M G ; X2: raw moments of Zb and of the output-LayerNorm backward
       IO::mma(zb, tokens_k(G), nM);
       const f32x4 gx2 = oo * gam;
-      float S2[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+      float S2[4];
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        S2[0] += zb[r];
-        S2[1] += zb[r] * zb[r];
-        S2[2] += gx2[r];
-        S2[3] += gx2[r] * zb[r];
+        sum_term(S2[0], r == 0, zb[r]);
+        sum_term(S2[1], r == 0, zb[r], zb[r]);
+        sum_term(S2[2], r == 0, gx2[r]);
+        sum_term(S2[3], r == 0, gx2[r], zb[r]);
       }
       xpub(SUMp + 8 * 16 * NW, S2);
       xcol(SUMp + 8 * 16 * NW, S2);
@@ -682,17 +683,17 @@ __global__ void __launch_bounds__(64 * (D / 16 + 1)) ttt_linear_bwd_pair_kernel(
     const f32x4 xh = own(L::XH), gx = own(L::GX), G = frk(L::GF, w);
     const float last = te_last * lr_c;
     const f32x4 u = (own(L::DGM) + last * S) * rstd1;  // u = -dG rstd1
-    float S4[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    float S4[6];
     {
       const f32x4 au = a2 * u;
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        S4[0] += u[r];
-        S4[1] += u[r] * xh[r];
-        S4[2] += au[r];
-        S4[3] += au[r] * xh[r];
-        S4[4] += u[r] * gx[r];
-        S4[5] += G[r] * S[r];
+        sum_term(S4[0], r == 0, u[r]);
+        sum_term(S4[1], r == 0, u[r], xh[r]);
+        sum_term(S4[2], r == 0, au[r]);
+        sum_term(S4[3], r == 0, au[r], xh[r]);
+        sum_term(S4[4], r == 0, u[r], gx[r]);
+        sum_term(S4[5], r == 0, G[r], S[r]);
       }
     }
     xpub(SUMp, S4);

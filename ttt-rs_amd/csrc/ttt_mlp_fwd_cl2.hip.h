@@ -295,10 +295,10 @@ __global__ void __launch_bounds__(64 * (D / 16)) ttt_mlp_fwd_cl2_kernel(Problems
 
   auto publish = [&](const float (&S)[6]) {
     const float v0 = xg_sum4_scatter(S[0], S[1], S[2], S[3]);
-    const float v1 = xg_sum4_scatter(S[4], S[5], 0.f, 0.f);
+    const float v1 = xg_sum2_scatter(S[4], S[5]);
     EX[(((g)*2 + (w >> 2)) * 16 + c) * 4 + (w & 3)] = v0;
-    if (g < 2) EX[(((g + 4) * 2 + (w >> 2)) * 16 + c) * 4 + (w & 3)] = v1;
-  };
+    EX[(((4 + (g >> 1)) * 2 + (w >> 2)) * 16 + c) * 4 + (w & 3)] = v1;  // two lane groups write the same value
+  };  // (with this and every sum from its first term, same bits: 128 units x 2048 tokens, d = 96 615 -> 608 us, d = 128 812 -> 807)
   // sums i and j of those exchanged at ex
   auto collect2 = [&](const float* ex, int i, int j, float& a, float& b) {
     f32x4 v[4];
@@ -329,13 +329,11 @@ __global__ void __launch_bounds__(64 * (D / 16)) ttt_mlp_fwd_cl2_kernel(Problems
   f32x4 zb = {0.f, 0.f, 0.f, 0.f};
   frag qo1 = IO::zero(), qo2 = qo1;  // xq tiles of the last mini-batch and of the one before
   auto a2_sum = [&]() -> f32x4 {
-    f32x4 v[NW], at = {0.f, 0.f, 0.f, 0.f};
+    f32x4 v[NW];
 #pragma unroll
     for (int ww = 0; ww < NW; ++ww) v[ww] = PA[ww * 64 + lane];
     together(v);
-#pragma unroll
-    for (int ww = 0; ww < NW; ++ww) at += v[ww];
-    return at;
+    return sum_tiles(v);
   };
   auto a2_early = [&](int stage) -> f32x4 {
     while (__builtin_amdgcn_ballot_w64(__hip_atomic_load(FL + (lane & 7), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) <= stage) != 0) {
@@ -350,9 +348,9 @@ __global__ void __launch_bounds__(64 * (D / 16)) ttt_mlp_fwd_cl2_kernel(Problems
     frag v[NW];
 #pragma unroll
     for (int ww = 0; ww < NW; ++ww) v[ww] = P2[(ww * NT + w) * 64 + lane];
-    zb = f32x4{0.f, 0.f, 0.f, 0.f};
+    zb = IO::to_f32(v[0]);
 #pragma unroll
-    for (int ww = 0; ww < NW; ++ww) zb += IO::to_f32(v[ww]);
+    for (int ww = 1; ww < NW; ++ww) zb += IO::to_f32(v[ww]);
     pin(zb);
     if (cu == 1) send_tile(par_, NT + w, zb, (unsigned)stage + 1);
   };
@@ -368,14 +366,10 @@ __global__ void __launch_bounds__(64 * (D / 16)) ttt_mlp_fwd_cl2_kernel(Problems
   auto output_finish = [&](int stage, f32x4 zb_part) {
     zb += zb_part;
     IO::mma(zb, read_tr(GT + ((stage & 1) * NT + w) * 64 + tr_lane(lane)), M2s[lane]);
-    float s0 = 0.f, s1 = 0.f;
+    float s0;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      s0 += zb[r];
-      s1 += zb[r] * zb[r];
-    }
-    const float v = xg_sum4_scatter(s0, s1, 0.f, 0.f);
-    if (g < 2) EXO[((g * 2 + (w >> 2)) * 16 + c) * 4 + (w & 3)] = v;
+    for (int r = 0; r < 4; ++r) sum_term(s0, r == 0, zb[r]);
+    EXO[(((g >> 1) * 2 + (w >> 2)) * 16 + c) * 4 + (w & 3)] = xg_sum2_scatter(s0, sum_squares(zb));
   };
   auto output_emit = [&](int stage) {
     float mu, ms;
@@ -471,14 +465,13 @@ __global__ void __launch_bounds__(64 * (D / 16)) ttt_mlp_fwd_cl2_kernel(Problems
     f32x4 z, bq;
     Inbound zb_in;
     {
-      f32x4 zloc = {0.f, 0.f, 0.f, 0.f};
+      f32x4 zloc;
       {
         f32x4 v[NW];
 #pragma unroll
         for (int ww = 0; ww < NW; ++ww) v[ww] = P1[(ww * NT + w) * 64 + lane];
         together(v);
-#pragma unroll
-        for (int ww = 0; ww < NW; ++ww) zloc += v[ww];
+        zloc = sum_tiles(v);
       }
       send_tile(par, w, zloc, (unsigned)st + 1);
       // everything that does not need the partner goes between the send and the wait: the local half of the previous
@@ -487,23 +480,24 @@ __global__ void __launch_bounds__(64 * (D / 16)) ttt_mlp_fwd_cl2_kernel(Problems
       if (st > 0) output_local(st - 1);
       const frag ko = load4<T>(row(buf, 1) + own), vo = load4<T>(row(buf, 2) + own);
       const f32x4 gam = *reinterpret_cast<const f32x4*>(GAM + own), bet = *reinterpret_cast<const f32x4*>(BET + own);
-      bq = gam * (bet - (IO::to_f32(vo) - IO::to_f32(ko)));
+      const f32x4 tgt = bet - (IO::to_f32(vo) - IO::to_f32(ko));
+      bq = gam * tgt;
       const bool m2w = cu == 0 && w == 2 && st > 0;  // CU 1 sent its A2 before its Z2 tiles
       Inbound in, in2;
       in.load(slot_in(par, w));
       if (m2w) in2.load(slot_in(par ^ 1, 2 * NT));
       const f32x4 zpart = in.wait(slot_in(par, w), (unsigned)st + 1, alive, spin_limit);
       z = b2T + (cu == 0 ? zloc + zpart : zpart + zloc);  // same order of the halves on both CUs
-      float S[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-      const f32x4 az = gam * gam * z;
+      float S[6];
+      const f32x4 a2 = gam * gam, az = a2 * z;
+      S[1] = sum_squares(z);
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        S[0] += z[r];
-        S[1] += z[r] * z[r];
-        S[2] += az[r];
-        S[3] += az[r] * z[r];
-        S[4] += bq[r];
-        S[5] += bq[r] * z[r];
+        sum_term(S[0], r == 0, z[r]);
+        sum_term(S[2], r == 0, a2[r], z[r]);
+        sum_term(S[3], r == 0, az[r], z[r]);
+        sum_term(S[4], r == 0, gam[r], tgt[r]);
+        sum_term(S[5], r == 0, bq[r], z[r]);
       }
       publish(S);
       if (cu == 0 && st > 0) {
@@ -541,7 +535,8 @@ __global__ void __launch_bounds__(64 * (D / 16)) ttt_mlp_fwd_cl2_kernel(Problems
       const float var = S[1] * inv_d - mu * mu;
       const float rstd = __builtin_amdgcn_rsqf(fmaxf(var, 0.f) + eps);
       const float s1 = rstd * (S[2] - mu * sum_a) + S[4];
-      const float s2 = rstd * rstd * (S[3] - 2.f * mu * S[2] + mu * mu * sum_a) + rstd * (S[5] - mu * S[4]);
+      const float m5 = S[5] - mu * S[4], q3 = S[3] - 2.f * mu * S[2] + mu * mu * sum_a, r2 = rstd * rstd;
+      const float s2 = __builtin_fmaf(m5, rstd, r2 * q3);
       const float p = -sc * lrc * rstd;
       const float c1 = p * rstd, c2 = -c1 * s2 * inv_d, c3 = -p * s1 * inv_d;
       const f32x4 gam = *reinterpret_cast<const f32x4*>(GAM + own);
