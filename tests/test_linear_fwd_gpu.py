@@ -170,6 +170,23 @@ def test_sequence_windows_in_place(P, d):
     assert torch.isnan(out_full[:, :, :lo]).all() and torch.isnan(out_full[:, :, hi:]).all()
 
 
+@pytest.mark.parametrize("N", [1, 2, 3, 4, 7])
+@pytest.mark.parametrize("d", [32, 64])
+def test_f32_forward_with_control_wave_without_checkpoints(P, d, N):
+    """The control-wave kernel has a variant without the code for checkpoints: the same bits as the one that writes them
+    (same arithmetic in the same order), at lengths around its ring of three mini-batches."""
+    print(f"case f32 fwd control wave, no checkpoints d{d} N{N}", flush=True)
+    K = 16
+    dv = to_dev(P.synthetic.reference_test_inputs(17 + d + N, 2, 3, N * K, d, K))
+
+    def run(ckpt):
+        return P.ttt_linear_forward_raw(dv["xq"], dv["xk"], dv["xv"], dv["W0"], dv["b0"], dv["token_eta"], dv["lr"],
+                                        dv["gamma"], dv["beta"], K, 1e-6, 1, want_checkpoints=ckpt)
+
+    for name, x, y in zip(("out", "W", "b"), run(False), run(True)):
+        assert torch.equal(x, y), name
+
+
 @pytest.mark.parametrize("fmt", [0, 1], ids=["rowmajor", "packed"])
 @pytest.mark.parametrize("B,H,d,N", [(1, 4, 64, 16), (3, 2, 64, 5), (2, 3, 32, 3), (1, 1, 64, 1), (2, 2, 32, 2), (1, 2, 64, 9)])
 def test_f32_forward_with_control_wave_equals_forward_with_own_loads(P, B, H, d, N, fmt):

@@ -129,7 +129,9 @@ int device_cus(int* cus);
 
 // ctl_wave: f32 I/O, one feature tile per wave, whole mini-batches, a CU per workgroup: the variant with a control
 // wave that copies the operands global -> LDS, so that the compute waves issue no loads (same bits; config-2 forward
-// 246 -> 216 us, with packed checkpoints 278 -> 250 us)
+// 246 -> 216 us, with packed checkpoints 278 -> 250 us).  A launch in which no problem asks for checkpoints has no code for
+// them: the test and the cursor are instructions of every mini-batch (96 units x 2048 tokens 211.1 -> 207.2 us, d = 32
+// 151.1 -> 146.7 us, same bits).
 template <class T, int D, int NW>
 int launch_linear_fwd_nw(const ttt::LinearFwdArgs* probs, unsigned ny, hipStream_t s, bool own_loads = false,
                          bool ctl_wave = false) {
@@ -138,7 +140,13 @@ int launch_linear_fwd_nw(const ttt::LinearFwdArgs* probs, unsigned ny, hipStream
   const auto P = pack_of(probs, ny);
   if constexpr (sizeof(typename ttt::Io<T>::elem) == 4 && NW == D / 16 && NW > 1) {
     if (ctl_wave && a.K == 16 && !sums) {
-      hipLaunchKernelGGL((ttt::ttt_linear_fwd_dma_kernel<T, D, NW, 2>), dim3((unsigned)(a.B * a.H), ny), dim3(64 * (NW + 1)), 0, s, P);
+      const dim3 grid((unsigned)(a.B * a.H), ny), block(64 * (NW + 1));
+      bool ckpt = false;
+      for (unsigned y = 0; y < ny; ++y) ckpt = ckpt || probs[y].W_ckpt != nullptr;
+      if (ckpt)
+        hipLaunchKernelGGL((ttt::ttt_linear_fwd_dma_kernel<T, D, NW, 2, true>), grid, block, 0, s, P);
+      else
+        hipLaunchKernelGGL((ttt::ttt_linear_fwd_dma_kernel<T, D, NW, 2, false>), grid, block, 0, s, P);
       return hip_status(hipGetLastError(), "ttt_linear_fwd launch");
     }
   }

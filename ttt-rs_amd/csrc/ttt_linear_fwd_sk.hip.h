@@ -53,7 +53,7 @@ namespace ttt {
 // STATES: only the recurrence runs, from a given state, and the state entering every one of n_stages + 1 mini-batches is
 // written as a checkpoint: no output, no attention block, no final state (see ttt_linear_states_kernel).  The unit and the
 // index of its initial state are then given (unit, state) instead of following from the workgroup's index.
-template <class T, int D, int NW, int PF, bool FULL, bool FAC, int RAW, bool ADAM = false, bool STATES = false, bool COMPACT = false>
+template <class T, int D, int NW, int PF, bool FULL, bool FAC, int RAW, bool ADAM = false, bool STATES = false, bool COMPACT = false, bool CKPT = !ADAM>
 __device__ __forceinline__ void linear_fwd_sk_body(const LinearFwdArgs& a, const FusedInputsArgs* fip,
                                                    const AdamArgs* adam = nullptr, size_t unit = 0, size_t state = 0) {
   static_assert(!ADAM || (D <= 64 && !FAC && (RAW == 0 || RAW == 3 || RAW == 5)), "Adam inner optimiser: head_dim <= 64, operands given, no checkpoints");
@@ -654,7 +654,7 @@ __device__ __forceinline__ void linear_fwd_sk_body(const LinearFwdArgs& a, const
       }
       // ---- checkpoint of the state entering this mini-batch (W and b change only behind the barrier);
       // placed at the barrier so that its branch does not cut the stretch in two
-      if (!ADAM && ck.due()) {
+      if (CKPT && ck.due()) {
         if (ck.packed) {
           store_ckpt_packed<T, NT, TPW>(ck.W, Wc, w, lane);
           store_bias_true<D, TPW>(ck.b, bT, b_mean, w, c, g);
@@ -663,7 +663,9 @@ __device__ __forceinline__ void linear_fwd_sk_body(const LinearFwdArgs& a, const
         }
         ck.advance();
       }
-      if constexpr (!ADAM) ck.next_stage();
+      if constexpr (CKPT) ck.next_stage();
+      // (without checkpoints the stretch is cut here all the same: as one, 208.5 us instead of 206)
+      if constexpr (!CKPT && !ADAM) __builtin_amdgcn_sched_barrier(0);
       // The compiler does not count the wait states between a matrix instruction and a read of its result behind a branch,
       // and so few instructions are left in between that the read comes too early (isa_check.py).
       if constexpr (BF && !ADAM) {
@@ -974,9 +976,9 @@ __global__ void __launch_bounds__(64 * NW) ttt_linear_fwd_sk_kernel(Problems<Lin
 }
 
 // The forward with a control wave that brings the operands in: see RAW = 5 above.
-template <class T, int D, int NW, int PF>
+template <class T, int D, int NW, int PF, bool CKPT>
 __global__ void __launch_bounds__(64 * (NW + 1)) ttt_linear_fwd_dma_kernel(Problems<LinearFwdArgs> problems) {
-  linear_fwd_sk_body<T, D, NW, PF, true, false, 5>(problems.p[blockIdx.y], nullptr);
+  linear_fwd_sk_body<T, D, NW, PF, true, false, 5, false, false, false, CKPT>(problems.p[blockIdx.y], nullptr);
 }
 
 // TTT-Linear with the Adam inner optimiser: see ADAM above.  Bound by the chain of a mini-batch, and in it by the issue
