@@ -116,7 +116,7 @@ typedef struct ttt_desc {
 #define TTT_HINT_F32_PRODUCTS 0x4000
 /* ttt_mlp_bwd and its variants: with at most 128 (batch, head) units every unit is worked on by two workgroups on two
  * CUs (see ttt_mlp_bwd); TTT_HINT_ONE_WORKGROUP keeps a unit on one.  Same results bit for bit (d_token_eta, which
- * is summed over the units with atomic additions, aside); the workspace is smaller. */
+ * is summed over the units with atomic additions, aside); the workspace is smaller.  ttt_mlpn_fwd: likewise. */
 #define TTT_HINT_ONE_WORKGROUP 0x8000
 /* Testing only: the two workgroups that share a (batch, head) unit in ttt_mlp_fwd at head_dim 128 (bf16 I/O) give
  * up waiting for each other at once, as if the partner had never become resident.  Exercises the failure path
@@ -494,6 +494,11 @@ int ttt_linear_fwd_fused_inputs(const ttt_desc* desc, const void* xq, const void
  * Products are f32 for both I/O types.  head_dim 32 with 2 - 4 hidden layers, head_dim 64 with 2 (what fits the
  * LDS of a CU); ttt_mlpn_supported says so beforehand.  One hidden layer is ttt_mlp_fwd.  desc.seq_stride is
  * honoured (a window of a longer sequence in place).
+ * With at most half as many (batch, head) units as the device has CUs (in groups of eight) and four mini-batches or more, a unit
+ * is worked on by two workgroups on two CUs, where W_out is 16-byte aligned and overlaps no other argument: the same results
+ * bit for bit; TTT_HINT_ONE_WORKGROUP keeps it on one.  They wait for each other, a bounded time; a unit whose workgroups were
+ * never resident together has NaN in out, in W_out of the last layer and in every b_out, and is counted by
+ * ttt_mlp_fwd_lost_workgroups.
  */
 int ttt_mlpn_supported(const ttt_desc* desc, int n_hidden);
 int ttt_mlpn_fwd(const ttt_desc* desc, int n_hidden, const void* xq, const void* xk, const void* xv,

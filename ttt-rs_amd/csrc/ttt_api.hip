@@ -1006,6 +1006,54 @@ int ttt_linear_fwd(const ttt_desc* d, const void* xq, const void* xk, const void
   return dispatch_linear_fwd(d, &a, 1, static_cast<hipStream_t>(stream));
 }
 
+}  // extern "C"
+
+namespace {
+// Whether a unit of ttt_mlpn_fwd runs on two workgroups (see ttt_mlpn_fwd.hip.h), and what that form needs besides.  Both of
+// a unit's workgroups must be resident together and each fills a CU, so there may be half as many units as CUs, in groups of
+// eight.  The words are cleared by a launch of their own and the last mini-batch's output follows its state: 96 units, bf16, us on
+// one / two workgroups at 2, 4, 8 mini-batches: head_dim 64 82 / 90, 145 / 136, 273 / 229, head_dim 32 27 / 30, 49 / 47,
+// 91 / 78.  What crosses lies in the W_out buffers, 16 bytes to a lane, while
+// either side still reads its inputs: a caller's buffers that are not aligned so, or overlap an input, stay with one workgroup.
+int mlpn_on_pairs(const ttt_desc* d, int n_hidden, ttt::MlpNFwdArgs& a, bool* yes) {
+  *yes = false;
+  if (d->kernel_hint & TTT_HINT_ONE_WORKGROUP) return TTT_OK;
+  const size_t units = (size_t)a.B * a.H;
+  if (a.n_stages < 4) return TTT_OK;
+  int cus = 0;
+  int rc = device_cus(&cus);
+  if (rc != TTT_OK) return rc;
+  if ((units + 7) / 8 * 16 > (size_t)cus) return TTT_OK;
+  const size_t D = (size_t)d->head_dim, M = 4 * D, io = d->io_dtype == TTT_F32 ? 4 : 2;
+  const size_t tokens = (units - 1) * a.seq_stride + d->seq, states = d->state_per_batch ? units : (size_t)a.H;
+  const auto apart = [](const void* p, size_t n, const void* q, size_t m) {
+    const uintptr_t x = (uintptr_t)p, y = (uintptr_t)q;
+    return x + n <= y || y + m <= x;
+  };
+  for (int i = 0; i <= n_hidden; ++i) {
+    const size_t n = units * (i == 0 ? D : M) * (i == n_hidden ? D : M) * 4;
+    if (!aligned16(a.W[i])) return TTT_OK;
+    bool ok = apart(a.W[i], n, a.token_eta, 4 * a.K) && apart(a.W[i], n, a.gamma, 4 * a.H * D) &&
+              apart(a.W[i], n, a.beta, 4 * a.H * D) && apart(a.W[i], n, a.lr, tokens * io);
+    for (const void* x : {a.xq, a.xk, a.xv, (const void*)a.out}) ok = ok && apart(a.W[i], n, x, tokens * D * io);
+    for (int j = 0; j <= n_hidden; ++j) {
+      const size_t out = j == n_hidden ? D : M;
+      ok = ok && apart(a.W[i], n, a.W0[j], states * (j == 0 ? D : M) * out * 4) && apart(a.W[i], n, a.b0[j], states * out * 4) &&
+           apart(a.W[i], n, a.b[j], units * out * 4);
+    }
+    if (!ok) return TTT_OK;
+  }
+  rc = lost_word(&a.lost_count);
+  if (rc != TTT_OK) return rc;
+  a.spin_limit = (d->kernel_hint & TTT_HINT_TEST_LOST_PARTNER) ? 0u : 1u << 21;
+  a.agent_release = (d->kernel_hint & TTT_HINT_TEST_OTHER_XCD) ? 1 : 0;
+  *yes = true;
+  return TTT_OK;
+}
+}  // namespace
+
+extern "C" {
+
 int ttt_mlpn_supported(const ttt_desc* d, int n_hidden) {
   int rc = check_common(d);
   if (rc != TTT_OK) return rc;
@@ -1026,7 +1074,7 @@ int ttt_mlpn_fwd(const ttt_desc* d, int n_hidden, const void* xq, const void* xk
   if (rc != TTT_OK) return rc;
   if (!xq || !xk || !xv || !W0 || !b0 || !token_eta || !lr || !gamma || !beta || !out || !W_out || !b_out)
     return fail(TTT_ERR_NULL, "ttt_mlpn_fwd: a required pointer is NULL");
-  ttt::MlpNFwdArgs a;
+  ttt::MlpNFwdArgs a{};
   for (int i = 0; i < ttt::kMlpNMaxLayers; ++i) {
     a.W0[i] = a.b0[i] = nullptr;
     a.W[i] = a.b[i] = nullptr;
@@ -1043,8 +1091,11 @@ int ttt_mlpn_fwd(const ttt_desc* d, int n_hidden, const void* xq, const void* xk
   a.seq_stride = d->seq_stride > 0 ? d->seq_stride : d->seq;
   a.state_per_batch = d->state_per_batch ? 1 : 0;
   a.eps = d->eps;
+  bool pair = false;
+  rc = mlpn_on_pairs(d, n_hidden, a, &pair);
+  if (rc != TTT_OK) return rc;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  return hip_status(ttt::launch_mlpn_fwd(d->io_dtype == TTT_F32, d->head_dim, n_hidden, a, s), "ttt_mlpn_fwd launch");
+  return hip_status(ttt::launch_mlpn_fwd(d->io_dtype == TTT_F32, d->head_dim, n_hidden, pair, a, s), "ttt_mlpn_fwd launch");
 }
 
 }  // extern "C"

@@ -27,6 +27,19 @@
 // products.  96 units of 64 mini-batches, bf16: 3128 us with the state read from the L2 for every product and update,
 // 2062 so.  All products are f32 for both I/O types.  LDS bounds the shapes: head_dim 32 with up to four hidden layers,
 // head_dim 64 with two.
+//
+// A unit on two workgroups (ttt_mlpn_fwd_pair_kernel), where the device has two CUs for each.  Nothing of the output chain is
+// needed for the state, so one workgroup, the producer, runs the forward chain, the gradients and the updates; the other, the
+// consumer, takes X[i] and G[i] from it, runs the output chain and the same updates on a state of its own (542 and 424
+// matrix instructions per wave and mini-batch).  Nothing flows back, so neither waits for a round trip of the other: the
+// producer runs up to SLOTS mini-batches ahead.  Wave w hands over to wave w in the layout of its registers, through a ring in
+// the unit's W_out (MlpNPair); two words per pair of waves say how far each has come.  The producer's stores stay in the L2 that
+// both share (each publishes its XCD number) or are written back by a device-scope release while that is not known; the
+// consumer loads at device scope.  Every wait is bounded: a side that waits in vain marks its words, both run to their end
+// without waiting, the consumer makes out, W[NL] and every b of the unit NaN, and a status word counts both.
+// The arithmetic is that of one workgroup, bit for bit.  64 mini-batches of 16 tokens, bf16, us on one / on two workgroups:
+// head_dim 64, 12 units 2060 / 1502, 96 units 2080 / 1529, 128 units 2081 / 1570; head_dim 32, 96 units two hidden layers
+// 699 / 519, 48 units three 1057 / 778, 24 units four 1414 / 1040.
 #pragma once
 #include "ttt_engine_fwd.hip.h"
 
@@ -49,6 +62,10 @@ struct MlpNFwdArgs {
   void* out;
   int B, H, seq, seq_stride, K, n_stages, state_per_batch;  // seq_stride: tokens between consecutive (b, h) units
   float eps;
+  // a unit on two workgroups
+  unsigned spin_limit;   // polls before a wait for the partner gives up; 0: give up at once (tests of that path)
+  int agent_release;     // 1: always publish with a device-scope release
+  unsigned* lost_count;  // counts workgroups that waited in vain
 };
 
 template <int D, int NL>
@@ -72,6 +89,23 @@ struct MlpNLds {
   static_assert(BYTES <= 160 * 1024, "exceeds the 160 KiB of LDS of a gfx950 CU");
 };
 
+// What crosses between the two workgroups of a unit lies in its W_out until the consumer stores the final state over it: a
+// ring of SLOTS mini-batches of X[1 .. NL] and G[0 .. NL-1] (W[1], W[2]), the same of G[NL], and the progress words.  W[0] and
+// W[NL] are taken at head_dim 64, where W[0] waits in memory on either side.
+template <int D, int NL>
+struct MlpNPair {
+  using L = MlpNLds<D, NL>;
+  static constexpr bool STREAM = D == 64;
+  static constexpr int SLOTS = STREAM ? 3 : 2, NJD = D / 32;
+  static constexpr int PIECE = 512 * 4 * 2 * L::NBM, PP = L::M * L::M / PIECE;  // floats of a layer's X and G; pieces to a W[i]
+  static constexpr int GR = STREAM ? (SLOTS * NL) * PIECE : 0, GSLOT = 512 * NJD;  // G[NL], in W[1] or W[0]
+  static constexpr int FL = GR + SLOTS * GSLOT, FL_WORDS = 64;
+  static_assert(SLOTS * NL <= (NL == 2 ? 1 : 2) * PP && FL + FL_WORDS <= (STREAM ? L::M : D) * L::M, "the hand-over must fit");
+  // words: progress of the producer's waves, its XCD; the same of the consumer
+  enum { COUNT = 0, XCD = 8, SIDE = 32 };
+};
+constexpr unsigned kMlpNPoison = 0xffffffffu;
+
 // acc += A B over 16 k: k step r takes the four k with index 4 g + r
 __device__ __forceinline__ void mlpn_mma(f32x4& acc, f32x4 a, f32x4 b) {
 #pragma unroll
@@ -88,20 +122,31 @@ __device__ __forceinline__ void mlpn_wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-template <class T, int D, int NL>
-__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) ttt_mlpn_fwd_kernel(MlpNFwdArgs a) {
+// a wave's own piece of the ring, stored by another CU: two device-scope loads, which do not look in the CU's vector cache
+__device__ __forceinline__ f32x4 mlpn_ld4_dev(const float* p) {
+  const unsigned long long* q = reinterpret_cast<const unsigned long long*>(p);
+  const unsigned long long u = __hip_atomic_load(q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  const unsigned long long v = __hip_atomic_load(q + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  return f32x4{__uint_as_float((unsigned)u), __uint_as_float((unsigned)(u >> 32)), __uint_as_float((unsigned)v),
+               __uint_as_float((unsigned)(v >> 32))};
+}
+
+// ROLE 0: the whole unit.  1: the producer of a unit on two workgroups, 2: its consumer.
+template <class T, int D, int NL, int ROLE>
+__device__ __forceinline__ void mlpn_fwd_body(const MlpNFwdArgs& a, const size_t bh) {
   using IO = Io<T>;
   using elem = typename IO::elem;
   using L = MlpNLds<D, NL>;
+  using P = MlpNPair<D, NL>;
   constexpr int M = L::M, LD = L::LD, LM = L::LM, TM = L::TM, NW = L::NW;
   constexpr int GW = 32, NJD = D / GW, NTD = L::NTD, NTM = L::NTM, NBM = L::NBM;
   constexpr int CH = L::CH, NCH = NTM / CH, SPLIT = NW / CH;
   constexpr bool STREAM = D == 64;  // W[0] waits in the output buffer while the other products run
+  constexpr int W0S = ROLE == 2 ? NL : 0;  // (the consumer's copy in that of W[NL], of the same size)
   static_assert(NTM % NW == 0 && NTM % CH == 0 && NW % CH == 0 && (SPLIT > 1 || NBM == 1), "tiles must divide among the waves");
   extern __shared__ __attribute__((aligned(16))) float lds[];
   int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   int t = tid >> 5, cg = tid & 31, c = lane & 15, g = lane >> 4;
-  const size_t bh = blockIdx.x;
   const int h = (int)(bh % a.H), K = a.K;
   float *sbl = lds + L::bl, *sgam = lds + L::gam, *sbet = lds + L::bet, *slr = lds + L::lr, *ste = lds + L::te;
   const size_t sbase = a.state_per_batch ? bh : (size_t)h;
@@ -128,7 +173,7 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))
 #pragma unroll
     for (int q = 0; q < NTD; ++q) {
       w0[q][j] = load_tile(a.W0[0] + sbase * D * M, M, q, j, oc);
-      if (STREAM) store_tile(a.W[0] + bh * D * M, M, q, j, oc, w0[q][j]);
+      if (STREAM) store_tile(a.W[W0S] + bh * D * M, M, q, j, oc, w0[q][j]);
     }
 #pragma unroll
     for (int i = 1; i < NL; ++i)
@@ -148,6 +193,54 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))
   __syncthreads();
   const float te_last = ste[K - 1];
 
+  // ---- the partner: wave w hands over to wave w, in the layout of the registers, so the only barriers are those of the products
+  float* const gring = STREAM ? a.W[1] + bh * M * M + P::GR : a.W[0] + bh * D * M + P::GR;
+  unsigned* const fl = reinterpret_cast<unsigned*>(gring + P::SLOTS * P::GSLOT);
+  unsigned* const mine = fl + (ROLE == 2 ? P::SIDE : 0);
+  unsigned* const theirs = fl + (ROLE == 2 ? 0 : P::SIDE);
+  unsigned known = 0, my_xcd = 0;
+  bool lost = false, fast = false;  // fast: the partner is known to sit behind the same L2
+  if constexpr (ROLE != 0) {
+    asm volatile("s_getreg_b32 %0, hwreg(HW_REG_XCC_ID)" : "=s"(my_xcd));
+    my_xcd = 0x100u | (my_xcd & 15u);
+    lost = a.spin_limit == 0;
+    if (tid == 0) __hip_atomic_store(mine + P::XCD, my_xcd, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  auto look = [&](const unsigned* p) {
+    return (unsigned)__builtin_amdgcn_readfirstlane((int)__hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+  };
+  auto wait_partner = [&](unsigned want) {  // until the partner's wave has come so far
+    if (lost || known >= want) return;
+    for (unsigned n = 0; ; ++n) {
+      const unsigned v = look(theirs + P::COUNT + (threadIdx.x >> 6));
+      if (v == kMlpNPoison || n >= a.spin_limit) {
+        lost = true;
+        return;
+      }
+      if (v >= want) {
+        known = v;
+        return;
+      }
+      __builtin_amdgcn_s_sleep(2);
+    }
+  };
+  auto publish = [&](unsigned count) {  // every store of this wave has been acknowledged, or written back
+    if (ROLE == 1 && !fast && a.agent_release == 0) fast = look(theirs + P::XCD) == my_xcd;
+    if (ROLE == 1 && !fast) __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    if ((threadIdx.x & 63) == 0)
+      __hip_atomic_store(mine + P::COUNT + (threadIdx.x >> 6), lost ? kMlpNPoison : count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  };
+  int slot = 0;
+  auto hand = [&](int i, int kind, int j) {  // X[i+1] (kind 0) or G[i] (1), tile j of the own columns
+    const int p = slot * NL + i;
+    float* base = NL > 2 && p >= P::PP ? a.W[NL > 2 ? 2 : 1] + bh * M * M + (p - P::PP) * P::PIECE : a.W[1] + bh * M * M + p * P::PIECE;
+    return base + (unsigned)(4 * ((kind * NBM + j) * 512 + tid));
+  };
+
+  // Where the staged rows wait: what the role does not use otherwise, or X[1]
+  constexpr int SQ = ROLE == 2 ? L::GT : L::XI, SK = ROLE == 1 ? L::XQ : SQ + L::TD;
+  constexpr int ST = ROLE == 1 ? L::ZBL : SQ + 2 * L::TD, SL = ROLE == 1 ? L::PART : SQ + 3 * L::TD;
   // The next mini-batch's xq/xk/xv/lr are fetched into registers while the last W[i] is updated, wait where X[1] lay while
   // W[0] is in registers, and go to their places when the mini-batch begins.  All by the thread that fetched them.
   elem pq[NJD], pk[NJD], pv[NJD], plr;
@@ -162,22 +255,22 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))
     const unsigned o = ((x >> 5) < K ? x >> 5 : 0) * D + (x & 31);
 #pragma unroll
     for (int j = 0; j < NJD; ++j) {
-      pq[j] = xq[o + GW * j];
+      if (ROLE != 1) pq[j] = xq[o + GW * j];
       pk[j] = xk[o + GW * j];
-      pv[j] = xv[o + GW * j];
+      if (ROLE != 2) pv[j] = xv[o + GW * j];
     }
     plr = lr[(unsigned)((x & 15) < K ? x & 15 : 0)];
   };
   auto stage_rows = [&]() {
-    float* S = lds + L::XI + t * LD + cg;
+    float* S = lds + SQ + t * LD + cg;
 #pragma unroll
     for (int j = 0; j < NJD; ++j) {
       const float k = IO::load1(pk + j);
-      S[GW * j] = t < K ? IO::load1(pq + j) : 0.f;
-      S[L::TD + GW * j] = t < K ? k : 0.f;
-      S[2 * L::TD + GW * j] = t < K ? IO::load1(pv + j) - k : 0.f;
+      if (ROLE != 1) S[GW * j] = t < K ? IO::load1(pq + j) : 0.f;
+      S[SK - SQ + GW * j] = t < K ? k : 0.f;
+      if (ROLE != 2) S[ST - SQ + GW * j] = t < K ? IO::load1(pv + j) - k : 0.f;
     }
-    if (tid < 16) lds[L::XI + 3 * L::TD + tid] = tid < K ? IO::load1(&plr) : 0.f;
+    if (tid < 16) lds[SL + tid] = tid < K ? IO::load1(&plr) : 0.f;
   };
   static_assert(3 * L::TD + 16 <= TM, "the staged rows take the place of X[1]");
   fetch(0);
@@ -194,11 +287,11 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))
 #pragma unroll
     for (int j = 0; j < NJD; ++j) {
       const int o = t * LD + cg + GW * j;
-      lds[L::XQ + o] = lds[L::XI + o];
-      lds[L::XK + o] = lds[L::XI + L::TD + o];
-      lds[L::TG + o] = lds[L::XI + 2 * L::TD + o];
+      if (ROLE != 1) lds[L::XQ + o] = lds[SQ + o];
+      lds[L::XK + o] = lds[SK + o];
+      if (ROLE != 2) lds[L::TG + o] = lds[ST + o];
     }
-    if (tid < 16) slr[tid] = lds[L::XI + 3 * L::TD + tid];
+    if (tid < 16) slr[tid] = lds[SL + tid];
     __syncthreads();
 
     // ---- forward chain: Z[i] = X[i] W[i]; X[i+1] = gelu(Z[i] + b[i]); gelu' stays in registers.  XQ W[0] rides along.
@@ -207,14 +300,18 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))
     auto hidden = [&](int i, const f32x4 (&z)[NBM]) {
       float* X = lds + L::XI + i * TM + own;
 #pragma unroll
-      for (int j = 0; j < NBM; ++j)
+      for (int j = 0; j < NBM; ++j) {
+        f32x4 x;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           float y, dy;
           gelu_tanh_pair(z[j][r] + bias[i][j], y, dy);
           X[um + r * LM + 16 * j] = y;
+          if constexpr (ROLE == 1) x[r] = y;
           G[i][j][r] = dy;
         }
+        if constexpr (ROLE == 1) mlpn_st4(hand(i, 0, j), x);
+      }
     };
     // X W over k = M, the operand read one tile ahead (the compiler, short of registers, would wait for each read)
     auto product = [&](f32x4 (&z)[NBM], const float* X, const f32x4 (&W)[NTM][NBM]) {
@@ -231,15 +328,29 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))
         fx = nx;
       }
     };
-    {
-      f32x4 z[NBM], at = {0.f, 0.f, 0.f, 0.f};
+    if (ROLE == 1 && st >= P::SLOTS) wait_partner((unsigned)(st - P::SLOTS + 1));  // the slot is free
+    if constexpr (ROLE == 1) {
+      f32x4 z[NBM];
 #pragma unroll
-      for (int j = 0; j < NBM; ++j) z[j] = zq[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int j = 0; j < NBM; ++j) z[j] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int q = 0; q < NTD; ++q) {
         const f32x4 fk = mlpn_ld4(lds + L::XK + ad + 16 * q);
 #pragma unroll
         for (int j = 0; j < NBM; ++j) mlpn_mma(z[j], fk, w0[q][j]);
+      }
+      hidden(0, z);
+    } else {
+      f32x4 z[NBM], at = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int j = 0; j < NBM; ++j) z[j] = zq[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+      if (ROLE == 0) {
+#pragma unroll
+      for (int q = 0; q < NTD; ++q) {
+        const f32x4 fk = mlpn_ld4(lds + L::XK + ad + 16 * q);
+#pragma unroll
+        for (int j = 0; j < NBM; ++j) mlpn_mma(z[j], fk, w0[q][j]);
+      }
       }
       // the attention block XQ XK^T: the waves share its k steps
 #pragma unroll
@@ -255,6 +366,7 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))
 #pragma unroll
       for (int e = 0; e < 4 * NBM; ++e) {
         if (e < NTD * NBM) mlpn_mma(zq[e % NBM], mlpn_ld4(lds + L::XQ + ad + 16 * (e / NBM)), w0[e / NBM][e % NBM]);
+        if (ROLE == 2) continue;
         float y, dy;
         gelu_tanh_pair(z[e >> 2][e & 3] + bias[0][e >> 2], y, dy);
         X[um + (e & 3) * LM + 16 * (e >> 2)] = y;
@@ -262,15 +374,49 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))
         __builtin_amdgcn_sched_barrier(0);
       }
     }
-    __syncthreads();
+    if constexpr (ROLE == 2) {
+      // what the producer has made of this mini-batch
+      wait_partner((unsigned)(st + 1));
+      if (!fast) {
+        if (a.agent_release == 0) fast = look(theirs + P::XCD) == my_xcd;
+        if (!fast) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+      }
+      f32x4 x[NL][NBM];
+      unsigned long long gv = 0;
 #pragma unroll
-    for (int i = 1; i < NL; ++i) {
-      f32x4 z[NBM];
-      product(z, lds + L::XI + (i - 1) * TM, w[i - 1]);
-      hidden(i, z);
-      if (i + 1 < NL) __syncthreads();
+      for (int i = 0; i < NL; ++i)
+#pragma unroll
+        for (int j = 0; j < NBM; ++j) {
+          x[i][j] = mlpn_ld4_dev(hand(i, 0, j));
+          G[i][j] = mlpn_ld4_dev(hand(i, 1, j));
+        }
+      const float* gp = gring + slot * P::GSLOT + NJD * tid;
+      if constexpr (NJD == 2)
+        gv = __hip_atomic_load(reinterpret_cast<const unsigned long long*>(gp), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      else
+        gv = __hip_atomic_load(reinterpret_cast<const unsigned*>(gp), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      publish((unsigned)(st + 1));  // all of it has landed
+      slot = slot + 1 < P::SLOTS ? slot + 1 : 0;
+#pragma unroll
+      for (int i = 0; i < NL; ++i)
+#pragma unroll
+        for (int j = 0; j < NBM; ++j)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) lds[L::XI + i * TM + own + um + r * LM + 16 * j] = x[i][j][r];
+#pragma unroll
+      for (int j = 0; j < NJD; ++j) lds[L::ZL + t * LD + cg + GW * j] = __uint_as_float((unsigned)(gv >> (32 * j)));
     }
-    mlpn_wave_sync();
+    __syncthreads();
+    if constexpr (ROLE != 2) {
+#pragma unroll
+      for (int i = 1; i < NL; ++i) {
+        f32x4 z[NBM];
+        product(z, lds + L::XI + (i - 1) * TM, w[i - 1]);
+        hidden(i, z);
+        if (i + 1 < NL) __syncthreads();
+      }
+      mlpn_wave_sync();
+    }
     // X W[NL] over the wave's own rows
     auto last_product = [&](const float* X) {
       f32x4 z[NTD];
@@ -285,6 +431,7 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))
 #pragma unroll
       for (int n = 0; n < NTD; ++n) mlpn_st4(lds + L::PZ + (wave * NTD + n) * 256 + 4 * lane, z[n]);
     };
+    if constexpr (ROLE != 2) {
     // ---- Z[NL] = X[NL] W[NL]; G[NL] = LN-L2 gradient of Z[NL] + b[NL] against the target
     last_product(lds + L::XI + (NL - 1) * TM);
     __syncthreads();
@@ -307,6 +454,13 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))
       ln_l2_grad<D, GW>(lds + L::ZL + t * LD, sbl, lds + L::TG + t * LD, sgam, sbet, cg, a.eps, Gv);
 #pragma unroll
       for (int j = 0; j < NJD; ++j) lds[L::ZL + t * LD + cg + GW * j] = Gv[j];
+      if constexpr (ROLE == 1) {
+        float* gp = gring + slot * P::GSLOT + NJD * tid;
+        if constexpr (NJD == 2)
+          *reinterpret_cast<float2*>(gp) = float2{Gv[0], Gv[1]};
+        else
+          *gp = Gv[0];
+      }
     }
     __syncthreads();
     // ---- G[NL-1] = (G[NL] W[NL]^T) * gelu'(Z[NL-1]): own rows, transposed in the wave's own part of the pool
@@ -331,6 +485,7 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))
 #pragma unroll
       for (int j = 0; j < NBM; ++j) {
         G[NL - 1][j] *= z[j];
+        if (ROLE == 1) mlpn_st4(hand(NL - 1, 1, j), G[NL - 1][j]);
 #pragma unroll
         for (int r = 0; r < 4; ++r) lds[L::GT + um + r * LM + own + 16 * j] = G[NL - 1][j][r];
       }
@@ -388,12 +543,16 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))
             G[i][j][r] *= p[0] + p[TM];
           }
       }
+      if (ROLE == 1)
+#pragma unroll
+        for (int j = 0; j < NBM; ++j) mlpn_st4(hand(i, 1, j), G[i][j]);
       if (i > 0) {
 #pragma unroll
         for (int r = 0; r < 4; ++r)
 #pragma unroll
           for (int j = 0; j < NBM; ++j) lds[L::GT + um + r * LM + own + 16 * j] = G[i][j][r];
       }
+    }
     }
     // ---- output chain; W[i] is updated right behind its last product of the mini-batch
     auto last = [&]() { return te_last * mlpn_ld4(slr + 4 * g); };  // of rows 4 g ..
@@ -415,6 +574,17 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))
       for (int r = 0; r < 4; ++r) mx[r] = 4 * g + r <= c ? te * l[r] * (1.f + at[r]) : 0.f;
       return mx;
     };
+    auto step = [&](int i) {  // the update's gradient and the bias
+      const f32x4 lst = last();
+#pragma unroll
+      for (int j = 0; j < NBM; ++j) {
+        G[i][j] *= lst;
+        float s = (G[i][j][0] + G[i][j][1]) + (G[i][j][2] + G[i][j][3]);
+        s += __shfl_xor(s, 16);
+        s += __shfl_xor(s, 32);
+        bias[i][j] -= s;
+      }
+    };
     auto hidden_out = [&](int i, f32x4 (&z)[NBM]) {  // z -> Xb[i+1] and the own part of its attention block
       const f32x4 mx = attention(i);
       float* X = lds + L::POOL + (i & 1) * TM + own;
@@ -434,24 +604,24 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))
       for (int j = 0; j < NBM; ++j)
         mlpn_mma(p, mlpn_ld4(lds + L::XI + i * TM + am + own + 16 * j), mlpn_ld4(X + am + 16 * j));
       mlpn_st4(lds + L::PART + ((i + 1) & 1) * NW * 256 + wave * 256 + 4 * lane, p);
-      // the update's gradient and the bias
-      const f32x4 lst = last();
-#pragma unroll
-      for (int j = 0; j < NBM; ++j) {
-        G[i][j] *= lst;
-        float s = (G[i][j][0] + G[i][j][1]) + (G[i][j][2] + G[i][j][3]);
-        s += __shfl_xor(s, 16);
-        s += __shfl_xor(s, 32);
-        bias[i][j] -= s;
-      }
+      step(i);
     };
-    hidden_out(0, zq);
+    if constexpr (ROLE == 1) {
+      if (st + 1 == a.n_stages) publish((unsigned)(st + 1));  // (otherwise behind the updates, where nothing waits for the stores)
+      step(0);
+    } else {
+      hidden_out(0, zq);
+    }
 #pragma unroll
     for (int i = 1; i < NL; ++i) {
-      __syncthreads();
-      f32x4 z[NBM];
-      product(z, lds + L::POOL + ((i - 1) & 1) * TM, w[i - 1]);
-      hidden_out(i, z);
+      if constexpr (ROLE == 1) {
+        step(i);
+      } else {
+        __syncthreads();
+        f32x4 z[NBM];
+        product(z, lds + L::POOL + ((i - 1) & 1) * TM, w[i - 1]);
+        hidden_out(i, z);
+      }
       if (i == NL - 1) fetch(st + 1 < a.n_stages ? st + 1 : st);  // no branch: the registers would be kept through it
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -461,10 +631,12 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))
         for (int j = 0; j < NBM; ++j) mlpn_mma(w[i - 1][q][j], fx, G[i][j]);
       }
     }
-    last_product(lds + L::POOL + ((NL - 1) & 1) * TM);
-    __syncthreads();
+    if constexpr (ROLE != 1) {
+      last_product(lds + L::POOL + ((NL - 1) & 1) * TM);
+      __syncthreads();
+    }
     stage_rows();
-    if (wave < NTD) {
+    if (ROLE != 1 && wave < NTD) {
       f32x4 z = sum8(lds + L::PZ + wave * 256 + 4 * lane, NTD * 256);
       mlpn_mma(z, attention(NL), mlpn_col4(lds + L::ZL + ud + 16 * wave, LD));
 #pragma unroll
@@ -474,7 +646,7 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))
 #pragma unroll
       for (int q = 0; q < NTD; ++q)
 #pragma unroll
-        for (int j = 0; j < NBM; ++j) w0[q][j] = load_tile(a.W[0] + bh * D * M, M, q, j, lane_off(M, 0, own));
+        for (int j = 0; j < NBM; ++j) w0[q][j] = load_tile(a.W[W0S] + bh * D * M, M, q, j, lane_off(M, 0, own));
     }
     __builtin_amdgcn_sched_barrier(0);
     {
@@ -489,13 +661,17 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))
         for (int j = 0; j < NBM; ++j) mlpn_mma(wl[j][n], fx[j], gl);
       }
     }
+    if constexpr (ROLE == 1) {
+      if (st + 1 < a.n_stages) publish((unsigned)(st + 1));
+      slot = slot + 1 < P::SLOTS ? slot + 1 : 0;
+    }
 #pragma unroll
     for (int q = 0; q < NTD; ++q) {
       const f32x4 fx = -mlpn_col4(lds + L::XK + ud + 16 * q, LD);
 #pragma unroll
       for (int j = 0; j < NBM; ++j) {
         mlpn_mma(w0[q][j], fx, G[0][j]);
-        if (STREAM) store_tile(a.W[0] + bh * D * M, M, q, j, lane_off(M, 0, own), w0[q][j]);
+        if (STREAM) store_tile(a.W[W0S] + bh * D * M, M, q, j, lane_off(M, 0, own), w0[q][j]);
       }
     }
     float db = 0.f;
@@ -504,7 +680,7 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))
       for (int r = 0; r < 16; ++r) db += lds[L::ZL + r * LD + tid - (512 - D)] * (te_last * slr[r]);
     __syncthreads();
     // ---- out = XQ + LN(Zb[NL] + b[NL])
-    {
+    if constexpr (ROLE != 1) {
       const size_t row = bh * (size_t)a.seq_stride + (size_t)st * K + t;
       float xh[NJD], rstd;
       ln_stats<D, GW>(lds + L::ZBL + t * LD, sbl, cg, a.eps, xh, rstd);
@@ -515,33 +691,87 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))
           IO::store1(static_cast<elem*>(a.out) + row * D + o, lds[L::XQ + t * LD + o] + (sgam[o] * xh[j] + sbet[o]));
       }
     }
-    __syncthreads();
+    if (ROLE != 1) __syncthreads();
     if (tid >= 512 - D) sbl[tid - (512 - D)] -= db;
   }
 
+  bool poison = false;  // a wait was in vain: nothing of this unit passes for a result
+  if constexpr (ROLE != 0) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this side's stores into W_out lie in front of the final state's
+    lane = tid & 63, wave = tid >> 6;
+    float* S = lds + L::PZ;
+    __syncthreads();
+    if (lane == 0) S[wave] = lost ? 1.f : 0.f;
+    __syncthreads();
+    float any = 0.f;
+#pragma unroll
+    for (int v = 0; v < NW; ++v) any += S[v];
+    poison = __builtin_amdgcn_readfirstlane((int)any) != 0;
+    if (poison && tid == 0) atomicAdd(a.lost_count, 1u);
+    if (ROLE == 1) return;
+    if (poison) {
+      const size_t n = (size_t)a.n_stages * K * D;
+      for (size_t e = tid; e < n; e += 512)
+        IO::store1(static_cast<elem*>(a.out) + bh * (size_t)a.seq_stride * D + e, __builtin_nanf(""));
+    }
+  }
+
   // ---- final state
+  const float nan = __builtin_nanf("");
+  auto final_value = [&](f32x4 v) { return ROLE == 2 && poison ? f32x4{nan, nan, nan, nan} : v; };
   const unsigned oc1 = lane_off(M, 0, 16 * NBM * wave), orow1 = lane_off(D, 16 * NBM * wave, 0);
 #pragma unroll
   for (int j = 0; j < NBM; ++j) {
     const int n = wave * NBM + j;
     if (!STREAM) {
 #pragma unroll
-      for (int q = 0; q < NTD; ++q) store_tile(a.W[0] + bh * D * M, M, q, j, oc1, w0[q][j]);
+      for (int q = 0; q < NTD; ++q) store_tile(a.W[0] + bh * D * M, M, q, j, oc1, final_value(w0[q][j]));
     }
 #pragma unroll
     for (int i = 1; i < NL; ++i)
 #pragma unroll
-      for (int q = 0; q < NTM; ++q) store_tile(a.W[i] + bh * M * M, M, q, j, oc1, w[i - 1][q][j]);
+      for (int q = 0; q < NTM; ++q) store_tile(a.W[i] + bh * M * M, M, q, j, oc1, final_value(w[i - 1][q][j]));
 #pragma unroll
-    for (int q = 0; q < NTD; ++q) store_tile(a.W[NL] + bh * M * D, D, j, q, orow1, wl[j][q]);
+    for (int q = 0; q < NTD; ++q) store_tile(a.W[NL] + bh * M * D, D, j, q, orow1, final_value(wl[j][q]));
 #pragma unroll
     for (int i = 0; i < NL; ++i)
-      if (g == 0) a.b[i][bh * M + 16 * n + c] = bias[i][j];
+      if (g == 0) a.b[i][bh * M + 16 * n + c] = ROLE == 2 && poison ? nan : bias[i][j];
   }
   __syncthreads();
-  if (tid < D) a.b[NL][bh * D + tid] = sbl[tid];
+  if (tid < D) a.b[NL][bh * D + tid] = ROLE == 2 && poison ? nan : sbl[tid];
 }
 
-hipError_t launch_mlpn_fwd(bool f32, int head_dim, int n_hidden, const MlpNFwdArgs& a, hipStream_t s);  // ttt_mlpn_fwd.hip
+// The arguments where they lie in the argument segment: through the parameter the compiler loads all of them at the start, and
+// the f32 kernel at head_dim 64 spills 200 registers instead of 20.
+__device__ __forceinline__ const MlpNFwdArgs& mlpn_args() {
+  return *(const MlpNFwdArgs*)__builtin_amdgcn_kernarg_segment_ptr();
+}
+
+template <class T, int D, int NL>
+__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) ttt_mlpn_fwd_kernel(MlpNFwdArgs) {
+  mlpn_fwd_body<T, D, NL, 0>(mlpn_args(), blockIdx.x);
+}
+
+// Workgroups b and b + 8 of every 16 share a unit: consecutive workgroups go to the XCDs in turn, so both run behind one L2.
+template <class T, int D, int NL>
+__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) ttt_mlpn_fwd_pair_kernel(MlpNFwdArgs) {
+  const MlpNFwdArgs& a = mlpn_args();
+  const size_t bh = (size_t)(blockIdx.x >> 4) * 8 + (blockIdx.x & 7);
+  if (bh >= (size_t)a.B * a.H) return;
+  if (((blockIdx.x >> 3) & 1) == 0)
+    mlpn_fwd_body<T, D, NL, 1>(a, bh);
+  else
+    mlpn_fwd_body<T, D, NL, 2>(a, bh);
+}
+
+template <int D, int NL>
+__global__ void ttt_mlpn_fwd_clear_kernel(MlpNFwdArgs a) {  // the progress words of every unit
+  using P = MlpNPair<D, NL>;
+  constexpr int M = 4 * D;
+  float* fl = (P::STREAM ? a.W[1] + (size_t)blockIdx.x * M * M : a.W[0] + (size_t)blockIdx.x * D * M) + P::FL;
+  fl[threadIdx.x] = 0.f;
+}
+
+hipError_t launch_mlpn_fwd(bool f32, int head_dim, int n_hidden, bool pair, const MlpNFwdArgs& a, hipStream_t s);  // ttt_mlpn_fwd.hip
 
 }  // namespace ttt
