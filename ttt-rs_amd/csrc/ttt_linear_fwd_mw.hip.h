@@ -158,6 +158,17 @@ __device__ __forceinline__ void store_state_tiles(float* Wd, float* bd, const f3
   }
 }
 
+// Wc[I][jj][r] = W[feat(I, 4 g + r)][feat(w TPW + jj, c)]
+template <int D, int TPW>
+__device__ __forceinline__ void load_state_slice(f32x4 (&W)[D / 16][TPW], const float* W0, int w, int c, int g) {
+#pragma unroll
+  for (int I = 0; I < D / 16; ++I)
+#pragma unroll
+    for (int jj = 0; jj < TPW; ++jj)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) W[I][jj][r] = W0[feat(I, 4 * g + r) * D + feat(w * TPW + jj, c)];
+}
+
 // ---- State centring -------------------------------------------------------------------------------------------
 // LayerNorm does not see a shift common to all d features of a row, and the inner loop looks at the state only
 // through LayerNorm: Z1 = XK W + b feeds the LN-L2 gradient, Zbar = XQ W + b - (...) G the output LayerNorm.  With
@@ -172,12 +183,20 @@ __device__ __forceinline__ void store_state_tiles(float* Wd, float* bd, const f3
 //
 // centre_state: centres the wave's column slice Wc[I][jj] and its bias features in place.  m0s (LDS, D + 1 floats)
 // receives m at index 16 I + p for row feat(I, p), and mean(b) at index D.  Every lane subtracts the numbers it
-// reads back from m0s, so a whole row is shifted by one and the same float.  xch: LDS scratch of NW * D floats.
-// Ends with a workgroup barrier.
+// reads back from m0s, so a whole row is shifted by one and the same float.  xch: LDS scratch of (NW + 2) * D floats,
+// 16-byte aligned.  Ends with a workgroup barrier.  sum_a receives the sum of gamma^2 of the head, in every lane.
+// Both sums over the features go in one chain each from LDS, where the lanes put b0 and gamma: read from memory in the chain,
+// sixteen at a time, they were 2 d / 16 round trips one after the other.
+constexpr int kCentreBarriers = 3;  // of centre_state, for a wave that takes no part in it
 template <int D, int NW, int TPW>
 __device__ __forceinline__ void centre_state(f32x4 (&Wc)[D / 16][TPW], f32x4 (&bT)[TPW], const float* b0, float* m0s,
-                                             float* xch, int w, int c, int g) {
+                                             const float* gamma, float& sum_a, float* xch, int w, int c, int g) {
   constexpr int NT = D / 16;
+  float* const bg = xch + NW * D;
+  for (int i = threadIdx.x; i < D; i += 64 * NW) {
+    bg[i] = b0[i];
+    bg[D + i] = gamma[i];
+  }
 #pragma unroll
   for (int I = 0; I < NT; ++I)
 #pragma unroll
@@ -195,10 +214,24 @@ __device__ __forceinline__ void centre_state(f32x4 (&Wc)[D / 16][TPW], f32x4 (&b
     for (int ww = 0; ww < NW; ++ww) s += xch[i * NW + ww];
     m0s[i] = s * (1.0f / D);
   }
-  if (threadIdx.x == 0) {
-    float s = 0.f;
-    for (int f = 0; f < D; ++f) s += b0[f];
+  if (threadIdx.x == 64 * (NW - 1)) {  // (the row means are the first wave's)
+    float s = 0.f, sa = 0.f;
+#pragma unroll 1
+    for (int f = 0; f < D; f += 32) {
+      f32x4 b[8], ga[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        b[i] = *reinterpret_cast<const f32x4*>(bg + f + 4 * i);
+        ga[i] = *reinterpret_cast<const f32x4*>(bg + D + f + 4 * i);
+      }
+#pragma unroll
+      for (int i = 0; i < 32; ++i) {
+        s += b[i >> 2][i & 3];
+        sa += ga[i >> 2][i & 3] * ga[i >> 2][i & 3];
+      }
+    }
     m0s[D] = s * (1.0f / D);
+    m0s[D + 1] = sa;
   }
   __syncthreads();
 #pragma unroll
@@ -210,6 +243,7 @@ __device__ __forceinline__ void centre_state(f32x4 (&Wc)[D / 16][TPW], f32x4 (&b
   const float bb = m0s[D];
 #pragma unroll
   for (int jj = 0; jj < TPW; ++jj) bT[jj] -= bb;
+  sum_a = m0s[D + 1];
   __syncthreads();
 }
 
@@ -252,9 +286,9 @@ __device__ __forceinline__ void store_bias_true(float* bd, const f32x4 (&bT)[TPW
 
 // The final state: initial state + (centred state now - centred state at the start).  The start value is formed
 // again exactly as centre_state formed it, so a sequence that never updates the state (lr = 0, token_eta[K-1] = 0)
-// returns the initial state bit for bit.
+// returns the initial state bit for bit.  W0: the wave's slice of it, laid out as Wc (load_state_slice).
 template <int D, int TPW>
-__device__ __forceinline__ void store_state_final(float* Wd, float* bd, const float* W0, const float* b0,
+__device__ __forceinline__ void store_state_final(float* Wd, float* bd, const f32x4 (&W0)[D / 16][TPW], const float* b0,
                                                   const f32x4 (&Wc)[D / 16][TPW], const f32x4 (&bT)[TPW],
                                                   const float* m0s, int w, int c, int g) {
   constexpr int NT = D / 16;
@@ -266,7 +300,7 @@ __device__ __forceinline__ void store_state_final(float* Wd, float* bd, const fl
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int at = feat(I, 4 * g + r) * D + feat(w * TPW + jj, c);
-        const float w0 = W0[at];
+        const float w0 = W0[I][jj][r];
         const float start = w0 - m[r];
         Wd[at] = w0 + (Wc[I][jj][r] - start);
       }
@@ -394,7 +428,6 @@ __global__ void __launch_bounds__(64 * NW) ttt_linear_fwd_mw_kernel(Problems<Lin
   const frag ones = splat_frag<T>(1.f);
   const size_t sb = a.state_per_batch ? bh : (size_t)h;
   f32x4 gam[TPW], bet[TPW], bT[TPW], a2[TPW];
-  float sum_a = 0.f;
 #pragma unroll
   for (int jj = 0; jj < TPW; ++jj)
 #pragma unroll
@@ -405,22 +438,14 @@ __global__ void __launch_bounds__(64 * NW) ttt_linear_fwd_mw_kernel(Problems<Lin
       bT[jj][r] = a.b0[sb * D + f];
       a2[jj][r] = gam[jj][r] * gam[jj][r];
     }
-  for (int f = 0; f < D; ++f) sum_a += a.gamma[h * D + f] * a.gamma[h * D + f];
   // Wc[I][jj][r] = W[feat(I,4g+r)][feat(w*TPW+jj, c)]
   f32x4 Wc[NT][TPW];
-  {
-    const float* W0 = a.W0 + sb * D * D;
-#pragma unroll
-    for (int I = 0; I < NT; ++I)
-#pragma unroll
-      for (int jj = 0; jj < TPW; ++jj)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) Wc[I][jj][r] = W0[feat(I, 4 * g + r) * D + feat(w * TPW + jj, c)];
-  }
+  load_state_slice<D, TPW>(Wc, a.W0 + sb * D * D, w, c, g);
   // the kernel carries the centred state (see centre_state)
   __shared__ __attribute__((aligned(16))) float m0s[D + 4];
-  __shared__ float cxch[NW * D];
-  centre_state<D, NW, TPW>(Wc, bT, a.b0 + sb * D, m0s, cxch, w, c, g);
+  __shared__ __attribute__((aligned(16))) float cxch[(NW + 2) * D];
+  float sum_a;
+  centre_state<D, NW, TPW>(Wc, bT, a.b0 + sb * D, m0s, a.gamma + h * D, sum_a, cxch, w, c, g);
 
   // Ring of R = PF+1 register sets, loop unrolled by R: step u consumes set u and refills the set
   // that step u-1 consumed, so every set has fixed registers and a load is never copied (a copy
@@ -614,7 +639,9 @@ __global__ void __launch_bounds__(64 * NW) ttt_linear_fwd_mw_kernel(Problems<Lin
     }
   }
 
-  store_state_final<D, TPW>(a.W_out + bh * D * D, a.b_out + bh * D, a.W0 + sb * D * D, a.b0 + sb * D, Wc, bT, m0s, w, c, g);
+  f32x4 W0[NT][TPW];
+  load_state_slice<D, TPW>(W0, a.W0 + sb * D * D, w, c, g);
+  store_state_final<D, TPW>(a.W_out + bh * D * D, a.b_out + bh * D, W0, a.b0 + sb * D, Wc, bT, m0s, w, c, g);
   if constexpr (FAC)
     store_state_tiles<D, TPW>(a.W_ckpt + bh * (size_t)a.n_ckpt * (D * D), a.b_ckpt + bh * (size_t)a.n_ckpt * D, Wc, bT, w, lane);
 }

@@ -65,7 +65,7 @@ __device__ __forceinline__ void linear_fwd_sk_body(const LinearFwdArgs& a, const
   constexpr bool BF = sizeof(elem) == 2;
   constexpr float inv_d = 1.0f / D;
   static_assert(NW > 1, "the skewed kernel is for two or more waves per unit");
-  __shared__ float ex[2][8 * 16 * NW];
+  __shared__ __attribute__((aligned(16))) float ex[2][8 * 16 * NW];
   // f32 products with one feature tile per wave are bound by the f32 matrix instructions: the waves then share what
   // each would otherwise compute for itself.  Every wave transposes its own XK tile and forms the attention block over
   // its own 16 features; both cross LDS with the row sums (same barrier, same double buffering) and are read back
@@ -83,7 +83,7 @@ __device__ __forceinline__ void linear_fwd_sk_body(const LinearFwdArgs& a, const
   constexpr bool TRK = RAW >= 3 && !DMA && BF && !ADAM;
   const int lane = threadIdx.x & 63, w = (threadIdx.x >> 6) % NW;
   // RAW = 5: the wave behind the compute waves is the control wave; up to the point where it branches off it does what
-  // wave 0 does (w == 0: valid loads, LDS writes of the same values) and it stores nothing
+  // wave 0 does (w == 0: valid loads) and it stores nothing
   const bool ctlw = DMA && __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) == NW;
   const int c = lane & 15, g = lane >> 4;
   const size_t bh = STATES ? unit : blockIdx.x;
@@ -114,7 +114,6 @@ __device__ __forceinline__ void linear_fwd_sk_body(const LinearFwdArgs& a, const
   const frag ones = splat_frag<T>(1.f);
   const size_t sb = STATES ? state : a.state_per_batch ? bh : (size_t)h;
   f32x4 gam[TPW], bet[TPW], bT[TPW], a2[TPW];
-  float sum_a = 0.f;
 #pragma unroll
   for (int jj = 0; jj < TPW; ++jj)
 #pragma unroll
@@ -125,21 +124,12 @@ __device__ __forceinline__ void linear_fwd_sk_body(const LinearFwdArgs& a, const
       bT[jj][r] = a.b0[sb * D + f];
       a2[jj][r] = gam[jj][r] * gam[jj][r];
     }
-  for (int f = 0; f < D; ++f) sum_a += a.gamma[h * D + f] * a.gamma[h * D + f];
   f32x4 Wc[NT][TPW];
-  {
-    const float* W0 = a.W0 + sb * D * D;
-#pragma unroll
-    for (int I = 0; I < NT; ++I)
-#pragma unroll
-      for (int jj = 0; jj < TPW; ++jj)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) Wc[I][jj][r] = W0[feat(I, 4 * g + r) * D + feat(w * TPW + jj, c)];
-  }
+  load_state_slice<D, TPW>(Wc, a.W0 + sb * D * D, w, c, g);
   // the kernel carries the centred state (see centre_state): row means in LDS, the exchange buffer as scratch
   __shared__ __attribute__((aligned(16))) float m0s[D + 4];
-  static_assert(NW * D <= 2 * 8 * 16 * NW, "the exchange buffer doubles as scratch of centre_state");
-  centre_state<D, NW, TPW>(Wc, bT, a.b0 + sb * D, m0s, &ex[0][0], w, c, g);
+  static_assert((NW + 2) * D <= 2 * 8 * 16 * NW, "the exchange buffer doubles as scratch of centre_state");
+  float sum_a;  // of gamma^2, from centre_state
 
   // ADAM: first and second moments of this wave's W tiles and bias rows, and the running powers beta^step
   f32x4 Wm[ADAM ? NT : 1][TPW], Wv[ADAM ? NT : 1][TPW], bm[TPW], bv[TPW];
@@ -527,6 +517,18 @@ __device__ __forceinline__ void linear_fwd_sk_body(const LinearFwdArgs& a, const
       dst.lr = ringlr_s[sl][c];
     }
   };
+  // The first rows are asked for before the state is centred: a launch of few mini-batches consists of round trips to memory, and
+  // this one then overlaps those of the state (and sums over d features go through LDS, see centre_state, and the final state's
+  // reference is read while the last output is exchanged).  One mini-batch, 12 units, launch to launch (an empty kernel 3.7): bf16
+  // d = 64 10.3 -> 6.8 us, d = 128 17.0 -> 10.8, f32 d = 64 9.5 -> 6.6, d = 128 26.3 -> 19.9; 384 units x 2048 tokens, bf16, d = 64
+  // 117.8 -> 114.0.
+  if constexpr (RAW != 0 && !DMA) {
+#pragma unroll
+    for (int u = 0; u < R; ++u) load_raw(raw[u], u);
+  } else if constexpr (!DMA) {
+#pragma unroll
+    for (int u = 0; u < PF; ++u) load_stage_mw<T, D, NW, FULL>(buf[u], ub, K, n_stages_, u, c, g, w);
+  }
   if constexpr (DMA) {
     if (ctlw) {
       const unsigned ring0 = (unsigned)(size_t)(__attribute__((address_space(3))) unsigned char*)&ring_s[0][0][0][0];
@@ -548,6 +550,8 @@ __device__ __forceinline__ void linear_fwd_sk_body(const LinearFwdArgs& a, const
       };
 #pragma unroll
       for (int u = 0; u < RS; ++u) copy_in(u);
+#pragma unroll
+      for (int i = 0; i < kCentreBarriers; ++i) asm volatile("s_barrier" ::: "memory");  // the compute waves centre the state
       asm volatile("s_waitcnt vmcnt(%0)" ::"n"((RS - 1) * kCopies) : "memory");  // mini-batch 0 has landed
       asm volatile("s_barrier" ::: "memory");
       for (int st = 0; st < n_stages_; ++st) {
@@ -562,21 +566,17 @@ __device__ __forceinline__ void linear_fwd_sk_body(const LinearFwdArgs& a, const
       return;
     }
   }
+  centre_state<D, NW, TPW>(Wc, bT, a.b0 + sb * D, m0s, a.gamma + h * D, sum_a, &ex[0][0], w, c, g);
   if constexpr (DMA) {
     lds_barrier();
     gather_dma(buf[0], 0);
   } else if constexpr (RAW != 0) {
     // mini-batch 0 complete, mini-batch 1 rotated and on its way through LDS (read behind the first barrier of the
     // loop), the raw rows of mini-batch 2 in flight
-#pragma unroll
-    for (int u = 0; u < R; ++u) load_raw(raw[u], u);
     rotate_share(raw[0], buf[0], 0, 0);
     lds_barrier();
     gather_rows(buf[0], 0);
     rotate_share(raw[1], buf[1], 1, 1);
-  } else {
-#pragma unroll
-    for (int u = 0; u < PF; ++u) load_stage_mw<T, D, NW, FULL>(buf[u], ub, K, n_stages_, u, c, g, w);
   }
 
   // One pass over R mini-batches (the ring of prefetch registers is indexed at compile time).  CHECKED:
@@ -936,6 +936,8 @@ __device__ __forceinline__ void linear_fwd_sk_body(const LinearFwdArgs& a, const
     return;
   }
   // ---- flush the last mini-batch's output
+  f32x4 W0[NT][TPW];
+  load_state_slice<D, TPW>(W0, a.W0 + sb * D * D, w, c, g);
   {
     float S[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     pend_sums(zbp, S[6], S[7]);
@@ -943,7 +945,7 @@ __device__ __forceinline__ void linear_fwd_sk_body(const LinearFwdArgs& a, const
     if (n_st() >= 2) emit_output(so0, so1, n_st() - 2, zbo, qoo);
     emit_output(S[6], S[7], n_st() - 1, zbp, qop);
   }
-  store_state_final<D, TPW>(a.W_out + bh * D * D, a.b_out + bh * D, a.W0 + sb * D * D, a.b0 + sb * D, Wc, bT, m0s, w, c, g);
+  store_state_final<D, TPW>(a.W_out + bh * D * D, a.b_out + bh * D, W0, a.b0 + sb * D, Wc, bT, m0s, w, c, g);
   if constexpr (ADAM) {
 #pragma unroll
     for (int I = 0; I < NT; ++I)
@@ -1028,7 +1030,7 @@ __global__ void __launch_bounds__(64 * NW, 2) ttt_linear_states_kernel(LinearFwd
   b.b0 = sg.b_in;
   b.W_ckpt = a.W_ckpt + at * (D * D);
   b.b_ckpt = a.b_ckpt + at * D;
-  b.n_stages = min(sg.every, a.n_ckpt - (int)at) - 1;
+  b.n_stages = __builtin_amdgcn_readfirstlane(min(sg.every, a.n_ckpt - (int)at) - 1);  // (the division leaves it in a vector register)
   linear_fwd_sk_body<T, D, NW, 2, FULL, false, 0, false, true>(b, nullptr, nullptr, unit,
                                                                unit * (size_t)sg.n_in + sg.first + seg);
 }
