@@ -126,6 +126,24 @@ __device__ __forceinline__ f32x4 over_tokens(f32x4 v) {
 // of a row must hold the SAME number (a pivot subtracted from a whole matrix row), one lane's result is shared.
 __device__ __forceinline__ float row16_first(float v) { return __shfl(v, (int)(threadIdx.x & 48u), 64); }
 
+// The sum of D floats in memory, or of their squares, in ascending order, the same float in every lane; for whole waves.  One load,
+// then a chain over the lanes: with the loads in the chain, sixteen floats at a time, it was D / 16 round trips to memory.
+template <int D, bool SQUARES = false>
+__device__ __forceinline__ float sum_in_order(const float* p) {
+  const int lane = threadIdx.x & 63;
+  float s = 0.f;
+#pragma unroll
+  for (int i = 0; i < D; i += 64) {
+    const int v = lane < D - i ? __float_as_int(p[i + lane]) : 0;
+#pragma unroll 16
+    for (int f = 0; f < (D - i < 64 ? D - i : 64); ++f) {
+      const float x = __int_as_float(__builtin_amdgcn_readlane(v, f));
+      s = SQUARES ? __builtin_fmaf(x, x, s) : s + x;
+    }
+  }
+  return s;
+}
+
 // A kernel argument in a scalar register from here on.  Short of scalar registers the compiler otherwise loads it again where
 // it is used, in every mini-batch: a round trip through the scalar cache, behind a barrier in the middle of the chain.
 __device__ __forceinline__ float held(float x) {

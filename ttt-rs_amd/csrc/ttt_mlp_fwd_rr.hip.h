@@ -213,7 +213,6 @@ __global__ void __launch_bounds__(512, D == 32 ? 4 : 2) ttt_mlp_fwd_rr_kernel(Pr
     }
   }
   f32x4 b2T;
-  float sum_a = 0.f;
   if (tid < 16) RHO[tid] = tid < K ? a.token_eta[tid] / sc : 0.f;
   if (w == 0) IDs[lane] = identity_frag<T>(c, g);
 #pragma unroll
@@ -225,9 +224,12 @@ __global__ void __launch_bounds__(512, D == 32 ? 4 : 2) ttt_mlp_fwd_rr_kernel(Pr
 #pragma unroll
     for (int I = 0; I < NT; ++I) W2c[j][I] -= m;
   }
-  b2T -= mean_of(a.b2_0 + sb * D, D, inv_d);
-  for (int f = 0; f < D; ++f) sum_a += a.gamma[h * D + f] * a.gamma[h * D + f];
-  sum_a = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(sum_a)));
+  // Formed by whole waves from one load each; in the chain of loads 128 units x 2048 tokens took 647 instead of 637 us (d = 96).  Not
+  // so in the backward kernels and on pairs of CUs, where it changes nothing or costs 0.2 %.
+  float b2_mean = sum_in_order<D>(a.b2_0 + sb * D) * inv_d;  // as mean_of
+  asm volatile("" : "+v"(b2_mean));
+  b2T -= b2_mean;
+  const float sum_a = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(sum_in_order<D, true>(a.gamma + h * D))));
   for (int i = tid; i < D; i += 512) {
     GAM[i] = a.gamma[h * D + i];
     BET[i] = a.beta[h * D + i];
