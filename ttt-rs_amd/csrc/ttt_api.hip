@@ -268,7 +268,11 @@ int launch_linear_fwd_wide(const ttt::LinearFwdArgs* probs, unsigned ny, hipStre
   const auto P = pack_of(probs, ny);
   constexpr int NW = D / 32;
   constexpr bool f32 = sizeof(typename ttt::Io<T>::elem) == 4;
-  constexpr int PF = f32 ? 1 : 2;  // f32 fragments are twice as large: prefetch one mini-batch ahead
+  // f32 fragments are twice as large.  d = 96 holds the rows of one mini-batch ahead.  At d = 128 two sets of rows do not fit: the
+  // compiler moves some of the loaded rows on at once, which waits for all of them in every other mini-batch.  There is one set
+  // there, filled anew behind the products (PF = 0): 128 mini-batches, 12 units 836 -> 740 us, 64 865 -> 767, 512 1766 -> 1570; one
+  // mini-batch, 12 units 19.9 -> 16.0.  At d = 96 that gives 13.7 -> 12.4 for one mini-batch and costs 575 -> 580 for 128, 256 units.
+  constexpr int PF = f32 ? (D == 128 ? 0 : 1) : 2;
   const dim3 grid((unsigned)(a.B * a.H), ny), block(64 * NW);
   if constexpr (!f32 && D == 128) {
     if (any_input_sums(probs, ny)) {

@@ -527,7 +527,7 @@ __device__ __forceinline__ void linear_fwd_sk_body(const LinearFwdArgs& a, const
     for (int u = 0; u < R; ++u) load_raw(raw[u], u);
   } else if constexpr (!DMA) {
 #pragma unroll
-    for (int u = 0; u < PF; ++u) load_stage_mw<T, D, NW, FULL>(buf[u], ub, K, n_stages_, u, c, g, w);
+    for (int u = 0; u < (PF > 0 ? PF : 1); ++u) load_stage_mw<T, D, NW, FULL>(buf[u], ub, K, n_stages_, u, c, g, w);
   }
   if constexpr (DMA) {
     if (ctlw) {
@@ -803,7 +803,7 @@ __device__ __forceinline__ void linear_fwd_sk_body(const LinearFwdArgs& a, const
         const int st = st0 + u;
         if constexpr (RAW != 0)
           load_raw(raw[u], st + R);
-        else
+        else if (PF > 0)
           load_stage_mw<T, D, NW, FULL>(buf[(u + PF) % R], ub, K, n_stages_, st + PF, c, g, w);
         if (st >= n_st()) continue;
         const StageInMw<T, NT, TPW>& cur = buf[u];
@@ -867,6 +867,12 @@ __device__ __forceinline__ void linear_fwd_sk_body(const LinearFwdArgs& a, const
           moments(S, jj, z1[jj], uu, bq[jj]);
         }
         pend_sums(zbp, S[6], S[7]);
+        const float lr_st = cur.lr;
+        frag qo_st[TPW];
+#pragma unroll
+        for (int jj = 0; jj < TPW; ++jj) qo_st[jj] = cur.qo[jj];
+        // PF = 0: one set of rows, filled anew as soon as its products are done
+        if constexpr (PF == 0) load_stage_mw<T, D, NW, FULL>(buf[0], ub, K, n_stages_, st + 1, c, g, w);
         exchange8_publish(S, st & 1);
         if (st > 1) emit_output(so0, so1, st - 2, zbo, qoo);  // inside the exchange window, as above
         exchange8_collect(S, st & 1);
@@ -887,7 +893,7 @@ __device__ __forceinline__ void linear_fwd_sk_body(const LinearFwdArgs& a, const
           const float rstd = __builtin_amdgcn_rsqf(fmaxf(var, 0.f) + eps());
           const float s1 = rstd * (S[2] - mu * sum_a) + S[4];
           const float s2 = g_norm_sum(S, mu, rstd, FULL && u == 2);
-          const float p = -sc * cur.lr * rstd;
+          const float p = -sc * lr_st * rstd;
           const float c1 = p * rstd, c2 = -c1 * s2 * inv_d, c3 = -p * s1 * inv_d;
 #pragma unroll
           for (int jj = 0; jj < TPW; ++jj) G[jj] = (z1[jj] - mu) * (a2[jj] * c1 + c2) + (bq[jj] * p + c3);
@@ -922,7 +928,7 @@ __device__ __forceinline__ void linear_fwd_sk_body(const LinearFwdArgs& a, const
 #pragma unroll
         for (int jj = 0; jj < TPW; ++jj) {
           zbp[jj] = zb[jj];
-          qop[jj] = cur.qo[jj];
+          qop[jj] = qo_st[jj];
         }
         if constexpr (RAW != 0) rotate_share(raw[(u + 2) % R], buf[(u + 2) % R], st + 2, st & 1);
       }
