@@ -170,6 +170,22 @@ def test_sequence_windows_in_place(P, d):
     assert torch.isnan(out_full[:, :, :lo]).all() and torch.isnan(out_full[:, :, hi:]).all()
 
 
+@pytest.mark.parametrize("K,N", [(16, 1), (16, 2), (16, 5), (5, 1), (5, 4)])
+@pytest.mark.parametrize("d", [96, 128])
+def test_f32_wide_heads_match_oracle_with_and_without_checkpoints(P, d, K, N):
+    """Wide heads hold one set of rows (d = 128, filled anew behind the products) or two: lengths around both, short mini-batches;
+    the mean of an offset bias and of gamma^2 go into it."""
+    print(f"case f32 wide d{d} K{K} N{N}", flush=True)
+    c = P.synthetic.reference_test_inputs(29 + d + K + N, 2, 3, N * K, d, K)
+    c["b0"] = c["b0"] + 0.5
+    c["gamma"] = c["gamma"] * torch.linspace(0.5, 1.5, d)
+    got, ref = run_case(P, c, K), oracle_case(c, K)
+    for name, x, r in zip(("out", "W", "b"), got, ref):
+        assert_close(x, r, TOL[torch.float32], name)
+    for name, x, y in zip(("out", "W", "b"), got, run_case(P, c, K, ckpt=True)):
+        assert torch.equal(x, y), name
+
+
 @pytest.mark.parametrize("N", [1, 2, 3, 4, 7])
 @pytest.mark.parametrize("d", [32, 64])
 def test_f32_forward_with_control_wave_without_checkpoints(P, d, N):
