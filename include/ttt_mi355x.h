@@ -120,7 +120,8 @@ typedef struct ttt_desc {
 #define TTT_HINT_ONE_WORKGROUP 0x8000
 /* Testing only: the two workgroups that share a (batch, head) unit in ttt_mlp_fwd at head_dim 128 (bf16 I/O) give
  * up waiting for each other at once, as if the partner had never become resident.  Exercises the failure path
- * described at ttt_mlp_fwd: every output of the affected units is NaN.  All kernels still run to their end. */
+ * described at ttt_mlp_fwd: every output of the affected units is NaN.  All kernels still run to their end.  (ttt_mlpn_fwd:
+ * likewise, and the units are computed again.) */
 #define TTT_HINT_TEST_LOST_PARTNER 0x200
 /* Testing only: the same two workgroups treat each other as running on different XCDs whatever they find at start,
  * i.e. take the path of a pair that was not placed on one XCD: every word they exchange is stored at device scope
@@ -261,7 +262,8 @@ int ttt_linear_bwd_ws(const ttt_desc* desc, const void* xq, const void* xk, cons
  * TTT_HINT_LDS_TILES to use the single-workgroup kernel (slower, f32 products).
  *
  * ttt_mlp_fwd_lost_workgroups: the device's status word of that kernel (and of the kernels of ttt_mlp_bwd and
- * ttt_linear_bwd_ws on two workgroups per unit, see there), the number of workgroups whose wait for
+ * ttt_linear_bwd_ws on two workgroups per unit, see there; and of ttt_mlpn_fwd, whose results a wait in vain does not
+ * harm), the number of workgroups whose wait for
  * their partner ran out since the library was loaded on the current device (0 on a healthy run; it never
  * decreases, compare with the value before the call).  A blocking copy from the device: call it after the
  * stream's work has finished.  No counterpart in the reference.
@@ -495,10 +497,12 @@ int ttt_linear_fwd_fused_inputs(const ttt_desc* desc, const void* xq, const void
  * LDS of a CU); ttt_mlpn_supported says so beforehand.  One hidden layer is ttt_mlp_fwd.  desc.seq_stride is
  * honoured (a window of a longer sequence in place).
  * With at most half as many (batch, head) units as the device has CUs (in groups of eight) and four mini-batches or more, a unit
- * is worked on by two workgroups on two CUs, where W_out is 16-byte aligned and overlaps no other argument: the same results
- * bit for bit; TTT_HINT_ONE_WORKGROUP keeps it on one.  They wait for each other, a bounded time; a unit whose workgroups were
- * never resident together has NaN in out, in W_out of the last layer and in every b_out, and is counted by
- * ttt_mlp_fwd_lost_workgroups.
+ * is worked on by two workgroups on two CUs, where W_out is 16-byte aligned and overlaps no other argument and out overlaps no
+ * input: the same results bit for bit; TTT_HINT_ONE_WORKGROUP keeps it on one.  During the call every W_out[i] also carries what
+ * the two hand over, and must be ordinary device memory (hipMalloc); for memory of another kind pass the hint.  The two wait
+ * for each other, a bounded time; a unit whose workgroups were not resident together in that time (2^21 polls, seconds: CUs held
+ * by other processes or streams) is computed again on one workgroup before the call's work ends, so the results are right all the
+ * same, and ttt_mlp_fwd_lost_workgroups counts the workgroups that waited in vain.
  */
 int ttt_mlpn_supported(const ttt_desc* desc, int n_hidden);
 int ttt_mlpn_fwd(const ttt_desc* desc, int n_hidden, const void* xq, const void* xk, const void* xv,

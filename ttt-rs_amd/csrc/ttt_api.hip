@@ -1018,7 +1018,8 @@ namespace {
 // eight.  The words are cleared by a launch of their own and the last mini-batch's output follows its state: 96 units, bf16, us on
 // one / two workgroups at 2, 4, 8 mini-batches: head_dim 64 82 / 90, 145 / 136, 273 / 229, head_dim 32 27 / 30, 49 / 47,
 // 91 / 78.  What crosses lies in the W_out buffers, 16 bytes to a lane, while
-// either side still reads its inputs: a caller's buffers that are not aligned so, or overlap an input, stay with one workgroup.
+// either side still reads its inputs, and a unit whose workgroups wait for each other in vain is done again from them: a caller's
+// buffers that are not aligned so, or outputs that overlap an input, stay with one workgroup.
 int mlpn_on_pairs(const ttt_desc* d, int n_hidden, ttt::MlpNFwdArgs& a, bool* yes) {
   *yes = false;
   if (d->kernel_hint & TTT_HINT_ONE_WORKGROUP) return TTT_OK;
@@ -1030,23 +1031,30 @@ int mlpn_on_pairs(const ttt_desc* d, int n_hidden, ttt::MlpNFwdArgs& a, bool* ye
   if ((units + 7) / 8 * 16 > (size_t)cus) return TTT_OK;
   const size_t D = (size_t)d->head_dim, M = 4 * D, io = d->io_dtype == TTT_F32 ? 4 : 2;
   const size_t tokens = (units - 1) * a.seq_stride + d->seq, states = d->state_per_batch ? units : (size_t)a.H;
-  const auto apart = [](const void* p, size_t n, const void* q, size_t m) {
-    const uintptr_t x = (uintptr_t)p, y = (uintptr_t)q;
-    return x + n <= y || y + m <= x;
-  };
-  for (int i = 0; i <= n_hidden; ++i) {
-    const size_t n = units * (i == 0 ? D : M) * (i == n_hidden ? D : M) * 4;
-    if (!aligned16(a.W[i])) return TTT_OK;
-    bool ok = apart(a.W[i], n, a.token_eta, 4 * a.K) && apart(a.W[i], n, a.gamma, 4 * a.H * D) &&
-              apart(a.W[i], n, a.beta, 4 * a.H * D) && apart(a.W[i], n, a.lr, tokens * io);
-    for (const void* x : {a.xq, a.xk, a.xv, (const void*)a.out}) ok = ok && apart(a.W[i], n, x, tokens * D * io);
+  // whether [p, p + n) overlaps no input
+  const auto clear_of_inputs = [&](const void* p, size_t n) {
+    const auto apart = [&](const void* q, size_t m) {
+      const uintptr_t x = (uintptr_t)p, y = (uintptr_t)q;
+      return x + n <= y || y + m <= x;
+    };
+    bool ok = apart(a.token_eta, 4 * a.K) && apart(a.gamma, 4 * a.H * D) && apart(a.beta, 4 * a.H * D) && apart(a.lr, tokens * io);
+    for (const void* x : {a.xq, a.xk, a.xv}) ok = ok && apart(x, tokens * D * io);
     for (int j = 0; j <= n_hidden; ++j) {
       const size_t out = j == n_hidden ? D : M;
-      ok = ok && apart(a.W[i], n, a.W0[j], states * (j == 0 ? D : M) * out * 4) && apart(a.W[i], n, a.b0[j], states * out * 4) &&
-           apart(a.W[i], n, a.b[j], units * out * 4);
+      ok = ok && apart(a.W0[j], states * (j == 0 ? D : M) * out * 4) && apart(a.b0[j], states * out * 4);
     }
-    if (!ok) return TTT_OK;
+    return ok;
+  };
+  const auto overlap = [](const void* p, size_t n, const void* q, size_t m) {
+    return (uintptr_t)p < (uintptr_t)q + m && (uintptr_t)q < (uintptr_t)p + n;
+  };
+  bool ok = clear_of_inputs(a.out, tokens * D * io);
+  for (int i = 0; ok && i <= n_hidden; ++i) {
+    const size_t n = units * (i == 0 ? D : M) * (i == n_hidden ? D : M) * 4;
+    ok = aligned16(a.W[i]) && clear_of_inputs(a.W[i], n) && !overlap(a.W[i], n, a.out, tokens * D * io);
+    for (int j = 0; j <= n_hidden; ++j) ok = ok && !overlap(a.W[i], n, a.b[j], units * (j == n_hidden ? D : M) * 4);
   }
+  if (!ok) return TTT_OK;
   rc = lost_word(&a.lost_count);
   if (rc != TTT_OK) return rc;
   a.spin_limit = (d->kernel_hint & TTT_HINT_TEST_LOST_PARTNER) ? 0u : 1u << 21;

@@ -7,11 +7,20 @@ template <class T, int D, int NL>
 static hipError_t launch(bool pair, const MlpNFwdArgs& a, hipStream_t s) {
   constexpr int bytes = (int)MlpNLds<D, NL>::BYTES;
   const unsigned units = (unsigned)(a.B * a.H);
-  const auto kern = pair ? ttt_mlpn_fwd_pair_kernel<T, D, NL> : ttt_mlpn_fwd_kernel<T, D, NL>;
-  const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+  const auto launch_lds = [&](auto kern, unsigned blocks, const MlpNFwdArgs& args) {
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+    if (e == hipSuccess) hipLaunchKernelGGL(kern, dim3(blocks), dim3(512), bytes, s, args);
+    return e;
+  };
+  MlpNFwdArgs one = a;
+  one.only_lost = pair ? 1 : 0;
+  if (pair) {
+    hipLaunchKernelGGL((ttt_mlpn_fwd_clear_kernel<D, NL>), dim3(units), dim3(MlpNPair<D, NL>::FL_WORDS), 0, s, a);
+    const hipError_t e = launch_lds(ttt_mlpn_fwd_pair_kernel<T, D, NL>, (units + 7) / 8 * 16, a);
+    if (e != hipSuccess) return e;
+  }
+  const hipError_t e = launch_lds(ttt_mlpn_fwd_kernel<T, D, NL>, units, one);
   if (e != hipSuccess) return e;
-  if (pair) hipLaunchKernelGGL((ttt_mlpn_fwd_clear_kernel<D, NL>), dim3(units), dim3(MlpNPair<D, NL>::FL_WORDS), 0, s, a);
-  hipLaunchKernelGGL(kern, dim3(pair ? (units + 7) / 8 * 16 : units), dim3(512), bytes, s, a);
   return hipGetLastError();
 }
 

@@ -36,7 +36,9 @@
 // the unit's W_out (MlpNPair); two words per pair of waves say how far each has come.  The producer's stores stay in the L2 that
 // both share (each publishes its XCD number) or are written back by a device-scope release while that is not known; the
 // consumer loads at device scope.  Every wait is bounded: a side that waits in vain marks its words, both run to their end
-// without waiting, the consumer makes out, W[NL] and every b of the unit NaN, and a status word counts both.
+// without waiting, the consumer marks the unit in W[NL], and a status word counts both.  A launch of the one-workgroup kernel
+// behind the pair's does the marked units again, from inputs that no output overlaps (the caller's rule), and finds none where
+// nothing held the device's CUs for seconds: 4 us.
 // The arithmetic is that of one workgroup, bit for bit.  64 mini-batches of 16 tokens, bf16, us on one / on two workgroups:
 // head_dim 64, 12 units 2060 / 1502, 96 units 2080 / 1529, 128 units 2081 / 1570; head_dim 32, 96 units two hidden layers
 // 699 / 519, 48 units three 1057 / 778, 24 units four 1414 / 1040.
@@ -66,6 +68,7 @@ struct MlpNFwdArgs {
   unsigned spin_limit;   // polls before a wait for the partner gives up; 0: give up at once (tests of that path)
   int agent_release;     // 1: always publish with a device-scope release
   unsigned* lost_count;  // counts workgroups that waited in vain
+  int only_lost;         // 1: the launch behind the pair's, for the units marked kMlpNLost
 };
 
 template <int D, int NL>
@@ -105,6 +108,8 @@ struct MlpNPair {
   enum { COUNT = 0, XCD = 8, SIDE = 32 };
 };
 constexpr unsigned kMlpNPoison = 0xffffffffu;
+constexpr unsigned kMlpNLost = 0x7fc60b5eu;  // first word of a unit's W[NL], which no producer writes (a NaN that comes to have these
+                                             // bits by itself costs a computation, not the result)
 
 // acc += A B over 16 k: k step r takes the four k with index 4 g + r
 __device__ __forceinline__ void mlpn_mma(f32x4& acc, f32x4 a, f32x4 b) {
@@ -695,7 +700,6 @@ __device__ __forceinline__ void mlpn_fwd_body(const MlpNFwdArgs& a, const size_t
     if (tid >= 512 - D) sbl[tid - (512 - D)] -= db;
   }
 
-  bool poison = false;  // a wait was in vain: nothing of this unit passes for a result
   if constexpr (ROLE != 0) {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this side's stores into W_out lie in front of the final state's
     lane = tid & 63, wave = tid >> 6;
@@ -706,39 +710,37 @@ __device__ __forceinline__ void mlpn_fwd_body(const MlpNFwdArgs& a, const size_t
     float any = 0.f;
 #pragma unroll
     for (int v = 0; v < NW; ++v) any += S[v];
-    poison = __builtin_amdgcn_readfirstlane((int)any) != 0;
-    if (poison && tid == 0) atomicAdd(a.lost_count, 1u);
-    if (ROLE == 1) return;
-    if (poison) {
-      const size_t n = (size_t)a.n_stages * K * D;
-      for (size_t e = tid; e < n; e += 512)
-        IO::store1(static_cast<elem*>(a.out) + bh * (size_t)a.seq_stride * D + e, __builtin_nanf(""));
+    if (__builtin_amdgcn_readfirstlane((int)any) != 0) {  // a wait was in vain: the unit is done again
+      if (tid == 0) {
+        atomicAdd(a.lost_count, 1u);
+        if (ROLE == 2) *reinterpret_cast<unsigned*>(a.W[NL] + bh * M * D) = kMlpNLost;
+      }
+      return;
     }
+    if (ROLE == 1) return;
   }
 
   // ---- final state
-  const float nan = __builtin_nanf("");
-  auto final_value = [&](f32x4 v) { return ROLE == 2 && poison ? f32x4{nan, nan, nan, nan} : v; };
   const unsigned oc1 = lane_off(M, 0, 16 * NBM * wave), orow1 = lane_off(D, 16 * NBM * wave, 0);
 #pragma unroll
   for (int j = 0; j < NBM; ++j) {
     const int n = wave * NBM + j;
     if (!STREAM) {
 #pragma unroll
-      for (int q = 0; q < NTD; ++q) store_tile(a.W[0] + bh * D * M, M, q, j, oc1, final_value(w0[q][j]));
+      for (int q = 0; q < NTD; ++q) store_tile(a.W[0] + bh * D * M, M, q, j, oc1, w0[q][j]);
     }
 #pragma unroll
     for (int i = 1; i < NL; ++i)
 #pragma unroll
-      for (int q = 0; q < NTM; ++q) store_tile(a.W[i] + bh * M * M, M, q, j, oc1, final_value(w[i - 1][q][j]));
+      for (int q = 0; q < NTM; ++q) store_tile(a.W[i] + bh * M * M, M, q, j, oc1, w[i - 1][q][j]);
 #pragma unroll
-    for (int q = 0; q < NTD; ++q) store_tile(a.W[NL] + bh * M * D, D, j, q, orow1, final_value(wl[j][q]));
+    for (int q = 0; q < NTD; ++q) store_tile(a.W[NL] + bh * M * D, D, j, q, orow1, wl[j][q]);
 #pragma unroll
     for (int i = 0; i < NL; ++i)
-      if (g == 0) a.b[i][bh * M + 16 * n + c] = ROLE == 2 && poison ? nan : bias[i][j];
+      if (g == 0) a.b[i][bh * M + 16 * n + c] = bias[i][j];
   }
   __syncthreads();
-  if (tid < D) a.b[NL][bh * D + tid] = ROLE == 2 && poison ? nan : sbl[tid];
+  if (tid < D) a.b[NL][bh * D + tid] = sbl[tid];
 }
 
 // The arguments where they lie in the argument segment: through the parameter the compiler loads all of them at the start, and
@@ -749,7 +751,12 @@ __device__ __forceinline__ const MlpNFwdArgs& mlpn_args() {
 
 template <class T, int D, int NL>
 __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) ttt_mlpn_fwd_kernel(MlpNFwdArgs) {
-  mlpn_fwd_body<T, D, NL, 0>(mlpn_args(), blockIdx.x);
+  const MlpNFwdArgs& a = mlpn_args();
+  if (a.only_lost != 0) {
+    const unsigned* mark = reinterpret_cast<const unsigned*>(a.W[NL] + blockIdx.x * (size_t)(4 * D * D));
+    if (__builtin_amdgcn_readfirstlane((int)*mark) != (int)kMlpNLost) return;
+  }
+  mlpn_fwd_body<T, D, NL, 0>(a, blockIdx.x);
 }
 
 // Workgroups b and b + 8 of every 16 share a unit: consecutive workgroups go to the XCDs in turn, so both run behind one L2.

@@ -462,9 +462,11 @@ def ttt_stack_workspace_bytes(B: int, H: int, seq: int, d: int, mini_batch: int,
 
 
 def mlp_fwd_lost_workgroups() -> int:
-    """ttt_mlp_fwd_lost_workgroups of the current device: how many workgroups of the two-CU TTT-MLP forward
-    (head_dim 128, bf16 I/O) gave up waiting for their partner since the library was loaded.  A blocking copy from
-    the device; meaningful once the work in question has finished."""
+    """ttt_mlp_fwd_lost_workgroups of the current device: how many workgroups of the kernels that put a unit on two of them
+    (TTT-MLP forward at head_dim 128 with bf16 I/O, TTT-MLP backward, TTT-Linear backward with f32 I/O, TTT-MLP with several hidden
+    layers) gave up waiting for their partner since the library was loaded.  The unit's results are then NaN as those calls
+    say; ttt_mlpn_forward_raw's are right all the same.  A blocking copy from the device; meaningful once the work in
+    question has finished."""
     n = C.c_int64(0)
     check(lib().ttt_mlp_fwd_lost_workgroups(C.byref(n)))
     return n.value
