@@ -313,12 +313,11 @@ __device__ __forceinline__ void linear_fwd_sk_body(const LinearFwdArgs& a, const
       return f;
     }
   };
-  // s2 of the LN-L2 gradient, a sum of two products of which one is rounded before the other is added.  Written out, `second`
-  // as the callers have it: left open, the compiler decides it in each copy of the body, anew after every change of the
-  // code around it, and a stack of layers carries a last bit on to 1 % of its outputs.
-  auto g_norm_sum = [&](const float (&S)[8], float mu, float rstd, bool second) {
-    const float m = S[5] - mu * S[4], q = S[3] - 2.f * mu * S[2] + mu * mu * sum_a, r2 = rstd * rstd;
-    return second ? __builtin_fmaf(r2, q, rstd * m) : __builtin_fmaf(m, rstd, r2 * q);
+  // s2 of the LN-L2 gradient, a sum of two products of which one is rounded before the other is added: written out, or the
+  // compiler decides it in each copy of the body, and a mini-batch is rounded by its place in the loop.
+  auto g_norm_sum = [&](const float (&S)[8], float mu, float rstd) {
+    const float m = S[5] - mu * S[4], q = S[3] - 2.f * mu * S[2] + mu * mu * sum_a;
+    return __builtin_fmaf(rstd * rstd, q, rstd * m);
   };
   const frag ident_upd = upd ? ident : IO::zero();
   const frag ones_upd = upd ? ones : IO::zero();
@@ -589,8 +588,8 @@ __device__ __forceinline__ void linear_fwd_sk_body(const LinearFwdArgs& a, const
   const float b_mean = __builtin_amdgcn_readfirstlane(m0s[D]);  // mean of the initial bias (split off by centre_state)
   static_assert(!FAC || BF, "update factors are saved with bf16 I/O only");
   unsigned char* fac = FAC ? factor_base<D>(a.W_ckpt, a.n_ckpt, bh) : nullptr;
-  auto pass = [&](auto checked_tag, auto later_tag, int st0) {
-    constexpr bool CHECKED = decltype(checked_tag)::value, LATER = decltype(later_tag)::value;
+  auto pass = [&](auto checked_tag, int st0) {
+    constexpr bool CHECKED = decltype(checked_tag)::value;
 #pragma unroll
     for (int u = 0; u < R; ++u) {
       const int st = st0 + u;
@@ -713,7 +712,7 @@ __device__ __forceinline__ void linear_fwd_sk_body(const LinearFwdArgs& a, const
         const float var = S[1] * inv_d - mu * mu;
         const float rstd = __builtin_amdgcn_rsqf(fmaxf(var, 0.f) + eps());
         const float s1 = rstd * (S[2] - mu * sum_a) + S[4];
-        const float s2 = g_norm_sum(S, mu, rstd, ADAM || FORM || STATES || (FULL && (u == 2 || LATER)));
+        const float s2 = g_norm_sum(S, mu, rstd);
         const float p = -sc * cur.lr * rstd;
         const float c1 = p * rstd, c2 = -c1 * s2 * inv_d, c3 = -p * s1 * inv_d;
 #pragma unroll
@@ -788,12 +787,12 @@ __device__ __forceinline__ void linear_fwd_sk_body(const LinearFwdArgs& a, const
     }
   };
   if constexpr (COMPACT) {
-    for (int st0 = 0; st0 < n_st(); st0 += R) pass(std::true_type{}, std::false_type{}, st0);
+    for (int st0 = 0; st0 < n_st(); st0 += R) pass(std::true_type{}, st0);
   } else if constexpr (NT <= 4) {
     int st0 = 0;
-    pass(std::true_type{}, std::false_type{}, st0);
-    for (st0 = R; st0 + R <= n_st(); st0 += R) pass(std::false_type{}, std::true_type{}, st0);
-    if (st0 < n_st()) pass(std::true_type{}, std::true_type{}, st0);
+    pass(std::true_type{}, st0);
+    for (st0 = R; st0 + R <= n_st(); st0 += R) pass(std::false_type{}, st0);
+    if (st0 < n_st()) pass(std::true_type{}, st0);
   } else {
     // Wide heads (d = 96, 128) keep the loop with its branches: in one long basic block the scheduler overlaps
     // so much that the state tiles no longer fit the register file (d = 128: 30 spilled registers).
@@ -892,7 +891,7 @@ __device__ __forceinline__ void linear_fwd_sk_body(const LinearFwdArgs& a, const
           const float var = S[1] * inv_d - mu * mu;
           const float rstd = __builtin_amdgcn_rsqf(fmaxf(var, 0.f) + eps());
           const float s1 = rstd * (S[2] - mu * sum_a) + S[4];
-          const float s2 = g_norm_sum(S, mu, rstd, FULL && u == 2);
+          const float s2 = g_norm_sum(S, mu, rstd);
           const float p = -sc * lr_st * rstd;
           const float c1 = p * rstd, c2 = -c1 * s2 * inv_d, c3 = -p * s1 * inv_d;
 #pragma unroll
