@@ -162,7 +162,7 @@ __device__ __forceinline__ void linear_fwd_sk_body(const LinearFwdArgs& a, const
   }
   // One Adam step on a tile: gneg = -gradient (what the plain kernel would add to the state).  The moments are carried
   // as m / (1 - beta1) and v / (1 - beta2), so that each decays and takes its new term in one or two instructions, and
-  // lr m^ / (sqrt(v^) + eps()) is taken as ad_k m / (sqrt(v) + ad_e) with the bias corrections in the two scalars: eight
+  // lr m^ / (sqrt(v^) + eps) is taken as ad_k m / (sqrt(v) + ad_e) with the bias corrections in the two scalars: eight
   // instructions per element, two of them transcendental, where the step as written has eleven.
   float ad_k = 0.f, ad_e = 0.f;
   auto adam_tile = [&](f32x4& x, f32x4& m, f32x4& v, f32x4 gneg) {
@@ -741,7 +741,7 @@ __device__ __forceinline__ void linear_fwd_sk_body(const LinearFwdArgs& a, const
         pw1 *= adam->beta1;
         pw2 *= adam->beta2;
         {
-          // v^ = v c2, m^ = m c1: lr m^ / (sqrt(v^) + eps()) = (lr c1 / sqrt(c2)) m / (sqrt(v) + eps / sqrt(c2))
+          // v^ = v c2, m^ = m c1: lr m^ / (sqrt(v^) + eps) = (lr c1 / sqrt(c2)) m / (sqrt(v) + eps / sqrt(c2))
           const float c1 = (1.f - adam->beta1) / (1.f - pw1), rc2 = sqrtf((1.f - pw2) / (1.f - adam->beta2));
           ad_k = -adam->lr * c1 * rc2;
           ad_e = adam->eps * rc2;
