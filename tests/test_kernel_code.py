@@ -84,3 +84,12 @@ def test_mlp_backward_reads_its_look_ahead_from_lds(tmp_path):
             f"ttt_mlp_bwd_rp_kernel<{d}>(MlpBwdRpArgs)" for d in (32, 64)]).items():
         flat = [s for s in body if s.startswith("flat_")]
         assert not flat, f"{name}: {flat}"
+
+
+def test_linear_adam_keeps_no_addresses_through_its_loop(tmp_path):
+    """f32 I/O, head_dim 64: state, moments and rows fill the registers, and what is spilled besides is spilled around the loop.  The
+    addresses of the initial state, 32 registers, were kept from the prologue for the final state (44 to 63 spilled, now 18 to 36)."""
+    for name, (_, figures) in compile_kernels(tmp_path, "ttt_linear_fwd_sk.hip.h", [
+            f"ttt_linear_adam_fwd_kernel<F32, 64, 4, {k}, 2>(LinearFwdArgs, AdamArgs)" for k in (
+                "2, true, 5, false", "1, true, 0, true", "1, false, 0, true")]).items():
+        assert figures["vgpr_spill_count"] <= 40, f"{name}: {figures}"
