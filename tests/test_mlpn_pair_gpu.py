@@ -68,6 +68,36 @@ def test_units_that_wait_in_vain_are_done_again(n_hidden, B, H, d, K, N):
         assert torch.equal(a, b), i
 
 
+def test_one_workgroup_can_be_asked_for_from_python():
+    """kernel_hint reaches the library from the call and from the layer object: no workgroup waits where one was asked for."""
+    P = importlib.import_module("ttt-rs_amd")
+    B, H, d, K, N = 1, 2, 32, 16, 5
+    c, Ws, bs = make_case(P, 2450, B, H, N * K, d, K, 2, torch.float32)
+    dv, dev = to_dev(c), lambda ts: [t.to("cuda:0") for t in ts]
+    x = (dv["xq"], dv["xk"], dv["xv"])
+    before = P.mlp_fwd_lost_workgroups()
+
+    def raw(hint):
+        out, W, b = P.ttt_mlpn_forward_raw(*x, dev(Ws), dev(bs), dv["token_eta"], dv["lr"], dv["gamma"], dv["beta"], K, kernel_hint=hint)
+        return [out, *W, *b]
+
+    def layer(hint):
+        m = P.FusedMlpN(P.ModelConfig(H, d, P.TTTConfig(mini_batch_size=K)), dev(Ws), dev(bs), dv["gamma"], dv["beta"], kernel_hint=hint)
+        state = m.init_state(B)
+        out = m.forward(state, P.TTTInputsInner(P.Qkv(*x), dv["token_eta"].repeat(N), dv["lr"]))
+        return [out, *state.weights, *state.biases]
+
+    want = raw(ONE | LOST)
+    for f in (raw, layer):
+        for a, b in zip(f(ONE | LOST), want):
+            assert torch.equal(a, b)
+    assert P.mlp_fwd_lost_workgroups() == before
+    for i, f in enumerate((raw, layer)):
+        for a, b in zip(f(LOST), want):
+            assert torch.equal(a, b)
+        assert P.mlp_fwd_lost_workgroups() == before + 2 * B * H * (i + 1)
+
+
 def test_two_workgroups_in_a_graph():
     P = importlib.import_module("ttt-rs_amd")
     B, H, d, K, N = 2, 3, 64, 16, 5

@@ -1015,9 +1015,9 @@ int ttt_linear_fwd(const ttt_desc* d, const void* xq, const void* xk, const void
 namespace {
 // Whether a unit of ttt_mlpn_fwd runs on two workgroups (see ttt_mlpn_fwd.hip.h), and what that form needs besides.  Both of
 // a unit's workgroups must be resident together and each fills a CU, so there may be half as many units as CUs, in groups of
-// eight.  The words are cleared by a launch of their own and the last mini-batch's output follows its state: 96 units, bf16, us on
-// one / two workgroups at 2, 4, 8 mini-batches: head_dim 64 82 / 90, 145 / 136, 273 / 229, head_dim 32 27 / 30, 49 / 47,
-// 91 / 78.  What crosses lies in the W_out buffers, 16 bytes to a lane, while
+// eight.  The words are cleared by a launch of their own, the last mini-batch's output follows its state, and the launch for units
+// to do again comes behind: 96 units, bf16, us on one / two workgroups at 2 (without that launch), 4, 8 mini-batches: head_dim 64
+// 82 / 90, 146 / 131, 276 / 224, head_dim 32 27 / 30, 49 / 47.5, 93 / 78.  What crosses lies in the W_out buffers, 16 bytes to a lane, while
 // either side still reads its inputs, and a unit whose workgroups wait for each other in vain is done again from them: a caller's
 // buffers that are not aligned so, or outputs that overlap an input, stay with one workgroup.
 int mlpn_on_pairs(const ttt_desc* d, int n_hidden, ttt::MlpNFwdArgs& a, bool* yes) {

@@ -38,10 +38,10 @@
 // consumer loads at device scope.  Every wait is bounded: a side that waits in vain marks its words, both run to their end
 // without waiting, the consumer marks the unit in W[NL], and a status word counts both.  A launch of the one-workgroup kernel
 // behind the pair's does the marked units again, from inputs that no output overlaps (the caller's rule), and finds none where
-// nothing held the device's CUs for seconds: 4 us.
+// nothing held the device's CUs for seconds: 1.5 us.
 // The arithmetic is that of one workgroup, bit for bit.  64 mini-batches of 16 tokens, bf16, us on one / on two workgroups:
-// head_dim 64, 12 units 2060 / 1502, 96 units 2080 / 1529, 128 units 2081 / 1570; head_dim 32, 96 units two hidden layers
-// 699 / 519, 48 units three 1057 / 778, 24 units four 1414 / 1040.
+// head_dim 64, 12 units 2066 / 1505, 96 units 2094 / 1533, 128 units 2093 / 1543; head_dim 32, 96 units two hidden layers
+// 704 / 523, three 1069 / 804, four 1429 / 1063.
 #pragma once
 #include "ttt_engine_fwd.hip.h"
 

@@ -583,7 +583,7 @@ PyObject* mlp_backward(PyObject* const* a) {
   return r;
 }
 
-// (xq, xk, xv, weights list, biases list, token_eta, lr, ln_weight, ln_bias, mini_batch, eps)
+// (xq, xk, xv, weights list, biases list, token_eta, lr, ln_weight, ln_bias, mini_batch, eps, kernel_hint)
 PyObject* mlpn_forward(PyObject* const* a) {
   Keep keep;
   keep.reserve(24);
@@ -619,7 +619,7 @@ PyObject* mlpn_forward(PyObject* const* a) {
   void* pl = need(a[6], gates, q.dtype, "ttt_lr_eta", keep);
   const float* gam = need_f32(a[7], hd, "ln_weight", keep);
   const float* bet = need_f32(a[8], hd, "ln_bias", keep);
-  const ttt_desc desc = desc_of(B, H, seq, d, K, real(a[10]), 1, io_of(q.t), per_batch, 0, 0, 0);
+  const ttt_desc desc = desc_of(B, H, seq, d, K, real(a[10]), 1, io_of(q.t), per_batch, 0, 0, integer(a[11]));
   check(ttt_mlpn_supported(&desc, hidden));
   at::Tensor out = empty(rows, q.dtype, q.dev), W[8], b[8];
   for (int i = 0; i < layers; ++i) {
@@ -911,7 +911,7 @@ PyMethodDef methods[] = {
     ENTRY(linear_backward, 20),
     ENTRY(mlp_forward, 15),
     ENTRY(mlp_backward, 19),
-    ENTRY(mlpn_forward, 11),
+    ENTRY(mlpn_forward, 12),
     ENTRY(stack_forward, 9),
     ENTRY(inner_inputs, 13),
     ENTRY(linear_forward_fused_inputs, 22),

@@ -140,12 +140,15 @@ def ttt_mlp_forward_raw(xq, xk, xv, w1, b1, w2, b2, token_eta, ttt_lr_eta, ln_we
 
 
 def ttt_mlpn_forward_raw(xq, xk, xv, weights, biases, token_eta, ttt_lr_eta, ln_weight, ln_bias, mini_batch: int,
-                         eps: float = 1e-6):
+                         eps: float = 1e-6, kernel_hint: int = 0):
     """One call of ttt_mlpn_fwd on the current stream: TTTMLP2/3/4::forward (rust/core/src/mlp2.rs, mlp3.rs, mlp4.rs
     looped as rust/core/src/inner.rs:25-50).  weights / biases: lists of the n_hidden + 1 layers, [H,in,out] / [H,out] or
-    with a leading batch dimension.  Returns (output, weights_out, biases_out), state per batch element."""
+    with a leading batch dimension.  Returns (output, weights_out, biases_out), state per batch element.
+    kernel_hint: with at most half as many (batch, head) units as the device has CUs and four mini-batches or more a unit
+    runs on two workgroups that wait for each other; TTT_HINT_ONE_WORKGROUP keeps it on one (the same bits), for a device
+    that other work holds for seconds, where the wait would be in vain and the unit computed again on one workgroup."""
     return host().mlpn_forward(xq, xk, xv, list(weights), list(biases), token_eta, ttt_lr_eta, ln_weight, ln_bias,
-                               mini_batch, eps)
+                               mini_batch, eps, int(kernel_hint))
 
 
 def ttt_mlp_backward_raw(xq, xk, xv, w1, b1, w2, b2, token_eta, ttt_lr_eta, ln_weight, ln_bias, d_out,
@@ -396,15 +399,16 @@ class TTTMLPNState:
 
 class FusedMlpN:
     """TTTMLP2 / TTTMLP3 / TTTMLP4 (rust/core/src/mlp2.rs, mlp3.rs, mlp4.rs) on the fused kernel: d -> 4d -> ... -> 4d
-    -> d with 2, 3 or 4 hidden layers, the TTTInnerModel interface of rust/core/src/inner.rs:13-58."""
+    -> d with 2, 3 or 4 hidden layers, the TTTInnerModel interface of rust/core/src/inner.rs:13-58.  kernel_hint: that of
+    ttt_mlpn_forward_raw, for every call."""
 
-    def __init__(self, config: ModelConfig, weights_init, biases_init, ln_weight, ln_bias):
+    def __init__(self, config: ModelConfig, weights_init, biases_init, ln_weight, ln_bias, kernel_hint: int = 0):
         H, d = config.num_heads, config.head_dim
         n = len(weights_init) - 1
         if n < 2 or n > 4 or len(biases_init) != n + 1:
             raise _lib.TttError(_lib.TTT_ERR_UNSUPPORTED, "FusedMlpN: 2, 3 or 4 hidden layers")
         dims = [d] + [4 * d] * n + [d]
-        self.config, self.n_hidden = config, n
+        self.config, self.n_hidden, self.kernel_hint = config, n, kernel_hint
         self.weights_init = [_need(w, (H, dims[i], dims[i + 1]), torch.float32, f"weights_init[{i}]")
                              for i, w in enumerate(weights_init)]
         self.biases_init = [_need(b, (H, dims[i + 1]), torch.float32, f"biases_init[{i}]")
@@ -426,7 +430,7 @@ class FusedMlpN:
     def _launch(self, state: TTTMLPNState, inputs: TTTInputsInner, mini_batch: int):
         out, ws, bs = ttt_mlpn_forward_raw(inputs.qkv.xq, inputs.qkv.xk, inputs.qkv.xv, state.weights, state.biases,
                                            inputs.token_eta, inputs.ttt_lr_eta, self.ln_weight, self.ln_bias,
-                                           mini_batch, self.config.ttt.epsilon)
+                                           mini_batch, self.config.ttt.epsilon, self.kernel_hint)
         state.weights, state.biases = ws, bs
         return out
 
