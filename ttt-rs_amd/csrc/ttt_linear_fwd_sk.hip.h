@@ -314,10 +314,13 @@ __device__ __forceinline__ void linear_fwd_sk_body(const LinearFwdArgs& a, const
     }
   };
   // s2 of the LN-L2 gradient, a sum of two products of which one is rounded before the other is added: written out, or the
-  // compiler decides it in each copy of the body, and a mini-batch is rounded by its place in the loop.
-  auto g_norm_sum = [&](const float (&S)[8], float mu, float rstd) {
-    const float m = S[5] - mu * S[4], q = S[3] - 2.f * mu * S[2] + mu * mu * sum_a;
-    return __builtin_fmaf(rstd * rstd, q, rstd * m);
+  // compiler decides it in each copy of the body, and a mini-batch is rounded by its place in the loop.  Wide heads keep what
+  // the compiler once chose for their loop (two of three mini-batches the other way): any other rounding there is as good, but a
+  // stack of six TTT-Linear and two TTT-MLP layers at d = 128 carries a last bit on to 1.0 % of its output, as much as callers who
+  // compare one version's results with the next's allow for.
+  auto g_norm_sum = [&](const float (&S)[8], float mu, float rstd, bool square_fused) {
+    const float m = S[5] - mu * S[4], q = S[3] - 2.f * mu * S[2] + mu * mu * sum_a, r2 = rstd * rstd;
+    return square_fused ? __builtin_fmaf(r2, q, rstd * m) : __builtin_fmaf(m, rstd, r2 * q);
   };
   const frag ident_upd = upd ? ident : IO::zero();
   const frag ones_upd = upd ? ones : IO::zero();
@@ -712,7 +715,7 @@ __device__ __forceinline__ void linear_fwd_sk_body(const LinearFwdArgs& a, const
         const float var = S[1] * inv_d - mu * mu;
         const float rstd = __builtin_amdgcn_rsqf(fmaxf(var, 0.f) + eps());
         const float s1 = rstd * (S[2] - mu * sum_a) + S[4];
-        const float s2 = g_norm_sum(S, mu, rstd);
+        const float s2 = g_norm_sum(S, mu, rstd, true);
         const float p = -sc * cur.lr * rstd;
         const float c1 = p * rstd, c2 = -c1 * s2 * inv_d, c3 = -p * s1 * inv_d;
 #pragma unroll
@@ -891,7 +894,7 @@ __device__ __forceinline__ void linear_fwd_sk_body(const LinearFwdArgs& a, const
           const float var = S[1] * inv_d - mu * mu;
           const float rstd = __builtin_amdgcn_rsqf(fmaxf(var, 0.f) + eps());
           const float s1 = rstd * (S[2] - mu * sum_a) + S[4];
-          const float s2 = g_norm_sum(S, mu, rstd);
+          const float s2 = g_norm_sum(S, mu, rstd, FULL && u == 2);
           const float p = -sc * lr_st * rstd;
           const float c1 = p * rstd, c2 = -c1 * s2 * inv_d, c3 = -p * s1 * inv_d;
 #pragma unroll
