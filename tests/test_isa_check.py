@@ -137,19 +137,41 @@ def test_mixed_shapes_five_wait_states_apart_are_exact():
     assert P.lib().ttt_selftest_mfma_mixed(4, 5, C.c_void_p(out.data_ptr()), stream) == P.TTT_ERR_SHAPE
 
 
-def test_scanner_flags_a_result_read_too_early_behind_a_branch():
-    """The compiler counts the wait states between a matrix instruction and a read of its result in straight code, not
-    across a branch: one instruction (the branch) in between read garbage on MI355X, one more did not."""
-    def code(between, behind):
-        return [K32.format(c="0")] + between + ["\ts_cbranch_vccnz .LBB0_2", "\ts_branch .LBB0_1", ".LBB0_1:", "\ts_nop 7", ".LBB0_2:"] + behind
+def test_scanner_flags_a_result_used_too_early():
+    """A read, and a write, by anything but a matrix instruction: eight wait states behind a four-pass instruction, ten behind an
+    eight-pass one, as the compiler keeps them in straight code."""
+    read = "\tv_mul_f32_e32 v40, v41, v{r}"
+    assert [h[4] for h in flagged([K32.format(c="0"), "\ts_nop 6", read.format(r=1)])] == [7]
+    assert flagged([K32.format(c="0"), "\ts_nop 7", read.format(r=1)]) == []
+    assert [h[4] for h in flagged([F32, "\ts_nop 7", "\ts_nop 0", read.format(r=1)])] == [9]
+    assert flagged([F32, "\ts_nop 7", "\ts_nop 1", read.format(r=1)]) == []
+    assert flagged([K32.format(c="0"), read.format(r=12)]) == []
+
+
+def test_scanner_flags_a_result_used_too_early_behind_a_branch():
+    """The compiler counts the wait states along one way into a block, not along the shortest: one instruction (the branch) in
+    between read garbage on MI355X.  A branch is one state like any instruction."""
+    def code(between, behind, first=K32.format(c="0")):
+        return [first] + between + ["\ts_cbranch_vccnz .LBB0_2", "\ts_branch .LBB0_1", ".LBB0_1:", "\ts_nop 7", "\ts_nop 7", ".LBB0_2:"] + behind
     read = "\tv_mul_f32_e32 v40, v41, v{r}"
     assert [h[4] for h in flagged(code([], [read.format(r=0)]))] == [1]
     assert [h[4] for h in flagged(code([], ["\tds_write_b32 v9, v3"]))] == [1]
     assert [h[4] for h in flagged(code([], ["\tv_mov_b32_e32 v2, 0"]))] == [1]  # a write is overtaken as well
-    assert flagged(code(["\ts_add_i32 s0, s1, s2"], [read.format(r=0)])) == []
-    assert flagged(code([], ["\ts_nop 4", read.format(r=0)])) == []
+    assert [h[4] for h in flagged(code(["\ts_add_i32 s0, s1, s2"], [read.format(r=0)]))] == [2]
+    assert [h[4] for h in flagged(code([], ["\ts_nop 5", read.format(r=0)]))] == [7]
+    assert flagged(code([], ["\ts_nop 6", read.format(r=0)])) == []
+    assert flagged(code(["\ts_nop 6"], [read.format(r=0)])) == []
+    assert [h[4] for h in flagged(code(["\ts_nop 7"], [read.format(r=0)], F32))] == [9]
+    assert flagged(code(["\ts_nop 7", "\ts_nop 0"], [read.format(r=0)], F32)) == []
     assert flagged(code([], [read.format(r=12)])) == []
-    # straight code, and code behind a branch that is always taken, which the text order does not reach
-    assert [h[4] for h in flagged([K32.format(c="0"), "\ts_nop 2", read.format(r=1)])] == [3]
-    assert flagged([K32.format(c="0"), "\ts_nop 3", "\ts_nop 0", read.format(r=1)]) == []
+    # matrix instructions: the result as SrcA or SrcB, or written over by another opcode; not as the same opcode's accumulator
+    assert [h[4] for h in flagged(code([], ["\tv_mfma_f32_16x16x32_bf16 v[20:23], v[0:3], v[4:7], 0"]))] == [1]
+    assert [h[4] for h in flagged(code([], ["\tv_mfma_f32_16x16x4_f32 v[20:23], v30, v0, v[20:23]"]))] == [1]
+    assert [h[4] for h in flagged(code([], [K16.format(d="v[2:5]", c="0")]))] == [1]
+    assert flagged(code([], [K32.format(c="v[0:3]")])) == []
+    assert flagged(code([], ["\ts_nop 6", "\tv_mfma_f32_16x16x32_bf16 v[20:23], v[0:3], v[4:7], 0"])) == []
+    # a branch behind the branch, and code behind a branch that is always taken, which the text order does not reach
+    far = [K32.format(c="0"), "\ts_cbranch_scc1 .LBB0_1", "\ts_nop 7", ".LBB0_1:", "\ts_cbranch_vccz .LBB0_2", "\ts_nop 7", ".LBB0_2:"]
+    assert [h[4] for h in flagged(far + [read.format(r=0)])] == [2]
+    assert flagged(far + ["\ts_nop 5", read.format(r=0)]) == []
     assert flagged([K32.format(c="0"), "\ts_branch .LBB0_9", read.format(r=1), ".LBB0_9:", "\ts_endpgm"]) == []

@@ -155,6 +155,22 @@ __device__ __forceinline__ int held(int x) {
   return x;
 }
 
+// In front of a branch behind which the results x ... are read or written over: the wait states that the compiler keeps between a
+// matrix instruction and such a use, of which it loses count behind a branch (isa_check.py).  Eight, for bf16 operands.
+__device__ __forceinline__ void settle() { asm volatile("s_nop 7"); }
+template <class V, class... Rest>
+__device__ __forceinline__ void settle(V& x, Rest&... rest) {
+  asm volatile("" : "+v"(x));
+  settle(rest...);
+}
+// Ten, behind v_mfma_f32_16x16x4_f32.
+__device__ __forceinline__ void settle_f32() { asm volatile("s_nop 7\n\ts_nop 1"); }
+template <class V, class... Rest>
+__device__ __forceinline__ void settle_f32(V& x, Rest&... rest) {
+  asm volatile("" : "+v"(x));
+  settle_f32(rest...);
+}
+
 // Workgroup barrier for LDS exchanges only: waits for this wave's LDS traffic, not for the
 // global prefetches in flight (a full __syncthreads() would drain those every mini-batch).
 __device__ __forceinline__ void lds_barrier() {

@@ -804,7 +804,10 @@ __global__ void __launch_bounds__(64 * NW, (D <= 64 && D / 16 == NW && (PK || si
     for (int jj = 0; jj < TPW; ++jj) {
       if constexpr (!TDB) IO::mma2(dbT[jj], Zd[jj], Z1d[jj], ones, ones);
     }
-    if constexpr (!FM) single_wave_outputs();
+    if constexpr (!FM) {
+      if constexpr (!BF && D == 64 && TPW == 2) settle_f32(dbT[0], dbT[1]);
+      single_wave_outputs();
+    }
     // FM: the state entering the next mini-batch of the scan.  Placed last: its short dependent chain (transposes,
     // products, conversions, LDS writes) then runs behind the state-gradient products instead of in front of the
     // dXK products and stores (measured 479 -> 463 us).  Behind the first mini-batch of the sequence nothing new is

@@ -733,6 +733,7 @@ __global__ void __launch_bounds__(64 * (D / 16 + 1)) ttt_linear_bwd_pair_kernel(
           Wn[J] = *reinterpret_cast<const f32x4*>(sl + L::C_W + (w * NT + J) * 1024) - mrowo;
       }
       mma_all(dK, Wn, Z1fa);
+      if constexpr (D == 32) settle_f32(dK);  // (a wider head's next use of the registers is further away)
       if (tok_ok) store_own(a.d_xk, tokoff, dK);
     }
     // ---- d lr (first wave), d token_eta (last wave)

@@ -654,6 +654,7 @@ __device__ __forceinline__ void linear_fwd_sk_body(const LinearFwdArgs& a, const
           uu[jj] = bet[jj] - (IO::to_f32(cur.vo[jj]) - IO::to_f32(cur.ko[jj]));
         }
       }
+      if constexpr (FORM && NT == 2) settle(kd[0], kd[1]);
       // ---- checkpoint of the state entering this mini-batch (W and b change only behind the barrier);
       // placed at the barrier so that its branch does not cut the stretch in two
       if (CKPT && ck.due()) {
@@ -668,11 +669,10 @@ __device__ __forceinline__ void linear_fwd_sk_body(const LinearFwdArgs& a, const
       if constexpr (CKPT) ck.next_stage();
       // (without checkpoints the stretch is cut here all the same: as one, 208.5 us instead of 206)
       if constexpr (!CKPT && !ADAM) __builtin_amdgcn_sched_barrier(0);
-      // The compiler does not count the wait states between a matrix instruction and a read of its result behind a branch,
-      // and so few instructions are left in between that the read comes too early (isa_check.py).
+      // The wait states of settle() for what the sums read, but behind the branch, which counts as one of them
       if constexpr (BF && !ADAM) {
-        if constexpr (TPW == 1) asm volatile("s_nop 4" : "+v"(z1[0]), "+v"(uu[0]));
-        else asm volatile("s_nop 4" : "+v"(z1[0]), "+v"(uu[0]), "+v"(z1[1]), "+v"(uu[1]));
+        if constexpr (TPW == 1) asm volatile("s_nop 5" : "+v"(z1[0]), "+v"(uu[0]));
+        else asm volatile("s_nop 5" : "+v"(z1[0]), "+v"(uu[0]), "+v"(z1[1]), "+v"(uu[1]));
       }
       // ---- row sums: six raw moments of Z1 (this mini-batch), two of the pending Zbar
       float S[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, ps0, ps1};  // the pending Zbar's in-lane sums are ready

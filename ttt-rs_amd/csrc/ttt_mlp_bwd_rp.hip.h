@@ -527,6 +527,11 @@ __device__ __forceinline__ void producer(const MlpBwdRpArgs& a, unsigned char* s
       for (int I = 0; I < NT; ++I) IO::mma(W2c[j][I], nx, x.GS[I * 64 + lane]);
       RP_FENCE();
     }
+    if constexpr (D < 96) {  // (d = 96: more instructions of the loop above lie behind the first products than the states)
+#pragma unroll
+      for (int I = 0; I < NT; ++I) asm volatile("" : "+v"(W2c[HT - 1][I]));
+      settle();
+    }
     if (red) IO::mma(b2T, upd ? neg(x.GS[w * 64 + lane]) : IO::zero(), x.ones);
 #pragma unroll
     for (int I = 0; I < NT; ++I) {
