@@ -187,64 +187,75 @@ __device__ __forceinline__ void load_state_slice(f32x4 (&W)[D / 16][TPW], const 
 // 16-byte aligned.  Ends with a workgroup barrier.  sum_a receives the sum of gamma^2 of the head, in every lane.
 // Both sums over the features go in one chain each from LDS, where the lanes put b0 and gamma: read from memory in the chain,
 // sixteen at a time, they were 2 d / 16 round trips one after the other.
-constexpr int kCentreBarriers = 3;  // of centre_state, for a wave that takes no part in it
-template <int D, int NW, int TPW>
+// WORK = false: a wave that takes no part (the control wave of the forward kernel) goes through the same barriers and does nothing
+// else; it does not wait for its copies in flight there.
+template <int D, int NW, int TPW, bool WORK = true>
 __device__ __forceinline__ void centre_state(f32x4 (&Wc)[D / 16][TPW], f32x4 (&bT)[TPW], const float* b0, float* m0s,
                                              const float* gamma, float& sum_a, float* xch, int w, int c, int g) {
   constexpr int NT = D / 16;
   float* const bg = xch + NW * D;
-  for (int i = threadIdx.x; i < D; i += 64 * NW) {
-    bg[i] = b0[i];
-    bg[D + i] = gamma[i];
-  }
-#pragma unroll
-  for (int I = 0; I < NT; ++I)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      float p = 0.f;
-#pragma unroll
-      for (int jj = 0; jj < TPW; ++jj) p += Wc[I][jj][r];
-      p = row16_sum_dpp(p);
-      if (c == 0) xch[(I * 16 + 4 * g + r) * NW + w] = p;
+  const auto barrier = []() {
+    if constexpr (WORK) __syncthreads();
+    else asm volatile("s_barrier" ::: "memory");
+  };
+  if constexpr (WORK) {
+    for (int i = threadIdx.x; i < D; i += 64 * NW) {
+      bg[i] = b0[i];
+      bg[D + i] = gamma[i];
     }
-  __syncthreads();
-  for (int i = threadIdx.x; i < D; i += 64 * NW) {
-    float s = 0.f;
 #pragma unroll
-    for (int ww = 0; ww < NW; ++ww) s += xch[i * NW + ww];
-    m0s[i] = s * (1.0f / D);
+    for (int I = 0; I < NT; ++I)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        float p = 0.f;
+#pragma unroll
+        for (int jj = 0; jj < TPW; ++jj) p += Wc[I][jj][r];
+        p = row16_sum_dpp(p);
+        if (c == 0) xch[(I * 16 + 4 * g + r) * NW + w] = p;
+      }
   }
-  if (threadIdx.x == 64 * (NW - 1)) {  // (the row means are the first wave's)
-    float s = 0.f, sa = 0.f;
+  barrier();
+  if constexpr (WORK) {
+    for (int i = threadIdx.x; i < D; i += 64 * NW) {
+      float s = 0.f;
+#pragma unroll
+      for (int ww = 0; ww < NW; ++ww) s += xch[i * NW + ww];
+      m0s[i] = s * (1.0f / D);
+    }
+    if (threadIdx.x == 64 * (NW - 1)) {  // (the row means are the first wave's)
+      float s = 0.f, sa = 0.f;
 #pragma unroll 1
-    for (int f = 0; f < D; f += 32) {
-      f32x4 b[8], ga[8];
+      for (int f = 0; f < D; f += 32) {
+        f32x4 b[8], ga[8];
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        b[i] = *reinterpret_cast<const f32x4*>(bg + f + 4 * i);
-        ga[i] = *reinterpret_cast<const f32x4*>(bg + D + f + 4 * i);
-      }
+        for (int i = 0; i < 8; ++i) {
+          b[i] = *reinterpret_cast<const f32x4*>(bg + f + 4 * i);
+          ga[i] = *reinterpret_cast<const f32x4*>(bg + D + f + 4 * i);
+        }
 #pragma unroll
-      for (int i = 0; i < 32; ++i) {
-        s += b[i >> 2][i & 3];
-        sa += ga[i >> 2][i & 3] * ga[i >> 2][i & 3];
+        for (int i = 0; i < 32; ++i) {
+          s += b[i >> 2][i & 3];
+          sa += ga[i >> 2][i & 3] * ga[i >> 2][i & 3];
+        }
       }
+      m0s[D] = s * (1.0f / D);
+      m0s[D + 1] = sa;
     }
-    m0s[D] = s * (1.0f / D);
-    m0s[D + 1] = sa;
   }
-  __syncthreads();
+  barrier();
+  if constexpr (WORK) {
 #pragma unroll
-  for (int I = 0; I < NT; ++I) {
-    const f32x4 m = *reinterpret_cast<const f32x4*>(m0s + I * 16 + 4 * g);
+    for (int I = 0; I < NT; ++I) {
+      const f32x4 m = *reinterpret_cast<const f32x4*>(m0s + I * 16 + 4 * g);
 #pragma unroll
-    for (int jj = 0; jj < TPW; ++jj) Wc[I][jj] -= m;
+      for (int jj = 0; jj < TPW; ++jj) Wc[I][jj] -= m;
+    }
+    const float bb = m0s[D];
+#pragma unroll
+    for (int jj = 0; jj < TPW; ++jj) bT[jj] -= bb;
+    sum_a = m0s[D + 1];
   }
-  const float bb = m0s[D];
-#pragma unroll
-  for (int jj = 0; jj < TPW; ++jj) bT[jj] -= bb;
-  sum_a = m0s[D + 1];
-  __syncthreads();
+  barrier();
 }
 
 // The state as f32 row-major matrices from the centred registers (checkpoints): W = Wc + m 1^T, b = bc + mean(b).

@@ -552,8 +552,7 @@ __device__ __forceinline__ void linear_fwd_sk_body(const LinearFwdArgs& a, const
       };
 #pragma unroll
       for (int u = 0; u < RS; ++u) copy_in(u);
-#pragma unroll
-      for (int i = 0; i < kCentreBarriers; ++i) asm volatile("s_barrier" ::: "memory");  // the compute waves centre the state
+      centre_state<D, NW, TPW, false>(Wc, bT, a.b0 + sb * D, m0s, a.gamma + h * D, sum_a, &ex[0][0], w, c, g);  // (the others do)
       asm volatile("s_waitcnt vmcnt(%0)" ::"n"((RS - 1) * kCopies) : "memory");  // mini-batch 0 has landed
       asm volatile("s_barrier" ::: "memory");
       for (int st = 0; st < n_stages_; ++st) {
