@@ -25,12 +25,12 @@
 //
 // What bounds it.  Phases A and D (the products) by the issue of a SIMD's two waves: matrix instructions and vector
 // instructions of 16x16 tiles hardly overlap, not across waves either (probe: a matrix instruction and three FMAs, two
-// waves, 23.3 cycles against 16 + 7.5).  Phases B and C by latency.  Cycles of a mini-batch at d = 96 and 128 units,
-// before -> after the revision before last: A 4.9 -> 4.7 k (XQ W1 now shares the operands of XK W1), B 2.9 -> 2.0 k, C 2.2 -> 1.3 k
-// (sums by lane group), D 7.4 -> 6.4 k (independent products side by side, transposes read from LDS).  The last one took the
-// output out of B (three tiles of sums by two waves were its longest path, 2.1 k) and D, the staging copies from the younger
-// waves and a load of eps through the scalar cache from C.  8 x 16 units x 2048 tokens: d = 96 840 -> 661 -> 640 us, d = 64 488 -> 428 ->
-// 416, d = 32 286 -> 260 -> 247; saving d = 96 715 -> 687, d = 64 467 -> 444, d = 32 284 -> 270.
+// waves, 23.3 cycles against 16 + 7.5).  Phases B and C by latency.  Cycles of a mini-batch at d = 96 and 128 units:
+// XQ W1 sharing the operands of XK W1 took A from 4.9 to 4.7 k, sums by lane group B from 2.9 to 2.0 k and C from 2.2 to 1.3 k,
+// independent products side by side and transposes read from LDS D from 7.4 to 6.4 k: 8 x 16 units x 2048 tokens, d = 96 840 -> 661 us,
+// d = 64 488 -> 428, d = 32 286 -> 260.  The output taken out of B (three tiles of sums by two waves were its longest path, 2.1 k) and
+// D, the staging copies from the younger waves, a load of eps through the scalar cache from C and the sums of the prologue from
+// one load each: 636, 413, 247; saving d = 96 715 -> 674, d = 64 467 -> 444, d = 32 284 -> 270.
 //
 // An odd hidden tile at the end of a split-k chain is issued as a k = 32 MFMA with a zero second
 // half, not as a k = 16 one: a 16x16x16 bf16 MFMA accumulating straight onto the result of a

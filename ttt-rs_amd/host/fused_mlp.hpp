@@ -195,7 +195,8 @@ class FusedMlp {
 class LostWorkgroupGuard {
  public:
   LostWorkgroupGuard() { check(ttt_mlp_fwd_lost_workgroups(&before_)); }
-  /// Throws if the word moved since construction: the outputs of the affected units are NaN.
+  /// Throws if the word moved since construction: the outputs of the affected units are NaN (unless it was a ttt_mlpn_fwd on the
+  /// same device whose workgroups waited in vain: those units are computed again, and only this word says so).
   void verify() const {
     std::int64_t now = 0;
     check(ttt_mlp_fwd_lost_workgroups(&now));

@@ -112,7 +112,9 @@ struct TTTMLPNState {
   }
 };
 
-/// TTT-MLP with 2, 3 or 4 hidden layers of width 4 d on the fused kernel (ttt_mlpn_fwd).
+/// TTT-MLP with 2, 3 or 4 hidden layers of width 4 d on the fused kernel (ttt_mlpn_fwd).  The next_ weights carry what two
+/// workgroups of a unit hand over during a call: ordinary device memory, or TTT_HINT_ONE_WORKGROUP in config.ttt.kernel_hint.  No
+/// LostWorkgroupGuard is needed: a unit whose workgroups waited in vain is computed again.
 class FusedMlpN {
  public:
   /// weight_init[i] [H,in_i,out_i], bias_init[i] [H,out_i] for the n_hidden + 1 layers (device pointers, f32).
