@@ -116,12 +116,13 @@ typedef struct ttt_desc {
 #define TTT_HINT_F32_PRODUCTS 0x4000
 /* ttt_mlp_bwd and its variants: with at most 128 (batch, head) units every unit is worked on by two workgroups on two
  * CUs (see ttt_mlp_bwd); TTT_HINT_ONE_WORKGROUP keeps a unit on one.  Same results bit for bit (d_token_eta, which
- * is summed over the units with atomic additions, aside); the workspace is smaller.  ttt_mlpn_fwd: likewise. */
+ * is summed over the units with atomic additions, aside); the workspace is smaller.  ttt_mlpn_fwd, and ttt_linear_fwd with f32
+ * I/O at head_dim 32 / 64 (see there): likewise. */
 #define TTT_HINT_ONE_WORKGROUP 0x8000
 /* Testing only: the two workgroups that share a (batch, head) unit in ttt_mlp_fwd at head_dim 128 (bf16 I/O) give
  * up waiting for each other at once, as if the partner had never become resident.  Exercises the failure path
- * described at ttt_mlp_fwd: every output of the affected units is NaN.  All kernels still run to their end.  (ttt_mlpn_fwd:
- * likewise, and the units are computed again.) */
+ * described at ttt_mlp_fwd: every output of the affected units is NaN.  All kernels still run to their end.  (ttt_mlpn_fwd and
+ * ttt_linear_fwd: likewise, and the units are computed again.) */
 #define TTT_HINT_TEST_LOST_PARTNER 0x200
 /* Testing only: the same two workgroups treat each other as running on different XCDs whatever they find at start,
  * i.e. take the path of a pair that was not placed on one XCD: every word they exchange is stored at device scope
@@ -169,6 +170,10 @@ int ttt_linear_best_checkpoint_format(const ttt_desc* desc);
  *  W_ckpt [B,H,C,d,d] f32, b_ckpt [B,H,C,d] f32 with C = ttt_linear_num_checkpoints();
  *  both may be NULL (no checkpoints written).  Checkpoint c holds the state ENTERING
  *  stage c*checkpoint_interval (forward/kernel.rs:143-150).
+ * f32 I/O at head_dim 32 / 64, mini_batch 16, 16 or more mini-batches: where the device has two CUs per (batch, head) unit, a
+ * unit runs on two workgroups, unless an output overlaps an input or another output (the same results bit for bit;
+ * TTT_HINT_ONE_WORKGROUP keeps it on one).  During the call `out` and W_out then also carry what crosses between the two; a
+ * unit whose second workgroup waited for the first in vain is computed again behind them.
  */
 int ttt_linear_fwd(const ttt_desc* desc, const void* xq, const void* xk, const void* xv,
                    const float* W0, const float* b0, const float* token_eta, const void* lr,

@@ -19,6 +19,7 @@
 #include "ttt_linear_bwd_rr.hip.h"
 #include "ttt_linear_fwd.hip.h"
 #include "ttt_linear_fwd_mw.hip.h"
+#include "ttt_linear_fwd_pair.hip.h"
 #include "ttt_linear_fwd_sk.hip.h"
 #include "ttt_mlp_bwd.hip.h"
 #include "ttt_mlp_bwd_rp.hip.h"
@@ -987,6 +988,45 @@ int dispatch_linear_fwd_pack(const ttt_desc* d, const ttt::LinearFwdArgs* a, uns
   return f32 ? launch_linear_fwd_wide<ttt::F32, 128>(a, ny, s) : launch_linear_fwd_wide<ttt::BF16, 128>(a, ny, s);
 }
 
+// Whether a unit of ttt_linear_fwd runs on two workgroups (see ttt_linear_fwd_pair.hip.h).  What crosses between them lies in the rows
+// of `out` and in W_out, and a unit whose workgroups did not find each other is done again from its inputs: outputs that
+// overlap an input or each other stay with one workgroup.  Both workgroups need a CU each, in groups of eight.  The launches that
+// clear the words and look for units to do again, and the consumer's last output behind the producer's last G'', cost 4 - 5 us:
+// on one / two workgroups, d = 64, 24 units, 8 mini-batches 17.9 / 18.6 us, 12 23.6 / 22.8, 16 29.9 / 27.1, 63 102 / 76, 128 202 / 144;
+// 128 units, 12 24.8 / 24.4, 16 31.0 / 28.7; d = 32, 24 units, 12 17.1 / 17.4, 16 21.4 / 20.4, 63 72.6 / 56.5, 128 143.5 / 105.5.
+bool linear_fwd_on_pairs(const ttt_desc* d, const ttt::LinearFwdArgs& a, ttt::LinearPairArgs* pa) {
+  if (d->io_dtype != TTT_F32 || d->head_dim > 64 || a.K != 16) return false;
+  if (d->kernel_hint & (TTT_HINT_WAVES_MASK | TTT_HINT_ALL_LOADS | TTT_HINT_ONE_WORKGROUP)) return false;
+  if (a.n_stages < 16) return false;
+  const size_t units = (size_t)a.B * a.H;
+  int cus = 0;
+  if (device_cus(&cus) != TTT_OK || (units + 7) / 8 * 16 > (size_t)cus) return false;
+  const size_t D = (size_t)d->head_dim, tokens = (units - 1) * a.seq_stride + d->seq, states = d->state_per_batch ? units : (size_t)a.H;
+  const size_t saved = a.W_ckpt != nullptr ? units * a.n_ckpt : 0;
+  struct Range {
+    const void* p;
+    size_t n;
+  };
+  const Range in[] = {{a.xq, tokens * D * 4}, {a.xk, tokens * D * 4}, {a.xv, tokens * D * 4}, {a.lr, tokens * 4}, {a.token_eta, 64},
+                      {a.W0, states * D * D * 4}, {a.b0, states * D * 4}, {a.gamma, a.H * D * 4}, {a.beta, a.H * D * 4}};
+  const Range res[] = {{a.out, tokens * D * 4}, {a.W_out, units * D * D * 4}, {a.b_out, units * D * 4}, {a.W_ckpt, saved * D * D * 4},
+                       {a.b_ckpt, saved * D * 4}};
+  const auto apart = [](const Range& x, const Range& y) {
+    const uintptr_t p = (uintptr_t)x.p, q = (uintptr_t)y.p;
+    return p + x.n <= q || q + y.n <= p;
+  };
+  for (const Range& r : res) {
+    if (r.n == 0) continue;
+    for (const Range& i : in)
+      if (!apart(r, i)) return false;
+    for (const Range& o : res)
+      if (&o != &r && o.n != 0 && !apart(r, o)) return false;
+  }
+  pa->spin_limit = (d->kernel_hint & TTT_HINT_TEST_LOST_PARTNER) ? 0u : 1u << 21;
+  pa->agent_release = (d->kernel_hint & TTT_HINT_TEST_OTHER_XCD) ? 1 : 0;
+  return true;
+}
+
 // n problems of one shape: kMaxProblems per launch
 int dispatch_linear_fwd(const ttt_desc* d, const ttt::LinearFwdArgs* probs, int n, hipStream_t s) {
   for (int p = 0; p < n; p += ttt::kMaxProblems) {
@@ -1007,6 +1047,9 @@ int ttt_linear_fwd(const ttt_desc* d, const void* xq, const void* xk, const void
   ttt::LinearFwdArgs a;
   int rc = prepare_linear_fwd(d, xq, xk, xv, W0, b0, token_eta, lr, gamma, beta, out, W_out, b_out, W_ckpt, b_ckpt, &a);
   if (rc != TTT_OK) return rc;
+  ttt::LinearPairArgs pa;
+  if (linear_fwd_on_pairs(d, a, &pa))
+    return hip_status(ttt::launch_linear_fwd_pair(d->head_dim, a, pa, static_cast<hipStream_t>(stream)), "ttt_linear_fwd launch");
   return dispatch_linear_fwd(d, &a, 1, static_cast<hipStream_t>(stream));
 }
 

@@ -233,6 +233,17 @@ __device__ __forceinline__ void lds_dma16(const void* base, unsigned lane_off, u
       : "v"(lane_off), "s"(uniform_ptr(base)), "s"(lds_base)
       : "memory");
 }
+// lds_dma16 with a device-scope load (sc1): the load does not look in the CU's vector cache, so it sees what another
+// CU behind the same L2 stored and had acknowledged, without the cache being dropped first.
+__device__ __forceinline__ void lds_dma16_dev(const void* base, unsigned lane_off, unsigned lds_base) {
+  unsigned saved;
+  asm volatile(
+      "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 sc1\n\ts_nop 0\n\ts_mov_b32 m0, %0"
+      : "=&s"(saved)
+      : "v"(lane_off), "s"(uniform_ptr(base)), "s"(lds_base)
+      : "memory");
+}
+
 // One 2-byte element per lane, zero-extended to a dword at lds_base + 4 * lane.
 __device__ __forceinline__ void lds_dma2(const void* src, unsigned lds_base) {
   unsigned saved;

@@ -41,17 +41,6 @@
 
 namespace ttt {
 
-// lds_dma16 with a device-scope load (sc1): the load does not look in the CU's vector cache, so it sees what another
-// CU behind the same L2 stored and had acknowledged, without the cache being dropped first.
-__device__ __forceinline__ void lds_dma16_dev(const void* base, unsigned lane_off, unsigned lds_base) {
-  unsigned saved;
-  asm volatile(
-      "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 sc1\n\ts_nop 0\n\ts_mov_b32 m0, %0"
-      : "=&s"(saved)
-      : "v"(lane_off), "s"(uniform_ptr(base)), "s"(lds_base)
-      : "memory");
-}
-
 // lds_dma16 with a non-temporal load: for rows that nothing reads again (the producer's xv and d_out, everything the
 // consumer takes from the inputs, which the producer has read before it).  Lines brought in this way do not push the
 // hand-over slots out of the L2, where they are meant to stay between their store and their one read: 170 MB per

@@ -1,0 +1,400 @@
+// TTT-Linear forward with f32 I/O, a (batch, head) unit on two workgroups on two CUs (head_dim 32 / 64, mini-batches of 16).
+//
+// The f32 matrix instructions bound the kernel with one workgroup per unit (ttt_linear_fwd_dma_kernel): 68 of 32 cycles per
+// wave and mini-batch at head_dim 64, 24 of them for the output, of which nothing is needed for the state.  Here a PRODUCER
+// runs the recurrence alone (44 instructions) and hands G'' of every mini-batch to a CONSUMER on a second CU, which follows with
+// the same updates on a state of its own and forms the output (44).  Nothing flows back: the producer waits for nobody.
+//
+// G'' of a mini-batch [16 x d] is as large as that mini-batch's rows of `out`, which nobody reads before the consumer writes
+// them: it is handed over there, in register layout, so there is no ring to run full.  One word per unit, in W_out, says how many
+// mini-batches have been handed over; the consumer writes the final state over it at the end.  The producer's stores stay in the
+// L2 that both share (the consumer publishes its XCD number) or are written back by a device-scope release while that is not
+// known; the consumer loads at device scope.  The consumer's wait is bounded: if it was in vain it runs to its end without
+// waiting and marks the unit in W_out, and a launch of the one-workgroup form behind the pair's does the marked units
+// again, from inputs that no output overlaps (the caller's rule).
+//
+// Beside its NW = d / 16 compute waves a workgroup has two that only move data, so that the compute waves issue no global load and,
+// in the producer, no store but checkpoints: one copies rows global -> LDS (as in ttt_linear_fwd_dma_kernel), the
+// COURIER stores G'' and the word, or watches the word and copies G'' global -> LDS.  One barrier per mini-batch.
+//
+// The arithmetic is that of one workgroup, bit for bit.
+#pragma once
+#include "ttt_linear_fwd_sk.hip.h"
+
+namespace ttt {
+
+struct LinearPairArgs {
+  unsigned spin_limit;  // polls before the consumer gives up; 0: at once (tests of that path)
+  int agent_release;    // 1: always publish with a device-scope release
+};
+// words of the last 64 floats of a unit's W_out, and the mark in its first (a final state that comes to have these bits by
+// itself costs a computation, not the result)
+constexpr int kLinPairWords = 64, kLinPairCount = 0, kLinPairXcd = 32;
+constexpr unsigned kLinPairLost = 0x7fc60b5fu;
+
+template <int D>
+struct LinearPairLds {
+  static constexpr int NT = D / 16, RS = 4;
+  f32x4 rows[RS][2][NT][64];  // producer: xk, xv; consumer: xq, xk
+  f32x4 g[RS][NT][64];        // G'' with tokens along k: on its way out (two slots) or in
+  f32x4 kd[2][NT][64];        // XK with tokens along k
+  f32x4 at[2][NT][64];        // consumer: a wave's share of the attention block
+  float lr[RS][64];
+  __attribute__((aligned(16))) float ex[2][8 * 16 * NT];
+  __attribute__((aligned(16))) float m0s[D + 4];
+  int lost;
+};
+
+template <class V>
+__device__ __forceinline__ unsigned lds_addr(const V* p) {
+  return (unsigned)(size_t)(const __attribute__((address_space(3))) V*)p;
+}
+
+template <int D, bool PRODUCER, bool CKPT>
+__device__ __forceinline__ void linear_fwd_pair_body(const LinearFwdArgs& a, const LinearPairArgs& pa, LinearPairLds<D>& L, size_t bh) {
+  using IO = Io<F32>;
+  constexpr int NT = D / 16, NW = NT, RS = LinearPairLds<D>::RS;
+  constexpr float inv_d = 1.0f / D;
+  constexpr int K = 16;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int w = wave % NW, c = lane & 15, g = lane >> 4;  // (the two other waves do what a compute wave does up to where they branch off)
+  const int h = (int)(bh % a.H), n = a.n_stages;
+  const UnitBase<F32, D> ub(a, bh);
+  unsigned* const words = reinterpret_cast<unsigned*>(a.W_out + bh * D * D + (D * D - kLinPairWords));
+
+  if (wave >= NW) {
+    float sum_a;
+    f32x4 Wn[NT][1], bn[1];
+    const auto centre = [&]() { centre_state<D, NW, 1, false>(Wn, bn, a.b0, L.m0s, a.gamma, sum_a, &L.ex[0][0], w, c, g); };
+    if (wave == NW) {  // rows: mini-batch st + RS behind the barrier of mini-batch st
+      constexpr int kCopies = 2 * NT + (PRODUCER ? 1 : 0);
+      const unsigned rows0 = lds_addr(&L.rows[0][0][0][0]), lr0 = lds_addr(&L.lr[0][0]);
+      const auto copy_in = [&](int stage) {  // (past the end: the last one again, into a slot nobody reads)
+        const unsigned slot = (unsigned)(stage & (RS - 1)), dst = rows0 + slot * (2 * NT * 1024);
+        const int st_ld = min(stage, n - 1);
+        const unsigned off = UnitBase<F32, D>::row_off(st_ld, K, c);
+#pragma unroll
+        for (int J = 0; J < NT; ++J) {
+          const unsigned fo = (unsigned)(32 * (J >> 1) + 8 * g + 4 * (J & 1)) * 4u;  // the lane's four features of tile J
+          lds_dma16(PRODUCER ? ub.xk : ub.xq, off + fo, dst + J * 1024);
+          lds_dma16(PRODUCER ? ub.xv : ub.xk, off + fo, dst + (NT + J) * 1024);
+        }
+        if constexpr (PRODUCER) lds_dma4(ub.lr, ((unsigned)st_ld * (unsigned)K + (unsigned)c) * 4u, lr0 + slot * 256u);
+      };
+#pragma unroll
+      for (int u = 0; u < RS; ++u) copy_in(u);
+      centre();
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"((RS - 1) * kCopies) : "memory");  // mini-batch 0 has landed
+      asm volatile("s_barrier" ::: "memory");
+      for (int st = 0; st < n; ++st) {
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"((RS - 2) * kCopies) : "memory");  // mini-batch st + 1 has landed
+        asm volatile("s_barrier" ::: "memory");
+        copy_in(st + RS);
+      }
+      asm volatile("s_barrier" ::: "memory");
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      return;
+    }
+    // the courier
+    const auto look = [&](const unsigned* p) {
+      return (unsigned)__builtin_amdgcn_readfirstlane((int)__hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+    };
+    unsigned xcd;
+    asm volatile("s_getreg_b32 %0, hwreg(HW_REG_XCC_ID)" : "=s"(xcd));
+    xcd = 0x100u | (xcd & 15u);
+    const unsigned lane16 = (unsigned)lane * 16u;
+    if constexpr (PRODUCER) {
+      bool fast = false;  // the consumer is known to sit behind the same L2
+      const auto hand_over = [&](int st) {
+#pragma unroll
+        for (int J = 0; J < NT; ++J)
+          *reinterpret_cast<f32x4*>(ub.out + (unsigned)st * (unsigned)(K * D * 4) + J * 1024 + lane16) = L.g[st & 1][J][lane];
+        if (!fast && pa.agent_release == 0) fast = look(words + kLinPairXcd) == xcd;
+        if (!fast) __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        if (lane == 0) __hip_atomic_store(words + kLinPairCount, (unsigned)(st + 1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      };
+      centre();
+      asm volatile("s_barrier" ::: "memory");
+      // G'' of mini-batch st lies in LDS behind the barrier of st + 1, until behind that of st + 2
+      asm volatile("s_barrier" ::: "memory");
+      for (int st = 1; st <= n; ++st) {
+        asm volatile("s_barrier" ::: "memory");
+        hand_over(st - 1);
+      }
+    } else {
+      if (lane == 0) __hip_atomic_store(words + kLinPairXcd, xcd, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      const unsigned g0 = lds_addr(&L.g[0][0][0]);
+      bool lost = pa.spin_limit == 0;
+      int known = 0, next = 0;  // mini-batches handed over; the next to copy
+      centre();
+      asm volatile("s_barrier" ::: "memory");
+      for (int st = 0; st < n; ++st) {
+        // G'' of mini-batch st in LDS in front of the barrier of st, and of the next two if they are there: the slot of st + 2 was
+        // last read behind the barrier of st - 2, which every wave left in front of that of st - 1
+        if (!lost && known < n) {
+          for (unsigned polls = 0;; ++polls) {
+            known = (int)look(words + kLinPairCount);
+            if (known > st) break;
+            if (polls >= pa.spin_limit) {
+              lost = true;
+              break;
+            }
+            __builtin_amdgcn_s_sleep(1);
+          }
+        }
+        if (!lost) {
+          for (; next < known && next <= st + 2; ++next) {
+#pragma unroll
+            for (int J = 0; J < NT; ++J)
+              lds_dma16_dev(ub.out + (unsigned)next * (unsigned)(K * D * 4), J * 1024u + lane16,
+                            g0 + (unsigned)(next & (RS - 1)) * (NT * 1024) + J * 1024);
+          }
+          asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        }
+        asm volatile("s_barrier" ::: "memory");
+      }
+      if (lane == 0) L.lost = lost ? 1 : 0;
+      lds_done();
+      asm volatile("s_barrier" ::: "memory");
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    return;
+  }
+
+  // ---- compute waves: tile w of the features (the names are those of linear_fwd_sk_body)
+  const float te_last = a.token_eta[K - 1];
+  const bool upd = te_last != 0.f;
+  const float sc = upd ? te_last : 1.f;
+  const float rho_c = a.token_eta[c] / sc;
+  const f32x4 ident = identity_frag<F32>(c, g), ones = splat_frag<F32>(1.f);
+  const f32x4 ident_upd = upd ? ident : IO::zero(), ones_upd = upd ? ones : IO::zero();
+  const size_t sb = a.state_per_batch ? bh : (size_t)h;
+  const float eps = held(a.eps);
+  const int fo = own_offset<1>(w, 0, g);
+  f32x4 gam, bet, a2, bT[1], Wc[NT][1];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    gam[r] = a.gamma[h * D + fo + r];
+    bet[r] = a.beta[h * D + fo + r];
+    bT[0][r] = a.b0[sb * D + fo + r];
+    a2[r] = gam[r] * gam[r];
+  }
+  load_state_slice<D, 1>(Wc, a.W0 + sb * D * D, w, c, g);
+  float sum_a;  // of gamma^2
+  centre_state<D, NW, 1>(Wc, bT, a.b0 + sb * D, L.m0s, a.gamma + h * D, sum_a, &L.ex[0][0], w, c, g);
+  lds_barrier();
+
+  // rows of a mini-batch: full rows of what is multiplied by the state, own features of the others
+  f32x4 x[2][NT], xo[2], yo[2];  // producer: xk, own xk, own xv; consumer: xq, own xq, own xk
+  float lr[2];
+  const auto gather = [&](int u, int stage) {
+    const int sl = stage & (RS - 1);
+#pragma unroll
+    for (int J = 0; J < NT; ++J) x[u][J] = L.rows[sl][0][J][lane];
+    xo[u] = L.rows[sl][0][w][lane];
+    yo[u] = L.rows[sl][1][w][lane];
+    if constexpr (PRODUCER) lr[u] = L.lr[sl][c];
+  };
+  gather(0, 0);
+
+  if constexpr (PRODUCER) {
+    CkptCursor<D> ck(a, bh);
+    const float b_mean = __builtin_amdgcn_readfirstlane(L.m0s[D]);
+    const auto mini_batch = [&](auto u_tag, int st) {
+      constexpr int u = decltype(u_tag)::value;
+      f32x4 t = {0.f, 0.f, 0.f, 0.f};
+      IO::mma(t, xo[u], ident_upd);  // XK with tokens along k, the own tile
+      L.kd[u][w][lane] = t;
+      f32x4 z1 = bT[0];
+#pragma unroll
+      for (int J = 0; J < NT; ++J) IO::mma(z1, Wc[J][0], x[u][J]);
+      const f32x4 uu = bet - (yo[u] - xo[u]);
+      if (CKPT && ck.due()) {
+        if (ck.packed) {
+          store_ckpt_packed<F32, NT, 1>(ck.W, Wc, w, lane);
+          store_bias_true<D, 1>(ck.b, bT, b_mean, w, c, g);
+        } else {
+          store_state_f32<D, 1>(ck.W, ck.b, Wc, bT, L.m0s, w, c, g);
+        }
+        ck.advance();
+      }
+      if constexpr (CKPT) {
+        ck.next_stage();
+        settle_f32(z1);
+      }
+      // the six moments of Z1
+      float S[6];
+      const f32x4 bq = gam * uu;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float az = a2[r] * z1[r];
+        if (r == 0) {
+          S[0] = z1[0];
+          S[2] = az;
+          S[3] = az * z1[0];
+          S[4] = bq[0];
+          S[5] = bq[0] * z1[0];
+        } else {
+          S[0] += z1[r];
+          S[1] = r == 1 ? __builtin_fmaf(z1[0], z1[0], z1[1] * z1[1]) : __builtin_fmaf(z1[r], z1[r], S[1]);
+          S[2] = __builtin_fmaf(a2[r], z1[r], S[2]);
+          S[3] = __builtin_fmaf(az, z1[r], S[3]);
+          S[4] = __builtin_fmaf(gam[r], uu[r], S[4]);
+          S[5] = __builtin_fmaf(bq[r], z1[r], S[5]);
+        }
+      }
+      float* const e = L.ex[u];
+      const float v0 = xg_sum4_scatter(S[0], S[1], S[2], S[3]), v1 = xg_sum2_scatter(S[4], S[5]);
+      e[(g * 16 + c) * NW + w] = v0;
+      if ((g & 1) == 0) e[((4 + (g >> 1)) * 16 + c) * NW + w] = v1;
+      lds_barrier();
+#pragma unroll
+      for (int i = 0; i < 6; ++i) {
+        float s = e[(i * 16 + c) * NW];
+#pragma unroll
+        for (int ww = 1; ww < NW; ++ww) s += e[(i * 16 + c) * NW + ww];
+        S[i] = s;
+      }
+      f32x4 kd[NT];
+#pragma unroll
+      for (int I = 0; I < NT; ++I) kd[I] = L.kd[u][I][lane];
+      gather(u ^ 1, st + 1);
+      const float mu = S[0] * inv_d;
+      const float var = S[1] * inv_d - mu * mu;
+      const float rstd = __builtin_amdgcn_rsqf(fmaxf(var, 0.f) + eps);
+      const float s1 = rstd * (S[2] - mu * sum_a) + S[4];
+      const float m = S[5] - mu * S[4], q = S[3] - 2.f * mu * S[2] + mu * mu * sum_a, r2 = rstd * rstd;
+      const float s2 = __builtin_fmaf(r2, q, rstd * m);
+      const float p = -sc * lr[u] * rstd;
+      const float c1 = p * rstd, c2 = -c1 * s2 * inv_d, c3 = -p * s1 * inv_d;
+      const f32x4 G = (z1 - mu) * (a2 * c1 + c2) + (bq * p + c3);
+      f32x4 Gd = {0.f, 0.f, 0.f, 0.f};
+      IO::mma(Gd, G, ident);
+#pragma unroll
+      for (int I = 0; I < NT; ++I) IO::mma(Wc[I][0], kd[I], Gd);
+      IO::mma(bT[0], Gd, ones_upd);
+      L.g[u][w][lane] = Gd;
+    };
+    int st = 0;
+    for (; st + 2 <= n; st += 2) {
+      mini_batch(std::integral_constant<int, 0>{}, st);
+      mini_batch(std::integral_constant<int, 1>{}, st + 1);
+    }
+    if (st < n) mini_batch(std::integral_constant<int, 0>{}, st);
+    lds_barrier();  // the last G''
+  } else {
+    // pending output of the last mini-batch (its sums travel in the next exchange) and of the one before (sums known)
+    f32x4 zbp = {0.f, 0.f, 0.f, 0.f}, zbo = zbp, qop = zbp, qoo = zbp;
+    float so0 = 0.f, so1 = 0.f;
+    const auto publish = [&](int u) {
+      const float s0 = ((zbp[0] + zbp[1]) + zbp[2]) + zbp[3];
+      const float s1 = __builtin_fmaf(zbp[3], zbp[3], __builtin_fmaf(zbp[2], zbp[2], __builtin_fmaf(zbp[1], zbp[1], zbp[0] * zbp[0])));
+      const float v = xg_sum2_scatter(s0, s1);
+      if ((g & 1) == 0) L.ex[u][((g >> 1) * 16 + c) * NW + w] = v;
+    };
+    const auto collect = [&](int u, float& s0, float& s1) {
+      const float* e = L.ex[u];
+      s0 = e[c * NW];
+      s1 = e[(16 + c) * NW];
+#pragma unroll
+      for (int ww = 1; ww < NW; ++ww) {
+        s0 += e[c * NW + ww];
+        s1 += e[(16 + c) * NW + ww];
+      }
+    };
+    const auto emit = [&](float s0, float s1, int stage, const f32x4& zb, const f32x4& qo) {
+      const float mu = s0 * inv_d;
+      const float rstd = __builtin_amdgcn_rsqf(fmaxf(s1 * inv_d - mu * mu, 0.f) + eps);
+      float* po = reinterpret_cast<float*>(ub.out + UnitBase<F32, D>::row_off(stage, K, c));
+      const f32x4 qb = qo + bet;
+      *reinterpret_cast<f32x4*>(po + fo) = qb + gam * ((zb - mu) * rstd);
+    };
+    const auto mini_batch = [&](auto u_tag, int st) {
+      constexpr int u = decltype(u_tag)::value;
+      f32x4 t = {0.f, 0.f, 0.f, 0.f}, At = {0.f, 0.f, 0.f, 0.f};
+      IO::mma(t, yo[u], ident_upd);
+      IO::mma(At, yo[u], xo[u]);
+      L.kd[u][w][lane] = t;
+      L.at[u][w][lane] = At;
+      f32x4 zb = bT[0];
+#pragma unroll
+      for (int J = 0; J < NT; ++J) IO::mma(zb, Wc[J][0], x[u][J]);
+      publish(u);
+      if (st > 1) emit(so0, so1, st - 2, zbo, qoo);
+      lds_barrier();
+      collect(u, so0, so1);
+      f32x4 kd[NT];
+#pragma unroll
+      for (int I = 0; I < NT; ++I) kd[I] = L.kd[u][I][lane];
+      At = L.at[u][0][lane];
+#pragma unroll
+      for (int ww = 1; ww < NW; ++ww) At += L.at[u][ww][lane];
+      const f32x4 Gd = L.g[st & (RS - 1)][w][lane];
+      gather(u ^ 1, st + 1);
+      zbo = zbp;
+      qoo = qop;
+      f32x4 m;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) m[r] = (4 * g + r <= c) ? rho_c * (1.f + At[r]) : 0.f;
+#pragma unroll
+      for (int I = 0; I < NT; ++I) IO::mma(Wc[I][0], kd[I], Gd);
+      IO::mma(bT[0], Gd, ones_upd);
+      IO::mma(zb, Gd, m);
+      zbp = zb;
+      qop = xo[u];
+    };
+    int st = 0;
+    for (; st + 2 <= n; st += 2) {
+      mini_batch(std::integral_constant<int, 0>{}, st);
+      mini_batch(std::integral_constant<int, 1>{}, st + 1);
+    }
+    if (st < n) mini_batch(std::integral_constant<int, 0>{}, st);
+    f32x4 W0[NT][1];
+    load_state_slice<D, 1>(W0, a.W0 + sb * D * D, w, c, g);
+    publish(n & 1);
+    lds_barrier();
+    float s0, s1;
+    collect(n & 1, s0, s1);
+    if (n >= 2) emit(so0, so1, n - 2, zbo, qoo);
+    emit(s0, s1, n - 1, zbp, qop);
+    store_state_final<D, 1>(a.W_out + bh * D * D, a.b_out + bh * D, W0, a.b0 + sb * D, Wc, bT, L.m0s, w, c, g);
+    // element (0, 0) of W_out is written by the lane that marks the unit
+    if (L.lost != 0 && threadIdx.x == 0) *reinterpret_cast<unsigned*>(a.W_out + bh * D * D) = kLinPairLost;
+  }
+}
+
+// Workgroups b and b + 8 of every 16 share a unit: consecutive workgroups go to the XCDs in turn, so both run behind one L2, and
+// the producer, which waits for nobody, is dispatched first.
+template <int D, bool CKPT>
+__global__ void __launch_bounds__(64 * (D / 16 + 2)) ttt_linear_fwd_pair_kernel(LinearFwdArgs a, LinearPairArgs pa) {
+  __shared__ LinearPairLds<D> L;
+  const size_t bh = (size_t)(blockIdx.x >> 4) * 8 + (blockIdx.x & 7);
+  if (bh >= (size_t)a.B * a.H) return;
+  if (((blockIdx.x >> 3) & 1) == 0)
+    linear_fwd_pair_body<D, true, CKPT>(a, pa, L, bh);
+  else
+    linear_fwd_pair_body<D, false, false>(a, pa, L, bh);
+}
+
+// the word of every unit, and the consumer's XCD number
+template <int D>
+__global__ void ttt_linear_fwd_pair_clear_kernel(float* W_out, int units) {
+  const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+  if (i < units) {
+    float* words = W_out + (size_t)i * D * D + (D * D - kLinPairWords);
+    words[kLinPairCount] = words[kLinPairXcd] = 0.f;
+  }
+}
+
+// the units whose consumer waited in vain, on one workgroup
+template <int D, bool CKPT>
+__global__ void __launch_bounds__(64 * (D / 16 + 1)) ttt_linear_fwd_redo_kernel(LinearFwdArgs a) {
+  const unsigned* mark = reinterpret_cast<const unsigned*>(a.W_out + blockIdx.x * (size_t)(D * D));
+  if (__builtin_amdgcn_readfirstlane((int)*mark) != (int)kLinPairLost) return;
+  linear_fwd_sk_body<F32, D, D / 16, 2, true, false, 5, false, false, false, CKPT>(a, nullptr);
+}
+
+hipError_t launch_linear_fwd_pair(int head_dim, const LinearFwdArgs& a, const LinearPairArgs& pa, hipStream_t s);  // ttt_linear_fwd_pair.hip
+
+}  // namespace ttt

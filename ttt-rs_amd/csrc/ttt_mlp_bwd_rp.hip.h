@@ -168,15 +168,7 @@ __device__ __forceinline__ V& at(const unsigned char* base, unsigned off) {
   return *reinterpret_cast<V*>(const_cast<unsigned char*>(base) + off);
 }
 
-// lds_dma16 and lds_dma4 with device scope (see Slot)
-__device__ __forceinline__ void lds_dma16_dev(const void* base, unsigned lane_off, unsigned lds_base) {
-  unsigned saved;
-  asm volatile(
-      "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 sc1\n\ts_nop 0\n\ts_mov_b32 m0, %0"
-      : "=&s"(saved)
-      : "v"(lane_off), "s"(uniform_ptr(base)), "s"(lds_base)
-      : "memory");
-}
+// lds_dma4 with device scope (see Slot)
 __device__ __forceinline__ void lds_dma4_dev(const void* base, unsigned lane_off, unsigned lds_base) {
   unsigned saved;
   asm volatile(
