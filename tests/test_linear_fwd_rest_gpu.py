@@ -1,0 +1,102 @@
+"""ttt_linear_fwd_with_rest: the whole mini-batches of a sequence and the short one behind them in one launch, against the two
+launches it takes the place of.  The state between the two is centred anew in the second launch, one f32 rounding of
+every element: outputs may differ by a few of those (2^-24), carried through one mini-batch, 1e-5 of the largest value at most.
+Where the consumer waits in vain the units are computed as the two launches would: the same bits."""
+import ctypes
+import importlib
+
+import pytest
+import torch
+
+from helpers import to_dev
+
+pytestmark = pytest.mark.gpu
+
+ONE, LOST, OTHER_XCD = 0x8000, 0x200, 0x800
+K = 16
+
+
+@pytest.fixture(scope="module")
+def P():
+    return importlib.import_module("ttt-rs_amd")
+
+
+def inputs(P, d, B, H, N, rest):
+    seq = N * K + rest
+    v = to_dev(P.synthetic.reference_test_inputs(5500 + d + N + rest, B, H, (N + 1) * K, d, K, io_dtype=torch.float32))
+    for k in ("xq", "xk", "xv", "lr"):
+        v[k] = v[k][:, :, :seq].contiguous()
+    te = v["token_eta"]
+    v["token_eta"] = torch.cat([te[:K].repeat(N), te[:rest] * 1.25]).contiguous()
+    return v
+
+
+def run(P, v, d, B, H, N, rest, hint, one_launch):
+    seq, dev = N * K + rest, "cuda:0"
+    buf = torch.full((B * H * seq * d + 16 * d,), 7.0, device=dev)  # behind the last row nothing may be written
+    W, b = (torch.full(s, 7.0, device=dev) for s in ((2, B, H, d, d), (2, B, H, d)))
+    p = lambda t, at=0: ctypes.c_void_p(t.data_ptr() + 4 * at)
+    s = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+
+    def desc(n, k, per_batch):
+        ds = P.TttDesc(B, H, n, d, k, 1e-6, 1, P.TTT_F32)
+        ds.kernel_hint, ds.seq_stride, ds.state_per_batch = hint, seq, per_batch
+        return ctypes.byref(ds)
+
+    def rows(at):
+        return [p(v[k], at * d) for k in ("xq", "xk", "xv")]
+
+    L, full = P.lib(), N * K
+    if one_launch:
+        rc = L.ttt_linear_fwd_with_rest(desc(full, K, 0), rest, *rows(0), p(v["W0"]), p(v["b0"]), p(v["token_eta"]), p(v["lr"]),
+                                        p(v["gamma"]), p(v["beta"]), p(buf), p(W[1]), p(b[1]), s)
+        assert rc == 0, L.ttt_last_error()
+    else:
+        for n, k, at, i in ((full, K, 0, 0), (rest, rest, full, 1)):
+            state = (p(W[0]), p(b[0])) if i else (p(v["W0"]), p(v["b0"]))
+            rc = L.ttt_linear_fwd(desc(n, k, i), *rows(at), *state, p(v["token_eta"], at), p(v["lr"], at), p(v["gamma"]),
+                                  p(v["beta"]), p(buf, at * d), p(W[i]), p(b[i]), None, None, s)
+            assert rc == 0, L.ttt_last_error()
+    torch.cuda.synchronize()
+    assert (buf[B * H * seq * d:] == 7.0).all(), "written behind the last row"
+    return buf[:B * H * seq * d], W[1], b[1]
+
+
+# one token, one short of a mini-batch; odd and even numbers of mini-batches; the fewest; units beyond a group of eight
+@pytest.mark.parametrize("d,B,H,N,rest", [(64, 1, 1, 4, 1), (64, 3, 3, 5, 15), (64, 2, 12, 63, 5), (64, 8, 16, 8, 8), (32, 1, 2, 5, 1),
+                                          (32, 3, 11, 16, 15), (32, 2, 4, 7, 7)])
+@pytest.mark.parametrize("no_update", [False, True])
+def test_equals_two_launches(P, d, B, H, N, rest, no_update):
+    print(f"case linear rest d{d} B{B} H{H} N{N} rest{rest} {no_update}", flush=True)
+    v = inputs(P, d, B, H, N, rest)
+    if no_update:  # the short mini-batch leaves the state as it is
+        v["token_eta"][-1] = 0.0
+    two = run(P, v, d, B, H, N, rest, ONE, False)
+    for hint in (0, OTHER_XCD):
+        for i, (x, y) in enumerate(zip(two, run(P, v, d, B, H, N, rest, hint, True))):
+            assert (x - y).abs().max() <= 1e-5 * x.abs().max(), f"output {i}, hint {hint:#x}"
+    for i, (x, y) in enumerate(zip(two, run(P, v, d, B, H, N, rest, LOST, True))):
+        assert torch.equal(x, y), f"output {i}, lost"
+
+
+def test_calls_without_one_launch_are_refused(P):
+    v = inputs(P, 64, 1, 2, 3, 5)
+    with pytest.raises(AssertionError, match="no single launch"):
+        run(P, v, 64, 1, 2, 3, 5, 0, True)
+    with pytest.raises(AssertionError, match="no single launch"):
+        run(P, v, 64, 1, 2, 3, 5, ONE, True)
+
+
+def test_layer_on_a_state_that_goes_on(P):
+    """The layer's forward over a ragged sequence, twice, against its mini-batches one call each."""
+    d, B, H, N, rest = 64, 2, 3, 6, 9
+    v = inputs(P, d, B, H, N, rest)
+    layer = P.FusedTileMulti(P.ModelConfig(H, d, P.TTTConfig(mini_batch_size=K)), v["W0"], v["b0"], v["gamma"], v["beta"])
+    x = P.TTTInputsInner(P.Qkv(v["xq"], v["xk"], v["xv"]), v["token_eta"], v["lr"])
+    seq = N * K + rest
+    got, want = layer.init_state(B), layer.init_state(B)
+    for _ in range(2):
+        out = layer.forward(got, x)
+        ref = torch.cat([layer.forward_mini_batch(want, x, range(i, min(i + K, seq))) for i in range(0, seq, K)], 2)
+        for a, r in ((out, ref), (got.weight, want.weight), (got.bias, want.bias)):
+            assert (a - r).abs().max() <= 1e-4 * r.abs().max()

@@ -994,20 +994,23 @@ int dispatch_linear_fwd_pack(const ttt_desc* d, const ttt::LinearFwdArgs* a, uns
 // clear the words and look for units to do again, and the consumer's last output behind the producer's last G'', cost 4 - 5 us:
 // on one / two workgroups, d = 64, 24 units, 8 mini-batches 17.9 / 18.6 us, 12 23.6 / 22.8, 16 29.9 / 27.1, 63 102 / 76, 128 202 / 144;
 // 128 units, 12 24.8 / 24.4, 16 31.0 / 28.7; d = 32, 24 units, 12 17.1 / 17.4, 16 21.4 / 20.4, 63 72.6 / 56.5, 128 143.5 / 105.5.
-bool linear_fwd_on_pairs(const ttt_desc* d, const ttt::LinearFwdArgs& a, ttt::LinearPairArgs* pa) {
+// `rest` tokens of a short mini-batch behind save the launch that they would take otherwise, and pay from four mini-batches on (the
+// fewest tried): 24 units, d = 64, 4 19.2 / 15.5, 8 25.7 / 19.7, 16 37.7 / 28.1; d = 32, 4 14.0 / 12.3, 16 27.1 / 21.1; 128 units, d = 64, 4
+// 20.1 / 16.2.
+bool linear_fwd_on_pairs(const ttt_desc* d, const ttt::LinearFwdArgs& a, ttt::LinearPairArgs* pa, int rest = 0) {
   if (d->io_dtype != TTT_F32 || d->head_dim > 64 || a.K != 16) return false;
   if (d->kernel_hint & (TTT_HINT_WAVES_MASK | TTT_HINT_ALL_LOADS | TTT_HINT_ONE_WORKGROUP)) return false;
-  if (a.n_stages < 16) return false;
+  if (a.n_stages < (rest > 0 ? 4 : 16)) return false;
   const size_t units = (size_t)a.B * a.H;
   int cus = 0;
   if (device_cus(&cus) != TTT_OK || (units + 7) / 8 * 16 > (size_t)cus) return false;
-  const size_t D = (size_t)d->head_dim, tokens = (units - 1) * a.seq_stride + d->seq, states = d->state_per_batch ? units : (size_t)a.H;
+  const size_t D = (size_t)d->head_dim, tokens = (units - 1) * a.seq_stride + d->seq + rest, states = d->state_per_batch ? units : (size_t)a.H;
   const size_t saved = a.W_ckpt != nullptr ? units * a.n_ckpt : 0;
   struct Range {
     const void* p;
     size_t n;
   };
-  const Range in[] = {{a.xq, tokens * D * 4}, {a.xk, tokens * D * 4}, {a.xv, tokens * D * 4}, {a.lr, tokens * 4}, {a.token_eta, 64},
+  const Range in[] = {{a.xq, tokens * D * 4}, {a.xk, tokens * D * 4}, {a.xv, tokens * D * 4}, {a.lr, tokens * 4}, {a.token_eta, rest > 0 ? (size_t)(d->seq + rest) * 4 : 64},
                       {a.W0, states * D * D * 4}, {a.b0, states * D * 4}, {a.gamma, a.H * D * 4}, {a.beta, a.H * D * 4}};
   const Range res[] = {{a.out, tokens * D * 4}, {a.W_out, units * D * D * 4}, {a.b_out, units * D * 4}, {a.W_ckpt, saved * D * D * 4},
                        {a.b_ckpt, saved * D * 4}};
@@ -1024,6 +1027,7 @@ bool linear_fwd_on_pairs(const ttt_desc* d, const ttt::LinearFwdArgs& a, ttt::Li
   }
   pa->spin_limit = (d->kernel_hint & TTT_HINT_TEST_LOST_PARTNER) ? 0u : 1u << 21;
   pa->agent_release = (d->kernel_hint & TTT_HINT_TEST_OTHER_XCD) ? 1 : 0;
+  pa->rest = rest;
   return true;
 }
 
@@ -1051,6 +1055,20 @@ int ttt_linear_fwd(const ttt_desc* d, const void* xq, const void* xk, const void
   if (linear_fwd_on_pairs(d, a, &pa))
     return hip_status(ttt::launch_linear_fwd_pair(d->head_dim, a, pa, static_cast<hipStream_t>(stream)), "ttt_linear_fwd launch");
   return dispatch_linear_fwd(d, &a, 1, static_cast<hipStream_t>(stream));
+}
+
+int ttt_linear_fwd_with_rest(const ttt_desc* d, int32_t rest, const void* xq, const void* xk, const void* xv,
+                             const float* W0, const float* b0, const float* token_eta, const void* lr,
+                             const float* gamma, const float* beta, void* out, float* W_out, float* b_out, void* stream) {
+  ttt::LinearFwdArgs a;
+  int rc = prepare_linear_fwd(d, xq, xk, xv, W0, b0, token_eta, lr, gamma, beta, out, W_out, b_out, nullptr, nullptr, &a);
+  if (rc != TTT_OK) return rc;
+  if (rest < 1 || rest >= d->mini_batch) return fail(TTT_ERR_SHAPE, "%d tokens behind mini-batches of %d", (int)rest, d->mini_batch);
+  if (a.seq_stride < d->seq + rest)
+    return fail(TTT_ERR_SHAPE, "seq_stride %d is shorter than %d + %d tokens", a.seq_stride, d->seq, (int)rest);
+  ttt::LinearPairArgs pa;
+  if (!linear_fwd_on_pairs(d, a, &pa, rest)) return fail(TTT_ERR_UNSUPPORTED, "no single launch for this call");
+  return hip_status(ttt::launch_linear_fwd_pair(d->head_dim, a, pa, static_cast<hipStream_t>(stream)), "ttt_linear_fwd_with_rest launch");
 }
 
 }  // extern "C"

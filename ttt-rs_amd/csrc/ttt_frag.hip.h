@@ -184,6 +184,11 @@ __device__ __forceinline__ void lds_done() { asm volatile("s_waitcnt lgkmcnt(0)"
 // (isa_check.py refuses code that has one).
 typedef __attribute__((address_space(3))) int lds_int;
 
+template <class V>
+__device__ __forceinline__ unsigned lds_addr(const V* p) {
+  return (unsigned)(size_t)(const __attribute__((address_space(3))) V*)p;
+}
+
 // A fragment's transpose: element (m, k) of the tile that lies in LDS as a fragment (lane order) -> the fragment with the
 // two axes exchanged.  Within each group of sixteen lanes the instruction takes four rows of sixteen elements, a row from
 // four lanes, and gives every lane a column.

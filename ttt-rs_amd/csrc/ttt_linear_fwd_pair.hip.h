@@ -17,6 +17,10 @@
 // in the producer, no store but checkpoints: one copies rows global -> LDS (as in ttt_linear_fwd_dma_kernel), the
 // COURIER stores G'' and the word, or watches the word and copies G'' global -> LDS.  One barrier per mini-batch.
 //
+// A sequence may end in a short mini-batch (REST), which is then the last one of both workgroups instead of a launch of its own:
+// its rows are read once more for the lanes without a token, with a learning rate of zero.  A launch of one short mini-batch took 8 us:
+// 63 mini-batches and five tokens, 24 units, head_dim 64, 89.6 -> 83.8 us.
+//
 // The arithmetic is that of one workgroup, bit for bit.
 #pragma once
 #include "ttt_linear_fwd_sk.hip.h"
@@ -26,6 +30,7 @@ namespace ttt {
 struct LinearPairArgs {
   unsigned spin_limit;  // polls before the consumer gives up; 0: at once (tests of that path)
   int agent_release;    // 1: always publish with a device-scope release
+  int rest;             // REST: tokens of the short mini-batch behind the a.n_stages whole ones, 1 .. 15
 };
 // words of the last 64 floats of a unit's W_out, and the mark in its first (a final state that comes to have these bits by
 // itself costs a computation, not the result)
@@ -45,12 +50,7 @@ struct LinearPairLds {
   int lost;
 };
 
-template <class V>
-__device__ __forceinline__ unsigned lds_addr(const V* p) {
-  return (unsigned)(size_t)(const __attribute__((address_space(3))) V*)p;
-}
-
-template <int D, bool PRODUCER, bool CKPT>
+template <int D, bool PRODUCER, bool CKPT, bool REST>
 __device__ __forceinline__ void linear_fwd_pair_body(const LinearFwdArgs& a, const LinearPairArgs& pa, LinearPairLds<D>& L, size_t bh) {
   using IO = Io<F32>;
   constexpr int NT = D / 16, NW = NT, RS = LinearPairLds<D>::RS;
@@ -58,9 +58,16 @@ __device__ __forceinline__ void linear_fwd_pair_body(const LinearFwdArgs& a, con
   constexpr int K = 16;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int w = wave % NW, c = lane & 15, g = lane >> 4;  // (the two other waves do what a compute wave does up to where they branch off)
-  const int h = (int)(bh % a.H), n = a.n_stages;
+  const int h = (int)(bh % a.H), n = a.n_stages + (REST ? 1 : 0);
   const UnitBase<F32, D> ub(a, bh);
   unsigned* const words = reinterpret_cast<unsigned*>(a.W_out + bh * D * D + (D * D - kLinPairWords));
+  // where G'' of a mini-batch crosses: its rows of `out`; a short one has fewer rows than G'', which goes into W_out, behind the
+  // mark (a producer may write it when a consumer that waited in vain has set the mark)
+  const auto crossing = [&](int st) {
+    return REST && st == n - 1 ? reinterpret_cast<unsigned char*>(a.W_out + bh * D * D + kLinPairWords)
+                               : ub.out + (unsigned)st * (unsigned)(K * D * 4);
+  };
+  static_assert(kLinPairWords + 16 * D <= D * D - kLinPairWords, "G'' lies between the mark and the words");
 
   if (wave >= NW) {
     float sum_a;
@@ -72,14 +79,16 @@ __device__ __forceinline__ void linear_fwd_pair_body(const LinearFwdArgs& a, con
       const auto copy_in = [&](int stage) {  // (past the end: the last one again, into a slot nobody reads)
         const unsigned slot = (unsigned)(stage & (RS - 1)), dst = rows0 + slot * (2 * NT * 1024);
         const int st_ld = min(stage, n - 1);
-        const unsigned off = UnitBase<F32, D>::row_off(st_ld, K, c);
+        // a short mini-batch's last token again in the lanes without one, whose learning rate is made zero: nothing comes of them
+        const int row = REST && st_ld == n - 1 ? min(c, pa.rest - 1) : c;
+        const unsigned off = UnitBase<F32, D>::row_off(st_ld, K, row);
 #pragma unroll
         for (int J = 0; J < NT; ++J) {
           const unsigned fo = (unsigned)(32 * (J >> 1) + 8 * g + 4 * (J & 1)) * 4u;  // the lane's four features of tile J
           lds_dma16(PRODUCER ? ub.xk : ub.xq, off + fo, dst + J * 1024);
           lds_dma16(PRODUCER ? ub.xv : ub.xk, off + fo, dst + (NT + J) * 1024);
         }
-        if constexpr (PRODUCER) lds_dma4(ub.lr, ((unsigned)st_ld * (unsigned)K + (unsigned)c) * 4u, lr0 + slot * 256u);
+        if constexpr (PRODUCER) lds_dma4(ub.lr, ((unsigned)st_ld * (unsigned)K + (unsigned)row) * 4u, lr0 + slot * 256u);
       };
 #pragma unroll
       for (int u = 0; u < RS; ++u) copy_in(u);
@@ -108,7 +117,7 @@ __device__ __forceinline__ void linear_fwd_pair_body(const LinearFwdArgs& a, con
       const auto hand_over = [&](int st) {
 #pragma unroll
         for (int J = 0; J < NT; ++J)
-          *reinterpret_cast<f32x4*>(ub.out + (unsigned)st * (unsigned)(K * D * 4) + J * 1024 + lane16) = L.g[st & 1][J][lane];
+          *reinterpret_cast<f32x4*>(crossing(st) + J * 1024 + lane16) = L.g[st & 1][J][lane];
         if (!fast && pa.agent_release == 0) fast = look(words + kLinPairXcd) == xcd;
         if (!fast) __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -147,8 +156,7 @@ __device__ __forceinline__ void linear_fwd_pair_body(const LinearFwdArgs& a, con
           for (; next < known && next <= st + 2; ++next) {
 #pragma unroll
             for (int J = 0; J < NT; ++J)
-              lds_dma16_dev(ub.out + (unsigned)next * (unsigned)(K * D * 4), J * 1024u + lane16,
-                            g0 + (unsigned)(next & (RS - 1)) * (NT * 1024) + J * 1024);
+              lds_dma16_dev(crossing(next), J * 1024u + lane16, g0 + (unsigned)(next & (RS - 1)) * (NT * 1024) + J * 1024);
           }
           asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         }
@@ -164,11 +172,24 @@ __device__ __forceinline__ void linear_fwd_pair_body(const LinearFwdArgs& a, con
 
   // ---- compute waves: tile w of the features (the names are those of linear_fwd_sk_body)
   const float te_last = a.token_eta[K - 1];
-  const bool upd = te_last != 0.f;
-  const float sc = upd ? te_last : 1.f;
-  const float rho_c = a.token_eta[c] / sc;
+  bool upd = te_last != 0.f;
+  float sc = upd ? te_last : 1.f, rho_c = a.token_eta[c] / sc;
   const f32x4 ident = identity_frag<F32>(c, g), ones = splat_frag<F32>(1.f);
-  const f32x4 ident_upd = upd ? ident : IO::zero(), ones_upd = upd ? ones : IO::zero();
+  f32x4 ident_upd = upd ? ident : IO::zero(), ones_upd = upd ? ones : IO::zero();
+  // the short mini-batch's token_eta, loaded here and taken up in front of it
+  float te_rest_last = 0.f, te_rest_c = 0.f;
+  if constexpr (REST) {
+    const float* te = a.token_eta + a.n_stages * K;
+    te_rest_last = te[pa.rest - 1];
+    te_rest_c = te[min(c, pa.rest - 1)];
+  }
+  const auto take_rest = [&]() {
+    upd = te_rest_last != 0.f;
+    sc = upd ? te_rest_last : 1.f;
+    rho_c = te_rest_c / sc;
+    ident_upd = upd ? ident : IO::zero();
+    ones_upd = upd ? ones : IO::zero();
+  };
   const size_t sb = a.state_per_batch ? bh : (size_t)h;
   const float eps = held(a.eps);
   const int fo = own_offset<1>(w, 0, g);
@@ -197,6 +218,28 @@ __device__ __forceinline__ void linear_fwd_pair_body(const LinearFwdArgs& a, con
     if constexpr (PRODUCER) lr[u] = L.lr[sl][c];
   };
   gather(0, 0);
+
+  // all mini-batches; `mask` comes in front of a short one
+  const auto run = [&](const auto& mini_batch, const auto& mask) {
+    constexpr std::integral_constant<int, 0> even{};
+    constexpr std::integral_constant<int, 1> odd{};
+    int st = 0;
+    for (; st + 2 <= a.n_stages; st += 2) {
+      mini_batch(even, st);
+      mini_batch(odd, st + 1);
+    }
+    if (st < a.n_stages) mini_batch(even, st);
+    if constexpr (REST) {
+      take_rest();
+      if (st < a.n_stages) {
+        mask(odd);
+        mini_batch(odd, n - 1);
+      } else {
+        mask(even);
+        mini_batch(even, n - 1);
+      }
+    }
+  };
 
   if constexpr (PRODUCER) {
     CkptCursor<D> ck(a, bh);
@@ -276,12 +319,9 @@ __device__ __forceinline__ void linear_fwd_pair_body(const LinearFwdArgs& a, con
       IO::mma(bT[0], Gd, ones_upd);
       L.g[u][w][lane] = Gd;
     };
-    int st = 0;
-    for (; st + 2 <= n; st += 2) {
-      mini_batch(std::integral_constant<int, 0>{}, st);
-      mini_batch(std::integral_constant<int, 1>{}, st + 1);
-    }
-    if (st < n) mini_batch(std::integral_constant<int, 0>{}, st);
+    run(mini_batch, [&](auto u_tag) {
+      if (c >= pa.rest) lr[decltype(u_tag)::value] = 0.f;
+    });
     lds_barrier();  // the last G''
   } else {
     // pending output of the last mini-batch (its sums travel in the next exchange) and of the one before (sums known)
@@ -344,12 +384,7 @@ __device__ __forceinline__ void linear_fwd_pair_body(const LinearFwdArgs& a, con
       zbp = zb;
       qop = xo[u];
     };
-    int st = 0;
-    for (; st + 2 <= n; st += 2) {
-      mini_batch(std::integral_constant<int, 0>{}, st);
-      mini_batch(std::integral_constant<int, 1>{}, st + 1);
-    }
-    if (st < n) mini_batch(std::integral_constant<int, 0>{}, st);
+    run(mini_batch, [](auto) {});
     f32x4 W0[NT][1];
     load_state_slice<D, 1>(W0, a.W0 + sb * D * D, w, c, g);
     publish(n & 1);
@@ -357,7 +392,7 @@ __device__ __forceinline__ void linear_fwd_pair_body(const LinearFwdArgs& a, con
     float s0, s1;
     collect(n & 1, s0, s1);
     if (n >= 2) emit(so0, so1, n - 2, zbo, qoo);
-    emit(s0, s1, n - 1, zbp, qop);
+    if (!REST || c < pa.rest) emit(s0, s1, n - 1, zbp, qop);
     store_state_final<D, 1>(a.W_out + bh * D * D, a.b_out + bh * D, W0, a.b0 + sb * D, Wc, bT, L.m0s, w, c, g);
     // element (0, 0) of W_out is written by the lane that marks the unit
     if (L.lost != 0 && threadIdx.x == 0) *reinterpret_cast<unsigned*>(a.W_out + bh * D * D) = kLinPairLost;
@@ -366,15 +401,15 @@ __device__ __forceinline__ void linear_fwd_pair_body(const LinearFwdArgs& a, con
 
 // Workgroups b and b + 8 of every 16 share a unit: consecutive workgroups go to the XCDs in turn, so both run behind one L2, and
 // the producer, which waits for nobody, is dispatched first.
-template <int D, bool CKPT>
+template <int D, bool CKPT, bool REST>
 __global__ void __launch_bounds__(64 * (D / 16 + 2)) ttt_linear_fwd_pair_kernel(LinearFwdArgs a, LinearPairArgs pa) {
   __shared__ LinearPairLds<D> L;
   const size_t bh = (size_t)(blockIdx.x >> 4) * 8 + (blockIdx.x & 7);
   if (bh >= (size_t)a.B * a.H) return;
   if (((blockIdx.x >> 3) & 1) == 0)
-    linear_fwd_pair_body<D, true, CKPT>(a, pa, L, bh);
+    linear_fwd_pair_body<D, true, CKPT, REST>(a, pa, L, bh);
   else
-    linear_fwd_pair_body<D, false, false>(a, pa, L, bh);
+    linear_fwd_pair_body<D, false, false, REST>(a, pa, L, bh);
 }
 
 // the word of every unit, and the consumer's XCD number
@@ -393,6 +428,29 @@ __global__ void __launch_bounds__(64 * (D / 16 + 1)) ttt_linear_fwd_redo_kernel(
   const unsigned* mark = reinterpret_cast<const unsigned*>(a.W_out + blockIdx.x * (size_t)(D * D));
   if (__builtin_amdgcn_readfirstlane((int)*mark) != (int)kLinPairLost) return;
   linear_fwd_sk_body<F32, D, D / 16, 2, true, false, 5, false, false, false, CKPT>(a, nullptr);
+}
+
+// the same where a short mini-batch of `rest` tokens follows: as two calls would, without the wave that copies rows
+template <int D>
+__global__ void __launch_bounds__(64 * (D / 16)) ttt_linear_fwd_redo_rest_kernel(LinearFwdArgs a, int rest) {
+  const unsigned* mark = reinterpret_cast<const unsigned*>(a.W_out + blockIdx.x * (size_t)(D * D));
+  if (__builtin_amdgcn_readfirstlane((int)*mark) != (int)kLinPairLost) return;
+  linear_fwd_sk_body<F32, D, D / 16, 2, true, false, 0, false, false, false, false>(a, nullptr);
+  __threadfence();  // the state in between goes from wave to wave through memory
+  __syncthreads();
+  const size_t at = (size_t)a.n_stages * a.K, row = at * (D * 4);
+  a.xq = static_cast<const unsigned char*>(a.xq) + row;
+  a.xk = static_cast<const unsigned char*>(a.xk) + row;
+  a.xv = static_cast<const unsigned char*>(a.xv) + row;
+  a.lr = static_cast<const unsigned char*>(a.lr) + at * 4;
+  a.out = static_cast<unsigned char*>(a.out) + row;
+  a.token_eta += at;
+  a.W0 = a.W_out;
+  a.b0 = a.b_out;
+  a.state_per_batch = 1;
+  a.seq = a.K = rest;
+  a.n_stages = 1;
+  linear_fwd_sk_body<F32, D, D / 16, 2, false, false, 0, false, false, false, false>(a, nullptr);
 }
 
 hipError_t launch_linear_fwd_pair(int head_dim, const LinearFwdArgs& a, const LinearPairArgs& pa, hipStream_t s);  // ttt_linear_fwd_pair.hip

@@ -254,7 +254,7 @@ PyObject* linear_forward(PyObject* const* a) {
 }
 
 // A layer's pass over the tokens start .. stop of its inputs: whole mini-batches in one launch, a remainder as one
-// short mini-batch behind it.  (xq, xk, xv, weight, bias, token_eta, lr, ln_weight, ln_bias, mini_batch, eps,
+// short mini-batch in the same launch where the library has one, or behind it.  (xq, xk, xv, weight, bias, token_eta, lr, ln_weight, ln_bias, mini_batch, eps,
 // checkpoint_interval, start, stop) -> (out, weight, bias); of token_eta the first K entries from start on are read, and
 // those of a remainder; the state goes in shared over the batch ([H,d,d], [H,d]) or per
 // batch element and comes out per batch element.
@@ -300,11 +300,20 @@ PyObject* linear_layer_forward(PyObject* const* a) {
   if (rest > 0) desc[calls++] = desc_of(B, H, rest, d, rest, eps, ci, io, per_batch || full > 0, full > 0 ? n : 0, 0, 0);
   for (int i = 0; i < calls; ++i) check(ttt_linear_supported(&desc[i]));
   at::Tensor out = empty(rows, q.dtype, q.dev), W[2], b[2];
-  for (int i = 0; i < calls; ++i) {
-    W[i] = empty(W4, at::kFloat, q.dev);
-    b[i] = empty(b3, at::kFloat, q.dev);
-  }
   char* po = static_cast<char*>(out.data_ptr());
+  W[0] = empty(W4, at::kFloat, q.dev);
+  b[0] = empty(b3, at::kFloat, q.dev);
+  if (calls == 2) {  // in one launch where there is one
+    bool one = true;
+    enqueue(q.dev, [&](void* s) {
+      const int rc = ttt_linear_fwd_with_rest(&desc[0], (int32_t)rest, pq, pk, pv, W0, b0, te, pl, gam, bet, po, ptr(W[0]), ptr(b[0]), s);
+      one = rc != TTT_ERR_UNSUPPORTED;
+      return one ? rc : (int)TTT_OK;
+    });
+    if (one) return wrap_tuple({&out, &W[0], &b[0]});
+    W[1] = empty(W4, at::kFloat, q.dev);
+    b[1] = empty(b3, at::kFloat, q.dev);
+  }
   enqueue(q.dev, [&](void* s) {
     for (int i = 0; i < calls; ++i) {
       const int64_t at = i == 0 ? 0 : full, rb = at * d * size;

@@ -300,7 +300,8 @@ class FusedTileMulti:
 
     def forward(self, state: TTTLinearState, inputs: TTTInputsInner) -> torch.Tensor:
         """wrapper.rs:102-164: all full mini-batches in one launch; a trailing remainder is one
-        short mini-batch, as the Burn-op model does it (inner.rs:40-47).  Both launches read and write
+        short mini-batch, as the Burn-op model does it (inner.rs:40-47), of the same launch where the library has one
+        (ttt_linear_fwd_with_rest) and of a second one elsewhere.  Both launches read and write
         windows of the sequence in place.  A sequence without tokens leaves the state as it is."""
         seq = inputs.qkv.xq.shape[2]
         return self._pass(state, inputs, 0, seq) if seq > 0 else torch.empty_like(inputs.qkv.xq)
