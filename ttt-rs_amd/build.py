@@ -18,7 +18,8 @@ LIB_PATH = os.path.join(LIB_DIR, "libttt_mi355x.so")
 TRACKERS = ("-mllvm", "-amdgpu-use-amdgpu-trackers=1")
 # translation units, compiled side by side, and what each is compiled with besides HIPCC_FLAGS
 SOURCES = {os.path.join(HERE, "csrc", f): flags for f, flags in (
-    ("ttt_api.hip", ()), ("ttt_mlp_bwd_rp.hip", ()), ("ttt_mlp_bwd_rp_d96.hip", TRACKERS), ("ttt_mlpn_fwd.hip", ()), ("ttt_linear_fwd_pair.hip", ()))}
+    ("ttt_api.hip", ()), ("ttt_mlp_bwd_rp.hip", ()), ("ttt_mlp_bwd_rp_d96.hip", TRACKERS), ("ttt_mlpn_fwd.hip", ()), ("ttt_linear_fwd_pair.hip", ()),
+    ("ttt_linear_fwd_roles.hip", ()))}
 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC",

@@ -20,6 +20,7 @@
 #include "ttt_linear_fwd.hip.h"
 #include "ttt_linear_fwd_mw.hip.h"
 #include "ttt_linear_fwd_pair.hip.h"
+#include "ttt_linear_fwd_roles.hip.h"
 #include "ttt_linear_fwd_sk.hip.h"
 #include "ttt_mlp_bwd.hip.h"
 #include "ttt_mlp_bwd_rp.hip.h"
@@ -217,6 +218,19 @@ int launch_linear_fwd_nw(const ttt::LinearFwdArgs* probs, unsigned ny, hipStream
   return hip_status(hipGetLastError(), "ttt_linear_fwd launch");
 }
 
+// bf16 I/O, head_dim 32 / 64, mini-batches of 16: whether the waves of a unit take roles (ttt_linear_fwd_roles.hip.h), the same bits.
+// head_dim 64 up to a unit per CU, 32 up to two (both measured there).  Few mini-batches at head_dim 32 lose to the longer
+// way into the loop, more so where the launch saves: two waves / in roles, 12 units, 1 mini-batch 5.4 / 5.8, 3 5.92 / 5.97, 4 6.5 / 5.8,
+// 384 units 4 7.7 / 6.8; saving 4 6.7 / 7.1, 8 8.5 / 7.1; head_dim 64, 12 units, 1 6.9 / 6.1, saving 1 7.0 / 7.1, 2 7.8 / 7.2.
+bool linear_fwd_in_roles(int D, const ttt::LinearFwdArgs* probs, int hint, unsigned ny, int rest, int* cus) {
+  const ttt::LinearFwdArgs& a = probs[0];
+  if (a.K != 16 || (hint & (TTT_HINT_WAVES_MASK | TTT_HINT_ALL_LOADS | TTT_HINT_ONE_WORKGROUP)) != 0 || any_input_sums(probs, ny)) return false;
+  bool saves = false;
+  for (unsigned y = 0; y < ny; ++y) saves = saves || probs[y].W_ckpt != nullptr;
+  if (a.n_stages < (rest > 0 ? 4 : D == 64 ? (saves ? 2 : 1) : (saves ? 8 : 4))) return false;
+  return device_cus(cus) == TTT_OK && (long)a.B * a.H * ny <= (D == 64 ? 1L : 2L) * *cus;
+}
+
 template <class T, int D>
 int launch_linear_fwd(const ttt::LinearFwdArgs* probs, int hint, unsigned ny, hipStream_t s) {
   const int waves_hint = hint & TTT_HINT_WAVES_MASK;
@@ -248,6 +262,11 @@ int launch_linear_fwd(const ttt::LinearFwdArgs* probs, int hint, unsigned ny, hi
   }
   if constexpr (max_nw >= 4) {
     if (nw >= 4) return launch_linear_fwd_nw<T, D, 4>(probs, ny, s, false, ctl_wave);
+  }
+  if constexpr (!f32) {
+    int cus = 0;
+    if (linear_fwd_in_roles(D, probs, hint, ny, 0, &cus))
+      return hip_status(ttt::launch_linear_fwd_roles(D, probs, ny, cus, 0, s), "ttt_linear_fwd launch");
   }
   // bf16: own-feature loads.  Every wave's loads of whole rows -> own features, 2048 tokens, d = 64: 4 units 112.4 -> 113.2 us, 8
   // 112.6 -> 113.4, 12 116.0 -> 113.9, 24 114.5 -> 114.2, 48 120.5 -> 115.7, 128 124.4 -> 118.4, 256 127.6 -> 118.1, saving
@@ -1066,6 +1085,10 @@ int ttt_linear_fwd_with_rest(const ttt_desc* d, int32_t rest, const void* xq, co
   if (rest < 1 || rest >= d->mini_batch) return fail(TTT_ERR_SHAPE, "%d tokens behind mini-batches of %d", (int)rest, d->mini_batch);
   if (a.seq_stride < d->seq + rest)
     return fail(TTT_ERR_SHAPE, "seq_stride %d is shorter than %d + %d tokens", a.seq_stride, d->seq, (int)rest);
+  int cus = 0;
+  if (d->io_dtype == TTT_BF16 && d->head_dim <= 64 && linear_fwd_in_roles(d->head_dim, &a, d->kernel_hint, 1, rest, &cus))
+    return hip_status(ttt::launch_linear_fwd_roles(d->head_dim, &a, 1, cus, rest, static_cast<hipStream_t>(stream)),
+                      "ttt_linear_fwd_with_rest launch");
   ttt::LinearPairArgs pa;
   if (!linear_fwd_on_pairs(d, a, &pa, rest)) return fail(TTT_ERR_UNSUPPORTED, "no single launch for this call");
   return hip_status(ttt::launch_linear_fwd_pair(d->head_dim, a, pa, static_cast<hipStream_t>(stream)), "ttt_linear_fwd_with_rest launch");
