@@ -133,3 +133,25 @@ def test_rest_equals_two_launches(P, d, B, H, N, rest, no_update):
         assert (x - y).abs().max() <= 2.0 ** -7 * x.abs().max(), name
     unit = lambda t: t[:B * H * seq * d].view(B, H, seq, d)[:, :, :full]
     assert torch.equal(unit(bufs[0]), unit(bufs[1])), "the whole mini-batches"
+
+
+# one mini-batch, around the ring of eight; more than a unit per CU (head_dim 32)
+@pytest.mark.parametrize("rope", [False, True])
+@pytest.mark.parametrize("d,B,H,N", [(64, 1, 3, 1), (64, 2, 5, 2), (64, 2, 3, 9), (64, 1, 12, 20), (32, 2, 3, 4), (32, 1, 5, 7), (32, 20, 16, 10)])
+def test_operands_formed_from_projections(P, d, B, H, N, rope):
+    """The fused call without copies of the operands against forming them first: the same bits."""
+    print(f"case linear roles formed d{d} B{B} H{H} N{N} rope{rope}", flush=True)
+    dev, seq = "cuda:0", N * K
+    g = torch.Generator(device=dev).manual_seed(5800 + d + N)
+    r = lambda *s: torch.randn(*s, generator=g, device=dev)
+    x = [r(B, seq, H, d).bfloat16() for _ in range(3)]
+    args = (*x, r(B, seq, H).bfloat16(), r(H) * 0.5, 0.8, 1.0 / torch.arange(1, K + 1, dtype=torch.float32, device=dev), r(K) * 0.1)
+    state = (r(H, d, d) * 0.02, r(H, d) * 0.02, 1.0 + 0.1 * r(H, d), 0.1 * r(H, d))
+    pos = dict(rope=P.rope_cos_sin(K, 0, None, d, dev), pos_offset=5, pos_wrap=K) if rope else {}
+    got = P.ttt_linear_forward_fused_inputs_raw(*args, *state, K, **pos)
+    ins = P.inner_loop_inputs_raw(*args, K, **pos)
+    want = P.ttt_linear_forward_raw(ins.qkv.xq, ins.qkv.xk, ins.qkv.xv, state[0], state[1], ins.token_eta, ins.ttt_lr_eta, *state[2:], K,
+                                    kernel_hint=TWO_WAVES)
+    torch.cuda.synchronize()
+    for i, (a, b) in enumerate(zip(got, want)):
+        assert torch.equal(a, b), f"output {i}"

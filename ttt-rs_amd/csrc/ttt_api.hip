@@ -1335,6 +1335,10 @@ int ttt_linear_fwd_fused_inputs(const ttt_desc* d, const void* xq, const void* x
   const bool full = d->mini_batch == 16;
   const dim3 grid((unsigned)(a.B * a.H)), block(128);
   hipStream_t s = static_cast<hipStream_t>(stream);
+  int cus = 0;
+  if (!per_token && !W_ckpt && !xq_out && !xk_out && !xv_out && !lr_out && !token_eta_out && aligned16(xq) && aligned16(xk) && aligned16(xv) &&
+      linear_fwd_in_roles(d->head_dim, &a, d->kernel_hint, 1, 0, &cus))
+    return hip_status(ttt::launch_linear_fwd_roles_form(d->head_dim, a, fi, cus, s), "ttt_linear_fwd_fused_inputs launch");
 #define TTT_FI_LAUNCH(D_, FULL_, RAW_) \
   hipLaunchKernelGGL((ttt::ttt_linear_fwd_fi_kernel<ttt::BF16, D_, 2, 2, FULL_, false, RAW_>), grid, block, 0, s, a, fi)
   if (d->head_dim == 64) {

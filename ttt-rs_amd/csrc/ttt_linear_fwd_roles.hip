@@ -23,6 +23,17 @@ static hipError_t launch(const LinearFwdArgs* probs, unsigned ny, int cus, int r
   return hipGetLastError();
 }
 
+hipError_t launch_linear_fwd_roles_form(int head_dim, const LinearFwdArgs& a, const FusedInputsArgs& fi, int cus, hipStream_t s) {
+  const dim3 grid((unsigned)(a.B * a.H)), block(64 * 6);
+  if (head_dim == 64)
+    hipLaunchKernelGGL((ttt_linear_fwd_roles_form_kernel<64, false>), grid, block, 0, s, a, fi, cus);
+  else if ((long)a.B * a.H <= cus)
+    hipLaunchKernelGGL((ttt_linear_fwd_roles_form_kernel<32, false>), grid, block, 0, s, a, fi, cus);
+  else
+    hipLaunchKernelGGL((ttt_linear_fwd_roles_form_kernel<32, true>), grid, block, 0, s, a, fi, cus);
+  return hipGetLastError();
+}
+
 hipError_t launch_linear_fwd_roles(int head_dim, const LinearFwdArgs* probs, unsigned ny, int cus, int rest, hipStream_t s) {
   if (head_dim == 64) return launch<64, false>(probs, ny, cus, rest, s);
   return (long)probs[0].B * probs[0].H * ny > cus ? launch<32, true>(probs, ny, cus, rest, s) : launch<32, false>(probs, ny, cus, rest, s);

@@ -16,6 +16,10 @@
 // more registers than five waves of two workgroups leave it (two rounds, 164 us), and without the copy wave it is even with two
 // waves per unit: 272 units 113.1 / 107.3, 384 113.8 / 114.0, 512 121.0 / 130.2.
 //
+// FORM: head split, rotary embedding and lr gate go to a second copy wave, which forms the operands of the next mini-batch in LDS, in
+// place; in the two-wave kernel (RAW = 1) they are instructions of the waves that carry the recurrence.  128 mini-batches, head_dim 64, 12
+// units 135.0 -> 78.1 us, 256 138.6 -> 81.6; head_dim 32, 256 units 97.1 -> 53.7, 384 126.8 -> 73.3.
+//
 // REST: a short mini-batch behind the whole ones is the last one, as in ttt_linear_fwd_pair.hip.h.
 //
 // The arithmetic is that of ttt_linear_fwd_sk_kernel, bit for bit.
@@ -36,8 +40,11 @@ struct LinearRolesLds {
 };
 
 // SAVE 0: nothing.  1: states.  2: update factors.
-template <int D, int SAVE, bool TWO, bool REST>
-__device__ __forceinline__ void linear_fwd_roles_body(const LinearFwdArgs& a, LinearRolesLds<D>& L, bool flip, int rest) {
+// FORM: the operands are formed from the projections (FusedInputsArgs, no copies of them asked for, positions that repeat with the
+// mini-batch), by a second copy wave.
+template <int D, int SAVE, bool TWO, bool REST, bool FORM = false>
+__device__ __forceinline__ void linear_fwd_roles_body(const LinearFwdArgs& a, LinearRolesLds<D>& L, bool flip, int rest,
+                                                      const FusedInputsArgs* fi = nullptr) {
   using IO = Io<BF16>;
   using frag = IO::frag;
   using LD = LinearRolesLds<D>;
@@ -53,33 +60,78 @@ __device__ __forceinline__ void linear_fwd_roles_body(const LinearFwdArgs& a, Li
   static_assert(64 * NW >= D, "centre_state's sums are the first NW waves'");
   float sum_a;  // of gamma^2
 
+  if (FORM && wave == 2 * NW + 1) {  // xq, xk and the learning rates of mini-batch st + 1 between the barriers of st - 1 and st, in place
+    const size_t pos = fi->cos != nullptr ? (size_t)((fi->pos_offset + c) % fi->pos_wrap) * (D / 2) + 4 * g : 0;
+    f32x4 cs[NT / 2], sn[NT / 2];
+#pragma unroll
+    for (int q = 0; q < NT / 2; ++q)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        cs[q][i] = fi->cos != nullptr ? fi->cos[pos + 16 * q + i] : 1.f;
+        sn[q][i] = fi->cos != nullptr ? fi->sin[pos + 16 * q + i] : 0.f;
+      }
+    const float bias = fi->lr_bias[h], scale = fi->lr_scale;
+    const auto form = [&](int stage) {
+      const int sl = stage & (RS - 1);
+#pragma unroll
+      for (int what = 0; what < 2; ++what)
+#pragma unroll
+        for (int q = 0; q < NT / 2; ++q) {
+          const u32x4 v = L.rows[sl][what][q][lane];
+          const f32x4 lo = IO::to_f32(__builtin_bit_cast(frag, u32x2{v[0], v[1]})), hi = IO::to_f32(__builtin_bit_cast(frag, u32x2{v[2], v[3]}));
+          const u32x2 x = __builtin_bit_cast(u32x2, IO::to_frag(rope_rotate4(lo, f32x2{cs[q][0], cs[q][1]}, f32x2{sn[q][0], sn[q][1]})));
+          const u32x2 y = __builtin_bit_cast(u32x2, IO::to_frag(rope_rotate4(hi, f32x2{cs[q][2], cs[q][3]}, f32x2{sn[q][2], sn[q][3]})));
+          L.rows[sl][what][q][lane] = u32x4{x[0], x[1], y[0], y[1]};
+        }
+      const float z = __uint_as_float(L.lr[sl][lane] << 16);
+      L.lr[sl][lane] = __float_as_uint(IO::rounded(lr_gate(z + bias, scale))) >> 16;
+    };
+    f32x4 Wn[NT][TPW], bn[TPW];
+    centre_state<D, NW, TPW, false>(Wn, bn, a.b0, L.m0s, a.gamma, sum_a, scratch, w, c, g);
+    asm volatile("s_barrier" ::: "memory");
+    form(0);
+    lds_barrier();
+    for (int st = 0; st < n; ++st) {
+      form(st + 1);
+      lds_barrier();
+    }
+    asm volatile("s_barrier\n\ts_barrier" ::: "memory");
+    return;
+  }
   if (wave == 2 * NW) {  // rows: mini-batch st + RS - 2 behind the barrier of mini-batch st
     constexpr int kCopies = 3 * (NT / 2) + 1;
+    // (FORM: token t of the unit is row (b seq + t) H + h of the [B,seq,H,d] projections and of the [B,seq,H] logits)
+    const size_t row0 = FORM ? bh / a.H * (size_t)a.seq * a.H + h : 0;
+    const unsigned char* const xq = FORM ? static_cast<const unsigned char*>(fi->xq) + row0 * (D * 2) : ub.xq;
+    const unsigned char* const xk = FORM ? static_cast<const unsigned char*>(fi->xk) + row0 * (D * 2) : ub.xk;
+    const unsigned char* const xv = FORM ? static_cast<const unsigned char*>(fi->xv) + row0 * (D * 2) : ub.xv;
+    const unsigned char* const lr = FORM ? static_cast<const unsigned char*>(fi->lr_logits) + row0 * 2 : ub.lr;
+    const unsigned pitch = FORM ? (unsigned)a.H : 1u;
     const unsigned rows0 = lds_addr(&L.rows[0][0][0][0]), lr0 = lds_addr(&L.lr[0][0]);
     const auto copy_in = [&](int stage) {  // (past the end: the last one again, into a slot nobody reads)
       const unsigned slot = (unsigned)(stage & (RS - 1)), dst = rows0 + slot * (3 * (NT / 2) * 1024);
       const int st_ld = min(stage, n - 1);
       // a short mini-batch's last token again in the lanes without one, whose learning rate is made zero: nothing comes of them
       const int row = REST && st_ld == n - 1 ? min(c, rest - 1) : c;
-      const unsigned off = UnitBase<BF16, D>::row_off(st_ld, K, row) + 16u * (unsigned)g;
+      const unsigned t = ((unsigned)st_ld * (unsigned)K + (unsigned)row) * pitch, off = t * (D * 2u) + 16u * (unsigned)g;
 #pragma unroll
       for (int q = 0; q < NT / 2; ++q) {
-        lds_dma16(ub.xk, off + 64u * q, dst + (1 * (NT / 2) + q) * 1024);
-        lds_dma16(ub.xv, off + 64u * q, dst + (2 * (NT / 2) + q) * 1024);
-        lds_dma16(ub.xq, off + 64u * q, dst + (0 * (NT / 2) + q) * 1024);
+        lds_dma16(xk, off + 64u * q, dst + (1 * (NT / 2) + q) * 1024);
+        lds_dma16(xv, off + 64u * q, dst + (2 * (NT / 2) + q) * 1024);
+        lds_dma16(xq, off + 64u * q, dst + (0 * (NT / 2) + q) * 1024);
       }
-      lds_dma2(ub.lr, ((unsigned)st_ld * (unsigned)K + (unsigned)row) * 2u, lr0 + slot * 256u);
+      lds_dma2(lr, t * 2u, lr0 + slot * 256u);
     };
 #pragma unroll
     for (int u = 0; u < RS - 2; ++u) copy_in(u);
     f32x4 Wn[NT][TPW], bn[TPW];
     centre_state<D, NW, TPW, false>(Wn, bn, a.b0, L.m0s, a.gamma, sum_a, scratch, w, c, g);
-    constexpr int kAhead = (RS - 3) * kCopies < 63 ? (RS - 3) * kCopies : 63;
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kAhead) : "memory");  // mini-batch 0 has landed
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"((RS - (FORM ? 4 : 3)) * kCopies) : "memory");  // mini-batch 0 has landed (FORM: and 1)
     asm volatile("s_barrier" ::: "memory");
+    if constexpr (FORM) asm volatile("s_barrier" ::: "memory");
     for (int st = 0; st < n; ++st) {
-      // mini-batch st + 1 has landed; the slot of mini-batch st - 2 was last read in front of this barrier, by the output waves
-      asm volatile("s_waitcnt vmcnt(%0)" ::"n"((RS - 4) * kCopies) : "memory");
+      // mini-batch st + 1 has landed (FORM: st + 2); the slot of mini-batch st - 2 was last read in front of this barrier, by the output waves
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"((RS - (FORM ? 5 : 4)) * kCopies) : "memory");
       asm volatile("s_barrier" ::: "memory");
       copy_in(st + RS - 2);
     }
@@ -88,9 +140,13 @@ __device__ __forceinline__ void linear_fwd_roles_body(const LinearFwdArgs& a, Li
     return;
   }
 
-  const float te_last = a.token_eta[K - 1];
+  const auto tok_eta = [&](int i) {
+    if constexpr (FORM) return fmaxf(fi->token_idx[i] + fi->learnable_token_idx[i], 0.f);
+    else return a.token_eta[i];
+  };
+  const float te_last = tok_eta(K - 1);
   bool upd = te_last != 0.f;
-  float sc = upd ? te_last : 1.f, rho_c = a.token_eta[c] / sc;
+  float sc = upd ? te_last : 1.f, rho_c = tok_eta(c) / sc;
   const frag ident = identity_frag<BF16>(c, g), nident = identity_frag<BF16>(c, g, -1.f), ones = splat_frag<BF16>(1.f);
   frag ones_upd = upd ? ones : IO::zero();
   unsigned upd_mask = upd ? ~0u : 0u;
@@ -124,6 +180,7 @@ __device__ __forceinline__ void linear_fwd_roles_body(const LinearFwdArgs& a, Li
   load_state_slice<D, TPW>(Wc, a.W0 + sb * D * D, w, c, g);
   centre_state<D, NW, TPW>(Wc, bT, a.b0 + sb * D, L.m0s, a.gamma + h * D, sum_a, scratch, w, c, g);
   lds_barrier();
+  if constexpr (FORM) lds_barrier();
 
   const auto full_rows = [&](frag (&x)[NT], int sl, int what) {
 #pragma unroll
@@ -366,6 +423,13 @@ __global__ void __launch_bounds__(64 * 5, TWO ? 3 : 2) ttt_linear_fwd_roles_kern
   linear_fwd_roles_body<D, SAVE, TWO, REST>(P.p[blockIdx.y], L, TWO && (int)(blockIdx.y * gridDim.x + blockIdx.x) >= cus, rest);
 }
 
+template <int D, bool TWO>
+__global__ void __launch_bounds__(64 * 6, TWO ? 3 : 2) ttt_linear_fwd_roles_form_kernel(LinearFwdArgs a, FusedInputsArgs fi, int cus) {
+  __shared__ LinearRolesLds<D> L;
+  linear_fwd_roles_body<D, 0, TWO, false, true>(a, L, TWO && (int)blockIdx.x >= cus, 0, &fi);
+}
+
+hipError_t launch_linear_fwd_roles_form(int head_dim, const LinearFwdArgs& a, const FusedInputsArgs& fi, int cus, hipStream_t s);
 // rest: tokens of a short mini-batch behind the whole ones (no checkpoints then), or 0
 hipError_t launch_linear_fwd_roles(int head_dim, const LinearFwdArgs* probs, unsigned ny, int cus, int rest, hipStream_t s);  // ttt_linear_fwd_roles.hip
 
