@@ -58,10 +58,10 @@ def make(P, d, B, H, N, no_update=False):
     return c
 
 
-# one mini-batch, around the ring of eight, odd and even; one unit per CU, one more, two per CU
+# one mini-batch, around the ring of eight, odd and even; a unit per CU, more (an odd number too), two per CU
 @pytest.mark.parametrize("d", [32, 64])
 @pytest.mark.parametrize("B,H,N", [(1, 1, 1), (1, 2, 2), (1, 3, 3), (2, 3, 7), (2, 3, 8), (3, 3, 9), (2, 5, 18), (16, 16, 5), (17, 16, 4),
-                                   (24, 16, 11), (32, 16, 3)])
+                                   (24, 16, 11), (32, 16, 3), (257, 1, 3)])
 def test_same_bits_as_two_waves(P, d, B, H, N):
     print(f"case linear roles d{d} B{B} H{H} N{N}", flush=True)
     c = make(P, d, B, H, N)
@@ -137,7 +137,7 @@ def test_rest_equals_two_launches(P, d, B, H, N, rest, no_update):
 
 # one mini-batch, around the ring of eight; more than a unit per CU (head_dim 32)
 @pytest.mark.parametrize("rope", [False, True])
-@pytest.mark.parametrize("d,B,H,N", [(64, 1, 3, 1), (64, 2, 5, 2), (64, 2, 3, 9), (64, 1, 12, 20), (32, 2, 3, 4), (32, 1, 5, 7), (32, 20, 16, 10)])
+@pytest.mark.parametrize("d,B,H,N", [(64, 1, 3, 1), (64, 2, 5, 2), (64, 2, 3, 9), (64, 1, 12, 20), (64, 24, 16, 9), (32, 2, 3, 4), (32, 1, 5, 7), (32, 20, 16, 10)])
 def test_operands_formed_from_projections(P, d, B, H, N, rope):
     """The fused call without copies of the operands against forming them first: the same bits."""
     print(f"case linear roles formed d{d} B{B} H{H} N{N} rope{rope}", flush=True)

@@ -2,8 +2,8 @@
 //
 // The f32 matrix instructions bound the kernel with one workgroup per unit (ttt_linear_fwd_dma_kernel): 68 of 32 cycles per
 // wave and mini-batch at head_dim 64, 24 of them for the output, of which nothing is needed for the state.  Here a PRODUCER
-// runs the recurrence alone (44 instructions) and hands G'' of every mini-batch to a CONSUMER on a second CU, which follows with
-// the same updates on a state of its own and forms the output (44).  Nothing flows back: the producer waits for nobody.
+// runs the recurrence alone (40 instructions) and hands G'' of every mini-batch to a CONSUMER on a second CU, which follows with
+// the same updates on a state of its own and forms the output (40).  Nothing flows back: the producer waits for nobody.
 //
 // G'' of a mini-batch [16 x d] is as large as that mini-batch's rows of `out`, which nobody reads before the consumer writes
 // them: it is handed over there, in register layout, so there is no ring to run full.  One word per unit, in W_out, says how many
@@ -40,9 +40,8 @@ constexpr unsigned kLinPairLost = 0x7fc60b5fu;
 template <int D>
 struct LinearPairLds {
   static constexpr int NT = D / 16, RS = 4;
-  f32x4 rows[RS][2][NT][64];  // producer: xk, xv; consumer: xq, xk
+  f32x4 rows[RS][2][NT][64];  // producer: xk, xv; consumer: xq, xk.  Four features of a token each, see `at_row`
   f32x4 g[RS][NT][64];        // G'' with tokens along k: on its way out (two slots) or in
-  f32x4 kd[2][NT][64];        // XK with tokens along k
   f32x4 at[2][NT][64];        // consumer: a wave's share of the attention block
   float lr[RS][64];
   __attribute__((aligned(16))) float ex[2][8 * 16 * NT];
@@ -80,8 +79,8 @@ __device__ __forceinline__ void linear_fwd_pair_body(const LinearFwdArgs& a, con
         const unsigned slot = (unsigned)(stage & (RS - 1)), dst = rows0 + slot * (2 * NT * 1024);
         const int st_ld = min(stage, n - 1);
         // a short mini-batch's last token again in the lanes without one, whose learning rate is made zero: nothing comes of them
-        const int row = REST && st_ld == n - 1 ? min(c, pa.rest - 1) : c;
-        const unsigned off = UnitBase<F32, D>::row_off(st_ld, K, row);
+        const int last = REST && st_ld == n - 1 ? pa.rest - 1 : K - 1, row = min(c, last);
+        const unsigned off = UnitBase<F32, D>::row_off(st_ld, K, min((c - g) & 15, last));
 #pragma unroll
         for (int J = 0; J < NT; ++J) {
           const unsigned fo = (unsigned)(32 * (J >> 1) + 8 * g + 4 * (J & 1)) * 4u;  // the lane's four features of tile J
@@ -175,7 +174,8 @@ __device__ __forceinline__ void linear_fwd_pair_body(const LinearFwdArgs& a, con
   bool upd = te_last != 0.f;
   float sc = upd ? te_last : 1.f, rho_c = a.token_eta[c] / sc;
   const f32x4 ident = identity_frag<F32>(c, g), ones = splat_frag<F32>(1.f);
-  f32x4 ident_upd = upd ? ident : IO::zero(), ones_upd = upd ? ones : IO::zero();
+  f32x4 ones_upd = upd ? ones : IO::zero();
+  unsigned upd_mask = upd ? ~0u : 0u;  // zero token_eta[K-1]: no update
   // the short mini-batch's token_eta, loaded here and taken up in front of it
   float te_rest_last = 0.f, te_rest_c = 0.f;
   if constexpr (REST) {
@@ -187,8 +187,13 @@ __device__ __forceinline__ void linear_fwd_pair_body(const LinearFwdArgs& a, con
     upd = te_rest_last != 0.f;
     sc = upd ? te_rest_last : 1.f;
     rho_c = te_rest_c / sc;
-    ident_upd = upd ? ident : IO::zero();
     ones_upd = upd ? ones : IO::zero();
+    upd_mask = upd ? ~0u : 0u;
+  };
+  const auto masked = [&](const f32x4& x) {
+    u32x4 v = __builtin_bit_cast(u32x4, x);
+    v &= upd_mask;
+    return __builtin_bit_cast(f32x4, v);
   };
   const size_t sb = a.state_per_batch ? bh : (size_t)h;
   const float eps = held(a.eps);
@@ -206,15 +211,29 @@ __device__ __forceinline__ void linear_fwd_pair_body(const LinearFwdArgs& a, con
   centre_state<D, NW, 1>(Wc, bT, a.b0 + sb * D, L.m0s, a.gamma + h * D, sum_a, &L.ex[0][0], w, c, g);
   lds_barrier();
 
+  // Features 4 j .. of a tile of token s lie at 16 j + (s + j) mod 16: sixteen lanes that read a row's features and sixteen that read a
+  // feature of four tokens (four lanes each, all four j) both meet all banks.
+  const int at_row = 16 * g + ((c + g) & 15);
+  // XK with tokens along k, from the rows, not by four matrix instructions in front of Z1, and a write for the other waves (24 units, 63 mini-
+  // batches and five tokens 83.9 -> 82.4 us, a training step of 96 units x 2048 tokens 619 -> 617): element r is feature c of a tile of token 4 g + r
+  const auto tokens_along_k = [&](f32x4 (&kd)[NT], int stage) {
+    const float* const x = reinterpret_cast<const float*>(&L.rows[stage & (RS - 1)][PRODUCER ? 0 : 1][0][0]);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int o = 4 * (16 * (c >> 2) + ((4 * g + r + (c >> 2)) & 15)) + (c & 3);
+#pragma unroll
+      for (int I = 0; I < NT; ++I) kd[I][r] = x[256 * I + o];
+    }
+  };
   // rows of a mini-batch: full rows of what is multiplied by the state, own features of the others
   f32x4 x[2][NT], xo[2], yo[2];  // producer: xk, own xk, own xv; consumer: xq, own xq, own xk
   float lr[2];
   const auto gather = [&](int u, int stage) {
     const int sl = stage & (RS - 1);
 #pragma unroll
-    for (int J = 0; J < NT; ++J) x[u][J] = L.rows[sl][0][J][lane];
-    xo[u] = L.rows[sl][0][w][lane];
-    yo[u] = L.rows[sl][1][w][lane];
+    for (int J = 0; J < NT; ++J) x[u][J] = L.rows[sl][0][J][at_row];
+    xo[u] = L.rows[sl][0][w][at_row];
+    yo[u] = L.rows[sl][1][w][at_row];
     if constexpr (PRODUCER) lr[u] = L.lr[sl][c];
   };
   gather(0, 0);
@@ -246,9 +265,8 @@ __device__ __forceinline__ void linear_fwd_pair_body(const LinearFwdArgs& a, con
     const float b_mean = __builtin_amdgcn_readfirstlane(L.m0s[D]);
     const auto mini_batch = [&](auto u_tag, int st) {
       constexpr int u = decltype(u_tag)::value;
-      f32x4 t = {0.f, 0.f, 0.f, 0.f};
-      IO::mma(t, xo[u], ident_upd);  // XK with tokens along k, the own tile
-      L.kd[u][w][lane] = t;
+      f32x4 kd[NT];
+      tokens_along_k(kd, st);
       f32x4 z1 = bT[0];
 #pragma unroll
       for (int J = 0; J < NT; ++J) IO::mma(z1, Wc[J][0], x[u][J]);
@@ -299,9 +317,6 @@ __device__ __forceinline__ void linear_fwd_pair_body(const LinearFwdArgs& a, con
         for (int ww = 1; ww < NW; ++ww) s += e[(i * 16 + c) * NW + ww];
         S[i] = s;
       }
-      f32x4 kd[NT];
-#pragma unroll
-      for (int I = 0; I < NT; ++I) kd[I] = L.kd[u][I][lane];
       gather(u ^ 1, st + 1);
       const float mu = S[0] * inv_d;
       const float var = S[1] * inv_d - mu * mu;
@@ -315,7 +330,7 @@ __device__ __forceinline__ void linear_fwd_pair_body(const LinearFwdArgs& a, con
       f32x4 Gd = {0.f, 0.f, 0.f, 0.f};
       IO::mma(Gd, G, ident);
 #pragma unroll
-      for (int I = 0; I < NT; ++I) IO::mma(Wc[I][0], kd[I], Gd);
+      for (int I = 0; I < NT; ++I) IO::mma(Wc[I][0], kd[I], masked(Gd));
       IO::mma(bT[0], Gd, ones_upd);
       L.g[u][w][lane] = Gd;
     };
@@ -352,10 +367,9 @@ __device__ __forceinline__ void linear_fwd_pair_body(const LinearFwdArgs& a, con
     };
     const auto mini_batch = [&](auto u_tag, int st) {
       constexpr int u = decltype(u_tag)::value;
-      f32x4 t = {0.f, 0.f, 0.f, 0.f}, At = {0.f, 0.f, 0.f, 0.f};
-      IO::mma(t, yo[u], ident_upd);
+      f32x4 At = {0.f, 0.f, 0.f, 0.f}, kd[NT];
+      tokens_along_k(kd, st);
       IO::mma(At, yo[u], xo[u]);
-      L.kd[u][w][lane] = t;
       L.at[u][w][lane] = At;
       f32x4 zb = bT[0];
 #pragma unroll
@@ -364,9 +378,6 @@ __device__ __forceinline__ void linear_fwd_pair_body(const LinearFwdArgs& a, con
       if (st > 1) emit(so0, so1, st - 2, zbo, qoo);
       lds_barrier();
       collect(u, so0, so1);
-      f32x4 kd[NT];
-#pragma unroll
-      for (int I = 0; I < NT; ++I) kd[I] = L.kd[u][I][lane];
       At = L.at[u][0][lane];
 #pragma unroll
       for (int ww = 1; ww < NW; ++ww) At += L.at[u][ww][lane];
@@ -378,7 +389,7 @@ __device__ __forceinline__ void linear_fwd_pair_body(const LinearFwdArgs& a, con
 #pragma unroll
       for (int r = 0; r < 4; ++r) m[r] = (4 * g + r <= c) ? rho_c * (1.f + At[r]) : 0.f;
 #pragma unroll
-      for (int I = 0; I < NT; ++I) IO::mma(Wc[I][0], kd[I], Gd);
+      for (int I = 0; I < NT; ++I) IO::mma(Wc[I][0], kd[I], masked(Gd));
       IO::mma(bT[0], Gd, ones_upd);
       IO::mma(zb, Gd, m);
       zbp = zb;
