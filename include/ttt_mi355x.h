@@ -101,8 +101,9 @@ typedef struct ttt_desc {
 #define TTT_HINT_TWO_CU 0x400
 /* ttt_linear_fwd, bf16 I/O at head_dim 32 / 64 with two waves per unit: TTT_HINT_OWN_LOADS = every wave loads only the
  * features it owns of xq, xk, xv and the full rows reach the waves through LDS (half the vector loads; the library's
- * choice); TTT_HINT_ALL_LOADS = every wave loads every row.  Same results bit for bit.  Ignored where only one of the two
- * exists (head_dim 96 / 128: own-feature loads).
+ * choice of the two); TTT_HINT_ALL_LOADS = every wave loads every row.  Same results bit for bit.  Ignored where only one of the two
+ * exists (head_dim 96 / 128: own-feature loads).  Without either hint and without a number of waves, mini-batches of 16 run on a
+ * kernel whose waves have roles (recurrence, output, copies) up to one unit per CU at head_dim 64 and two at 32: the same bits.
  * ttt_linear_fwd, f32 I/O with one wave per feature tile (head_dim 32 / 64), whole mini-batches of 16 tokens and at
  * most one (batch, head) unit per CU: the library's choice is a kernel with a fifth wave that copies the operands
  * global -> LDS, so that the four compute waves issue no loads; TTT_HINT_ALL_LOADS keeps the loads in the compute

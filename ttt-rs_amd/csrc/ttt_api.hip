@@ -224,7 +224,7 @@ int launch_linear_fwd_nw(const ttt::LinearFwdArgs* probs, unsigned ny, hipStream
 // 384 units 4 7.7 / 6.8; saving 4 6.7 / 7.1, 8 8.5 / 7.1; head_dim 64, 12 units, 1 6.9 / 6.1, saving 1 7.0 / 7.1, 2 7.8 / 7.2.
 bool linear_fwd_in_roles(int D, const ttt::LinearFwdArgs* probs, int hint, unsigned ny, int rest, int* cus) {
   const ttt::LinearFwdArgs& a = probs[0];
-  if (a.K != 16 || (hint & (TTT_HINT_WAVES_MASK | TTT_HINT_ALL_LOADS | TTT_HINT_ONE_WORKGROUP)) != 0 || any_input_sums(probs, ny)) return false;
+  if (a.K != 16 || (hint & (TTT_HINT_WAVES_MASK | TTT_HINT_ALL_LOADS | TTT_HINT_OWN_LOADS)) != 0 || any_input_sums(probs, ny)) return false;
   bool saves = false;
   for (unsigned y = 0; y < ny; ++y) saves = saves || probs[y].W_ckpt != nullptr;
   if (a.n_stages < (rest > 0 ? 4 : D == 64 ? (saves ? 2 : 1) : (saves ? 8 : 4))) return false;
