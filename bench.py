@@ -222,9 +222,12 @@ class LinearCalls:
 
 
 def fwd_kernel_name(io, units):
-    """The TTT-Linear forward kernel the library picks at head_dim 64 and mini_batch 16: with f32 I/O and a CU per
-    (batch, head) unit the variant with a control wave that copies the operands global -> LDS."""
-    return "ttt_linear_fwd_dma_kernel" if io == "f32" and units <= 256 else "ttt_linear_fwd_sk_kernel"
+    """The TTT-Linear forward kernel the library picks at head_dim 64, mini_batch 16 and 16 or more mini-batches: with f32 I/O and
+    two CUs per (batch, head) unit the one on two workgroups, with one CU the variant with a control wave that copies the
+    operands global -> LDS; with bf16 I/O and a CU per unit the one whose waves have roles."""
+    if io == "f32":
+        return "ttt_linear_fwd_pair_kernel" if units <= 128 else "ttt_linear_fwd_dma_kernel" if units <= 256 else "ttt_linear_fwd_sk_kernel"
+    return "ttt_linear_fwd_roles_kernel" if units <= 256 else "ttt_linear_fwd_sk_kernel"
 
 
 def measured_counters(workload):
