@@ -40,10 +40,12 @@ def dt(P, t):
     return P.TTT_BF16 if t.dtype == torch.bfloat16 else P.TTT_F32
 
 
+# (from four whole mini-batches on the Python mirror makes one launch)
+@pytest.mark.parametrize("N", [3, 8])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["f32", "bf16"])
-def test_cpp_linear_forward_with_remainder_equals_python_mirror(P, drv, dtype):
-    B, H, d, K, seq = 2, 2, 64, 16, 16 * 3 + 5
-    print(f"case host C++ linear forward+remainder {dtype}", flush=True)
+def test_cpp_linear_forward_with_remainder_equals_python_mirror(P, drv, dtype, N):
+    B, H, d, K, seq = 2, 2, 64, 16, 16 * N + 5
+    print(f"case host C++ linear forward+remainder {dtype} N{N}", flush=True)
     c = to_dev(P.synthetic.reference_test_inputs(13, B, H, seq, d, K, io_dtype=dtype))
     te_seq = c["token_eta"].repeat(seq // K + 1)[:seq].contiguous()
     model = P.FusedTileMulti(P.ModelConfig(H, d, P.TTTConfig(mini_batch_size=K)), c["W0"], c["b0"], c["gamma"], c["beta"])

@@ -1014,8 +1014,8 @@ int dispatch_linear_fwd_pack(const ttt_desc* d, const ttt::LinearFwdArgs* a, uns
 // on one / two workgroups, d = 64, 24 units, 8 mini-batches 17.9 / 18.6 us, 12 23.6 / 22.8, 16 29.9 / 27.1, 63 102 / 76, 128 202 / 144;
 // 128 units, 12 24.8 / 24.4, 16 31.0 / 28.7; d = 32, 24 units, 12 17.1 / 17.4, 16 21.4 / 20.4, 63 72.6 / 56.5, 128 143.5 / 105.5.
 // `rest` tokens of a short mini-batch behind save the launch that they would take otherwise, and pay from four mini-batches on (the
-// fewest tried): 24 units, d = 64, 4 19.2 / 15.5, 8 25.7 / 19.7, 16 37.7 / 28.1; d = 32, 4 14.0 / 12.3, 16 27.1 / 21.1; 128 units, d = 64, 4
-// 20.1 / 16.2.
+// fewest tried): on one workgroup and two launches / on two workgroups and one, 24 units, d = 64, 4 19.1 / 16.7, 8 25.7 / 20.9, 16 37.8 /
+// 29.1; d = 32, 4 13.8 / 12.8, 16 27.1 / 21.3; 128 units, d = 64, 4 20.2 / 18.3.
 bool linear_fwd_on_pairs(const ttt_desc* d, const ttt::LinearFwdArgs& a, ttt::LinearPairArgs* pa, int rest = 0) {
   if (d->io_dtype != TTT_F32 || d->head_dim > 64 || a.K != 16) return false;
   if (d->kernel_hint & (TTT_HINT_WAVES_MASK | TTT_HINT_ALL_LOADS | TTT_HINT_ONE_WORKGROUP)) return false;

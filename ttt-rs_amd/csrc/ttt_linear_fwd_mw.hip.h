@@ -329,6 +329,118 @@ __device__ __forceinline__ void store_state_final(float* Wd, float* bd, const f3
   }
 }
 
+// ---- The state between the whole mini-batches of a sequence and a short one in the same launch ---------------------
+// Two launches write the state in between (store_state_final) and centre it anew (centre_state): two roundings that belong to the
+// result, which must not depend on how many launches a caller's shape takes.  One launch does the same to its registers:
+// the initial state waits in LDS (keep), `form` makes the state as it would be written and leaves row sums and bias, and behind a
+// barrier `centre` takes the means off, in centre_state's order of additions.  For the NW waves that carry the recurrence.
+template <int D, int NW, int TPW>
+struct StateBetween {
+  static constexpr int NT = D / 16;
+  f32x4 W0[NT][TPW][NW][64], b0[TPW][NW][64];  // the initial state, in lane order; W0 from `form` on: the weights in between
+  __attribute__((aligned(16))) float sums[D * NW];
+  __attribute__((aligned(16))) float b[D];        // the bias in between
+  __attribute__((aligned(16))) float m0s[D + 4];  // the new means, as centre_state leaves them
+
+  // before centre_state
+  __device__ __forceinline__ void keep(const f32x4 (&Wc)[NT][TPW], const f32x4 (&bT)[TPW], int w, int lane) {
+#pragma unroll
+    for (int jj = 0; jj < TPW; ++jj) {
+#pragma unroll
+      for (int I = 0; I < NT; ++I) W0[I][jj][w][lane] = Wc[I][jj];
+      b0[jj][w][lane] = bT[jj];
+    }
+  }
+  // m0s_now: the means that Wc and bT are centred by
+  __device__ __forceinline__ void form(f32x4 (&Wc)[NT][TPW], f32x4 (&bT)[TPW], const float* m0s_now, int w, int c, int g) {
+    const int lane = 16 * g + c;
+    const float bb = m0s_now[D];
+#pragma unroll
+    for (int jj = 0; jj < TPW; ++jj) {
+      const f32x4 v0 = b0[jj][w][lane];
+      f32x4 start = v0;
+      start -= bb;
+      bT[jj] = v0 + (bT[jj] - start);
+      if (c == 0) *reinterpret_cast<f32x4*>(b + own_offset<TPW>(w, jj, g)) = bT[jj];
+    }
+#pragma unroll
+    for (int I = 0; I < NT; ++I) {
+      const f32x4 m = *reinterpret_cast<const f32x4*>(m0s_now + I * 16 + 4 * g);
+      f32x4 p;
+#pragma unroll
+      for (int jj = 0; jj < TPW; ++jj) {
+        const f32x4 w0 = W0[I][jj][w][lane];
+        const f32x4 start = w0 - m;
+        Wc[I][jj] = w0 + (Wc[I][jj] - start);
+        W0[I][jj][w][lane] = Wc[I][jj];
+        p = jj == 0 ? Wc[I][0] : p + Wc[I][jj];
+      }
+      p = over_tokens(p);
+      if (c == 0) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) sums[(I * 16 + 4 * g + r) * NW + w] = p[r];
+      }
+    }
+  }
+  // behind a barrier
+  __device__ __forceinline__ void centre(f32x4 (&Wc)[NT][TPW], f32x4 (&bT)[TPW], int w, int c, int g) {
+    float s = 0.f;
+#pragma unroll
+    for (int f = 0; f < D; f += 4) {
+      const f32x4 v = *reinterpret_cast<const f32x4*>(b + f);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) s += v[i];
+    }
+    const float bb = s * (1.0f / D);
+#pragma unroll
+    for (int jj = 0; jj < TPW; ++jj) bT[jj] -= bb;
+#pragma unroll
+    for (int I = 0; I < NT; ++I) {
+      f32x4 m;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        float t = sums[(I * 16 + 4 * g + r) * NW];
+#pragma unroll
+        for (int ww = 1; ww < NW; ++ww) t += sums[(I * 16 + 4 * g + r) * NW + ww];
+        m[r] = t * (1.0f / D);
+      }
+      if (w == 0 && c == 0) *reinterpret_cast<f32x4*>(m0s + I * 16 + 4 * g) = m;
+#pragma unroll
+      for (int jj = 0; jj < TPW; ++jj) Wc[I][jj] -= m;
+    }
+    if (w == 0 && c == 0 && g == 0) m0s[D] = bb;
+  }
+  __device__ __forceinline__ void weights(f32x4 (&W)[NT][TPW], int w, int lane) const {
+#pragma unroll
+    for (int I = 0; I < NT; ++I)
+#pragma unroll
+      for (int jj = 0; jj < TPW; ++jj) W[I][jj] = W0[I][jj][w][lane];
+  }
+};
+// ... where other waves of the workgroup follow with a state of their own: they take the centred one over, behind a barrier
+template <int D, int NW, int TPW>
+struct StateBetweenShared : StateBetween<D, NW, TPW> {
+  static constexpr int NT = D / 16;
+  f32x4 W1[NT][TPW][NW][64], b1[TPW][NW][64];
+  __device__ __forceinline__ void give(const f32x4 (&Wc)[NT][TPW], const f32x4 (&bT)[TPW], int w, int lane) {
+#pragma unroll
+    for (int jj = 0; jj < TPW; ++jj) {
+#pragma unroll
+      for (int I = 0; I < NT; ++I) W1[I][jj][w][lane] = Wc[I][jj];
+      b1[jj][w][lane] = bT[jj];
+    }
+  }
+  __device__ __forceinline__ void take(f32x4 (&Wc)[NT][TPW], f32x4 (&bT)[TPW], int w, int lane) const {
+#pragma unroll
+    for (int jj = 0; jj < TPW; ++jj) {
+#pragma unroll
+      for (int I = 0; I < NT; ++I) Wc[I][jj] = W1[I][jj][w][lane];
+      bT[jj] = b1[jj][w][lane];
+    }
+  }
+};
+struct NoStateBetween {};
+
 // Where one (batch, head) unit's rows start, as wave-uniform byte pointers formed once; a token's row is then a
 // 32-bit byte offset from them (a unit spans at most seq_stride * d * 4 bytes), which is what the addressing of
 // global loads and stores takes directly: scalar base plus 32-bit lane offset, no 64-bit arithmetic and no renewed

@@ -18,10 +18,11 @@
 // COURIER stores G'' and the word, or watches the word and copies G'' global -> LDS.  One barrier per mini-batch.
 //
 // A sequence may end in a short mini-batch (REST), which is then the last one of both workgroups instead of a launch of its own:
-// its rows are read once more for the lanes without a token, with a learning rate of zero.  A launch of one short mini-batch took 8 us:
-// 63 mini-batches and five tokens, 24 units, head_dim 64, 89.6 -> 83.8 us.
+// the lanes without a token have rows of zeros and a learning rate of zero, and the state in front of it is what two launches would hand
+// over (StateBetween, 1.3 us of the call).  63 mini-batches and five tokens, 24 units, head_dim 64, with a launch of its own 89.6 us, in
+// this one 83.3.
 //
-// The arithmetic is that of one workgroup, bit for bit.
+// The arithmetic is that of one workgroup, and with a short mini-batch that of two launches, bit for bit.
 #pragma once
 #include "ttt_linear_fwd_sk.hip.h"
 
@@ -37,7 +38,7 @@ struct LinearPairArgs {
 constexpr int kLinPairWords = 64, kLinPairCount = 0, kLinPairXcd = 32;
 constexpr unsigned kLinPairLost = 0x7fc60b5fu;
 
-template <int D>
+template <int D, bool REST>
 struct LinearPairLds {
   static constexpr int NT = D / 16, RS = 4;
   f32x4 rows[RS][2][NT][64];  // producer: xk, xv; consumer: xq, xk.  Four features of a token each, see `at_row`
@@ -46,13 +47,14 @@ struct LinearPairLds {
   float lr[RS][64];
   __attribute__((aligned(16))) float ex[2][8 * 16 * NT];
   __attribute__((aligned(16))) float m0s[D + 4];
+  std::conditional_t<REST, StateBetween<D, NT, 1>, NoStateBetween> between;
   int lost;
 };
 
 template <int D, bool PRODUCER, bool CKPT, bool REST>
-__device__ __forceinline__ void linear_fwd_pair_body(const LinearFwdArgs& a, const LinearPairArgs& pa, LinearPairLds<D>& L, size_t bh) {
+__device__ __forceinline__ void linear_fwd_pair_body(const LinearFwdArgs& a, const LinearPairArgs& pa, LinearPairLds<D, REST>& L, size_t bh) {
   using IO = Io<F32>;
-  constexpr int NT = D / 16, NW = NT, RS = LinearPairLds<D>::RS;
+  constexpr int NT = D / 16, NW = NT, RS = LinearPairLds<D, REST>::RS;
   constexpr float inv_d = 1.0f / D;
   constexpr int K = 16;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
@@ -78,7 +80,7 @@ __device__ __forceinline__ void linear_fwd_pair_body(const LinearFwdArgs& a, con
       const auto copy_in = [&](int stage) {  // (past the end: the last one again, into a slot nobody reads)
         const unsigned slot = (unsigned)(stage & (RS - 1)), dst = rows0 + slot * (2 * NT * 1024);
         const int st_ld = min(stage, n - 1);
-        // a short mini-batch's last token again in the lanes without one, whose learning rate is made zero: nothing comes of them
+        // (a short mini-batch's last token again in the lanes without one, until they are cleared below)
         const int last = REST && st_ld == n - 1 ? pa.rest - 1 : K - 1, row = min(c, last);
         const unsigned off = UnitBase<F32, D>::row_off(st_ld, K, min((c - g) & 15, last));
 #pragma unroll
@@ -95,7 +97,17 @@ __device__ __forceinline__ void linear_fwd_pair_body(const LinearFwdArgs& a, con
       asm volatile("s_waitcnt vmcnt(%0)" ::"n"((RS - 1) * kCopies) : "memory");  // mini-batch 0 has landed
       asm volatile("s_barrier" ::: "memory");
       for (int st = 0; st < n; ++st) {
+        if (REST && st == n - 1) asm volatile("s_barrier" ::: "memory");           // of StateBetween
         asm volatile("s_waitcnt vmcnt(%0)" ::"n"((RS - 2) * kCopies) : "memory");  // mini-batch st + 1 has landed
+        if (REST && st == n - 2) {  // the short one: zeros in the lanes without a token
+          const int sl = (n - 1) & (RS - 1);
+          if (((c - g) & 15) >= pa.rest) {
+#pragma unroll
+            for (int i = 0; i < 2 * NT; ++i) L.rows[sl][i / NT][i % NT][lane] = f32x4{0.f, 0.f, 0.f, 0.f};
+          }
+          if (PRODUCER && c >= pa.rest) L.lr[sl][lane] = 0.f;
+          lds_done();
+        }
         asm volatile("s_barrier" ::: "memory");
         copy_in(st + RS);
       }
@@ -129,6 +141,12 @@ __device__ __forceinline__ void linear_fwd_pair_body(const LinearFwdArgs& a, con
       for (int st = 1; st <= n; ++st) {
         asm volatile("s_barrier" ::: "memory");
         hand_over(st - 1);
+        if (REST && st == n - 2) {  // StateBetween has a barrier: G'' of n - 2 need not wait for the next, nor the consumer's state
+          asm volatile("s_barrier" ::: "memory");
+          hand_over(st);
+          ++st;
+          asm volatile("s_barrier" ::: "memory");
+        }
       }
     } else {
       if (lane == 0) __hip_atomic_store(words + kLinPairXcd, xcd, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -138,6 +156,7 @@ __device__ __forceinline__ void linear_fwd_pair_body(const LinearFwdArgs& a, con
       centre();
       asm volatile("s_barrier" ::: "memory");
       for (int st = 0; st < n; ++st) {
+        if (REST && st == n - 1) asm volatile("s_barrier" ::: "memory");  // of StateBetween
         // G'' of mini-batch st in LDS in front of the barrier of st, and of the next two if they are there: the slot of st + 2 was
         // last read behind the barrier of st - 2, which every wave left in front of that of st - 1
         if (!lost && known < n) {
@@ -207,6 +226,7 @@ __device__ __forceinline__ void linear_fwd_pair_body(const LinearFwdArgs& a, con
     a2[r] = gam[r] * gam[r];
   }
   load_state_slice<D, 1>(Wc, a.W0 + sb * D * D, w, c, g);
+  if constexpr (REST) L.between.keep(Wc, bT, w, lane);
   float sum_a;  // of gamma^2
   centre_state<D, NW, 1>(Wc, bT, a.b0 + sb * D, L.m0s, a.gamma + h * D, sum_a, &L.ex[0][0], w, c, g);
   lds_barrier();
@@ -238,8 +258,8 @@ __device__ __forceinline__ void linear_fwd_pair_body(const LinearFwdArgs& a, con
   };
   gather(0, 0);
 
-  // all mini-batches; `mask` comes in front of a short one
-  const auto run = [&](const auto& mini_batch, const auto& mask) {
+  // all mini-batches
+  const auto run = [&](const auto& mini_batch) {
     constexpr std::integral_constant<int, 0> even{};
     constexpr std::integral_constant<int, 1> odd{};
     int st = 0;
@@ -250,13 +270,13 @@ __device__ __forceinline__ void linear_fwd_pair_body(const LinearFwdArgs& a, con
     if (st < a.n_stages) mini_batch(even, st);
     if constexpr (REST) {
       take_rest();
-      if (st < a.n_stages) {
-        mask(odd);
+      L.between.form(Wc, bT, L.m0s, w, c, g);
+      lds_barrier();
+      L.between.centre(Wc, bT, w, c, g);
+      if (st < a.n_stages)
         mini_batch(odd, n - 1);
-      } else {
-        mask(even);
+      else
         mini_batch(even, n - 1);
-      }
     }
   };
 
@@ -334,9 +354,7 @@ __device__ __forceinline__ void linear_fwd_pair_body(const LinearFwdArgs& a, con
       IO::mma(bT[0], Gd, ones_upd);
       L.g[u][w][lane] = Gd;
     };
-    run(mini_batch, [&](auto u_tag) {
-      if (c >= pa.rest) lr[decltype(u_tag)::value] = 0.f;
-    });
+    run(mini_batch);
     lds_barrier();  // the last G''
   } else {
     // pending output of the last mini-batch (its sums travel in the next exchange) and of the one before (sums known)
@@ -395,16 +413,21 @@ __device__ __forceinline__ void linear_fwd_pair_body(const LinearFwdArgs& a, con
       zbp = zb;
       qop = xo[u];
     };
-    run(mini_batch, [](auto) {});
+    run(mini_batch);
     f32x4 W0[NT][1];
-    load_state_slice<D, 1>(W0, a.W0 + sb * D * D, w, c, g);
+    if constexpr (!REST) load_state_slice<D, 1>(W0, a.W0 + sb * D * D, w, c, g);
     publish(n & 1);
     lds_barrier();
     float s0, s1;
     collect(n & 1, s0, s1);
     if (n >= 2) emit(so0, so1, n - 2, zbo, qoo);
     if (!REST || c < pa.rest) emit(s0, s1, n - 1, zbp, qop);
-    store_state_final<D, 1>(a.W_out + bh * D * D, a.b_out + bh * D, W0, a.b0 + sb * D, Wc, bT, L.m0s, w, c, g);
+    if constexpr (REST) {
+      L.between.weights(W0, w, lane);
+      store_state_final<D, 1>(a.W_out + bh * D * D, a.b_out + bh * D, W0, L.between.b, Wc, bT, L.between.m0s, w, c, g);
+    } else {
+      store_state_final<D, 1>(a.W_out + bh * D * D, a.b_out + bh * D, W0, a.b0 + sb * D, Wc, bT, L.m0s, w, c, g);
+    }
     // element (0, 0) of W_out is written by the lane that marks the unit
     if (L.lost != 0 && threadIdx.x == 0) *reinterpret_cast<unsigned*>(a.W_out + bh * D * D) = kLinPairLost;
   }
@@ -414,7 +437,7 @@ __device__ __forceinline__ void linear_fwd_pair_body(const LinearFwdArgs& a, con
 // the producer, which waits for nobody, is dispatched first.
 template <int D, bool CKPT, bool REST>
 __global__ void __launch_bounds__(64 * (D / 16 + 2)) ttt_linear_fwd_pair_kernel(LinearFwdArgs a, LinearPairArgs pa) {
-  __shared__ LinearPairLds<D> L;
+  __shared__ LinearPairLds<D, REST> L;
   const size_t bh = (size_t)(blockIdx.x >> 4) * 8 + (blockIdx.x & 7);
   if (bh >= (size_t)a.B * a.H) return;
   if (((blockIdx.x >> 3) & 1) == 0)

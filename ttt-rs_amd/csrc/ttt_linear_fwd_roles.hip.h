@@ -20,15 +20,17 @@
 // place; in the two-wave kernel (RAW = 1) they are instructions of the waves that carry the recurrence.  128 mini-batches, head_dim 64, 12
 // units 135.0 -> 78.1 us, 256 138.6 -> 81.6; head_dim 32, 256 units 97.1 -> 53.7, 384 126.8 -> 73.3.
 //
-// REST: a short mini-batch behind the whole ones is the last one, as in ttt_linear_fwd_pair.hip.h.
+// REST: a short mini-batch behind the whole ones is the last one, as in ttt_linear_fwd_pair.hip.h; the chain waves form the state in
+// front of it (StateBetween) and the output waves take it over.  24 units, five tokens behind four mini-batches, two launches with two
+// waves / one in roles: head_dim 64 16.0 / 10.1 us, 32 11.1 / 6.4; behind 63 63.8 / 44.4 and 42.4 / 29.3.
 //
-// The arithmetic is that of ttt_linear_fwd_sk_kernel, bit for bit.
+// The arithmetic is that of ttt_linear_fwd_sk_kernel, and with a short mini-batch that of two launches of it, bit for bit.
 #pragma once
 #include "ttt_linear_fwd_sk.hip.h"
 
 namespace ttt {
 
-template <int D>
+template <int D, bool REST = false>
 struct LinearRolesLds {
   static constexpr int NT = D / 16, NW = 2, TPW = NT / NW, RS = 8;
   u32x4 rows[RS][3][NT / 2][64];  // xq, xk, xv: lane (c, g) the features 32 q + 8 g .. + 7 of token c
@@ -37,17 +39,18 @@ struct LinearRolesLds {
   __attribute__((aligned(16))) float ex[2][6 * 16 * NW];
   __attribute__((aligned(16))) float ez[2][2 * 16 * NW];
   __attribute__((aligned(16))) float m0s[D + 4];
+  std::conditional_t<REST, StateBetweenShared<D, NW, TPW>, NoStateBetween> between;
 };
 
 // SAVE 0: nothing.  1: states.  2: update factors.
 // FORM: the operands are formed from the projections (FusedInputsArgs, no copies of them asked for, positions that repeat with the
 // mini-batch), by a second copy wave.
 template <int D, int SAVE, bool TWO, bool REST, bool FORM = false>
-__device__ __forceinline__ void linear_fwd_roles_body(const LinearFwdArgs& a, LinearRolesLds<D>& L, bool flip, int rest,
+__device__ __forceinline__ void linear_fwd_roles_body(const LinearFwdArgs& a, LinearRolesLds<D, REST>& L, bool flip, int rest,
                                                       const FusedInputsArgs* fi = nullptr) {
   using IO = Io<BF16>;
   using frag = IO::frag;
-  using LD = LinearRolesLds<D>;
+  using LD = LinearRolesLds<D, REST>;
   constexpr int NT = D / 16, NW = LD::NW, TPW = LD::TPW, RS = LD::RS, K = 16;
   constexpr float inv_d = 1.0f / D;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
@@ -111,7 +114,7 @@ __device__ __forceinline__ void linear_fwd_roles_body(const LinearFwdArgs& a, Li
     const auto copy_in = [&](int stage) {  // (past the end: the last one again, into a slot nobody reads)
       const unsigned slot = (unsigned)(stage & (RS - 1)), dst = rows0 + slot * (3 * (NT / 2) * 1024);
       const int st_ld = min(stage, n - 1);
-      // a short mini-batch's last token again in the lanes without one, whose learning rate is made zero: nothing comes of them
+      // (a short mini-batch's last token again in the lanes without one, until they are cleared below)
       const int row = REST && st_ld == n - 1 ? min(c, rest - 1) : c;
       const unsigned t = ((unsigned)st_ld * (unsigned)K + (unsigned)row) * pitch, off = t * (D * 2u) + 16u * (unsigned)g;
 #pragma unroll
@@ -130,8 +133,18 @@ __device__ __forceinline__ void linear_fwd_roles_body(const LinearFwdArgs& a, Li
     asm volatile("s_barrier" ::: "memory");
     if constexpr (FORM) asm volatile("s_barrier" ::: "memory");
     for (int st = 0; st < n; ++st) {
+      if (REST && st == n - 1) asm volatile("s_barrier" ::: "memory");  // of StateBetween
       // mini-batch st + 1 has landed (FORM: st + 2); the slot of mini-batch st - 2 was last read in front of this barrier, by the output waves
       asm volatile("s_waitcnt vmcnt(%0)" ::"n"((RS - (FORM ? 5 : 4)) * kCopies) : "memory");
+      if (REST && st == n - 2) {  // the short one: zeros in the lanes without a token
+        const int sl = (n - 1) & (RS - 1);
+        if (c >= rest) {
+#pragma unroll
+          for (int i = 0; i < 3 * (NT / 2); ++i) L.rows[sl][i / (NT / 2)][i % (NT / 2)][lane] = u32x4{0u, 0u, 0u, 0u};
+          L.lr[sl][lane] = 0u;
+        }
+        lds_done();
+      }
       asm volatile("s_barrier" ::: "memory");
       copy_in(st + RS - 2);
     }
@@ -178,6 +191,7 @@ __device__ __forceinline__ void linear_fwd_roles_body(const LinearFwdArgs& a, Li
       a2[jj][r] = gam[jj][r] * gam[jj][r];
     }
   load_state_slice<D, TPW>(Wc, a.W0 + sb * D * D, w, c, g);
+  if constexpr (REST) L.between.keep(Wc, bT, w, lane);
   centre_state<D, NW, TPW>(Wc, bT, a.b0 + sb * D, L.m0s, a.gamma + h * D, sum_a, scratch, w, c, g);
   lds_barrier();
   if constexpr (FORM) lds_barrier();
@@ -312,7 +326,10 @@ __device__ __forceinline__ void linear_fwd_roles_body(const LinearFwdArgs& a, Li
     if (st < whole) mini_batch(std::integral_constant<int, 0>{}, st);
     if constexpr (REST) {
       take_rest();
-      if (c >= rest) lr_next = 0.f;
+      L.between.form(Wc, bT, L.m0s, w, c, g);
+      lds_barrier();
+      L.between.centre(Wc, bT, w, c, g);
+      L.between.give(Wc, bT, w, lane);
       if (st < whole)
         mini_batch(std::integral_constant<int, 1>{}, whole);
       else
@@ -320,9 +337,16 @@ __device__ __forceinline__ void linear_fwd_roles_body(const LinearFwdArgs& a, Li
     }
     lds_barrier();
     f32x4 W0[NT][TPW];
-    load_state_slice<D, TPW>(W0, a.W0 + sb * D * D, w, c, g);
+    if constexpr (!REST) load_state_slice<D, TPW>(W0, a.W0 + sb * D * D, w, c, g);
     lds_barrier();
-    store_state_final<D, TPW>(a.W_out + bh * D * D, a.b_out + bh * D, W0, a.b0 + sb * D, Wc, bT, L.m0s, w, c, g);
+    if constexpr (REST) {
+      int c_end = c, g_end = g;  // (or the addresses, formed from the same lane indices as the prologue's, are kept: 16 spilled registers)
+      asm volatile("" : "+v"(c_end), "+v"(g_end));
+      L.between.weights(W0, w, lane);
+      store_state_final<D, TPW>(a.W_out + bh * D * D, a.b_out + bh * D, W0, L.between.b, Wc, bT, L.between.m0s, w, c_end, g_end);
+    } else {
+      store_state_final<D, TPW>(a.W_out + bh * D * D, a.b_out + bh * D, W0, a.b0 + sb * D, Wc, bT, L.m0s, w, c, g);
+    }
     if constexpr (SAVE == 2)
       store_state_tiles<D, TPW>(a.W_ckpt + bh * (size_t)a.n_ckpt * (D * D), a.b_ckpt + bh * (size_t)a.n_ckpt * D, Wc, bT, w, lane);
     return;
@@ -359,7 +383,12 @@ __device__ __forceinline__ void linear_fwd_roles_body(const LinearFwdArgs& a, Li
   for (int m = 0; m < n; ++m) {
     const int sl = m & (RS - 1);
     if (m > 0) emit(m - 1);
-    if (REST && m == whole) take_rest();
+    if constexpr (REST) {
+      if (m == whole) {  // the recurrence left its state two barriers ago
+        take_rest();
+        L.between.take(Wc, bT, w, lane);
+      }
+    }
     frag q[NT], k[NT], kd[NT], Gd[TPW];
     full_rows(q, sl, 0);
     full_rows(k, sl, 1);
@@ -402,6 +431,7 @@ __device__ __forceinline__ void linear_fwd_roles_body(const LinearFwdArgs& a, Li
 #pragma unroll
     for (int jj = 0; jj < TPW; ++jj) IO::mma(zb[jj], Gd[jj], Mf);
     update(kd, Gd);
+    if (REST && m == n - 3) asm volatile("s_barrier" ::: "memory");  // of StateBetween (the recurrence is two mini-batches ahead)
     float s0 = 0.f, s1 = 0.f;
 #pragma unroll
     for (int jj = 0; jj < TPW; ++jj)
@@ -419,7 +449,7 @@ __device__ __forceinline__ void linear_fwd_roles_body(const LinearFwdArgs& a, Li
 
 template <int D, int SAVE, bool TWO, bool REST>
 __global__ void __launch_bounds__(64 * 5, TWO ? 3 : 2) ttt_linear_fwd_roles_kernel(Problems<LinearFwdArgs> P, int cus, int rest) {
-  __shared__ LinearRolesLds<D> L;
+  __shared__ LinearRolesLds<D, REST> L;
   linear_fwd_roles_body<D, SAVE, TWO, REST>(P.p[blockIdx.y], L, TWO && (int)(blockIdx.y * gridDim.x + blockIdx.x) >= cus, rest);
 }
 
