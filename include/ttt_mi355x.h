@@ -185,7 +185,7 @@ int ttt_linear_fwd(const ttt_desc* desc, const void* xq, const void* xk, const v
  * ttt_linear_fwd on desc->seq tokens and, in the same launch, on the `rest` tokens behind them (1 .. mini_batch - 1) as one short
  * mini-batch: bit for bit what a second call with seq = mini_batch = rest on the windows behind the first would give.  desc->seq_stride >= seq + rest; token_eta: the entries [0, K) and
  * [seq, seq + rest) are read.  For calls of four or more mini-batches that run a unit on two workgroups (see above),
- * and with bf16 I/O at head_dim 64 up to one unit per CU, at head_dim 32 up to two;
+ * W_out on a 16-byte boundary, and with bf16 I/O at head_dim 64 up to one unit per CU, at head_dim 32 up to two;
  * any other call returns TTT_ERR_UNSUPPORTED with nothing enqueued, and two calls of ttt_linear_fwd do the work.
  */
 int ttt_linear_fwd_with_rest(const ttt_desc* desc, int32_t rest, const void* xq, const void* xk, const void* xv,

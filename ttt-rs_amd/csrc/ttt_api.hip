@@ -1020,6 +1020,7 @@ bool linear_fwd_on_pairs(const ttt_desc* d, const ttt::LinearFwdArgs& a, ttt::Li
   if (d->io_dtype != TTT_F32 || d->head_dim > 64 || a.K != 16) return false;
   if (d->kernel_hint & (TTT_HINT_WAVES_MASK | TTT_HINT_ALL_LOADS | TTT_HINT_ONE_WORKGROUP)) return false;
   if (a.n_stages < (rest > 0 ? 4 : 16)) return false;
+  if (rest > 0 && !aligned16(a.W_out)) return false;  // the short mini-batch's G'' crosses there, 16 bytes a lane; else W_out goes by elements
   const size_t units = (size_t)a.B * a.H;
   int cus = 0;
   if (device_cus(&cus) != TTT_OK || (units + 7) / 8 * 16 > (size_t)cus) return false;
