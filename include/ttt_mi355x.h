@@ -187,7 +187,10 @@ int ttt_linear_fwd(const ttt_desc* desc, const void* xq, const void* xk, const v
  * [seq, seq + rest) are read.  For calls of four or more mini-batches that run a unit on two workgroups (see above),
  * W_out on a 16-byte boundary, and with bf16 I/O at head_dim 64 up to one unit per CU, at head_dim 32 up to two;
  * any other call returns TTT_ERR_UNSUPPORTED with nothing enqueued, and two calls of ttt_linear_fwd do the work.
+ * ttt_linear_fwd_takes_rest: 1 where the current device has the one launch for this shape, otherwise 0 (also for a desc that no call
+ * takes); ttt_last_error() stays as it was.  What depends on the buffers (overlaps, the alignment of W_out) is not part of the answer.
  */
+int ttt_linear_fwd_takes_rest(const ttt_desc* desc, int32_t rest);
 int ttt_linear_fwd_with_rest(const ttt_desc* desc, int32_t rest, const void* xq, const void* xk, const void* xv,
                              const float* W0, const float* b0, const float* token_eta, const void* lr,
                              const float* gamma, const float* beta, void* out, float* W_out, float* b_out, void* stream);

@@ -74,6 +74,19 @@ def test_shape_validation(P):
     assert b"checkpoint_format" in L.ttt_last_error()
 
 
+def test_asking_for_the_one_launch_leaves_no_error_text(P):
+    """ttt_linear_fwd_takes_rest says no (here there is no device at all) without a failure of the thread's last call."""
+    L = P.lib()
+    assert L.ttt_linear_supported(C.byref(desc(P, checkpoint_interval=0))) == P.TTT_ERR_SHAPE
+    before = L.ttt_last_error()
+    ask = lambda rest=5, **kw: L.ttt_linear_fwd_takes_rest(C.byref(desc(P, **{"seq": 64, "seq_stride": 69, **kw})), rest)
+    for answer in (ask(rest=0), ask(rest=16), ask(seq=33), ask(head_dim=48), ask(head_dim=96), ask(seq_stride=0), ask(seq_stride=68),
+                   ask(mini_batch=32, head_dim=32, seq_stride=99), L.ttt_linear_fwd_takes_rest(None, 5)):
+        assert answer == 0
+    assert ask() in (0, 1)
+    assert before and L.ttt_last_error() == before
+
+
 def test_best_checkpoint_format(P):
     L = P.lib()
     best = lambda **kw: L.ttt_linear_best_checkpoint_format(C.byref(desc(P, **kw)))

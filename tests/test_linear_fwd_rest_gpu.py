@@ -111,6 +111,44 @@ def test_bits_do_not_depend_on_the_batch(P, dtype, d, few, many):
         assert torch.equal(x, y[:few]), f"output {i}"
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_the_question_agrees_with_the_call(P, dtype):
+    """ttt_linear_fwd_takes_rest against what ttt_linear_fwd_with_rest answers, around the limits in mini-batches, units and head_dim."""
+    L, io, dev, rest = P.lib(), P.TTT_F32 if dtype == torch.float32 else P.TTT_BF16, "cuda:0", 3
+    p = lambda t: ctypes.c_void_p(t.data_ptr())
+    s = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    said = []
+    for d in (32, 64, 96, 128):
+        for B, H, N in ((1, 2, 3), (1, 2, 4), (8, 16, 4), (43, 3, 4), (16, 16, 4), (257, 1, 4), (32, 16, 4), (57, 9, 4)):
+            seq = N * K + rest
+            x, lr = torch.zeros(B, H, seq, d, device=dev, dtype=dtype), torch.zeros(B, H, seq, device=dev, dtype=dtype)
+            out, te, one = torch.empty_like(x), torch.ones(seq, device=dev), torch.ones(H, d, d, device=dev)
+            W, b = torch.empty(B, H, d, d, device=dev), torch.empty(B, H, d, device=dev)
+            ds = P.TttDesc(B, H, N * K, d, K, 1e-6, 1, io)
+            ds.seq_stride = seq
+            print(f"case linear rest asked {dtype} d{d} B{B} H{H} N{N}", flush=True)
+            asked = L.ttt_linear_fwd_takes_rest(ctypes.byref(ds), rest)
+            rc = L.ttt_linear_fwd_with_rest(ctypes.byref(ds), rest, p(x), p(x), p(x), p(one), p(one), p(te), p(lr), p(one), p(one), p(out),
+                                            p(W), p(b), s)
+            torch.cuda.synchronize()
+            assert rc == (P.TTT_OK if asked else P.TTT_ERR_UNSUPPORTED), (d, B, H, N)
+            said.append(asked)
+    assert 0 in said and 1 in said
+
+
+def test_a_call_that_succeeds_leaves_no_error_text(P):
+    """A layer's pass over a ragged sequence whose shape has no single launch."""
+    v = inputs(P, 64, 1, 2, 3, 5)
+    layer = P.FusedTileMulti(P.ModelConfig(2, 64, P.TTTConfig(mini_batch_size=K)), v["W0"], v["b0"], v["gamma"], v["beta"])
+    print("case linear rest error text", flush=True)
+    L = P.lib()
+    assert L.ttt_linear_supported(None) == P.TTT_ERR_NULL
+    before = L.ttt_last_error()
+    layer.forward(layer.init_state(1), P.TTTInputsInner(P.Qkv(v["xq"], v["xk"], v["xv"]), v["token_eta"], v["lr"]))
+    torch.cuda.synchronize()
+    assert before and L.ttt_last_error() == before
+
+
 def test_calls_without_one_launch_are_refused(P):
     v = inputs(P, 64, 1, 2, 3, 5)
     with pytest.raises(AssertionError, match="no single launch"):

@@ -222,13 +222,17 @@ int launch_linear_fwd_nw(const ttt::LinearFwdArgs* probs, unsigned ny, hipStream
 // head_dim 64 up to a unit per CU, 32 up to two (both measured there).  Few mini-batches at head_dim 32 lose to the longer
 // way into the loop, more so where the launch saves: two waves / in roles, 12 units, 1 mini-batch 5.4 / 5.8, 3 5.92 / 5.97, 4 6.5 / 5.8,
 // 384 units 4 7.7 / 6.8; saving 4 6.7 / 7.1, 8 8.5 / 7.1; head_dim 64, 12 units, 1 6.9 / 6.1, saving 1 7.0 / 7.1, 2 7.8 / 7.2.
+bool linear_fwd_shape_in_roles(int D, int K, int n_stages, long units, int hint, bool saves, int rest, int* cus) {
+  if (K != 16 || (hint & (TTT_HINT_WAVES_MASK | TTT_HINT_ALL_LOADS | TTT_HINT_OWN_LOADS)) != 0) return false;
+  if (n_stages < (rest > 0 ? 4 : D == 64 ? (saves ? 2 : 1) : (saves ? 8 : 4))) return false;
+  return device_cus(cus) == TTT_OK && units <= (D == 64 ? 1L : 2L) * *cus;
+}
 bool linear_fwd_in_roles(int D, const ttt::LinearFwdArgs* probs, int hint, unsigned ny, int rest, int* cus) {
   const ttt::LinearFwdArgs& a = probs[0];
-  if (a.K != 16 || (hint & (TTT_HINT_WAVES_MASK | TTT_HINT_ALL_LOADS | TTT_HINT_OWN_LOADS)) != 0 || any_input_sums(probs, ny)) return false;
+  if (any_input_sums(probs, ny)) return false;
   bool saves = false;
   for (unsigned y = 0; y < ny; ++y) saves = saves || probs[y].W_ckpt != nullptr;
-  if (a.n_stages < (rest > 0 ? 4 : D == 64 ? (saves ? 2 : 1) : (saves ? 8 : 4))) return false;
-  return device_cus(cus) == TTT_OK && (long)a.B * a.H * ny <= (D == 64 ? 1L : 2L) * *cus;
+  return linear_fwd_shape_in_roles(D, a.K, a.n_stages, (long)a.B * a.H * ny, hint, saves, rest, cus);
 }
 
 template <class T, int D>
@@ -1016,15 +1020,17 @@ int dispatch_linear_fwd_pack(const ttt_desc* d, const ttt::LinearFwdArgs* a, uns
 // `rest` tokens of a short mini-batch behind save the launch that they would take otherwise, and pay from four mini-batches on (the
 // fewest tried): on one workgroup and two launches / on two workgroups and one, 24 units, d = 64, 4 19.1 / 16.7, 8 25.7 / 20.9, 16 37.8 /
 // 29.1; d = 32, 4 13.8 / 12.8, 16 27.1 / 21.3; 128 units, d = 64, 4 20.2 / 18.3.
-bool linear_fwd_on_pairs(const ttt_desc* d, const ttt::LinearFwdArgs& a, ttt::LinearPairArgs* pa, int rest = 0) {
-  if (d->io_dtype != TTT_F32 || d->head_dim > 64 || a.K != 16) return false;
+bool linear_fwd_shape_on_pairs(const ttt_desc* d, int rest) {
+  if (d->io_dtype != TTT_F32 || d->head_dim > 64 || d->mini_batch != 16) return false;
   if (d->kernel_hint & (TTT_HINT_WAVES_MASK | TTT_HINT_ALL_LOADS | TTT_HINT_ONE_WORKGROUP)) return false;
-  if (a.n_stages < (rest > 0 ? 4 : 16)) return false;
-  if (rest > 0 && !aligned16(a.W_out)) return false;  // the short mini-batch's G'' crosses there, 16 bytes a lane; else W_out goes by elements
-  const size_t units = (size_t)a.B * a.H;
+  if (d->seq / 16 < (rest > 0 ? 4 : 16)) return false;
   int cus = 0;
-  if (device_cus(&cus) != TTT_OK || (units + 7) / 8 * 16 > (size_t)cus) return false;
-  const size_t D = (size_t)d->head_dim, tokens = (units - 1) * a.seq_stride + d->seq + rest, states = d->state_per_batch ? units : (size_t)a.H;
+  return device_cus(&cus) == TTT_OK && ((size_t)d->batch * d->heads + 7) / 8 * 16 <= (size_t)cus;
+}
+bool linear_fwd_on_pairs(const ttt_desc* d, const ttt::LinearFwdArgs& a, ttt::LinearPairArgs* pa, int rest = 0) {
+  if (!linear_fwd_shape_on_pairs(d, rest)) return false;
+  if (rest > 0 && !aligned16(a.W_out)) return false;  // the short mini-batch's G'' crosses there, 16 bytes a lane; else W_out goes by elements
+  const size_t units = (size_t)a.B * a.H, D = (size_t)d->head_dim, tokens = (units - 1) * a.seq_stride + d->seq + rest, states = d->state_per_batch ? units : (size_t)a.H;
   const size_t saved = a.W_ckpt != nullptr ? units * a.n_ckpt : 0;
   struct Range {
     const void* p;
@@ -1075,6 +1081,20 @@ int ttt_linear_fwd(const ttt_desc* d, const void* xq, const void* xk, const void
   if (linear_fwd_on_pairs(d, a, &pa))
     return hip_status(ttt::launch_linear_fwd_pair(d->head_dim, a, pa, static_cast<hipStream_t>(stream)), "ttt_linear_fwd launch");
   return dispatch_linear_fwd(d, &a, 1, static_cast<hipStream_t>(stream));
+}
+
+int ttt_linear_fwd_takes_rest(const ttt_desc* d, int32_t rest) {
+  char kept[sizeof(g_err)];  // "no" is an answer, not a failure of the thread's
+  memcpy(kept, g_err, sizeof(kept));
+  bool takes = ttt_linear_supported(d) == TTT_OK && rest > 0 && rest < d->mini_batch && d->seq_stride >= (int64_t)d->seq + rest;
+  if (takes) {
+    int cus = 0;
+    takes = d->io_dtype == TTT_F32 ? linear_fwd_shape_on_pairs(d, rest)
+                                   : d->head_dim <= 64 && linear_fwd_shape_in_roles(d->head_dim, d->mini_batch, d->seq / d->mini_batch,
+                                                                                   (long)d->batch * d->heads, d->kernel_hint, false, rest, &cus);
+  }
+  memcpy(g_err, kept, sizeof(kept));
+  return takes ? 1 : 0;
 }
 
 int ttt_linear_fwd_with_rest(const ttt_desc* d, int32_t rest, const void* xq, const void* xk, const void* xv,

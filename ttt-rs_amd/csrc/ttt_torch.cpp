@@ -306,9 +306,9 @@ PyObject* linear_layer_forward(PyObject* const* a) {
   if (calls == 2) {  // in one launch where there is one
     bool one = true;
     enqueue(q.dev, [&](void* s) {
-      const int rc = ttt_linear_fwd_with_rest(&desc[0], (int32_t)rest, pq, pk, pv, W0, b0, te, pl, gam, bet, po, ptr(W[0]), ptr(b[0]), s);
-      one = rc != TTT_ERR_UNSUPPORTED;
-      return one ? rc : (int)TTT_OK;
+      one = ttt_linear_fwd_takes_rest(&desc[0], (int32_t)rest) == 1;
+      return one ? ttt_linear_fwd_with_rest(&desc[0], (int32_t)rest, pq, pk, pv, W0, b0, te, pl, gam, bet, po, ptr(W[0]), ptr(b[0]), s)
+                 : (int)TTT_OK;
     });
     if (one) return wrap_tuple({&out, &W[0], &b[0]});
     W[1] = empty(W4, at::kFloat, q.dev);
