@@ -125,6 +125,9 @@ typedef struct ttt_desc {
  * described at ttt_mlp_fwd: every output of the affected units is NaN.  All kernels still run to their end.  (ttt_mlpn_fwd and
  * ttt_linear_fwd: likewise, and the units are computed again.) */
 #define TTT_HINT_TEST_LOST_PARTNER 0x200
+/* Testing only, ttt_linear_fwd on two workgroups per unit: the second gives up waiting half way through the mini-batches, when it has
+ * put final rows where the first still writes. */
+#define TTT_HINT_TEST_LOST_HALFWAY 0x10000
 /* Testing only: the same two workgroups treat each other as running on different XCDs whatever they find at start,
  * i.e. take the path of a pair that was not placed on one XCD: every word they exchange is stored at device scope
  * instead of staying in the XCD's L2.  Slower; results identical. */

@@ -1,6 +1,6 @@
 """ttt_linear_fwd, f32 I/O, with a unit on two workgroups: the same bits as on one (TTT_HINT_ONE_WORKGROUP), output, final state and
 checkpoints, also where the two do not share an L2 (a release per mini-batch), where buffers that do not qualify keep a unit
-on one, and where the consumer waits in vain and the unit is computed again."""
+on one, and where the consumer waits in vain, from the start or half way, and the unit is computed again."""
 import ctypes
 import importlib
 
@@ -12,7 +12,7 @@ from test_linear_fwd_gpu import oracle_case
 
 pytestmark = pytest.mark.gpu
 
-ONE, LOST, OTHER_XCD = 0x8000, 0x200, 0x800
+ONE, LOST, OTHER_XCD, HALFWAY = 0x8000, 0x200, 0x800, 0x10000
 K = 16
 
 
@@ -75,7 +75,7 @@ def test_same_bits_as_on_one_workgroup(P, d, B, H, N):
     print(f"case linear pair d{d} B{B} H{H} N{N}", flush=True)
     c = make(P, d, B, H, N, 5100 + d + N)
     one = call(P, c, d, B, H, N, ONE)
-    for hint in (0, OTHER_XCD, LOST):
+    for hint in (0, OTHER_XCD, LOST, HALFWAY):
         for i, (x, y) in enumerate(zip(one, call(P, c, d, B, H, N, hint))):
             assert torch.equal(x, y), f"output {i}, hint {hint:#x}"
     for name, got, ref in zip(("out", "W", "b"), one, oracle_case(c, K)):
@@ -88,7 +88,7 @@ def test_checkpoints(P, d, B, H, N, ckpt, ci):
     print(f"case linear pair checkpoints d{d} N{N} fmt{ckpt} ci{ci}", flush=True)
     c = make(P, d, B, H, N, 5200 + d)
     one = call(P, c, d, B, H, N, ONE, ckpt, ci)
-    for hint in (0, LOST):
+    for hint in (0, LOST, HALFWAY):
         for i, (x, y) in enumerate(zip(one, call(P, c, d, B, H, N, hint, ckpt, ci))):
             assert torch.equal(x, y), f"output {i}, hint {hint:#x}"
 
@@ -100,7 +100,7 @@ def test_other_calls(P, what):
     c = make(P, d, B, H, N, 5300, no_update=what == "no update")
     kw = {"window": 16} if what == "window" else {"in_place": (what.split()[0],)} if "in place" in what else {}
     one = call(P, c, d, B, H, N, ONE, **kw)
-    for hint in (0, OTHER_XCD, LOST):
+    for hint in (0, OTHER_XCD, LOST, HALFWAY):
         for i, (x, y) in enumerate(zip(one, call(P, c, d, B, H, N, hint, **kw))):
             assert torch.equal(x, y), f"output {i}, hint {hint:#x}"
     if what == "no update":

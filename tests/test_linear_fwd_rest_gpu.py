@@ -11,7 +11,7 @@ from helpers import to_dev
 
 pytestmark = pytest.mark.gpu
 
-ONE, LOST, OTHER_XCD = 0x8000, 0x200, 0x800
+ONE, LOST, OTHER_XCD, HALFWAY = 0x8000, 0x200, 0x800, 0x10000
 K = 16
 
 
@@ -73,7 +73,7 @@ def test_equals_two_launches(P, d, B, H, N, rest, no_update):
     if no_update:  # the short mini-batch leaves the state as it is
         v["token_eta"][-1] = 0.0
     two = run(P, v, d, B, H, N, rest, ONE, False)
-    for hint in (0, OTHER_XCD, LOST):
+    for hint in (0, OTHER_XCD, LOST, HALFWAY):
         for i, (x, y) in enumerate(zip(two, run(P, v, d, B, H, N, rest, hint, True))):
             assert torch.equal(x, y), f"output {i}, hint {hint:#x}"
 

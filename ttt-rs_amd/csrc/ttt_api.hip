@@ -4,6 +4,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <climits>
 #include <cstdarg>
 #include <cstdio>
 #include <cstdlib>
@@ -1051,7 +1052,10 @@ bool linear_fwd_on_pairs(const ttt_desc* d, const ttt::LinearFwdArgs& a, ttt::Li
     for (const Range& o : res)
       if (&o != &r && o.n != 0 && !apart(r, o)) return false;
   }
-  pa->spin_limit = (d->kernel_hint & TTT_HINT_TEST_LOST_PARTNER) ? 0u : 1u << 21;
+  pa->spin_limit = 1u << 21;
+  pa->lose_at = (d->kernel_hint & TTT_HINT_TEST_LOST_PARTNER)   ? 0
+                : (d->kernel_hint & TTT_HINT_TEST_LOST_HALFWAY) ? (a.n_stages + (rest > 0 ? 1 : 0)) / 2
+                                                                : INT_MAX;
   pa->agent_release = (d->kernel_hint & TTT_HINT_TEST_OTHER_XCD) ? 1 : 0;
   pa->rest = rest;
   return true;

@@ -29,7 +29,8 @@
 namespace ttt {
 
 struct LinearPairArgs {
-  unsigned spin_limit;  // polls before the consumer gives up; 0: at once (tests of that path)
+  unsigned spin_limit;  // polls before the consumer gives up
+  int lose_at;          // the mini-batch from which on it does not wait at all (tests of that path), or INT_MAX
   int agent_release;    // 1: always publish with a device-scope release
   int rest;             // REST: tokens of the short mini-batch behind the a.n_stages whole ones, 1 .. 15
 };
@@ -151,7 +152,7 @@ __device__ __forceinline__ void linear_fwd_pair_body(const LinearFwdArgs& a, con
     } else {
       if (lane == 0) __hip_atomic_store(words + kLinPairXcd, xcd, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       const unsigned g0 = lds_addr(&L.g[0][0][0]);
-      bool lost = pa.spin_limit == 0;
+      bool lost = false;
       int known = 0, next = 0;  // mini-batches handed over; the next to copy
       centre();
       asm volatile("s_barrier" ::: "memory");
@@ -159,6 +160,7 @@ __device__ __forceinline__ void linear_fwd_pair_body(const LinearFwdArgs& a, con
         if (REST && st == n - 1) asm volatile("s_barrier" ::: "memory");  // of StateBetween
         // G'' of mini-batch st in LDS in front of the barrier of st, and of the next two if they are there: the slot of st + 2 was
         // last read behind the barrier of st - 2, which every wave left in front of that of st - 1
+        if (st >= pa.lose_at) lost = true;
         if (!lost && known < n) {
           for (unsigned polls = 0;; ++polls) {
             known = (int)look(words + kLinPairCount);
