@@ -58,7 +58,8 @@ def make(P, d, B, H, N, no_update=False):
     return c
 
 
-# one mini-batch, around the ring of eight, odd and even; a unit per CU, more (an odd number too), two per CU
+# one mini-batch, around the ring of eight, odd and even; a unit per CU, more (an odd number too), two per CU (head_dim 32; at 64 these
+# are the two-wave kernel's)
 @pytest.mark.parametrize("d", [32, 64])
 @pytest.mark.parametrize("B,H,N", [(1, 1, 1), (1, 2, 2), (1, 3, 3), (2, 3, 7), (2, 3, 8), (3, 3, 9), (2, 5, 18), (16, 16, 5), (17, 16, 4),
                                    (24, 16, 11), (32, 16, 3), (257, 1, 3)])
@@ -76,7 +77,7 @@ def test_same_bits_as_two_waves(P, d, B, H, N):
 
 @pytest.mark.parametrize("d", [32, 64])
 @pytest.mark.parametrize("ckpt,ci", [(0, 1), (0, 3), (1, 1), (2, 1)])
-@pytest.mark.parametrize("B,H,N", [(2, 3, 10), (18, 16, 3)])
+@pytest.mark.parametrize("B,H,N", [(2, 3, 10), (18, 16, 3), (1, 3, 1), (2, 3, 2), (3, 3, 3), (257, 1, 10), (32, 16, 9), (16, 16, 7)])
 def test_saved(P, d, B, H, N, ckpt, ci):
     print(f"case linear roles saved d{d} B{B} H{H} N{N} fmt{ckpt} ci{ci}", flush=True)
     v = to_dev(make(P, d, B, H, N))
@@ -133,7 +134,8 @@ def test_rest_equals_two_launches(P, d, B, H, N, rest, no_update):
 
 # one mini-batch, around the ring of eight; more than a unit per CU (head_dim 32)
 @pytest.mark.parametrize("rope", [False, True])
-@pytest.mark.parametrize("d,B,H,N", [(64, 1, 3, 1), (64, 2, 5, 2), (64, 2, 3, 9), (64, 1, 12, 20), (64, 24, 16, 9), (32, 2, 3, 4), (32, 1, 5, 7), (32, 20, 16, 10)])
+@pytest.mark.parametrize("d,B,H,N", [(64, 1, 3, 1), (64, 2, 5, 2), (64, 2, 3, 9), (64, 1, 12, 20), (64, 24, 16, 9), (32, 2, 3, 4), (32, 1, 5, 7), (32, 20, 16, 10),
+                                     (32, 1, 3, 1), (32, 2, 3, 2), (32, 257, 1, 3)])
 def test_operands_formed_from_projections(P, d, B, H, N, rope):
     """The fused call without copies of the operands against forming them first: the same bits."""
     print(f"case linear roles formed d{d} B{B} H{H} N{N} rope{rope}", flush=True)
@@ -143,7 +145,10 @@ def test_operands_formed_from_projections(P, d, B, H, N, rope):
     x = [r(B, seq, H, d).bfloat16() for _ in range(3)]
     args = (*x, r(B, seq, H).bfloat16(), r(H) * 0.5, 0.8, 1.0 / torch.arange(1, K + 1, dtype=torch.float32, device=dev), r(K) * 0.1)
     state = (r(H, d, d) * 0.02, r(H, d) * 0.02, 1.0 + 0.1 * r(H, d), 0.1 * r(H, d))
-    pos = dict(rope=P.rope_cos_sin(K, 0, None, d, dev), pos_offset=5, pos_wrap=K) if rope else {}
+    _same_formed(P, args, state, dict(rope=P.rope_cos_sin(K, 0, None, d, dev), pos_offset=5, pos_wrap=K) if rope else {})
+
+
+def _same_formed(P, args, state, pos):
     got = P.ttt_linear_forward_fused_inputs_raw(*args, *state, K, **pos)
     ins = P.inner_loop_inputs_raw(*args, K, **pos)
     want = P.ttt_linear_forward_raw(ins.qkv.xq, ins.qkv.xk, ins.qkv.xv, state[0], state[1], ins.token_eta, ins.ttt_lr_eta, *state[2:], K,

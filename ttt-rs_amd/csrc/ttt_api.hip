@@ -220,20 +220,18 @@ int launch_linear_fwd_nw(const ttt::LinearFwdArgs* probs, unsigned ny, hipStream
 }
 
 // bf16 I/O, head_dim 32 / 64, mini-batches of 16: whether the waves of a unit take roles (ttt_linear_fwd_roles.hip.h), the same bits.
-// head_dim 64 up to a unit per CU, 32 up to two (both measured there).  Few mini-batches at head_dim 32 lose to the longer
-// way into the loop, more so where the launch saves: two waves / in roles, 12 units, 1 mini-batch 5.4 / 5.8, 3 5.92 / 5.97, 4 6.5 / 5.8,
-// 384 units 4 7.7 / 6.8; saving 4 6.7 / 7.1, 8 8.5 / 7.1; head_dim 64, 12 units, 1 6.9 / 6.1, saving 1 7.0 / 7.1, 2 7.8 / 7.2.
-bool linear_fwd_shape_in_roles(int D, int K, int n_stages, long units, int hint, bool saves, int rest, int* cus) {
+// head_dim 64 up to a unit per CU, 32 up to two (both measured there), from one mini-batch on: us with two waves / in roles, head_dim 32, 12 units,
+// 1 mini-batch 4.7 / 3.9, 2 5.2 / 4.4, 4 6.2 / 5.1, saving states 1 4.8 / 4.0, 4 6.5 / 5.3; 384 units 1 5.8 / 5.5, 4 7.7 / 7.0, saving 1 5.9 / 5.5, 4
+// 8.3 / 7.5; head_dim 64, 12 units, 1 6.7 / 6.2, saving 1 7.0 / 6.3, 4 9.8 / 8.2; 256 units 1 7.6 / 6.8, saving 1 8.1 / 7.3.  With a short mini-batch
+// behind from four on (the fewest tried).
+bool linear_fwd_shape_in_roles(int D, int K, int n_stages, long units, int hint, int rest, int* cus) {
   if (K != 16 || (hint & (TTT_HINT_WAVES_MASK | TTT_HINT_ALL_LOADS | TTT_HINT_OWN_LOADS)) != 0) return false;
-  if (n_stages < (rest > 0 ? 4 : D == 64 ? (saves ? 2 : 1) : (saves ? 8 : 4))) return false;
+  if (rest > 0 && n_stages < 4) return false;
   return device_cus(cus) == TTT_OK && units <= (D == 64 ? 1L : 2L) * *cus;
 }
 bool linear_fwd_in_roles(int D, const ttt::LinearFwdArgs* probs, int hint, unsigned ny, int rest, int* cus) {
   const ttt::LinearFwdArgs& a = probs[0];
-  if (any_input_sums(probs, ny)) return false;
-  bool saves = false;
-  for (unsigned y = 0; y < ny; ++y) saves = saves || probs[y].W_ckpt != nullptr;
-  return linear_fwd_shape_in_roles(D, a.K, a.n_stages, (long)a.B * a.H * ny, hint, saves, rest, cus);
+  return !any_input_sums(probs, ny) && linear_fwd_shape_in_roles(D, a.K, a.n_stages, (long)a.B * a.H * ny, hint, rest, cus);
 }
 
 template <class T, int D>
@@ -1095,7 +1093,7 @@ int ttt_linear_fwd_takes_rest(const ttt_desc* d, int32_t rest) {
     int cus = 0;
     takes = d->io_dtype == TTT_F32 ? linear_fwd_shape_on_pairs(d, rest)
                                    : d->head_dim <= 64 && linear_fwd_shape_in_roles(d->head_dim, d->mini_batch, d->seq / d->mini_batch,
-                                                                                   (long)d->batch * d->heads, d->kernel_hint, false, rest, &cus);
+                                                                                   (long)d->batch * d->heads, d->kernel_hint, rest, &cus);
   }
   memcpy(g_err, kept, sizeof(kept));
   return takes ? 1 : 0;
