@@ -156,3 +156,99 @@ def _same_formed(P, args, state, pos):
     torch.cuda.synchronize()
     for i, (a, b) in enumerate(zip(got, want)):
         assert torch.equal(a, b), f"output {i}"
+
+
+@pytest.mark.parametrize("wrap", [1, 2, 8])
+def test_operands_formed_with_positions_that_repeat_within_the_mini_batch(P, wrap):
+    d, B, H, N = 64, 1, 3, 3
+    print(f"case linear roles formed wrap {wrap}", flush=True)
+    dev, seq = "cuda:0", N * K
+    g = torch.Generator(device=dev).manual_seed(5900 + wrap)
+    r = lambda *s: torch.randn(*s, generator=g, device=dev)
+    x = [r(B, seq, H, d).bfloat16() for _ in range(3)]
+    args = (*x, r(B, seq, H).bfloat16(), r(H) * 0.5, 0.8, 1.0 / torch.arange(1, K + 1, dtype=torch.float32, device=dev), r(K) * 0.1)
+    state = (r(H, d, d) * 0.02, r(H, d) * 0.02, 1.0 + 0.1 * r(H, d), 0.1 * r(H, d))
+    _same_formed(P, args, state, dict(rope=P.rope_cos_sin(K, 0, None, d, dev), pos_offset=3, pos_wrap=wrap))
+
+
+@pytest.mark.parametrize("in_place", [False, True])
+@pytest.mark.parametrize("d,B,H", [(64, 2, 3), (32, 2, 3), (32, 20, 16)])
+def test_a_state_per_batch_element_carried_through_windows(P, d, B, H, in_place):
+    """Windows of 1, 3, 2 and 5 mini-batches of one sequence, each on the state the one before left, also over it in place."""
+    print(f"case linear roles carried d{d} B{B} {in_place}", flush=True)
+    N = 11
+    v = to_dev(make(P, d, B, H, N))
+    p = lambda t, at=0: ctypes.c_void_p(t.data_ptr() + t.element_size() * at)
+    s = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    res = []
+    for hint in (TWO_WAVES, 0):
+        out = torch.full_like(v["xq"], 7.0)
+        W, b = v["W0"].expand(B, H, d, d).contiguous(), v["b0"].expand(B, H, d).contiguous()
+        at = 0
+        for n in (1, 3, 2, 5):
+            desc = P.TttDesc(B, H, n * K, d, K, 1e-6, 1, P.TTT_BF16)
+            desc.kernel_hint, desc.seq_stride, desc.state_per_batch = hint, N * K, 1
+            Wn, bn = (W, b) if in_place else (torch.empty_like(W), torch.empty_like(b))
+            rc = P.lib().ttt_linear_fwd(ctypes.byref(desc), *[p(v[k], at * d) for k in ("xq", "xk", "xv")], p(W), p(b), p(v["token_eta"]),
+                                        p(v["lr"], at), p(v["gamma"]), p(v["beta"]), p(out, at * d), p(Wn), p(bn), None, None, s)
+            assert rc == 0, P.lib().ttt_last_error()
+            W, b, at = Wn, bn, at + n * K
+        torch.cuda.synchronize()
+        res.append((out, W, b))
+    for i, (x, y) in enumerate(zip(*res)):
+        assert torch.equal(x, y), f"output {i}"
+
+
+@pytest.mark.parametrize("what", ["xq", "xk", "xv", "lr"])
+@pytest.mark.parametrize("value", [float("inf"), float("nan"), 3e38])
+def test_extremes(P, what, value):
+    """In the last token of a mini-batch and, for a sequence that ends in a short one, in its last token."""
+    d, B, H, N, rest = 64, 1, 2, 5, 6
+    print(f"case linear roles extremes {what} {value}", flush=True)
+    v = to_dev(make(P, d, B, H, N))
+    v[what][:, 0, 2 * K - 1] = value
+    same = lambda x, y: torch.equal(x.isnan(), y.isnan()) and torch.equal(x.nan_to_num(0.0, 1.0, -1.0), y.nan_to_num(0.0, 1.0, -1.0))
+    for i, (x, y) in enumerate(zip(call(P, v, d, B, H, N, TWO_WAVES), call(P, v, d, B, H, N, 0))):
+        assert same(x.float(), y.float()), f"output {i}"
+    c = to_dev(P.synthetic.reference_test_inputs(5950, B, H, N * K + rest, d, K, io_dtype=torch.bfloat16))
+    c[what][:, 0, -1] = value
+    te = c["token_eta"].repeat(N + 1)[:N * K + rest].contiguous()
+    layer = P.FusedTileMulti(P.ModelConfig(H, d, P.TTTConfig(mini_batch_size=K)), c["W0"], c["b0"], c["gamma"], c["beta"])
+    x = P.TTTInputsInner(P.Qkv(c["xq"], c["xk"], c["xv"]), te, c["lr"])
+    one, two = layer.init_state(B), layer.init_state(B)
+    a = layer.forward(one, x)
+    whole = layer._pass(two, x, 0, N * K)
+    b = torch.cat([whole, layer.forward_mini_batch(two, x, range(N * K, N * K + rest))], 2)
+    for i, (p, q) in enumerate(((a, b), (one.weight, two.weight), (one.bias, two.bias))):
+        assert same(p.float(), q.float()), f"ragged, output {i}"
+
+
+def test_two_streams_and_replays(P):
+    """Calls at once that do not fit side by side; a captured call, replayed between eager ones."""
+    d, B, H, N = 64, 12, 16, 6
+    print("case linear roles streams, graph", flush=True)
+    v = to_dev(make(P, d, B, H, N))
+    args = (v["xq"], v["xk"], v["xv"], v["W0"], v["b0"], v["token_eta"], v["lr"], v["gamma"], v["beta"], K)
+    want = P.ttt_linear_forward_raw(*args, kernel_hint=TWO_WAVES)
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    got = []
+    for s in streams * 3:
+        with torch.cuda.stream(s):
+            got.append(P.ttt_linear_forward_raw(*args))
+    torch.cuda.synchronize()
+    for r in got:
+        for x, y in zip(r, want):
+            assert torch.equal(x, y)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        res = P.ttt_linear_forward_raw(*args)
+    for _ in range(3):
+        for t in res:
+            t.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        eager = P.ttt_linear_forward_raw(*args)
+        torch.cuda.synchronize()
+        for x, y, z in zip(res, want, eager):
+            assert torch.equal(x, y) and torch.equal(z, y)
