@@ -105,9 +105,16 @@ typedef struct ttt_desc {
  * exists (head_dim 96 / 128: own-feature loads).  Without either hint and without a number of waves, mini-batches of 16 run on a
  * kernel whose waves have roles (recurrence, output, copies) up to one unit per CU at head_dim 64 and two at 32: the same bits.
  * ttt_linear_fwd, f32 I/O with one wave per feature tile (head_dim 32 / 64), whole mini-batches of 16 tokens and at
- * most one (batch, head) unit per CU: the library's choice is a kernel with a fifth wave that copies the operands
+ * most one (batch, head) unit per CU: the library's choice is, with two CUs per unit and 16 or more mini-batches, two workgroups
+ * per unit (see ttt_linear_fwd), otherwise a kernel with a fifth wave that copies the operands
  * global -> LDS, so that the four compute waves issue no loads; TTT_HINT_ALL_LOADS keeps the loads in the compute
- * waves.  Same results bit for bit. */
+ * waves of one workgroup.  Same results bit for bit.
+ * Several callers on one GPU at a time (streams of their own): the library chooses for a launch that has the device to itself.  A unit
+ * whose waves have roles fills a CU at head_dim 64 and half of one at 32, a unit on two workgroups two CUs, and what does not fit
+ * beside other work waits for it.  Calls of 2048 tokens, us for both of two callers, as chosen / with TTT_HINT_OWN_LOADS: bf16,
+ * head_dim 64, 128 units each 89 / 122, 192 142 / 123, 256 168 / 137; head_dim 32, 256 83 / 101, 512 158 / 143; with
+ * TTT_HINT_ONE_WORKGROUP: f32, head_dim 64, 64 161 / 213, 96 259 / 214, 128 331 / 215.  So a caller whose streams together
+ * have more units than the device has room for sets the hint. */
 #define TTT_HINT_OWN_LOADS 0x1000
 #define TTT_HINT_ALL_LOADS 0x2000
 /* ttt_mlp_bwd / ttt_mlp_bwd_static, bf16 I/O up to head_dim 96: the reverse scan normally rounds the operands of its
@@ -130,7 +137,8 @@ typedef struct ttt_desc {
 #define TTT_HINT_TEST_LOST_HALFWAY 0x10000
 /* Testing only: the same two workgroups treat each other as running on different XCDs whatever they find at start,
  * i.e. take the path of a pair that was not placed on one XCD: every word they exchange is stored at device scope
- * instead of staying in the XCD's L2.  Slower; results identical. */
+ * instead of staying in the XCD's L2.  Slower; results identical.  (ttt_linear_fwd on two workgroups and the backward passes on
+ * two: likewise, what the first hands over is written back to memory.) */
 #define TTT_HINT_TEST_OTHER_XCD 0x800
 
 /* Library / build identification. */
